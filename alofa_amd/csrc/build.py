@@ -206,4 +206,5 @@ def load() -> ctypes.CDLL:
         except OSError as e:
             raise AlofaError("not_initialized", "the HIP library cannot be loaded", f"path={path} reason={e}") from None
         _lib.alofa_last_error.restype = ctypes.c_char_p
+        _lib.alofa_gemm_exact_parts.restype = ctypes.c_int64
     return _lib

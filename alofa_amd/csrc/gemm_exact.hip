@@ -1,0 +1,298 @@
+// Matrix products of the 32-bit path: out[m, n] = sum_k A[m, k] * W[n, k], float operands, every product and every sum in
+// float64 on the matrix cores (v_mfma_f64_16x16x4_f64), rounded to float once. W is stored [out, in].
+//
+// Lane l of the instruction holds A[row l % 16][k l / 16], B[k l / 16][column l % 16] and D[rows 4 v + l / 16, v = 0..3][column l % 16].
+// Which four k an instruction takes is free as long as both operands agree, so a lane takes four consecutive k (one 16-byte
+// load) for four instructions in a row.
+//
+// An output is the sum over k in a few float64 partial sums (waves, parts of K), added in a fixed order that depends on the sizes
+// only: two orders differ by some 2^-50 of the sum, which the one rounding to float hides but for one output in some ten million.
+//
+//   up to 16 rows (exact_rows_kernel): a block owns 16 weight rows (16 of gate and 16 of up), its waves take runs of 32 k in turn,
+//   straight from memory, and meet in LDS. Bound by reading the weights once: a wave's matrix instructions take 64 cycles for 64
+//   weights, half of what the memory brings. 8 rows, us before (a tile of 64 x 64 on the vector units, one block per 64 columns) and
+//   now: see the numbers at launch_exact.
+//
+//   more rows (exact_tile_kernel): slabs of 32 k through LDS, a wave owns 32 rows x 32 weight rows (four instructions for two
+//   loads of either operand), a block 64 x 64 (32 x 128 up to 32 rows). Bound by the matrix cores (69 TFLOP/s measured with
+//   nothing else in the loop): the slab's traffic hides behind 2,048 cycles of instructions. K is shared out over blocks
+//   where the tiles are fewer than twice the compute units; the shares' float64 sums go to a buffer of the caller's (not to the library's
+//   workspace, which one stream at a time may use) and a second launch adds them.
+#include "common.h"
+
+namespace alofa {
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kExactStore = 0, kExactResidual = 1;
+constexpr int kExactRows = 16;       // rows that exact_rows_kernel takes at most
+
+// four consecutive k of a row from `k` on: one 16-byte load, or, where rows are not 16-byte aligned, value by value; zeros beyond K
+template <bool kVec>
+__device__ __forceinline__ float4 quad(const float* row, int k, int K) {
+  if constexpr (kVec) {
+    return k < K ? *reinterpret_cast<const float4*>(row + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+  } else {
+    return make_float4(k < K ? row[k] : 0.f, k + 1 < K ? row[k + 1] : 0.f, k + 2 < K ? row[k + 2] : 0.f, k + 3 < K ? row[k + 3] : 0.f);
+  }
+}
+
+__device__ __forceinline__ f64x4 fma_quad(float4 a, float4 b, f64x4 acc) {
+  acc = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(a.x), static_cast<double>(b.x), acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(a.y), static_cast<double>(b.y), acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(a.z), static_cast<double>(b.z), acc, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(a.w), static_cast<double>(b.w), acc, 0, 0, 0);
+}
+
+template <int kEpilogue>
+__device__ __forceinline__ void put(float* dst, double sum) {
+  const float v = static_cast<float>(sum);
+  *dst = kEpilogue == kExactResidual ? *dst + v : v;
+}
+
+// both products are rounded to float first, then the activation and the product in float64
+__device__ __forceinline__ float gated(double g, double u, int gelu) {
+  return static_cast<float>(gate_of(static_cast<double>(static_cast<float>(g)), gelu != 0) * static_cast<double>(static_cast<float>(u)));
+}
+
+// NW waves; kMats = 2: gate and up. NT tiles of 16 weight rows a block (of each matrix).
+template <int NW, int NT, int kMats, int kEpilogue, bool kVec>
+__global__ void __launch_bounds__(64 * NW) exact_rows_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ A, int64_t lda,
+                                                             const float* __restrict__ W, const float* __restrict__ W2, int64_t ldw,
+                                                             const float* __restrict__ bias, int M, int N, int K, int gelu) {
+  constexpr int kTiles = NT * kMats;
+  __shared__ double sums[NW][kTiles][4][64];
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
+  const int n0 = blockIdx.x * 16 * NT;
+  const bool row_ok = r < M;
+  const float* a_row = A + static_cast<int64_t>(row_ok ? r : 0) * lda;
+  const float* w_row[kTiles];
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) {
+    const int n = n0 + (t / kMats) * 16 + r;
+    w_row[t] = (t % kMats ? W2 : W) + static_cast<int64_t>(n < N ? n : N - 1) * ldw;      // (rows beyond N: the last one again, not stored)
+  }
+  f64x4 acc[kTiles];
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) acc[t] = f64x4{0, 0, 0, 0};
+  // runs of 32 k: a lane takes 8 g .. 8 g + 7 of each; the next run is on its way while one is multiplied
+  float4 a0, a1, w0[kTiles], w1[kTiles];
+  auto fetch = [&](int k) __attribute__((always_inline)) {
+    a0 = quad<kVec>(a_row, k, K), a1 = quad<kVec>(a_row, k + 4, K);
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) w0[t] = quad<kVec>(w_row[t], k, K), w1[t] = quad<kVec>(w_row[t], k + 4, K);
+  };
+  int k = wave * 32 + g * 8;
+  if (wave * 32 < K) fetch(k);
+  for (int k0 = wave * 32; k0 < K; k0 += NW * 32) {
+    float4 ca0 = a0, ca1 = a1, cw0[kTiles], cw1[kTiles];
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) cw0[t] = w0[t], cw1[t] = w1[t];
+    k += NW * 32;
+    if (k0 + NW * 32 < K) fetch(k);
+    if (!row_ok) ca0 = ca1 = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+      acc[t] = fma_quad(cw0[t], ca0, acc[t]);
+      acc[t] = fma_quad(cw1[t], ca1, acc[t]);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) sums[wave][t][v][lane] = acc[t][v];
+  __syncthreads();
+  // an output a thread: tile, weight row i = 4 v + g', row of A j: place (v, 16 g' + j)
+  for (int i = threadIdx.x; i < NT * 256; i += 64 * NW) {
+    const int tile = i / 256, v = i / 64 % 4, at = i % 64, m = at % 16, n = n0 + tile * 16 + 4 * v + at / 16;
+    if (m >= M || n >= N) continue;
+    double s[kMats];
+#pragma unroll
+    for (int x = 0; x < kMats; ++x) {
+      s[x] = bias ? static_cast<double>(bias[n]) : 0.0;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) s[x] += sums[w][tile * kMats + x][v][at];
+    }
+    float* dst = out + static_cast<int64_t>(m) * ldo + n;
+    if constexpr (kMats == 2) *dst = gated(s[0], s[1], gelu);
+    else put<kEpilogue>(dst, s[0]);
+  }
+}
+
+// A block of WM x (4 / WM) waves, each 32 rows x 32 weight rows; kMats = 2: the weight rows of a wave are 16 of gate and the same 16 of up.
+// parts (with gridDim.z > 1): this share's sums, [share][M][N]; the epilogue is then the second launch's.
+template <int WM, int kMats, int kEpilogue, bool kVec>
+__global__ void __launch_bounds__(256) exact_tile_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ A, int64_t lda,
+                                                         const float* __restrict__ W, const float* __restrict__ W2, int64_t ldw,
+                                                         const float* __restrict__ bias, double* __restrict__ parts, int M, int N, int K, int k_share, int gelu) {
+  constexpr int WN = 4 / WM, BM = 32 * WM, BW = 32 * WN, BK = 32, kPad = 4;
+  constexpr int kOwn = 32 / kMats;                     // outputs of a wave along N
+  __shared__ __attribute__((aligned(16))) float As[BM][BK + kPad], Ws[BW][BK + kPad];
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
+  const int wm = wave / WN, wn = wave % WN;
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * WN * kOwn;
+  const int k_begin = blockIdx.z * k_share, k_end = k_begin + k_share < K ? k_begin + k_share : K;
+  constexpr int kA = BM * BK / 4 / 256, kW = BW * BK / 4 / 256;      // quads a thread brings of either operand
+  float4 fa[kA], fw[kW];
+  auto fetch = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kA; ++i) {
+      const int at = threadIdx.x + i * 256, row = at / 8, m = m0 + row;
+      fa[i] = quad<kVec>(A + static_cast<int64_t>(m < M ? m : M - 1) * lda, k0 + at % 8 * 4, k_end);
+    }
+#pragma unroll
+    for (int i = 0; i < kW; ++i) {
+      const int at = threadIdx.x + i * 256, row = at / 8, n = n0 + row / 32 * kOwn + row % kOwn;
+      fw[i] = quad<kVec>((kMats == 2 && row % 32 >= 16 ? W2 : W) + static_cast<int64_t>(n < N ? n : N - 1) * ldw, k0 + at % 8 * 4, k_end);
+    }
+  };
+  f64x4 acc[2][2];      // [rows of A][weight rows]
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f64x4{0, 0, 0, 0};
+  fetch(k_begin);
+  for (int k0 = k_begin; k0 < k_end; k0 += BK) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kA; ++i) *reinterpret_cast<float4*>(&As[(threadIdx.x + i * 256) / 8][threadIdx.x % 8 * 4]) = fa[i];
+#pragma unroll
+    for (int i = 0; i < kW; ++i) *reinterpret_cast<float4*>(&Ws[(threadIdx.x + i * 256) / 8][threadIdx.x % 8 * 4]) = fw[i];
+    __syncthreads();
+    if (k0 + BK < k_end) fetch(k0 + BK);
+#pragma unroll
+    for (int q = 0; q < BK / 16; ++q) {
+      float4 a[2], w[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        a[i] = *reinterpret_cast<const float4*>(&As[wm * 32 + i * 16 + r][q * 16 + g * 4]);
+        w[i] = *reinterpret_cast<const float4*>(&Ws[wn * 32 + i * 16 + r][q * 16 + g * 4]);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = fma_quad(a[i], w[j], acc[i][j]);
+    }
+  }
+  // D: rows of A 4 v + g, weight row r
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int m = m0 + wm * 32 + i * 16 + 4 * v + g;
+      if (m >= M) continue;
+      if constexpr (kMats == 2) {
+        const int n = n0 + wn * 16 + r;
+        if (n < N) out[static_cast<int64_t>(m) * ldo + n] = gated(acc[i][0][v], acc[i][1][v], gelu);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int n = n0 + wn * 32 + j * 16 + r;
+          if (n >= N) continue;
+          if (parts) parts[(static_cast<int64_t>(blockIdx.z) * M + m) * N + n] = acc[i][j][v];
+          else put<kEpilogue>(out + static_cast<int64_t>(m) * ldo + n, (bias ? static_cast<double>(bias[n]) : 0.0) + acc[i][j][v]);
+        }
+      }
+    }
+}
+
+// The shares' sums in their order, then the epilogue.
+template <int kEpilogue>
+__global__ void __launch_bounds__(256) exact_sum_kernel(float* __restrict__ out, int64_t ldo, const double* __restrict__ parts, const float* __restrict__ bias,
+                                                        int M, int N, int shares) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, all = static_cast<int64_t>(M) * N;
+  if (i >= all) return;
+  const int n = i % N;
+  double s = bias ? static_cast<double>(bias[n]) : 0.0;
+  double p[16];
+#pragma unroll
+  for (int x = 0; x < 16; ++x) p[x] = x < shares ? parts[x * all + i] : 0.0;
+#pragma unroll
+  for (int x = 0; x < 16; ++x) s += p[x];
+  put<kEpilogue>(out + i / N * ldo + n, s);
+}
+
+// Up to 16 rows: blocks of eight waves (four in the gated form, whose blocks are many), sixteen where the blocks of 16 weight rows are fewer than
+// half the compute units; four tiles of weight rows a block against a matrix as long as a vocabulary, so that the rows of A are read a quarter as often.
+template <int kMats, int kEpilogue, bool kVec>
+static int launch_exact_rows(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, const float* W2, int64_t ldw, const float* bias,
+                             int M, int N, int K, int gelu, hipStream_t stream) {
+  const int tiles = (N + 15) / 16, cus = compute_units();
+  if (kMats == 1 && tiles >= 16 * cus)
+    exact_rows_kernel<4, 4, 1, kEpilogue, kVec><<<(tiles + 3) / 4, 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, gelu);
+  else if (kMats == 1 && tiles * 2 < cus && K >= 2048)
+    exact_rows_kernel<16, 1, kMats, kEpilogue, kVec><<<tiles, 1024, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, gelu);
+  else if (kMats == 1 || tiles < cus)
+    exact_rows_kernel<8, 1, kMats, kEpilogue, kVec><<<tiles, 512, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, gelu);
+  else
+    exact_rows_kernel<4, 1, kMats, kEpilogue, kVec><<<tiles, 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, gelu);
+  return check_launch("gemm_exact_rows");
+}
+
+// How K is shared out over blocks: blocks for two rounds of the compute units, at least 128 k a share, at most 16 shares. Returns k a share (a multiple
+// of a slab). Up to 16 rows and in the gated form K is not shared out.
+static int exact_share(int M, int N, int K) {
+  const int BM = M <= 32 ? 32 : 64, BW = M <= 32 ? 128 : 64;
+  const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BW - 1) / BW);
+  int64_t shares = (2 * compute_units() + tiles - 1) / tiles;
+  shares = shares < K / 128 ? shares : K / 128;
+  shares = M <= kExactRows || shares < 1 ? 1 : shares > 16 ? 16 : shares;
+  return static_cast<int>(((K + shares - 1) / shares + 31) / 32 * 32);
+}
+
+template <int WM, int kMats, int kEpilogue, bool kVec>
+static int launch_exact_tile(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, const float* W2, int64_t ldw, const float* bias,
+                             double* parts, int M, int N, int K, int gelu, hipStream_t stream) {
+  constexpr int BM = 32 * WM, kOut = 32 * (4 / WM) / kMats;
+  const int k_share = kMats == 1 ? exact_share(M, N, K) : K, shares = (K + k_share - 1) / k_share;
+  dim3 grid((N + kOut - 1) / kOut, (M + BM - 1) / BM, shares);
+  exact_tile_kernel<WM, kMats, kEpilogue, kVec><<<grid, 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, shares > 1 ? parts : nullptr, M, N, K, k_share, gelu);
+  if (shares > 1) {
+    const int64_t all = static_cast<int64_t>(M) * N;
+    exact_sum_kernel<kEpilogue><<<static_cast<unsigned>((all + 255) / 256), 256, 0, stream>>>(out, ldo, parts, bias, M, N, shares);
+  }
+  return check_launch("gemm_exact_tile");
+}
+
+template <int kMats, int kEpilogue>
+static int launch_exact(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, const float* W2, int64_t ldw, const float* bias,
+                        double* parts, int M, int N, int K, int gelu, hipStream_t stream) {
+  auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && aligned(A) && aligned(W) && aligned(W2);
+  if (M <= kExactRows)
+    return vec ? launch_exact_rows<kMats, kEpilogue, true>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, gelu, stream)
+               : launch_exact_rows<kMats, kEpilogue, false>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, gelu, stream);
+  if (M <= 32)
+    return vec ? launch_exact_tile<1, kMats, kEpilogue, true>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, stream)
+               : launch_exact_tile<1, kMats, kEpilogue, false>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, stream);
+  return vec ? launch_exact_tile<2, kMats, kEpilogue, true>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, stream)
+             : launch_exact_tile<2, kMats, kEpilogue, false>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, stream);
+}
+
+}  // namespace alofa
+
+using namespace alofa;
+
+// Float64 sums that alofa_gemm_exact needs room for with these sizes (0: none).
+extern "C" int64_t alofa_gemm_exact_parts(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const int k_share = exact_share(M, N, K), shares = (K + k_share - 1) / k_share;
+  return shares > 1 ? static_cast<int64_t>(shares) * M * N : 0;
+}
+
+extern "C" int alofa_gemm_exact(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, int64_t ldw, const float* bias, double* parts, int64_t room,
+                                int M, int N, int K, int epilogue, hipStream_t stream) {
+  ALOFA_REQUIRE(M > 0 && N > 0 && K > 0, "gemm: M=%d N=%d K=%d must be positive", M, N, K);
+  ALOFA_REQUIRE(epilogue == kExactStore || epilogue == kExactResidual, "gemm: unknown epilogue %d", epilogue);
+  ALOFA_REQUIRE(lda >= K && ldw >= K && ldo >= N, "gemm: a leading dimension is shorter than its row");
+  ALOFA_REQUIRE(room >= alofa_gemm_exact_parts(M, N, K), "gemm: no room for the sums of the shares of K");
+  if (epilogue == kExactStore) return launch_exact<1, kExactStore>(out, ldo, A, lda, W, W, ldw, bias, parts, M, N, K, 0, stream);
+  return launch_exact<1, kExactResidual>(out, ldo, A, lda, W, W, ldw, bias, parts, M, N, K, 0, stream);
+}
+
+extern "C" int alofa_gemm_swiglu_exact(float* out, int64_t ldo, const float* A, int64_t lda, const float* Wg, const float* Wu, int64_t ldw, int M, int N, int K,
+                                       int gelu, hipStream_t stream) {
+  ALOFA_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_swiglu: M=%d N=%d K=%d must be positive", M, N, K);
+  ALOFA_REQUIRE(lda >= K && ldw >= K && ldo >= N, "gemm_swiglu: a leading dimension is shorter than its row");
+  return launch_exact<2, kExactStore>(out, ldo, A, lda, Wg, Wu, ldw, nullptr, nullptr, M, N, K, gelu, stream);
+}

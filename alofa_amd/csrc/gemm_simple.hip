@@ -5,9 +5,9 @@
 // Every output element has one accumulator that starts at the bias and takes
 // the products in ascending k, whatever M is and wherever the row lies in the
 // batch: a row's result does not depend on what else is computed with it.
-// Acc = double gives the float32 model with float64 accumulation; Acc = float is
-// the plain float path. These kernels are the slow, always-valid path; the
-// MFMA and skinny kernels take over where their shapes fit.
+// These kernels are the slow, always-valid path with float sums; the MFMA and
+// skinny kernels take over where their shapes fit, and the 32-bit path with
+// float64 sums has kernels of its own (gemm_exact.hip).
 #include "common.h"
 
 namespace alofa {
@@ -169,7 +169,7 @@ static int launch_gemm_swiglu(void* out, int64_t ldo, const void* A, int64_t lda
 
 using namespace alofa;
 
-// Dtypes: a = activations in, w = weights, o = out. exact != 0 needs all float.
+// Dtypes: a = activations in, w = weights, o = out. exact != 0 is refused: such calls with float operands go to alofa_gemm_exact.
 extern "C" int alofa_gemm_simple(void* out, int o_dtype, int64_t ldo, const void* A, int a_dtype, int64_t lda,
                                  const void* W, int w_dtype, int64_t ldw, const float* bias, int M, int N, int K,
                                  int epilogue, int exact, hipStream_t stream) {
@@ -177,10 +177,7 @@ extern "C" int alofa_gemm_simple(void* out, int o_dtype, int64_t ldo, const void
   ALOFA_REQUIRE(epilogue == kStore || epilogue == kAddToResidual, "gemm: unknown epilogue %d", epilogue);
   ALOFA_REQUIRE(epilogue != kAddToResidual || o_dtype == kF32, "gemm: the residual stream is float");
   ALOFA_REQUIRE(lda >= K && ldw >= K && ldo >= N, "gemm: a leading dimension is shorter than its row");
-  if (exact) {
-    ALOFA_REQUIRE(a_dtype == kF32 && w_dtype == kF32 && o_dtype == kF32, "gemm: the exact path takes float operands only");
-    return launch_gemm<float, float, float, double>(out, ldo, A, lda, W, ldw, bias, M, N, K, epilogue, stream);
-  }
+  ALOFA_REQUIRE(!exact, "gemm: the exact path takes float operands only");
 #define ALOFA_GEMM_CASE(ad, wd, od, TA, TW, TO) \
   if (a_dtype == ad && w_dtype == wd && o_dtype == od) \
     return launch_gemm<TA, TW, TO, float>(out, ldo, A, lda, W, ldw, bias, M, N, K, epilogue, stream);
@@ -198,10 +195,7 @@ extern "C" int alofa_gemm_swiglu_simple(void* out, int o_dtype, int64_t ldo, con
                                         int K, int gelu, int exact, hipStream_t stream) {
   ALOFA_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_swiglu: M=%d N=%d K=%d must be positive", M, N, K);
   ALOFA_REQUIRE(lda >= K && ldw >= K && ldo >= N, "gemm_swiglu: a leading dimension is shorter than its row");
-  if (exact) {
-    ALOFA_REQUIRE(a_dtype == kF32 && w_dtype == kF32 && o_dtype == kF32, "gemm_swiglu: the exact path takes float operands only");
-    return launch_gemm_swiglu<float, float, float, double>(out, ldo, A, lda, Wg, Wu, ldw, M, N, K, gelu, stream);
-  }
+  ALOFA_REQUIRE(!exact, "gemm_swiglu: the exact path takes float operands only");
   if (a_dtype == kBF16 && w_dtype == kBF16 && o_dtype == kBF16)
     return launch_gemm_swiglu<bf16_t, bf16_t, bf16_t, float>(out, ldo, A, lda, Wg, Wu, ldw, M, N, K, gelu, stream);
   if (a_dtype == kBF16 && w_dtype == kF32 && o_dtype == kBF16)

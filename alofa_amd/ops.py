@@ -407,6 +407,14 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[tor
         if then_rows is not None and not done.value:
             rmsnorm(then_rows, out, then_w, then_eps, False)
         return
+    if exact and a.dtype is torch.float32 and w.dtype is torch.float32 and out.dtype is torch.float32:
+        room = load().alofa_gemm_exact_parts(_I(M), _I(N), _I(K))      # (sums of the shares of K, where the tiles are too few for the chip)
+        parts = torch.empty(room, dtype=torch.float64, device=out.device) if room else None
+        _call("alofa_gemm_exact", _ptr(out), _L(_rows("out", out)), _ptr(a), _L(_rows("a", a)), _ptr(w), _L(_rows("w", w)), _ptr(bias), _ptr(parts), _L(room),
+              _I(M), _I(N), _I(K), _I(ADD_TO_RESIDUAL if add_to_out else STORE), _stream())
+        if then_rows is not None:
+            rmsnorm(then_rows, out, then_w, then_eps, exact)
+        return
     _call("alofa_gemm_simple", _ptr(out), _I(dtype_code(out)), _L(_rows("out", out)), _ptr(a), _I(dtype_code(a)), _L(_rows("a", a)),
           _ptr(w), _I(dtype_code(w)), _L(_rows("w", w)), _ptr(bias), _I(M), _I(N), _I(K),
           _I(ADD_TO_RESIDUAL if add_to_out else STORE), _I(int(exact)), _stream())
@@ -438,6 +446,10 @@ def gemm_swiglu(out: torch.Tensor, a: torch.Tensor, w_gate: torch.Tensor, w_up: 
         more = (_ptr(None), _F(0.0)) if entry != "alofa_gemm_mfma" else (_ptr(None), _F(0.0), _ptr(None), _L(0), _ptr(None))
         _call(entry, _ptr(out), _I(BF16), _L(_rows("out", out)), _ptr(a), _L(_rows("a", a)), _ptr(w_gate), _ptr(w_up),
               _L(_rows("w_gate", w_gate)), _ptr(None), _I(M), _I(N), _I(K), _I(GATED[act]), *more, _stream())
+        return
+    if exact and a.dtype is torch.float32 and w_gate.dtype is torch.float32 and out.dtype is torch.float32:
+        _call("alofa_gemm_swiglu_exact", _ptr(out), _L(_rows("out", out)), _ptr(a), _L(_rows("a", a)), _ptr(w_gate), _ptr(w_up), _L(_rows("w_gate", w_gate)),
+              _I(M), _I(N), _I(K), _I(int(act == "gelu_tanh")), _stream())
         return
     _call("alofa_gemm_swiglu_simple", _ptr(out), _I(dtype_code(out)), _L(_rows("out", out)), _ptr(a), _I(dtype_code(a)), _L(_rows("a", a)),
           _ptr(w_gate), _ptr(w_up), _I(dtype_code(w_gate)), _L(_rows("w_gate", w_gate)), _I(M), _I(N), _I(K), _I(int(act == "gelu_tanh")), _I(int(exact)), _stream())
@@ -654,6 +666,10 @@ def paged_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v
             and _rows("q", q) % 8 == 0 and q.data_ptr() % 16 == 0 and bs >= MIN_FAST_PAGE and bs & (bs - 1) == 0):
         attention_decode(out, q, k_cache, v_cache, block_table, req_of_token, positions, heads, kv_heads, d, window, scale,
                          max_context or 1 << 30, scratch)
+        return
+    if exact and q.dtype is torch.float32 and load().alofa_attention_exact_takes(_ptr(q), _L(_rows("q", q)), _ptr(k_cache), _ptr(v_cache), _I(d), _I(bs)):
+        _call("alofa_attention_exact", _ptr(out), _L(_rows("out", out)), _ptr(q), _L(_rows("q", q)), _ptr(k_cache), _ptr(v_cache), _ptr(block_table),
+              _I(block_table.shape[1]), _ptr(req_of_token), _ptr(positions), _I(T), _I(heads), _I(kv_heads), _I(d), _I(bs), _I(int(window or 0)), _F(scale), _stream())
         return
     _call("alofa_attention_simple", _ptr(out), _L(_rows("out", out)), _ptr(q), _L(_rows("q", q)), _ptr(k_cache), _ptr(v_cache),
           _I(dtype_code(q)), _ptr(block_table), _I(block_table.shape[1]), _ptr(req_of_token), _ptr(positions), _I(T),

@@ -1,0 +1,83 @@
+"""The 32-bit path's kernels with float64 sums on the matrix cores, at the edges of their tiles, against float64 on the host."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+ONCE = 2.0 ** -23      # an output is rounded to float once (half a unit in the last place), a sum with the residual stream twice
+
+
+def ops():
+    from alofa_amd import ops as o
+    return o
+
+
+def t(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+def within(got, want, parts):
+    """|got - want| <= parts roundings of the terms' size."""
+    got, want = got.cpu().double().numpy(), np.asarray(want, dtype=np.float64)
+    assert np.all(np.isfinite(got)) and np.all(np.abs(got - want) <= ONCE * parts), np.abs((got - want) / parts).max()
+
+
+# rows up to 16, 32 and beyond (three kernels' forms), tiles' edges, K short, ragged and shared out, unaligned rows
+@pytest.mark.parametrize("M,N,K,shift", [(1, 16, 32, 0), (8, 896, 4864, 0), (16, 17, 31, 0), (16, 5000, 36, 0), (5, 70000, 64, 0), (17, 33, 260, 0), (32, 129, 1000, 0),
+                                         (33, 64, 128, 0), (64, 896, 4864, 0), (65, 130, 2056, 0), (200, 97, 1030, 0), (8, 130, 200, 1), (40, 70, 512, 1), (450, 1152, 896, 0)])
+def test_exact_products(M, N, K, shift):
+    rng = np.random.default_rng(M * 1000 + N)
+    a, w, w2, b, res = (rng.standard_normal(s).astype(np.float32) for s in ((M, K + shift), (N, K + shift), (N, K + shift), (N,), (M, N)))
+    ta, tw, tw2 = t(a)[:, shift:], t(w)[:, shift:], t(w2)[:, shift:]
+    want = a[:, shift:].astype(np.float64) @ w[:, shift:].astype(np.float64).T
+    up = a[:, shift:].astype(np.float64) @ w2[:, shift:].astype(np.float64).T
+    out = torch.full((M, N + 3), 7.0, device=DEV)
+    ops().gemm(out[:, :N], ta, tw, t(b), exact=True)
+    within(out[:, :N], want + b, np.abs(want + b) + 1e-7)
+    assert bool((out[:, N:] == 7.0).all())
+    acc = t(res)
+    ops().gemm(acc, ta, tw, add_to_out=True, exact=True)
+    within(acc, want + res, np.abs(want) + np.abs(want + res) + 1e-7)
+    ops().gemm_swiglu(out[:, :N], ta, tw, tw2, exact=True)
+    gate = want / (1.0 + np.exp(-want))
+    within(out[:, :N], gate * up, 4 * np.abs(gate * up) * (1 + np.abs(want)) + 1e-7)      # (gate and up are rounded before the activation, whose slope is its size at most)
+    again = torch.empty(M, N, device=DEV)
+    ops().gemm(again, ta, tw, t(b), exact=True)
+    ops().gemm(out[:, :N], ta, tw, t(b), exact=True)
+    assert torch.equal(again, out[:, :N])      # a fixed order, whatever the timing
+
+
+@pytest.mark.parametrize("heads,kv_heads,d,bs,requests", [(14, 2, 64, 16, 3), (20, 1, 32, 4, 2), (33, 1, 16, 12, 2), (4, 4, 112, 16, 2), (2, 1, 160, 8, 2), (8, 2, 128, 64, 70)])
+@pytest.mark.parametrize("window", [None, 19])
+def test_exact_attention(heads, kv_heads, d, bs, requests, window):
+    rng = np.random.default_rng(heads + d)
+    lens = [1 + (i * 37) % 90 + (100 if i == 0 else 0) for i in range(requests)]      # from one key on, past a page's and a tile's end
+    brings = [n if i == 1 else min(n, 1 + i % 2) for i, n in enumerate(lens)]      # a whole prompt and single tokens
+    per = [(n + bs - 1) // bs for n in lens]
+    order = rng.permutation(sum(per) + 1)
+    kc = torch.full((sum(per) + 1, kv_heads, bs, d), float("nan"), dtype=torch.float32)      # (what no token has written is never read into a result)
+    vc = torch.full((sum(per) + 1, kv_heads, d, bs), float("nan"), dtype=torch.float32)
+    table = torch.full((requests, max(per)), -1, dtype=torch.int32)
+    rows, req, pos, want, used = [], [], [], [], 0
+    for i, (n, m) in enumerate(zip(lens, brings)):
+        pages = order[used:used + per[i]]
+        used += per[i]
+        lowest = 0 if window is None else max(0, n - m - window + 1)
+        k, v, q = (torch.from_numpy(rng.standard_normal(s).astype(np.float32)) for s in ((n, kv_heads, d), (n, kv_heads, d), (m, heads, d)))
+        for j in range(n):
+            kc[pages[j // bs], :, j % bs], vc[pages[j // bs], :, :, j % bs] = k[j], v[j]
+        for j, page in enumerate(pages):
+            table[i, j] = -1 if (j + 1) * bs <= lowest else int(page)      # (pages that a window has passed are given back)
+        rows.append(q.reshape(m, heads * d)), req.extend([i] * m), pos.extend(range(n - m, n))
+        for j in range(m):
+            p = n - m + j
+            lo = 0 if window is None else max(0, p - window + 1)
+            kk, vv = (x[lo:p + 1].double().repeat_interleave(heads // kv_heads, 1) for x in (k, v))
+            s = torch.einsum("hd,khd->hk", q[j].double(), kk) * float(np.float32(d ** -0.5))
+            want.append(torch.einsum("hk,khd->hd", torch.softmax(s, -1), vv).reshape(-1))
+    out = torch.empty(len(req), heads * d, device=DEV)
+    to = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)      # noqa: E731
+    ops().paged_attention(out, torch.cat(rows).to(DEV), kc.to(DEV), vc.to(DEV), table.to(DEV), to(req), to(pos), heads, kv_heads, d, window, float(np.float32(d ** -0.5)), True)
+    # a weight: its score's rounding (some units of 2^-23 at scores of up to six), expf's two units; the values are of order one
+    within(out, torch.stack(want).numpy(), 12.0)
