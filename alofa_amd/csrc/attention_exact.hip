@@ -14,7 +14,7 @@
 //
 // Bound by the chain table -> keys -> scores -> weights -> values of few tiles in decode steps and by the matrix cores in prompts
 // (half of the columns idle with seven heads to a key head). us before (a wave a (token, head), one key a lane, every score twice)
-// and now, 14/2 heads of 64: 8 tokens at 130 to 260 keys 85 and 10; prompts of 64, 128 and 256 tokens 145 and 24.
+// and now, 14/2 heads of 64: 8 tokens at 130 to 260 keys 85 and 12; prompts of 64, 128 and 256 tokens 145 and 22.
 // Cache layout: keys [block, kv_head, slot_in_block, d], values transposed [block, kv_head, d, slot_in_block].
 #include "common.h"
 
@@ -31,7 +31,7 @@ __global__ void __launch_bounds__(64 * NW) attention_exact_kernel(
     const float* __restrict__ v_cache, const int32_t* __restrict__ block_table, int max_blocks, const int32_t* __restrict__ req_of_token,
     const int32_t* __restrict__ positions, int heads, int kv_heads, int block_size, int window, float scale) {
   constexpr int d = NT * 16;
-  __shared__ double sums[16][d + 1];      // per head: the channels' sums, then the weights'
+  __shared__ double sums[NW][16][d + 1];      // per wave and head: the channels' sums, then the weights'
   __shared__ float maxima[NW][16];
   const int group = heads / kv_heads, chunks = (group + 15) / 16;
   const int t = blockIdx.x, hk = blockIdx.y / chunks, h0 = (blockIdx.y % chunks) * 16;
@@ -108,24 +108,23 @@ __global__ void __launch_bounds__(64 * NW) attention_exact_kernel(
   l += __shfl_xor(l, 16);
   l += __shfl_xor(l, 32);
   if (g == 0) maxima[wave][r] = m;
-  for (int i = threadIdx.x; i < 16 * (d + 1); i += 64 * NW) sums[i / (d + 1)][i % (d + 1)] = 0.0;
   __syncthreads();
   float most = maxima[0][r];
 #pragma unroll
   for (int w = 1; w < NW; ++w) most = fmaxf(most, maxima[w][r]);
   const double f = exp(static_cast<double>(m) - static_cast<double>(most));      // (0 for a wave that saw no key)
-  for (int w = 0; w < NW; ++w) {
-    if (wave == w) {
 #pragma unroll
-      for (int i = 0; i < NT; ++i)
+  for (int i = 0; i < NT; ++i)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) sums[r][i * 16 + 4 * v + g] += o[i][v] * f;
-      if (g == 0) sums[r][d] += l * f;
-    }
-    __syncthreads();
+    for (int v = 0; v < 4; ++v) sums[wave][r][i * 16 + 4 * v + g] = o[i][v] * f;
+  if (g == 0) sums[wave][r][d] = l * f;
+  __syncthreads();
+  for (int i = threadIdx.x; i < served * d; i += 64 * NW) {
+    double value = 0, weight = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) value += sums[w][i / d][i % d], weight += sums[w][i / d][d];
+    out[static_cast<int64_t>(t) * out_stride + static_cast<int64_t>(hk * group + h0 + i / d) * d + i % d] = static_cast<float>(value / weight);
   }
-  for (int i = threadIdx.x; i < served * d; i += 64 * NW)
-    out[static_cast<int64_t>(t) * out_stride + static_cast<int64_t>(hk * group + h0 + i / d) * d + i % d] = static_cast<float>(sums[i / d][i % d] / sums[i / d][d]);
 }
 
 template <int NT>

@@ -9,15 +9,17 @@
 // only: two orders differ by some 2^-50 of the sum, which the one rounding to float hides but for one output in some ten million.
 //
 //   up to 16 rows (exact_rows_kernel): a block owns 16 weight rows (16 of gate and 16 of up), its waves take runs of 32 k in turn,
-//   straight from memory, and meet in LDS. Bound by reading the weights once: a wave's matrix instructions take 64 cycles for 64
-//   weights, half of what the memory brings. 8 rows, us before (a tile of 64 x 64 on the vector units, one block per 64 columns) and
-//   now: see the numbers at launch_exact.
+//   straight from memory, and meet in LDS. Bound by the rate at which a compute unit takes its weights in and, within it, by the matrix
+//   cores (64 cycles an instruction, 64 weights), so K is shared out over blocks where blocks are few. 8 rows, us, a tile of 64 x 64
+//   on the vector units (one block per 64 columns) / this: 9,728 x 896 with the gate 270 / 14.6, 896 x 4,864 920 / 7.8 and 4.5 for the second
+//   launch, 896 x 896 168 / 6.8, 1,152 x 896 170 / 7.3, 151,936 x 896 658 / 113.
 //
 //   more rows (exact_tile_kernel): slabs of 32 k through LDS, a wave owns 32 rows x 32 weight rows (four instructions for two
 //   loads of either operand), a block 64 x 64 (32 x 128 up to 32 rows). Bound by the matrix cores (69 TFLOP/s measured with
-//   nothing else in the loop): the slab's traffic hides behind 2,048 cycles of instructions. K is shared out over blocks
-//   where the tiles are fewer than twice the compute units; the shares' float64 sums go to a buffer of the caller's (not to the library's
-//   workspace, which one stream at a time may use) and a second launch adds them.
+//   nothing else in the loop; 46 of useful work at 450 rows, whose last tile is padding): the slab's traffic hides behind 2,048 cycles of
+//   instructions. K is shared out over blocks where the tiles are few; the shares' float64 sums go to a buffer of the caller's (not to the
+//   library's workspace, which one stream at a time may use) and a second launch adds them. 450 rows, us, as above: 9,728 x 896 with the gate
+//   377 / 169, 896 x 4,864 1,000 / 101 + 5, 896 x 896 185 / 25, 1,152 x 896 185 / 30 + 5.
 #include "common.h"
 
 namespace alofa {
@@ -27,14 +29,17 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 constexpr int kExactStore = 0, kExactResidual = 1;
 constexpr int kExactRows = 16;       // rows that exact_rows_kernel takes at most
 
-// four consecutive k of a row from `k` on: one 16-byte load, or, where rows are not 16-byte aligned, value by value; zeros beyond K
+// four consecutive k of a row from `k` on, all of them within the row: one 16-byte load, or, where rows are not 16-byte aligned, value by value
 template <bool kVec>
-__device__ __forceinline__ float4 quad(const float* row, int k, int K) {
-  if constexpr (kVec) {
-    return k < K ? *reinterpret_cast<const float4*>(row + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-  } else {
-    return make_float4(k < K ? row[k] : 0.f, k + 1 < K ? row[k + 1] : 0.f, k + 2 < K ? row[k + 2] : 0.f, k + 3 < K ? row[k + 3] : 0.f);
-  }
+__device__ __forceinline__ float4 quad(const float* row, int k) {
+  if constexpr (kVec) return *reinterpret_cast<const float4*>(row + k);
+  else return make_float4(row[k], row[k + 1], row[k + 2], row[k + 3]);
+}
+// the same with zeros beyond K
+template <bool kVec>
+__device__ __forceinline__ float4 quad_within(const float* row, int k, int K) {
+  if constexpr (kVec) return k < K ? quad<kVec>(row, k) : make_float4(0.f, 0.f, 0.f, 0.f);
+  else return make_float4(k < K ? row[k] : 0.f, k + 1 < K ? row[k + 1] : 0.f, k + 2 < K ? row[k + 2] : 0.f, k + 3 < K ? row[k + 3] : 0.f);
 }
 
 __device__ __forceinline__ f64x4 fma_quad(float4 a, float4 b, f64x4 acc) {
@@ -59,42 +64,66 @@ __device__ __forceinline__ float gated(double g, double u, int gelu) {
 template <int NW, int NT, int kMats, int kEpilogue, bool kVec>
 __global__ void __launch_bounds__(64 * NW) exact_rows_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ A, int64_t lda,
                                                              const float* __restrict__ W, const float* __restrict__ W2, int64_t ldw,
-                                                             const float* __restrict__ bias, int M, int N, int K, int gelu) {
+                                                             const float* __restrict__ bias, double* __restrict__ parts, int k_share, int M, int N, int K, int gelu) {
   constexpr int kTiles = NT * kMats;
   __shared__ double sums[NW][kTiles][4][64];
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
   const int n0 = blockIdx.x * 16 * NT;
+  const int k_first = blockIdx.y * k_share;      // (shares of K: blockIdx.y, their sums in `parts` as [share][M][N])
+  K = K - k_first < k_share ? K - k_first : k_share;
   const bool row_ok = r < M;
-  const float* a_row = A + static_cast<int64_t>(row_ok ? r : 0) * lda;
+  const float* a_row = A + static_cast<int64_t>(row_ok ? r : 0) * lda + k_first;
   const float* w_row[kTiles];
 #pragma unroll
   for (int t = 0; t < kTiles; ++t) {
     const int n = n0 + (t / kMats) * 16 + r;
-    w_row[t] = (t % kMats ? W2 : W) + static_cast<int64_t>(n < N ? n : N - 1) * ldw;      // (rows beyond N: the last one again, not stored)
+    w_row[t] = (t % kMats ? W2 : W) + static_cast<int64_t>(n < N ? n : N - 1) * ldw + k_first;      // (rows beyond N: the last one again, not stored)
   }
   f64x4 acc[kTiles];
 #pragma unroll
   for (int t = 0; t < kTiles; ++t) acc[t] = f64x4{0, 0, 0, 0};
-  // runs of 32 k: a lane takes 8 g .. 8 g + 7 of each; the next run is on its way while one is multiplied
-  float4 a0, a1, w0[kTiles], w1[kTiles];
-  auto fetch = [&](int k) __attribute__((always_inline)) {
-    a0 = quad<kVec>(a_row, k, K), a1 = quad<kVec>(a_row, k + 4, K);
+  // Runs of 32 k: a lane takes 4 g .. 4 g + 3 of either half (an instruction's lanes fetch 64 bytes of a row side by side). kSets runs are on their
+  // way or in work; each set of registers is filled again as soon as its run is multiplied, without a branch around the loads (a run past
+  // the last is the last one again), so that the compiler waits for the oldest only.
+  constexpr int kSets = kTiles == 1 ? 4 : kTiles == 2 ? 3 : 2;
+  const int runs = K / 32, mine = (runs - wave + NW - 1) / NW;      // whole runs, and those of this wave: wave, wave + NW, ...
+  float4 a[kSets][2], w[kSets][kTiles][2];
+  auto fetch = [&](int s, int i) __attribute__((always_inline)) {
+    const int k = (wave + (i < mine ? i : mine - 1) * NW) * 32 + g * 4;
 #pragma unroll
-    for (int t = 0; t < kTiles; ++t) w0[t] = quad<kVec>(w_row[t], k, K), w1[t] = quad<kVec>(w_row[t], k + 4, K);
+    for (int h = 0; h < 2; ++h) {
+      a[s][h] = quad<kVec>(a_row, k + 16 * h);
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t) w[s][t][h] = quad<kVec>(w_row[t], k + 16 * h);
+    }
   };
-  int k = wave * 32 + g * 8;
-  if (wave * 32 < K) fetch(k);
-  for (int k0 = wave * 32; k0 < K; k0 += NW * 32) {
-    float4 ca0 = a0, ca1 = a1, cw0[kTiles], cw1[kTiles];
+  auto multiply = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
-    for (int t = 0; t < kTiles; ++t) cw0[t] = w0[t], cw1[t] = w1[t];
-    k += NW * 32;
-    if (k0 + NW * 32 < K) fetch(k);
-    if (!row_ok) ca0 = ca1 = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int h = 0; h < 2; ++h) {
+      if (!row_ok) a[s][h] = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-      acc[t] = fma_quad(cw0[t], ca0, acc[t]);
-      acc[t] = fma_quad(cw1[t], ca1, acc[t]);
+      for (int t = 0; t < kTiles; ++t) acc[t] = fma_quad(w[s][t][h], a[s][h], acc[t]);
+    }
+  };
+  if (mine > 0) {
+#pragma unroll
+    for (int s = 0; s < kSets; ++s) fetch(s, s);
+    int i = 0;
+    for (; i + kSets <= mine; i += kSets)
+#pragma unroll
+      for (int s = 0; s < kSets; ++s) {
+        multiply(s);
+        fetch(s, i + kSets + s);
+      }
+#pragma unroll
+    for (int s = 0; s < kSets - 1; ++s)
+      if (i + s < mine) multiply(s);
+  }
+  if (runs % NW == wave) {      // what is left of K beyond the whole runs
+    for (int k = runs * 32; k < K; k += 16) {
+      const float4 left = row_ok ? quad_within<kVec>(a_row, k + g * 4, K) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t) acc[t] = fma_quad(quad_within<kVec>(w_row[t], k + g * 4, K), left, acc[t]);
     }
   }
 #pragma unroll
@@ -109,12 +138,13 @@ __global__ void __launch_bounds__(64 * NW) exact_rows_kernel(float* __restrict__
     double s[kMats];
 #pragma unroll
     for (int x = 0; x < kMats; ++x) {
-      s[x] = bias ? static_cast<double>(bias[n]) : 0.0;
+      s[x] = bias && !parts ? static_cast<double>(bias[n]) : 0.0;
 #pragma unroll
       for (int w = 0; w < NW; ++w) s[x] += sums[w][tile * kMats + x][v][at];
     }
     float* dst = out + static_cast<int64_t>(m) * ldo + n;
     if constexpr (kMats == 2) *dst = gated(s[0], s[1], gelu);
+    else if (parts) parts[(static_cast<int64_t>(blockIdx.y) * M + m) * N + n] = s[0];
     else put<kEpilogue>(dst, s[0]);
   }
 }
@@ -127,7 +157,7 @@ __global__ void __launch_bounds__(256) exact_tile_kernel(float* __restrict__ out
                                                          const float* __restrict__ bias, double* __restrict__ parts, int M, int N, int K, int k_share, int gelu) {
   constexpr int WN = 4 / WM, BM = 32 * WM, BW = 32 * WN, BK = 32, kPad = 4;
   constexpr int kOwn = 32 / kMats;                     // outputs of a wave along N
-  __shared__ __attribute__((aligned(16))) float As[BM][BK + kPad], Ws[BW][BK + kPad];
+  __shared__ __attribute__((aligned(16))) float As[BM][BK + kPad], Ws[BW][BK + kPad];      // (as doubles, widened once as they are brought: 174 us where this takes 169)
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
   const int wm = wave / WN, wn = wave % WN;
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * WN * kOwn;
@@ -138,12 +168,12 @@ __global__ void __launch_bounds__(256) exact_tile_kernel(float* __restrict__ out
 #pragma unroll
     for (int i = 0; i < kA; ++i) {
       const int at = threadIdx.x + i * 256, row = at / 8, m = m0 + row;
-      fa[i] = quad<kVec>(A + static_cast<int64_t>(m < M ? m : M - 1) * lda, k0 + at % 8 * 4, k_end);
+      fa[i] = quad_within<kVec>(A + static_cast<int64_t>(m < M ? m : M - 1) * lda, k0 + at % 8 * 4, k_end);
     }
 #pragma unroll
     for (int i = 0; i < kW; ++i) {
       const int at = threadIdx.x + i * 256, row = at / 8, n = n0 + row / 32 * kOwn + row % kOwn;
-      fw[i] = quad<kVec>((kMats == 2 && row % 32 >= 16 ? W2 : W) + static_cast<int64_t>(n < N ? n : N - 1) * ldw, k0 + at % 8 * 4, k_end);
+      fw[i] = quad_within<kVec>((kMats == 2 && row % 32 >= 16 ? W2 : W) + static_cast<int64_t>(n < N ? n : N - 1) * ldw, k0 + at % 8 * 4, k_end);
     }
   };
   f64x4 acc[2][2];      // [rows of A][weight rows]
@@ -212,32 +242,52 @@ __global__ void __launch_bounds__(256) exact_sum_kernel(float* __restrict__ out,
   put<kEpilogue>(out + i / N * ldo + n, s);
 }
 
-// Up to 16 rows: blocks of eight waves (four in the gated form, whose blocks are many), sixteen where the blocks of 16 weight rows are fewer than
-// half the compute units; four tiles of weight rows a block against a matrix as long as a vocabulary, so that the rows of A are read a quarter as often.
-template <int kMats, int kEpilogue, bool kVec>
-static int launch_exact_rows(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, const float* W2, int64_t ldw, const float* bias,
-                             int M, int N, int K, int gelu, hipStream_t stream) {
-  const int tiles = (N + 15) / 16, cus = compute_units();
-  if (kMats == 1 && tiles >= 16 * cus)
-    exact_rows_kernel<4, 4, 1, kEpilogue, kVec><<<(tiles + 3) / 4, 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, gelu);
-  else if (kMats == 1 && tiles * 2 < cus && K >= 2048)
-    exact_rows_kernel<16, 1, kMats, kEpilogue, kVec><<<tiles, 1024, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, gelu);
-  else if (kMats == 1 || tiles < cus)
-    exact_rows_kernel<8, 1, kMats, kEpilogue, kVec><<<tiles, 512, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, gelu);
-  else
-    exact_rows_kernel<4, 1, kMats, kEpilogue, kVec><<<tiles, 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, gelu);
-  return check_launch("gemm_exact_rows");
+// How K is shared out over blocks: the number of shares (at most 16, at least 128 k each) with the least time of the compute unit that has the most
+// blocks: 27 ns a k of a block (64 cycles of its SIMDs' matrix cores) and some 1.5 us a block, a third more with one block to a compute unit (nothing
+// fills its waits), and for the second launch 4 us and 16 bytes a sum at 4 TB/s. Returns k a share (a multiple of a slab). Up to 16 rows and in the
+// gated form K is not shared out. Up to 16 rows: shares of 1,024 k and more for one block to a compute unit, where the
+// blocks of 16 weight rows are fewer than half the compute units and K is long (896 x 4,864, 8 rows: 19.0 us in 56 blocks of 16 waves).
+static int exact_share(int M, int N, int K) {
+  if (M <= kExactRows) {
+    const int blocks = (N + 15) / 16, cus = compute_units();
+    if (blocks * 2 >= cus || K < 2048) return K;
+    const int shares = cus / blocks < K / 1024 ? cus / blocks : K / 1024;
+    return ((K + shares - 1) / shares + 31) / 32 * 32;
+  }
+  const int BM = M <= 32 ? 32 : 64, BW = M <= 32 ? 128 : 64, cus = compute_units();
+  const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BW - 1) / BW);
+  int best = K;
+  double least = 1e30;
+  for (int shares = 1; shares <= 16 && (shares == 1 || K / shares >= 128); ++shares) {
+    const int k = ((K + shares - 1) / shares + 31) / 32 * 32, got = (K + k - 1) / k;
+    const int64_t rounds = (tiles * got + cus - 1) / cus;
+    const double us = rounds * (0.027 * k + 1.5) * (rounds == 1 ? 1.33 : 1.0) + (got > 1 ? 4.0 + 4e-6 * got * M * N : 0.0);
+    if (us < least) least = us, best = got > 1 ? k : K;
+  }
+  return best;
 }
 
-// How K is shared out over blocks: blocks for two rounds of the compute units, at least 128 k a share, at most 16 shares. Returns k a share (a multiple
-// of a slab). Up to 16 rows and in the gated form K is not shared out.
-static int exact_share(int M, int N, int K) {
-  const int BM = M <= 32 ? 32 : 64, BW = M <= 32 ? 128 : 64;
-  const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BW - 1) / BW);
-  int64_t shares = (2 * compute_units() + tiles - 1) / tiles;
-  shares = shares < K / 128 ? shares : K / 128;
-  shares = M <= kExactRows || shares < 1 ? 1 : shares > 16 ? 16 : shares;
-  return static_cast<int>(((K + shares - 1) / shares + 31) / 32 * 32);
+template <int kEpilogue>
+static void launch_exact_sum(float* out, int64_t ldo, const double* parts, const float* bias, int M, int N, int shares, hipStream_t stream) {
+  const int64_t all = static_cast<int64_t>(M) * N;
+  exact_sum_kernel<kEpilogue><<<static_cast<unsigned>((all + 255) / 256), 256, 0, stream>>>(out, ldo, parts, bias, M, N, shares);
+}
+
+// Up to 16 rows: blocks of eight waves (four in the gated form, whose blocks are many); four tiles of weight rows a block against a matrix as long as a
+// vocabulary, so that the rows of A are read a quarter as often.
+template <int kMats, int kEpilogue, bool kVec>
+static int launch_exact_rows(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, const float* W2, int64_t ldw, const float* bias,
+                             double* parts, int M, int N, int K, int gelu, hipStream_t stream) {
+  const int tiles = (N + 15) / 16, cus = compute_units();
+  const int k_share = kMats == 1 ? exact_share(M, N, K) : K, shares = (K + k_share - 1) / k_share;
+  if (kMats == 1 && tiles >= 16 * cus)
+    exact_rows_kernel<4, 4, 1, kEpilogue, kVec><<<(tiles + 3) / 4, 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, nullptr, K, M, N, K, gelu);
+  else if (kMats == 1 || tiles < cus)
+    exact_rows_kernel<8, 1, kMats, kEpilogue, kVec><<<dim3(tiles, shares), 512, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, shares > 1 ? parts : nullptr, k_share, M, N, K, gelu);
+  else
+    exact_rows_kernel<4, 1, kMats, kEpilogue, kVec><<<tiles, 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, nullptr, K, M, N, K, gelu);
+  if (shares > 1) launch_exact_sum<kEpilogue>(out, ldo, parts, bias, M, N, shares, stream);
+  return check_launch("gemm_exact_rows");
 }
 
 template <int WM, int kMats, int kEpilogue, bool kVec>
@@ -247,10 +297,7 @@ static int launch_exact_tile(float* out, int64_t ldo, const float* A, int64_t ld
   const int k_share = kMats == 1 ? exact_share(M, N, K) : K, shares = (K + k_share - 1) / k_share;
   dim3 grid((N + kOut - 1) / kOut, (M + BM - 1) / BM, shares);
   exact_tile_kernel<WM, kMats, kEpilogue, kVec><<<grid, 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, shares > 1 ? parts : nullptr, M, N, K, k_share, gelu);
-  if (shares > 1) {
-    const int64_t all = static_cast<int64_t>(M) * N;
-    exact_sum_kernel<kEpilogue><<<static_cast<unsigned>((all + 255) / 256), 256, 0, stream>>>(out, ldo, parts, bias, M, N, shares);
-  }
+  if (shares > 1) launch_exact_sum<kEpilogue>(out, ldo, parts, bias, M, N, shares, stream);
   return check_launch("gemm_exact_tile");
 }
 
@@ -260,8 +307,8 @@ static int launch_exact(float* out, int64_t ldo, const float* A, int64_t lda, co
   auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && aligned(A) && aligned(W) && aligned(W2);
   if (M <= kExactRows)
-    return vec ? launch_exact_rows<kMats, kEpilogue, true>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, gelu, stream)
-               : launch_exact_rows<kMats, kEpilogue, false>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, gelu, stream);
+    return vec ? launch_exact_rows<kMats, kEpilogue, true>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, stream)
+               : launch_exact_rows<kMats, kEpilogue, false>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, stream);
   if (M <= 32)
     return vec ? launch_exact_tile<1, kMats, kEpilogue, true>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, stream)
                : launch_exact_tile<1, kMats, kEpilogue, false>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, stream);
