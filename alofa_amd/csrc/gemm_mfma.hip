@@ -24,43 +24,12 @@
 // Epilogues: store (+ bias), add to the float residual stream, and SwiGLU, for
 // which a block computes the gate and the up product of the same columns (its
 // W slab holds as many rows of each) and writes silu(gate) * up (or the tanh form of gelu in silu's place).
-#include "common.h"
-
-#include <cstdlib>
+#include "gemm_tiles.h"
 
 namespace alofa {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-enum MfmaEpilogue : int { kMfStore = 0, kMfResidual = 1, kMfSwiglu = 2, kMfArgmax = 3, kMfGeglu = 4 };
-
 constexpr int TK = 64, PAD = 8;
 constexpr int kRow = TK + PAD;  // LDS row length in elements
-
-// Which tile a block computes. The chip is eight dies, each with an L2 of its own, and blocks go to the
-// dies in turn (block i to die i % 8). Dealt out row by row, every die computes tiles from all over the
-// output and pulls all of A and all of W through its L2: fine while both fit there, and measured a few
-// percent faster then than the path below; with operands beyond the L2s (projections of 7B-sized models
-// and up) it costs up to a fifth of the time. For those (by_die) the tiles are numbered along a path that
-// stays within squares of 8 x 8 tiles (8 tile rows at a time, column by column), every die takes one
-// contiguous stretch of the path, and the blocks resident on a die together share a handful of A and W
-// panels. With K shared out, the shares are the slowest index (blocks of different shares have nothing
-// in common).
-struct TilePlace {
-  int bm, bn, share;
-};
-__device__ __forceinline__ TilePlace place_tile(int block, int tiles_m, int tiles_n, int shares, bool by_die) {
-  constexpr int kDies = 8, kGroup = 8;
-  const int tiles = tiles_m * tiles_n, total = tiles * shares;
-  if (!by_die) return {block % tiles / tiles_n, block % tiles_n, block / tiles};
-  const int die = block % kDies, local = block / kDies;
-  const int step = die * (total / kDies) + min(die, total % kDies) + local;   // dies before this one hold that many blocks
-  const int t = step % tiles;
-  const int per_group = kGroup * tiles_n, first_m = (t / per_group) * kGroup, within = t % per_group;
-  const int rows = min(tiles_m - first_m, kGroup);
-  return {first_m + within % rows, within / rows, step / tiles};
-}
 
 // Instead of the outputs, a wave leaves per row the highest of its columns and that column's number (the lowest
 // among equals): candidate 2 bn + wn of `parts` per row, values at out[m * parts + ..], column numbers as int32
@@ -93,48 +62,6 @@ __device__ __forceinline__ void tile_argmax(f32x16 (&acc)[WTM][WTN], float* __re
       if (col == 0 && m < M) {
         out[static_cast<int64_t>(m) * parts + 2 * bn + wn] = bv;
         numbers[static_cast<int64_t>(m) * parts + 2 * bn + wn] = bi;
-      }
-    }
-  }
-}
-
-// What a wave does with its finished tiles (WTM x WTN of 32 x 32, the block's tile at m0, n0 of the output).
-template <int kEpilogue, typename TO, int WTM, int WTN>
-__device__ __forceinline__ void tile_epilogue(f32x16 (&acc)[WTM][WTN], TO* __restrict__ out, int64_t ldo,
-                                              const float* __restrict__ bias, int M, int N, int m0, int n0, int wm, int wn, int lane) {
-  constexpr int kGateTiles = WTN / 2;
-  const int col = lane % 32, row_base = (lane / 32) * 4;
-  constexpr int kOutTiles = is_gated(kEpilogue) ? kGateTiles : WTN;
-#pragma unroll
-  for (int i = 0; i < WTM; ++i) {
-#pragma unroll
-    for (int j = 0; j < kOutTiles; ++j) {
-      const int n = n0 + wn * 32 * kOutTiles + j * 32 + col;
-      if (n >= N) continue;
-      const float b = (bias && kEpilogue == kMfStore) ? bias[n] : 0.f;
-      const int m_first = m0 + wm * 32 * WTM + i * 32 + row_base;      // element e: row m_first + 8 * (e / 4) + e % 4
-      TO* column = out + n;
-      float old[16];
-      if (kEpilogue == kMfResidual) {      // all sixteen old values set out before any is needed
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int m = m_first + 8 * (e / 4) + e % 4;
-          old[e] = m < M ? load_f32(column + static_cast<int64_t>(m) * ldo) : 0.f;
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int m = m_first + 8 * (e / 4) + e % 4;
-        if (m >= M) continue;
-        TO* dst = column + static_cast<int64_t>(m) * ldo;
-        if (kEpilogue == kMfStore) {
-          store_f32(dst, acc[i][j][e] + b);
-        } else if (kEpilogue == kMfResidual) {
-          store_f32(dst, old[e] + acc[i][j][e]);
-        } else {
-          const float g = acc[i][j][e];
-          store_f32(dst, gate_of<kEpilogue == kMfGeglu>(g) * acc[i][(j + kGateTiles) % WTN][e]);
-        }
       }
     }
   }
@@ -356,7 +283,6 @@ __global__ void __launch_bounds__(256) gemm_mfma_kernel(TO* __restrict__ out, in
 // of row r undoes by fetching chunk p ^ swz(r), so that the 16 or 32 rows whose fragments are read together
 // fall on distinct banks.
 // Rows beyond M or N are fetched from the last valid row (their results are never stored).
-__device__ __forceinline__ int swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
 // kSplitK = 2: a block leaves its share's sums as they are, tile by tile, in part `share` of `out` (float
 // [shares, M, ldo]); a second kernel (split_sum_kernel) adds the parts and runs the epilogue.
@@ -561,148 +487,6 @@ __global__ void __launch_bounds__(256) gemm_dma_kernel(TO* __restrict__ out, int
       }
   }
   tile_epilogue<kEpilogue, TO, WTM, WTN>(acc, out, ldo, bias, M, n_end, m0, n0, wm, wn, lane);
-}
-
-// The tiled product for many rows against a wide matrix: eight waves (WM x WN) on a tile of TM x TN outputs, slabs of 32
-// along K straight from memory into a ring of S in LDS. Against the four waves and slabs of 64 above: a wave's share of
-// a slab is small enough (a tile of 256 x 256 in 128 KB of ring) for two waves a SIMD, which fill one another's waits
-// at the barrier and for LDS, and a slab carries twice the products per byte fetched. The sums are the same numbers in
-// the same order as in the kernels above (one accumulator an output, ascending k). K a multiple of 32.
-// A slab is TM rows of A and TN rows of W, 64 bytes each; the four 16-byte chunks of a row are permuted by the row's
-// number (chunk c of row r lies at place c ^ ((r >> 2) & 3)), so that the sixteen rows whose fragments a quarter of a
-// wave reads together fall on distinct banks. kMfSwiglu: the slab's W rows are TN / 2 gate rows, then the up rows of the
-// same columns, and a wave holds gate and up of the same columns.
-__device__ __forceinline__ int swz32(int r) { return (r >> 2) & 3; }
-
-template <int kEpilogue, typename TO, int TM, int TN, int WM, int WN, int S>
-__global__ void __launch_bounds__(64 * WM * WN) gemm_wide_kernel(TO* __restrict__ out, int64_t ldo, const bf16_t* __restrict__ A, int64_t lda,
-                                                                 const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2, int64_t ldw,
-                                                                 const float* __restrict__ bias, int M, int N, int K, int tiles_m, int tiles_n) {
-  constexpr int kSlabK = 32, kRows = TM + TN, kStageBytes = kRows * 64, kWaves = WM * WN;
-  constexpr int kLoads = kRows / 16 / kWaves;        // fetch instructions per wave and slab (each brings sixteen rows)
-  constexpr int TI = TM / 32 / WM, TJ = TN / 32 / WN;   // 32 x 32 tiles a wave
-  static_assert(kRows % (16 * kWaves) == 0 && TM % (32 * WM) == 0 && TN % (32 * WN) == 0, "the tile must divide among the waves");
-  static_assert(!is_gated(kEpilogue) || TJ % 2 == 0, "the swiglu epilogue needs gate and up tiles in every wave");
-  constexpr int kGateTiles = TJ / 2;
-  __shared__ __attribute__((aligned(1024))) char ring[S * kStageBytes];
-  const TilePlace place = place_tile(blockIdx.x, tiles_m, tiles_n, 1, true);
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const int wm = wave / WN, wn = wave % WN;
-  constexpr int kOutCols = is_gated(kEpilogue) ? TN / 2 : TN;
-  const int m0 = place.bm * TM, n0 = place.bn * kOutCols;
-
-  // what this lane fetches: instruction j of this wave brings slab rows 16 (kWaves j + wave) .. + 15, lane l place l % 4 of row l / 4
-  const bf16_t* src[kLoads];
-#pragma unroll
-  for (int j = 0; j < kLoads; ++j) {
-    const int r = 16 * (kWaves * j + wave) + lane / 4, c = (lane % 4) ^ swz32(r);
-    if (r < TM) {
-      src[j] = A + static_cast<int64_t>(min(m0 + r, M - 1)) * lda + c * 8;
-    } else {
-      const int row = r - TM;
-      int n = n0 + row;
-      const bf16_t* base = W;
-      if (is_gated(kEpilogue) && row >= TN / 2) {
-        n = n0 + row - TN / 2;
-        base = W2;
-      }
-      src[j] = base + static_cast<int64_t>(min(n, N - 1)) * ldw + c * 8;
-    }
-  }
-  const unsigned ring_at = static_cast<unsigned>(reinterpret_cast<uintptr_t>(ring));
-  auto fetch = [&](int slab) {     // uniform over the block
-    const unsigned stage = ring_at + (slab % S) * kStageBytes + wave * 1024;
-#pragma unroll
-    for (int j = 0; j < kLoads; ++j) {
-      const bf16_t* from = src[j] + static_cast<int64_t>(slab) * kSlabK;
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                   :: "s"(__builtin_amdgcn_readfirstlane(stage + j * kWaves * 1024)), "v"(from), "r"(ring) : "memory", "m0");
-    }
-  };
-
-  f32x16 acc[TI][TJ];
-#pragma unroll
-  for (int i = 0; i < TI; ++i)
-#pragma unroll
-    for (int j = 0; j < TJ; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-  // fragments: lane l reads row l % 32 of its 32-row group, chunk 2 q + l / 32 in step q of the slab's two
-  const int sw = swz32(lane % 32), half = lane / 32;
-  const int a_row = (wm * 32 * TI + lane % 32) * 64;
-  const int w_row = (TM + lane % 32) * 64;
-  int place_of[2];
-#pragma unroll
-  for (int q = 0; q < 2; ++q) place_of[q] = ((2 * q + half) ^ sw) * 16;
-  auto w_group = [&](int j) {      // byte offset of this wave's j-th 32-row group within the slab's W rows
-    if (is_gated(kEpilogue)) return ((j < kGateTiles ? 0 : TN / 2) + (wn * kGateTiles + j % kGateTiles) * 32) * 64;
-    return (wn * TJ + j) * 32 * 64;
-  };
-  auto step = [&](int slab) {
-    const char* stage = ring + (slab % S) * kStageBytes;
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      bf16x8 a[TI], w[TJ];
-#pragma unroll
-      for (int i = 0; i < TI; ++i) a[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(stage + a_row + i * 32 * 64 + place_of[q]));
-#pragma unroll
-      for (int j = 0; j < TJ; ++j) w[j] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(stage + w_row + w_group(j) + place_of[q]));
-#pragma unroll
-      for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], w[j], acc[i][j], 0, 0, 0);
-    }
-  };
-
-  // Slab k + S - 1 takes the place of slab k - 1, which every wave has read before the barrier of step k; a wave waits
-  // for its own fetches of slab k (the S - 2 slabs behind it stay on their way) before that barrier.
-  const int slabs = K / kSlabK;
-  constexpr int kLead = S - 1;
-#pragma unroll
-  for (int p = 0; p < kLead; ++p)
-    if (p < slabs) fetch(p);
-  int k = 0;
-  for (; k + kLead < slabs; ++k) {
-    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kLoads * (kLead - 1)) : "memory");
-    __syncthreads();
-    fetch(k + kLead);
-    step(k);
-  }
-  for (; k < slabs; ++k) {      // nothing more to set out: the last slabs as they come
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    step(k);
-  }
-  tile_epilogue<kEpilogue, TO, TI, TJ>(acc, out, ldo, bias, M, N, m0, n0, wm, wn, lane);
-}
-
-template <int kEpilogue, typename TO, int TM, int TN, int WM, int WN, int S>
-static int launch_wide(void* out, int64_t ldo, const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, int M, int N, int K,
-                       hipStream_t stream, const void* W2 = nullptr) {
-  constexpr int kOutCols = is_gated(kEpilogue) ? TN / 2 : TN;
-  const int tiles_n = (N + kOutCols - 1) / kOutCols, tiles_m = (M + TM - 1) / TM;
-  gemm_wide_kernel<kEpilogue, TO, TM, TN, WM, WN, S><<<tiles_n * tiles_m, 64 * WM * WN, 0, stream>>>(
-      static_cast<TO*>(out), ldo, static_cast<const bf16_t*>(A), lda, static_cast<const bf16_t*>(W), static_cast<const bf16_t*>(W2), ldw, bias, M, N, K,
-      tiles_m, tiles_n);
-  return 0;
-}
-
-// Where the tiles of 256 x 256 with eight waves are the tiled product's choice: many rows against a long K, and so many
-// tiles that their rounds of one a compute unit are at least four fifths full. Measured against the forms below
-// (2,048 rows, us): gate/up + SwiGLU of the 7B sizes 524 against 586, of the 32B sizes 1,043 against 1,169 (4,096 rows:
-// 2,086 against 2,268; 256 rows, 216 tiles: 174 against 254); 7,168 x 5,120 150 against 183 (4,096 rows: 293 against
-// 350); 3,584 x 3,584 at 4,096 rows 116 against 142, 3,584 x 18,944 538 against 592. With rounds less full the forms
-// below stay ahead (7B gate/up at 512 rows, 296 tiles: 210 against 176; 5,120 x 27,648 at 4,096 rows, 320 tiles: 1,507
-// against 1,285), and so they do with a short K (0.5B gate/up at 2,048 rows 60.6 against 46.3).
-template <int kEpilogue>
-static bool wide_pays(int M, int N, int K) {
-  static const bool switched_off = [] { const char* e = getenv("ALOFA_WIDE_TILES"); return e != nullptr && e[0] == '0'; }();     // (for measurements)
-  if (switched_off || M <= 128 || K % 32 != 0 || K < 2048) return false;
-  constexpr int kOutCols = is_gated(kEpilogue) ? 128 : 256;
-  const int64_t tiles = static_cast<int64_t>((M + 255) / 256) * ((N + kOutCols - 1) / kOutCols), units = compute_units();
-  const int64_t rounds = (tiles + units - 1) / units;
-  return tiles * 5 >= rounds * units * 4;
 }
 
 template <int kEpilogue, typename TO, int WTM, int WTN, int PF, bool kSplitK>
@@ -928,10 +712,7 @@ template <int kEpilogue, typename TO>
 static int launch_mfma(void* out, int64_t ldo, const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw,
                        const float* bias, int M, int N, int K, hipStream_t stream, const ThenNorm& then, int* then_done) {
   if constexpr (kEpilogue != kMfArgmax) {
-    if (wide_pays<kEpilogue>(M, N, K)) {
-      if (launch_wide<kEpilogue, TO, 256, 256, 4, 2, 4>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2)) return 1;
-      return check_launch("gemm_wide");
-    }
+    if (tall_pays(M, N, K, is_gated(kEpilogue))) return launch_tall(kEpilogue, sizeof(TO) == 4 ? kF32 : kBF16, out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream);
   }
   if constexpr (is_gated(kEpilogue)) {
     // A block computes gate and up of the same 64 columns. With K a multiple of 64 and tiles that do not fill the
@@ -1005,24 +786,6 @@ static int launch_mfma(void* out, int64_t ldo, const void* A, int64_t lda, const
     // unit, were slower here even with four slabs ahead. Where even the small tiles are too few, K is
     // shared out among blocks as well.
     const int64_t big_blocks = static_cast<int64_t>((N + 127) / 128) * ((M + 127) / 128);
-    const int64_t tiles_192 = static_cast<int64_t>((N + 191) / 192) * ((M + 127) / 128);
-    const int64_t tiles_256 = static_cast<int64_t>((N + 255) / 256) * ((M + 127) / 128);
-    const int64_t rounds_192 = (tiles_192 + 255) / 256, rounds_256 = (tiles_256 + 255) / 256;
-    if (M > 64 && K % TK == 0 && K >= 2048 && rounds_192 * 192 < rounds_256 * 256 &&
-        (rounds_192 == 1 ? tiles_192 >= 128 : tiles_192 * 16 >= rounds_192 * 256 * 13)) {
-      // tiles of 128 x 192, a ring of three, one block per compute unit, where their rounds of the chip cover
-      // fewer columns than those of the 256-wide tiles below and are full enough: a single round on half of the
-      // compute units or more (1,024 rows: 235 against 307 us for N = 3,584, K = 18,944, 390 against 500 for
-      // N = 5,120, K = 27,648, 61 against 75 for N = 4,608, K = 3,584), or several at least 13/16 full (2,048 rows:
-      // 762 against 825 for N = 5,120, K = 27,648; 4,096 rows: 189 against 203 for N = 4,608, K = 3,584)
-      if (launch_dma<kEpilogue, TO, 2, 3, 3>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream)) return 1;
-    } else
-    if (M > 64 && K % TK == 0 && K >= 2048 && big_blocks >= 256 && fills_rounds(tiles_256)) {
-      // tiles of 128 x 256, a ring of three, one block per compute unit, where such tiles come out in nearly full
-      // rounds of the chip (2,048 rows: 343 against 368 us for N = 3,584, K = 18,944, 198 against 234 for N = 7,168,
-      // K = 5,120; where the last round is half empty they lose: 138 against 121 for N = 4,608, K = 3,584)
-      if (launch_dma<kEpilogue, TO, 2, 4, 3>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream)) return 1;
-    } else
     if (M <= 64 && (N + 127) / 128 >= 256) {
       // one tile of rows against a long matrix (the vocabulary): tiles of 64 rows, so that no empty rows are staged
       if (launch_tile<kEpilogue, TO, 1, 2, 2, false>((N + 127) / 128, 1, 1, out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream)) return 1;
@@ -1149,28 +912,6 @@ extern "C" int alofa_gemm_mfma(void* out, int o_dtype, int64_t ldo, const void* 
     return launch_mfma<kMfGeglu, bf16_t>(out, ldo, A, lda, W, W2, ldw, nullptr, M, N, K, stream, kNoNorm, done);
   }
   ALOFA_REQUIRE(false, "gemm_mfma: unsupported epilogue %d with out dtype %d", epilogue, o_dtype);
-}
-
-// The same product by the tiles of 256 x 256 with eight waves whatever the sizes (alofa_gemm_mfma takes them where they
-// pay): K a multiple of 32. The operands as for alofa_gemm_mfma; norm_w and eps stand where alofa_gemm_skinny has them
-// and must be null and zero (no norm rides on this kernel).
-extern "C" int alofa_gemm_wide(void* out, int o_dtype, int64_t ldo, const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw,
-                               const float* bias, int M, int N, int K, int epilogue, const float* norm_w, float eps, hipStream_t stream) {
-  ALOFA_REQUIRE(M > 0 && N > 0 && K > 0 && K % 32 == 0, "gemm_wide: M=%d N=%d K=%d must be positive, K a multiple of 32", M, N, K);
-  ALOFA_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && lda >= K && ldw >= K && ldo >= N, "gemm_wide: lda=%lld, ldw=%lld must be multiples of 8 and cover K, ldo=%lld cover N",
-                static_cast<long long>(lda), static_cast<long long>(ldw), static_cast<long long>(ldo));
-  ALOFA_REQUIRE(reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0 && reinterpret_cast<uintptr_t>(W2) % 16 == 0,
-                "gemm_wide: operands must be 16-byte aligned");
-  ALOFA_REQUIRE(norm_w == nullptr && eps == 0.f, "gemm_wide: no norm rides on this kernel");
-  int failed = 1;
-  if (epilogue == kMfStore && o_dtype == kBF16) failed = launch_wide<kMfStore, bf16_t, 256, 256, 4, 2, 4>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream);
-  else if (epilogue == kMfStore && o_dtype == kF32) failed = launch_wide<kMfStore, float, 256, 256, 4, 2, 4>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream);
-  else if (epilogue == kMfResidual && o_dtype == kF32) failed = launch_wide<kMfResidual, float, 256, 256, 4, 2, 4>(out, ldo, A, lda, W, ldw, nullptr, M, N, K, stream);
-  else if (epilogue == kMfSwiglu && o_dtype == kBF16 && W2 != nullptr) failed = launch_wide<kMfSwiglu, bf16_t, 256, 256, 4, 2, 4>(out, ldo, A, lda, W, ldw, nullptr, M, N, K, stream, W2);
-  else if (epilogue == kMfGeglu && o_dtype == kBF16 && W2 != nullptr) failed = launch_wide<kMfGeglu, bf16_t, 256, 256, 4, 2, 4>(out, ldo, A, lda, W, ldw, nullptr, M, N, K, stream, W2);
-  else ALOFA_REQUIRE(false, "gemm_wide: unsupported epilogue %d with out dtype %d", epilogue, o_dtype);
-  if (failed) return 1;
-  return check_launch("gemm_wide");
 }
 
 // out[m] = the column n with the highest sum_k A[m, k] * W[n, k] (the lowest n among equals), for M <= 64 rows

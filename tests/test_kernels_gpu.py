@@ -1178,3 +1178,28 @@ def test_gemm_with_operands_beyond_the_l2():
     out = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
     ops().gemm_swiglu(out, t(a, torch.bfloat16), t(g, torch.bfloat16), t(u, torch.bfloat16), kernel="tiled")
     close(out, pm.swiglu(pm.linear(a, g), pm.linear(a, u)), BF16, "swiglu")
+
+
+# every form of the product for many rows (the last gated one too), edges in both directions, whole and half slabs along K, as few slabs as the ring holds and fewer
+@pytest.mark.parametrize("M,N,K,form", [(2045, 10230, 2080, 0), (2045, 8187, 224, 1), (2045, 6140, 96, 2), (2045, 5117, 192, 3), (2045, 4091, 256, 4), (1021, 6140, 320, 5), (517, 4093, 64, 6), (517, 4093, 320, 6), (300, 5120, 32, 6)])
+def test_forms_of_the_product_for_many_rows(M, N, K, form):
+    from alofa_amd.csrc.build import load
+    assert load().alofa_gemm_wide_form(M, N, K, 0) == form
+    gen = torch.Generator(device=DEV).manual_seed(M + N + K)
+    a, w, w2 = (torch.randn(s, generator=gen, device=DEV).bfloat16() for s in ((M, K), (N, K), (N, K)))
+    out = torch.full((M, N + 5), 3.0, device=DEV)      # (what lies beyond a row's end stays as it was)
+    ops().gemm(out[:, :N], a, w, kernel="wide")
+    want = a.float() @ w.float().t()
+    # float sums of K products of order one: 2^-24 a sum, K sums, of numbers of order sqrt(K)
+    bound = K ** 1.5 * 2.0 ** -24 * 4
+    assert (out[:, :N] - want).abs().max().item() <= bound and bool((out[:, N:] == 3.0).all())
+    res = torch.randn(M, N, generator=gen, device=DEV)
+    acc = res.clone()
+    ops().gemm(acc, a, w, add_to_out=True, kernel="wide")
+    assert (acc - (res + want)).abs().max().item() <= bound + 2e-6 * (res + want).abs().max().item()
+    for n in (N // 2, N):      # gate and up: both gated forms
+        gated = torch.full((M, n + 5), 3.0, device=DEV, dtype=torch.bfloat16)
+        ops().gemm_swiglu(gated[:, :n], a, w[:n], w2[:n], kernel="wide")
+        up = a.float() @ w2[:n].float().t()
+        ref = torch.nn.functional.silu(want[:, :n]) * up
+        assert (gated[:, :n].float() - ref).abs().max().item() <= (2.0 ** -8 + 1e-5) * ref.abs().max().item() and bool((gated[:, n:] == 3.0).all())
