@@ -859,6 +859,30 @@ def pair_tiles(runs: list, window: Optional[int] = None, heads: Optional[int] = 
     return out
 
 
+TALL_ROWS = 256     # query rows a block of the attention kernel for many rows serves
+
+
+def attention_tall_pays(heads: int, d: int, block_size: int, scale: float, runs: int) -> bool:
+    """Whether ``runs`` runs of up to ``TALL_ROWS`` query rows go to the kernel with blocks of that many rows of one head: heads of 128,
+    pages of 16 tokens or more, and blocks for five eighths of the compute units. us, the kernel with blocks of 64 rows / this: 28/4 heads, four
+    portions of some 480 rows on 256 to 1,536 keys (224 blocks) 82 / 63, 16/16 heads, three prompts of 1,024 (192 blocks) 60 / 36, 40/8
+    heads, one prompt of 2,048 (320) 118 / 68; with fewer blocks the longest of them is what the launch waits for: 16/2 heads, one prompt of 2,048 (128) 47 / 57, 12/2 heads (96) 45 / 55."""
+    return d == 128 and block_size >= 16 and scale > 0 and runs * heads * 8 >= 5 * compute_units()
+
+
+def attention_tall(out, q, k_cache, v_cache, block_table, runs, heads, kv_heads, d, window, scale) -> None:
+    """bfloat16 attention for launches of many query rows (head size 128). ``runs`` is int32 [n, 4]: (request index, first row,
+    rows <= ``TALL_ROWS``, position of the first row), the ones that see most keys first; a block serves one run and one query head."""
+    T, bs = _attention_operands(out, q, k_cache, v_cache, block_table, heads, kv_heads, d)
+    if out.dtype is not torch.bfloat16:
+        raise AlofaError("unsupported", "the attention kernel for many rows leaves bfloat16 rows", f"out={out.dtype}")
+    _gpu("runs", runs, torch.int32, 2), _contig("runs", runs)
+    if runs.shape[1] != 4 or runs.shape[0] == 0:
+        raise AlofaError("shape_mismatch", "runs must be [n, 4]", f"runs={tuple(runs.shape)}")
+    _call("alofa_attention_tall", _ptr(out), _L(_rows("out", out)), _ptr(q), _L(_rows("q", q)), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), _I(block_table.shape[1]),
+          _ptr(runs), _I(runs.shape[0]), _I(heads), _I(kv_heads), _I(d), _I(bs), _I(int(window or 0)), _F(scale), _stream())
+
+
 def attention_prefill(out, q, k_cache, v_cache, block_table, tiles, heads, kv_heads, d, window, scale, share: int = 0,
                       rows: int = 16, v_head: Optional[int] = None, fine_weights: bool = False, all_value_heads: bool = False,
                       sink: Optional[torch.Tensor] = None) -> None:

@@ -31,7 +31,7 @@ class RowPlan:
     Built once per step from the spans and used by every attention layer."""
 
     def __init__(self, ctx):
-        spans = ctx.spans
+        spans = self.spans = ctx.spans
         self.device = ctx.device
         self.n_short = sum(s.n for s in spans if s.n <= SHORT)
         self.short_rows = None      # int32 indices of the short rows; None when every row is short (or none is)
@@ -43,6 +43,17 @@ class RowPlan:
             if self.n_short:
                 self.short_rows = torch.tensor([r for s in spans if s.n <= SHORT for r in range(s.row0, s.row0 + s.n)],
                                                dtype=torch.int32, device=self.device)
+
+    @property
+    def n_tall(self) -> int:
+        """How many runs of up to ``ops.TALL_ROWS`` rows the long portions make."""
+        return sum(-(-s.n // ops.TALL_ROWS) for s in self.spans if s.n > SHORT)
+
+    def tall_runs(self):
+        """The long portions in runs of up to ``ops.TALL_ROWS`` rows, the ones that see most keys first: int32 [n, 4] (request index, first row, rows, position of the first row)."""
+        size = ops.TALL_ROWS
+        runs = [(i, s.row0 + q0, min(size, s.n - q0), s.pos0 + q0) for i, s in enumerate(self.spans) if s.n > SHORT for q0 in range(0, s.n, size)]
+        return torch.tensor(sorted(runs, key=lambda r: -(r[3] + r[2])), dtype=torch.int32, device=self.device)
 
     def runs_of_sixteen(self):
         """The runs in pieces of up to sixteen rows: int32 [n, 3] (request index, first row, rows)."""
@@ -96,7 +107,9 @@ def paged_attend(ctx, entry, qkv, attn, heads, kv_heads, d, window, scale, posit
         # the exact path, and page or head sizes the bfloat16 kernels are not built for
         ops.paged_attention(attn, qkv, kv.k, kv.v, kv.block_table, ctx.req_of_token, ctx.positions, *common, exact)
     else:
-        if plan.long_runs is not None:      # portions of prompts
+        if plan.long_runs is not None and ops.attention_tall_pays(heads, d, kv.k.shape[2], scale, plan.n_tall):      # portions of prompts, many rows
+            ops.attention_tall(attn, qkv, kv.k, kv.v, kv.block_table, ctx.memo("gqa_attention.tall_runs", plan.tall_runs), *common)
+        elif plan.long_runs is not None:      # portions of prompts
             tiles, share, rows = plan.tiles(heads, kv_heads, d, window)
             ops.attention_prefill(attn, qkv, kv.k, kv.v, kv.block_table, tiles, *common, share=share, rows=rows)
         if plan.n_short:                    # single tokens and very short portions, all query heads of a key head together

@@ -1203,3 +1203,43 @@ def test_forms_of_the_product_for_many_rows(M, N, K, form):
         up = a.float() @ w2[:n].float().t()
         ref = torch.nn.functional.silu(want[:, :n]) * up
         assert (gated[:, :n].float() - ref).abs().max().item() <= (2.0 ** -8 + 1e-5) * ref.abs().max().item() and bool((gated[:, n:] == 3.0).all())
+
+
+# runs that end within a tile, within a wave's rows and at either's edge; one row; history in whole and ragged tiles; windows shorter than a tile, than a block and longer; larger pages
+@pytest.mark.parametrize("heads,kv_heads,bs,window", [(5, 1, 16, None), (4, 2, 16, 40), (16, 8, 64, 300), (3, 3, 32, None), (2, 1, 16, 1)])
+def test_attention_of_many_rows(heads, kv_heads, bs, window):
+    d, size = 128, ops().TALL_ROWS
+    portions = [(1, 0), (size, 0), (size + 1, 77), (31, 500), (65, 64), (300, 5)]      # rows brought, keys before them
+    gen = torch.Generator(device=DEV).manual_seed(heads * 10 + bs)
+    per = [-(-(n + h) // bs) for n, h in portions]
+    order = torch.randperm(sum(per) + 2, generator=torch.Generator().manual_seed(1)).tolist()
+    kc = torch.full((len(order), kv_heads, bs, d), float("nan"), device=DEV, dtype=torch.bfloat16)      # (what no token has written is never read into a result)
+    vc = torch.full((len(order), kv_heads, d, bs), float("nan"), device=DEV, dtype=torch.bfloat16)
+    table = torch.full((len(portions), max(per) + 1), -1, dtype=torch.int32)
+    T = sum(n for n, _ in portions)
+    q = torch.randn(T, heads * d, generator=gen, device=DEV).bfloat16()
+    want, runs, row, used = [], [], 0, 0
+    scale = d ** -0.5 * 4      # (scores far apart: maxima that move)
+    for r, (n, h) in enumerate(portions):
+        pages = order[used:used + per[r]]
+        used += per[r]
+        k, v = (torch.randn(n + h, kv_heads, d, generator=gen, device=DEV).bfloat16() for _ in range(2))
+        for j in range(n + h):
+            kc[pages[j // bs], :, j % bs], vc[pages[j // bs], :, :, j % bs] = k[j], v[j]
+        lowest = 0 if window is None else max(0, h - window + 1)
+        for j, page in enumerate(pages):
+            table[r, j] = -1 if (j + 1) * bs <= lowest else page      # (pages that a window has passed are given back)
+        runs += [(r, row + o, min(size, n - o), h + o) for o in range(0, n, size)]
+        kk, vv = (x.float().repeat_interleave(heads // kv_heads, 1) for x in (k, v))
+        s = torch.einsum("nhd,khd->hnk", q[row:row + n].float().view(n, heads, d), kk) * scale
+        at, key = torch.arange(h, h + n, device=DEV)[:, None], torch.arange(n + h, device=DEV)[None]
+        s.masked_fill_((key > at) | (key <= at - window if window is not None else torch.zeros_like(key > at)), float("-inf"))
+        want.append(torch.einsum("hnk,khd->nhd", torch.softmax(s, -1), vv).reshape(n, heads * d))
+        row += n
+    out = torch.zeros(T, heads * d, device=DEV, dtype=torch.bfloat16)
+    runs = torch.tensor(sorted(runs, key=lambda x: -(x[3] + x[2])), dtype=torch.int32, device=DEV)
+    ops().attention_tall(out, q, kc, vc, table.to(DEV), runs, heads, kv_heads, d, window, scale)
+    close(out, torch.cat(want).cpu().numpy(), BF16, "many rows")
+    again = torch.zeros_like(out)
+    ops().attention_tall(again, q, kc, vc, table.to(DEV), runs, heads, kv_heads, d, window, scale)
+    assert torch.equal(again, out)
