@@ -1,5 +1,5 @@
-"""Builds the HIP sources of this folder into one shared library for gfx950
-and the C++ host runtime (host/) into another, and loads them. The library's file name carries a hash of the sources and flags,
+"""Builds the HIP sources of this folder into one shared library for gfx950,
+the C++ host runtime (host/) into another and the way from Python to the kernels' entries (host/binding/) into a third, and loads them. The library's file name carries a hash of the sources and flags,
 so a stale build is never loaded: when no file of the current hash exists, it
 is compiled at the first call (a line is printed for every file meanwhile)."""
 from __future__ import annotations
@@ -92,6 +92,85 @@ def build_host(force: bool = False) -> Path:
             except OSError:
                 pass
     return out
+
+
+_binding = None
+BINDING_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+BINDING_LIBS = ["-ltorch_python", "-ltorch_cpu", "-lc10"]      # (in the process already when it is loaded: no search path is kept)
+
+
+def binding_sources() -> list:
+    return sorted((HERE / "host" / "binding").glob("*.cpp"))
+
+
+def _binding_name() -> str:
+    import torch
+    # (it is built against torch's and the interpreter's headers: another version of either needs a build of its own)
+    h = hashlib.sha256(" ".join([*BINDING_FLAGS, *BINDING_LIBS, torch.__version__, sys.implementation.cache_tag]).encode())
+    for p in binding_sources():
+        h.update(p.name.encode())
+        h.update(p.read_bytes())
+    return f"libalofa_binding_{h.hexdigest()[:12]}.so"
+
+
+def find_built_binding():
+    name = _binding_name()
+    for d in _candidate_dirs():
+        if (d / name).is_file():
+            return d / name
+    return None
+
+
+def build_binding(force: bool = False) -> Path:
+    """Compile the binding (plain C++, no GPU code) against torch's and Python's headers."""
+    if not force:
+        found = find_built_binding()
+        if found:
+            return found
+    import sysconfig
+    from torch.utils import cpp_extension      # (it knows where torch's headers lie)
+    cxx = next((c for c in (os.environ.get("CXX"), shutil.which("g++"), shutil.which("c++"), shutil.which("clang++")) if c), None)
+    if cxx is None:
+        raise AlofaError("not_initialized", "no C++ compiler was found; the binding cannot be built")
+    target_dir = next((d for d in _candidate_dirs() if _writable(d)), None)
+    if target_dir is None:
+        raise AlofaError("io", "no writable folder for the built library", f"tried={[str(d) for d in _candidate_dirs()]}")
+    import torch
+    out = target_dir / _binding_name()
+    tmp = target_dir / (out.name + f".tmp{os.getpid()}")
+    where = [f"-I{p}" for p in [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]]]
+    _say(f"compiling the binding into {target_dir}")
+    r = subprocess.run([cxx, *BINDING_FLAGS, f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *where, "-o", str(tmp), *map(str, binding_sources()),
+                        *(f"-L{p}" for p in cpp_extension.library_paths()), *BINDING_LIBS],
+                       capture_output=True, text=True)
+    if r.returncode != 0:
+        raise AlofaError("io", "compiling the binding failed (it needs Python's development headers)", r.stderr[-4000:])
+    os.replace(tmp, out)
+    for old in target_dir.glob("libalofa_binding_*.so"):
+        if old != out:
+            try:
+                old.unlink()
+            except OSError:
+                pass
+    return out
+
+
+def load_binding():
+    """The binding's module (csrc/host/binding/fastcall.cpp); built first when missing."""
+    global _binding
+    if _binding is None:
+        import importlib.machinery
+        import importlib.util
+        import torch  # noqa: F401  (its libraries are what the binding's symbols resolve to)
+        path = find_built_binding() or build_binding()
+        loader = importlib.machinery.ExtensionFileLoader("alofa_fastcall", str(path))
+        try:
+            _binding = importlib.util.module_from_spec(importlib.util.spec_from_loader("alofa_fastcall", loader))
+            loader.exec_module(_binding)
+        except ImportError as e:
+            _binding = None
+            raise AlofaError("not_initialized", "the binding cannot be loaded", f"path={path} reason={e}") from None
+    return _binding
 
 
 def load_host() -> ctypes.CDLL:

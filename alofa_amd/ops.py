@@ -5,22 +5,21 @@ fallback: a tensor that is not on the GPU, or a missing library, is an error."""
 from __future__ import annotations
 
 import ctypes
+import operator
 import os
 from typing import Optional
 
 import torch
 
-from .csrc.build import load
+from .csrc.build import load, load_binding
 from .errors import AlofaError
 
 F32, BF16 = 0, 1
 STORE, ADD_TO_RESIDUAL = 0, 1
 MAX_HEAD_DIM = 256
 
-_P = ctypes.c_void_p
-_I = ctypes.c_int
-_L = ctypes.c_int64
-_F = ctypes.c_float
+_I = _L = operator.index      # (what the binding's ``call`` takes: integers, floats, tensors and None as they are)
+_F = float
 
 
 def dtype_code(t: torch.Tensor) -> int:
@@ -61,13 +60,13 @@ def _contig(name: str, t: torch.Tensor) -> torch.Tensor:
     return t
 
 
-_scoped_stream: Optional[ctypes.c_void_p] = None
+_scoped_stream: Optional[int] = None
 
 
-def _stream() -> ctypes.c_void_p:
+def _stream() -> int:
     if _scoped_stream is not None:
         return _scoped_stream
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch.cuda.current_stream().cuda_stream
 
 
 class stream_scope:
@@ -79,7 +78,7 @@ class stream_scope:
     def __enter__(self):
         global _scoped_stream
         self._outer = _scoped_stream
-        _scoped_stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        _scoped_stream = torch.cuda.current_stream().cuda_stream
         return self
 
     def __exit__(self, *exc):
@@ -88,19 +87,42 @@ class stream_scope:
         return False
 
 
-_entries: dict = {}      # the library's entry points by name (looked up once: a step makes some two hundred calls)
+_entries: dict = {}      # addresses of the library's entry points by name (looked up once: a step makes some two hundred calls)
+_binding = None
+
+
+def _native():
+    """The binding (csrc/host/binding): the calls themselves and the checks of the operations that every layer runs."""
+    global _binding
+    if _binding is None:
+        _binding = load_binding()
+    return _binding
+
+
+def _answer(fn_name: str, *args) -> int:
+    """The entry's own answer. A parameter is a tensor (its memory), None (a null pointer), an integer or a float, as ``_ptr``, ``_I``, ``_L`` and ``_F`` leave them."""
+    address = _entries.get(fn_name)
+    if address is None:
+        address = _entries[fn_name] = ctypes.cast(getattr(load(), fn_name), ctypes.c_void_p).value
+    return _native().call(address, *args)
 
 
 def _call(fn_name: str, *args) -> None:
-    fn = _entries.get(fn_name)
-    if fn is None:
-        fn = _entries[fn_name] = getattr(load(), fn_name)
-    if fn(*args) != 0:
+    if _answer(fn_name, *args) != 0:
         raise AlofaError("invalid_argument", "kernel refused its arguments", load().alofa_last_error().decode())
 
 
-def _ptr(t: Optional[torch.Tensor]) -> ctypes.c_void_p:
-    return _P(t.data_ptr() if t is not None else None)
+def _ptr(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    return t
+
+
+def upload(values, device) -> torch.Tensor:
+    """Whole numbers that the host has laid out (nested lists), as an int32 tensor on the device. On the GPU by way of pinned memory and a copy on the
+    current stream that the host does not wait for: a plain ``torch.tensor`` there stops the host until everything in front of it on the stream has run (0.45 ms in
+    the middle of a step of prompts with 3 ms of kernels)."""
+    if torch.device(device).type != "cuda":
+        return torch.tensor(values, dtype=torch.int32, device=device)
+    return torch.tensor(values, dtype=torch.int32, pin_memory=True).to(device, non_blocking=True)      # (the pinned block is used again only after the copy)
 
 
 # ----------------------------------------------------------------- embedding
@@ -126,20 +148,24 @@ def embed_gather(out: torch.Tensor, table: torch.Tensor, ids: torch.Tensor, stor
 def rmsnorm(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, eps: float, exact: bool,
             rows: Optional[torch.Tensor] = None) -> None:
     """out[r] = rmsnorm(x[rows[r]] if rows is given else x[r]) * w."""
-    _gpu("out", out, None, 2), _gpu("x", x, torch.float32, 2), _gpu("w", w, torch.float32, 1)
-    _contig("out", out), _contig("x", x), _contig("w", w)
-    n, h = out.shape
-    if x.shape[1] != h or w.shape[0] != h:
-        raise AlofaError("shape_mismatch", "norm width does not fit", f"out={tuple(out.shape)} x={tuple(x.shape)} w={tuple(w.shape)}")
-    if rows is not None:
-        _gpu("rows", rows, torch.int32, 1), _contig("rows", rows)
-        if rows.shape[0] != n:
-            raise AlofaError("shape_mismatch", "one row index per output row", f"rows={tuple(rows.shape)} out={tuple(out.shape)}")
-    elif x.shape[0] != n:
-        raise AlofaError("shape_mismatch", "norm row count does not fit", f"out={tuple(out.shape)} x={tuple(x.shape)}")
-    if exact and out.dtype is not torch.float32:
+    sizes = _native().norm(out, x, w, rows)
+    if sizes is None:
+        _gpu("out", out, None, 2), _gpu("x", x, torch.float32, 2), _gpu("w", w, torch.float32, 1)
+        _contig("out", out), _contig("x", x), _contig("w", w)
+        n, h = out.shape
+        if x.shape[1] != h or w.shape[0] != h:
+            raise AlofaError("shape_mismatch", "norm width does not fit", f"out={tuple(out.shape)} x={tuple(x.shape)} w={tuple(w.shape)}")
+        if rows is not None:
+            _gpu("rows", rows, torch.int32, 1), _contig("rows", rows)
+            if rows.shape[0] != n:
+                raise AlofaError("shape_mismatch", "one row index per output row", f"rows={tuple(rows.shape)} out={tuple(out.shape)}")
+        elif x.shape[0] != n:
+            raise AlofaError("shape_mismatch", "norm row count does not fit", f"out={tuple(out.shape)} x={tuple(x.shape)}")
+        sizes = n, h, dtype_code(out)
+    n, h, code = sizes
+    if exact and code != F32:
         raise AlofaError("invalid_argument", "the exact path is float32 throughout", f"out={out.dtype}")
-    _call("alofa_rmsnorm", _ptr(out), _I(dtype_code(out)), _ptr(x), _ptr(w), _ptr(rows), _I(n), _I(h), _F(eps), _I(int(exact)), _stream())
+    _call("alofa_rmsnorm", _ptr(out), code, _ptr(x), _ptr(w), _ptr(rows), n, h, _F(eps), _I(int(exact)), _stream())
 
 
 # ------------------------------------------------------------ matrix product
@@ -286,16 +312,6 @@ def _ensure_workspace(device) -> None:
         _workspace_ready = True
 
 
-def _mfma_operands(a: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether the bfloat16 MFMA kernels can take these operands: 16-byte loads
-    along K need K and the leading dimensions in multiples of 8 and aligned bases."""
-    if a.dtype is not torch.bfloat16 or w.dtype is not torch.bfloat16:
-        return False
-    K = a.shape[1]
-    return (K % 8 == 0 and _rows("a", a) % 8 == 0 and _rows("w", w) % 8 == 0
-            and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
-
-
 def norm_goes_apart(M: int, N: int, K: int) -> bool:
     """Whether a norm in front of a plain product of at most eight rows should run as a kernel of its own although
     a product could take it along: the vector-unit kernel reads every row once per four columns, float32 rows
@@ -357,9 +373,13 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[tor
     activation dtype) holds the RMSNorm of out's new rows. Where the product's last launch has whole
     rows in hand (the tiled kernel with K shared out and a launch that adds the shares) the norm rides
     on it; everywhere else it is the norm kernel, run here: the values are the same either way."""
-    _gpu("out", out, None, 2), _gpu("a", a, None, 2), _gpu("w", w, None, 2)
-    M, K = a.shape
-    N = w.shape[0]
+    sizes = None if exact or norm is not None else _native().product(out, a, w, None, bias)      # (bfloat16 operands that 16-byte loads along K can read)
+    if sizes is not None:
+        M, N, K, ldo, lda, ldw, code = sizes
+    else:
+        _gpu("out", out, None, 2), _gpu("a", a, None, 2), _gpu("w", w, None, 2)
+        M, K = a.shape
+        N = w.shape[0]
     then_w = then_rows = None
     then_eps = 0.0
     if then_norm is not None:
@@ -379,31 +399,30 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[tor
         _call(_product_entry(kernel, M, N, K, normed=True), _ptr(out), _I(BF16), _L(_rows("out", out)), _ptr(a), _L(_rows("a", a)), _ptr(w), _ptr(None), _L(_rows("w", w)),
               _ptr(bias), _I(M), _I(N), _I(K), _I(STORE), *_norm_operands(a, norm, K), _stream())
         return
-    if w.shape[1] != K or tuple(out.shape) != (M, N):
-        raise AlofaError("shape_mismatch", "matrix product shapes do not fit", f"a={tuple(a.shape)} w={tuple(w.shape)} out={tuple(out.shape)}")
-    if bias is not None:
-        _gpu("bias", bias, torch.float32, 1), _contig("bias", bias)
-        if bias.shape[0] != N:
-            raise AlofaError("shape_mismatch", "bias length does not fit", f"bias={tuple(bias.shape)} N={N}")
+    if sizes is None:
+        if w.shape[1] != K or tuple(out.shape) != (M, N):
+            raise AlofaError("shape_mismatch", "matrix product shapes do not fit", f"a={tuple(a.shape)} w={tuple(w.shape)} out={tuple(out.shape)}")
+        if bias is not None:
+            _gpu("bias", bias, torch.float32, 1), _contig("bias", bias)
+            if bias.shape[0] != N:
+                raise AlofaError("shape_mismatch", "bias length does not fit", f"bias={tuple(bias.shape)} N={N}")
     if add_to_out and out.dtype is not torch.float32:
         raise AlofaError("invalid_argument", "the residual stream is float32", f"out={out.dtype}")
     if add_to_out and bias is not None:
         # no kernel's residual epilogue adds a bias: the same call would otherwise give different results by dtype
         raise AlofaError("unsupported", "a product that adds to the residual stream takes no bias; add the bias in a buffer of its own")
-    if not exact and _mfma_operands(a, w):
+    if sizes is not None:
         _ensure_workspace(a.device)
         if kernel is None and then_rows is not None and then_rows.dtype is torch.bfloat16 and FUSE_NORMS and norm_rides_on_shares(M, N, K):
             kernel = "tiled"
         entry = _product_entry(kernel, M, N, K)
-        done = _I(0)
+        done = ctypes.c_int(0)
         if entry == "alofa_gemm_mfma":
             ride = then_rows is not None and then_rows.dtype is torch.bfloat16 and FUSE_NORMS
-            more = (_ptr(then_w if ride else None), _F(then_eps), _ptr(then_rows if ride else None), _L(N), ctypes.byref(done))
+            more = (then_w if ride else None, _F(then_eps), then_rows if ride else None, N, ctypes.addressof(done))
         else:
-            more = (_ptr(None), _F(0.0))
-        _call(entry, _ptr(out), _I(dtype_code(out)), _L(_rows("out", out)),
-              _ptr(a), _L(_rows("a", a)), _ptr(w), _ptr(None), _L(_rows("w", w)), _ptr(bias), _I(M), _I(N), _I(K),
-              _I(ADD_TO_RESIDUAL if add_to_out else STORE), *more, _stream())
+            more = (None, 0.0)
+        _call(entry, out, code, ldo, a, lda, w, None, ldw, bias, M, N, K, ADD_TO_RESIDUAL if add_to_out else STORE, *more, _stream())
         if then_rows is not None and not done.value:
             rmsnorm(then_rows, out, then_w, then_eps, False)
         return
@@ -427,6 +446,14 @@ def gemm_swiglu(out: torch.Tensor, a: torch.Tensor, w_gate: torch.Tensor, w_up: 
     """out = act(a @ w_gate.T) * (a @ w_up.T), act "silu" or "gelu_tanh". ``kernel`` and ``norm`` as for ``gemm``."""
     if act not in GATED:
         raise AlofaError("unsupported", "no such activation of a gate", f"act={act}")
+    sizes = None if exact or norm is not None else _native().product(out, a, w_gate, w_up, None)      # (bfloat16 operands that 16-byte loads along K can read)
+    if sizes is not None:
+        M, N, K, ldo, lda, ldw, _ = sizes
+        _ensure_workspace(a.device)
+        entry = _product_entry(kernel, M, 2 * N, K, True)
+        more = (None, 0.0) if entry != "alofa_gemm_mfma" else (None, 0.0, None, 0, None)
+        _call(entry, out, BF16, ldo, a, lda, w_gate, w_up, ldw, None, M, N, K, GATED[act], *more, _stream())
+        return
     _gpu("out", out, None, 2), _gpu("a", a, None, 2), _gpu("w_gate", w_gate, None, 2), _gpu("w_up", w_up, None, 2)
     M, K = a.shape
     N = w_gate.shape[0]
@@ -439,13 +466,6 @@ def gemm_swiglu(out: torch.Tensor, a: torch.Tensor, w_gate: torch.Tensor, w_up: 
             raise AlofaError("unsupported", "no kernel takes a norm with this product", f"a={tuple(a.shape)} gate={tuple(w_gate.shape)} out={out.dtype}")
         _call(_product_entry(kernel, M, 2 * N, K, True, normed=True), _ptr(out), _I(BF16), _L(_rows("out", out)), _ptr(a), _L(_rows("a", a)), _ptr(w_gate), _ptr(w_up),
               _L(_rows("w_gate", w_gate)), _ptr(None), _I(M), _I(N), _I(K), _I(GATED[act]), *_norm_operands(a, norm, K), _stream())
-        return
-    if not exact and out.dtype is torch.bfloat16 and _mfma_operands(a, w_gate) and _mfma_operands(a, w_up):
-        _ensure_workspace(a.device)
-        entry = _product_entry(kernel, M, 2 * N, K, True)
-        more = (_ptr(None), _F(0.0)) if entry != "alofa_gemm_mfma" else (_ptr(None), _F(0.0), _ptr(None), _L(0), _ptr(None))
-        _call(entry, _ptr(out), _I(BF16), _L(_rows("out", out)), _ptr(a), _L(_rows("a", a)), _ptr(w_gate), _ptr(w_up),
-              _L(_rows("w_gate", w_gate)), _ptr(None), _I(M), _I(N), _I(K), _I(GATED[act]), *more, _stream())
         return
     if exact and a.dtype is torch.float32 and w_gate.dtype is torch.float32 and out.dtype is torch.float32:
         _call("alofa_gemm_swiglu_exact", _ptr(out), _L(_rows("out", out)), _ptr(a), _L(_rows("a", a)), _ptr(w_gate), _ptr(w_up), _L(_rows("w_gate", w_gate)),
@@ -475,23 +495,11 @@ def check_cache(name: str, cache: torch.Tensor, kv_heads: int, d: int, transpose
     return bs
 
 
-_checked_caches: dict = {}      # id(key cache) -> (key cache, value cache, kv_heads, d, block size): what has been checked already
-
-
 def check_caches(k_cache: torch.Tensor, v_cache: torch.Tensor, kv_heads: int, d: int) -> int:
-    """Key cache and (transposed) value cache of one layer; returns block_size. (A layer's caches are the same
-    two tensors step after step, and three kernels a layer ask: what has been checked is remembered by object.)"""
-    known = _checked_caches.get(id(k_cache))
-    if known is not None and known[0] is k_cache and known[1] is v_cache and known[2] == kv_heads and known[3] == d:
-        return known[4]
-    bs = _check_caches(k_cache, v_cache, kv_heads, d)
-    if len(_checked_caches) > 4096:
-        _checked_caches.clear()
-    _checked_caches[id(k_cache)] = (k_cache, v_cache, kv_heads, d, bs)
-    return bs
-
-
-def _check_caches(k_cache: torch.Tensor, v_cache: torch.Tensor, kv_heads: int, d: int) -> int:
+    """Key cache and (transposed) value cache of one layer; returns block_size."""
+    known = _native().caches(k_cache, v_cache, kv_heads, d)
+    if known is not None:
+        return known
     bs = check_cache("k_cache", k_cache, kv_heads, d)
     if check_cache("v_cache", v_cache, kv_heads, d, transposed=True) != bs or k_cache.shape[0] != v_cache.shape[0] or k_cache.dtype is not v_cache.dtype:
         raise AlofaError("shape_mismatch", "key and value caches must agree in blocks, block size and dtype",
@@ -507,6 +515,11 @@ def rope_kv_write(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, posit
     the rotated keys and the values to each token's slot. ``cos``/``sin`` are
     float32 [positions, d/2]. Positions and slots are checked by the caller
     against the table and the cache."""
+    sizes = None if k_cache is None else _native().turn(qkv, cos, sin, positions, slots, k_cache, v_cache, heads, kv_heads, d)
+    if sizes is not None:
+        T, ld, code, bs = sizes
+        _call("alofa_rope_kv_write", qkv, code, ld, cos, sin, positions, slots, k_cache, v_cache, T, heads, kv_heads, d, bs, 1, _stream())
+        return
     _gpu("qkv", qkv, None, 2)
     T = qkv.shape[0]
     write = k_cache is not None
@@ -667,7 +680,7 @@ def paged_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v
         attention_decode(out, q, k_cache, v_cache, block_table, req_of_token, positions, heads, kv_heads, d, window, scale,
                          max_context or 1 << 30, scratch)
         return
-    if exact and q.dtype is torch.float32 and load().alofa_attention_exact_takes(_ptr(q), _L(_rows("q", q)), _ptr(k_cache), _ptr(v_cache), _I(d), _I(bs)):
+    if exact and q.dtype is torch.float32 and _answer("alofa_attention_exact_takes", _ptr(q), _L(_rows("q", q)), _ptr(k_cache), _ptr(v_cache), _I(d), _I(bs)):
         _call("alofa_attention_exact", _ptr(out), _L(_rows("out", out)), _ptr(q), _L(_rows("q", q)), _ptr(k_cache), _ptr(v_cache), _ptr(block_table),
               _I(block_table.shape[1]), _ptr(req_of_token), _ptr(positions), _I(T), _I(heads), _I(kv_heads), _I(d), _I(bs), _I(int(window or 0)), _F(scale), _stream())
         return
@@ -678,6 +691,9 @@ def paged_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v
 
 def _attention_operands(out, q, k_cache, v_cache, block_table, heads, kv_heads, d):
     # (float32 ``out``: the kernels leave their results unrounded there)
+    known = _native().attention(out, q, k_cache, v_cache, block_table, heads, kv_heads, d)
+    if known is not None:
+        return known
     _gpu("out", out, torch.float32 if out.dtype is torch.float32 else torch.bfloat16, 2), _gpu("q", q, torch.bfloat16, 2)
     T = q.shape[0]
     if out.shape[0] != T or out.shape[1] < heads * d or q.shape[1] < heads * d:
@@ -1372,8 +1388,8 @@ def linear_recurrence(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: to
         _gpu("bonus", bonus, torch.float32, 2), _contig("bonus", bonus)
         if tuple(bonus.shape) != (heads, dk) or not before_update:
             raise AlofaError("shape_mismatch", "the bonus is [heads, dk] and goes with the read-out before the update", f"bonus={tuple(bonus.shape)}")
-    used = _I(1)
-    _call("alofa_linear_recurrence", _ptr(out), _I(max_parts), _L(part_stride), ctypes.byref(used), _ptr(q), _L(_rows("q", q)), _ptr(k), _L(_rows("k", k)), _ptr(v), _L(_rows("v", v)), _I(dtype_code(q)),
+    used = ctypes.c_int(1)
+    _call("alofa_linear_recurrence", _ptr(out), _I(max_parts), _L(part_stride), ctypes.addressof(used), _ptr(q), _L(_rows("q", q)), _ptr(k), _L(_rows("k", k)), _ptr(v), _L(_rows("v", v)), _I(dtype_code(q)),
           _ptr(None if per_head else decay), _L(0 if per_head else _rows("decay", decay)), _ptr(decay if per_head else None), _ptr(bonus), _ptr(state),
           _ptr(rows.slots), _ptr(rows.offsets), _I(rows.requests), _I(T), _I(heads), _I(dk), _I(dv), _I(decay_kind), _F(tau), _F(q_scale), _F(k_scale),
           _I(int(before_update)), _stream())
@@ -1395,7 +1411,7 @@ class Chunks:
             of_request.append((len(chunks), -(-n // CHUNK_ROWS)))
             chunks += [(r, row0 + a, min(CHUNK_ROWS, n - a), 0) for a in range(0, n, CHUNK_ROWS)]
         self.requests, self.count, self.rows = len(of_request), len(chunks), sum(n for _, n in spans)
-        both = torch.tensor([x for c in chunks for x in c] + [x for c in of_request for x in c], dtype=torch.int32, device=device)
+        both = upload([x for c in chunks for x in c] + [x for c in of_request for x in c], device)
         self.chunks, self.of_request = both[:4 * self.count], both[4 * self.count:]
 
 

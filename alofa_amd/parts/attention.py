@@ -41,8 +41,7 @@ class RowPlan:
             self.long_runs = [(i, s.row0 + q0, min(TILE_ROWS, s.n - q0), s.pos0 + q0)
                               for i, s in enumerate(spans) if s.n > SHORT for q0 in range(0, s.n, TILE_ROWS)]
             if self.n_short:
-                self.short_rows = torch.tensor([r for s in spans if s.n <= SHORT for r in range(s.row0, s.row0 + s.n)],
-                                               dtype=torch.int32, device=self.device)
+                self.short_rows = ops.upload([r for s in spans if s.n <= SHORT for r in range(s.row0, s.row0 + s.n)], self.device)
 
     @property
     def n_tall(self) -> int:
@@ -53,11 +52,11 @@ class RowPlan:
         """The long portions in runs of up to ``ops.TALL_ROWS`` rows, the ones that see most keys first: int32 [n, 4] (request index, first row, rows, position of the first row)."""
         size = ops.TALL_ROWS
         runs = [(i, s.row0 + q0, min(size, s.n - q0), s.pos0 + q0) for i, s in enumerate(self.spans) if s.n > SHORT for q0 in range(0, s.n, size)]
-        return torch.tensor(sorted(runs, key=lambda r: -(r[3] + r[2])), dtype=torch.int32, device=self.device)
+        return ops.upload(sorted(runs, key=lambda r: -(r[3] + r[2])), self.device)
 
     def runs_of_sixteen(self):
         """The runs in pieces of up to sixteen rows: int32 [n, 3] (request index, first row, rows)."""
-        return torch.tensor([(r, row0 + q0, min(16, n - q0)) for r, row0, n, _ in self.long_runs for q0 in range(0, n, 16)], dtype=torch.int32, device=self.device)
+        return ops.upload([(r, row0 + q0, min(16, n - q0)) for r, row0, n, _ in self.long_runs for q0 in range(0, n, 16)], self.device)
 
     def tiles(self, heads: int, kv_heads: int, d: int, window, plain: bool = False, fine: bool = False):
         """The runs as blocks of the prefill kernel for a mixer with these head counts, how many heads
@@ -70,7 +69,7 @@ class RowPlan:
             share = 0 if plain else ops.prefill_share(heads, kv_heads, d, len(self.long_runs))
             rows = 16 if plain or fine else ops.prefill_rows(heads, kv_heads, d, share, len(self.long_runs))
             per_run = ops.prefill_blocks_per_run(heads, kv_heads, share, rows)
-            self._tiles[key] = (torch.tensor(ops.pair_tiles(self.long_runs, window, per_run), dtype=torch.int32, device=self.device), share, rows)
+            self._tiles[key] = (ops.upload(ops.pair_tiles(self.long_runs, window, per_run), self.device), share, rows)
         return self._tiles[key]
 
 

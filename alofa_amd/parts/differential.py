@@ -141,7 +141,7 @@ class DifferentialAttention(Mixer):
             return
         common = (H, G, D, self.window, self.keep_first, self.scale, self.softcap, self.end)
         if plan.long_runs is not None:      # portions of prompts
-            tiles = ctx.memo("runs of 64 rows", lambda: torch.tensor(plan.long_runs, dtype=torch.int32, device=ctx.device))
+            tiles = ctx.memo("runs of 64 rows", lambda: ops.upload(plan.long_runs, ctx.device))
             ops.maps_prefill(attn, q, kv.k, kv.v, kv.block_table, tiles, *common)
         if plan.n_short:                    # single tokens and very short portions
             parts = ops.maps_decode_plan(plan.n_short, H, G, D, ctx.max_context, self.window, self.keep_first)

@@ -45,7 +45,7 @@ USE_SPAN_MFMA = os.environ.get("ALOFA_SPAN_MFMA", "1") != "0"      # 0 (for meas
 def _runs_of_sixteen(ctx) -> torch.Tensor:
     """The step's rows as runs of up to sixteen rows of one request: int32 [n, 3] (request index, first row, rows)."""
     runs = [(i, s.row0 + q0, min(16, s.n - q0)) for i, s in enumerate(ctx.spans) for q0 in range(0, s.n, 16)]
-    return torch.tensor(runs, dtype=torch.int32, device=ctx.device)
+    return ops.upload(runs, ctx.device)
 
 
 def distance_buckets(rows: int, far: float, upto: int) -> list:
