@@ -16,11 +16,14 @@
 //
 //   more rows (exact_tile_kernel): slabs of 32 k through LDS, a wave owns 32 rows x 32 weight rows (four instructions for two
 //   loads of either operand), a block 64 x 64 (32 x 128 up to 32 rows). Bound by the matrix cores (69 TFLOP/s measured with
-//   nothing else in the loop; 46 of useful work at 450 rows, whose last tile is padding): the slab's traffic hides behind 2,048 cycles of
-//   instructions. K is shared out over blocks where the tiles are few; the shares' float64 sums go to a buffer of the caller's (not to the
-//   library's workspace, which one stream at a time may use) and a second launch adds them. 450 rows, us, as above: 9,728 x 896 with the gate
-//   377 / 169, 896 x 4,864 1,000 / 101 + 5, 896 x 896 185 / 25, 1,152 x 896 185 / 30 + 5.
+//   nothing else in the loop; 58 reached, 50 of them useful at 450 rows, whose last tile is padding) and by the widening, which the same SIMD does between the
+//   products. Two slabs are on their way in registers and two lie in LDS: with one of either, a slab that came late (1.4 us from a busy memory against 0.9 us of
+//   products) held up the block, 9,728 x 896 with the gate 167, 896 x 4,864 102 + 5. K is shared out over blocks where the tiles are few; the shares' float64 sums
+//   go to a buffer of the caller's (not to the library's workspace, which one stream at a time may use) and a second launch adds them. 450 rows, us, as above:
+//   9,728 x 896 with the gate 377 / 154, 896 x 4,864 1,000 / 84 both launches, 896 x 896 185 / 26, 1,152 x 896 185 / 31.
 #include "common.h"
+
+#include <type_traits>
 
 namespace alofa {
 
@@ -152,57 +155,105 @@ __global__ void __launch_bounds__(64 * NW) exact_rows_kernel(float* __restrict__
 // A block of WM x (4 / WM) waves, each 32 rows x 32 weight rows; kMats = 2: the weight rows of a wave are 16 of gate and the same 16 of up.
 // parts (with gridDim.z > 1): this share's sums, [share][M][N]; the epilogue is then the second launch's.
 template <int WM, int kMats, int kEpilogue, bool kVec>
-__global__ void __launch_bounds__(256) exact_tile_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ A, int64_t lda,
+__global__ void __launch_bounds__(256, WM == 2 ? 3 : 2) exact_tile_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ A, int64_t lda,
                                                          const float* __restrict__ W, const float* __restrict__ W2, int64_t ldw,
                                                          const float* __restrict__ bias, double* __restrict__ parts, int M, int N, int K, int k_share, int gelu) {
   constexpr int WN = 4 / WM, BM = 32 * WM, BW = 32 * WN, BK = 32, kPad = 4;
   constexpr int kOwn = 32 / kMats;                     // outputs of a wave along N
-  __shared__ __attribute__((aligned(16))) float As[BM][BK + kPad], Ws[BW][BK + kPad];      // (as doubles, widened once as they are brought: 174 us where this takes 169)
+  __shared__ __attribute__((aligned(16))) float As[2][BM][BK + kPad], Ws[2][BW][BK + kPad];      // (as doubles, widened once as they are brought: 174 us where this took 169)
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
   const int wm = wave / WN, wn = wave % WN;
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * WN * kOwn;
   const int k_begin = blockIdx.z * k_share, k_end = k_begin + k_share < K ? k_begin + k_share : K;
   constexpr int kA = BM * BK / 4 / 256, kW = BW * BK / 4 / 256;      // quads a thread brings of either operand
-  float4 fa[kA], fw[kW];
-  auto fetch = [&](int k0) __attribute__((always_inline)) {
+  const float *a_row[kA], *w_row[kW];      // (rows past the end: the last one again, its results are not stored)
 #pragma unroll
-    for (int i = 0; i < kA; ++i) {
-      const int at = threadIdx.x + i * 256, row = at / 8, m = m0 + row;
-      fa[i] = quad_within<kVec>(A + static_cast<int64_t>(m < M ? m : M - 1) * lda, k0 + at % 8 * 4, k_end);
-    }
+  for (int i = 0; i < kA; ++i) {
+    const int m = m0 + (threadIdx.x + i * 256) / 8;
+    a_row[i] = A + static_cast<int64_t>(m < M ? m : M - 1) * lda;
+  }
 #pragma unroll
-    for (int i = 0; i < kW; ++i) {
-      const int at = threadIdx.x + i * 256, row = at / 8, n = n0 + row / 32 * kOwn + row % kOwn;
-      fw[i] = quad_within<kVec>((kMats == 2 && row % 32 >= 16 ? W2 : W) + static_cast<int64_t>(n < N ? n : N - 1) * ldw, k0 + at % 8 * 4, k_end);
-    }
-  };
+  for (int i = 0; i < kW; ++i) {
+    const int row = (threadIdx.x + i * 256) / 8, n = n0 + row / 32 * kOwn + row % kOwn;
+    w_row[i] = (kMats == 2 && row % 32 >= 16 ? W2 : W) + static_cast<int64_t>(n < N ? n : N - 1) * ldw;
+  }
+  const int k_own = threadIdx.x % 8 * 4;      // (threadIdx.x + 256 i has the same place in its row)
   f64x4 acc[2][2];      // [rows of A][weight rows]
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f64x4{0, 0, 0, 0};
-  fetch(k_begin);
-  for (int k0 = k_begin; k0 < k_end; k0 += BK) {
-    __syncthreads();
+  // Two slabs in registers, on their way, while a third is worked on: a slab comes in some 1.4 us when the chip is busy, and its own products last 0.9.
+  // (The loads of whole slabs are issued whatever the thread: under a condition each would be waited for by itself.)
+  float4 fa[2][kA], fw[2][kW];
+  auto fetch = [&](auto set, int slab) __attribute__((always_inline)) {
+    constexpr int x = decltype(set)::value;
 #pragma unroll
-    for (int i = 0; i < kA; ++i) *reinterpret_cast<float4*>(&As[(threadIdx.x + i * 256) / 8][threadIdx.x % 8 * 4]) = fa[i];
+    for (int i = 0; i < kA; ++i) fa[x][i] = quad<kVec>(a_row[i], k_begin + slab * BK + k_own);
 #pragma unroll
-    for (int i = 0; i < kW; ++i) *reinterpret_cast<float4*>(&Ws[(threadIdx.x + i * 256) / 8][threadIdx.x % 8 * 4]) = fw[i];
-    __syncthreads();
-    if (k0 + BK < k_end) fetch(k0 + BK);
+    for (int i = 0; i < kW; ++i) fw[x][i] = quad<kVec>(w_row[i], k_begin + slab * BK + k_own);
+  };
+  auto keep = [&](auto set) __attribute__((always_inline)) {
+    constexpr int x = decltype(set)::value;
+#pragma unroll
+    for (int i = 0; i < kA; ++i) *reinterpret_cast<float4*>(&As[x][(threadIdx.x + i * 256) / 8][k_own]) = fa[x][i];
+#pragma unroll
+    for (int i = 0; i < kW; ++i) *reinterpret_cast<float4*>(&Ws[x][(threadIdx.x + i * 256) / 8][k_own]) = fw[x][i];
+  };
+  auto multiply = [&](auto set) __attribute__((always_inline)) {
+    constexpr int x = decltype(set)::value;
 #pragma unroll
     for (int q = 0; q < BK / 16; ++q) {
       float4 a[2], w[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        a[i] = *reinterpret_cast<const float4*>(&As[wm * 32 + i * 16 + r][q * 16 + g * 4]);
-        w[i] = *reinterpret_cast<const float4*>(&Ws[wn * 32 + i * 16 + r][q * 16 + g * 4]);
+        a[i] = *reinterpret_cast<const float4*>(&As[x][wm * 32 + i * 16 + r][q * 16 + g * 4]);
+        w[i] = *reinterpret_cast<const float4*>(&Ws[x][wn * 32 + i * 16 + r][q * 16 + g * 4]);
       }
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = fma_quad(a[i], w[j], acc[i][j]);
     }
+  };
+  // (two slabs in LDS: a slab's place is written again two barriers after the barrier behind which it is read)
+  auto step = [&](auto set, int slab, auto more) __attribute__((always_inline)) {
+    keep(set);
+    if constexpr (decltype(more)::value) fetch(set, slab + 2);
+    __syncthreads();
+    multiply(set);
+  };
+  constexpr std::integral_constant<int, 0> first{};
+  constexpr std::integral_constant<int, 1> second{};
+  constexpr std::true_type more{};
+  constexpr std::false_type done{};
+  const int whole = (k_end - k_begin) / BK;
+  if (whole > 0) fetch(first, 0);
+  if (whole > 1) fetch(second, 1);
+  int slab = 0;
+  for (; slab + 3 < whole; slab += 2) {
+    step(first, slab, more);
+    step(second, slab + 1, more);
+  }
+  if (whole - slab == 3) {
+    step(first, slab, more);
+    step(second, slab + 1, done);
+    step(first, slab + 2, done);
+  } else if (whole - slab == 2) {
+    step(first, slab, done);
+    step(second, slab + 1, done);
+  } else if (whole - slab == 1) {
+    step(first, slab, done);
+  }
+  if (k_begin + whole * BK < k_end) {      // the last k, fewer than a slab
+#pragma unroll
+    for (int i = 0; i < kA; ++i) fa[0][i] = quad_within<kVec>(a_row[i], k_begin + whole * BK + k_own, k_end);
+#pragma unroll
+    for (int i = 0; i < kW; ++i) fw[0][i] = quad_within<kVec>(w_row[i], k_begin + whole * BK + k_own, k_end);
+    __syncthreads();
+    keep(first);
+    __syncthreads();
+    multiply(first);
   }
   // D: rows of A 4 v + g, weight row r
 #pragma unroll
@@ -243,8 +294,9 @@ __global__ void __launch_bounds__(256) exact_sum_kernel(float* __restrict__ out,
 }
 
 // How K is shared out over blocks: the number of shares (at most 16, at least 128 k each) with the least time of the compute unit that has the most
-// blocks: 27 ns a k of a block (64 cycles of its SIMDs' matrix cores) and some 1.5 us a block, a third more with one block to a compute unit (nothing
-// fills its waits), and for the second launch 4 us and 16 bytes a sum at 4 TB/s. Returns k a share (a multiple of a slab). Up to 16 rows and in the
+// blocks: 35.5 ns a k of a block (30 of them its SIMDs' matrix cores) and some 0.5 us a block, a twentieth more with one block to a compute unit, and
+// for the second launch 4 us and 0.7 us a million sums. Measured / by that count, us, 896 x 4,864: 450 rows in 4 shares 91.5 / 92.5, in 9 83.6 / 85.8; 200 rows in 4
+// 52.3 / 50.4, in 9 46.5 / 44.7, in 16 54.4 / 53; 768 rows in 2 173.7 / 179, in 3 121.1 / 122. Returns k a share (a multiple of a slab). Up to 16 rows and in the
 // gated form K is not shared out. Up to 16 rows: shares of 1,024 k and more for one block to a compute unit, where the
 // blocks of 16 weight rows are fewer than half the compute units and K is long (896 x 4,864, 8 rows: 19.0 us in 56 blocks of 16 waves).
 static int exact_share(int M, int N, int K) {
@@ -261,7 +313,7 @@ static int exact_share(int M, int N, int K) {
   for (int shares = 1; shares <= 16 && (shares == 1 || K / shares >= 128); ++shares) {
     const int k = ((K + shares - 1) / shares + 31) / 32 * 32, got = (K + k - 1) / k;
     const int64_t rounds = (tiles * got + cus - 1) / cus;
-    const double us = rounds * (0.027 * k + 1.5) * (rounds == 1 ? 1.33 : 1.0) + (got > 1 ? 4.0 + 4e-6 * got * M * N : 0.0);
+    const double us = rounds * (0.0355 * k + 0.5) * (rounds == 1 ? 1.05 : 1.0) + (got > 1 ? 4.0 + 0.7e-6 * got * M * N : 0.0);
     if (us < least) least = us, best = got > 1 ? k : K;
   }
   return best;

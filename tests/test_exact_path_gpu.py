@@ -81,3 +81,15 @@ def test_exact_attention(heads, kv_heads, d, bs, requests, window):
     ops().paged_attention(out, torch.cat(rows).to(DEV), kc.to(DEV), vc.to(DEV), table.to(DEV), to(req), to(pos), heads, kv_heads, d, window, float(np.float32(d ** -0.5)), True)
     # a weight: its score's rounding (some units of 2^-23 at scores of up to six), expf's two units; the values are of order one
     within(out, torch.stack(want).numpy(), 12.0)
+
+
+# slabs of 32 k: none whole, one to seven, with and without a rest, rows that are not 16-byte aligned, shares of unequal length
+@pytest.mark.parametrize("M,N,K,shift", [(17, 40, 20, 0), (33, 70, 32, 0), (33, 70, 52, 0), (65, 70, 64, 0), (20, 140, 96, 0), (65, 70, 99, 0), (40, 64, 128, 0), (64, 64, 160, 1), (90, 70, 190, 1),
+                                         (40, 70, 228, 0), (200, 64, 1100, 0)])
+def test_exact_products_by_slabs(M, N, K, shift):
+    rng = np.random.default_rng(K)
+    a, w = (rng.standard_normal(s).astype(np.float32) for s in ((M, K + shift), (N, K + shift)))
+    want = a[:, shift:].astype(np.float64) @ w[:, shift:].astype(np.float64).T
+    out = torch.empty(M, N, device=DEV)
+    ops().gemm(out, t(a)[:, shift:], t(w)[:, shift:], exact=True)
+    within(out, want, np.abs(want) + 1e-7)
