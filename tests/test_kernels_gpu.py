@@ -719,6 +719,22 @@ def close_at_own_scale(got, ref, what):
     assert np.isfinite(got).all() and err <= 1.5e-2 * scale, f"{what}: {err:.3e} > 1.5e-2 x {scale:.3e}"
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kv_heads,d,block_heads", [(16, 1, 128, 16), (9, 1, 128, 16), (28, 4, 128, None), (16, 1, 128, 5), (11, 1, 96, None), (7, 1, 256, 16), (3, 1, 112, None)])
+def test_parts_that_the_last_block_combines(heads, kv_heads, d, block_heads):
+    """Wide heads, whose outputs are several a thread: one to sixteen heads a block (one pass over the outputs or two, the last one ragged), two to eight parts
+    whose reads set out together, and more, which are read in turn."""
+    rng = np.random.default_rng(heads * d)
+    c = paged_case(rng, [600, 37, 1], [1, 2, 1], heads, kv_heads, d, 16, torch.bfloat16)
+    ref = np.concatenate([pm.attention(c["q"][r], c["k"][r], c["v"][r], heads, kv_heads, d, None) for r in range(3)])
+    o = ops()
+    for parts in (2, 3, 4, 5, 8, 9):
+        out = torch.zeros(4, heads * d, device=DEV, dtype=torch.bfloat16)
+        o.attention_decode(out, c["qcat"], c["kc"], c["vc"], c["table"], c["req"], c["pos"], heads, kv_heads, d, None, float(np.float32(1) / np.sqrt(np.float32(d))), 600,
+                           None, n_splits=parts, hand_over=True, block_heads=block_heads)
+        close(out, ref, BF16, f"{parts} parts combined by the last block")
+
+
 @pytest.mark.parametrize("batch", [1, 8])
 @pytest.mark.parametrize("context", [8192, 16384, 32768])
 @pytest.mark.parametrize("heads,kv_heads,d", [(14, 2, 64), (28, 4, 128)])
