@@ -9,8 +9,8 @@
 // piece as it is). Nothing passes through registers, one barrier a tile. What is left is the softmax on the vector unit (some 1,000
 // cycles a wave and tile) beside 1,024 cycles of products; the two waves of a SIMD fill one another's gaps.
 //
-// 40/8 heads, 2 x 2,048 rows on 6,144 and 10,240 keys 1,310 -> 725 us (1.07 PFLOP/s); 28/4 heads, 2,048 rows on 8,192 keys 550 -> 268. Measured
-// and not kept: the two waves of a SIMD half a tile apart by barriers, one with the products while the other has the weights (788 and 301 us: their
+// 40/8 heads, 2 x 2,048 rows on 6,144 and 10,240 keys 1,315 -> 766 us (1.01 PFLOP/s); 28/4 heads, 2,048 rows on 8,192 keys 538 -> 282. Measured
+// and not kept (beside 725 and 268 us, with one state a row): the two waves of a SIMD half a tile apart by barriers, one with the products while the other has the weights (788 and 301 us: their
 // slots come out unequal, and the slower of eight waves ends each); the fetches behind the first product (774 and 285); a higher wave priority for the
 // products (no difference); head size 64, 256 or 128 rows (14/2 heads, 8,192 rows 241 and 292 us against 212: half the products for the same softmax).
 //
@@ -18,9 +18,12 @@
 // l % 32 and rows 8 j + 4 (l / 32) + r): S^T = K Q^T, O^T += V^T P^T. Row i = 16 y + 8 jj + 4 h + r of a 32-key half is key 16 y + 8 h + 4 jj + r, so that the
 // weights a lane holds for one instruction of the second product are eight consecutive keys: its values are one 16-byte read.
 //
-// Scores, maximum, weights and their sum are float, the weights are rounded to bfloat16 as operands only. A row's maximum is followed only where
-// a tile passes it by more than 2^8 (weights up to 256 keep the same relative precision, in float and in bfloat16; the sums hold them), so that
-// most tiles leave the outputs alone.
+// Scores, maximum, weights and their sum are float, the weights are rounded to bfloat16 as operands only. A row's maximum is followed in every tile
+// that raises it, so that the weight that counts most is one, which no rounding touches; a tile that raises no row's maximum leaves the outputs alone. A row has
+// two running states, of the even and of the odd tiles, which meet at the end: the highest weight of either is exact, as it is with the two teams of the blocks of
+// 64 rows, and the results are as far from 64 bits as theirs (40/8 heads, 1,024 rows on 3,072 keys, scores times 1, 2, 4 and 8: 0.002246, 0.001869,
+// 0.001708 and 0.001655 here and there; with one state 0.002270, 0.001916, 0.001736 and 0.001672; with one state that follows the maximum only where a tile passes it by
+// more than 2^8 0.002342, 0.002306, 0.002142 and 0.001976). The times of the three: 766, 759 and 722 us, 282, 276 and 265.
 //
 // Blocks of one key head go to one die where there are eight of them (the dies take blocks in turn): its keys and values then stay in that
 // die's L2 for all the rows and heads that read them.
@@ -107,19 +110,21 @@ __global__ void __launch_bounds__(512) attention_tall_kernel(bf16_t* __restrict_
     const bf16_t* vb = v_cache + ((static_cast<int64_t>(page) * kv_heads + hk) * d << bs_shift) + slot;
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                   :: "s"(__builtin_amdgcn_readfirstlane(k_to[j] + stage)), "v"(kb + k_off[j]), "r"(ring) : "memory", "m0");
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                   :: "s"(__builtin_amdgcn_readfirstlane(v_to[j] + stage)), "v"(vb + v_off[j]), "r"(ring) : "memory", "m0");
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                   :: "s"(__builtin_amdgcn_readfirstlane(k_to[j] + stage)), "v"(2u * k_off[j]), "s"(kb), "r"(ring) : "memory", "m0");
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                   :: "s"(__builtin_amdgcn_readfirstlane(v_to[j] + stage)), "v"(2u * v_off[j]), "s"(vb), "r"(ring) : "memory", "m0");
     }
   };
 
-  f32x16 o[OT];
+  f32x16 o[2][OT];      // of the even tiles and of the odd ones, counted from the block's first
 #pragma unroll
-  for (int nt = 0; nt < OT; ++nt)
+  for (int x = 0; x < 2; ++x)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) o[nt][e] = 0.f;
-  float m = -FLT_MAX, l = 0.f;
+    for (int nt = 0; nt < OT; ++nt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[x][nt][e] = 0.f;
+  float m[2] = {-FLT_MAX, -FLT_MAX}, l[2] = {0.f, 0.f};
   const float scale2 = scale * 1.44269504088896340736f;   // scores in units of log2(e)
 
   // fragments: keys row 32 kh + (r32's key), chunk 2 ds + h; values channel 32 nt + r32, keys 16 x + 8 h ..
@@ -129,7 +134,7 @@ __global__ void __launch_bounds__(512) attention_tall_kernel(bf16_t* __restrict_
   bf16x8 pf[4];
   // n products with a read from LDS each: kAhead reads set out before the first product, then one with every product
   auto reads_ahead = [](auto n) __attribute__((always_inline)) {
-    constexpr int kAhead = 6;
+    constexpr int kAhead = 4;
     __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
 #pragma unroll
     for (int i = 0; i < n.value - kAhead; ++i) {
@@ -138,13 +143,14 @@ __global__ void __launch_bounds__(512) attention_tall_kernel(bf16_t* __restrict_
     }
     __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
   };
-  auto take_values = [&](const char* st) __attribute__((always_inline)) {
+  auto take_values = [&](const char* st, auto which) __attribute__((always_inline)) {
+    constexpr int w = decltype(which)::value;
 #pragma unroll
     for (int x = 0; x < 4; ++x)
 #pragma unroll
       for (int nt = 0; nt < OT; ++nt) {
         const uint4 vv = *reinterpret_cast<const uint4*>(st + kKeyBytes + ((x * d + nt * 32 + r32) * 2 + h) * 16);
-        o[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vv), pf[x], o[nt], 0, 0, 0);
+        o[w][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vv), pf[x], o[w][nt], 0, 0, 0);
       }
     reads_ahead(std::integral_constant<int, 4 * OT>{});
   };
@@ -162,7 +168,8 @@ __global__ void __launch_bounds__(512) attention_tall_kernel(bf16_t* __restrict_
       }
     reads_ahead(std::integral_constant<int, 2 * DT>{});
   };
-  auto take_weights = [&](int t, bool whole) __attribute__((always_inline)) {
+  auto take_weights = [&](int t, bool whole, auto which) __attribute__((always_inline)) {
+    constexpr int w = decltype(which)::value;
     if (!whole) {      // (uniform) what a row does not see: minus infinity, whose weight is zero against any maximum
 #pragma unroll
       for (int i = 0; i < 32; ++i) {
@@ -175,12 +182,12 @@ __global__ void __launch_bounds__(512) attention_tall_kernel(bf16_t* __restrict_
 #pragma unroll
     for (int i = 1; i < 32; ++i) top = fmaxf(top, s[i / 16][i % 16]);
     top = two_halves_max(top) * scale2;
-    if (__any(top > m + 8.f)) {
-      const float m_new = fmaxf(m, top), corr = __builtin_amdgcn_exp2f(m - m_new);      // (1 while a row has seen nothing yet: m stays -FLT_MAX)
-      m = m_new;
-      l *= corr;
+    if (__any(top > m[w])) {
+      const float m_new = fmaxf(m[w], top), corr = __builtin_amdgcn_exp2f(m[w] - m_new);      // (1 where a row's maximum stays, and while it has seen nothing yet: m is -FLT_MAX)
+      m[w] = m_new;
+      l[w] *= corr;
 #pragma unroll
-      for (int nt = 0; nt < OT; ++nt) o[nt] *= corr;
+      for (int nt = 0; nt < OT; ++nt) o[w][nt] *= corr;
     }
     float sum = 0.f;
 #pragma unroll
@@ -188,12 +195,12 @@ __global__ void __launch_bounds__(512) attention_tall_kernel(bf16_t* __restrict_
       float p[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[x / 2][x % 2 * 8 + i], scale2, -m));
+        p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[x / 2][x % 2 * 8 + i], scale2, -m[w]));
         sum += p[i];
       }
       pf[x] = __builtin_bit_cast(bf16x8, make_uint4(pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]), pack_bf16x2(p[6], p[7])));
     }
-    l += sum;
+    l[w] += sum;
   };
   // Values beyond the block's visible keys (in its first and last tiles) are not data: cleared, so that a weight of zero times them is zero.
   auto clear = [&](int t, char* st) {
@@ -215,7 +222,7 @@ __global__ void __launch_bounds__(512) attention_tall_kernel(bf16_t* __restrict_
   for (int p = 0; p < S - 1; ++p)
     if (t_begin + p <= t_end) fetch(t_begin + p, page_of(t_begin + p), p * kStage);
   unsigned stage = 0;
-  for (int t = t_begin; t <= t_end; ++t) {
+  auto step = [&](int t, auto which) __attribute__((always_inline)) {
     if (t + S - 2 <= t_end) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * kLoads * (S - 2)) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
@@ -232,21 +239,28 @@ __global__ void __launch_bounds__(512) attention_tall_kernel(bf16_t* __restrict_
       __syncthreads();
     }
     // (uniform over the wave) a tile of which no row of the wave sees a key; one that every row sees whole
-    if (t * KT > last_row_pos || (window > 0 && t * KT + KT - 1 <= first_row_pos - window)) continue;
+    if (t * KT > last_row_pos || (window > 0 && t * KT + KT - 1 <= first_row_pos - window)) return;
     take_keys(st);
-    take_weights(t, t * KT + KT - 1 <= first_row_pos && (window <= 0 || t * KT > last_row_pos - window));
-    take_values(st);
+    take_weights(t, t * KT + KT - 1 <= first_row_pos && (window <= 0 || t * KT > last_row_pos - window), which);
+    take_values(st, which);
+  };
+  for (int t = t_begin; t <= t_end; t += 2) {
+    step(t, std::integral_constant<int, 0>{});
+    if (t + 1 <= t_end) step(t + 1, std::integral_constant<int, 1>{});
   }
-  l = two_halves_sum(l);
+  const float most = fmaxf(m[0], m[1]), even = __builtin_amdgcn_exp2f(m[0] - most), odd = __builtin_amdgcn_exp2f(m[1] - most);
+  const float all = two_halves_sum(l[0] * even + l[1] * odd);
+#pragma unroll
+  for (int nt = 0; nt < OT; ++nt) o[0][nt] = o[0][nt] * even + o[1][nt] * odd;
   if (row_ok) {
-    const float inv = 1.f / l;
+    const float inv = 1.f / all;
     bf16_t* dst = out + static_cast<int64_t>(row0 + my_row) * out_stride + static_cast<int64_t>(head) * d;
 #pragma unroll
     for (int nt = 0; nt < OT; ++nt)
 #pragma unroll
       for (int j = 0; j < 4; ++j)      // four consecutive channels
         *reinterpret_cast<uint2*>(dst + nt * 32 + 8 * j + 4 * h) =
-            make_uint2(pack_bf16x2(o[nt][4 * j] * inv, o[nt][4 * j + 1] * inv), pack_bf16x2(o[nt][4 * j + 2] * inv, o[nt][4 * j + 3] * inv));
+            make_uint2(pack_bf16x2(o[0][nt][4 * j] * inv, o[0][nt][4 * j + 1] * inv), pack_bf16x2(o[0][nt][4 * j + 2] * inv, o[0][nt][4 * j + 3] * inv));
   }
 }
 

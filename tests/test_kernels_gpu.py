@@ -1259,3 +1259,31 @@ def test_attention_of_many_rows(heads, kv_heads, bs, window):
     again = torch.zeros_like(out)
     ops().attention_tall(again, q, kc, vc, table.to(DEV), runs, heads, kv_heads, d, window, scale)
     assert torch.equal(again, out)
+
+
+# sharper and sharper softmaxes: where one key counts, its weight is one exactly, and only the others' are rounded
+@pytest.mark.parametrize("heads,kv_heads,n,history", [(8, 2, 700, 900), (6, 6, 512, 0), (16, 2, 300, 3000)])
+@pytest.mark.parametrize("sharp", [1, 2, 4, 8, 16])
+def test_attention_of_many_rows_is_as_exact_as_the_kernel_for_all_sizes(heads, kv_heads, n, history, sharp):
+    d, bs, L = 128, 16, n + history
+    gen = torch.Generator(device=DEV).manual_seed(sharp + n)
+    pages = -(-L // bs)
+    q = (torch.randn(n, heads * d, generator=gen, device=DEV) * sharp).bfloat16()
+    kc, vc = torch.randn(pages, kv_heads, bs, d, generator=gen, device=DEV).bfloat16(), torch.randn(pages, kv_heads, d, bs, generator=gen, device=DEV).bfloat16()
+    table = torch.arange(pages, dtype=torch.int32, device=DEV)[None].contiguous()
+    common = (heads, kv_heads, d, None, d ** -0.5)
+    few, many = (torch.zeros(n, heads * d, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    runs = [(0, o, min(64, n - o), history + o) for o in range(0, n, 64)]
+    ops().attention_prefill(few, q, kc, vc, table, torch.tensor(ops().pair_tiles(runs), dtype=torch.int32, device=DEV), *common)
+    runs = [(0, o, min(ops().TALL_ROWS, n - o), history + o) for o in reversed(range(0, n, ops().TALL_ROWS))]
+    ops().attention_tall(many, q, kc, vc, table, torch.tensor(runs, dtype=torch.int32, device=DEV), *common)
+    k, v = kc.permute(1, 0, 2, 3).reshape(kv_heads, -1, d)[:, :L].double(), vc.permute(1, 0, 3, 2).reshape(kv_heads, -1, d)[:, :L].double()
+    hidden = torch.arange(L, device=DEV)[None] > history + torch.arange(n, device=DEV)[:, None]
+    far = [0.0, 0.0]
+    for h in range(heads):
+        s = (q[:, h * d:(h + 1) * d].double() @ k[h * kv_heads // heads].T.contiguous()) * d ** -0.5
+        want = torch.softmax(s.masked_fill_(hidden, float("-inf")), -1) @ v[h * kv_heads // heads]
+        for i, got in enumerate((few, many)):
+            far[i] += ((got[:, h * d:(h + 1) * d].double() - want) ** 2).sum().item()
+    # both follow the maxima of the even and of the odd tiles and round the same weights and results; what differs is the order of float sums
+    assert far[1] <= 1.005 ** 2 * far[0], (far[0] ** 0.5, far[1] ** 0.5)
