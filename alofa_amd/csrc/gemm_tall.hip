@@ -228,12 +228,22 @@ static int pick_tall(int M, int N, int K, bool gated, double* fill) {
 //   ahead: 5,120 x 5,120 against 512 (160) 67 / 56, 5,120 x 13,824 against 512 170 / 130, 3,584 x 3,584 against 1,024 (224) 53 / 41, against 2,000 70 / 60, 5,120 x 27,648 against 4,096 1,299 / 891,
 //   5,120 x 5,120 260 / 184, 4,608 x 3,584 against 2,000 100 / 72, 2,560 x 2,048 against 1,536 (240) 35 / 25; with the gate: 18,944 x 3,584 against 65 (148 of 128 x 128) 79 / 62, against 2,048
 //   523 / 463, 27,648 x 5,120 against 2,048 1,090 / 920, 8,960 x 1,536 against 300 (210) 35 / 29, 13,824 x 5,120 against 2,048 573 / 493.
+// Small matrices (under 20 M elements, 40 MB) whose K is not long stay with the other forms until their tiles fill seven and a half tenths: 180 tiles of 128 x 128, 1,280 x 2,048 against 2,262 rows
+// 24.5 / 26.3, 2,304 x 4,864 against 1,191 47.0 / 49.6, 2,560 x 4,096 against 1,090 40.6 / 43.3; 154 and 162 tiles, 896 x 8,192 against 2,706 73.3 / 76.4, 2,304 x 8,192 against 1,053 73.1 / 76.5; 189 and 192,
+// 896 x 2,560 against 3,432 44.3 / 31.2, 2,048 x 3,072 against 1,465 47.4 / 35.4.
+// Where tiles of 128 x 128 are more than one round of the chip, the others' K is not shared out and their second round is nearly empty, while 128 x 192 still come out in one: 11,008 x 4,096 against
+// 315 rows (174 tiles of 128 x 192) 82 / 56, 11,008 x 2,048 against 303 47 / 34, 4,224 x 3,584 against 957 (176) 64 / 47, 3,072 x 4,864 against 1,323 78 / 60, 3,072 x 2,560 against 1,385 51 / 38.
 bool tall_pays(int M, int N, int K, bool gated) {
   static const bool switched_off = [] { const char* e = getenv("ALOFA_WIDE_TILES"); return e != nullptr && e[0] == '0'; }();     // (for measurements)
   if (switched_off || M <= 64 || K % 32 != 0 || K < 1536) return false;
   double fill = 0;
   pick_tall(M, N, K, gated, &fill);
-  return fill >= (K < 2048 ? 0.80 : K < 3072 || (K < 5120 && !gated) ? 0.70 : 0.57);
+  if (K < 2048) return fill >= 0.80;
+  if (!gated) {
+    if (static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128) > compute_units()) return true;
+    if (K < 8960 && static_cast<int64_t>(N) * K < 20000000) return fill >= 0.735;
+  }
+  return fill >= (K < 3072 || (K < 5120 && !gated) ? 0.70 : 0.57);
 }
 
 template <int kEpilogue, typename TO, typename T>
@@ -284,6 +294,9 @@ extern "C" int alofa_gemm_wide_form(int M, int N, int K, int gated) {
   double fill = 0;
   return pick_tall(M, N, K, gated != 0, &fill);
 }
+
+// Whether alofa_gemm_mfma takes these tiles.
+extern "C" int alofa_gemm_wide_pays(int M, int N, int K, int gated) { return tall_pays(M, N, K, gated != 0); }
 
 // The same product by these tiles whatever the sizes (alofa_gemm_mfma takes them where they pay): K a multiple of 32. The operands as for
 // alofa_gemm_mfma; norm_w and eps stand where alofa_gemm_skinny has them and must be null and zero (no norm rides on this kernel).

@@ -1221,6 +1221,17 @@ def test_forms_of_the_product_for_many_rows(M, N, K, form):
         assert (gated[:, :n].float() - ref).abs().max().item() <= (2.0 ** -8 + 1e-5) * ref.abs().max().item() and bool((gated[:, n:] == 3.0).all())
 
 
+# which forms take a product (256 compute units): a little more than one round of tiles of 128 x 128; small matrices on either side of their line; few tiles of a long K; a short K; the gate
+@pytest.mark.parametrize("M,N,K,gated,taken", [(315, 11008, 4096, 0, 1), (303, 11008, 2048, 0, 1), (957, 4224, 3584, 0, 1), (1385, 3072, 2560, 0, 1), (2262, 1280, 2048, 0, 0), (1170, 2304, 8192, 0, 0),
+                                               (2706, 896, 8192, 0, 0), (3432, 896, 2560, 0, 1), (439, 5120, 5120, 0, 1), (512, 3584, 18944, 0, 0), (2674, 896, 18944, 0, 1), (900, 4224, 1600, 0, 0),
+                                               (64, 11008, 4096, 0, 0), (2048, 18944, 3584, 1, 1), (256, 8960, 1536, 1, 0)])
+def test_which_products_the_forms_for_many_rows_take(M, N, K, gated, taken):
+    from alofa_amd.csrc.build import load
+    if ops().compute_units() != 256:
+        pytest.skip("the sizes are those of 256 compute units")
+    assert load().alofa_gemm_wide_pays(M, N, K, gated) == taken
+
+
 # runs that end within a tile, within a wave's rows and at either's edge; one row; history in whole and ragged tiles; windows shorter than a tile, than a block and longer; larger pages
 @pytest.mark.parametrize("heads,kv_heads,bs,window", [(5, 1, 16, None), (4, 2, 16, 40), (16, 8, 64, 300), (3, 3, 32, None), (2, 1, 16, 1)])
 def test_attention_of_many_rows(heads, kv_heads, bs, window):
