@@ -31,6 +31,7 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kExactStore = 0, kExactResidual = 1;
 constexpr int kExactRows = 16;       // rows that exact_rows_kernel takes at most
+constexpr int kMaxShares = 16;       // shares of K that exact_sum_kernel adds at most
 
 // four consecutive k of a row from `k` on, all of them within the row: one 16-byte load, or, where rows are not 16-byte aligned, value by value
 template <bool kVec>
@@ -285,11 +286,11 @@ __global__ void __launch_bounds__(256) exact_sum_kernel(float* __restrict__ out,
   if (i >= all) return;
   const int n = i % N;
   double s = bias ? static_cast<double>(bias[n]) : 0.0;
-  double p[16];
+  double p[kMaxShares];
 #pragma unroll
-  for (int x = 0; x < 16; ++x) p[x] = x < shares ? parts[x * all + i] : 0.0;
+  for (int x = 0; x < kMaxShares; ++x) p[x] = x < shares ? parts[x * all + i] : 0.0;
 #pragma unroll
-  for (int x = 0; x < 16; ++x) s += p[x];
+  for (int x = 0; x < kMaxShares; ++x) s += p[x];
   put<kEpilogue>(out + i / N * ldo + n, s);
 }
 
@@ -303,14 +304,14 @@ static int exact_share(int M, int N, int K) {
   if (M <= kExactRows) {
     const int blocks = (N + 15) / 16, cus = compute_units();
     if (blocks * 2 >= cus || K < 2048) return K;
-    const int shares = cus / blocks < K / 1024 ? cus / blocks : K / 1024;
+    const int room = cus / blocks < kMaxShares ? cus / blocks : kMaxShares, shares = room < K / 1024 ? room : K / 1024;
     return ((K + shares - 1) / shares + 31) / 32 * 32;
   }
   const int BM = M <= 32 ? 32 : 64, BW = M <= 32 ? 128 : 64, cus = compute_units();
   const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BW - 1) / BW);
   int best = K;
   double least = 1e30;
-  for (int shares = 1; shares <= 16 && (shares == 1 || K / shares >= 128); ++shares) {
+  for (int shares = 1; shares <= kMaxShares && (shares == 1 || K / shares >= 128); ++shares) {
     const int k = ((K + shares - 1) / shares + 31) / 32 * 32, got = (K + k - 1) / k;
     const int64_t rounds = (tiles * got + cus - 1) / cus;
     const double us = rounds * (0.0355 * k + 0.5) * (rounds == 1 ? 1.05 : 1.0) + (got > 1 ? 4.0 + 0.7e-6 * got * M * N : 0.0);
@@ -385,6 +386,7 @@ extern "C" int alofa_gemm_exact(float* out, int64_t ldo, const float* A, int64_t
   ALOFA_REQUIRE(epilogue == kExactStore || epilogue == kExactResidual, "gemm: unknown epilogue %d", epilogue);
   ALOFA_REQUIRE(lda >= K && ldw >= K && ldo >= N, "gemm: a leading dimension is shorter than its row");
   ALOFA_REQUIRE(room >= alofa_gemm_exact_parts(M, N, K), "gemm: no room for the sums of the shares of K");
+  ALOFA_REQUIRE(alofa_gemm_exact_parts(M, N, K) <= static_cast<int64_t>(kMaxShares) * M * N, "gemm: more shares of K than are added up");
   if (epilogue == kExactStore) return launch_exact<1, kExactStore>(out, ldo, A, lda, W, W, ldw, bias, parts, M, N, K, 0, stream);
   return launch_exact<1, kExactResidual>(out, ldo, A, lda, W, W, ldw, bias, parts, M, N, K, 0, stream);
 }

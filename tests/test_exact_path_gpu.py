@@ -93,3 +93,17 @@ def test_exact_products_by_slabs(M, N, K, shift):
     out = torch.empty(M, N, device=DEV)
     ops().gemm(out, t(a)[:, shift:], t(w)[:, shift:], exact=True)
     within(out, want, np.abs(want) + 1e-7)
+
+
+# up to 16 rows against few columns and K so long that a share of 1,024 k a block would make more shares than are added up
+@pytest.mark.parametrize("M,N,K", [(8, 64, 18944), (1, 128, 27648), (16, 16, 32768), (3, 240, 17408), (16, 31, 17500)])
+def test_exact_products_of_few_rows_and_very_long_k(M, N, K):
+    gen = torch.Generator(device=DEV).manual_seed(K + N)
+    a, w, b, res = (torch.randn(s, generator=gen, device=DEV) for s in ((M, K), (N, K), (N,), (M, N)))
+    want = (a.double() @ w.double().T.contiguous()).cpu().numpy()
+    out = torch.empty(M, N, device=DEV)
+    ops().gemm(out, a, w, b, exact=True)
+    within(out, want + b.cpu().numpy(), np.abs(want + b.cpu().numpy()) + 1e-7)
+    acc = res.clone()
+    ops().gemm(acc, a, w, add_to_out=True, exact=True)
+    within(acc, want + res.cpu().numpy(), np.abs(want) + np.abs(want + res.cpu().numpy()) + 1e-7)
