@@ -5,24 +5,28 @@
 // Which four k an instruction takes is free as long as both operands agree, so a lane takes four consecutive k (one 16-byte
 // load) for four instructions in a row.
 //
-// An output is the sum over k in a few float64 partial sums (waves, parts of K), added in a fixed order that depends on the sizes
-// only: two orders differ by some 2^-50 of the sum, which the one rounding to float hides but for one output in some ten million.
+// An output is bias + c0 + c1 + ...: K is cut into chains of 128 values and more, sixteen at most, by K alone; a chain's products are summed in ascending k, four by
+// an instruction, and the chains' float64 sums are added in their order. Every form below does so, whichever wave or block has a chain: a row's
+// result is the same bits whatever rows are computed with it.
 //
-//   up to 16 rows (exact_rows_kernel): a block owns 16 weight rows (16 of gate and 16 of up), its waves take runs of 32 k in turn,
+//   up to 16 rows (exact_rows_kernel): a block owns 16 weight rows (16 of gate and 16 of up), its waves take a chain each, in runs of 32 k
 //   straight from memory, and meet in LDS. Bound by the rate at which a compute unit takes its weights in and, within it, by the matrix
-//   cores (64 cycles an instruction, 64 weights), so K is shared out over blocks where blocks are few. 8 rows, us, a tile of 64 x 64
-//   on the vector units (one block per 64 columns) / this: 9,728 x 896 with the gate 270 / 14.6, 896 x 4,864 920 / 7.8 and 4.5 for the second
-//   launch, 896 x 896 168 / 6.8, 1,152 x 896 170 / 7.3, 151,936 x 896 658 / 113.
+//   cores (64 cycles an instruction, 64 weights), so the chains are dealt out over blocks where blocks are few. 8 rows, us, a tile of 64 x 64
+//   on the vector units (one block per 64 columns) / this: 9,728 x 896 with the gate 270 / 14.9, 896 x 4,864 920 / 10.2 with the second
+//   launch, 896 x 896 168 / 6.5, 1,152 x 896 170 / 6.5, 151,936 x 896 658 / 113.
 //
 //   more rows (exact_tile_kernel): slabs of 32 k through LDS, a wave owns 32 rows x 32 weight rows (four instructions for two
 //   loads of either operand), a block 64 x 64 (32 x 128 up to 32 rows). Bound by the matrix cores (69 TFLOP/s measured with
 //   nothing else in the loop; 58 reached, 50 of them useful at 450 rows, whose last tile is padding) and by the widening, which the same SIMD does between the
 //   products. Two slabs are on their way in registers and two lie in LDS: with one of either, a slab that came late (1.4 us from a busy memory against 0.9 us of
-//   products) held up the block, 9,728 x 896 with the gate 167, 896 x 4,864 102 + 5. K is shared out over blocks where the tiles are few; the shares' float64 sums
-//   go to a buffer of the caller's (not to the library's workspace, which one stream at a time may use) and a second launch adds them. 450 rows, us, as above:
-//   9,728 x 896 with the gate 377 / 154, 896 x 4,864 1,000 / 84 both launches, 896 x 896 185 / 26, 1,152 x 896 185 / 31.
+//   products) held up the block, 9,728 x 896 with the gate 167, 896 x 4,864 102 + 5. The chains are dealt out over blocks where the tiles are few; their float64 sums
+//   go to a buffer of the caller's (not to the library's workspace, which one stream at a time may use) and a second launch adds them. Else a block adds them up in
+//   registers, two blocks to a compute unit where three fit without. 450 rows, us, as above: 9,728 x 896 with the gate 377 / 154, 896 x 4,864 1,000 / 89 both launches,
+//   896 x 896 185 / 30, 1,152 x 896 185 / 31. (With shares of K by the number of rows 84, 26 and 31: then a row's sums depend on the others. A block that takes several chains
+//   of few, each to its own place: 89, 31, 31.)
 #include "common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace alofa {
@@ -31,7 +35,8 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kExactStore = 0, kExactResidual = 1;
 constexpr int kExactRows = 16;       // rows that exact_rows_kernel takes at most
-constexpr int kMaxShares = 16;       // shares of K that exact_sum_kernel adds at most
+constexpr int kMaxChains = 16;       // chains that K is cut into at most, and exact_sum_kernel adds
+constexpr int64_t kMostBytes = int64_t{64} << 20;      // of the chains' sums in memory
 
 // four consecutive k of a row from `k` on, all of them within the row: one 16-byte load, or, where rows are not 16-byte aligned, value by value
 template <bool kVec>
@@ -64,108 +69,140 @@ __device__ __forceinline__ float gated(double g, double u, int gelu) {
   return static_cast<float>(gate_of(static_cast<double>(static_cast<float>(g)), gelu != 0) * static_cast<double>(static_cast<float>(u)));
 }
 
-// NW waves; kMats = 2: gate and up. NT tiles of 16 weight rows a block (of each matrix).
+// How K is cut into chains (see the head of this file): `count` of them, `length` values each, the last one what is left. By K alone.
+struct Cut {
+  int length, count;
+};
+static Cut cut_of(int K) {
+  const int length = std::max(128, ((K + kMaxChains - 1) / kMaxChains + 63) / 64 * 64);
+  return {length, (K + length - 1) / length};
+}
+
+// NW waves; kMats = 2: gate and up. NT tiles of 16 weight rows a block (of each matrix). blockIdx.y: which `per` chains; parts, where those are not all: the chains' sums, [chain][M][N].
 template <int NW, int NT, int kMats, int kEpilogue, bool kVec>
 __global__ void __launch_bounds__(64 * NW) exact_rows_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ A, int64_t lda,
                                                              const float* __restrict__ W, const float* __restrict__ W2, int64_t ldw,
-                                                             const float* __restrict__ bias, double* __restrict__ parts, int k_share, int M, int N, int K, int gelu) {
-  constexpr int kTiles = NT * kMats;
+                                                             const float* __restrict__ bias, double* __restrict__ parts, Cut cut, int per, int M, int N, int K, int gelu) {
+  constexpr int kTiles = NT * kMats, kOut = (NT * 256 + 64 * NW - 1) / (64 * NW);
   __shared__ double sums[NW][kTiles][4][64];
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
   const int n0 = blockIdx.x * 16 * NT;
-  const int k_first = blockIdx.y * k_share;      // (shares of K: blockIdx.y, their sums in `parts` as [share][M][N])
-  K = K - k_first < k_share ? K - k_first : k_share;
   const bool row_ok = r < M;
-  const float* a_row = A + static_cast<int64_t>(row_ok ? r : 0) * lda + k_first;
+  const float* a_row = A + static_cast<int64_t>(row_ok ? r : 0) * lda;
   const float* w_row[kTiles];
 #pragma unroll
   for (int t = 0; t < kTiles; ++t) {
     const int n = n0 + (t / kMats) * 16 + r;
-    w_row[t] = (t % kMats ? W2 : W) + static_cast<int64_t>(n < N ? n : N - 1) * ldw + k_first;      // (rows beyond N: the last one again, not stored)
+    w_row[t] = (t % kMats ? W2 : W) + static_cast<int64_t>(n < N ? n : N - 1) * ldw;      // (rows beyond N: the last one again, not stored)
   }
-  f64x4 acc[kTiles];
-#pragma unroll
-  for (int t = 0; t < kTiles; ++t) acc[t] = f64x4{0, 0, 0, 0};
-  // Runs of 32 k: a lane takes 4 g .. 4 g + 3 of either half (an instruction's lanes fetch 64 bytes of a row side by side). kSets runs are on their
-  // way or in work; each set of registers is filled again as soon as its run is multiplied, without a branch around the loads (a run past
-  // the last is the last one again), so that the compiler waits for the oldest only.
-  constexpr int kSets = kTiles == 1 ? 4 : kTiles == 2 ? 3 : 2;
-  const int runs = K / 32, mine = (runs - wave + NW - 1) / NW;      // whole runs, and those of this wave: wave, wave + NW, ...
-  float4 a[kSets][2], w[kSets][kTiles][2];
-  auto fetch = [&](int s, int i) __attribute__((always_inline)) {
-    const int k = (wave + (i < mine ? i : mine - 1) * NW) * 32 + g * 4;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      a[s][h] = quad<kVec>(a_row, k + 16 * h);
-#pragma unroll
-      for (int t = 0; t < kTiles; ++t) w[s][t][h] = quad<kVec>(w_row[t], k + 16 * h);
-    }
+  // what this thread adds up: output o is place i = threadIdx.x + 64 NW o: tile, weight row 4 v + g', row of A j: (v, 16 g' + j)
+  auto place = [&](int o, int& tile, int& v, int& at, int& m, int& n) __attribute__((always_inline)) {
+    const int i = threadIdx.x + 64 * NW * o;
+    tile = i / 256, v = i / 64 % 4, at = i % 64, m = at % 16, n = n0 + tile * 16 + 4 * v + at / 16;
+    return i < NT * 256 && m < M && n < N;
   };
-  auto multiply = [&](int s) __attribute__((always_inline)) {
+  double total[kOut][kMats];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      if (!row_ok) a[s][h] = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int o = 0; o < kOut; ++o) {
+    int tile, v, at, m, n;
+    const bool ok = place(o, tile, v, at, m, n);
 #pragma unroll
-      for (int t = 0; t < kTiles; ++t) acc[t] = fma_quad(w[s][t][h], a[s][h], acc[t]);
-    }
-  };
-  if (mine > 0) {
+    for (int x = 0; x < kMats; ++x) total[o][x] = ok && bias ? static_cast<double>(bias[n]) : 0.0;
+  }
+  const int from = blockIdx.y * per, last = min(from + per, cut.count);
+  for (int first = from; first < last; first += NW) {      // the next NW chains, one a wave
+    f64x4 acc[kTiles];
 #pragma unroll
-    for (int s = 0; s < kSets; ++s) fetch(s, s);
-    int i = 0;
-    for (; i + kSets <= mine; i += kSets)
+    for (int t = 0; t < kTiles; ++t) acc[t] = f64x4{0, 0, 0, 0};
+    const int begin = (first + wave) * cut.length, end = first + wave < last ? min(begin + cut.length, K) : begin;
+    // Runs of 32 k: a lane takes 4 g .. 4 g + 3 of either half (an instruction's lanes fetch 64 bytes of a row side by side). Two runs are on their
+    // way or in work; each set of registers is filled again as soon as its run is multiplied, without a branch around the loads (in the last round of them a run past
+    // the last is the last one again), so that the compiler waits for the oldest only.
+    constexpr int kSets = 2;
+    const int runs = end > begin ? (end - begin) / 32 : 0;
+    float4 a[kSets][2], w[kSets][kTiles][2];
+    auto fetch = [&](int s, int i) __attribute__((always_inline)) {
+      const int k = begin + (i < runs ? i : runs - 1) * 32 + g * 4;
 #pragma unroll
-      for (int s = 0; s < kSets; ++s) {
-        multiply(s);
-        fetch(s, i + kSets + s);
+      for (int h = 0; h < 2; ++h) {
+        a[s][h] = quad<kVec>(a_row, k + 16 * h);
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) w[s][t][h] = quad<kVec>(w_row[t], k + 16 * h);
       }
+    };
+    auto multiply = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < kSets - 1; ++s)
-      if (i + s < mine) multiply(s);
-  }
-  if (runs % NW == wave) {      // what is left of K beyond the whole runs
-    for (int k = runs * 32; k < K; k += 16) {
+      for (int h = 0; h < 2; ++h) {
+        if (!row_ok) a[s][h] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) acc[t] = fma_quad(w[s][t][h], a[s][h], acc[t]);
+      }
+    };
+    if (runs > 0) {
+#pragma unroll
+      for (int s = 0; s < kSets; ++s) fetch(s, s);
+      int i = 0;
+      for (; i + kSets < runs; i += kSets)
+#pragma unroll
+        for (int s = 0; s < kSets; ++s) {
+          multiply(s);
+          fetch(s, i + kSets + s);
+        }
+#pragma unroll
+      for (int s = 0; s < kSets; ++s)
+        if (i + s < runs) multiply(s);
+    }
+    for (int k = begin + runs * 32; k < end; k += 16) {      // what is left of K beyond the whole runs
       const float4 left = row_ok ? quad_within<kVec>(a_row, k + g * 4, K) : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
       for (int t = 0; t < kTiles; ++t) acc[t] = fma_quad(quad_within<kVec>(w_row[t], k + g * 4, K), left, acc[t]);
     }
-  }
+    if (first > from) __syncthreads();      // (the chains before have been added up)
 #pragma unroll
-  for (int t = 0; t < kTiles; ++t)
+    for (int t = 0; t < kTiles; ++t)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) sums[wave][t][v][lane] = acc[t][v];
-  __syncthreads();
-  // an output a thread: tile, weight row i = 4 v + g', row of A j: place (v, 16 g' + j)
-  for (int i = threadIdx.x; i < NT * 256; i += 64 * NW) {
-    const int tile = i / 256, v = i / 64 % 4, at = i % 64, m = at % 16, n = n0 + tile * 16 + 4 * v + at / 16;
-    if (m >= M || n >= N) continue;
-    double s[kMats];
+      for (int v = 0; v < 4; ++v) sums[wave][t][v][lane] = acc[t][v];
+    __syncthreads();
 #pragma unroll
-    for (int x = 0; x < kMats; ++x) {
-      s[x] = bias && !parts ? static_cast<double>(bias[n]) : 0.0;
+    for (int o = 0; o < kOut; ++o) {
+      int tile, v, at, m, n;
+      const bool ok = place(o, tile, v, at, m, n);
+      if (!ok) continue;
 #pragma unroll
-      for (int w = 0; w < NW; ++w) s[x] += sums[w][tile * kMats + x][v][at];
+      for (int w = 0; w < NW; ++w) {
+        if (first + w >= last) break;      // (uniform)
+#pragma unroll
+        for (int x = 0; x < kMats; ++x) {
+          const double sum = sums[w][tile * kMats + x][v][at];
+          if (parts) parts[(static_cast<int64_t>(first + w) * M + m) * N + n] = sum;
+          else total[o][x] += sum;
+        }
+      }
     }
+  }
+  if (parts) return;
+#pragma unroll
+  for (int o = 0; o < kOut; ++o) {
+    int tile, v, at, m, n;
+    if (!place(o, tile, v, at, m, n)) continue;
     float* dst = out + static_cast<int64_t>(m) * ldo + n;
-    if constexpr (kMats == 2) *dst = gated(s[0], s[1], gelu);
-    else if (parts) parts[(static_cast<int64_t>(blockIdx.y) * M + m) * N + n] = s[0];
-    else put<kEpilogue>(dst, s[0]);
+    if constexpr (kMats == 2) *dst = gated(total[o][0], total[o][1], gelu);
+    else put<kEpilogue>(dst, total[o][0]);
   }
 }
 
 // A block of WM x (4 / WM) waves, each 32 rows x 32 weight rows; kMats = 2: the weight rows of a wave are 16 of gate and the same 16 of up.
-// parts (with gridDim.z > 1): this share's sums, [share][M][N]; the epilogue is then the second launch's.
-template <int WM, int kMats, int kEpilogue, bool kVec>
-__global__ void __launch_bounds__(256, WM == 2 ? 3 : 2) exact_tile_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ A, int64_t lda,
+// kFold: the block takes all chains and adds them up; else chain blockIdx.z, whose sums go to parts, [chain][M][N], and the epilogue is the second launch's.
+template <int WM, int kMats, int kEpilogue, bool kVec, bool kFold>
+__global__ void __launch_bounds__(256, WM == 2 && !kFold ? 3 : 2) exact_tile_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ A, int64_t lda,
                                                          const float* __restrict__ W, const float* __restrict__ W2, int64_t ldw,
-                                                         const float* __restrict__ bias, double* __restrict__ parts, int M, int N, int K, int k_share, int gelu) {
+                                                         const float* __restrict__ bias, double* __restrict__ parts, Cut cut, int M, int N, int K, int gelu) {
   constexpr int WN = 4 / WM, BM = 32 * WM, BW = 32 * WN, BK = 32, kPad = 4;
   constexpr int kOwn = 32 / kMats;                     // outputs of a wave along N
   __shared__ __attribute__((aligned(16))) float As[2][BM][BK + kPad], Ws[2][BW][BK + kPad];      // (as doubles, widened once as they are brought: 174 us where this took 169)
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
   const int wm = wave / WN, wn = wave % WN;
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * WN * kOwn;
-  const int k_begin = blockIdx.z * k_share, k_end = k_begin + k_share < K ? k_begin + k_share : K;
   constexpr int kA = BM * BK / 4 / 256, kW = BW * BK / 4 / 256;      // quads a thread brings of either operand
   const float *a_row[kA], *w_row[kW];      // (rows past the end: the last one again, its results are not stored)
 #pragma unroll
@@ -179,11 +216,29 @@ __global__ void __launch_bounds__(256, WM == 2 ? 3 : 2) exact_tile_kernel(float*
     w_row[i] = (kMats == 2 && row % 32 >= 16 ? W2 : W) + static_cast<int64_t>(n < N ? n : N - 1) * ldw;
   }
   const int k_own = threadIdx.x % 8 * 4;      // (threadIdx.x + 256 i has the same place in its row)
-  f64x4 acc[2][2];      // [rows of A][weight rows]
+  const int k_begin = kFold ? 0 : blockIdx.z * cut.length, k_end = kFold ? K : min(k_begin + cut.length, K);
+  static_assert(kFold || kMats == 1, "gate and up meet in the block");
+  f64x4 acc[2][2], sum[2][2];      // [rows of A][weight rows]: of this chain, of the chains before (kFold)
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f64x4{0, 0, 0, 0};
+    for (int j = 0; j < 2; ++j) acc[i][j] = sum[i][j] = f64x4{0, 0, 0, 0};
+  if constexpr (kFold && kMats == 1)
+    if (bias) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int n = n0 + wn * 32 + j * 16 + r;
+        const double b = n < N ? bias[n] : 0.0;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) sum[i][j] = f64x4{b, b, b, b};
+      }
+    }
+  auto end_chain = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) sum[i][j] += acc[i][j], acc[i][j] = f64x4{0, 0, 0, 0};
+  };
   // Two slabs in registers, on their way, while a third is worked on: a slab comes in some 1.4 us when the chip is busy, and its own products last 0.9.
   // (The loads of whole slabs are issued whatever the thread: under a condition each would be waited for by itself.)
   float4 fa[2][kA], fw[2][kW];
@@ -217,6 +272,14 @@ __global__ void __launch_bounds__(256, WM == 2 ? 3 : 2) exact_tile_kernel(float*
         for (int j = 0; j < 2; ++j) acc[i][j] = fma_quad(a[i], w[j], acc[i][j]);
     }
   };
+  int left = cut.length / (2 * BK);      // pairs of slabs of this chain
+  auto end_pair = [&]() __attribute__((always_inline)) {
+    if constexpr (kFold)
+      if (--left == 0) {      // (uniform)
+        end_chain();
+        left = cut.length / (2 * BK);
+      }
+  };
   // (two slabs in LDS: a slab's place is written again two barriers after the barrier behind which it is read)
   auto step = [&](auto set, int slab, auto more) __attribute__((always_inline)) {
     keep(set);
@@ -235,14 +298,17 @@ __global__ void __launch_bounds__(256, WM == 2 ? 3 : 2) exact_tile_kernel(float*
   for (; slab + 3 < whole; slab += 2) {
     step(first, slab, more);
     step(second, slab + 1, more);
+    end_pair();
   }
   if (whole - slab == 3) {
     step(first, slab, more);
     step(second, slab + 1, done);
+    end_pair();
     step(first, slab + 2, done);
   } else if (whole - slab == 2) {
     step(first, slab, done);
     step(second, slab + 1, done);
+    end_pair();
   } else if (whole - slab == 1) {
     step(first, slab, done);
   }
@@ -256,6 +322,7 @@ __global__ void __launch_bounds__(256, WM == 2 ? 3 : 2) exact_tile_kernel(float*
     __syncthreads();
     multiply(first);
   }
+  end_chain();      // (the last one; zeros where its end was a pair's)
   // D: rows of A 4 v + g, weight row r
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -265,81 +332,78 @@ __global__ void __launch_bounds__(256, WM == 2 ? 3 : 2) exact_tile_kernel(float*
       if (m >= M) continue;
       if constexpr (kMats == 2) {
         const int n = n0 + wn * 16 + r;
-        if (n < N) out[static_cast<int64_t>(m) * ldo + n] = gated(acc[i][0][v], acc[i][1][v], gelu);
+        if (n < N) out[static_cast<int64_t>(m) * ldo + n] = gated(sum[i][0][v], sum[i][1][v], gelu);
       } else {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           const int n = n0 + wn * 32 + j * 16 + r;
           if (n >= N) continue;
-          if (parts) parts[(static_cast<int64_t>(blockIdx.z) * M + m) * N + n] = acc[i][j][v];
-          else put<kEpilogue>(out + static_cast<int64_t>(m) * ldo + n, (bias ? static_cast<double>(bias[n]) : 0.0) + acc[i][j][v]);
+          if constexpr (kFold) put<kEpilogue>(out + static_cast<int64_t>(m) * ldo + n, sum[i][j][v]);
+          else parts[(static_cast<int64_t>(blockIdx.z) * M + m) * N + n] = sum[i][j][v];
         }
       }
     }
 }
 
-// The shares' sums in their order, then the epilogue.
+// The chains' sums in their order, then the epilogue.
 template <int kEpilogue>
 __global__ void __launch_bounds__(256) exact_sum_kernel(float* __restrict__ out, int64_t ldo, const double* __restrict__ parts, const float* __restrict__ bias,
-                                                        int M, int N, int shares) {
+                                                        int M, int N, int chains) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, all = static_cast<int64_t>(M) * N;
   if (i >= all) return;
   const int n = i % N;
   double s = bias ? static_cast<double>(bias[n]) : 0.0;
-  double p[kMaxShares];
+  double p[kMaxChains];
 #pragma unroll
-  for (int x = 0; x < kMaxShares; ++x) p[x] = x < shares ? parts[x * all + i] : 0.0;
+  for (int x = 0; x < kMaxChains; ++x) p[x] = parts[(x < chains ? x : 0) * all + i];
 #pragma unroll
-  for (int x = 0; x < kMaxShares; ++x) s += p[x];
+  for (int x = 0; x < kMaxChains; ++x)
+    if (x < chains) s += p[x];
   put<kEpilogue>(out + i / N * ldo + n, s);
 }
 
-// How K is shared out over blocks: the number of shares (at most 16, at least 128 k each) with the least time of the compute unit that has the most
-// blocks: 35.5 ns a k of a block (30 of them its SIMDs' matrix cores) and some 0.5 us a block, a twentieth more with one block to a compute unit, and
-// for the second launch 4 us and 0.7 us a million sums. Measured / by that count, us, 896 x 4,864: 450 rows in 4 shares 91.5 / 92.5, in 9 83.6 / 85.8; 200 rows in 4
-// 52.3 / 50.4, in 9 46.5 / 44.7, in 16 54.4 / 53; 768 rows in 2 173.7 / 179, in 3 121.1 / 122. Returns k a share (a multiple of a slab). Up to 16 rows and in the
-// gated form K is not shared out. Up to 16 rows: shares of 1,024 k and more for one block to a compute unit, where the
-// blocks of 16 weight rows are fewer than half the compute units and K is long (896 x 4,864, 8 rows: 19.0 us in 56 blocks of 16 waves).
-static int exact_share(int M, int N, int K) {
-  if (M <= kExactRows) {
-    const int blocks = (N + 15) / 16, cus = compute_units();
-    if (blocks * 2 >= cus || K < 2048) return K;
-    const int room = cus / blocks < kMaxShares ? cus / blocks : kMaxShares, shares = room < K / 1024 ? room : K / 1024;
-    return ((K + shares - 1) / shares + 31) / 32 * 32;
-  }
+// Up to 16 rows: chains a block takes. Four where the blocks of 16 weight rows are fewer than half the compute units and the chains more than a block's eight
+// waves, else all of them.
+static int chains_per_block(int N, const Cut& cut) { return cut.count > 8 && (N + 15) / 16 * 2 < compute_units() ? 4 : cut.count; }
+
+// More rows: whether the chains are dealt out over blocks, for the least time of the compute unit that has the most blocks: 35.5 ns a k of a block (30 of them its SIMDs'
+// matrix cores) and some 0.5 us a block, a twentieth more with one block to a compute unit, and for the second launch 4 us and 0.7 us a million sums.
+// Not where the sums of 64 rows are more than kMostBytes.
+static bool chains_apart(int M, int N, int K, const Cut& cut) {
+  if (static_cast<int64_t>(cut.count) * N * std::min(M, 64) * 8 > kMostBytes) return false;
   const int BM = M <= 32 ? 32 : 64, BW = M <= 32 ? 128 : 64, cus = compute_units();
   const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BW - 1) / BW);
-  int best = K;
-  double least = 1e30;
-  for (int shares = 1; shares <= kMaxShares && (shares == 1 || K / shares >= 128); ++shares) {
-    const int k = ((K + shares - 1) / shares + 31) / 32 * 32, got = (K + k - 1) / k;
-    const int64_t rounds = (tiles * got + cus - 1) / cus;
-    const double us = rounds * (0.0355 * k + 0.5) * (rounds == 1 ? 1.05 : 1.0) + (got > 1 ? 4.0 + 0.7e-6 * got * M * N : 0.0);
-    if (us < least) least = us, best = got > 1 ? k : K;
-  }
-  return best;
+  auto us = [&](int64_t blocks, int k) { const int64_t rounds = (blocks + cus - 1) / cus; return rounds * (0.0355 * k + 0.5) * (rounds == 1 ? 1.05 : 1.0); };
+  return cut.count > 1 && us(tiles * cut.count, cut.length) + 4.0 + 0.7e-6 * cut.count * M * N < us(tiles, K);
+}
+
+// Rows that one launch takes where the chains' sums go to memory, in whole tiles.
+static int rows_at_once(int M, int N, const Cut& cut) {
+  const int64_t most = kMostBytes / (static_cast<int64_t>(cut.count) * N * 8);
+  return M <= most ? M : static_cast<int>(most / 64 * 64);
 }
 
 template <int kEpilogue>
-static void launch_exact_sum(float* out, int64_t ldo, const double* parts, const float* bias, int M, int N, int shares, hipStream_t stream) {
+static void launch_exact_sum(float* out, int64_t ldo, const double* parts, const float* bias, int M, int N, int chains, hipStream_t stream) {
   const int64_t all = static_cast<int64_t>(M) * N;
-  exact_sum_kernel<kEpilogue><<<static_cast<unsigned>((all + 255) / 256), 256, 0, stream>>>(out, ldo, parts, bias, M, N, shares);
+  exact_sum_kernel<kEpilogue><<<static_cast<unsigned>((all + 255) / 256), 256, 0, stream>>>(out, ldo, parts, bias, M, N, chains);
 }
 
-// Up to 16 rows: blocks of eight waves (four in the gated form, whose blocks are many); four tiles of weight rows a block against a matrix as long as a
-// vocabulary, so that the rows of A are read a quarter as often.
+// Up to 16 rows: blocks of eight waves; two tiles of weight rows and four waves a block against a matrix as long as a vocabulary, so that the rows of A are read half as
+// often (8 rows, 151,936 x 896: 113 us; four tiles 130, eight waves 143).
 template <int kMats, int kEpilogue, bool kVec>
 static int launch_exact_rows(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, const float* W2, int64_t ldw, const float* bias,
                              double* parts, int M, int N, int K, int gelu, hipStream_t stream) {
-  const int tiles = (N + 15) / 16, cus = compute_units();
-  const int k_share = kMats == 1 ? exact_share(M, N, K) : K, shares = (K + k_share - 1) / k_share;
-  if (kMats == 1 && tiles >= 16 * cus)
-    exact_rows_kernel<4, 4, 1, kEpilogue, kVec><<<(tiles + 3) / 4, 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, nullptr, K, M, N, K, gelu);
-  else if (kMats == 1 || tiles < cus)
-    exact_rows_kernel<8, 1, kMats, kEpilogue, kVec><<<dim3(tiles, shares), 512, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, shares > 1 ? parts : nullptr, k_share, M, N, K, gelu);
-  else
-    exact_rows_kernel<4, 1, kMats, kEpilogue, kVec><<<tiles, 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, nullptr, K, M, N, K, gelu);
-  if (shares > 1) launch_exact_sum<kEpilogue>(out, ldo, parts, bias, M, N, shares, stream);
+  const Cut cut = cut_of(K);
+  const int tiles = (N + 15) / 16;
+  if (kMats == 1 && chains_per_block(N, cut) < cut.count) {
+    exact_rows_kernel<4, 1, 1, kEpilogue, kVec><<<dim3(tiles, (cut.count + 3) / 4), 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, parts, cut, 4, M, N, K, gelu);
+    launch_exact_sum<kEpilogue>(out, ldo, parts, bias, M, N, cut.count, stream);
+  } else if (kMats == 1 && tiles >= 16 * compute_units()) {
+    exact_rows_kernel<4, 2, 1, kEpilogue, kVec><<<(tiles + 2 - 1) / 2, 64 * 4, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, nullptr, cut, cut.count, M, N, K, gelu);
+  } else {
+    exact_rows_kernel<8, 1, kMats, kEpilogue, kVec><<<tiles, 512, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, nullptr, cut, cut.count, M, N, K, gelu);
+  }
   return check_launch("gemm_exact_rows");
 }
 
@@ -347,10 +411,21 @@ template <int WM, int kMats, int kEpilogue, bool kVec>
 static int launch_exact_tile(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, const float* W2, int64_t ldw, const float* bias,
                              double* parts, int M, int N, int K, int gelu, hipStream_t stream) {
   constexpr int BM = 32 * WM, kOut = 32 * (4 / WM) / kMats;
-  const int k_share = kMats == 1 ? exact_share(M, N, K) : K, shares = (K + k_share - 1) / k_share;
-  dim3 grid((N + kOut - 1) / kOut, (M + BM - 1) / BM, shares);
-  exact_tile_kernel<WM, kMats, kEpilogue, kVec><<<grid, 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, shares > 1 ? parts : nullptr, M, N, K, k_share, gelu);
-  if (shares > 1) launch_exact_sum<kEpilogue>(out, ldo, parts, bias, M, N, shares, stream);
+  const Cut cut = cut_of(K);
+  if constexpr (kMats == 1) {
+    if (chains_apart(M, N, K, cut)) {
+      const int at_once = rows_at_once(M, N, cut);
+      for (int m = 0; m < M; m += at_once) {
+        const int rows = std::min(at_once, M - m);
+        float* dst = out + static_cast<int64_t>(m) * ldo;
+        exact_tile_kernel<WM, 1, kEpilogue, kVec, false><<<dim3((N + kOut - 1) / kOut, (rows + BM - 1) / BM, cut.count), 256, 0, stream>>>(
+            nullptr, 0, A + static_cast<int64_t>(m) * lda, lda, W, W2, ldw, bias, parts, cut, rows, N, K, gelu);
+        launch_exact_sum<kEpilogue>(dst, ldo, parts, bias, rows, N, cut.count, stream);
+      }
+      return check_launch("gemm_exact_tile");
+    }
+  }
+  exact_tile_kernel<WM, kMats, kEpilogue, kVec, true><<<dim3((N + kOut - 1) / kOut, (M + BM - 1) / BM), 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, nullptr, cut, M, N, K, gelu);
   return check_launch("gemm_exact_tile");
 }
 
@@ -376,8 +451,9 @@ using namespace alofa;
 // Float64 sums that alofa_gemm_exact needs room for with these sizes (0: none).
 extern "C" int64_t alofa_gemm_exact_parts(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  const int k_share = exact_share(M, N, K), shares = (K + k_share - 1) / k_share;
-  return shares > 1 ? static_cast<int64_t>(shares) * M * N : 0;
+  const Cut cut = cut_of(K);
+  if (M <= kExactRows ? chains_per_block(N, cut) == cut.count : !chains_apart(M, N, K, cut)) return 0;
+  return static_cast<int64_t>(cut.count) * (M <= kExactRows ? M : rows_at_once(M, N, cut)) * N;
 }
 
 extern "C" int alofa_gemm_exact(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, int64_t ldw, const float* bias, double* parts, int64_t room,
@@ -385,8 +461,7 @@ extern "C" int alofa_gemm_exact(float* out, int64_t ldo, const float* A, int64_t
   ALOFA_REQUIRE(M > 0 && N > 0 && K > 0, "gemm: M=%d N=%d K=%d must be positive", M, N, K);
   ALOFA_REQUIRE(epilogue == kExactStore || epilogue == kExactResidual, "gemm: unknown epilogue %d", epilogue);
   ALOFA_REQUIRE(lda >= K && ldw >= K && ldo >= N, "gemm: a leading dimension is shorter than its row");
-  ALOFA_REQUIRE(room >= alofa_gemm_exact_parts(M, N, K), "gemm: no room for the sums of the shares of K");
-  ALOFA_REQUIRE(alofa_gemm_exact_parts(M, N, K) <= static_cast<int64_t>(kMaxShares) * M * N, "gemm: more shares of K than are added up");
+  ALOFA_REQUIRE(room >= alofa_gemm_exact_parts(M, N, K), "gemm: no room for the sums of the chains of K");
   if (epilogue == kExactStore) return launch_exact<1, kExactStore>(out, ldo, A, lda, W, W, ldw, bias, parts, M, N, K, 0, stream);
   return launch_exact<1, kExactResidual>(out, ldo, A, lda, W, W, ldw, bias, parts, M, N, K, 0, stream);
 }

@@ -107,3 +107,50 @@ def test_exact_products_of_few_rows_and_very_long_k(M, N, K):
     acc = res.clone()
     ops().gemm(acc, a, w, add_to_out=True, exact=True)
     within(acc, want + res.cpu().numpy(), np.abs(want) + np.abs(want + res.cpu().numpy()) + 1e-7)
+
+
+# Every form (rows up to 16, 32 and beyond; chains of K in one block, over blocks, in rounds; two matrices; a vocabulary) adds up in one order: a row alone and the same row among
+# others are the same bits. Pairs of 2^40 that cancel exactly lie far apart in k: what is summed between them loses its low bits, and another order loses others.
+@pytest.mark.parametrize("N,K,shift", [(896, 896, 0), (896, 4864, 0), (17, 1030, 0), (130, 2056, 1), (70000, 200, 0), (33, 20000, 0), (4100, 3584, 0), (64, 127, 0), (48, 160, 0)])
+def test_a_row_of_an_exact_product_does_not_depend_on_the_others(N, K, shift):
+    gen = torch.Generator(device=DEV).manual_seed(N + K)
+    rows = 40 if N > 10000 else 300
+    a, w, b = (torch.randn(s, generator=gen, device=DEV) for s in ((rows, K + shift), (N, K + shift), (N,)))
+    order = torch.randperm(K, generator=gen, device=DEV)[:K // 8 * 2] + shift
+    plus, minus = order[::2], order[1::2]
+    w[:, minus] = w[:, plus]
+    a[:, plus] = torch.ldexp(a[:, plus], torch.tensor(40, device=DEV))
+    a[:, minus] = -a[:, plus]
+    a, w = a[:, shift:], w[:, shift:]
+    want = torch.empty(rows, N, device=DEV)
+    ops().gemm(want, a, w, b, exact=True)
+    gate = torch.empty(rows, N // 2, device=DEV)
+    ops().gemm_swiglu(gate, a, w[:N // 2], w[N // 2:N // 2 * 2], exact=True)
+    stream = torch.randn(rows, N, generator=gen, device=DEV)
+    added = stream.clone()
+    ops().gemm(added, a, w, add_to_out=True, exact=True)
+    for first, n in ((0, 1), (7, 5), (0, 16), (3, 17), (0, 32), (1, 33), (0, 64), (9, 65), (0, 200)):
+        if first + n > rows:
+            continue
+        part = slice(first, first + n)
+        out, half, acc = torch.empty(n, N, device=DEV), torch.empty(n, N // 2, device=DEV), stream[part].clone()
+        ops().gemm(out, a[part], w, b, exact=True)
+        ops().gemm_swiglu(half, a[part], w[:N // 2], w[N // 2:N // 2 * 2], exact=True)
+        ops().gemm(acc, a[part], w, add_to_out=True, exact=True)
+        assert torch.equal(out, want[part]) and torch.equal(acc, added[part]) and torch.equal(half, gate[part]), (first, n)
+
+
+def test_exact_sums_of_many_rows_stay_bounded():
+    from alofa_amd.csrc.build import load
+    for M, N, K in ((64, 152064, 3584), (4096, 896, 4864), (100000, 896, 4864), (64, 20000, 8192), (65, 8192, 8192), (1, 128, 27648), (16, 240, 17408)):
+        assert load().alofa_gemm_exact_parts(M, N, K) * 8 <= 64 << 20
+
+
+def test_exact_products_whose_sums_go_to_memory_in_pieces():
+    M, N, K = 1100, 500, 16384      # 16 chains, 64 KB of sums a row
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    a, w, res = (torch.randn(s, generator=gen, device=DEV) for s in ((M, K), (N, K), (M, N)))
+    acc = res.clone()
+    ops().gemm(acc, a, w, add_to_out=True, exact=True)
+    want = (a.double() @ w.double().T.contiguous()).cpu().numpy()
+    within(acc, want + res.cpu().numpy(), np.abs(want) + np.abs(want + res.cpu().numpy()) + 1e-7)
