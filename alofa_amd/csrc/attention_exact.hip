@@ -10,11 +10,12 @@
 //                             four consecutive keys of a channel, one 16-byte load.
 // A score is rounded to float and multiplied by the float scale, the weight is expf of its difference to the running maximum; the
 // sums of weights and of weighted values are float64, and where the maximum moves they take a float64 factor. The waves meet in
-// LDS in their order, so a row depends only on its own keys and the number of waves.
+// LDS in their order, and how many they are follows from the head size: a row's result depends on its own keys only, to the bit.
 //
 // Bound by the chain table -> keys -> scores -> weights -> values of few tiles in decode steps and by the matrix cores in prompts
 // (half of the columns idle with seven heads to a key head). us before (a wave a (token, head), one key a lane, every score twice)
-// and now, 14/2 heads of 64: 8 tokens at 130 to 260 keys 85 and 12; prompts of 64, 128 and 256 tokens 145 and 22.
+// and now, 14/2 heads of 64: 8 tokens at 130 to 260 keys 85 and 11; prompts of 64, 128 and 256 tokens 145 and 27 (23 with four waves a block
+// where blocks are many, and then a row depends on how many there are).
 // Cache layout: keys [block, kv_head, slot_in_block, d], values transposed [block, kv_head, d, slot_in_block].
 #include "common.h"
 
@@ -131,15 +132,11 @@ template <int NT>
 static void launch_attention_exact(float* out, int64_t out_stride, const float* q, int64_t q_stride, const float* k_cache, const float* v_cache,
                                    const int32_t* block_table, int max_blocks, const int32_t* req_of_token, const int32_t* positions, int tokens, int heads,
                                    int kv_heads, int block_size, int window, float scale, hipStream_t stream) {
-  // blocks that are fewer than the compute units get as many waves as the registers allow, the others four
-  constexpr int kMany = NT <= 3 ? 16 : NT <= 8 ? 8 : 4;
+  // (the number of waves, which decides whose running maximum a key's weight is taken against, follows from the head size alone: as many as the registers and LDS allow)
+  constexpr int kWaves = NT <= 8 ? 8 : 4;
   dim3 grid(tokens, kv_heads * ((heads / kv_heads + 15) / 16));
-  if (static_cast<int64_t>(grid.x) * grid.y < compute_units())
-    attention_exact_kernel<NT, kMany><<<grid, 64 * kMany, 0, stream>>>(out, out_stride, q, q_stride, k_cache, v_cache, block_table, max_blocks, req_of_token, positions,
-                                                                       heads, kv_heads, block_size, window, scale);
-  else
-    attention_exact_kernel<NT, 4><<<grid, 256, 0, stream>>>(out, out_stride, q, q_stride, k_cache, v_cache, block_table, max_blocks, req_of_token, positions, heads,
-                                                            kv_heads, block_size, window, scale);
+  attention_exact_kernel<NT, kWaves><<<grid, 64 * kWaves, 0, stream>>>(out, out_stride, q, q_stride, k_cache, v_cache, block_table, max_blocks, req_of_token, positions, heads, kv_heads,
+                                                                       block_size, window, scale);
 }
 
 }  // namespace alofa

@@ -154,3 +154,22 @@ def test_exact_products_whose_sums_go_to_memory_in_pieces():
     ops().gemm(acc, a, w, add_to_out=True, exact=True)
     want = (a.double() @ w.double().T.contiguous()).cpu().numpy()
     within(acc, want + res.cpu().numpy(), np.abs(want) + np.abs(want + res.cpu().numpy()) + 1e-7)
+
+
+@pytest.mark.parametrize("heads,kv_heads,d", [(14, 2, 64), (8, 1, 32), (6, 2, 160)])
+def test_a_row_of_exact_attention_does_not_depend_on_the_others(heads, kv_heads, d):
+    bs, rows, history = 16, 300, 500
+    gen = torch.Generator(device=DEV).manual_seed(d)
+    pages = -(-(rows + history) // bs)
+    q = torch.randn(rows, heads * d, generator=gen, device=DEV) * 2
+    kc, vc = torch.randn(pages, kv_heads, bs, d, generator=gen, device=DEV), torch.randn(pages, kv_heads, d, bs, generator=gen, device=DEV)
+    table = torch.arange(pages, dtype=torch.int32, device=DEV)[None].contiguous()
+    req, pos = torch.zeros(rows, dtype=torch.int32, device=DEV), torch.arange(history, history + rows, dtype=torch.int32, device=DEV)
+
+    def attend(part):
+        out = torch.empty_like(q[part])
+        ops().paged_attention(out, q[part], kc, vc, table, req[part], pos[part], heads, kv_heads, d, None, d ** -0.5, True)
+        return out
+    want = attend(slice(0, rows))
+    for first, n in ((0, 1), (299, 1), (5, 8), (17, 100), (100, 200)):
+        assert torch.equal(attend(slice(first, first + n)), want[first:first + n])
