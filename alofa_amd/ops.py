@@ -878,12 +878,23 @@ def pair_tiles(runs: list, window: Optional[int] = None, heads: Optional[int] = 
 TALL_ROWS = 256     # query rows a block of the attention kernel for many rows serves
 
 
-def attention_tall_pays(heads: int, d: int, block_size: int, scale: float, runs: int) -> bool:
-    """Whether ``runs`` runs of up to ``TALL_ROWS`` query rows go to the kernel with blocks of that many rows of one head: heads of 128,
-    pages of 16 tokens or more, and blocks for five eighths of the compute units. us, the kernel with blocks of 64 rows / this: 28/4 heads, four
-    portions of some 480 rows on 256 to 1,536 keys (224 blocks) 82 / 63, 16/16 heads, three prompts of 1,024 (192 blocks) 60 / 36, 40/8
-    heads, one prompt of 2,048 (320) 118 / 68; with fewer blocks the longest of them is what the launch waits for: 16/2 heads, one prompt of 2,048 (128) 47 / 57, 12/2 heads (96) 45 / 55."""
-    return d == 128 and block_size >= 16 and scale > 0 and runs * heads * 8 >= 5 * compute_units()
+def attention_tall_pays(heads: int, kv_heads: int, d: int, block_size: int, scale: float, portions: list) -> bool:
+    """Whether ``portions``, (rows brought, keys that the last of them sees) each, go to the kernel with blocks of ``TALL_ROWS`` query rows of one head:
+    heads of 128, pages of 16 tokens or more, blocks for five eighths of the compute units, and runs that are full enough. us, the kernel with blocks of
+    64 rows / this. Full runs: 28/4 heads, four portions of some 480 rows on 256 to 1,536 keys (224 blocks) 79 / 61, 16/16 heads, three prompts of 1,024 (192
+    blocks) 58 / 36, 40/8 heads, one prompt of 2,048 (320) 116 / 65; with fewer blocks the longest of them is what the launch waits for: 16/2 heads, one
+    prompt of 2,048 (128) 47 / 57, 12/2 heads (96) 45 / 55.
+    Runs of few rows: a block of this kernel fills a compute unit whatever its rows, and a wave walks all keys alone. 28/4 heads on 2,048 keys, 48 portions of 5 rows
+    132 / 226, of 17 135 / 234, 8 of 64 42 / 43; 40/8 heads, 48 of 64 295 / 336; from 96 rows a run on it is ahead (28/4 heads, 8 of 96 79 / 58; 40/8 heads, 48 of 96 on
+    512 keys 169 / 157), but where the heads of a group share the other kernel's tiles and the keys are few only from 150 on: 28/4 heads without history, 48 of 96 rows 39 / 47, 8 of
+    257 (128 a run) 29 / 32, 16 of 300 62 / 59; on 512 keys 8 of 257 73 / 57."""
+    if d != 128 or block_size < 16 or not scale > 0:
+        return False
+    runs, rows = sum(-(-n // TALL_ROWS) for n, _ in portions), sum(n for n, _ in portions)
+    if runs * heads * 8 < 5 * compute_units() or rows < 96 * runs:
+        return False
+    few_keys = sum(keys for _, keys in portions) < 512 * len(portions)
+    return not (few_keys and rows < 150 * runs and prefill_share(heads, kv_heads, d, sum(-(-n // 64) for n, _ in portions)))
 
 
 def attention_tall(out, q, k_cache, v_cache, block_table, runs, heads, kv_heads, d, window, scale) -> None:

@@ -37,16 +37,19 @@ class RowPlan:
         self.short_rows = None      # int32 indices of the short rows; None when every row is short (or none is)
         self.long_runs = None       # (request index, first row, rows, first position) per run; None when every row is short
         self._tiles: dict = {}
+        self._tall: dict = {}
         if self.n_short < ctx.tokens:
             self.long_runs = [(i, s.row0 + q0, min(TILE_ROWS, s.n - q0), s.pos0 + q0)
                               for i, s in enumerate(spans) if s.n > SHORT for q0 in range(0, s.n, TILE_ROWS)]
             if self.n_short:
                 self.short_rows = ops.upload([r for s in spans if s.n <= SHORT for r in range(s.row0, s.row0 + s.n)], self.device)
 
-    @property
-    def n_tall(self) -> int:
-        """How many runs of up to ``ops.TALL_ROWS`` rows the long portions make."""
-        return sum(-(-s.n // ops.TALL_ROWS) for s in self.spans if s.n > SHORT)
+    def in_tall_blocks(self, heads: int, kv_heads: int, d: int, block_size: int, scale: float) -> bool:
+        """Whether the long portions go to the kernel with blocks of ``ops.TALL_ROWS`` rows for a mixer with these head counts."""
+        key = (heads, kv_heads, d, block_size, scale)
+        if key not in self._tall:
+            self._tall[key] = ops.attention_tall_pays(*key, [(s.n, s.pos0 + s.n) for s in self.spans if s.n > SHORT])
+        return self._tall[key]
 
     def tall_runs(self):
         """The long portions in runs of up to ``ops.TALL_ROWS`` rows, the ones that see most keys first: int32 [n, 4] (request index, first row, rows, position of the first row)."""
@@ -106,7 +109,7 @@ def paged_attend(ctx, entry, qkv, attn, heads, kv_heads, d, window, scale, posit
         # the exact path, and page or head sizes the bfloat16 kernels are not built for
         ops.paged_attention(attn, qkv, kv.k, kv.v, kv.block_table, ctx.req_of_token, ctx.positions, *common, exact)
     else:
-        if plan.long_runs is not None and ops.attention_tall_pays(heads, d, kv.k.shape[2], scale, plan.n_tall):      # portions of prompts, many rows
+        if plan.long_runs is not None and plan.in_tall_blocks(heads, kv_heads, d, kv.k.shape[2], scale):      # portions of prompts, many rows
             ops.attention_tall(attn, qkv, kv.k, kv.v, kv.block_table, ctx.memo("gqa_attention.tall_runs", plan.tall_runs), *common)
         elif plan.long_runs is not None:      # portions of prompts
             tiles, share, rows = plan.tiles(heads, kv_heads, d, window)

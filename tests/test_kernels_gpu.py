@@ -1272,6 +1272,18 @@ def test_attention_of_many_rows(heads, kv_heads, bs, window):
     assert torch.equal(again, out)
 
 
+# which launches take the blocks of 256 rows (256 compute units): enough full runs; runs of few rows, however many; runs half full, with and without tiles that heads share, on few keys and on many
+@pytest.mark.parametrize("heads,kv_heads,portions,taken", [(40, 8, [(2048, 2048)], True), (12, 2, [(2048, 2048)], False), (28, 4, [(480, 1000)] * 4, True), (28, 4, [(5, 2053)] * 48, False),
+                                                           (28, 4, [(17, 17)] * 48, False), (40, 8, [(64, 2112)] * 48, False), (40, 8, [(33, 8225)] * 4, False), (28, 4, [(96, 608)] * 16, True),
+                                                           (28, 4, [(96, 96)] * 48, False), (28, 4, [(257, 257)] * 8, False), (28, 4, [(257, 769)] * 8, True), (28, 4, [(257, 257)] * 4, True),
+                                                           (40, 8, [(257, 257)] * 8, True), (28, 4, [(300, 300)] * 16, True), (16, 16, [(2048, 2048), (5, 9)], False)])
+def test_which_portions_the_blocks_of_many_rows_take(heads, kv_heads, portions, taken):
+    if ops().compute_units() != 256:
+        pytest.skip("the sizes are those of 256 compute units")
+    assert ops().attention_tall_pays(heads, kv_heads, 128, 16, 128 ** -0.5, portions) == taken
+    assert not ops().attention_tall_pays(heads, kv_heads, 64, 16, 0.125, portions) and not ops().attention_tall_pays(heads, kv_heads, 128, 8, 0.1, portions)
+
+
 # sharper and sharper softmaxes: where one key counts, its weight is one exactly, and only the others' are rounded
 @pytest.mark.parametrize("heads,kv_heads,n,history", [(8, 2, 700, 900), (6, 6, 512, 0), (16, 2, 300, 3000)])
 @pytest.mark.parametrize("sharp", [1, 2, 4, 8, 16])
