@@ -363,7 +363,7 @@ def _norm_operands(a: torch.Tensor, norm: tuple, K: int):
 
 def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
          add_to_out: bool = False, exact: bool = False, kernel: Optional[str] = None, norm: Optional[tuple] = None,
-         then_norm: Optional[tuple] = None) -> None:
+         then_norm: Optional[tuple] = None, scratch=None) -> None:
     """out = a @ w.T (+ bias), or out += a @ w.T when ``add_to_out`` (out is then
     the float32 residual stream). w is [out_features, in_features]. ``kernel``
     names the bfloat16 kernel ("rows", "stream" or "tiled") instead of ``few_rows_kernel``.
@@ -372,7 +372,9 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[tor
     ``then_norm`` = (weight, eps, rows) with ``add_to_out``: afterwards ``rows`` (out's shape, the
     activation dtype) holds the RMSNorm of out's new rows. Where the product's last launch has whole
     rows in hand (the tiled kernel with K shared out and a launch that adds the shares) the norm rides
-    on it; everywhere else it is the norm kernel, run here: the values are the same either way."""
+    on it; everywhere else it is the norm kernel, run here: the values are the same either way.
+    ``scratch``: (name, shape, dtype) -> a buffer of the caller's stream that the call may use and leave (a step's, which its captured graphs share and
+    the memory account sees); without it, the products that need one allocate it."""
     sizes = None if exact or norm is not None else _native().product(out, a, w, None, bias)      # (bfloat16 operands that 16-byte loads along K can read)
     if sizes is not None:
         M, N, K, ldo, lda, ldw, code = sizes
@@ -427,8 +429,10 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[tor
             rmsnorm(then_rows, out, then_w, then_eps, False)
         return
     if exact and a.dtype is torch.float32 and w.dtype is torch.float32 and out.dtype is torch.float32:
-        room = load().alofa_gemm_exact_parts(_I(M), _I(N), _I(K))      # (sums of the shares of K, where the tiles are too few for the chip)
-        parts = torch.empty(room, dtype=torch.float64, device=out.device) if room else None
+        room = load().alofa_gemm_exact_parts(_I(M), _I(N), _I(K))      # (sums of the chains of K, where the tiles are too few for the chip)
+        parts = None
+        if room:
+            parts = torch.empty(room, dtype=torch.float64, device=out.device) if scratch is None else scratch("product_sums", (room,), torch.float64)
         _call("alofa_gemm_exact", _ptr(out), _L(_rows("out", out)), _ptr(a), _L(_rows("a", a)), _ptr(w), _L(_rows("w", w)), _ptr(bias), _ptr(parts), _L(room),
               _I(M), _I(N), _I(K), _I(ADD_TO_RESIDUAL if add_to_out else STORE), _stream())
         if then_rows is not None:

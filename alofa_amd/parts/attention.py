@@ -265,17 +265,17 @@ class GQAAttention(Mixer):
         if norm is not None:      # the input norm rides on the product
             ops.gemm(qkv, residual, self.w_qkv, self.b_qkv, norm=norm.as_rmsnorm())
         else:
-            ops.gemm(qkv, x, self.w_qkv, self.b_qkv, exact=exact)
+            ops.gemm(qkv, x, self.w_qkv, self.b_qkv, exact=exact, scratch=ctx.scratch)
         attn = ctx.scratch("attn", (T, self.heads * self.d), self.rt.dtype)
         paged_attend(ctx, entry, qkv, attn, self.heads, self.kv_heads, self.d, self.window, self.scale, self.position, self.rt)
         if out is not None:
-            ops.gemm(out, attn, self.w_o, self.b_o, exact=exact)
+            ops.gemm(out, attn, self.w_o, self.b_o, exact=exact, scratch=ctx.scratch)
         elif self.b_o is not None:
             proj = ctx.scratch("attn_proj", (T, self.hidden), torch.float32)
-            ops.gemm(proj, attn, self.w_o, self.b_o, exact=exact)
+            ops.gemm(proj, attn, self.w_o, self.b_o, exact=exact, scratch=ctx.scratch)
             residual.add_(proj)
         else:      # (then: the norm behind this part, left in the rows given with it)
-            ops.gemm(residual, attn, self.w_o, add_to_out=True, exact=exact, then_norm=_then(then))
+            ops.gemm(residual, attn, self.w_o, add_to_out=True, exact=exact, scratch=ctx.scratch, then_norm=_then(then))
 
 
 def _then(then):

@@ -111,7 +111,7 @@ class DifferentialAttention(Mixer):
         kv = ctx.kv(where)
         H, G, D = self.heads, self.kv_heads, self.d
         proj = ctx.scratch("maps_proj", (T, self.w_in.shape[0]), self.rt.dtype)
-        ops.gemm(proj, x, self.w_in, self.b_in, exact=exact)
+        ops.gemm(proj, x, self.w_in, self.b_in, exact=exact, scratch=ctx.scratch)
         table, qkv = self.position.table(ctx.n_positions), proj[:, :self.width]
         fast = not exact and ops.maps_attention_fast(D, self.dm, kv.k.shape[2], self.keep_first, self.rt.dtype)
         plan = ctx.memo("gqa_attention.rows", lambda: RowPlan(ctx)) if fast else None
@@ -126,9 +126,9 @@ class DifferentialAttention(Mixer):
         attn = ctx.scratch("maps_out", (T, H * D), self.rt.dtype)
         self._attend(ctx, qkv if turns else proj[:, :2 * H * self.dm], kv, attn, plan, (*table, kv.slots) if turns else None)
         if out is not None:
-            ops.gemm(out, attn, self.w_o, exact=exact)
+            ops.gemm(out, attn, self.w_o, exact=exact, scratch=ctx.scratch)
         else:
-            ops.gemm(residual, attn, self.w_o, add_to_out=True, exact=exact)
+            ops.gemm(residual, attn, self.w_o, add_to_out=True, exact=exact, scratch=ctx.scratch)
 
     def _attend(self, ctx, q, kv, attn, plan, rope) -> None:
         T, H, G, D = q.shape[0], self.heads, self.kv_heads, self.d

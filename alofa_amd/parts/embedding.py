@@ -105,7 +105,7 @@ class LMHead(Part):
 
     def forward(self, ctx, y):
         logits = ctx.scratch("logits", (y.shape[0], self.vocab), torch.float32)
-        ops.gemm(logits, y, self.weight, exact=self.rt.exact)
+        ops.gemm(logits, y, self.weight, exact=self.rt.exact, scratch=ctx.scratch)
         if self.scale != 1.0:
             ops.scale_(logits, self.scale)
         if self.softcap is not None:

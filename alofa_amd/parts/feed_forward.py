@@ -61,13 +61,13 @@ class SwiGLU(FeedForward):
         else:
             ops.gemm_swiglu(act, x, self.w_gate, self.w_up, exact=self.rt.exact, act=self.activation)
         if out is not None:
-            ops.gemm(out, act, self.w_down, exact=self.rt.exact)
+            ops.gemm(out, act, self.w_down, exact=self.rt.exact, scratch=ctx.scratch)
             return
         then_norm = None
         if then is not None:      # the norm behind this part, left in the rows given with it
             weight, eps = then[0].as_rmsnorm()
             then_norm = (weight, eps, then[1])
-        ops.gemm(residual, act, self.w_down, add_to_out=True, exact=self.rt.exact, then_norm=then_norm)
+        ops.gemm(residual, act, self.w_down, add_to_out=True, exact=self.rt.exact, scratch=ctx.scratch, then_norm=then_norm)
 
 
 def _softplus(z: float) -> float:
@@ -117,7 +117,7 @@ class DenseActivated(FeedForward):
         if norm is not None:      # the norm in front rides on the product
             ops.gemm(act, residual, self.w_up, self.b_up, norm=norm.as_rmsnorm())
         else:
-            ops.gemm(act, x, self.w_up, self.b_up, exact=self.rt.exact)
+            ops.gemm(act, x, self.w_up, self.b_up, exact=self.rt.exact, scratch=ctx.scratch)
         if self.activation == "xielu":
             ops.activation(act, act, ops.XIELU, self.a, self.b, self.rt.exact)
         elif self.activation == "gelu_tanh":
@@ -125,12 +125,12 @@ class DenseActivated(FeedForward):
         else:
             ops.relu_squared(act, act)
         if scale is None and self.b_down is None:
-            ops.gemm(residual, act, self.w_down, add_to_out=True, exact=self.rt.exact)
+            ops.gemm(residual, act, self.w_down, add_to_out=True, exact=self.rt.exact, scratch=ctx.scratch)
             if then is not None:
                 ops.rmsnorm(then[2], residual, then[0], then[1], self.rt.exact)
         elif scale is None:
             apart = ctx.scratch("sub_out", tuple(residual.shape), torch.float32)
-            ops.gemm(apart, act, self.w_down, self.b_down, exact=self.rt.exact)
+            ops.gemm(apart, act, self.w_down, self.b_down, exact=self.rt.exact, scratch=ctx.scratch)
             ops.add_scaled(residual, apart, 1.0, exact=self.rt.exact)
             if then is not None:
                 ops.rmsnorm(then[2], residual, then[0], then[1], self.rt.exact)

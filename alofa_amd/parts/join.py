@@ -28,7 +28,7 @@ class ConcatProjection(Join):
     def forward(self, ctx, hidden, first):
         both = ctx.scratch("joined", (hidden.shape[0], 2 * self.width), self.rt.dtype)
         ops.concat_rows(both, hidden, first)
-        ops.gemm(hidden, both, self.weight, exact=self.rt.exact)
+        ops.gemm(hidden, both, self.weight, exact=self.rt.exact, scratch=ctx.scratch)
 
 
 register_part("join", "concat_projection", ConcatProjection)

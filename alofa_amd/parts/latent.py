@@ -216,7 +216,7 @@ class LatentAttention(Mixer):
         """The step's latents, normed, ``copies`` times side by side in ``out`` (each widened to ``pad`` channels with zeros)."""
         if down is None:
             down = ctx.scratch("latent_down", (x.shape[0], self.r), torch.float32)
-            ops.gemm(down, x, self.w_down, exact=self.rt.exact)
+            ops.gemm(down, x, self.w_down, exact=self.rt.exact, scratch=ctx.scratch)
         w, eps = self.norm
         ops.rmsnorm_spread(out, down, w, eps, pad, copies, self.rt.exact)
 
@@ -237,15 +237,15 @@ class LatentAttention(Mixer):
                 if norm is not None:
                     ops.gemm(qg, residual, self.w_in, norm=norm.as_rmsnorm())
                 else:
-                    ops.gemm(qg, x, self.w_in, exact=exact)
+                    ops.gemm(qg, x, self.w_in, exact=exact, scratch=ctx.scratch)
                 q, gate = qg[:, :H * self.dk], (qg[:, H * self.dk:H * (self.dk + self.dv)] if self.gated else None)
                 down = qg[:, qg.shape[1] - self.r:]
             else:
                 q, gate = ctx.scratch("latent_q", (T, H * self.dk), self.rt.dtype), None
-                ops.gemm(q, x, self.w_q, exact=exact)
+                ops.gemm(q, x, self.w_q, exact=exact, scratch=ctx.scratch)
                 if self.gated:
                     gate = ctx.scratch("latent_gate", (T, H * self.dv), self.rt.dtype)
-                    ops.gemm(gate, x, self.w_gate, exact=exact)
+                    ops.gemm(gate, x, self.w_gate, exact=exact, scratch=ctx.scratch)
             # [a query per head | the latent as key | the latent as value]
             qkv = ctx.scratch("qkv", (T, (H + 2) * d), self.rt.dtype)
             self._latent(ctx, x, qkv[:, H * d:], d, 2, down)
@@ -255,20 +255,20 @@ class LatentAttention(Mixer):
             ops.head_project(heads_out, attn, self.w_result, exact, gate=gate)
         else:
             qkv = ctx.scratch("qkv", (T, 3 * H * d), self.rt.dtype)
-            ops.gemm(qkv[:, :H * d], x, self.w_q, exact=exact)
+            ops.gemm(qkv[:, :H * d], x, self.w_q, exact=exact, scratch=ctx.scratch)
             c = ctx.scratch("latent", (T, self.r), self.rt.dtype)
             self._latent(ctx, x, c, self.r, 1)
-            ops.gemm(qkv[:, H * d:], c, self.w_kv, exact=exact)
+            ops.gemm(qkv[:, H * d:], c, self.w_kv, exact=exact, scratch=ctx.scratch)
             paged_attend(ctx, where, qkv, attn, H, H, d, self.window, self.scale, self.position, self.rt)
             if self.gated:
                 gate = ctx.scratch("latent_gate", (T, H * d), self.rt.dtype)
-                ops.gemm(gate, x, self.w_gate, exact=exact)
+                ops.gemm(gate, x, self.w_gate, exact=exact, scratch=ctx.scratch)
                 ops.sigmoid_gate(attn, gate, exact)
             heads_out = attn
         if out is not None:
-            ops.gemm(out, heads_out, self.w_o, exact=exact)
+            ops.gemm(out, heads_out, self.w_o, exact=exact, scratch=ctx.scratch)
         elif scale is None:
-            ops.gemm(residual, heads_out, self.w_o, add_to_out=True, exact=exact)
+            ops.gemm(residual, heads_out, self.w_o, add_to_out=True, exact=exact, scratch=ctx.scratch)
         else:
             ops.gemm_channel_scaled(residual, heads_out, self.w_o, scale, ctx.scratch("sub_out", tuple(residual.shape), torch.float32), exact, then_norm=then)
 
@@ -281,7 +281,7 @@ class LatentAttention(Mixer):
         if norm is not None:
             ops.gemm(proj, residual, self.w_in, norm=norm.as_rmsnorm())
         else:
-            ops.gemm(proj, x, self.w_in, exact=exact)
+            ops.gemm(proj, x, self.w_in, exact=exact, scratch=ctx.scratch)
         table = self.angles.table(ctx.n_positions) if t else None
         queries, q = None, proj[:, :self.first_width]
         if self.q_rank:
@@ -293,7 +293,7 @@ class LatentAttention(Mixer):
             ops.latent_rows(proj, queries, keys, t, ctx.positions, table, pages=(kv.slots, kv.k, kv.v), exact=exact)
             if self.q_rank:
                 q = ctx.scratch("latent_q", (T, H * q_size), self.rt.dtype)
-                ops.gemm(q, cq, self.w_uq, exact=exact)
+                ops.gemm(q, cq, self.w_uq, exact=exact, scratch=ctx.scratch)
             ql = ctx.scratch("qkv", (T, H * d), self.rt.dtype)
             ops.head_project(ql, q, self.w_query, exact, turn=(ctx.positions, *table) if t else None)
             attend_pages(ctx, kv, ql, attn, H, 1, d, self.window, self.scale, self.rt, sink=self.sink)
@@ -304,10 +304,10 @@ class LatentAttention(Mixer):
         c = ctx.scratch("latent", (T, self.c_width), self.rt.dtype)
         ops.latent_rows(proj, queries, keys, t, rows=c, exact=exact)
         if self.q_rank:
-            ops.gemm(qkv[:, :H * d], cq, self.w_uq, exact=exact)
+            ops.gemm(qkv[:, :H * d], cq, self.w_uq, exact=exact, scratch=ctx.scratch)
         else:
             qkv[:, :H * d].copy_(q)
-        ops.gemm(qkv[:, H * d:], c, self.w_kv, exact=exact)
+        ops.gemm(qkv[:, H * d:], c, self.w_kv, exact=exact, scratch=ctx.scratch)
         ops.norm_turn_write(qkv, ctx.positions, table, H, H, d, d, ops.NORM_NONE, None, None, 0.0, exact, kv.slots, kv.k, kv.v)
         attend_pages(ctx, kv, qkv[:, :H * d], attn, H, H, d, self.window, self.scale, self.rt, sink=self.sink)
         return attn

@@ -124,7 +124,7 @@ class RoutedExperts(FeedForward):
         The shared expert's weights, where it has a gate, are left in the scratch buffer ``router_shared``."""
         T = x.shape[0]
         z = ctx.scratch("router_z", (T, self.w_router.shape[0]), torch.float32)
-        ops.gemm(z, x, self.w_router, self.b_router, exact=self.rt.exact)
+        ops.gemm(z, x, self.w_router, self.b_router, exact=self.rt.exact, scratch=ctx.scratch)
         dense = ctx.scratch("router_dense", (T, self.experts), torch.float32)
         chosen, weights = ctx.scratch("router_chosen", (T, self.top), torch.int32), ctx.scratch("router_weights", (T, self.top), torch.float32)
         if self.score != "softmax":
@@ -177,26 +177,26 @@ class RoutedExperts(FeedForward):
             return
         # every expert's gate and up for every row, the rows an expert is not taken by weighted with zero
         u, act = ctx.scratch("experts_up", (T, self.channels), self.rt.dtype), ctx.scratch("ff_act", (T, self.channels), self.rt.dtype)
-        ops.gemm(u, x, self.w_up, exact=exact)
+        ops.gemm(u, x, self.w_up, exact=exact, scratch=ctx.scratch)
         if self.activation == "relu_squared":
             ops.weighted_relu_squared(act, u, dense, shared_weight, self.experts, self.ff, self.shared_ff, exact)
         else:
             g = ctx.scratch("experts_gate", (T, self.channels), self.rt.dtype)
-            ops.gemm(g, x, self.w_gate, exact=exact)
+            ops.gemm(g, x, self.w_gate, exact=exact, scratch=ctx.scratch)
             ops.clamped_glu(act, g, u, dense, self.experts, self.ff, self.shared_ff, self.limit, self.shared_limit, self.slope, exact, self.offset)
         if post is not None:
             apart = ctx.scratch("sub_out", tuple(residual.shape), torch.float32)
-            ops.gemm(apart, act, self.w_down, exact=exact)
+            ops.gemm(apart, act, self.w_down, exact=exact, scratch=ctx.scratch)
             ops.rmsnorm_add(residual, apart, *post, exact=exact)
             return
         if out is not None:
-            ops.gemm(out, act, self.w_down, exact=exact)
+            ops.gemm(out, act, self.w_down, exact=exact, scratch=ctx.scratch)
             if scale is not None:
                 out.mul_(scale)
             if passed is not None:
                 ops.add_row_scaled(out, x, passed, exact)
         elif scale is None:
-            ops.gemm(residual, act, self.w_down, add_to_out=True, exact=exact)
+            ops.gemm(residual, act, self.w_down, add_to_out=True, exact=exact, scratch=ctx.scratch)
             if passed is not None:
                 ops.add_row_scaled(residual, x, passed, exact)
         else:

@@ -83,9 +83,9 @@ class RecurrentMixer(Mixer):
         y = ctx.scratch("recurrent_gated", (o.shape[1], self.heads * self.dv), self.rt.dtype)
         ops.headnorm_gate(y, o, gate, weight, self.heads, self.dv, self.eps, self.rt.exact, parts=parts)
         if out is not None:
-            ops.gemm(out, y, self.w_o, exact=self.rt.exact)
+            ops.gemm(out, y, self.w_o, exact=self.rt.exact, scratch=ctx.scratch)
         else:
-            ops.gemm(residual, y, self.w_o, add_to_out=True, exact=self.rt.exact)
+            ops.gemm(residual, y, self.w_o, add_to_out=True, exact=self.rt.exact, scratch=ctx.scratch)
 
 
 class Retention(RecurrentMixer):
@@ -126,7 +126,7 @@ class Retention(RecurrentMixer):
     def forward(self, ctx, where, x, residual, out=None):
         T, kd, vd = x.shape[0], self.heads * self.dk, self.heads * self.dv
         proj = ctx.scratch("recurrent_proj", (T, 2 * kd + 2 * vd), self.rt.dtype)
-        ops.gemm(proj, x, self.w_in, exact=self.rt.exact)
+        ops.gemm(proj, x, self.w_in, exact=self.rt.exact, scratch=ctx.scratch)
         table = self.position.table(ctx.n_positions) if self.position is not None else None
         if self.position is None:
             pass
@@ -167,9 +167,9 @@ class GatedLinearAttention(RecurrentMixer):
     def forward(self, ctx, where, x, residual, out=None):
         T, kd, vd = x.shape[0], self.heads * self.dk, self.heads * self.dv
         proj = ctx.scratch("recurrent_proj", (T, 2 * kd + 2 * vd + self.rank), self.rt.dtype)
-        ops.gemm(proj, x, self.w_in, exact=self.rt.exact)
+        ops.gemm(proj, x, self.w_in, exact=self.rt.exact, scratch=ctx.scratch)
         z = ctx.scratch("recurrent_decay", (T, kd), torch.float32)
-        ops.gemm(z, proj[:, 2 * kd + 2 * vd:], self.w_a2, self.b_a2, exact=self.rt.exact)
+        ops.gemm(z, proj[:, 2 * kd + 2 * vd:], self.w_a2, self.b_a2, exact=self.rt.exact, scratch=ctx.scratch)
         o = self._readouts(ctx, T)
         parts = ops.linear_recurrence(o, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:2 * kd + vd], ctx.state(where), rows_of_requests(ctx),
                                       self.heads, self.dk, self.dv, ops.DECAY_SIGMOID_ROOT, z, tau=self.tau, q_scale=self.q_scale)
@@ -200,7 +200,7 @@ class LightningAttention(RecurrentMixer):
     def forward(self, ctx, where, x, residual, out=None):
         T, kd, vd = x.shape[0], self.heads * self.dk, self.heads * self.dv
         proj = ctx.scratch("recurrent_proj", (T, 2 * kd + 2 * vd), self.rt.dtype)
-        ops.gemm(proj, x, self.w_in, exact=self.rt.exact)
+        ops.gemm(proj, x, self.w_in, exact=self.rt.exact, scratch=ctx.scratch)
         qkv = proj[:, :2 * kd + vd]
         ops.activation(qkv, qkv, ops.SILU, exact=self.rt.exact)
         o = self._readouts(ctx, T)
@@ -209,9 +209,9 @@ class LightningAttention(RecurrentMixer):
         y = ctx.scratch("recurrent_gated", (T, vd), self.rt.dtype)
         ops.headnorm_gate(y, o, proj[:, 2 * kd + vd:], self.norm, 1, vd, self.eps, self.rt.exact, parts=parts, gate_kind="sigmoid")
         if out is not None:
-            ops.gemm(out, y, self.w_o, exact=self.rt.exact)
+            ops.gemm(out, y, self.w_o, exact=self.rt.exact, scratch=ctx.scratch)
         else:
-            ops.gemm(residual, y, self.w_o, add_to_out=True, exact=self.rt.exact)
+            ops.gemm(residual, y, self.w_o, add_to_out=True, exact=self.rt.exact, scratch=ctx.scratch)
 
 
 class GateMaximum(Mixer):
@@ -266,9 +266,9 @@ class MatrixMemory(RecurrentMixer):
         entry, k = where if isinstance(where, tuple) else (where, 0)
         exact, rows = self.rt.exact, rows_of_requests(ctx)
         proj = ctx.scratch("recurrent_proj", (T, 2 * kd + 2 * vd), self.rt.dtype)
-        ops.gemm(proj, x, self.w_in, exact=exact)
+        ops.gemm(proj, x, self.w_in, exact=exact, scratch=ctx.scratch)
         z = ctx.scratch("memory_gate_z", (T, 2 * H), torch.float32)
-        ops.gemm(z, x, self.w_gates, self.b_gates, exact=exact)
+        ops.gemm(z, x, self.w_gates, self.b_gates, exact=exact, scratch=ctx.scratch)
         gates = ctx.scratch("memory_gates", (3, T, H), torch.float32)
         ops.gate_scan(gates, z, ctx.state((entry, k + 1)), rows, H, self.cap)
         qf, kf = ctx.scratch("memory_q", (T, kd), torch.float32), ctx.scratch("memory_k", (T, kd), torch.float32)
@@ -279,9 +279,9 @@ class MatrixMemory(RecurrentMixer):
         y = ctx.scratch("recurrent_gated", (T, vd), self.rt.dtype)
         ops.headnorm_gate(y, o, proj[:, 2 * kd + vd:], self.norm, H, self.dv, self.eps, exact, parts=parts, gate_kind="sigmoid", extra=1, floor=gates[2])
         if out is not None:
-            ops.gemm(out, y, self.w_o, exact=exact)
+            ops.gemm(out, y, self.w_o, exact=exact, scratch=ctx.scratch)
         else:
-            ops.gemm(residual, y, self.w_o, add_to_out=True, exact=exact)
+            ops.gemm(residual, y, self.w_o, add_to_out=True, exact=exact, scratch=ctx.scratch)
 
 
 class ConvTail(Mixer):
@@ -337,7 +337,7 @@ class StateSpace(RecurrentMixer):
         entry, k = where if isinstance(where, tuple) else (where, 0)
         exact, rows = self.rt.exact, rows_of_requests(ctx)
         proj = ctx.scratch("recurrent_proj", (T, self.w_in.shape[0]), self.rt.dtype)
-        ops.gemm(proj, x, self.w_in, exact=exact)
+        ops.gemm(proj, x, self.w_in, exact=exact, scratch=ctx.scratch)
         z, raw, dt = proj[:, :inner], proj[:, inner:inner + self.conv_width], proj[:, inner + self.conv_width:inner + self.conv_width + H]
         xbc = ctx.scratch("state_space_conv", (T, self.conv_width), self.rt.dtype)
         qf, kf = ctx.scratch("memory_q", (T, H * N), torch.float32), ctx.scratch("memory_k", (T, H * N), torch.float32)
@@ -358,9 +358,9 @@ class StateSpace(RecurrentMixer):
         y = ctx.scratch("recurrent_gated", (T, inner), self.rt.dtype)
         ops.ssd_finish(y, o, xbc[:, :inner], z, self.skip, self.norm, H, dv, self.norm_parts, self.eps, exact, parts=parts)
         if out is not None:
-            ops.gemm(out, y, self.w_o, exact=exact)
+            ops.gemm(out, y, self.w_o, exact=exact, scratch=ctx.scratch)
         else:
-            ops.gemm(residual, y, self.w_o, add_to_out=True, exact=exact)
+            ops.gemm(residual, y, self.w_o, add_to_out=True, exact=exact, scratch=ctx.scratch)
 
 
 MIXES = ("r", "k", "v", "g", "w")
@@ -433,12 +433,12 @@ class TimeMix(RecurrentMixer):
         self.shift.forward(ctx, (entry, k + 1), mixes, x)
         proj = ctx.scratch("time_mix_proj", (T, 4 * kd), self.rt.dtype)
         for i, n in enumerate(("r", "k", "v", "g")):
-            ops.gemm(proj[:, i * kd:(i + 1) * kd], mixes[i], self.w[n], exact=exact)
+            ops.gemm(proj[:, i * kd:(i + 1) * kd], mixes[i], self.w[n], exact=exact, scratch=ctx.scratch)
         low = ctx.scratch("time_mix_low", (T, self.rank), self.rt.dtype)
-        ops.gemm(low, mixes[4], self.w["w1"], exact=exact)
+        ops.gemm(low, mixes[4], self.w["w1"], exact=exact, scratch=ctx.scratch)
         ops.activation(low, low, ops.TANH, exact=exact)
         z = ctx.scratch("recurrent_decay", (T, kd), torch.float32)
-        ops.gemm(z, low, self.w["w2"], self.w0, exact=exact)
+        ops.gemm(z, low, self.w["w2"], self.w0, exact=exact, scratch=ctx.scratch)
         o = self._readouts(ctx, T)
         parts = ops.linear_recurrence(o, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:3 * kd], ctx.state((entry, k)), rows_of_requests(ctx),
                                       self.heads, self.dk, self.dv, ops.DECAY_EXP_NEG_EXP, z, bonus=self.bonus, before_update=True)

@@ -126,7 +126,7 @@ class TalkingAttention(Mixer):
         if kv.owner != self.owns:
             raise AlofaError("invalid_argument", "a layer with key and value projections owns its pages, one without reads another's", f"where={where} owns={self.owns}")
         proj = ctx.scratch("talking_proj", (T, self.w_in.shape[0]), self.rt.dtype)
-        ops.gemm(proj, x, self.w_in, exact=exact)
+        ops.gemm(proj, x, self.w_in, exact=exact, scratch=ctx.scratch)
         v_table = self.value_position.table(ctx.n_positions) if self.value_position is not None else None
         kc, vc = kv.tensors["k"], kv.tensors["v"]
         ops.turn_norm_write(proj[:, :self.qkv_width], ctx.positions, self.position.table(ctx.n_positions), v_table, self.heads,
@@ -140,9 +140,9 @@ class TalkingAttention(Mixer):
             ops.talking_attention(attn, proj[:, :self.q_width], kc, vc, kv.block_table, ctx.req_of_token, ctx.positions, self.heads, self.kv_heads,
                                   self.d, self.dv, self.window, self.scale, self.talk, v_table, gate, exact)
         if out is not None:
-            ops.gemm(out, attn, self.w_o, exact=exact)
+            ops.gemm(out, attn, self.w_o, exact=exact, scratch=ctx.scratch)
         else:
-            ops.gemm(residual, attn, self.w_o, add_to_out=True, exact=exact)
+            ops.gemm(residual, attn, self.w_o, add_to_out=True, exact=exact, scratch=ctx.scratch)
 
 
 register_part("mixer", "talking_attention", TalkingAttention)

@@ -213,7 +213,7 @@ class WindowAttention(Mixer):
         kv = ctx.kv((entry, k))
         H, G, D = self.heads, self.kv_heads, self.d
         proj = ctx.scratch("window_proj", (T, self.w_in.shape[0]), self.rt.dtype)
-        ops.gemm(proj, x, self.w_in, exact=exact)
+        ops.gemm(proj, x, self.w_in, exact=exact, scratch=ctx.scratch)
         table = self.position.table(ctx.n_positions) if self.position is not None else None
         factors = ctx.scratch("window_row_factors", (T, 2), torch.float64) if self.scope == ops.NORM_ALL else None
         # (the norms average over the channels the design has: the widened ones are zeros and are not counted)
@@ -247,9 +247,9 @@ class WindowAttention(Mixer):
             ops.span_attention(attn, proj[:, :H * D], kv.k, kv.v, kv.block_table, ctx.req_of_token, ctx.positions, H, G, D, D, self.window, self.scale, exact,
                                pooled=pooled, bias=self.bias, sink=self.sink, gate=gate, gate_kind=kind)
         if out is not None:
-            ops.gemm(out, attn, self.w_o, exact=exact)
+            ops.gemm(out, attn, self.w_o, exact=exact, scratch=ctx.scratch)
         else:
-            ops.gemm(residual, attn, self.w_o, add_to_out=True, exact=exact)
+            ops.gemm(residual, attn, self.w_o, add_to_out=True, exact=exact, scratch=ctx.scratch)
 
 
 register_part("mixer", "window_attention", WindowAttention)

@@ -173,3 +173,25 @@ def test_a_row_of_exact_attention_does_not_depend_on_the_others(heads, kv_heads,
     want = attend(slice(0, rows))
     for first, n in ((0, 1), (299, 1), (5, 8), (17, 100), (100, 200)):
         assert torch.equal(attend(slice(first, first + n)), want[first:first + n])
+
+
+def test_sums_of_chains_lie_in_the_callers_buffers(tiny_dirs):
+    a, w, out = torch.ones(64, 4864, device=DEV), torch.ones(896, 4864, device=DEV), torch.empty(64, 896, device=DEV)
+    room, asked = torch.empty(1 << 23, dtype=torch.float64, device=DEV), []
+
+    def scratch(name, shape, dtype):
+        asked.append((name, dtype))
+        return room[:shape[0]]
+    ops().gemm(out, a, w, exact=True)
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    ops().gemm(out, a, w, exact=True, scratch=scratch)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] == before and asked == [("product_sums", torch.float64)] and bool((out == 4864).all())
+    # an engine's steps, cut kernel by kernel and captured: the sums are among the buffers that its account of memory counts
+    from alofa_amd.replay import Replayer
+    r = Replayer(tiny_dirs["D"], "float32", 128)
+    r.step({"step": 0, "entries": [{"id": "a", "tokens": list(range(20)), "want": []}], "end": []})
+    for i in range(2):
+        r.step({"step": 1 + i, "entries": [{"id": "a", "tokens": [7], "want": [0]}], "end": ["a"] if i else []})
+    fn = r.fn
+    eager, captured = fn._eager_scratch["product_sums", torch.float64], fn._graph_buffers[1]["scratch"]["product_sums", torch.float64]
+    assert fn.graph_replays == 1 and fn.scratch_bytes() > 8 * (eager.numel() + captured.numel())
