@@ -361,6 +361,12 @@ def _norm_operands(a: torch.Tensor, norm: tuple, K: int):
     return _ptr(weight), _F(eps)
 
 
+def _exact_operands(**operands) -> None:
+    for name, t in operands.items():
+        if t.dtype is not torch.float32:
+            raise AlofaError("invalid_argument", "the exact path takes float32 operands only", f"operand={name} dtype={t.dtype}")
+
+
 def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
          add_to_out: bool = False, exact: bool = False, kernel: Optional[str] = None, norm: Optional[tuple] = None,
          then_norm: Optional[tuple] = None, scratch=None) -> None:
@@ -428,7 +434,8 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[tor
         if then_rows is not None and not done.value:
             rmsnorm(then_rows, out, then_w, then_eps, False)
         return
-    if exact and a.dtype is torch.float32 and w.dtype is torch.float32 and out.dtype is torch.float32:
+    if exact:
+        _exact_operands(a=a, w=w, out=out)
         room = load().alofa_gemm_exact_parts(_I(M), _I(N), _I(K))      # (sums of the chains of K, where the tiles are too few for the chip)
         parts = None
         if room:
@@ -440,7 +447,7 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[tor
         return
     _call("alofa_gemm_simple", _ptr(out), _I(dtype_code(out)), _L(_rows("out", out)), _ptr(a), _I(dtype_code(a)), _L(_rows("a", a)),
           _ptr(w), _I(dtype_code(w)), _L(_rows("w", w)), _ptr(bias), _I(M), _I(N), _I(K),
-          _I(ADD_TO_RESIDUAL if add_to_out else STORE), _I(int(exact)), _stream())
+          _I(ADD_TO_RESIDUAL if add_to_out else STORE), _stream())
     if then_rows is not None:
         rmsnorm(then_rows, out, then_w, then_eps, exact)
 
@@ -471,12 +478,13 @@ def gemm_swiglu(out: torch.Tensor, a: torch.Tensor, w_gate: torch.Tensor, w_up: 
         _call(_product_entry(kernel, M, 2 * N, K, True, normed=True), _ptr(out), _I(BF16), _L(_rows("out", out)), _ptr(a), _L(_rows("a", a)), _ptr(w_gate), _ptr(w_up),
               _L(_rows("w_gate", w_gate)), _ptr(None), _I(M), _I(N), _I(K), _I(GATED[act]), *_norm_operands(a, norm, K), _stream())
         return
-    if exact and a.dtype is torch.float32 and w_gate.dtype is torch.float32 and out.dtype is torch.float32:
+    if exact:
+        _exact_operands(a=a, w_gate=w_gate, w_up=w_up, out=out)
         _call("alofa_gemm_swiglu_exact", _ptr(out), _L(_rows("out", out)), _ptr(a), _L(_rows("a", a)), _ptr(w_gate), _ptr(w_up), _L(_rows("w_gate", w_gate)),
               _I(M), _I(N), _I(K), _I(int(act == "gelu_tanh")), _stream())
         return
     _call("alofa_gemm_swiglu_simple", _ptr(out), _I(dtype_code(out)), _L(_rows("out", out)), _ptr(a), _I(dtype_code(a)), _L(_rows("a", a)),
-          _ptr(w_gate), _ptr(w_up), _I(dtype_code(w_gate)), _L(_rows("w_gate", w_gate)), _I(M), _I(N), _I(K), _I(int(act == "gelu_tanh")), _I(int(exact)), _stream())
+          _ptr(w_gate), _ptr(w_up), _I(dtype_code(w_gate)), _L(_rows("w_gate", w_gate)), _I(M), _I(N), _I(K), _I(int(act == "gelu_tanh")), _stream())
 
 
 def swiglu(out: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, exact: bool = False) -> None:

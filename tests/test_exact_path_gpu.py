@@ -195,3 +195,15 @@ def test_sums_of_chains_lie_in_the_callers_buffers(tiny_dirs):
     fn = r.fn
     eager, captured = fn._eager_scratch["product_sums", torch.float64], fn._graph_buffers[1]["scratch"]["product_sums", torch.float64]
     assert fn.graph_replays == 1 and fn.scratch_bytes() > 8 * (eager.numel() + captured.numel())
+
+
+def test_exact_products_name_the_operand_that_is_not_float32():
+    from alofa_amd.errors import AlofaError
+    f, h = torch.ones(8, 64, device=DEV), torch.ones(8, 64, device=DEV, dtype=torch.bfloat16)
+    out = torch.empty(8, 8, device=DEV)
+    for operands, name in (((out, h, f), "operand=a"), ((out, f, h), "operand=w"), ((out.bfloat16(), f, f), "operand=out")):
+        with pytest.raises(AlofaError, match=name):
+            ops().gemm(*operands, exact=True)
+    for operands, name in (((out, h, f, f), "operand=a"), ((out, f, h, h), "operand=w_gate"), ((out.bfloat16(), f, f, f), "operand=out")):
+        with pytest.raises(AlofaError, match=name):
+            ops().gemm_swiglu(*operands, exact=True)
