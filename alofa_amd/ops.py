@@ -7,6 +7,7 @@ from __future__ import annotations
 import ctypes
 import operator
 import os
+import sys
 from typing import Optional
 
 import torch
@@ -92,10 +93,16 @@ _binding = None
 
 
 def _native():
-    """The binding (csrc/host/binding): the calls themselves and the checks of the operations that every layer runs."""
+    """The binding (csrc/host/binding): the calls themselves and the checks of the operations that every layer runs. Where it can be neither
+    found nor built, ctypes and the checks in Python do the same, more slowly; a line says so once."""
     global _binding
     if _binding is None:
-        _binding = load_binding()
+        try:
+            _binding = load_binding()
+        except AlofaError as e:
+            from .csrc import calls
+            print(f"[alofa_amd] every launch takes some 10 us longer, by way of ctypes: {e}", file=sys.stderr, flush=True)
+            _binding = calls
     return _binding
 
 

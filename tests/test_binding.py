@@ -1,5 +1,6 @@
 """The binding: the calls of C entries, and the operand checks in front of them against the same rules written out here."""
 import ctypes
+import re
 import shutil
 import subprocess
 
@@ -7,6 +8,7 @@ import pytest
 import torch
 
 from alofa_amd import ops
+from alofa_amd.csrc import build, calls
 from alofa_amd.csrc.build import load_binding
 from alofa_amd.errors import AlofaError
 
@@ -146,3 +148,70 @@ def test_operands_of_attention_norm_and_rotation_are_told_apart_as_the_rules_say
         assert n.turn(*args, k, v, 4, 2, 64) is None
         with pytest.raises(AlofaError):
             ops.rope_kv_write(*args[:4], 4, 2, 64, args[4], k, v)
+
+
+def test_without_the_binding_ctypes_passes_the_same(entries):
+    assert calls.call(entries("mixed"), 1, 0.5, -2, None, 3, -4, 5, 1 << 40, 1.5, -7, 8, -2.5) == 1
+    assert calls.call(entries("nothing")) == -3
+    assert calls.call(entries("floats"), 1.0, 2.0, 3.0, 4.0, 5.0, 6.0, 7.0, 8.0, -9) == 1
+    assert calls.call(entries("many"), *range(-20, 28)) == 48
+    assert calls.call(entries("memory"), torch.arange(5, dtype=torch.float32), 5) == 10
+    for args, error in (((0,), ValueError), ((entries("nothing"), "x"), TypeError), ((entries("nothing"), 1 << 70), OverflowError)):
+        with pytest.raises(error):
+            calls.call(*args)
+
+
+def test_a_binding_that_cannot_be_built_is_done_without(monkeypatch, capsys):
+    def refuse():
+        raise AlofaError("not_initialized", "no C++ compiler was found; the binding cannot be built")
+    monkeypatch.setattr(build, "_binding", None)
+    monkeypatch.setattr(build, "find_built_binding", lambda: None)
+    monkeypatch.setattr(build, "build_binding", refuse)
+    monkeypatch.setattr(ops, "_binding", None)
+    assert ops._native() is calls and "no C++ compiler" in capsys.readouterr().err
+    t = torch.zeros(4, 16, dtype=torch.bfloat16)
+    with pytest.raises(AlofaError) as e:      # the check that says a tensor is not on the GPU needs no binding
+        ops.gemm(t, t, t)
+    assert e.value.name == "invalid_argument" and "GPU tensor" in str(e.value)
+
+
+def test_every_entry_can_be_called():
+    """The one signature behind ``call``: at most 48 integers and pointers, at most eight floats, and no double (it would be passed as a float)."""
+    seen = 0
+    for source in build.sources():
+        for name, parameters in re.findall(r'extern "C" [\w ]+?\b(alofa_\w+)\(([^)]*)\)', source.read_text()):
+            kinds = [re.sub(r"\b\w+$", "", p.strip()) for p in parameters.split(",") if p.strip()]
+            floats = [k for k in kinds if "*" not in k and "float" in k]
+            assert not any("double" in k and "*" not in k for k in kinds), name
+            assert len(floats) <= 8 and len(kinds) - len(floats) <= 48, name
+            seen += 1
+    assert seen > 50
+
+
+@pytest.mark.gpu
+def test_without_the_binding_the_results_are_the_same(monkeypatch):
+    dev = "cuda"
+    gen = torch.Generator(device=dev).manual_seed(1)
+
+    def results():
+        gen.manual_seed(1)
+        rand = lambda *s: torch.randn(*s, generator=gen, device=dev)      # noqa: E731
+        a, w, w2, x = rand(70, 256).bfloat16(), rand(192, 256).bfloat16(), rand(192, 256).bfloat16(), rand(70, 192)
+        out, gated, normed = torch.empty(70, 192, device=dev), torch.empty(70, 192, device=dev, dtype=torch.bfloat16), torch.empty(70, 192, device=dev, dtype=torch.bfloat16)
+        ops.gemm(out, a, w, rand(192))
+        ops.gemm_swiglu(gated, a, w, w2)
+        ops.gemm(x, a, w, add_to_out=True, then_norm=(rand(192), 1e-6, normed))
+        exact = torch.empty(70, 192, device=dev)
+        ops.gemm(exact, a.float(), w.float(), exact=True)
+        kc, vc = rand(5, 1, 16, 64).bfloat16(), rand(5, 1, 64, 16).bfloat16()
+        qkv, cos = rand(70, 6 * 64).bfloat16(), rand(80, 32)
+        at, slots = torch.arange(70, dtype=torch.int32, device=dev), torch.arange(70, dtype=torch.int64, device=dev)
+        ops.rope_kv_write(qkv, cos, cos, at, 4, 1, 64, slots, kc, vc)
+        attn, table = torch.empty(70, 256, device=dev, dtype=torch.bfloat16), torch.arange(5, dtype=torch.int32, device=dev)[None]
+        tiles = torch.tensor(ops.pair_tiles([(0, 0, 64, 0), (0, 64, 6, 64)]), dtype=torch.int32, device=dev)
+        ops.attention_prefill(attn, qkv[:, :256], kc, vc, table, tiles, 4, 1, 64, None, 0.125)
+        return [out, gated, x, normed, exact, qkv, kc, vc, attn]
+    want = results()
+    monkeypatch.setattr(ops, "_binding", calls)
+    for got, expected in zip(results(), want):
+        assert torch.equal(got, expected)
