@@ -62,9 +62,12 @@ __global__ void __launch_bounds__(512) attention_tall_kernel(bf16_t* __restrict_
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   const int r32 = lane % 32, h = lane / 32;
   const int group = heads / kv_heads;
-  // die b % 8 takes one contiguous stretch of the blocks in the order key head, run, head of the group
+  // die b % 8 takes one contiguous stretch of the blocks in the order key head, run, head of the group; where that cuts a key head's blocks over several dies, each of them takes every
+  // so-manieth run, else one had all the longest
   const int total = gridDim.x, die = blockIdx.x % 8, at = die * (total / 8) + min(die, total % 8) + blockIdx.x / 8;
-  const int hk = at / (n_runs * group), run = at % (n_runs * group) / group, head = hk * group + at % group;
+  const int hk = at / (n_runs * group), place = at % (n_runs * group) / group, head = hk * group + at % group;
+  const int dies = 8 % kv_heads == 0 ? 8 / kv_heads : 1, each = n_runs / dies, larger = n_runs % dies * (each + 1);      // (the first dies of a key head may have a run more)
+  const int run = place < larger ? place % (each + 1) * dies + place / (each + 1) : (place - larger) % each * dies + n_runs % dies + (place - larger) / each;
   const int req = runs[4 * run], row0 = runs[4 * run + 1], n_rows = runs[4 * run + 2], pos0 = runs[4 * run + 3];
   const int32_t* table = block_table + static_cast<int64_t>(req) * max_blocks;
   const int my_row = wave * 32 + r32;

@@ -1272,6 +1272,24 @@ def test_attention_of_many_rows(heads, kv_heads, bs, window):
     assert torch.equal(again, out)
 
 
+# a key head's blocks on eight, four and two dies, each of which takes every so-manieth run: runs that come out even over the dies and that don't; every run as in a launch of its own
+@pytest.mark.parametrize("heads,kv_heads", [(3, 1), (4, 2), (8, 4), (6, 3)])
+@pytest.mark.parametrize("n_runs", [2, 3, 5, 8, 13])
+def test_every_run_of_many_rows_is_served_once(heads, kv_heads, n_runs):
+    d, bs, n, history = 128, 16, 70, 30
+    gen = torch.Generator(device=DEV).manual_seed(n_runs)
+    per = -(-(n + history) // bs)
+    q = torch.randn(n_runs * n, heads * d, generator=gen, device=DEV).bfloat16()
+    kc, vc = (torch.randn(n_runs * per, kv_heads, *page, generator=gen, device=DEV).bfloat16() for page in ((bs, d), (d, bs)))
+    table = torch.arange(n_runs * per, dtype=torch.int32, device=DEV).view(n_runs, per).contiguous()
+    runs = torch.tensor([(r, r * n, n - r, history) for r in range(n_runs)], dtype=torch.int32, device=DEV)
+    out, alone = (torch.full((n_runs * n, heads * d), 7.0, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    ops().attention_tall(out, q, kc, vc, table, runs, heads, kv_heads, d, None, d ** -0.5)
+    for r in range(n_runs):
+        ops().attention_tall(alone, q, kc, vc, table, runs[r:r + 1], heads, kv_heads, d, None, d ** -0.5)
+    assert torch.equal(out, alone) and int((out != 7).any(1).sum()) == sum(n - r for r in range(n_runs))
+
+
 # which launches take the blocks of 256 rows (256 compute units): enough full runs; runs of few rows, however many; runs half full, with and without tiles that heads share, on few keys and on many
 @pytest.mark.parametrize("heads,kv_heads,portions,taken", [(40, 8, [(2048, 2048)], True), (12, 2, [(2048, 2048)], False), (28, 4, [(480, 1000)] * 4, True), (28, 4, [(5, 2053)] * 48, False),
                                                            (28, 4, [(17, 17)] * 48, False), (40, 8, [(64, 2112)] * 48, False), (40, 8, [(33, 8225)] * 4, False), (28, 4, [(96, 608)] * 16, True),
