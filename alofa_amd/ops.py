@@ -897,7 +897,7 @@ def pair_tiles(runs: list, window: Optional[int] = None, heads: Optional[int] = 
 TALL_ROWS = 256     # query rows a block of the attention kernel for many rows serves
 
 
-def attention_tall_pays(heads: int, kv_heads: int, d: int, block_size: int, scale: float, portions: list) -> bool:
+def attention_tall_pays(heads: int, kv_heads: int, d: int, block_size: int, scale: float, portions: list, window: Optional[int] = None) -> bool:
     """Whether ``portions``, (rows brought, keys that the last of them sees) each, go to the kernel with blocks of ``TALL_ROWS`` query rows of one head:
     heads of 128, pages of 16 tokens or more, blocks for five eighths of the compute units, and runs that are full enough. us, the kernel with blocks of
     64 rows / this. Full runs: 28/4 heads, four portions of some 480 rows on 256 to 1,536 keys (224 blocks) 79 / 61, 16/16 heads, three prompts of 1,024 (192
@@ -906,14 +906,24 @@ def attention_tall_pays(heads: int, kv_heads: int, d: int, block_size: int, scal
     Runs of few rows: a block of this kernel fills a compute unit whatever its rows, and a wave walks all keys alone. 28/4 heads on 2,048 keys, 48 portions of 5 rows
     132 / 226, of 17 135 / 234, 8 of 64 42 / 43; 40/8 heads, 48 of 64 295 / 336; from 96 rows a run on it is ahead (28/4 heads, 8 of 96 79 / 58; 40/8 heads, 48 of 96 on
     512 keys 169 / 157), but where the heads of a group share the other kernel's tiles and the keys are few only from 150 on: 28/4 heads without history, 48 of 96 rows 39 / 47, 8 of
-    257 (128 a run) 29 / 32, 16 of 300 62 / 59; on 512 keys 8 of 257 73 / 57."""
+    257 (128 a run) 29 / 32, 16 of 300 62 / 59; on 512 keys 8 of 257 73 / 57.
+    A ``window`` of fewer than 512 keys: a block of a few rows takes nearly as long as a whole one. In one round, runs of less than half the rows beside whole ones don't count towards the
+    blocks that it takes, unless the other kernel's blocks are more than two rounds (28/4 heads, window 128, 3 of 300 rows 19.5 / 21.6; 24/2, 4 of 300 19.6 / 21.6, 4 of 360 35 / 21; 28/4, 6 of 300 45 / 41);
+    and whole runs of which the last round has few lose against tiles that heads share, windows under 256 (28/4, 128, 12 of 256 45 / 49, 6 of 512 45 / 49, 3 of 1,500 66 / 53)."""
     if d != 128 or block_size < 16 or not scale > 0:
         return False
     runs, rows = sum(-(-n // TALL_ROWS) for n, _ in portions), sum(n for n, _ in portions)
-    if runs * heads * 8 < 5 * compute_units() or rows < 96 * runs:
+    cus, pieces = compute_units(), sum(-(-n // 64) for n, _ in portions)
+    if runs * heads * 8 < 5 * cus or rows < 96 * runs:
         return False
+    if window and window < 512:
+        whole = sum(max(1, (n + TALL_ROWS // 2) // TALL_ROWS) for n, _ in portions)
+        if whole * heads * 8 < 5 * cus and pieces * heads <= 2 * cus:
+            return False
+        if window < 256 and rows >= 225 * runs and 5 * pieces * heads < 16 * cus * -(-runs * heads // cus) and prefill_share(heads, kv_heads, d, pieces):
+            return False
     few_keys = sum(keys for _, keys in portions) < 512 * len(portions)
-    return not (few_keys and rows < 150 * runs and prefill_share(heads, kv_heads, d, sum(-(-n // 64) for n, _ in portions)))
+    return not (few_keys and rows < 150 * runs and prefill_share(heads, kv_heads, d, pieces))
 
 
 def attention_tall(out, q, k_cache, v_cache, block_table, runs, heads, kv_heads, d, window, scale) -> None:

@@ -44,11 +44,11 @@ class RowPlan:
             if self.n_short:
                 self.short_rows = ops.upload([r for s in spans if s.n <= SHORT for r in range(s.row0, s.row0 + s.n)], self.device)
 
-    def in_tall_blocks(self, heads: int, kv_heads: int, d: int, block_size: int, scale: float) -> bool:
+    def in_tall_blocks(self, heads: int, kv_heads: int, d: int, block_size: int, scale: float, window) -> bool:
         """Whether the long portions go to the kernel with blocks of ``ops.TALL_ROWS`` rows for a mixer with these head counts."""
-        key = (heads, kv_heads, d, block_size, scale)
+        key = (heads, kv_heads, d, block_size, scale, window)
         if key not in self._tall:
-            self._tall[key] = ops.attention_tall_pays(*key, [(s.n, s.pos0 + s.n) for s in self.spans if s.n > SHORT])
+            self._tall[key] = ops.attention_tall_pays(*key[:-1], [(s.n, s.pos0 + s.n) for s in self.spans if s.n > SHORT], window)
         return self._tall[key]
 
     def tall_runs(self):
@@ -109,7 +109,7 @@ def paged_attend(ctx, entry, qkv, attn, heads, kv_heads, d, window, scale, posit
         # the exact path, and page or head sizes the bfloat16 kernels are not built for
         ops.paged_attention(attn, qkv, kv.k, kv.v, kv.block_table, ctx.req_of_token, ctx.positions, *common, exact)
     else:
-        if plan.long_runs is not None and plan.in_tall_blocks(heads, kv_heads, d, kv.k.shape[2], scale):      # portions of prompts, many rows
+        if plan.long_runs is not None and plan.in_tall_blocks(heads, kv_heads, d, kv.k.shape[2], scale, window):      # portions of prompts, many rows
             ops.attention_tall(attn, qkv, kv.k, kv.v, kv.block_table, ctx.memo("gqa_attention.tall_runs", plan.tall_runs), *common)
         elif plan.long_runs is not None:      # portions of prompts
             tiles, share, rows = plan.tiles(heads, kv_heads, d, window)

@@ -1302,6 +1302,15 @@ def test_which_portions_the_blocks_of_many_rows_take(heads, kv_heads, portions, 
     assert not ops().attention_tall_pays(heads, kv_heads, 64, 16, 0.125, portions) and not ops().attention_tall_pays(heads, kv_heads, 128, 8, 0.1, portions)
 
 
+# windows of fewer keys than a run has rows and more: nearly empty runs beside whole ones in one round of the chip and in two, whole runs in one round and a part of another with and without tiles that heads share
+@pytest.mark.parametrize("heads,kv_heads,n,count,window,taken", [(28, 4, 300, 3, 128, False), (28, 4, 300, 3, 512, True), (28, 4, 300, 3, None, True), (28, 4, 300, 6, 128, True), (24, 2, 360, 4, 128, True), (24, 2, 300, 4, 255, False),
+                                                                  (28, 4, 96, 6, 128, True), (28, 4, 256, 12, 128, False), (28, 4, 256, 12, 256, True), (40, 8, 256, 8, 128, True), (28, 4, 1500, 3, 128, True), (16, 16, 300, 5, 48, False)])
+def test_which_windows_the_blocks_of_many_rows_take(heads, kv_heads, n, count, window, taken):
+    if ops().compute_units() != 256:
+        pytest.skip("the sizes are those of 256 compute units")
+    assert ops().attention_tall_pays(heads, kv_heads, 128, 16, 128 ** -0.5, [(n, n + 2048)] * count, window) == taken
+
+
 # sharper and sharper softmaxes: where one key counts, its weight is one exactly, and only the others' are rounded
 @pytest.mark.parametrize("heads,kv_heads,n,history", [(8, 2, 700, 900), (6, 6, 512, 0), (16, 2, 300, 3000)])
 @pytest.mark.parametrize("sharp", [1, 2, 4, 8, 16])
