@@ -97,7 +97,7 @@ __device__ __forceinline__ Pair8 rotate8(uint4 lo, uint4 hi, float4 c_lo, float4
   return Pair8{make_uint4(ra[0], ra[1], ra[2], ra[3]), make_uint4(rb[0], rb[1], rb[2], rb[3])};
 }
 
-// Heads of 128: two blocks to a compute unit (the rotary form's 295 registers fit 256 without a spill): us, one / two, 28/4 heads, 32 tokens of 128 to 1,028 keys 21.9 / 21.2,
+// Heads of 128: two blocks to a compute unit (the rotary form's 295 registers come out as 256 and five that are spilled): us, one / two, 28/4 heads, 32 tokens of 128 to 1,028 keys 21.9 / 21.2,
 // 48 of 64 to 512 16.0 / 15.6.
 // DT = d / 16; NW: waves per block. blockIdx.y = key head * chunks + chunk of up to `block_heads` (<= 16) heads of its group.
 // kSplit: a weight enters the second product as two bfloat16 numbers, its rounding and what the rounding took away: sixteen bits of every weight count.
@@ -559,115 +559,166 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
     });
     return;
   }
-  const int here = min(block_heads, group - h0);      // heads of this block
-  auto states_of = [&](int i) { return partial + (static_cast<int64_t>(blockIdx.x) * heads + hk * group + h0 + i) * n_parts * (d + 2); };
-  auto finish = [&](int i, int c, float big, float total, float acc, float s2) {
-    if (sink) total += __builtin_amdgcn_exp2f(s2 - big);
-    put_out(out, out32, static_cast<int64_t>(t) * out_stride + static_cast<int64_t>(hk * group + h0 + i) * d + c, acc / total);
-  };
-  auto sink_of = [&](int i) { return sink ? sink[hk * group + h0 + i] * 1.44269504088896340736f : -FLT_MAX; };
-  // Up to eight parts (more are handed over only on a caller's word): everything that is read sets out together, since the states come from memory, a round trip
-  // of more than a microsecond. Where eight heads are several outputs a thread (heads of 128: four) the parts' maxima and sums are read once for
-  // the block and meet in LDS, and the sums of all those outputs set out at once: us, one output's loads at a time / this, 28/4 heads of 128: one token, 600 keys
-  // in five parts 11.8 / 10.2, eight of 500 to 800 in seven 12.9 / 11.8, four of 2,000 in eight 16.5 / 15.5. Where they are one output a thread it reads its own
-  // maxima and sums too: by way of LDS 14/2 heads of 64 take 7.8 us where this takes 7.5 (one token, 520 keys).
-  constexpr int kOutputs = (8 * d + 64 * NW - 1) / (64 * NW);
-  if (kOutputs == 1 && n_parts <= 8) {
-    auto at_once = [&](auto count) __attribute__((always_inline)) {
-      constexpr int kCount = decltype(count)::value;
-      for (int x = threadIdx.x; x < here * d; x += 64 * NW) {
-        const int i = x / d;
-        const float* src = states_of(i);
-        const float s2 = sink_of(i);
-        float ms[kCount], ls[kCount], vs[kCount];
+  if constexpr (DT > 4 && DT != 8) {
+    // Sizes whose kernels fill their registers: an output at a time, up to sixteen parts' numbers asked for at once. By what follows heads of 256 spill 76 bytes a lane where this spills
+    // 56, and 24 tokens of 5,800 keys take 40.1 us where they take 37.5 so; 16/4 heads of 96, two tokens of 640 7.1 and 6.9.
+    for (int x = threadIdx.x; x < block_heads * d; x += 64 * NW) {
+      const int i = x / d, c = x % d;
+      if (h0 + i >= group) break;
+      const int head = hk * group + h0 + i;
+      const float* src = partial + (static_cast<int64_t>(blockIdx.x) * heads + head) * n_parts * (d + 2);
+      const float s2 = sink ? sink[head] * 1.44269504088896340736f : -FLT_MAX;
+      float big = s2, total = 0.f, acc = 0.f;
+      if (n_parts <= 16) {
+        auto at_once = [&](auto count) {
+          constexpr int kCount = decltype(count)::value;
+          float ms[kCount], ls[kCount], vs[kCount];
 #pragma unroll
-        for (int u = 0; u < kCount; ++u) {
-          const float* part = src + min(u, n_parts - 1) * (d + 2);
-          ms[u] = __hip_atomic_load(part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          ls[u] = __hip_atomic_load(part + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          vs[u] = __hip_atomic_load(part + 2 + x % d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        float big = s2, total = 0.f, acc = 0.f;
-#pragma unroll
-        for (int u = 0; u < kCount; ++u)
-          if (u < n_parts) big = fmaxf(big, ms[u]);
-#pragma unroll
-        for (int u = 0; u < kCount; ++u)
-          if (u < n_parts) {
-            const float e = __builtin_amdgcn_exp2f(ms[u] - big);
-            total += ls[u] * e;
-            acc += vs[u] * e;
+          for (int u = 0; u < kCount; ++u) {
+            const float* part = src + min(u, n_parts - 1) * (d + 2);
+            ms[u] = __hip_atomic_load(part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ls[u] = __hip_atomic_load(part + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            vs[u] = __hip_atomic_load(part + 2 + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           }
-        finish(i, x % d, big, total, acc, s2);
-      }
-    };
-    if (n_parts <= 4) at_once(std::integral_constant<int, 4>());
-    else at_once(std::integral_constant<int, 8>());
-    return;
-  }
-  if constexpr (kOutputs > 1) if (n_parts <= 8) {
-    float* ml = &state[0][0][0];      // [head][part][2]; (the waves' states have been read)
-    auto at_once = [&](auto count) __attribute__((always_inline)) {
-      constexpr int kCount = decltype(count)::value;
-      for (int base = 0; base < here * d; base += kOutputs * 64 * NW) {      // uniform over the block
-        float part_m = 0.f, part_l = 0.f;
-        if (base == 0 && static_cast<int>(threadIdx.x) < here * n_parts) {      // (at most 128 of them)
-          const float* part = states_of(threadIdx.x / n_parts) + threadIdx.x % n_parts * (d + 2);
-          part_m = __hip_atomic_load(part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          part_l = __hip_atomic_load(part + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        float vs[kOutputs][kCount];
-#pragma unroll
-        for (int n = 0; n < kOutputs; ++n) {
-          const int x = min(base + n * 64 * NW + static_cast<int>(threadIdx.x), here * d - 1);
-          const float* src = states_of(x / d) + 2 + x % d;
-#pragma unroll
-          for (int u = 0; u < kCount; ++u) vs[n][u] = __hip_atomic_load(src + min(u, n_parts - 1) * (d + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (base == 0) {
-          if (static_cast<int>(threadIdx.x) < here * n_parts) ml[2 * threadIdx.x] = part_m, ml[2 * threadIdx.x + 1] = part_l;
-          __syncthreads();
-        }
-#pragma unroll
-        for (int n = 0; n < kOutputs; ++n) {
-          const int x = base + n * 64 * NW + threadIdx.x;
-          if (x >= here * d) break;
-          const int i = x / d;
-          const float* heads_ml = ml + 2 * i * n_parts;
-          const float s2 = sink_of(i);
-          float big = s2, total = 0.f, acc = 0.f;
 #pragma unroll
           for (int u = 0; u < kCount; ++u)
-            if (u < n_parts) big = fmaxf(big, heads_ml[2 * u]);
+            if (u < n_parts) big = fmaxf(big, ms[u]);
 #pragma unroll
           for (int u = 0; u < kCount; ++u)
             if (u < n_parts) {
-              const float e = __builtin_amdgcn_exp2f(heads_ml[2 * u] - big);
-              total += heads_ml[2 * u + 1] * e;
-              acc += vs[n][u] * e;
+              const float e = __builtin_amdgcn_exp2f(ms[u] - big);
+              total += ls[u] * e;
+              acc += vs[u] * e;
+            }
+        };
+        if (n_parts <= 4) at_once(std::integral_constant<int, 4>());
+        else if (n_parts <= 8) at_once(std::integral_constant<int, 8>());
+        else at_once(std::integral_constant<int, 16>());
+      } else {
+        for (int sp = 0; sp < n_parts; ++sp) big = fmaxf(big, __hip_atomic_load(src + sp * (d + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+#pragma unroll 4
+        for (int sp = 0; sp < n_parts; ++sp) {
+          const float* part = src + sp * (d + 2);
+          const float e = __builtin_amdgcn_exp2f(__hip_atomic_load(part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - big);
+          total += __hip_atomic_load(part + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * e;
+          acc += __hip_atomic_load(part + 2 + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * e;
+        }
+      }
+      if (sink) total += __builtin_amdgcn_exp2f(s2 - big);
+      put_out(out, out32, static_cast<int64_t>(t) * out_stride + static_cast<int64_t>(head) * d + c, acc / total);
+    }
+    return;
+  } else {
+    const int here = min(block_heads, group - h0);      // heads of this block
+    auto states_of = [&](int i) { return partial + (static_cast<int64_t>(blockIdx.x) * heads + hk * group + h0 + i) * n_parts * (d + 2); };
+    auto finish = [&](int i, int c, float big, float total, float acc, float s2) {
+      if (sink) total += __builtin_amdgcn_exp2f(s2 - big);
+      put_out(out, out32, static_cast<int64_t>(t) * out_stride + static_cast<int64_t>(hk * group + h0 + i) * d + c, acc / total);
+    };
+    auto sink_of = [&](int i) { return sink ? sink[hk * group + h0 + i] * 1.44269504088896340736f : -FLT_MAX; };
+    // Up to eight parts (more are handed over only on a caller's word): everything that is read sets out together, since the states come from memory, a round trip
+    // of more than a microsecond. Where eight heads are four outputs a thread (heads of 128) the parts' maxima and sums are read once for
+    // the block and meet in LDS, and the sums of all those outputs set out at once: us, one output's loads at a time / this, 28/4 heads of 128: one token, 600 keys
+    // in five parts 11.8 / 10.2, eight of 500 to 800 in seven 12.9 / 11.8, four of 2,000 in eight 16.5 / 15.5. Where they are one output a thread it reads its own
+    // maxima and sums too: by way of LDS 14/2 heads of 64 take 7.8 us where this takes 7.5 (one token, 520 keys).
+    constexpr int kOutputs = (8 * d + 64 * NW - 1) / (64 * NW);
+    if (kOutputs == 1 && n_parts <= 8) {
+      auto at_once = [&](auto count) __attribute__((always_inline)) {
+        constexpr int kCount = decltype(count)::value;
+        for (int x = threadIdx.x; x < here * d; x += 64 * NW) {
+          const int i = x / d;
+          const float* src = states_of(i);
+          const float s2 = sink_of(i);
+          float ms[kCount], ls[kCount], vs[kCount];
+#pragma unroll
+          for (int u = 0; u < kCount; ++u) {
+            const float* part = src + min(u, n_parts - 1) * (d + 2);
+            ms[u] = __hip_atomic_load(part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ls[u] = __hip_atomic_load(part + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            vs[u] = __hip_atomic_load(part + 2 + x % d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+          float big = s2, total = 0.f, acc = 0.f;
+#pragma unroll
+          for (int u = 0; u < kCount; ++u)
+            if (u < n_parts) big = fmaxf(big, ms[u]);
+#pragma unroll
+          for (int u = 0; u < kCount; ++u)
+            if (u < n_parts) {
+              const float e = __builtin_amdgcn_exp2f(ms[u] - big);
+              total += ls[u] * e;
+              acc += vs[u] * e;
             }
           finish(i, x % d, big, total, acc, s2);
         }
-      }
-    };
-    if (n_parts <= 4) at_once(std::integral_constant<int, 4>());
-    else at_once(std::integral_constant<int, 8>());
-    return;
-  }
-  for (int x = threadIdx.x; x < here * d; x += 64 * NW) {
-    const int i = x / d, c = x % d;
-    const float* src = states_of(i);
-    const float s2 = sink_of(i);
-    float big = s2, total = 0.f, acc = 0.f;
-    for (int sp = 0; sp < n_parts; ++sp) big = fmaxf(big, __hip_atomic_load(src + sp * (d + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-#pragma unroll 4
-    for (int sp = 0; sp < n_parts; ++sp) {
-      const float* part = src + sp * (d + 2);
-      const float e = __builtin_amdgcn_exp2f(__hip_atomic_load(part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - big);
-      total += __hip_atomic_load(part + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * e;
-      acc += __hip_atomic_load(part + 2 + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * e;
+      };
+      if (n_parts <= 4) at_once(std::integral_constant<int, 4>());
+      else at_once(std::integral_constant<int, 8>());
+      return;
     }
-    finish(i, c, big, total, acc, s2);
+    if constexpr (kOutputs > 1) if (n_parts <= 8) {
+      float* ml = &state[0][0][0];      // [head][part][2]; (the waves' states have been read)
+      auto at_once = [&](auto count) __attribute__((always_inline)) {
+        constexpr int kCount = decltype(count)::value;
+        for (int base = 0; base < here * d; base += kOutputs * 64 * NW) {      // uniform over the block
+          float part_m = 0.f, part_l = 0.f;
+          if (base == 0 && static_cast<int>(threadIdx.x) < here * n_parts) {      // (at most 128 of them)
+            const float* part = states_of(threadIdx.x / n_parts) + threadIdx.x % n_parts * (d + 2);
+            part_m = __hip_atomic_load(part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            part_l = __hip_atomic_load(part + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+          float vs[kOutputs][kCount];
+#pragma unroll
+          for (int n = 0; n < kOutputs; ++n) {
+            const int x = min(base + n * 64 * NW + static_cast<int>(threadIdx.x), here * d - 1);
+            const float* src = states_of(x / d) + 2 + x % d;
+#pragma unroll
+            for (int u = 0; u < kCount; ++u) vs[n][u] = __hip_atomic_load(src + min(u, n_parts - 1) * (d + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+          if (base == 0) {
+            if (static_cast<int>(threadIdx.x) < here * n_parts) ml[2 * threadIdx.x] = part_m, ml[2 * threadIdx.x + 1] = part_l;
+            __syncthreads();
+          }
+#pragma unroll
+          for (int n = 0; n < kOutputs; ++n) {
+            const int x = base + n * 64 * NW + threadIdx.x;
+            if (x >= here * d) break;
+            const int i = x / d;
+            const float* heads_ml = ml + 2 * i * n_parts;
+            const float s2 = sink_of(i);
+            float big = s2, total = 0.f, acc = 0.f;
+#pragma unroll
+            for (int u = 0; u < kCount; ++u)
+              if (u < n_parts) big = fmaxf(big, heads_ml[2 * u]);
+#pragma unroll
+            for (int u = 0; u < kCount; ++u)
+              if (u < n_parts) {
+                const float e = __builtin_amdgcn_exp2f(heads_ml[2 * u] - big);
+                total += heads_ml[2 * u + 1] * e;
+                acc += vs[n][u] * e;
+              }
+            finish(i, x % d, big, total, acc, s2);
+          }
+        }
+      };
+      if (n_parts <= 4) at_once(std::integral_constant<int, 4>());
+      else at_once(std::integral_constant<int, 8>());
+      return;
+    }
+    for (int x = threadIdx.x; x < here * d; x += 64 * NW) {
+      const int i = x / d, c = x % d;
+      const float* src = states_of(i);
+      const float s2 = sink_of(i);
+      float big = s2, total = 0.f, acc = 0.f;
+      for (int sp = 0; sp < n_parts; ++sp) big = fmaxf(big, __hip_atomic_load(src + sp * (d + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+#pragma unroll 4
+      for (int sp = 0; sp < n_parts; ++sp) {
+        const float* part = src + sp * (d + 2);
+        const float e = __builtin_amdgcn_exp2f(__hip_atomic_load(part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - big);
+        total += __hip_atomic_load(part + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * e;
+        acc += __hip_atomic_load(part + 2 + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * e;
+      }
+      finish(i, c, big, total, acc, s2);
+    }
   }
 }
 
