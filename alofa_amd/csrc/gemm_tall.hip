@@ -233,16 +233,24 @@ static int pick_tall(int M, int N, int K, bool gated, double* fill) {
 // 896 x 2,560 against 3,432 44.3 / 31.2, 2,048 x 3,072 against 1,465 47.4 / 35.4.
 // Where tiles of 128 x 128 are more than one round of the chip, the others' K is not shared out and their second round is nearly empty, while 128 x 192 still come out in one: 11,008 x 4,096 against
 // 315 rows (174 tiles of 128 x 192) 82 / 56, 11,008 x 2,048 against 303 47 / 34, 4,224 x 3,584 against 957 (176) 64 / 47, 3,072 x 4,864 against 1,323 78 / 60, 3,072 x 2,560 against 1,385 51 / 38.
+// With K of 1,536 too: 8,960 x 1,536 against 397 rows (188) 35 / 27, 18,944 x 1,536 against 150 33 / 27, 3,584 x 1,536 against 1,710 (196 of 256 x 128) 34 / 31.
+// But not 256 x 160 where the others come out in two rounds and K is short or the last rows are mostly padding: 8,960 x 1,536 against 787 36 / 41, 18,944 x 2,048 against 269 44 / 47, 18,944 x 5,120
+// against 330 89 / 95 (4,608 x 1,792 against 1,907, 540 of 128 x 128, 56 / 42); nor one round of 128 x 128 with that much padding and K under 4,096: 8,960 x 1,536 against 265 (210) 18.0 / 21.0, x 3,584
+// 35.4 / 38.0, 13,824 x 2,048 against 140 (216) 21.6 / 25.1 (against 1,536 x 1,536, 2,073 rows, 25 / 22).
 bool tall_pays(int M, int N, int K, bool gated) {
   static const bool switched_off = [] { const char* e = getenv("ALOFA_WIDE_TILES"); return e != nullptr && e[0] == '0'; }();     // (for measurements)
   if (switched_off || M <= 64 || K % 32 != 0 || K < 1536) return false;
   double fill = 0;
-  pick_tall(M, N, K, gated, &fill);
-  if (K < 2048) return fill >= 0.80;
+  const int form = pick_tall(M, N, K, gated, &fill), cus = compute_units();
   if (!gated) {
-    if (static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128) > compute_units()) return true;
-    if (K < 8960 && static_cast<int64_t>(N) * K < 20000000) return fill >= 0.735;
+    const int64_t small = static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128);
+    const int full = (M + kPlain[form].rows - 1) / kPlain[form].rows * kPlain[form].rows;      // rows with the last tile's padding
+    if (kPlain[form].columns == 160 && small <= 2 * cus && (K <= 2048 || 4 * M < 3 * full)) return false;
+    if (kPlain[form].rows == 128 && kPlain[form].columns == 128 && small <= cus && K < 4096 && 5 * M < 4 * full) return false;
+    if (small > cus) return K >= 2048 || fill >= 0.72;
   }
+  if (K < 2048) return fill >= 0.80;
+  if (!gated && K < 8960 && static_cast<int64_t>(N) * K < 20000000) return fill >= 0.735;
   return fill >= (K < 3072 || (K < 5120 && !gated) ? 0.70 : 0.57);
 }
 

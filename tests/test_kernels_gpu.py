@@ -1232,6 +1232,16 @@ def test_which_products_the_forms_for_many_rows_take(M, N, K, gated, taken):
     assert load().alofa_gemm_wide_pays(M, N, K, gated) == taken
 
 
+# tiles of 128 x 128 that are a little more than one round of a short K; tiles of 256 x 160 where those come out in two rounds and in more; one round of 128 x 128 with much padding and with little
+@pytest.mark.parametrize("M,N,K,taken", [(397, 8960, 1536, 1), (150, 18944, 1536, 1), (1710, 3584, 1536, 1), (787, 8960, 1536, 0), (282, 18944, 1536, 0), (269, 18944, 2048, 0), (1907, 4608, 1792, 1), (1920, 4608, 2048, 1), (2355, 4096, 1536, 1),
+                                           (330, 18944, 5120, 0), (265, 8960, 1536, 0), (265, 8960, 3584, 0), (140, 13824, 2048, 0), (2073, 1536, 1536, 0), (3388, 1024, 1536, 1)])
+def test_which_ragged_products_the_forms_for_many_rows_take(M, N, K, taken):
+    from alofa_amd.csrc.build import load
+    if ops().compute_units() != 256:
+        pytest.skip("the sizes are those of 256 compute units")
+    assert load().alofa_gemm_wide_pays(M, N, K, 0) == taken
+
+
 # runs that end within a tile, within a wave's rows and at either's edge; one row; history in whole and ragged tiles; windows shorter than a tile, than a block and longer; larger pages
 @pytest.mark.parametrize("heads,kv_heads,bs,window", [(5, 1, 16, None), (4, 2, 16, 40), (16, 8, 64, 300), (3, 3, 32, None), (2, 1, 16, 1)])
 def test_attention_of_many_rows(heads, kv_heads, bs, window):
