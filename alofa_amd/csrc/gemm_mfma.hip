@@ -712,7 +712,7 @@ template <int kEpilogue, typename TO>
 static int launch_mfma(void* out, int64_t ldo, const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw,
                        const float* bias, int M, int N, int K, hipStream_t stream, const ThenNorm& then, int* then_done) {
   if constexpr (kEpilogue != kMfArgmax) {
-    if (tall_pays(M, N, K, is_gated(kEpilogue))) return launch_tall(kEpilogue, sizeof(TO) == 4 ? kF32 : kBF16, out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream);
+    if (tall_pays(M, N, K, is_gated(kEpilogue) ? kTallGated : sizeof(TO) == 2 ? kTallRows16 : kTallFloat)) return launch_tall(kEpilogue, sizeof(TO) == 4 ? kF32 : kBF16, out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream);
   }
   if constexpr (is_gated(kEpilogue)) {
     // A block computes gate and up of the same 64 columns. With K a multiple of 64 and tiles that do not fill the

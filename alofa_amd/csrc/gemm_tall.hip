@@ -17,6 +17,11 @@
 // 4,096 x 27,648 x 5,120 with the gate 2,132 us (tiles of 256 x 256, eight waves, slabs of 32, all waves in step) -> 2,029 (the groups half a
 // phase apart) -> 1,880 (slabs of 64 in two units) -> 1,765 (fetches between the products): 1.31 PFLOP/s.
 //
+// A tile's way out counts as much as its way in where K is short. bfloat16 outputs are written as whole lines of rows by way of LDS (rows_epilogue), the gate's division takes what its range needs
+// (common.h), and gate and up share a group of 32 rows of W eight and eight, so that any tile does for them: 4,864 x 896 with the gate against 2,048 rows 47.6 us (tiles of 128 x 64 of gemm_mfma.hip; 53.1
+// with 256 x 128 here) -> 40.3 (256 x 160, one round of the chip) -> 37.2 (the division); 8,960 x 1,536 against 2,048 133 -> 102, 18,944 x 3,584 against 1,970 460 -> 441, 27,648 x 5,120
+// against 4,096 1,797 -> 1,756; stored as bfloat16 7,168 x 5,120 against 4,096 266 -> 243, 4,608 x 3,584 against 1,970 72.0 -> 65.7.
+//
 // Tiles (Tall<rows, columns, waves along rows, along columns, slabs in the ring, column groups of the phases>): the wider, the less a
 // product fetches; which one comes out best is a matter of how full its last round of the chip is: see pick_tall.
 //
@@ -51,12 +56,67 @@ struct Tall {
   static_assert(WM * WN == 8 && TM % (32 * WM) == 0 && TN % (32 * WN) == 0 && J0 + J1 + J2 == TJ && S * kStage <= 160 * 1024, "eight waves share the tile, the phases its columns");
 };
 
+// bfloat16 outputs leave by way of LDS, 32 rows of a wave at a time: the products are taken with W's rows first, so that a lane holds four
+// consecutive columns of one row (element e of a group: row lane % 32, column 8 (e / 4) + 4 (lane / 32) + e % 4); it writes them as eight bytes, and
+// the wave reads whole rows back, sixteen bytes a lane.
+template <int kEpilogue, int TJ>
+constexpr int kRowsStride = TJ * (is_gated(kEpilogue) ? 32 : 64) + 16;      // bytes of a wave's row in LDS
+template <int kEpilogue, int TJ>
+constexpr int kRowsBytes = 32 * kRowsStride<kEpilogue, TJ>;
+template <int kEpilogue, int TI, int TJ>
+__device__ __forceinline__ void rows_epilogue(f32x16 (&acc)[TI][TJ], char* mine, bf16_t* __restrict__ out, int64_t ldo, const float* __restrict__ bias, int M, int N, int m0,
+                                              int n0, int lane) {
+  constexpr bool kGated = is_gated(kEpilogue);
+  constexpr int kStride = kRowsStride<kEpilogue, TJ>, kChunks = TJ * (kGated ? 2 : 4);      // sixteen-byte chunks a row
+  const bool whole = ldo % 8 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+  char* to = mine + (lane % 32) * kStride + (lane / 32) * 8;
+#pragma unroll
+  for (int i = 0; i < TI; ++i) {
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+#pragma unroll
+      for (int e = 0; e < 16; e += kGated ? 8 : 4) {
+        float v[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          if constexpr (kGated) {
+            v[c] = gate_of<kEpilogue == kMfGeglu>(acc[i][j][e + c]) * acc[i][j][e + 4 + c];
+          } else {
+            v[c] = acc[i][j][e + c];
+            if (bias) v[c] += bias[min(n0 + j * 32 + e * 2 + (lane / 32) * 4 + c, N - 1)];
+          }
+        }
+        *reinterpret_cast<uint2*>(to + j * (kGated ? 32 : 64) + e * (kGated ? 2 : 4)) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+      }
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int x = 0; x < kChunks / 2; ++x) {
+      const int at = x * 64 + lane, r = at / kChunks, c = at % kChunks, m = m0 + i * 32 + r, n = n0 + c * 8;
+      const uint4 v = *reinterpret_cast<const uint4*>(mine + r * kStride + c * 16);
+      bf16_t* dst = out + static_cast<int64_t>(m) * ldo + n;
+      if (m < M) {
+        if (whole && n + 8 <= N) {
+          *reinterpret_cast<uint4*>(dst) = v;
+        } else {
+          const uint32_t word[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+          for (int u = 0; u < 8; ++u)
+            if (n + u < N) dst[u] = static_cast<bf16_t>(word[u / 2] >> (16 * (u % 2)));
+        }
+      }
+    }
+    wave_lds_sync();
+  }
+}
+
 template <int kEpilogue, typename TO, typename T>
 __global__ void __launch_bounds__(512) gemm_tall_kernel(TO* __restrict__ out, int64_t ldo, const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W,
                                                         const bf16_t* __restrict__ W2, int64_t ldw, const float* __restrict__ bias, int M, int N, int K, int tiles_m,
                                                         int tiles_n) {
-  constexpr int TM = T::TM, TN = T::TN, WN = T::WN, TI = T::TI, TJ = T::TJ, S = T::S, P = T::P, kGateTiles = TJ / 2;
-  static_assert(!is_gated(kEpilogue) || TJ % 2 == 0, "a wave's column groups are gate and up in turn");
+  constexpr int TM = T::TM, TN = T::TN, WN = T::WN, TI = T::TI, TJ = T::TJ, S = T::S, P = T::P;
+  constexpr bool kGated = is_gated(kEpilogue), kRows = sizeof(TO) == 2;      // kRows: a lane holds four consecutive columns of one row (bfloat16 outputs, see rows_epilogue)
+  static_assert(!kGated || kRows, "gated outputs are bfloat16");
   __shared__ __attribute__((aligned(1024))) char ring[S * T::kStage];
   const TilePlace place = place_tile(blockIdx.x, tiles_m, tiles_n, 1, true);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
@@ -79,9 +139,9 @@ __global__ void __launch_bounds__(512) gemm_tall_kernel(TO* __restrict__ out, in
         row = A + static_cast<int64_t>(min(m0 + r, M - 1)) * lda;
       } else {
         const int x = p == 0 ? r - TM : r, wcol = x / (T::J(p) * 32), j = T::before(p) + x / 32 % T::J(p);
-        // (gated: a wave's groups are gate, up, gate, up of 32 columns each)
-        const int n = n0 + (is_gated(kEpilogue) ? wcol * kGateTiles + j / 2 : wcol * TJ + j) * 32 + x % 32;
-        row = (is_gated(kEpilogue) && (j & 1) ? W2 : W) + static_cast<int64_t>(min(n, N - 1)) * ldw;
+        // (gated: a group of 32 is gate, up, gate, up of eight columns each, so that both halves of an output meet in one lane)
+        const int n = n0 + (kGated ? (wcol * TJ + j) * 16 + x % 32 / 16 * 8 + x % 8 : (wcol * TJ + j) * 32 + x % 32);
+        row = (kGated && (x & 8) ? W2 : W) + static_cast<int64_t>(min(n, N - 1)) * ldw;
       }
       src[p][i] = row + chunk * 8;
       to[p][i] = static_cast<unsigned>(reinterpret_cast<uintptr_t>(ring)) + (T::first_row(p) + at) * 128;
@@ -157,7 +217,8 @@ __global__ void __launch_bounds__(512) gemm_tall_kernel(TO* __restrict__ out, in
         for (int i = 0; i < TI; ++i)
 #pragma unroll
           for (int j = 0; j < n; ++j) {
-            acc[i][T::before(p) + j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[q][i], w[q][j], acc[i][T::before(p) + j], 0, 0, 0);
+            acc[i][T::before(p) + j] = kRows ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[q][j], a[q][i], acc[i][T::before(p) + j], 0, 0, 0)
+                                             : __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[q][i], w[q][j], acc[i][T::before(p) + j], 0, 0, 0);
             ++done;
             if (more && sent < loads && done * loads * 4 >= (sent + 1) * total * 3) {
               __builtin_amdgcn_sched_barrier(0);
@@ -182,31 +243,25 @@ __global__ void __launch_bounds__(512) gemm_tall_kernel(TO* __restrict__ out, in
   if (k + 1 < slabs) slab_step(k++, std::integral_constant<int, 1>{});
   slab_step(k, std::integral_constant<int, 0>{});
   if (!late) end_slot();
-  if constexpr (is_gated(kEpilogue)) {      // gate's groups first, as the epilogue wants them
-    f32x16 sorted[TI][TJ];
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-      for (int j = 0; j < TJ; ++j) sorted[i][j] = acc[i][j < kGateTiles ? 2 * j : 2 * (j - kGateTiles) + 1];
-    tile_epilogue<kEpilogue, TO, TI, TJ>(sorted, out, ldo, bias, M, N, m0, n0, wm, wn, lane);
-  } else {
-    tile_epilogue<kEpilogue, TO, TI, TJ>(acc, out, ldo, bias, M, N, m0, n0, wm, wn, lane);
-  }
+  // (behind the last slot's barrier nobody reads the ring any more, and no fetch is on its way)
+  if constexpr (kRows) rows_epilogue<kEpilogue, TI, TJ>(acc, ring + wave * kRowsBytes<kEpilogue, TJ>, out, ldo, bias, M, N, m0 + wm * TI * 32, n0 + wn * TJ * (kGated ? 16 : 32), lane);
+  else tile_epilogue<kEpilogue, TO, TI, TJ>(acc, out, ldo, bias, M, N, m0, n0, wm, wn, lane);
 }
 
 // The forms, and what a tile of each takes: us a slab of 64 with few and with all compute units at work, and us besides (way in and epilogue).
-// Measured at 512 to 4,096 rows against 3,584 to 13,824 values of K.
+// Measured at 512 to 4,096 rows against 3,584 to 13,824 values of K; with the gate (columns of outputs: half as many as rows of W) fitted to 330 launches of 65 to 4,240 rows against
+// K of 768 to 5,120, which it foretells within 3 to 6 %: the form picked is 0.2 % behind the best one on average.
 struct TallForm {
   int rows, columns;      // of outputs
   double slab_few, slab_all, besides;
 };
 constexpr TallForm kPlain[] = {{256, 320, 1.38, 1.95, 17}, {256, 256, 1.15, 1.50, 9}, {256, 192, 1.07, 1.20, 6}, {256, 160, 1.00, 1.13, 5}, {256, 128, 0.83, 0.92, 4}, {128, 192, 0.70, 0.78, 4}, {128, 128, 0.57, 0.60, 3}};
-constexpr TallForm kGated[] = {{256, 128, 1.15, 1.50, 12}, {128, 128, 0.83, 0.92, 6}};
+constexpr TallForm kGated[] = {{256, 160, 1.27, 1.91, 9.5}, {256, 128, 1.02, 1.53, 7.1}, {256, 96, 0.93, 1.26, 5.6}, {256, 80, 0.83, 1.14, 5.6}, {256, 64, 0.66, 0.90, 4.8}, {128, 128, 0.89, 0.99, 3.4}, {128, 96, 0.79, 0.84, 3.7}, {128, 64, 0.67, 0.65, 2.9}};
 
 // The form with the least time by that count: whole rounds of the chip, then what is left over; `fill`: its tiles against the compute units.
 static int pick_tall(int M, int N, int K, bool gated, double* fill) {
   const TallForm* forms = gated ? kGated : kPlain;
-  const int n_forms = gated ? 2 : 7, cus = compute_units();
+  const int n_forms = gated ? 8 : 7, cus = compute_units();
   const double slabs = (K + 63) / 64;
   int best = 0;
   double least = 1e30;
@@ -224,7 +279,7 @@ static int pick_tall(int M, int N, int K, bool gated, double* fill) {
 // Where the tiled product's other forms stay ahead: tiles that leave too much of the chip idle (their K can be shared out over blocks), all the more the
 // shorter K is (a tile is over before the ring has paid for its way in). us, the other forms / these:
 //   behind: 4,608 x 3,584 against 512 rows (144 tiles of 128 x 128) 38 / 39, 3,584 x 3,584 against 700 (168) 36 / 39, 3,584 x 18,944 against 512 (56 of 256 x 128) 105 / 237,
-//   2,560 x 2,048 against 1,024 (160 of 128 x 128) 21 / 24, 2,048 x 1,536 against 1,536 (192) 18 / 21, 8,960 x 1,536 with the gate against 256 (70) 31 / 36, 4,864 x 896 with the gate against 2,048 47 / 52;
+//   2,560 x 2,048 against 1,024 (160 of 128 x 128) 21 / 24, 2,048 x 1,536 against 1,536 (192) 18 / 21, 8,960 x 1,536 with the gate against 256 (70) 31 / 36;
 //   ahead: 5,120 x 5,120 against 512 (160) 67 / 56, 5,120 x 13,824 against 512 170 / 130, 3,584 x 3,584 against 1,024 (224) 53 / 41, against 2,000 70 / 60, 5,120 x 27,648 against 4,096 1,299 / 891,
 //   5,120 x 5,120 260 / 184, 4,608 x 3,584 against 2,000 100 / 72, 2,560 x 2,048 against 1,536 (240) 35 / 25; with the gate: 18,944 x 3,584 against 65 (148 of 128 x 128) 79 / 62, against 2,048
 //   523 / 463, 27,648 x 5,120 against 2,048 1,090 / 920, 8,960 x 1,536 against 300 (210) 35 / 29, 13,824 x 5,120 against 2,048 573 / 493.
@@ -237,21 +292,33 @@ static int pick_tall(int M, int N, int K, bool gated, double* fill) {
 // But not 256 x 160 where the others come out in two rounds and K is short or the last rows are mostly padding: 8,960 x 1,536 against 787 36 / 41, 18,944 x 2,048 against 269 44 / 47, 18,944 x 5,120
 // against 330 89 / 95 (4,608 x 1,792 against 1,907, 540 of 128 x 128, 56 / 42); nor one round of 128 x 128 with that much padding and K under 4,096: 8,960 x 1,536 against 265 (210) 18.0 / 21.0, x 3,584
 // 35.4 / 38.0, 13,824 x 2,048 against 140 (216) 21.6 / 25.1 (against 1,536 x 1,536, 2,073 rows, 25 / 22).
-bool tall_pays(int M, int N, int K, bool gated) {
+// K from 768 to 1,535 (us, the others / these; 0.5B sizes unless said). With the gate wherever the others' tiles of 64 rows x 64 outputs are more than one round: 4,864 x 896 against 171 rows (228 of
+// them) 10.9 / 12.9, against 202 (304) 14.3 / 13.1, 467 22.4 / 16.7, 1,041 31.6 / 25.0, 1,430 43.9 / 29.2, 2,048 46.9 / 37.2, 3,967 92.9 / 73.8; 2,816 x 1,024 against 200 (176) 10.1 / 13.0,
+// 370 (264) 13.8 / 13.3, 2,803 49.0 / 32.6; 3,072 x 768 against 279 (240) 9.0 / 11.1, 2,968 43.2 / 33.5. Stored as bfloat16 from seven tenths of a round of 128 x 128 on: 1,152 x 896 against 1,162 (90)
+// 9.8 / 12.1, 2,453 (180) 12.9 / 12.8, 3,209 (234) 19.1 / 13.5; 4,096 x 1,024 against 398 (128) 10.8 / 13.2, 988 (256) 23.4 / 14.6, 3,302 56.9 / 31.7; 4,864 x 896 against 3,039 55.5 / 29.4. Float outputs,
+// whose way out is longer, from eight tenths: 896 x 896 against 2,734 (154) 14.3 / 17.6, 3,760 (210) 20.9 / 18.6.
+// With the gate and K from 1,536 from 0.55 of a round on: 8,960 x 1,536 against 268 rows 37.9 / 27.5, 819 77.4 / 55.6, 2,021 140 / 107; 5,632 x 2,048 against 107 (88 tiles of 128 x 64) 22.4 / 23.7, 225 (176)
+// 26.4 / 24.4, 2,116 124 / 102. Up to 256 rows against K under 2,048 with few tiles of 128 x 128 stay where they were (5,632 x 1,536 and narrower are even there; 8,960 against 245 36.6 / 26.2 is left).
+bool tall_pays(int M, int N, int K, TallKind kind) {
   static const bool switched_off = [] { const char* e = getenv("ALOFA_WIDE_TILES"); return e != nullptr && e[0] == '0'; }();     // (for measurements)
-  if (switched_off || M <= 64 || K % 32 != 0 || K < 1536) return false;
+  if (switched_off || M <= 64 || K % 32 != 0 || K < 768) return false;
+  const bool gated = kind == kTallGated;
   double fill = 0;
   const int form = pick_tall(M, N, K, gated, &fill), cus = compute_units();
-  if (!gated) {
-    const int64_t small = static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128);
-    const int full = (M + kPlain[form].rows - 1) / kPlain[form].rows * kPlain[form].rows;      // rows with the last tile's padding
-    if (kPlain[form].columns == 160 && small <= 2 * cus && (K <= 2048 || 4 * M < 3 * full)) return false;
-    if (kPlain[form].rows == 128 && kPlain[form].columns == 128 && small <= cus && K < 4096 && 5 * M < 4 * full) return false;
-    if (small > cus) return K >= 2048 || fill >= 0.72;
+  const int64_t small = static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128);
+  if (gated) {
+    if (K < 1536) return static_cast<int64_t>((M + 63) / 64) * ((N + 63) / 64) > cus;
+    if (K < 2048 && M <= 256 && 10 * small < 8 * cus) return false;
+    return fill >= 0.55;
   }
+  if (K < 1536) return 10 * small >= (kind == kTallRows16 ? 7 : 8) * static_cast<int64_t>(cus);
+  const int full = (M + kPlain[form].rows - 1) / kPlain[form].rows * kPlain[form].rows;      // rows with the last tile's padding
+  if (kPlain[form].columns == 160 && small <= 2 * cus && (K <= 2048 || 4 * M < 3 * full)) return false;
+  if (kPlain[form].rows == 128 && kPlain[form].columns == 128 && small <= cus && K < 4096 && 5 * M < 4 * full) return false;
+  if (small > cus) return K >= 2048 || fill >= 0.72;
   if (K < 2048) return fill >= 0.80;
-  if (!gated && K < 8960 && static_cast<int64_t>(N) * K < 20000000) return fill >= 0.735;
-  return fill >= (K < 3072 || (K < 5120 && !gated) ? 0.70 : 0.57);
+  if (K < 8960 && static_cast<int64_t>(N) * K < 20000000) return fill >= 0.735;
+  return fill >= (K < 5120 ? 0.70 : 0.57);
 }
 
 template <int kEpilogue, typename TO, typename T>
@@ -268,8 +335,16 @@ static int launch_picked(void* out, int64_t ldo, const void* A, int64_t lda, con
   double fill = 0;
   const int form = pick_tall(M, N, K, is_gated(kEpilogue), &fill);
   if constexpr (is_gated(kEpilogue)) {
-    if (form == 0) return launch_form<kEpilogue, TO, Tall<256, 256, 4, 2, 2, 2, 2>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream);
-    return launch_form<kEpilogue, TO, Tall<128, 256, 2, 4, 3, 1, 1>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream);
+    switch (form) {
+      case 0: return launch_form<kEpilogue, TO, Tall<256, 320, 4, 2, 2, 2, 2, 1>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream);
+      case 1: return launch_form<kEpilogue, TO, Tall<256, 256, 4, 2, 2, 2, 2>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream);
+      case 2: return launch_form<kEpilogue, TO, Tall<256, 192, 4, 2, 2, 2, 1>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream);
+      case 3: return launch_form<kEpilogue, TO, Tall<256, 160, 8, 1, 3, 3, 2>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream);
+      case 4: return launch_form<kEpilogue, TO, Tall<256, 128, 4, 2, 3, 1, 1>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream);
+      case 5: return launch_form<kEpilogue, TO, Tall<128, 256, 2, 4, 3, 1, 1>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream);
+      case 6: return launch_form<kEpilogue, TO, Tall<128, 192, 4, 2, 3, 2, 1>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream);
+      default: return launch_form<kEpilogue, TO, Tall<128, 128, 4, 2, 3, 1, 1>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream);
+    }
   } else {
     switch (form) {
       case 0: return launch_form<kEpilogue, TO, Tall<256, 320, 4, 2, 2, 2, 2, 1>>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream);
@@ -303,8 +378,8 @@ extern "C" int alofa_gemm_wide_form(int M, int N, int K, int gated) {
   return pick_tall(M, N, K, gated != 0, &fill);
 }
 
-// Whether alofa_gemm_mfma takes these tiles.
-extern "C" int alofa_gemm_wide_pays(int M, int N, int K, int gated) { return tall_pays(M, N, K, gated != 0); }
+// Whether alofa_gemm_mfma takes these tiles (gated: 0 float outputs, 1 with the gate, 2 bfloat16 outputs without).
+extern "C" int alofa_gemm_wide_pays(int M, int N, int K, int gated) { return tall_pays(M, N, K, static_cast<TallKind>(gated)); }
 
 // The same product by these tiles whatever the sizes (alofa_gemm_mfma takes them where they pay): K a multiple of 32. The operands as for
 // alofa_gemm_mfma; norm_w and eps stand where alofa_gemm_skinny has them and must be null and zero (no norm rides on this kernel).

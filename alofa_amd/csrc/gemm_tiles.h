@@ -83,7 +83,8 @@ __device__ __forceinline__ void tile_epilogue(f32x16 (&acc)[WTM][WTN], TO* __res
 
 // (gemm_tall.hip) Tiles of up to 256 x 320 outputs by eight waves, for many rows. `pays`: whether they are the tiled product's choice for these sizes.
 // `launch`: the product with the epilogue as above and `out` of type o_dtype; K a multiple of 32. 0, or 1 with the error set.
-bool tall_pays(int M, int N, int K, bool gated);
+enum TallKind : int { kTallFloat = 0, kTallGated = 1, kTallRows16 = 2 };      // float outputs, with the gate, bfloat16 outputs
+bool tall_pays(int M, int N, int K, TallKind kind);
 int launch_tall(int epilogue, int o_dtype, void* out, int64_t ldo, const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, const float* bias,
                 int M, int N, int K, hipStream_t stream);
 

@@ -1221,6 +1221,57 @@ def test_forms_of_the_product_for_many_rows(M, N, K, form):
         assert (gated[:, :n].float() - ref).abs().max().item() <= (2.0 ** -8 + 1e-5) * ref.abs().max().item() and bool((gated[:, n:] == 3.0).all())
 
 
+# every form with the gate; edges in both directions, whole and half slabs, a column more than whole chunks of eight and rows that no 16-byte store can write; bfloat16 outputs without the gate by the same way out
+@pytest.mark.parametrize("M,N,K,form", [(2045, 5117, 320, 0), (2048, 4088, 224, 1), (2045, 3067, 96, 2), (2045, 2555, 192, 3), (2045, 2043, 1120, 4), (1021, 4091, 320, 5), (1021, 3072, 320, 6), (1021, 2043, 320, 7), (253, 2043, 32, 7)])
+@pytest.mark.parametrize("room", [0, 5, 8])
+def test_forms_with_the_gate_and_their_way_out(M, N, K, form, room):
+    from alofa_amd.csrc.build import load
+    assert load().alofa_gemm_wide_form(M, N, K, 1) == form
+    gen = torch.Generator(device=DEV).manual_seed(M + N + K)
+    a, w, w2 = (torch.randn(s, generator=gen, device=DEV).bfloat16() for s in ((M, K), (N, K), (N, K)))
+    bias = torch.randn(N, generator=gen, device=DEV)
+    want, up = a.float() @ w.float().t(), a.float() @ w2.float().t()
+    for ref, product in ((torch.nn.functional.silu(want) * up, lambda o: ops().gemm_swiglu(o, a, w, w2, kernel="wide")),
+                         (torch.nn.functional.gelu(want, approximate="tanh") * up, lambda o: ops().gemm_swiglu(o, a, w, w2, kernel="wide", act="gelu_tanh")),
+                         (want + bias, lambda o: ops().gemm(o, a, w, bias, kernel="wide"))):
+        out = torch.full((M, N + room), 3.0, device=DEV, dtype=torch.bfloat16)
+        product(out[:, :N])
+        # half a unit of bfloat16's last place, and the float sums' own error (K sums of 2^-24 each, of numbers of order sqrt(K), by as large an up)
+        bound = 2.0 ** -8 * ref.abs() + K ** 1.5 * 2.0 ** -24 * 4 * (1 + up.abs().max())
+        assert bool(((out[:, :N].float() - ref).abs() <= bound).all()) and bool((out[:, N:] == 3.0).all())
+
+
+def test_the_gates_own_division():
+    """Gates from far below to far above zero, infinite ones and NaN: z / (1 + exp(-z)) as the general division gives it, but for quotients under 1e-36."""
+    z = torch.cat([torch.linspace(-120, 120, 4090, device=DEV), torch.tensor([float("inf"), -float("inf"), float("nan"), 0.0, -0.0, 1e-30], device=DEV)])
+    w = torch.zeros(4096, 64, device=DEV, dtype=torch.bfloat16)
+    w[:, 0] = z.bfloat16()
+    a = torch.zeros(96, 64, device=DEV, dtype=torch.bfloat16)
+    a[:, 0] = 1.0
+    w[4090:4093, 1:] = 0
+    up = torch.zeros_like(w)
+    up[:, 0] = 1.0
+    out = torch.empty(96, 4096, device=DEV, dtype=torch.bfloat16)
+    ops().gemm_swiglu(out, a, w, up, kernel="wide")
+    x = w[:, 0].double()
+    want = (x / (1 + torch.exp(-x.float()).double()))
+    nan = torch.isnan(want.float())
+    assert bool((torch.isnan(out) == nan).all())
+    got, want = out[:, ~nan].double(), want[~nan]
+    fine = (got == want) | ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-36)
+    assert bool(fine.all())
+
+
+# with the gate and for bfloat16 and float outputs (kind 1, 2, 0) on either side of their lines: K under 1,536 and under 768
+@pytest.mark.parametrize("M,N,K,kind,taken", [(171, 4864, 896, 1, 0), (202, 4864, 896, 1, 1), (2048, 4864, 896, 1, 1), (2048, 4864, 736, 1, 0), (819, 8960, 1536, 1, 1), (107, 5632, 2048, 1, 0),
+                                              (2048, 1152, 896, 2, 0), (2453, 1152, 896, 2, 1), (2453, 1152, 896, 0, 0), (3760, 896, 896, 0, 1)])
+def test_which_products_of_a_short_k_the_forms_for_many_rows_take(M, N, K, kind, taken):
+    from alofa_amd.csrc.build import load
+    if ops().compute_units() != 256:
+        pytest.skip("the sizes are those of 256 compute units")
+    assert load().alofa_gemm_wide_pays(M, N, K, kind) == taken
+
+
 # which forms take a product (256 compute units): a little more than one round of tiles of 128 x 128; small matrices on either side of their line; few tiles of a long K; a short K; the gate
 @pytest.mark.parametrize("M,N,K,gated,taken", [(315, 11008, 4096, 0, 1), (303, 11008, 2048, 0, 1), (957, 4224, 3584, 0, 1), (1385, 3072, 2560, 0, 1), (2262, 1280, 2048, 0, 0), (1170, 2304, 8192, 0, 0),
                                                (2706, 896, 8192, 0, 0), (3432, 896, 2560, 0, 1), (439, 5120, 5120, 0, 1), (512, 3584, 18944, 0, 0), (2674, 896, 18944, 0, 1), (900, 4224, 1600, 0, 0),
