@@ -1,0 +1,112 @@
+"""Decode steps whose layers run in one launch (csrc/decode_resident.hip): what the launch needs beside the step's own tensors, kept by a step
+function: the table of the layers' matrices and caches, an area of memory that the launch's blocks exchange values in, and a word that the
+kernel sets if it gives a wait up."""
+from __future__ import annotations
+
+import ctypes
+import threading
+import weakref
+from typing import Optional
+
+import torch
+
+from .. import ops
+from ..errors import AlofaError
+from ..parts.attention import GQAAttention
+from ..parts.block import PreNormBlock
+from ..parts.feed_forward import SwiGLU
+
+
+class _Areas:
+    """Areas that step functions of this process have given back. They are never freed (uncached device memory must not be), so there are never
+    more of them than step functions lived at one time. One that changes hands has no launch in flight: the taker waits for the device first."""
+
+    def __init__(self):
+        self._lock = threading.Lock()
+        self._idle: dict = {}      # device -> addresses
+
+    def take(self, device: torch.device) -> int:
+        with self._lock:
+            idle = self._idle.get(device.index)
+            known = idle.pop() if idle else None
+        if known is not None:
+            torch.cuda.synchronize(device)
+            return known
+        with torch.cuda.device(device):
+            return ops.resident_area()
+
+    def give_back(self, device: torch.device, area: int) -> None:
+        with self._lock:
+            self._idle.setdefault(device.index, []).append(area)
+
+
+_areas = _Areas()
+
+
+class ResidentLayers:
+    """All layers of ``model`` over ``cache`` as one launch, for steps of at most ``MOST_ROWS`` rows of one new token each."""
+    MOST_ROWS = 16
+    MOST_LAYERS = 64      # whose addresses the kernel keeps at hand
+
+    @classmethod
+    def of(cls, model, cache) -> Optional["ResidentLayers"]:
+        """None where the model's layers are not what the kernel runs: pre-norm blocks of grouped-query attention over its own cache of every token (rotary, no
+        output bias) and a silu-gated feed-forward, all alike, sizes that fit a block's registers, bfloat16."""
+        rt, order = model.rt, model.order
+        if rt.exact or rt.dtype is not torch.bfloat16 or model.streams or model.joins or not 0 < len(order) <= cls.MOST_LAYERS:
+            return None
+        blocks = [model.blocks[e.layer] for e in order]
+        if any(e.cache_of is not None or e.join is not None for e in order) or any(type(b) is not PreNormBlock for b in blocks):
+            return None
+        first = blocks[0]
+        for i, b in enumerate(blocks):
+            m, f = b.mixer, b.feed_forward
+            if type(m) is not GQAAttention or type(f) is not SwiGLU or f.activation != "silu" or m.window is not None or m.b_o is not None:
+                return None
+            if any(n.as_rmsnorm() is None for n in b.norms) or m.position.table(1) is None or cache.group_of_entry.get((i, 0)) is None:
+                return None
+            same = [(x.mixer.heads, x.mixer.kv_heads, x.mixer.d, x.mixer.scale, x.mixer.b_qkv is None, x.mixer.hidden, x.feed_forward.intermediate, tuple(n.as_rmsnorm()[1] for n in x.norms),
+                     x.mixer.position.table(1)[0].data_ptr()) for x in (first, b)]
+            if same[0] != same[1] or cache.group_of_entry[(i, 0)] != cache.group_of_entry[(0, 0)]:
+                return None
+        m = first.mixer
+        if not ops.resident_takes(m.hidden, first.feed_forward.intermediate, m.heads, m.kv_heads, m.d, cache.block_size):
+            return None
+        return cls(blocks, cache, rt.device)
+
+    def __init__(self, blocks: list, cache, device):
+        self.blocks, self.device = blocks, device
+        m = blocks[0].mixer
+        self.heads, self.kv_heads, self.d, self.scale, self.position = m.heads, m.kv_heads, m.d, m.scale, m.position
+        self.hidden, self.intermediate, self.biased = m.hidden, blocks[0].feed_forward.intermediate, m.b_qkv is not None
+        self.eps = tuple(float(n.as_rmsnorm()[1]) for n in blocks[0].norms)
+        self.page, self.group = cache.block_size, cache.group_of_entry[(0, 0)]
+        # (what the table points to: the model's matrices and the cache's pages, which live as long as the step function that holds both)
+        rows = []
+        for i, b in enumerate(blocks):
+            kv = cache.tensors[(i, 0)]
+            ops.check_caches(kv["k"], kv["v"], self.kv_heads, self.d)
+            tensors = [b.mixer.w_qkv, b.mixer.b_qkv, b.mixer.w_o, b.feed_forward.w_gate, b.feed_forward.w_up, b.feed_forward.w_down,
+                       b.norms[0].as_rmsnorm()[0], b.norms[1].as_rmsnorm()[0], kv["k"], kv["v"]]
+            if any(t is not None and (not t.is_cuda or not t.is_contiguous()) for t in tensors):
+                raise AlofaError("shape_mismatch", "the layers' tensors must be contiguous and on the GPU", f"layer={i}")
+            rows.append([0 if t is None else t.data_ptr() for t in tensors])
+        self.layers = torch.tensor(rows, dtype=torch.int64, device=device)
+        self.area = _areas.take(device)
+        weakref.finalize(self, _areas.give_back, device, self.area)
+        self.failed = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self._failed = self.failed.numpy()
+
+    def takes(self, ctx, rows: int) -> bool:
+        """Whether this step runs in one launch: one new token for each of few requests."""
+        return rows <= self.MOST_ROWS and ctx.max_q_len == 1 and len(ctx.spans) == rows
+
+    def check(self) -> None:
+        if self._failed[0]:
+            raise AlofaError("not_initialized", "a decode step gave up waiting for blocks that another kernel kept off the GPU; its results are lost")
+
+    def forward(self, ctx, hidden: torch.Tensor) -> None:
+        self.check()
+        cos, sin = self.position.table(ctx.n_positions)
+        ops.decode_resident(hidden, self.layers, ctx.positions, ctx._tables[self.group], ctx._slots[self.group], cos, sin, self.area, self.failed, self.intermediate,
+                            self.heads, self.kv_heads, self.d, self.page, self.biased, self.scale, self.eps)

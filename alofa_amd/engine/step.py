@@ -17,6 +17,7 @@ import torch
 from .. import ops
 from ..cache.manager import CacheManager
 from ..errors import AlofaError
+from .resident import ResidentLayers
 
 
 def _pow2_ceil(n: int) -> int:
@@ -89,6 +90,7 @@ class StepContext:
         self._memo: dict = {}
         self.token_store = fn.token_store
         self.watch = fn.watch
+        self.resident = fn.resident
         self.request_slots: Optional[torch.Tensor] = None   # int32 [entries] on the device: the request slot of every entry
         self.row_offsets: Optional[torch.Tensor] = None     # int32 [entries + 1] on the device: entry i owns the rows [i] .. [i+1]-1; None: one row each (decode graphs)
         self.want_slots: Optional[torch.Tensor] = None      # int32 [wanted rows] on the device: the request slot behind every wanted row
@@ -180,6 +182,7 @@ class StepFunction:
         self.graph_replays = 0
         # what must not move once steps run (position tables up to the context bound) is built now
         model.prepare(self.n_positions)
+        self.resident = ResidentLayers.of(model, cache)      # None, or what runs the layers of small decode steps in one launch
 
     # ------------------------------------------------------------- scratch
     def scratch(self, name: str, shape: tuple, dtype: torch.dtype) -> torch.Tensor:
@@ -430,6 +433,8 @@ class StepFunction:
         the logits, int32 [wanted] with the first index of every wanted row's highest
         logit, and leaves the same in the token store at the row's request's slot.
         The buffer is re-used by the next step."""
+        if self.resident is not None:
+            self.resident.check()
         with ops.stream_scope():
             if self.use_graphs and self.watch is None and all(len(e.tokens) == 1 and list(e.want) == [0] for e in entries):
                 return self._run_decode_graph(entries, greedy)

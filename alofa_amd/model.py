@@ -125,6 +125,10 @@ class Model:
             first = ctx.scratch("hidden_first", tuple(hidden.shape), torch.float32)
             first.copy_(hidden)
         watch = getattr(ctx, "watch", None)      # (for tests and debugging: called with the stream after every run entry)
+        resident = getattr(ctx, "resident", None)
+        if resident is not None and watch is None and resident.takes(ctx, rows):      # few rows of one new token each: every layer in one launch
+            resident.forward(ctx, hidden)
+            return hidden
         stream = hidden
         if self.streams:      # the copies: spread, and read for the first block, in one launch
             stream = ctx.scratch("streams", (rows, self.streams, hidden.shape[1]), torch.float32)

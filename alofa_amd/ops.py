@@ -823,6 +823,44 @@ def attention_decode(out, q, k_cache, v_cache, block_table, req_of_token, positi
           _I(planes), _L(out.stride(0) if planes else 0), _ptr(_sink_of(sink, heads)), _I(block_heads), _I(0), _I(0), _F(0.0), _F(0.0), _F(0.0), _F(0.0), _I(d), _stream())
 
 
+# ---------------------------------------------------- decode steps in one launch
+
+def resident_takes(hidden: int, intermediate: int, heads: int, kv_heads: int, d: int, page: int) -> bool:
+    """Whether the layers of a model of these sizes fit the kernel that runs all of a decode step's layers in one launch."""
+    return bool(_answer("alofa_resident_takes", _I(hidden), _I(intermediate), _I(heads), _I(kv_heads), _I(d), _I(page)))
+
+
+def resident_area() -> int:
+    """A new area that the blocks of ``decode_resident`` exchange values in: its address. It is never freed."""
+    place = ctypes.c_void_p()
+    if load().alofa_resident_area(ctypes.byref(place)) != 0:
+        raise AlofaError("capacity", "no memory for an area", load().alofa_last_error().decode())
+    return place.value
+
+
+def decode_resident(hidden: torch.Tensor, layers: torch.Tensor, positions: torch.Tensor, block_table: torch.Tensor, slots: torch.Tensor, cos: torch.Tensor,
+                    sin: torch.Tensor, area: int, failed: torch.Tensor, intermediate: int, heads: int, kv_heads: int, d: int, page: int, biased: bool, scale: float, eps: tuple) -> None:
+    """Every layer of a decode step, one new token per row, row i request i: ``hidden`` float32 [rows, width], in and out. ``layers`` int64 [layers, 10]: the addresses of a
+    layer's matrices, norms and caches, which the caller keeps alive and has checked; ``area``: of ``resident_area``, used by one launch at a time; ``failed``: int32 [1] in
+    pinned memory, set if the kernel gives a wait up."""
+    _contig("hidden", _gpu("hidden", hidden, torch.float32, 2))
+    M, H = hidden.shape
+    _contig("layers", _gpu("layers", layers, torch.int64, 2))
+    if layers.shape[1] != 10:
+        raise AlofaError("shape_mismatch", "a layer has ten addresses", f"layers={tuple(layers.shape)}")
+    _contig("block_table", _gpu("block_table", block_table, torch.int32, 2))
+    for name, t, dtype in (("positions", positions, torch.int32), ("slots", slots, torch.int64)):
+        if tuple(_contig(name, _gpu(name, t, dtype, 1)).shape) != (M,):
+            raise AlofaError("shape_mismatch", "one number per row", f"operand={name} shape={tuple(t.shape)} rows={M}")
+    for name, t in (("cos", cos), ("sin", sin)):
+        if _contig(name, _gpu(name, t, torch.float32, 2)).shape[1] != d // 2:
+            raise AlofaError("shape_mismatch", "half a head of angles per position", f"operand={name} shape={tuple(t.shape)}")
+    if block_table.shape[0] < M or failed.dtype is not torch.int32 or not failed.is_pinned():
+        raise AlofaError("shape_mismatch", "a row of pages per request, and a pinned word", f"table={tuple(block_table.shape)} rows={M}")
+    _call("alofa_decode_resident", hidden, layers, positions, block_table, slots, cos, sin, _L(area), _L(failed.data_ptr()), _I(layers.shape[0]), _I(M), _I(H), _I(intermediate),
+          _I(heads), _I(kv_heads), _I(d), _I(page), _I(block_table.shape[1]), _I(bool(biased)), _F(scale), _F(eps[0]), _F(eps[1]), _L(_stream()))
+
+
 def can_fuse_rope_into_decode(d: int) -> bool:
     """Head sizes for which the decode attention kernel can rotate and write the new token itself."""
     return d % 64 == 0

@@ -1,0 +1,131 @@
+"""Decode steps whose layers run in one launch (csrc/decode_resident.hip), beside the kernels that run them one after the other and the 32-bit path."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+VOCAB, LAYERS = 512, 3
+
+
+def model(width, heads, kv_heads, ff, dtype, layers=LAYERS, window=None):
+    from alofa_amd.config import config_from_dict
+    from alofa_amd.model import Model, runtime
+    config = config_from_dict({"architectures": ["Qwen2ForCausalLM"], "model_type": "qwen2", "num_hidden_layers": layers, "hidden_size": width, "num_attention_heads": heads,
+                               "num_key_value_heads": kv_heads, "head_dim": width // heads, "intermediate_size": ff, "vocab_size": VOCAB, "rope_theta": 10000.0, "rms_norm_eps": 1e-6,
+                               "tie_word_embeddings": True, "use_sliding_window": window is not None, "max_position_embeddings": 4096,
+                               **({"sliding_window": window, "max_window_layers": 0} if window else {})})
+    gen = torch.Generator(device="cuda").manual_seed(7)
+
+    def draw(*shape, scale=1.0, shift=0.0):
+        return (torch.randn(shape, generator=gen, device="cuda") * scale + shift).to(torch.bfloat16)
+    d = width // heads
+    w = {"model.embed_tokens.weight": draw(VOCAB, width), "model.norm.weight": draw(width, scale=0.1, shift=1.0)}
+    for i in range(layers):
+        pre = f"model.layers.{i}."
+        for n, rows, cols in (("self_attn.q_proj", heads * d, width), ("self_attn.k_proj", kv_heads * d, width), ("self_attn.v_proj", kv_heads * d, width),
+                              ("self_attn.o_proj", width, heads * d), ("mlp.gate_proj", ff, width), ("mlp.up_proj", ff, width), ("mlp.down_proj", width, ff)):
+            w[pre + n + ".weight"] = draw(rows, cols, scale=cols ** -0.5)
+            if n[-6] in "qkv" and n.startswith("self"):
+                w[pre + n + ".bias"] = draw(rows, scale=0.5)
+        for n in ("input_layernorm", "post_attention_layernorm"):
+            w[pre + n + ".weight"] = draw(width, scale=0.1, shift=1.0)
+    return config, Model(config.spec(), w, runtime(dtype))
+
+
+def engine(m, rows, context, dtype, page=16):
+    from alofa_amd import Engine
+    return Engine(None, dtype=dtype, max_tokens=context + 8, max_batch=rows, kv_blocks=rows * ((context + 8) // page + 2), block_size=page, token_budget=4096, watermark_permille=1000, model=m)
+
+
+def stand(eng, lengths, seed):
+    """Requests 0.. with lengths[i] tokens in the cache."""
+    from alofa_amd.engine.step import StepEntry
+    rng = np.random.default_rng(seed)
+    for i, n in enumerate(lengths):
+        eng.cache.admit(i)
+        if n:
+            eng.step_fn.run([StepEntry(i, rng.integers(0, VOCAB, n).tolist())])
+
+
+def decode(eng, tokens):
+    from alofa_amd.engine.step import StepEntry
+    return [eng.step_fn.run([StepEntry(i, [int(t)], [0]) for i, t in enumerate(row)]).double().cpu() for row in tokens]
+
+
+# widths: the least, ones whose columns do not divide by the blocks, the most; keys at the edges of tiles, pages, parts and a wave's first step
+SHAPES = [(256, 4, 1, 512), (320, 5, 5, 768), (896, 14, 2, 4864), (1024, 16, 2, 6144)]
+CONTEXTS = [0, 1, 15, 16, 17, 31, 255, 256, 300, 511, 600, 1023, 7, 48, 130, 2100]
+
+
+@pytest.mark.parametrize("page", [16, 64])
+@pytest.mark.parametrize("rows", [1, 2, 3, 5, 8, 9, 16])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_one_launch_is_as_near_the_32_bit_path_as_the_kernels_it_replaces(shape, rows, page):
+    lengths = (CONTEXTS * 2)[rows:2 * rows] if rows < 16 else CONTEXTS
+    tokens = np.random.default_rng(rows).integers(0, VOCAB, (3, rows))
+    got = {}
+    for how in ("float32", "one by one", "one launch", "one launch, captured"):
+        dtype = "float32" if how == "float32" else "bfloat16"
+        m = model(*shape, dtype)
+        eng = engine(m, rows, max(lengths) + 4, dtype, page)
+        fn = eng.step_fn
+        assert (fn.resident is None) == (how == "float32")
+        if how == "one by one":
+            fn.resident = None
+        fn.use_graphs = how.endswith("captured")
+        stand(eng, lengths, 1)
+        got[how] = decode(eng, tokens)
+        if how.endswith("captured"):
+            assert fn.graph_replays > 0
+    for step in range(len(tokens)):
+        exact = got["float32"][step]
+        off = {how: ((x[step] - exact).norm() / exact.norm()).item() for how, x in got.items()}
+        # both round the same values to bfloat16 and add in float32 in orders of their own: roundings that fall the other way are as many on either side, and
+        # over at least 512 logits the two distances are alike within a third (the spread of a norm of that many independent errors, with those of a layer's rows shared)
+        assert off["one launch"] <= 1.34 * off["one by one"] + 1e-4, (step, off)
+        # the same kernel on the same cache, whether captured or not
+        assert torch.equal(got["one launch"][step], got["one launch, captured"][step])
+
+
+def test_steps_in_turn_do_not_disturb_one_another():
+    """Two engines with areas of their own, of different rows, and steps that are no decode steps in between."""
+    tokens = np.random.default_rng(3).integers(0, VOCAB, (12, 8))
+    m = model(896, 14, 2, 4864, "bfloat16")
+    alone = {}
+    for rows in (2, 8):
+        eng = engine(m, rows, 100, "bfloat16")
+        stand(eng, [33 + i for i in range(rows)], 5)
+        alone[rows] = decode(eng, tokens[:, :rows])
+    both = {rows: engine(m, rows, 100, "bfloat16") for rows in (2, 8)}
+    assert both[2].step_fn.resident.area != both[8].step_fn.resident.area
+    for rows, eng in both.items():
+        stand(eng, [33 + i for i in range(rows)], 5)
+    for k, row in enumerate(tokens):
+        for rows, eng in both.items():
+            assert torch.equal(decode(eng, row[None, :rows])[0], alone[rows][k]), (k, rows)
+
+
+def test_what_it_does_not_take_runs_kernel_by_kernel():
+    assert engine(model(896, 14, 2, 4864, "bfloat16"), 2, 64, "bfloat16").step_fn.resident is not None
+    assert engine(model(896, 14, 2, 4864, "float32"), 2, 64, "float32").step_fn.resident is None
+    assert engine(model(896, 14, 2, 4864, "bfloat16", window=32), 2, 64, "bfloat16").step_fn.resident is None
+    assert engine(model(896, 14, 2, 4864, "bfloat16"), 2, 64, "bfloat16", page=8).step_fn.resident is None      # (pages of fewer than 16 tokens)
+    assert engine(model(512, 4, 1, 1024, "bfloat16"), 2, 64, "bfloat16").step_fn.resident is None               # heads of 128
+    assert engine(model(192, 3, 1, 512, "bfloat16"), 2, 64, "bfloat16").step_fn.resident is None                # fewer columns than blocks
+    eng = engine(model(896, 14, 2, 4864, "bfloat16"), 24, 64, "bfloat16")
+    stand(eng, [5] * 17, 2)
+    before = eng.step_fn.resident.failed.item()
+    assert all(torch.isfinite(x).all() for x in decode(eng, np.ones((2, 17), dtype=int)))      # (17 rows)
+    assert before == 0 and eng.step_fn.resident.failed.item() == 0
+
+
+def test_areas_are_used_again():
+    import gc
+    from alofa_amd.engine.resident import _areas
+    m = model(256, 4, 1, 512, "bfloat16", layers=1)
+    area = engine(m, 1, 32, "bfloat16").step_fn.resident.area
+    gc.collect()
+    idle = [a for areas in _areas._idle.values() for a in areas]
+    assert area in idle
+    assert engine(m, 1, 32, "bfloat16").step_fn.resident.area in idle
