@@ -28,8 +28,11 @@
 // LDS), so that 256 of them fit beside 256 of another such launch, whatever process it belongs to; kernels that wait for nobody make room by ending.
 // No wait is without end: a wave that has asked kLimit times sets `stop` and `failed`, which end every other wait, and the step's rows are NaN.
 //
-// A step of the 0.5B sizes (24 layers of 896, 14/2 heads, 4,864; the head's 70 us among them), us, kernel by kernel / this: 1 row of 512 keys 641 / 491, 2 665 / 515,
-// 4 of 512 to 768 714 / 551, 8 782 / 664, 12 of 64 to 700 890 / 688, 16 of 128 to 1,024 937 / 734, 1 of 4,000 705 / 528, 8 of 3,000 to 4,000 860 / 701.
+// A step of the 0.5B sizes (24 layers of 896, 14/2 heads, 4,864; the head's 70 us among them), us, kernel by kernel / this: 1 row of 512 keys 643 / 455, 2 667 / 476,
+// 4 of 512 to 768 715 / 510, 8 785 / 549, 12 of 64 to 700 890 / 616, 16 of 128 to 1,024 937 / 663, 1 of 4,000 707 / 481, 8 of 3,000 to 4,000 860 / 589. What a layer takes (16 us at
+// one row, 20 at eight) is the exchanges, 1.1 to 2.2 us each with the loads that are waited for before them, and 0.5 to 1.3 us of dependent instructions in every phase. Where the
+// weights are asked for was found by trying: behind a phase's products and before its barrier, before the values leave, a phase earlier or later cost 1 to 5 %, a single register
+// that the compiler keeps in memory 10 (it is read back behind the weights on their way), and weights by pointers of any kind, which LDS's waits wait for too, 15.
 //
 // Numbers as in the kernels this replaces: the norm's weight on the row rounded to bfloat16 as an operand and the row's factor on the finished
 // sum, queries, keys, values, attention's result and act rounded to bfloat16, everything else float.
@@ -132,7 +135,8 @@ struct Wait {      // of one wave: the area as a buffer resource (reads past the
     do {
       asm volatile("" ::: "memory");      // (read anew every time)
 #pragma unroll
-      for (int i = 0; i < N; ++i) v[i] = two(at(i));
+      for (int i = 0; i < N; ++i)
+        v[i] = two(at(i));
       bool here = true;
 #pragma unroll
       for (int i = 0; i < N; ++i) here &= v[i][1] == stamp && v[i][3] == stamp;
@@ -148,6 +152,7 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
   constexpr int KS = kResMaxWidth / 32 / kResWaves;          // steps of 32 along K a wave takes at most (4)
   constexpr int GT = 3, DT = 2, DK = kResMaxFF / kResShares / 32 / kResWaves;      // tiles of gate and up, of down; down's steps a wave (3)
   constexpr int kRowWaves = MB >= 8 ? 1 : 8 / MB, kRounds = MB == 16 ? 2 : 1;      // waves that share a row on its way in; rows a wave takes one after the other
+  constexpr bool kEarlyDown = MB <= 4;                       // (more rows on their way in leave no registers for a part of down's weights as well)
   constexpr int kLdx = kResMaxWidth + 8;                     // bfloat16 numbers from row to row of the operand in LDS (not on the same banks)
   __shared__ __attribute__((aligned(16))) bf16_t xs[MB * kLdx];
   constexpr int kRed = 20;                                   // floats from row to row of a tile's sums
@@ -219,19 +224,16 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
     const bool up = r >= 2 * np;
     fetch_pairs(wg[t], layer.w_gate + static_cast<int64_t>(2 * p0) * H * 2, row_of(up ? r - 2 * np : r, H) + (up ? apart : 0), H);
   };
-  auto fetch_down = [&](gbytes matrix) __attribute__((always_inline)) {
+  auto fetch_down = [&](int t, gbytes matrix) __attribute__((always_inline)) {
     const auto [f0, nf] = down_columns();
     const int steps = share_length() / 32;
     gbytes from = matrix + (static_cast<int64_t>(f0) * FF + share_of() * share_length()) * 2;
+    const int r = t * 16 + c16;
+    const uint32_t row = row_of(r < nf ? r : nf - 1, FF);
 #pragma unroll
-    for (int t = 0; t < DT; ++t) {
-      const int r = t * 16 + c16;
-      const uint32_t row = row_of(r < nf ? r : nf - 1, FF);
-#pragma unroll
-      for (int j = 0; j < DK; ++j) {
-        const int s = wave + kResWaves * j;
-        wd[t][j] = load_global<u32x4>(from + (s < steps ? s : 0) * 64 + row);
-      }
+    for (int j = 0; j < DK; ++j) {
+      const int s = wave + kResWaves * j;
+      wd[t][j] = load_global<u32x4>(from + (s < steps ? s : 0) * 64 + row);
     }
   };
   // the operand's fragment: row c16 of the rows (beyond M: row M - 1, a column of the result that nobody reads); beyond the last step zeros
@@ -263,10 +265,13 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
   auto in_ok = [&](int i) __attribute__((always_inline)) { return i * 64 + lane < in_len() && in_at(i) < H / 2; };
   typedef float f32x2 __attribute__((ext_vector_type(2)));
   f32x2 nw[2];      // two weights of either norm, on their way to LDS
+  float bias = 0.f;    // of the column of queries, keys and values that this thread finishes
   auto fetch_norms = [&](const ResidentLayer& layer) __attribute__((always_inline)) {
     const int at = 2 * tid < H ? 2 * tid : 0;
     nw[0] = *reinterpret_cast<ALOFA_GLOBAL const f32x2*>(layer.norm0 + at);
     nw[1] = *reinterpret_cast<ALOFA_GLOBAL const f32x2*>(layer.norm1 + at);
+    const auto [q0, nq] = qkv_columns();
+    if (a.has_bias) bias = layer.b_qkv[q0 + ((tid & 15) < nq ? (tid & 15) : 0)];
   };
   auto leave_norms = [&]() __attribute__((always_inline)) {
     if (2 * tid < H) {
@@ -387,6 +392,7 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
   fetch_cols(wq, layer.w_qkv, qkv_columns().first, qkv_columns().n, H);
   fetch_norms(layer);
   leave_norms();
+  if (has_step) fetch_step(st, layer, first_tile, page0, page1);
   __syncthreads();
 
 #pragma unroll 1
@@ -398,25 +404,30 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
     anew();
     const int fn = tid & 15, fm = tid >> 4;      // the output this thread finishes: column, row
     const auto [q0, nq] = qkv_columns();
-    float bias = 0.f;
-    if (a.has_bias && fn < nq && fm < M) bias = layer.b_qkv[q0 + fn];
     __syncthreads();
+    const float factor_a = factor(ssq[0], fm < M ? fm : 0, a.eps0);
     {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      bf16x8 x[KS];
 #pragma unroll
-      for (int j = 0; j < KS; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wq[j]), operand(step_of(j), H / 32), acc, 0, 0, 0);
+      for (int j = 0; j < KS; ++j) x[j] = operand(step_of(j), H / 32);
+#pragma unroll
+      for (int j = 0; j < KS; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wq[j]), x[j], acc, 0, 0, 0);
       leave_sums(1, 0, acc);
     }
-    if (has_step) fetch_step(st, layer, first_tile, page0, page1);
-    else st = Step{};      // (nothing of the layer before is kept)
     __syncthreads();
     if (fn < nq && fm < M) {
-      const float v = sum_of(1, 0, fm, fn) * factor(ssq[0], fm, a.eps0) + bias;
+      const float v = sum_of(1, 0, fm, fn) * factor_a + bias;
       put(a.area + kAtQkv + fm * NQ + q0 + fn, static_cast<uint32_t>(f32_to_bf16(v)), w.stamp);
     }
 
     // ---- B
     anew();
+    auto fetch_ahead = [&]() __attribute__((always_inline)) {
+      fetch_cols(wo, layer.w_o, own_columns().first, own_columns().n, KO);
+      fetch_gate_up(0, layer);
+    };
+    if (!attends) fetch_ahead();
     if (attends) {
       const int item = tid / 16, chan = 2 * (tid % 16);      // head `item` (group: the key, group + 1: the value), channels chan, chan + 1 and their partners 32 on
       if (item < group + 2) {
@@ -514,6 +525,7 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
         tile += 2 * kResWaves;
         if (tile < tile_end) fetch_step(st, layer, tile, page_of(tile), page_of(tile + 1));
       }
+      fetch_ahead();
       sum = rows_sum(sum);
       float* mine = red + (wave * kResMaxGroup + c16) * (d + 4);
       if (g == 0 && c16 < kResMaxGroup) {
@@ -545,8 +557,6 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
 
     // ---- C
     anew();
-    fetch_cols(wo, layer.w_o, own_columns().first, own_columns().n, KO);
-    fetch_gate_up(0, layer);
     if (meets) {
       float big = -FLT_MAX, total = 0.f, acc = 0.f;
       float ms[2], ls[2], vs[2];
@@ -590,19 +600,22 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
         if ((lane & 1) == 0) put(a.area + kAtAttn + cm * (KO / 2) + ch * 32 + lane / 2, pack_bf16x2(x, y), w.stamp);
       }
     }
-    fetch_gate_up(1, layer);
 
     // ---- D
     anew();
+    fetch_gate_up(1, layer);
+    if (kEarlyDown) fetch_down(0, layer.w_down);
     take_packed(std::integral_constant<int, (kResMaxWidth / 4 / 64 + kRowWaves - 1) / kRowWaves>(), kAtAttn, KO / 2, KO / 4);
     __syncthreads();
     {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      bf16x8 x[KS];
 #pragma unroll
-      for (int j = 0; j < KS; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wo[j]), operand(step_of(j), KO / 32), acc, 0, 0, 0);
+      for (int j = 0; j < KS; ++j) x[j] = operand(step_of(j), KO / 32);
+#pragma unroll
+      for (int j = 0; j < KS; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wo[j]), x[j], acc, 0, 0, 0);
       leave_sums(1, 0, acc);
     }
-    fetch_gate_up(2, layer);
     __syncthreads();
     const int on = tid & 15, om = tid >> 4;
     const auto [h0, nh] = own_columns();
@@ -614,32 +627,32 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
 
     // ---- E
     anew();
+    fetch_gate_up(2, layer);
     take_rows(kAtRowsA, false, 1);
+    anew();
     __syncthreads();
+    const float factor_e = factor(ssq[1], (tid >> 5) < M ? tid >> 5 : 0, a.eps1);
     {
       f32x4 acc[GT];
+      bf16x8 x[KS];
 #pragma unroll
       for (int t = 0; t < GT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < KS; ++j) {
-        const bf16x8 x = operand(step_of(j), H / 32);
+      for (int j = 0; j < KS; ++j) x[j] = operand(step_of(j), H / 32);
 #pragma unroll
-        for (int t = 0; t < GT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wg[t][j]), x, acc[t], 0, 0, 0);
-      }
+      for (int j = 0; j < KS; ++j)
+#pragma unroll
+        for (int t = 0; t < GT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wg[t][j]), x[j], acc[t], 0, 0, 0);
 #pragma unroll
       for (int t = 0; t < GT; ++t) leave_sums(GT, t, acc[t]);
     }
-    fetch_down(layer.w_down);
-    const bool more = l + 1 < a.n_layers;
-    next_layer(more ? l + 1 : l);      // (behind the last layer its own once more: a load under a condition would keep the old registers)
-    fetch_norms(layer);
     __syncthreads();
     {
       const int n = tid & 31, m = tid >> 5;      // column 2 p0 + n of act
       const auto [p0, np] = act_pairs();
       if (n < 2 * np && m < M) {
         const int u = 2 * np + n;
-        const float f = factor(ssq[1], m, a.eps1);
+        const float f = factor_e;
         const float gate = sum_of(GT, n >> 4, m, n & 15) * f, up = sum_of(GT, u >> 4, m, u & 15) * f;
         const float x = gate_of<false>(gate) * up, y = lane_xor1(x);
         if ((n & 1) == 0) put(a.area + kAtAct + m * (FF / 2) + p0 + n / 2, pack_bf16x2(x, y), w.stamp);
@@ -648,8 +661,9 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
 
     // ---- F
     anew();
+    if (!kEarlyDown) fetch_down(0, layer.w_down);
+    fetch_down(1, layer.w_down);
     take_packed(std::integral_constant<int, (kResMaxFF / kResShares / 4 / 64 + kRowWaves - 1) / kRowWaves>(), kAtAct + share_of() * (share_length() / 2), FF / 2, share_length() / 4);
-    leave_norms();
     __syncthreads();
     {
       f32x4 acc[DT];
@@ -664,7 +678,6 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
 #pragma unroll
       for (int t = 0; t < DT; ++t) leave_sums(DT, t, acc[t]);
     }
-    fetch_cols(wq, layer.w_qkv, qkv_columns().first, qkv_columns().n, H);
     __syncthreads();
     {
       const int n = tid & 31, m = tid >> 5;
@@ -674,6 +687,10 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
 
     // ---- G
     anew();
+    const bool more = l + 1 < a.n_layers;
+    next_layer(more ? l + 1 : l);      // (behind the last layer its own once more: a load under a condition would keep the old registers)
+    fetch_cols(wq, layer.w_qkv, qkv_columns().first, qkv_columns().n, H);
+    fetch_norms(layer);
     {
       const int m = tid / 16, n = tid / 4 % 4, pair = tid % 4;      // two shares a thread
       const auto [h0, nh] = own_columns();
@@ -691,6 +708,10 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
         else a.hidden[static_cast<int64_t>(m) * H + h0 + n] = w.dead ? __uint_as_float(0x7fc00000u) : x;
       }
     }
+    if (has_step) fetch_step(st, layer, first_tile, page0, page1);
+    else st = Step{};      // (nothing of the layer before is kept)
+    leave_norms();
+    __syncthreads();      // (and the waves without a column wait here and not by asking for rows that cannot be there yet)
   }
   // the next step's stamps go on from here (every block has read `base` before this one could finish its last layer)
   if (b == 0 && tid == 0) __hip_atomic_store(a.area, static_cast<u64>(base + a.n_layers), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
