@@ -35,7 +35,7 @@
 // that the compiler keeps in memory 10 (it is read back behind the weights on their way), and weights by pointers of any kind, which LDS's waits wait for too, 15.
 //
 // Numbers as in the kernels this replaces: the norm's weight on the row rounded to bfloat16 as an operand and the row's factor on the finished
-// sum, queries, keys, values, attention's result and act rounded to bfloat16, everything else float.
+// sum, queries and keys (once, when they have been turned), values, attention's result and act rounded to bfloat16, everything else float.
 #include "common.h"
 
 #include <float.h>
@@ -418,7 +418,7 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
     __syncthreads();
     if (fn < nq && fm < M) {
       const float v = sum_of(1, 0, fm, fn) * factor_a + bias;
-      put(a.area + kAtQkv + fm * NQ + q0 + fn, static_cast<uint32_t>(f32_to_bf16(v)), w.stamp);
+      put(a.area + kAtQkv + fm * NQ + q0 + fn, v, w.stamp);
     }
 
     // ---- B
@@ -435,11 +435,10 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
         const int at = kAtQkv + am * NQ + row * d + chan;
         u32x4 v[2];
         if (!w.dead) w.pairs(v, [&](int i) { return at + 32 * i; });
-        uint32_t lo = v[0][0] | (v[0][2] << 16), hi = v[1][0] | (v[1][2] << 16);
+        const float a0 = __uint_as_float(v[0][0]), a1 = __uint_as_float(v[0][2]), b0 = __uint_as_float(v[1][0]), b1 = __uint_as_float(v[1][2]);
+        uint32_t lo = pack_bf16x2(a0, a1), hi = pack_bf16x2(b0, b1);
         if (item <= group) {
-#pragma clang fp contract(off)
           const float2 angle_c = *reinterpret_cast<const float2*>(angles[0] + chan), angle_s = *reinterpret_cast<const float2*>(angles[1] + chan);
-          const float a0 = __uint_as_float(lo << 16), a1 = __uint_as_float(lo & 0xffff0000u), b0 = __uint_as_float(hi << 16), b1 = __uint_as_float(hi & 0xffff0000u);
           lo = pack_bf16x2(a0 * angle_c.x - b0 * angle_s.x, a1 * angle_c.y - b1 * angle_s.y);
           hi = pack_bf16x2(b0 * angle_c.x + a0 * angle_s.x, b1 * angle_c.y + a1 * angle_s.y);
         }
