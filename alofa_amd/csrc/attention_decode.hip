@@ -76,6 +76,50 @@ struct MapsForm {
   int d_true;
 };
 
+// Blocks dealt out by length (`deal` blocks a token on average, at most 64 tokens, one lane each): a token's keys are cut into as many parts as it takes for none to have
+// more than a quota of tiles, the least of five quotas between an even share of all tiles and one that always fits for which the blocks suffice. Every wave finds the
+// same from the positions alone (four sums over the lanes, independent of one another, some 0.2 us). One number of parts for all leaves the launch
+// waiting for the longest request. us a step of the 0.5B sizes (24 layers, 14/2 heads of 64), so many parts each / dealt out: 64 tokens of 128 to 2,048 keys 1,410 / 1,379, 64 of 700
+// 1,317 / 1,314, 64 of 32 to 500 1,255 / 1,255, 48 of 16 to 300 1,213 / 1,215. Not where a token has four parts or more on average: 32 of 512 to 768 1,160 / 1,175 (24 of 64 to 1,500 1,178 / 1,154), and not
+// for heads of 128: 32 tokens of 28/4 heads, 128 to 1,024 keys, even; 8 of 500 to 800 1.4 % slower.
+constexpr int kMostDealt = 8;
+struct Dealt {
+  int token, position, part, parts;      // token -1: a block too many
+};
+__device__ __forceinline__ Dealt deal_out(const int32_t* __restrict__ positions, int tokens, int blocks, int block, int lane) {
+  const int position = positions[lane < tokens ? lane : 0];
+  const float tiles = lane < tokens ? static_cast<float>((position >> 4) + 1) : 0.f;
+  const float total = wave_sum(tiles);
+  const float least = total / static_cast<float>(blocks), most = total / static_cast<float>(blocks - tokens);
+  // (half a tile less: never a whole multiple of the quota, so that the division's rounding decides nothing)
+  auto cut = [&](float quota) { return tiles > 0.f ? fminf(floorf((tiles - 0.5f) * __builtin_amdgcn_rcpf(quota)) + 1.f, static_cast<float>(kMostDealt)) : 0.f; };
+  float parts = 0.f, quota = 0.f;
+  bool found = false;
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    constexpr float kSteps[5] = {0.f, 0.125f, 0.25f, 0.5f, 1.f};
+    const float tried = ceilf(least + (most - least) * kSteps[k] - 1e-3f), mine = cut(tried);
+    const bool fits = k == 4 || wave_sum(mine) <= static_cast<float>(blocks);
+    parts = fits && !found ? mine : parts;
+    quota = fits && !found ? tried : quota;
+    found = found || fits;
+  }
+  // (so many parts each where that leaves none with a fifth more: more parts of one token are more to add up)
+  const int each = blocks / tokens;
+  if (wave_max(tiles) <= 1.2f * quota * static_cast<float>(each)) parts = lane < tokens ? static_cast<float>(each) : 0.f;
+  float upto = parts;      // parts of the lanes up to this one
+  upto += dpp_move<kRowShr1, 0xf>(0.f, upto);
+  upto += dpp_move<kRowShr2, 0xf>(0.f, upto);
+  upto += dpp_move<kRowShr4, 0xf>(0.f, upto);
+  upto += dpp_move<kRowShr8, 0xf>(0.f, upto);
+  upto += dpp_move<kRowBcast15, 0xa>(0.f, upto);
+  upto += dpp_move<kRowBcast31, 0xc>(0.f, upto);
+  const int before = __popcll(__ballot(lane < tokens && upto <= static_cast<float>(block)));
+  if (before >= tokens) return Dealt{-1, 0, 0, 1};
+  const int parts_here = static_cast<int>(read_lane(parts, before));
+  return Dealt{before, __builtin_amdgcn_readlane(position, before), block - (static_cast<int>(read_lane(upto, before)) - parts_here), parts_here};
+}
+
 struct Pair8 {
   uint4 lo, hi;
 };
@@ -108,7 +152,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
     const int32_t* __restrict__ block_table, int max_blocks, const int32_t* __restrict__ req_of_token,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ rows, int heads, int kv_heads,
     int bs_shift, int window, float scale, RopeArgs rope, int* __restrict__ counters, int v_head, float* __restrict__ out32, int value_heads, int64_t plane,
-    const float* __restrict__ sink, int block_heads, MapsForm maps) {
+    const float* __restrict__ sink, int block_heads, MapsForm maps, int deal) {
   static_assert(!kMaps || kSplit, "two maps: with split weights");
   static_assert(!kRope || DT % (kMaps ? 8 : 4) == 0, "the rotation needs a channel and its partner in the same lane: d (of one map: d / 2) a multiple of 64");
   constexpr int d = DT * 16;
@@ -120,7 +164,18 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
   const int chunks = (group + block_heads - 1) / block_heads;
   // the tokens served are rows[0..gridDim.x) of the packed batch, or all of it
   // (value_heads > 0: blockIdx.x counts (token, value head) pairs: every value head in turn serves all key heads, and its results go to a plane of their own)
-  const int served = value_heads > 0 ? blockIdx.x / value_heads : blockIdx.x;
+  // (deal > 0: the blocks are dealt out by length, see deal_out)
+  int place = blockIdx.x, part = blockIdx.z, n_parts = gridDim.z, room = gridDim.z;      // where the token's parts are kept, which this is, how many, room for how many
+  int known_position = -1;
+  if constexpr (kRope && !kMaps) {
+    if (deal > 0) {
+      const Dealt dealt = deal_out(positions, gridDim.x / deal, gridDim.x, blockIdx.x, threadIdx.x % 64);
+      if (dealt.token < 0) return;      // (uniform over the block)
+      known_position = dealt.position;
+      place = dealt.token, part = dealt.part, n_parts = dealt.parts, room = kMostDealt;
+    }
+  }
+  const int served = value_heads > 0 ? place / value_heads : place;
   if (value_heads > 0) {
     v_head = blockIdx.x % value_heads;
     out32 += static_cast<int64_t>(v_head) * plane;
@@ -130,13 +185,13 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
   const int hv = v_head >= 0 ? v_head : hk;      // the value head whose values the weights meet (v_head >= 0: one for all key heads)
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int c16 = lane % 16, g = lane / 16;
-  const int n_parts = gridDim.z, n_splits = n_parts * NW, split = blockIdx.z * NW + wave;
+  const int n_splits = n_parts * NW, split = part * NW + wave;
   // The chain of dependent loads is what a short context's attention takes its time from: position and request ->
   // pages -> keys. With one token per request the request is the token's own number (req_of_token may be null
   // then), and the first 64 pages of its table set out at once, before the position says which pages are needed.
   const int32_t* table = block_table + static_cast<int64_t>(req_of_token ? req_of_token[t] : t) * max_blocks;
   int my_page = table[lane < max_blocks ? lane : max_blocks - 1];
-  const int p = positions[t];
+  const int p = known_position >= 0 ? known_position : positions[t];
   const int lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
   // the visible keys lo..p lie in the 16-key tiles first..last; a wave takes a contiguous run of tiles
   // (kMaps: first the tiles of the kept tokens, then the window's; a tile's number counts along both, and from `kept_tiles` on `gap` leads to its place)
@@ -502,7 +557,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
     if (n_parts == 1) {
       put_out(out, out32, static_cast<int64_t>(t) * out_stride + static_cast<int64_t>(h) * d + c, acc / total);
     } else {
-      float* dst = partial + ((static_cast<int64_t>(blockIdx.x) * heads + h) * n_parts + blockIdx.z) * (d + 2);
+      float* dst = partial + ((static_cast<int64_t>(place) * heads + h) * room + part) * (d + 2);
       if (counters) {   // (device scope: written through to memory, where blocks on every die find it)
         __hip_atomic_store(dst + 2 + c, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (c == 0) {
@@ -524,7 +579,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __syncthreads();
   if (threadIdx.x == 0) {
-    int* counter = counters + blockIdx.x * gridDim.y + blockIdx.y;
+    int* counter = counters + place * gridDim.y + blockIdx.y;
     const int arrived = atomicAdd(counter, 1);
     last_block = arrived == n_parts - 1;
     if (last_block) atomicExch(counter, 0);
@@ -534,7 +589,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
   if constexpr (kMaps) {
     head_end([&](int i, int c) {
-      const float* src = partial + (static_cast<int64_t>(blockIdx.x) * heads + hk * group + h0 + i) * n_parts * (d + 2);
+      const float* src = partial + (static_cast<int64_t>(place) * heads + hk * group + h0 + i) * room * (d + 2);
       float big = -FLT_MAX, total = 0.f, acc = 0.f;
       constexpr int kMost = 8;      // (parts that are handed over; their loads set out together)
       float ms[kMost], ls[kMost], vs[kMost];
@@ -566,7 +621,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
       const int i = x / d, c = x % d;
       if (h0 + i >= group) break;
       const int head = hk * group + h0 + i;
-      const float* src = partial + (static_cast<int64_t>(blockIdx.x) * heads + head) * n_parts * (d + 2);
+      const float* src = partial + (static_cast<int64_t>(place) * heads + head) * room * (d + 2);
       const float s2 = sink ? sink[head] * 1.44269504088896340736f : -FLT_MAX;
       float big = s2, total = 0.f, acc = 0.f;
       if (n_parts <= 16) {
@@ -610,7 +665,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
     return;
   } else {
     const int here = min(block_heads, group - h0);      // heads of this block
-    auto states_of = [&](int i) { return partial + (static_cast<int64_t>(blockIdx.x) * heads + hk * group + h0 + i) * n_parts * (d + 2); };
+    auto states_of = [&](int i) { return partial + (static_cast<int64_t>(place) * heads + hk * group + h0 + i) * room * (d + 2); };
     auto finish = [&](int i, int c, float big, float total, float acc, float s2) {
       if (sink) total += __builtin_amdgcn_exp2f(s2 - big);
       put_out(out, out32, static_cast<int64_t>(t) * out_stride + static_cast<int64_t>(hk * group + h0 + i) * d + c, acc / total);
@@ -849,19 +904,25 @@ extern "C" int alofa_attention_decode_v(void* out, int64_t out_stride, float* pa
   const int group = heads / kv_heads;
   const RopeArgs rope{cos_t, sin_t, slots};
   dim3 grid(tokens, kv_heads * ((group + block_heads - 1) / block_heads), n_splits);
+  // where one launch turns the new tokens of many requests, sees all their keys and hands two or three parts of each over, the same blocks go to the requests by their length (deal_out)
+  const int deal = fused && !two_maps && counters && n_splits > 1 && d == 64 && n_splits <= 3 && tokens > 32 && tokens <= kWave && !rows && window == 0 &&
+                           alofa_attention_decode_can_hand_over(tokens, heads, kv_heads, d, kMostDealt, block_heads)
+                       ? n_splits
+                       : 0;
+  if (deal) grid = dim3(tokens * n_splits, grid.y, 1);
 #define ALOFA_DECODE(DT, NW, ROPE)                                                                                        \
   if (two_maps) attention_decode_kernel<DT, NW, ROPE && DT % 8 == 0, true, true><<<grid, 64 * NW, 0, stream>>>(                 \
       static_cast<bf16_t*>(out), out_stride, partial, static_cast<const bf16_t*>(q), q_stride,                            \
       static_cast<bf16_t*>(k_cache), static_cast<bf16_t*>(v_cache), block_table, max_blocks, req_of_token,                \
-      positions, rows, heads, kv_heads, bs_shift, window, scale, rope, counters, v_head, out32, value_heads, plane, sink, block_heads, maps); \
+      positions, rows, heads, kv_heads, bs_shift, window, scale, rope, counters, v_head, out32, value_heads, plane, sink, block_heads, maps, deal); \
   else if (split && !ROPE) attention_decode_kernel<DT, NW, false, true><<<grid, 64 * NW, 0, stream>>>(                         \
       static_cast<bf16_t*>(out), out_stride, partial, static_cast<const bf16_t*>(q), q_stride,                            \
       static_cast<bf16_t*>(k_cache), static_cast<bf16_t*>(v_cache), block_table, max_blocks, req_of_token,                \
-      positions, rows, heads, kv_heads, bs_shift, window, scale, rope, counters, v_head, out32, value_heads, plane, sink, block_heads, maps);       \
+      positions, rows, heads, kv_heads, bs_shift, window, scale, rope, counters, v_head, out32, value_heads, plane, sink, block_heads, maps, deal);       \
   else attention_decode_kernel<DT, NW, ROPE><<<grid, 64 * NW, 0, stream>>>(                                                    \
       static_cast<bf16_t*>(out), out_stride, partial, static_cast<const bf16_t*>(q), q_stride,                            \
       static_cast<bf16_t*>(k_cache), static_cast<bf16_t*>(v_cache), block_table, max_blocks, req_of_token,                \
-      positions, rows, heads, kv_heads, bs_shift, window, scale, rope, counters, v_head, out32, value_heads, plane, sink, block_heads, maps)
+      positions, rows, heads, kv_heads, bs_shift, window, scale, rope, counters, v_head, out32, value_heads, plane, sink, block_heads, maps, deal)
   if (fused) {
     switch (d / 64) {
       case 1: ALOFA_DECODE(4, 8, true); break;

@@ -642,6 +642,48 @@ def test_decode_attention_that_rotates_and_writes_the_new_token(heads, kv_heads,
         o.attention_decode(again, t(qkv, torch.bfloat16), kc, vc, c["table"][:n - 1], None, c["pos"], heads, kv_heads, d, window, scale, bucket, scratch)
 
 
+@pytest.mark.parametrize("heads,kv_heads", [(14, 2), (20, 1), (3, 3)])
+@pytest.mark.parametrize("parts", [2, 3])
+@pytest.mark.parametrize("n,kind", [(33, "spread"), (33, "one long"), (40, "alike"), (63, "spread"), (64, "spread"), (64, "one long"), (64, "single keys")])
+def test_decode_attention_whose_blocks_are_dealt_out_by_length(n, kind, heads, kv_heads, parts):
+    """Many requests of one new token each, whose parts follow their lengths: against the plain attention, and the same bits again."""
+    d, bs = 64, 16
+    rng = np.random.default_rng(23)
+    lens = {"spread": [int(round(np.exp(rng.uniform(0, np.log(600))))) for _ in range(n)], "one long": [3 + r % 5 for r in range(n - 1)] + [1500],
+            "alike": [250 + r % 30 for r in range(n)], "single keys": [1] * n}[kind]
+    c = paged_case(rng, lens, [1] * n, heads, kv_heads, d, bs, torch.bfloat16)
+    cos, sin = pm.rope_table(max(lens), d, 1e4)
+    o = ops()
+    assert o.decode_hand_over(n, heads, kv_heads, d, 8)
+    qkv = np.zeros((n, (heads + 2 * kv_heads) * d), np.float32)
+    kc, vc, table = c["kc"].clone(), c["vc"].clone(), c["table"].cpu().numpy()
+    slots, refs = [], []
+    for r, L in enumerate(lens):
+        q_raw, k_raw = bf(rng.standard_normal((1, heads * d)).astype(np.float32)), bf(rng.standard_normal((1, kv_heads * d)).astype(np.float32))
+        q_rot, k_rot = (bf(pm.rope_apply(x, cos, sin, np.array([L - 1]), d).astype(np.float32)) for x in (q_raw, k_raw))
+        k = c["k"][r].copy()
+        k[L - 1] = k_rot[0]
+        qkv[r] = np.concatenate([q_raw[0], k_raw[0], c["v"][r][L - 1]])
+        slot = int(table[r, (L - 1) // bs]) * bs + (L - 1) % bs
+        slots.append(slot)
+        kc[slot // bs, :, slot % bs] = float("nan")
+        vc[slot // bs, :, :, slot % bs] = float("nan")
+        refs.append((pm.attention(q_rot, k, c["v"][r], heads, kv_heads, d, None), k_rot[0]))
+    scale = float(np.float32(1) / np.sqrt(np.float32(d)))
+    rope = (t(cos[:, :d // 2]), t(sin[:, :d // 2]), t(np.array(slots, np.int64), torch.int64))
+    outs = []
+    for _ in range(3):
+        out, kc2, vc2 = torch.full((n, heads * d), float("nan"), device=DEV, dtype=torch.bfloat16), kc.clone(), vc.clone()
+        o.attention_decode(out, t(qkv, torch.bfloat16), kc2, vc2, c["table"], None, c["pos"], heads, kv_heads, d, None, scale, 2048, None, rope=rope, n_splits=parts, hand_over=True)
+        outs.append(out)
+    close(outs[0], np.concatenate([a for a, _ in refs]), BF16, "attention")
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    got = kc2.float().cpu().numpy()
+    for (_, key), slot in zip(refs, slots):
+        close(got[slot // bs, :, slot % bs].reshape(-1), key, BF16, "new key in its slot")
+    assert torch.isfinite(vc2[[s // bs for s in slots], :, :, [s % bs for s in slots]].float()).all()
+
+
 @pytest.mark.parametrize("heads,kv_heads,d", [(5, 1, 80), (2, 2, 96), (3, 1, 64)])
 def test_decode_attention_with_many_splits(heads, kv_heads, d):
     """One token over 5,000 keys, the launch shaped for a far longer context: the keys are shared out
