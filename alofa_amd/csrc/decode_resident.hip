@@ -694,6 +694,8 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
       const int m = tid / 16, n = tid / 4 % 4, pair = tid % 4;      // two shares a thread
       const auto [h0, nh] = own_columns();
       const int first = h0, own = nh;
+      // (behind the last layer: whether any wave of the launch has given a wait up, asked together with the shares)
+      const u64 stopped = more ? 0 : __hip_atomic_load(a.area + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const bool mine = m < M && n < own;
       u32x4 v[1] = {u32x4{0u, 0u, 0u, 0u}};
       if (!w.dead && wave * 4 < M) w.pairs(v, [&](int) { return kAtDown + ((first + (n < own ? n : 0)) * M + (m < M ? m : 0)) * kResShares + 2 * pair; });
@@ -704,7 +706,7 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
         const float x = hs[m * 4 + n] + sum;
         hs[m * 4 + n] = x;
         if (more) put(a.area + kAtRowsB + m * H + h0 + n, x, w.stamp + 1);
-        else a.hidden[static_cast<int64_t>(m) * H + h0 + n] = w.dead ? __uint_as_float(0x7fc00000u) : x;
+        else a.hidden[static_cast<int64_t>(m) * H + h0 + n] = w.dead || stopped != 0 ? __uint_as_float(0x7fc00000u) : x;
       }
     }
     if (has_step) fetch_step(st, layer, first_tile, page0, page1);

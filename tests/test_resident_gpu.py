@@ -130,3 +130,14 @@ def test_areas_are_used_again():
     idle = [a for areas in _areas._idle.values() for a in areas]
     assert area in idle
     assert engine(m, 1, 32, "bfloat16").step_fn.resident.area in idle
+
+
+def test_a_wait_given_up_is_an_error_of_the_next_step():
+    """The word that the kernel sets, set by the host."""
+    from alofa_amd.errors import AlofaError
+    eng = engine(model(256, 4, 1, 512, "bfloat16", layers=1), 1, 32, "bfloat16")
+    stand(eng, [3], 1)
+    assert torch.isfinite(decode(eng, [[1]])[0]).all()
+    eng.step_fn.resident.failed[0] = 1
+    with pytest.raises(AlofaError):
+        decode(eng, [[1]])
