@@ -152,6 +152,10 @@ class CacheManager:
                                    for t in need.tensors}
             for i, need in state_needs.items():
                 self.state[i] = torch.zeros((max_requests, *need.shape), dtype=need.dtype, device=device)
+        self._slots = None      # on the GPU: every tensor's slot is cleared in one launch
+        if self.state and all(t.is_cuda for t in self.state.values()):
+            from ..ops import StateSlots
+            self._slots = StateSlots(list(self.state.values()))
 
     def device_bytes(self) -> int:
         """Bytes of device memory the pages and the state slots take."""
@@ -171,8 +175,11 @@ class CacheManager:
             raise AlofaError("invalid_argument", "duplicate request id", f"request={req}")
         slot = hostlib.check(self._lib.alofa_cache_admit(self._h))
         self.requests[req] = slot
-        for t in self.state.values():
-            t[slot].zero_()
+        if self._slots is not None:
+            self._slots.clear(slot)
+        else:
+            for t in self.state.values():
+                t[slot].zero_()
         return slot
 
     def has(self, req) -> bool:

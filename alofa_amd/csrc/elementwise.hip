@@ -309,3 +309,30 @@ extern "C" int alofa_swiglu(void* out, const void* gate, const void* up, int dty
     ALOFA_REQUIRE(false, "swiglu: unknown dtype %d", dtype);
   return check_launch("swiglu");
 }
+
+// ---- the state of a new request ---------------------------------------------------------------
+// One launch clears the slot in every tensor that keeps state: `places` holds per tensor the address of its first slot and the bytes of one (blockIdx.y: the tensor, blockIdx.x a run of
+// kClearRun bytes of its slot). A tensor at a time is a launch and some 8 us of the host each, 26 a request for eight layers that keep state: four prompts of 96 to 500 tokens and eight
+// decode steps at a width of 1,024 5,712 us a tensor at a time, 5,596 so, alone (nothing in front on the stream) 6,672 and 6,144.
+namespace alofa {
+constexpr int64_t kClearRun = 256 * 16 * 4;
+__global__ void __launch_bounds__(256) clear_slots_kernel(const int64_t* __restrict__ places, int slot) {
+  const int64_t bytes = places[2 * blockIdx.y + 1], begin = blockIdx.x * kClearRun;
+  if (begin >= bytes) return;
+  const int64_t end = begin + kClearRun < bytes ? begin + kClearRun : bytes;
+  char* at = reinterpret_cast<char*>(places[2 * blockIdx.y]) + slot * bytes;
+  if ((reinterpret_cast<uintptr_t>(at) | static_cast<uintptr_t>(bytes)) % 16 == 0) {
+    for (int64_t i = begin + threadIdx.x * 16; i < end; i += 256 * 16) *reinterpret_cast<uint4*>(at + i) = make_uint4(0, 0, 0, 0);
+  } else {      // (slots of no whole sixteen bytes)
+    for (int64_t i = begin + threadIdx.x; i < end; i += 256) at[i] = 0;
+  }
+}
+}  // namespace alofa
+
+// places [n, 2] in device memory; longest: the most bytes a slot has.
+extern "C" int alofa_clear_slots(const int64_t* places, int n, int slot, int64_t longest, hipStream_t stream) {
+  using namespace alofa;
+  ALOFA_REQUIRE(places && n > 0 && n <= 65535 && slot >= 0 && longest > 0, "clear_slots: n=%d slot=%d longest=%lld", n, slot, static_cast<long long>(longest));
+  clear_slots_kernel<<<dim3(static_cast<unsigned>((longest + kClearRun - 1) / kClearRun), n), 256, 0, stream>>>(places, slot);
+  return check_launch("clear_slots");
+}

@@ -823,6 +823,26 @@ def attention_decode(out, q, k_cache, v_cache, block_table, req_of_token, positi
           _I(planes), _L(out.stride(0) if planes else 0), _ptr(_sink_of(sink, heads)), _I(block_heads), _I(0), _I(0), _F(0.0), _F(0.0), _F(0.0), _F(0.0), _I(d), _stream())
 
 
+# ------------------------------------------------------------- state of requests
+
+class StateSlots:
+    """The tensors that keep state per request ([slots, ...], contiguous, on the GPU), whose slot of a new request is cleared in one launch."""
+
+    def __init__(self, tensors: list):
+        self.tensors = [_contig("state", _gpu("state", t)) for t in tensors if t.numel()]      # (kept: the table holds their addresses)
+        self.slots = min((t.shape[0] for t in self.tensors), default=0)
+        sizes = [t[0].numel() * t.element_size() for t in self.tensors]
+        self.longest = max(sizes, default=0)
+        self.places = torch.tensor([(t.data_ptr(), n) for t, n in zip(self.tensors, sizes)], dtype=torch.int64, device=self.tensors[0].device) if self.tensors else None
+
+    def clear(self, slot: int) -> None:
+        if self.places is None:
+            return
+        if not 0 <= slot < self.slots:
+            raise AlofaError("out_of_range", "no such slot", f"slot={slot} slots={self.slots}")
+        _call("alofa_clear_slots", self.places, _I(self.places.shape[0]), _I(slot), _L(self.longest), _L(_stream()))
+
+
 # ---------------------------------------------------- decode steps in one launch
 
 def resident_takes(hidden: int, intermediate: int, heads: int, kv_heads: int, d: int, page: int) -> bool:

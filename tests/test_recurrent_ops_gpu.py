@@ -262,3 +262,20 @@ def test_norm_filter_and_state_in_one_launch(taps, exact):
         ops.keep_last_rows(apart, normed, rows)
         ops.norm_conv_step(got, x, nw, nb, 1e-5, w, fused, rows, exact)
         assert torch.equal(got, want) and torch.equal(fused, apart)
+
+
+@pytest.mark.parametrize("shapes", [[(3, 4)], [(16, 64, 64), (3, 5), (1,), (1029,)], [(4097,), (7, 4096), (33, 257)]])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_the_slot_of_a_new_request_is_cleared_in_every_tensor_and_no_other(shapes, dtype):
+    from alofa_amd import ops
+    from alofa_amd.errors import AlofaError
+    tensors = [torch.randn((3, *s), device="cuda").to(dtype) for s in shapes]
+    want = [t.clone() for t in tensors]
+    slots = ops.StateSlots(tensors)
+    for slot in (1, 2, 0):
+        slots.clear(slot)
+        for w, t in zip(want, tensors):
+            w[slot].zero_()
+            assert torch.equal(w, t)
+    with pytest.raises(AlofaError):
+        slots.clear(3)
