@@ -3,7 +3,7 @@ function: the table of the layers' matrices and caches, an area of memory that t
 kernel sets if it gives a wait up."""
 from __future__ import annotations
 
-import ctypes
+import contextlib
 import threading
 import weakref
 from typing import Optional
@@ -41,6 +41,35 @@ class _Areas:
 
 
 _areas = _Areas()
+
+
+class _Turn:
+    """Steps that run in one launch go one after the other, whichever threads and streams of this process they come from: the launch's blocks hold half of
+    every compute unit until all of them have come, so that two launches fit (another process may have the other half), a third may not. A step on another stream than
+    the last one's waits for what that stream had been given; on the same stream nothing is added. Held while the step is launched, not while it runs."""
+    _lock = threading.Lock()
+    _last: dict = {}      # device -> the stream of the last such step
+
+    def __init__(self, device: torch.device):
+        self.device = device
+
+    def __enter__(self):
+        self._lock.acquire()
+        try:
+            here, last = torch.cuda.current_stream(self.device), self._last.get(self.device.index)
+            if last is not None and last != here:
+                reached = torch.cuda.Event()
+                reached.record(last)
+                here.wait_event(reached)
+            self._last[self.device.index] = here
+        except BaseException:
+            self._lock.release()
+            raise
+        return self
+
+    def __exit__(self, *exc):
+        self._lock.release()
+        return False
 
 
 class ResidentLayers:
@@ -100,6 +129,10 @@ class ResidentLayers:
     def takes(self, ctx, rows: int) -> bool:
         """Whether this step runs in one launch: one new token for each of few requests."""
         return rows <= self.MOST_ROWS and ctx.max_q_len == 1 and len(ctx.spans) == rows
+
+    def turn(self, entries: list):
+        """What a step of these entries is launched within."""
+        return _Turn(self.device) if len(entries) <= self.MOST_ROWS and all(len(e.tokens) == 1 for e in entries) else contextlib.nullcontext()
 
     def check(self) -> None:
         if self._failed[0]:

@@ -433,8 +433,13 @@ class StepFunction:
         the logits, int32 [wanted] with the first index of every wanted row's highest
         logit, and leaves the same in the token store at the row's request's slot.
         The buffer is re-used by the next step."""
-        if self.resident is not None:
-            self.resident.check()
+        if self.resident is None:
+            return self._run(entries, greedy)
+        self.resident.check()
+        with self.resident.turn(entries):
+            return self._run(entries, greedy)
+
+    def _run(self, entries: list, greedy: bool) -> Optional[torch.Tensor]:
         with ops.stream_scope():
             if self.use_graphs and self.watch is None and all(len(e.tokens) == 1 and list(e.want) == [0] for e in entries):
                 return self._run_decode_graph(entries, greedy)

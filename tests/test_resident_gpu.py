@@ -107,6 +107,40 @@ def test_steps_in_turn_do_not_disturb_one_another():
             assert torch.equal(decode(eng, row[None, :rows])[0], alone[rows][k]), (k, rows)
 
 
+def test_threads_with_streams_of_their_own_take_turns():
+    import threading
+    tokens = np.random.default_rng(4).integers(0, VOCAB, (40, 8))
+    m = model(896, 14, 2, 4864, "bfloat16")
+    sizes = (1, 3, 8, 2)
+    want = []
+    for rows in sizes:
+        eng = engine(m, rows, 100, "bfloat16")
+        stand(eng, [20 + i for i in range(rows)], 6)
+        want.append(torch.stack(decode(eng, tokens[:, :rows])))
+    engines = [engine(m, rows, 100, "bfloat16") for rows in sizes]
+    for rows, eng in zip(sizes, engines):
+        stand(eng, [20 + i for i in range(rows)], 6)
+        decode(eng, tokens[:1, :rows])      # (captured here: a capture forbids what other threads may be doing)
+    torch.cuda.synchronize()
+    got, start = {}, threading.Barrier(len(sizes))
+
+    def run(k):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                start.wait()
+                got[k] = torch.stack(decode(engines[k], tokens[1:, :sizes[k]]))
+        except BaseException as e:
+            got[k] = e
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(len(sizes))]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    for k in range(len(sizes)):
+        assert isinstance(got[k], torch.Tensor), got[k]
+        assert torch.equal(got[k], want[k][1:]), k
+
+
 def test_what_it_does_not_take_runs_kernel_by_kernel():
     assert engine(model(896, 14, 2, 4864, "bfloat16"), 2, 64, "bfloat16").step_fn.resident is not None
     assert engine(model(896, 14, 2, 4864, "float32"), 2, 64, "float32").step_fn.resident is None
