@@ -1304,6 +1304,25 @@ def test_the_gates_own_division():
     assert bool(fine.all())
 
 
+@pytest.mark.parametrize("act,exact", [("silu", lambda x: x / (1 + torch.exp(-x))), ("gelu_tanh", lambda x: x / (1 + torch.exp(-2 * (2 / np.pi) ** 0.5 * (x + 0.044715 * x ** 3))))])
+def test_gates_whose_quotient_is_far_below_one(act, exact):
+    """Divisors between 2^126 and the largest float: the quotient, 1e-38 to 1e-36, is as near as any other."""
+    lo, hi = (-88.6, -87.0) if act == "silu" else (-10.05, -9.9)
+    z = torch.linspace(lo, hi, 1024, device=DEV)
+    w = torch.zeros(1024, 64, device=DEV, dtype=torch.bfloat16)
+    w[:, 0] = z.bfloat16()
+    w[:, 1] = (z - w[:, 0].float()).bfloat16()      # (the two add up to sixteen bits of z)
+    a, up = torch.zeros(96, 64, device=DEV, dtype=torch.bfloat16), torch.zeros_like(w)
+    a[:, :2], up[:, 0] = 1.0, 1.0
+    out = torch.empty(96, 1024, device=DEV, dtype=torch.bfloat16)
+    ops().gemm_swiglu(out, a, w, up, kernel="wide", act=act)
+    x = w[:, 0].double() + w[:, 1].double()
+    # half a unit of bfloat16's last place, and what 32 bits leave of an exponent near 88 (2^-24 of it, in each of at most eight roundings) beside the quotient
+    bound = (2.0 ** -8 + 8 * 88 * 2.0 ** -24) * exact(x).abs()
+    assert bool(((out.double() - exact(x)).abs() <= bound).all())
+    assert bool((out != 0).all())
+
+
 # with the gate and for bfloat16 and float outputs (kind 1, 2, 0) on either side of their lines: K under 1,536 and under 768
 @pytest.mark.parametrize("M,N,K,kind,taken", [(171, 4864, 896, 1, 0), (202, 4864, 896, 1, 1), (2048, 4864, 896, 1, 1), (2048, 4864, 736, 1, 0), (819, 8960, 1536, 1, 1), (107, 5632, 2048, 1, 0),
                                               (2048, 1152, 896, 2, 0), (2453, 1152, 896, 2, 1), (2453, 1152, 896, 0, 0), (3760, 896, 896, 0, 1)])
