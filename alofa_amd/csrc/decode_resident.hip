@@ -500,7 +500,7 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
         float add = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          pw[i] = pw[i] > -FLT_MAX ? __builtin_amdgcn_exp2f(pw[i] - m_new) : 0.f;
+          pw[i] = pw[i] <= -FLT_MAX ? 0.f : __builtin_amdgcn_exp2f(pw[i] - m_new);      // (a score that is no number stays one)
           add += pw[i];
         }
         sum = sum * corr + add;

@@ -89,6 +89,25 @@ def test_one_launch_is_as_near_the_32_bit_path_as_the_kernels_it_replaces(shape,
         assert torch.equal(a, b), (step, (a != b).sum(1).tolist(), (a - b).abs().amax(1).tolist(), lengths)
 
 
+@pytest.mark.parametrize("name", ["k", "v"])
+def test_a_cached_key_or_value_that_is_no_number_reaches_the_logits(name):
+    """NaN in one request's cache, in its first tile of keys, one in the middle and its last: that row is NaN, the others keep their bits."""
+    lengths, page = [300, 40, 600], 16
+    tokens = [[5, 6, 7]]
+    m = model(896, 14, 2, 4864, "bfloat16")
+    eng = engine(m, 3, 700, "bfloat16", page)
+    stand(eng, lengths, 9)
+    clean = decode(eng, tokens)[0]
+    for at in (3, 299, 590):
+        eng = engine(m, 3, 700, "bfloat16", page)
+        stand(eng, lengths, 9)
+        block = eng.cache.table(2, 0)[at // page]
+        t = eng.cache.tensors[(1, 0)][name]
+        (t[block, 1, at % page] if name == "k" else t[block, 1, :, at % page]).fill_(float("nan"))
+        got = decode(eng, tokens)[0]
+        assert torch.isnan(got[2]).all() and torch.equal(got[:2], clean[:2]), at
+
+
 def test_steps_in_turn_do_not_disturb_one_another():
     """Two engines with areas of their own, of different rows, and steps that are no decode steps in between."""
     tokens = np.random.default_rng(3).integers(0, VOCAB, (12, 8))
