@@ -729,15 +729,24 @@ static int launch_resident(const ResidentArgs& a, hipStream_t stream) {
 // Bytes of an area (uncached device memory; it is never given back to the runtime: tensors that took the place of such memory have held wrong values).
 extern "C" int64_t alofa_resident_area_bytes() { return static_cast<int64_t>(alofa::kAreaPlaces) * 8; }
 
+// An area as it was when new, zeros, behind everything that the device has been given. Not to be called under graph capture.
+extern "C" int alofa_resident_area_clear(void* area) {
+  using namespace alofa;
+  ALOFA_REQUIRE(area, "resident_area_clear: no area");
+  hipError_t e = hipDeviceSynchronize();
+  if (e == hipSuccess) e = hipMemset(area, 0, kAreaPlaces * 8);
+  if (e == hipSuccess) e = hipDeviceSynchronize();
+  ALOFA_REQUIRE(e == hipSuccess, "resident_area_clear: %s", hipGetErrorString(e));
+  return 0;
+}
+
 // A new area, zeros. Not to be called under graph capture.
 extern "C" int alofa_resident_area(void** area) {
   using namespace alofa;
   *area = nullptr;
-  hipError_t e = hipExtMallocWithFlags(area, kAreaPlaces * 8, hipDeviceMallocUncached);
-  if (e == hipSuccess) e = hipMemset(*area, 0, kAreaPlaces * 8);
-  if (e == hipSuccess) e = hipDeviceSynchronize();
+  const hipError_t e = hipExtMallocWithFlags(area, kAreaPlaces * 8, hipDeviceMallocUncached);
   ALOFA_REQUIRE(e == hipSuccess, "resident_area: %s", hipGetErrorString(e));
-  return 0;
+  return alofa_resident_area_clear(*area);
 }
 
 // How many blocks share a row and key head's keys: as many as there are blocks for, at most sixteen.

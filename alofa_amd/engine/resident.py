@@ -17,25 +17,37 @@ from ..parts.block import PreNormBlock
 from ..parts.feed_forward import SwiGLU
 
 
+class _Area:
+    """Memory that the blocks of a launch exchange values in, and the pinned word that the kernel sets if it gives a wait up."""
+
+    def __init__(self):
+        self.address = ops.resident_area()
+        self.failed = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+
+
 class _Areas:
     """Areas that step functions of this process have given back. They are never freed (uncached device memory must not be), so there are never
-    more of them than step functions lived at one time. One that changes hands has no launch in flight: the taker waits for the device first."""
+    more of them than step functions lived at one time. One that changes hands has no launch in flight: the taker waits for the device first. One
+    whose owner failed is cleared then: the word that stops its launches is still set, and its counter and its values may not belong together."""
 
     def __init__(self):
         self._lock = threading.Lock()
-        self._idle: dict = {}      # device -> addresses
+        self._idle: dict = {}      # device -> areas
 
-    def take(self, device: torch.device) -> int:
+    def take(self, device: torch.device) -> _Area:
         with self._lock:
             idle = self._idle.get(device.index)
-            known = idle.pop() if idle else None
-        if known is not None:
-            torch.cuda.synchronize(device)
-            return known
+            area = idle.pop() if idle else None
         with torch.cuda.device(device):
-            return ops.resident_area()
+            if area is None:
+                return _Area()
+            torch.cuda.synchronize(device)
+            if area.failed.item():
+                ops.clear_resident_area(area.address)
+                area.failed.zero_()
+        return area
 
-    def give_back(self, device: torch.device, area: int) -> None:
+    def give_back(self, device: torch.device, area: _Area) -> None:
         with self._lock:
             self._idle.setdefault(device.index, []).append(area)
 
@@ -123,7 +135,7 @@ class ResidentLayers:
         self.layers = torch.tensor(rows, dtype=torch.int64, device=device)
         self.area = _areas.take(device)
         weakref.finalize(self, _areas.give_back, device, self.area)
-        self.failed = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self.failed = self.area.failed
         self._failed = self.failed.numpy()
 
     def takes(self, ctx, rows: int) -> bool:
@@ -141,5 +153,5 @@ class ResidentLayers:
     def forward(self, ctx, hidden: torch.Tensor) -> None:
         self.check()
         cos, sin = self.position.table(ctx.n_positions)
-        ops.decode_resident(hidden, self.layers, ctx.positions, ctx._tables[self.group], ctx._slots[self.group], cos, sin, self.area, self.failed, self.intermediate,
+        ops.decode_resident(hidden, self.layers, ctx.positions, ctx._tables[self.group], ctx._slots[self.group], cos, sin, self.area.address, self.failed, self.intermediate,
                             self.heads, self.kv_heads, self.d, self.page, self.biased, self.scale, self.eps)

@@ -858,6 +858,11 @@ def resident_area() -> int:
     return place.value
 
 
+def clear_resident_area(area: int) -> None:
+    """An area as it was when new; no launch that uses it may be in flight."""
+    _call("alofa_resident_area_clear", _L(area))
+
+
 def decode_resident(hidden: torch.Tensor, layers: torch.Tensor, positions: torch.Tensor, block_table: torch.Tensor, slots: torch.Tensor, cos: torch.Tensor,
                     sin: torch.Tensor, area: int, failed: torch.Tensor, intermediate: int, heads: int, kv_heads: int, d: int, page: int, biased: bool, scale: float, eps: tuple) -> None:
     """Every layer of a decode step, one new token per row, row i request i: ``hidden`` float32 [rows, width], in and out. ``layers`` int64 [layers, 10]: the addresses of a

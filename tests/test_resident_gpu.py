@@ -185,6 +185,40 @@ def test_areas_are_used_again():
     assert engine(m, 1, 32, "bfloat16").step_fn.resident.area in idle
 
 
+def write(address, words):
+    """64-bit words into device memory that no tensor stands for."""
+    import ctypes
+    hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+    block = (ctypes.c_uint64 * len(words))(*words)
+    assert hip.hipMemcpy(ctypes.c_void_p(address), block, ctypes.c_size_t(8 * len(words)), 1) == 0      # (1: host to device)
+
+
+def test_the_area_of_a_step_function_that_failed_serves_the_next_one():
+    """What such a launch leaves behind, written by the host: the stop word, a counter that has gone on, values that bear the numbers of steps to come."""
+    import gc
+    from alofa_amd.engine.resident import _areas
+    m = model(256, 4, 1, 512, "bfloat16", layers=2)
+    tokens = [[1], [2], [3]]
+
+    def run():
+        eng = engine(m, 1, 32, "bfloat16")
+        stand(eng, [3], 1)
+        return eng, decode(eng, tokens)
+    gc.collect()
+    _areas._idle.clear()      # (those of other tests stay out of it)
+    eng, want = run()
+    area, address = eng.step_fn.resident.area, eng.step_fn.resident.area.address
+    torch.cuda.synchronize()
+    write(address, [6, 1] + [0] * 30 + [(7 + i % 5) << 32 | 0x3f800000 for i in range(400000)])      # (all of the places, with numbers that come next)
+    area.failed[0] = 1
+    del eng, area
+    gc.collect()
+    eng, got = run()
+    assert eng.step_fn.resident.area.address == address
+    assert all(torch.equal(a, b) for a, b in zip(got, want)), [torch.isnan(x).any().item() for x in got]
+    assert eng.step_fn.resident.failed.item() == 0
+
+
 def test_a_wait_given_up_is_an_error_of_the_next_step():
     """The word that the kernel sets, set by the host."""
     from alofa_amd.errors import AlofaError
