@@ -34,7 +34,7 @@ import numpy as np
 import torch
 
 from .. import ops
-from ..errors import AlofaError
+from ..errors import AlofaError, LostResults
 from ..sampling.sampler import SampleParams, Sampler, SplitMix64
 from .scheduler import Action, SchedConfig, SchedInput, Scheduler
 from .step import TOKEN_ON_DEVICE, StepEntry, StepFunction
@@ -59,6 +59,7 @@ class Request:
     shared: int = 0                  # prompt tokens taken over from another request's pages
     pending: int = 0                 # tokens chosen on the device whose values have not been read back yet
     on_device: bool = False          # the last chosen token lies in the step function's token store
+    lost: bool = False               # ended because a step lost its results: no output
 
 
 class EngineCore:
@@ -74,6 +75,7 @@ class EngineCore:
         self.share_prefixes = bool(share_prefixes)
         self.shared_tokens = 0
         self.cache = step_fn.cache
+        self._steps_stand = getattr(step_fn, "check", None) or (lambda: None)      # an error where a step that has run lost its results
         # the scheduler counts the pages of every group of layers: one rule per group (a scheduler with a single
         # rule over several groups counts for all of them with it, so every pool must hold what it counts)
         rules, pools = sched_cfg.groups, [g.pool.n_blocks for g in self.cache.groups]
@@ -135,6 +137,8 @@ class EngineCore:
         return r.state == DONE and r.pending == 0
 
     def output(self, req: int) -> list:
+        if self.requests[req].lost:
+            raise LostResults("a step lost the results that this request's tokens come from", f"request={req}")
         return list(self.requests[req].out)
 
     def release(self, req: int) -> None:
@@ -243,6 +247,27 @@ class EngineCore:
         self.shared_tokens += got
         return got
 
+    def _check_steps(self) -> None:
+        """Asked behind every wait for a step's results, before they are used. Where some are lost, so are the requests that
+        have pages or tokens on their way (which of them the step was for is not known by then): they end without output, and the engine goes on with the others."""
+        try:
+            self._steps_stand()
+        except LostResults:
+            self._give_up()
+            raise
+
+    def _give_up(self) -> None:
+        self._inflight.clear()
+        for r in self.requests.values():
+            if r.state != RESIDENT and not r.pending:
+                continue
+            if r.state == RESIDENT:
+                self._drop(r)
+                if r.id not in self._cancels:
+                    self._cancels.append(r.id)
+                r.state = DONE
+            r.pending, r.on_device, r.lost = 0, False, True
+
     # ------------------------------------------------------------------ choice
     def _stage(self):
         """Small pinned blocks (taking turns, as a block's copy runs only when the GPU gets there)
@@ -334,6 +359,7 @@ class EngineCore:
             for i, tok in zip(order, sent[1][:sent[2]].tolist()):
                 values[i] = int(tok)
         rows = logits[torch.tensor(host, device=logits.device)].cpu().numpy()
+        self._check_steps()
         for k, i in enumerate(host):
             r = reqs[i]
             self.sampler.build(rows[k], r.params, r.prompt + r.out)
@@ -345,8 +371,9 @@ class EngineCore:
         """Read back the tokens that earlier choices sent on their way, oldest first, all but the
         newest ``keep`` sets. A request that was preempted since, or released, no longer takes its token."""
         while len(self._inflight) > keep:
-            owed, tokens, n, event = self._inflight.popleft()
-            event.synchronize()
+            self._inflight[0][3].synchronize()
+            self._check_steps()
+            owed, tokens, n, _ = self._inflight.popleft()
             for (rid, life), tok in zip(owed, tokens[:n].tolist()):
                 r = self.requests.get(rid)
                 if r is not None and r.preemptions == life and r.pending > 0:
@@ -384,6 +411,7 @@ class EngineCore:
     def tick(self) -> int:
         """One whole tick; returns the rows that ran. When it returns, the tokens of the tick
         before are in the outputs (all of them with ``run_ahead`` off)."""
+        self._check_steps()
         entries, owes = self.prepare()
         self.ticks += 1
         self.last_rows = sum(len(e.tokens) for e in entries)
@@ -392,7 +420,11 @@ class EngineCore:
             # where every request that is owed a token takes the first maximum, the step chooses by itself
             # (the vocabulary product leaves no logits then)
             by_step = bool(wanted) and all(self.requests[o].params.plain and r_is_greedy(self.requests[o]) for o in wanted)
-            result = self.fn.run(entries, greedy=by_step)
+            try:
+                result = self.fn.run(entries, greedy=by_step)
+            except LostResults:      # (those of a step before, known only now)
+                self._give_up()
+                raise
             chosen = (self.choose(None, wanted, result) if by_step else self.choose(result, wanted)) if wanted else []
             self.settle(owes, chosen)
             self.collect(keep=1 if self.run_ahead else 0)

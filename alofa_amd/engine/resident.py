@@ -11,7 +11,7 @@ from typing import Optional
 import torch
 
 from .. import ops
-from ..errors import AlofaError
+from ..errors import AlofaError, LostResults
 from ..parts.attention import GQAAttention
 from ..parts.block import PreNormBlock
 from ..parts.feed_forward import SwiGLU
@@ -148,7 +148,7 @@ class ResidentLayers:
 
     def check(self) -> None:
         if self._failed[0]:
-            raise AlofaError("not_initialized", "a decode step gave up waiting for blocks that another kernel kept off the GPU; its results are lost")
+            raise LostResults("a decode step gave up waiting for blocks that another kernel kept off the GPU; its results are lost")
 
     def forward(self, ctx, hidden: torch.Tensor) -> None:
         self.check()

@@ -432,12 +432,19 @@ class StepFunction:
         is wanted. With ``greedy`` the step chooses by itself: it returns, instead of
         the logits, int32 [wanted] with the first index of every wanted row's highest
         logit, and leaves the same in the token store at the row's request's slot.
-        The buffer is re-used by the next step."""
+        The buffer is re-used by the next step. The step runs when the GPU gets there; ``check`` says
+        afterwards whether its results stand."""
+        self.check()
         if self.resident is None:
             return self._run(entries, greedy)
-        self.resident.check()
         with self.resident.turn(entries):
             return self._run(entries, greedy)
+
+    def check(self) -> None:
+        """An error (``LostResults``) if a step that has run lost its results. To be called behind a copy or an event that
+        waits for the step, before what it left is used; every ``run`` asks for the steps before it."""
+        if self.resident is not None:
+            self.resident.check()
 
     def _run(self, entries: list, greedy: bool) -> Optional[torch.Tensor]:
         with ops.stream_scope():

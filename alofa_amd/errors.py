@@ -23,3 +23,10 @@ class AlofaError(Exception):
         if detail:
             text += f" [{detail}]"
         super().__init__(text)
+
+
+class LostResults(AlofaError):
+    """What steps that have been launched computed is not to be used: a kernel gave up before it was done."""
+
+    def __init__(self, message: str, detail: str = ""):
+        super().__init__("not_initialized", message, detail)

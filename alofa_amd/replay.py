@@ -98,6 +98,7 @@ class Replayer:
                 self.tokens[e.request].extend(e.tokens)
             if logits is not None:
                 out = logits.detach().cpu().numpy().astype("<f4")
+                self.fn.check()
         for r in rec.get("end", []):
             if self.cache.has(r):
                 self.cache.free(r)

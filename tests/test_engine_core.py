@@ -12,7 +12,8 @@ import pytest
 from alofa_amd.cache import CacheManager
 from alofa_amd.engine.core import EngineCore
 from alofa_amd.engine.scheduler import SchedConfig
-from alofa_amd.errors import AlofaError
+from alofa_amd.engine.step import TOKEN_ON_DEVICE, StepEntry
+from alofa_amd.errors import AlofaError, LostResults
 from alofa_amd.parts import CacheNeed
 
 VOCAB = 97
@@ -275,4 +276,65 @@ def test_many_requests_in_a_wide_batch():
     for i in range(40):
         assert core.output(i) == alone(prompts[i], 5 + i % 4)
         core.release(i)
+    nothing_held(core)
+
+
+class LateStep(FakeStep):
+    """The last token of every request stays with the step, as in the token store."""
+    kept: dict = {}
+
+    def run(self, entries, greedy=False):
+        entries = [StepEntry(e.request, [self.kept[e.request] if t == TOKEN_ON_DEVICE else t for t in e.tokens], e.want) for e in entries]
+        out = super().run(entries, greedy)
+        self.kept = {**self.kept, **dict(zip([e.request for e in entries if e.want], out or []))}
+        return out
+
+
+class LateCore(EngineCore):
+    """Tokens whose values arrive behind an event, as the device's choices do."""
+
+    def choose(self, logits, owes, by_step=None):
+        tokens = np.array(logits if by_step is None else by_step)
+        for o in owes:
+            self.requests[o].on_device = True
+        self._inflight.append(([(o, self.requests[o].preemptions) for o in owes], tokens, len(owes), SimpleNamespace(synchronize=lambda: None)))
+
+
+@pytest.mark.parametrize("when", ["a tick", "the flush behind the last step", "the step"])
+def test_tokens_of_a_step_that_lost_its_results_are_an_error_and_no_output(when):
+    fn = LateStep(64, 4)
+    lost = []
+    fn.check = lambda: lost and (_ for _ in ()).throw(LostResults(lost[0]))
+    core = LateCore(fn, SchedConfig(block_size=4, capacity_blocks=64))
+    core.submit(1, prompt_of(1, 6), 5)
+    core.submit(2, prompt_of(2, 9), 5 if when == "the flush behind the last step" else 9)
+    for _ in range(5 if when == "the flush behind the last step" else 3):
+        core.tick()
+    assert any(core.requests[r].pending for r in (1, 2))
+    had = {r: list(core.requests[r].out) for r in (1, 2)}
+    run = fn.run
+    if when == "the step":      # (known only when the next step is asked for)
+        def run_and_find_out(entries, greedy=False):
+            lost.append("lost")
+            fn.check()
+        fn.run = run_and_find_out
+    else:
+        lost.append("lost")
+    with pytest.raises(LostResults):
+        core.flush() if when == "the flush behind the last step" else core.tick()
+    lost.clear()
+    fn.run = run
+    ended = [r for r in (1, 2) if core.requests[r].lost]
+    assert ended and not core._inflight
+    for r in (1, 2):
+        assert core.is_done(r)
+        if r in ended:
+            assert core.requests[r].out == had[r]
+            with pytest.raises(LostResults):
+                core.output(r)
+        core.release(r)
+    core.submit(3, prompt_of(3, 7), 6)      # (the engine goes on)
+    core.run(50)
+    assert core.output(3) == alone(prompt_of(3, 7), 6)
+    core.release(3)
     nothing_held(core)

@@ -228,3 +228,26 @@ def test_a_wait_given_up_is_an_error_of_the_next_step():
     eng.step_fn.resident.failed[0] = 1
     with pytest.raises(AlofaError):
         decode(eng, [[1]])
+
+
+@pytest.mark.parametrize("how", [{}, {"temperature": 0.8}, {"temperature": 0.8, "top_k": 5}])
+@pytest.mark.parametrize("last", [True, False])
+def test_tokens_of_a_step_that_gave_up_do_not_come_out(how, last):
+    """The word that the kernel sets, set by the host while the step is on its way: the last step of a run, or one before it."""
+    from alofa_amd.errors import LostResults
+    eng = engine(model(256, 4, 1, 512, "bfloat16", layers=1), 2, 32, "bfloat16")
+    steps, run = [], eng.step_fn.run
+
+    def failing(entries, greedy=False):
+        out = run(entries, greedy)
+        steps.append(len(entries))
+        if len(steps) == (4 if last else 2):
+            eng.step_fn.resident.failed[0] = 1
+        return out
+    eng.step_fn.run = failing
+    with pytest.raises(LostResults):
+        eng.generate([[5, 6, 7], [8, 9]], max_new=4, **how)
+    assert len(steps) <= (4 if last else 3)
+    for r in eng.core.requests:
+        with pytest.raises(LostResults):
+            eng.core.output(r)
