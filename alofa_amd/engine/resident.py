@@ -11,7 +11,7 @@ from typing import Optional
 import torch
 
 from .. import ops
-from ..errors import AlofaError, LostResults
+from ..errors import AlofaError
 from ..parts.attention import GQAAttention
 from ..parts.block import PreNormBlock
 from ..parts.feed_forward import SwiGLU
@@ -146,12 +146,10 @@ class ResidentLayers:
         """What a step of these entries is launched within."""
         return _Turn(self.device) if len(entries) <= self.MOST_ROWS and all(len(e.tokens) == 1 for e in entries) else contextlib.nullcontext()
 
-    def check(self) -> None:
-        if self._failed[0]:
-            raise LostResults("a decode step gave up waiting for blocks that another kernel kept off the GPU; its results are lost")
+    def gave_up(self) -> bool:
+        return bool(self._failed[0])
 
     def forward(self, ctx, hidden: torch.Tensor) -> None:
-        self.check()
         cos, sin = self.position.table(ctx.n_positions)
         ops.decode_resident(hidden, self.layers, ctx.positions, ctx._tables[self.group], ctx._slots[self.group], cos, sin, self.area.address, self.failed, self.intermediate,
                             self.heads, self.kv_heads, self.d, self.page, self.biased, self.scale, self.eps)

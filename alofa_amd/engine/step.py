@@ -16,7 +16,7 @@ import torch
 
 from .. import ops
 from ..cache.manager import CacheManager
-from ..errors import AlofaError
+from ..errors import AlofaError, LostResults
 from .resident import ResidentLayers
 
 
@@ -442,9 +442,16 @@ class StepFunction:
 
     def check(self) -> None:
         """An error (``LostResults``) if a step that has run lost its results. To be called behind a copy or an event that
-        waits for the step, before what it left is used; every ``run`` asks for the steps before it."""
-        if self.resident is not None:
-            self.resident.check()
+        waits for the step, before what it left is used; every ``run`` asks for the steps before it. It is said once: from
+        then on all steps run kernel by kernel, which wait for nobody. What the lost steps wrote to their requests' pages is no
+        history to go on from."""
+        if self.resident is None or not self.resident.gave_up():
+            return
+        torch.cuda.synchronize(self.device)      # (what is in flight may be such a launch)
+        most = self.resident.MOST_ROWS
+        self._graphs = {key: graph for key, graph in self._graphs.items() if key[0] > most}
+        self.resident = None
+        raise LostResults("a decode step gave up waiting for blocks that another kernel kept off the GPU; its results are lost")
 
     def _run(self, entries: list, greedy: bool) -> Optional[torch.Tensor]:
         with ops.stream_scope():

@@ -3,6 +3,8 @@ import numpy as np
 import pytest
 import torch
 
+from alofa_amd.engine.step import StepEntry
+
 pytestmark = pytest.mark.gpu
 
 VOCAB, LAYERS = 512, 3
@@ -40,7 +42,6 @@ def engine(m, rows, context, dtype, page=16):
 
 def stand(eng, lengths, seed):
     """Requests 0.. with lengths[i] tokens in the cache."""
-    from alofa_amd.engine.step import StepEntry
     rng = np.random.default_rng(seed)
     for i, n in enumerate(lengths):
         eng.cache.admit(i)
@@ -49,7 +50,6 @@ def stand(eng, lengths, seed):
 
 
 def decode(eng, tokens):
-    from alofa_amd.engine.step import StepEntry
     return [eng.step_fn.run([StepEntry(i, [int(t)], [0]) for i, t in enumerate(row)]).double().cpu() for row in tokens]
 
 
@@ -251,3 +251,30 @@ def test_tokens_of_a_step_that_gave_up_do_not_come_out(how, last):
     for r in eng.core.requests:
         with pytest.raises(LostResults):
             eng.core.output(r)
+
+
+@pytest.mark.parametrize("captured", [True, False])
+def test_behind_a_step_that_gave_up_all_steps_run_kernel_by_kernel(captured):
+    from alofa_amd.errors import LostResults
+    m = model(896, 14, 2, 4864, "bfloat16")
+    tokens = np.random.default_rng(8).integers(0, VOCAB, (4, 3))
+    engines = {}
+    for how in ("one by one", "gave up"):
+        eng = engines[how] = engine(m, 3, 100, "bfloat16")
+        eng.step_fn.use_graphs = captured
+        if how == "one by one":
+            eng.step_fn.resident = None
+        else:
+            eng.cache.admit("before")
+            eng.step_fn.run([StepEntry("before", [5], [0])])
+            eng.step_fn.run([StepEntry("before", [6], [0])])
+            eng.step_fn.resident.failed[0] = 1
+            with pytest.raises(LostResults):
+                eng.step_fn.run([StepEntry("before", [7], [0])])
+            assert eng.step_fn.resident is None
+            eng.cache.free("before")
+        stand(eng, [33, 5, 70], 2)
+    replayed = engines["gave up"].step_fn.graph_replays
+    want, got = (decode(engines[how], tokens) for how in ("one by one", "gave up"))
+    assert all(torch.equal(a, b) for a, b in zip(want, got))
+    assert (engines["gave up"].step_fn.graph_replays > replayed) == captured
