@@ -4,6 +4,9 @@ kernel sets if it gives a wait up."""
 from __future__ import annotations
 
 import contextlib
+import fcntl
+import os
+import tempfile
 import threading
 import weakref
 from typing import Optional
@@ -55,6 +58,58 @@ class _Areas:
 _areas = _Areas()
 
 
+class _Seats:
+    """Which processes run such launches on a GPU: at most two, as many as fit on it at once (a third's blocks and theirs could keep one another waiting). A process
+    holds a lock on one of two files from its first such step function on until it ends, whichever way. Without one of them, or where the files cannot be had, steps
+    run kernel by kernel. (Processes that do not share the folder do not know of one another: there ``ALOFA_ONE_LAUNCH=0`` in all but two.)"""
+
+    def __init__(self, folder: Optional[str] = None):
+        self.folder = folder or tempfile.gettempdir()
+        self._lock = threading.Lock()
+        self._held: dict = {}      # (process, GPU) -> the open file whose lock this process has
+
+    @staticmethod
+    def _open(path: str) -> Optional[int]:
+        flags = os.O_RDWR | os.O_CLOEXEC | os.O_NOFOLLOW
+        for _ in range(2):      # (a file that is there is opened as it is: a sticky folder refuses O_CREAT for another user's)
+            try:
+                return os.open(path, flags)
+            except FileNotFoundError:
+                pass
+            except OSError:
+                return None
+            try:
+                fd = os.open(path, flags | os.O_CREAT | os.O_EXCL, 0o666)
+                os.fchmod(fd, 0o666)
+                return fd
+            except FileExistsError:
+                pass
+            except OSError:
+                return None
+        return None
+
+    def take(self, gpu: str) -> bool:
+        with self._lock:
+            key = (os.getpid(), gpu)      # (a fork has the open file, but not the lock)
+            if key in self._held:
+                return True
+            for n in range(2):
+                fd = self._open(os.path.join(self.folder, f"alofa_amd-one-launch-{gpu}-{n}.lock"))
+                if fd is None:
+                    continue
+                try:
+                    fcntl.lockf(fd, fcntl.LOCK_EX | fcntl.LOCK_NB)
+                except OSError:
+                    os.close(fd)
+                    continue
+                self._held[key] = fd
+                return True
+            return False
+
+
+_seats = _Seats()
+
+
 class _Turn:
     """Steps that run in one launch go one after the other, whichever threads and streams of this process they come from: the launch's blocks hold half of
     every compute unit until all of them have come, so that two launches fit (another process may have the other half), a third may not. A step on another stream than
@@ -92,9 +147,9 @@ class ResidentLayers:
     @classmethod
     def of(cls, model, cache) -> Optional["ResidentLayers"]:
         """None where the model's layers are not what the kernel runs: pre-norm blocks of grouped-query attention over its own cache of every token (rotary, no
-        output bias) and a silu-gated feed-forward, all alike, sizes that fit a block's registers, bfloat16."""
+        output bias) and a silu-gated feed-forward, all alike, sizes that fit a block's registers, bfloat16; or where ``ALOFA_ONE_LAUNCH=0`` or other processes say no."""
         rt, order = model.rt, model.order
-        if rt.exact or rt.dtype is not torch.bfloat16 or model.streams or model.joins or not 0 < len(order) <= cls.MOST_LAYERS:
+        if os.environ.get("ALOFA_ONE_LAUNCH", "1") == "0" or rt.exact or rt.dtype is not torch.bfloat16 or model.streams or model.joins or not 0 < len(order) <= cls.MOST_LAYERS:
             return None
         blocks = [model.blocks[e.layer] for e in order]
         if any(e.cache_of is not None or e.join is not None for e in order) or any(type(b) is not PreNormBlock for b in blocks):
@@ -112,6 +167,8 @@ class ResidentLayers:
                 return None
         m = first.mixer
         if not ops.resident_takes(m.hidden, first.feed_forward.intermediate, m.heads, m.kv_heads, m.d, cache.block_size):
+            return None
+        if not _seats.take(str(torch.cuda.get_device_properties(rt.device).uuid)):
             return None
         return cls(blocks, cache, rt.device)
 

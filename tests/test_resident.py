@@ -1,0 +1,74 @@
+"""Decode steps in one launch: what lies around the launch, without a GPU."""
+import os
+import signal
+
+from alofa_amd.engine.resident import _Seats
+
+
+def another(folder):
+    """Another process that asks for a seat and lives until ``end``: (process, what ends it, whether it has one)."""
+    (said, say), (told, tell) = os.pipe(), os.pipe()
+    pid = os.fork()
+    if pid == 0:
+        try:
+            os.close(tell)
+            os.write(say, b"1" if _Seats(str(folder)).take("gpu") else b"0")
+            os.read(told, 1)
+        finally:
+            os._exit(0)
+    os.close(say), os.close(told)
+    has = os.read(said, 1) == b"1"
+    os.close(said)
+    return (pid, tell), has
+
+
+def end(process, how=None):
+    pid, tell = process
+    if how:
+        os.kill(pid, how)
+    else:
+        os.write(tell, b".")      # (closing it would not do: processes forked later have it open too)
+    os.close(tell)
+    os.waitpid(pid, 0)
+
+
+def test_two_processes_have_a_seat_on_a_gpu_and_a_third_has_none(tmp_path):
+    mine = _Seats(str(tmp_path))
+    assert mine.take("gpu") and mine.take("gpu")      # (one seat, however often it is asked for)
+    second, has = another(tmp_path)
+    assert has
+    third, has = another(tmp_path)
+    assert not has
+    end(third)
+    assert mine.take("another gpu")
+    end(second)      # its seat is free again
+    fourth, has = another(tmp_path)
+    assert has
+    end(fourth, signal.SIGKILL)      # whichever way a process ends
+    fifth, has = another(tmp_path)
+    assert has
+    end(fifth)
+
+
+def test_a_fork_does_not_have_its_parents_seat(tmp_path):
+    seats = _Seats(str(tmp_path))
+    assert seats.take("gpu")
+    other, has = another(tmp_path)
+    assert has
+    pid = os.fork()
+    if pid == 0:
+        os._exit(0 if not seats.take("gpu") else 1)
+    assert os.waitpid(pid, 0)[1] == 0
+    end(other)
+    third, has = another(tmp_path)      # the parent's seat is still held: one was free
+    assert has
+    fourth, has = another(tmp_path)
+    assert not has
+    end(third), end(fourth)
+
+
+def test_no_seat_where_the_files_cannot_be_had(tmp_path):
+    assert not _Seats(str(tmp_path / "none")).take("gpu")
+    for n in range(2):
+        os.symlink("/dev/null", tmp_path / f"alofa_amd-one-launch-gpu-{n}.lock")
+    assert not _Seats(str(tmp_path)).take("gpu")

@@ -278,3 +278,15 @@ def test_behind_a_step_that_gave_up_all_steps_run_kernel_by_kernel(captured):
     want, got = (decode(engines[how], tokens) for how in ("one by one", "gave up"))
     assert all(torch.equal(a, b) for a, b in zip(want, got))
     assert (engines["gave up"].step_fn.graph_replays > replayed) == captured
+
+
+def test_without_a_seat_or_switched_off_steps_run_kernel_by_kernel(monkeypatch):
+    from alofa_amd.engine import resident
+    m = model(256, 4, 1, 512, "bfloat16", layers=1)
+    monkeypatch.setattr(resident._seats, "take", lambda gpu: False)
+    assert engine(m, 1, 32, "bfloat16").step_fn.resident is None
+    monkeypatch.undo()
+    monkeypatch.setenv("ALOFA_ONE_LAUNCH", "0")
+    assert engine(m, 1, 32, "bfloat16").step_fn.resident is None
+    monkeypatch.undo()
+    assert engine(m, 1, 32, "bfloat16").step_fn.resident is not None
