@@ -1,6 +1,8 @@
 """Decode steps in one launch: what lies around the launch, without a GPU."""
 import os
 import signal
+import threading
+from types import SimpleNamespace
 
 from alofa_amd.engine.resident import _Seats
 
@@ -72,3 +74,32 @@ def test_no_seat_where_the_files_cannot_be_had(tmp_path):
     for n in range(2):
         os.symlink("/dev/null", tmp_path / f"alofa_amd-one-launch-gpu-{n}.lock")
     assert not _Seats(str(tmp_path)).take("gpu")
+
+
+def test_a_scope_of_one_thread_leaves_the_streams_of_others_alone(monkeypatch):
+    """Two threads whose scopes overlap, neither within the other: each launches on its own stream inside and outside its scope."""
+    from alofa_amd import ops
+    current = threading.local()
+    monkeypatch.setattr(ops.torch.cuda, "current_stream", lambda *a: SimpleNamespace(cuda_stream=current.stream))
+    current.stream = 1
+    entered, leave, seen = threading.Event(), threading.Event(), {}
+
+    def other():
+        current.stream = 2
+        seen["before"] = ops._stream()
+        with ops.stream_scope():
+            entered.set()
+            leave.wait(30)
+            seen["within"] = ops._stream()
+        seen["behind"] = ops._stream()
+    with ops.stream_scope():
+        t = threading.Thread(target=other)
+        t.start()
+        assert entered.wait(30)
+        assert ops._stream() == 1
+    assert ops._stream() == 1
+    leave.set()
+    t.join(30)
+    assert seen == {"before": 2, "within": 2, "behind": 2}
+    current.stream = 3
+    assert ops._stream() == 3

@@ -290,3 +290,49 @@ def test_without_a_seat_or_switched_off_steps_run_kernel_by_kernel(monkeypatch):
     assert engine(m, 1, 32, "bfloat16").step_fn.resident is None
     monkeypatch.undo()
     assert engine(m, 1, 32, "bfloat16").step_fn.resident is not None
+
+
+def test_prompts_in_one_thread_and_decode_steps_in_others():
+    """Each with a stream of its own, the decode steps laid out and launched one by one (sizes whose kernels hand nothing over in the library's workspace, which is for one stream at a time)."""
+    import threading
+    m = model(256, 4, 1, 512, "bfloat16", layers=2)
+    rng = np.random.default_rng(12)
+    tokens, prompts = rng.integers(0, VOCAB, (30, 3)), rng.integers(0, VOCAB, (30, 9)).tolist()
+
+    def prompt_steps(eng):
+        out = []
+        for p in prompts:
+            eng.cache.admit(0)
+            out.append(eng.step_fn.run([StepEntry(0, p, [8])]).double().cpu())
+            eng.cache.free(0)
+        return torch.stack(out)
+
+    def engines():
+        made = {n: engine(m, 3, 64, "bfloat16") for n in ("prompts", 2, 3)}
+        for n, eng in made.items():
+            eng.step_fn.use_graphs = False
+            if n != "prompts":
+                stand(eng, [11 + i for i in range(n)], 7)
+        torch.cuda.synchronize()
+        return made
+
+    def work(n, eng):
+        return prompt_steps(eng) if n == "prompts" else torch.stack(decode(eng, tokens[:, :n]))
+    want = {n: work(n, eng) for n, eng in engines().items()}
+    got, start = {}, threading.Barrier(3)
+
+    def run(n, eng):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                start.wait()
+                got[n] = work(n, eng)
+        except BaseException as e:
+            got[n] = e
+    threads = [threading.Thread(target=run, args=x) for x in engines().items()]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    for n in want:
+        assert isinstance(got[n], torch.Tensor), got[n]
+        assert torch.equal(got[n], want[n]), n
