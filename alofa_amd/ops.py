@@ -4,6 +4,7 @@ only then launches on torch's current stream. There is no CPU or library
 fallback: a tensor that is not on the GPU, or a missing library, is an error."""
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import operator
 import os
@@ -829,10 +830,13 @@ def attention_decode(out, q, k_cache, v_cache, block_table, req_of_token, positi
 # ------------------------------------------------------------- state of requests
 
 class StateSlots:
-    """The tensors that keep state per request ([slots, ...], contiguous, on the GPU), whose slot of a new request is cleared in one launch."""
+    """The tensors that keep state per request ([slots, ...], contiguous, on one GPU), whose slot of a new request is cleared in one launch: on torch's
+    current stream of that GPU, as an operation of the tensors' own would be, whichever GPU is the current one and whatever scope the caller is in."""
 
     def __init__(self, tensors: list):
         self.tensors = [_contig("state", _gpu("state", t)) for t in tensors if t.numel()]      # (kept: the table holds their addresses)
+        if len({t.device for t in self.tensors}) > 1:
+            raise AlofaError("invalid_argument", "the tensors lie on several GPUs", f"devices={sorted({str(t.device) for t in self.tensors})}")
         self.slots = min((t.shape[0] for t in self.tensors), default=0)
         sizes = [t[0].numel() * t.element_size() for t in self.tensors]
         self.longest = max(sizes, default=0)
@@ -843,7 +847,9 @@ class StateSlots:
             return
         if not 0 <= slot < self.slots:
             raise AlofaError("out_of_range", "no such slot", f"slot={slot} slots={self.slots}")
-        _call("alofa_clear_slots", self.places, _I(self.places.shape[0]), _I(slot), _L(self.longest), _L(_stream()))
+        device = self.places.device
+        with contextlib.nullcontext() if torch.cuda.current_device() == device.index else torch.cuda.device(device):
+            _call("alofa_clear_slots", self.places, _I(self.places.shape[0]), _I(slot), _L(self.longest), _L(torch.cuda.current_stream(device).cuda_stream))
 
 
 # ---------------------------------------------------- decode steps in one launch

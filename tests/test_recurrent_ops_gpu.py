@@ -279,3 +279,25 @@ def test_the_slot_of_a_new_request_is_cleared_in_every_tensor_and_no_other(shape
             assert torch.equal(w, t)
     with pytest.raises(AlofaError):
         slots.clear(3)
+
+
+def test_a_slot_is_cleared_on_the_callers_stream():
+    """Within a scope of another stream, as where another part of the program is in the middle of a step."""
+    from alofa_amd import ops
+    t = torch.ones((3, 1000), device="cuda")
+    slots = ops.StateSlots([t])
+    busy, mine = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(busy):
+        scope = ops.stream_scope()
+        scope.__enter__()
+        torch.cuda._sleep(200_000_000)      # (a kernel that counts clock cycles, some 0.1 s, and ends)
+    try:
+        with torch.cuda.stream(mine):
+            slots.clear(1)
+            got = t.cpu()
+            assert not busy.query()
+    finally:
+        scope.__exit__(None, None, None)
+    busy.synchronize()
+    assert bool((got[1] == 0).all()) and bool((got[[0, 2]] == 1).all())
