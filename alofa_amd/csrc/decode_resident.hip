@@ -26,7 +26,7 @@
 //
 // All blocks have to be on the chip at once. A block takes at most half of a compute unit (eight waves of up to 128 registers, under 80 KB of
 // LDS), so that 256 of them fit beside 256 of another such launch, whatever process it belongs to; kernels that wait for nobody make room by ending.
-// No wait is without end: a wave that has asked kLimit times sets `stop` and `failed`, which end every other wait, and the step's rows are NaN.
+// No wait is without end: a wave that has asked kLimit times sets `stop` and `failed`, which end every other wait, and what it waited for is NaN from then on.
 //
 // A step of the 0.5B sizes (24 layers of 896, 14/2 heads, 4,864; the head's 70 us among them), us, kernel by kernel / this: 1 row of 512 keys 643 / 455, 2 667 / 476,
 // 4 of 512 to 768 715 / 510, 8 785 / 549, 12 of 64 to 700 890 / 616, 16 of 128 to 1,024 937 / 663, 1 of 4,000 707 / 481, 8 of 3,000 to 4,000 860 / 589. What a layer takes (16 us at
@@ -95,7 +95,7 @@ struct ResidentArgs {
   const float* sin_t;
   u64* area;
   int* failed;
-  int n_layers, M, H, FF, heads, kv_heads, max_blocks, bs_shift, parts, has_bias;
+  int n_layers, M, H, FF, heads, kv_heads, max_blocks, bs_shift, parts, has_bias, limit;
   float scale, eps0, eps1;
 };
 
@@ -108,6 +108,7 @@ struct Wait {      // of one wave: the area as a buffer resource (reads past the
   __amdgpu_buffer_rsrc_t area;
   u64* words;
   int* failed;
+  int limit;      // asks until a wait is given up
   uint32_t stamp;
   bool dead;
 
@@ -118,9 +119,9 @@ struct Wait {      // of one wave: the area as a buffer resource (reads past the
   }
   // whether to go on asking (uniform over the wave)
   __device__ __forceinline__ bool again(int& asked) {
-    if ((++asked & 255) == 0) {
+    if ((++asked & 255) == 0 || asked >= limit) {
       dead = __any(__hip_atomic_load(words + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0);
-      if (asked >= kLimit) {
+      if (asked >= limit) {
         __hip_atomic_store(words + 1, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         dead = true;
@@ -128,11 +129,14 @@ struct Wait {      // of one wave: the area as a buffer resource (reads past the
     }
     return !dead;
   }
-  // N pairs of places at first(i), until all bear the stamp
+  // N pairs of places at at(i), until all bear the stamp. Where waits are over the values are NaN, in 32 bits and as two numbers of 16: whatever is computed from
+  // them is NaN and leaves as such, so that no number that a row ends with comes from a wait that was given up, whichever wave gave it up and when.
+  // (told which way is the usual one, the compiler keeps no register in memory: a step of 8 rows 545 -> 529 us, of 12 617 -> 599)
   template <int N, typename At>
   __device__ __forceinline__ void pairs(u32x4 (&v)[N], At&& at) {
+    constexpr uint32_t kNaN = 0x7fc07fc0u;
     int asked = 0;
-    do {
+    if (__builtin_expect(!dead, 1)) do {
       asm volatile("" ::: "memory");      // (read anew every time)
 #pragma unroll
       for (int i = 0; i < N; ++i)
@@ -140,8 +144,10 @@ struct Wait {      // of one wave: the area as a buffer resource (reads past the
       bool here = true;
 #pragma unroll
       for (int i = 0; i < N; ++i) here &= v[i][1] == stamp && v[i][3] == stamp;
-      if (__all(here)) break;
+      if (__builtin_expect(__all(here), 1)) return;
     } while (again(asked));
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i][0] = kNaN, v[i][2] = kNaN;
   }
 };
 
@@ -178,6 +184,7 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
   w.area = __builtin_amdgcn_make_buffer_rsrc(a.area, 0, kAreaPlaces * 8, 0x00020000);
   w.words = a.area;
   w.failed = a.failed;
+  w.limit = a.limit;
   w.dead = false;
   const uint32_t base = static_cast<uint32_t>(__hip_atomic_load(a.area, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 
@@ -292,7 +299,7 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
           const float2 x = *reinterpret_cast<const float2*>(a.hidden + static_cast<int64_t>(m) * H + 2 * (in_ok(i) ? in_at(i) : 0));
           v[i] = u32x4{__float_as_uint(x.x), 0u, __float_as_uint(x.y), 0u};
         }
-      } else if (!w.dead) {
+      } else {
         w.pairs(v, [&](int i) { return from + m * H + 2 * (in_ok(i) ? in_at(i) : in_part_of() * in_len()); });
       }
       // (every lane reads and writes, one without a pair of its own the row's padding: nothing to wait for in between)
@@ -325,7 +332,7 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
       u32x4 v[N];
       auto at = [&](int i) { return in_part * len + i * 64 + lane; };
       auto ok = [&](int i) { return i * 64 + lane < len && at(i) < n; };
-      if (!w.dead) w.pairs(v, [&](int i) { return from + m * stride + 2 * (ok(i) ? at(i) : (in_part * len < n ? in_part * len : 0)); });
+      w.pairs(v, [&](int i) { return from + m * stride + 2 * (ok(i) ? at(i) : (in_part * len < n ? in_part * len : 0)); });
 #pragma unroll
       for (int i = 0; i < N; ++i) *reinterpret_cast<uint2*>(xs + m * kLdx + (ok(i) ? 4 * at(i) : kResMaxWidth)) = make_uint2(v[i][0], v[i][2]);
     }
@@ -430,11 +437,11 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
     if (!attends) fetch_ahead();
     if (attends) {
       const int item = tid / 16, chan = 2 * (tid % 16);      // head `item` (group: the key, group + 1: the value), channels chan, chan + 1 and their partners 32 on
-      if (item < group + 2) {
-        const int row = item < group ? ahk * group + item : item == group ? heads + ahk : heads + kv_heads + ahk;
+      if (wave * 4 < group + 2) {      // (all lanes of a wave ask, those without a head of their own for the first one: a wait is a wave's)
+        const int row = item < group || item > group + 1 ? ahk * group + (item < group ? item : 0) : item == group ? heads + ahk : heads + kv_heads + ahk;
         const int at = kAtQkv + am * NQ + row * d + chan;
         u32x4 v[2];
-        if (!w.dead) w.pairs(v, [&](int i) { return at + 32 * i; });
+        w.pairs(v, [&](int i) { return at + 32 * i; });
         const float a0 = __uint_as_float(v[0][0]), a1 = __uint_as_float(v[0][2]), b0 = __uint_as_float(v[1][0]), b1 = __uint_as_float(v[1][2]);
         uint32_t lo = pack_bf16x2(a0, a1), hi = pack_bf16x2(b0, b1);
         if (item <= group) {
@@ -443,8 +450,10 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
           hi = pack_bf16x2(b0 * angle_c.x + a0 * angle_s.x, b1 * angle_c.y + a1 * angle_s.y);
         }
         bf16_t* to = qs + (item < group ? item : item - group + kResMaxGroup) * 72 + chan;
-        *reinterpret_cast<uint32_t*>(to) = lo;
-        *reinterpret_cast<uint32_t*>(to + 32) = hi;
+        if (item < group + 2) {
+          *reinterpret_cast<uint32_t*>(to) = lo;
+          *reinterpret_cast<uint32_t*>(to + 32) = hi;
+        }
       }
     }
     if (attends) {
@@ -566,7 +575,7 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
         if (part < a.parts) {
           const int at = kAtParts + ((cm * heads + ch) * a.parts + part) * 66;
           u32x4 v[2];
-          if (!w.dead) w.pairs(v, [&](int n) { return at + (n == 0 ? 0 : 2 + (lane & ~1)); });
+          w.pairs(v, [&](int n) { return at + (n == 0 ? 0 : 2 + (lane & ~1)); });
           ms[i] = __uint_as_float(v[0][0]), ls[i] = __uint_as_float(v[0][2]), vs[i] = __uint_as_float((lane & 1) ? v[1][2] : v[1][0]);
         }
       }
@@ -694,11 +703,9 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
       const int m = tid / 16, n = tid / 4 % 4, pair = tid % 4;      // two shares a thread
       const auto [h0, nh] = own_columns();
       const int first = h0, own = nh;
-      // (behind the last layer: whether any wave of the launch has given a wait up, asked together with the shares)
-      const u64 stopped = more ? 0 : __hip_atomic_load(a.area + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const bool mine = m < M && n < own;
       u32x4 v[1] = {u32x4{0u, 0u, 0u, 0u}};
-      if (!w.dead && wave * 4 < M) w.pairs(v, [&](int) { return kAtDown + ((first + (n < own ? n : 0)) * M + (m < M ? m : 0)) * kResShares + 2 * pair; });
+      if (wave * 4 < M) w.pairs(v, [&](int) { return kAtDown + ((first + (n < own ? n : 0)) * M + (m < M ? m : 0)) * kResShares + 2 * pair; });
       float sum = __uint_as_float(v[0][0]) + __uint_as_float(v[0][2]);
       sum += lane_xor1(sum);
       sum += lane_xor2(sum);
@@ -706,7 +713,7 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
         const float x = hs[m * 4 + n] + sum;
         hs[m * 4 + n] = x;
         if (more) put(a.area + kAtRowsB + m * H + h0 + n, x, w.stamp + 1);
-        else a.hidden[static_cast<int64_t>(m) * H + h0 + n] = w.dead || stopped != 0 ? __uint_as_float(0x7fc00000u) : x;
+        else a.hidden[static_cast<int64_t>(m) * H + h0 + n] = x;
       }
     }
     if (has_step) fetch_step(st, layer, first_tile, page0, page1);
@@ -764,10 +771,11 @@ extern "C" int alofa_resident_takes(int H, int FF, int heads, int kv_heads, int 
 }
 
 // hidden [M, H] float32, in and out; layers: n_layers x ten pointers (ResidentLayer) in device memory; positions [M], table [M, max_blocks], slots [M]: the new token's
-// place per row, row i request i; cos, sin [positions, 32]; area: of alofa_resident_area, of one launch at a time; failed: an int in memory that the host reads, set if a wait is given up.
+// place per row, row i request i; cos, sin [positions, 32]; area: of alofa_resident_area, of one launch at a time; failed: an int in memory that the host reads, set if a wait is given up;
+// limit: after how many asks (0: kLimit).
 extern "C" int alofa_decode_resident(float* hidden, const void* layers, const int32_t* positions, const int32_t* table, const int64_t* slots, const float* cos_t,
                                      const float* sin_t, void* area, int* failed, int n_layers, int M, int H, int FF, int heads, int kv_heads, int d, int page, int max_blocks,
-                                     int has_bias, float scale, float eps0, float eps1, hipStream_t stream) {
+                                     int has_bias, int limit, float scale, float eps0, float eps1, hipStream_t stream) {
   using namespace alofa;
   ALOFA_REQUIRE(alofa_resident_takes(H, FF, heads, kv_heads, d, page) && M >= 1 && M <= kResMaxRows && M * kv_heads <= kResBlocks && M * heads <= kResBlocks && n_layers > 0 && n_layers <= kResMaxLayers && max_blocks > 0,
                 "decode_resident: sizes beyond what a block holds (M=%d H=%d FF=%d heads=%d/%d d=%d page=%d)", M, H, FF, heads, kv_heads, d, page);
@@ -775,7 +783,7 @@ extern "C" int alofa_decode_resident(float* hidden, const void* layers, const in
   int shift = 0;
   while ((1 << shift) < page) ++shift;
   const ResidentArgs a = {hidden, static_cast<const ResidentLayer*>(layers), positions, table, slots, cos_t, sin_t, static_cast<u64*>(area), failed, n_layers, M, H, FF, heads, kv_heads,
-                          max_blocks, shift, alofa_resident_parts(M, kv_heads), has_bias, scale, eps0, eps1};
+                          max_blocks, shift, alofa_resident_parts(M, kv_heads), has_bias, limit > 0 ? limit : kLimit, scale, eps0, eps1};
   if (M == 1) return launch_resident<1>(a, stream);
   if (M == 2) return launch_resident<2>(a, stream);
   if (M <= 4) return launch_resident<4>(a, stream);

@@ -873,10 +873,11 @@ def clear_resident_area(area: int) -> None:
 
 
 def decode_resident(hidden: torch.Tensor, layers: torch.Tensor, positions: torch.Tensor, block_table: torch.Tensor, slots: torch.Tensor, cos: torch.Tensor,
-                    sin: torch.Tensor, area: int, failed: torch.Tensor, intermediate: int, heads: int, kv_heads: int, d: int, page: int, biased: bool, scale: float, eps: tuple) -> None:
+                    sin: torch.Tensor, area: int, failed: torch.Tensor, intermediate: int, heads: int, kv_heads: int, d: int, page: int, biased: bool, scale: float, eps: tuple, limit: int = 0) -> None:
     """Every layer of a decode step, one new token per row, row i request i: ``hidden`` float32 [rows, width], in and out. ``layers`` int64 [layers, 10]: the addresses of a
     layer's matrices, norms and caches, which the caller keeps alive and has checked; ``area``: of ``resident_area``, used by one launch at a time; ``failed``: int32 [1] in
-    pinned memory, set if the kernel gives a wait up."""
+    pinned memory, set if the kernel gives a wait up: the numbers that hang on it are NaN then.
+    ``limit``: after how many asks, some microsecond each (0: the kernel's own limit, seconds)."""
     _contig("hidden", _gpu("hidden", hidden, torch.float32, 2))
     M, H = hidden.shape
     _contig("layers", _gpu("layers", layers, torch.int64, 2))
@@ -892,7 +893,7 @@ def decode_resident(hidden: torch.Tensor, layers: torch.Tensor, positions: torch
     if block_table.shape[0] < M or failed.dtype is not torch.int32 or not failed.is_pinned():
         raise AlofaError("shape_mismatch", "a row of pages per request, and a pinned word", f"table={tuple(block_table.shape)} rows={M}")
     _call("alofa_decode_resident", hidden, layers, positions, block_table, slots, cos, sin, _L(area), _L(failed.data_ptr()), _I(layers.shape[0]), _I(M), _I(H), _I(intermediate),
-          _I(heads), _I(kv_heads), _I(d), _I(page), _I(block_table.shape[1]), _I(bool(biased)), _F(scale), _F(eps[0]), _F(eps[1]), _L(_stream()))
+          _I(heads), _I(kv_heads), _I(d), _I(page), _I(block_table.shape[1]), _I(bool(biased)), _I(limit), _F(scale), _F(eps[0]), _F(eps[1]), _L(_stream()))
 
 
 def can_fuse_rope_into_decode(d: int) -> bool:

@@ -336,3 +336,40 @@ def test_prompts_in_one_thread_and_decode_steps_in_others():
     for n in want:
         assert isinstance(got[n], torch.Tensor), got[n]
         assert torch.equal(got[n], want[n]), n
+
+
+@pytest.mark.parametrize("shape,rows", [((256, 4, 1, 512), 1), ((320, 5, 5, 768), 5), ((896, 14, 2, 4864), 2), ((896, 14, 2, 4864), 9), ((1024, 16, 2, 6144), 16)])
+def test_no_number_comes_from_a_wait_that_was_given_up(shape, rows):
+    """Waits given up after 1 to 40 asks, of which an ordinary one takes a few: each row is the right one or has NaN in it, and if one is not the right one, the
+    word says that a wait was given up. Every launch ends."""
+    from alofa_amd import ops
+    m = model(*shape, "bfloat16")
+    lengths = (CONTEXTS * 2)[3:3 + rows]
+    eng = engine(m, rows, max(lengths) + 4, "bfloat16")
+    stand(eng, lengths, 4)
+    fn, res = eng.step_fn, eng.step_fn.resident
+    ctx, ids, _ = fn.begin([StepEntry(i, [7 + i], [0]) for i in range(rows)])
+    start = m[1].embedding.forward(ctx, ids).clone()
+    cos, sin = res.position.table(ctx.n_positions)
+
+    def run(limit):
+        ops.clear_resident_area(res.area.address)
+        res.failed.zero_()
+        hidden = start.clone()
+        ops.decode_resident(hidden, res.layers, ctx.positions, ctx._tables[res.group], ctx._slots[res.group], cos, sin, res.area.address, res.failed, res.intermediate,
+                            res.heads, res.kv_heads, res.d, res.page, res.biased, res.scale, res.eps, limit=limit)
+        torch.cuda.synchronize()
+        return hidden, bool(res.failed.item())
+    want, failed = run(0)
+    assert torch.isfinite(want).all() and not failed
+    given_up = 0
+    for limit in [*range(1, 41), 1, 1, 2, 2, 3, 3]:
+        got, failed = run(limit)
+        given_up += failed
+        right = (got == want).all(1)
+        assert (right | torch.isnan(got).any(1)).all(), (limit, failed)
+        assert failed or right.all(), limit
+    assert given_up > 0      # (a first ask that finds every value there, in every block and phase, is not to be had)
+    ops.clear_resident_area(res.area.address)
+    res.failed.zero_()
+    assert torch.equal(run(0)[0], want)
