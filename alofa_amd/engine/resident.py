@@ -110,25 +110,24 @@ class _Seats:
 _seats = _Seats()
 
 
-class _Turn:
-    """Steps that run in one launch go one after the other, whichever threads and streams of this process they come from: the launch's blocks hold half of
-    every compute unit until all of them have come, so that two launches fit (another process may have the other half), a third may not. A step on another stream than
-    the last one's waits for what that stream had been given; on the same stream nothing is added. Held while the step is launched, not while it runs."""
-    _lock = threading.Lock()
-    _last: dict = {}      # device -> the stream of the last such step
+class _Turns:
+    """Launches of one GPU's steps go one after the other, whichever threads and streams of this process they come from: a launch's blocks hold half of
+    every compute unit until all of them have come, so that two launches fit (another process may have the other half), a third may not. A launch on another stream than
+    the last one's waits for what that stream had been given; on the same stream nothing is added. Held for the launch alone: not while a step is laid out or captured, and not while it runs."""
 
     def __init__(self, device: torch.device):
-        self.device = device
+        self._device, self._lock = device, threading.Lock()
+        self._last: Optional[torch.cuda.Stream] = None      # the stream of the last launch
 
     def __enter__(self):
         self._lock.acquire()
         try:
-            here, last = torch.cuda.current_stream(self.device), self._last.get(self.device.index)
+            here, last = torch.cuda.current_stream(self._device), self._last
             if last is not None and last != here:
                 reached = torch.cuda.Event()
                 reached.record(last)
                 here.wait_event(reached)
-            self._last[self.device.index] = here
+            self._last = here
         except BaseException:
             self._lock.release()
             raise
@@ -137,6 +136,9 @@ class _Turn:
     def __exit__(self, *exc):
         self._lock.release()
         return False
+
+
+_turns: dict = {}      # GPU -> its launches' turns
 
 
 class ResidentLayers:
@@ -194,19 +196,17 @@ class ResidentLayers:
         weakref.finalize(self, _areas.give_back, device, self.area)
         self.failed = self.area.failed
         self._failed = self.failed.numpy()
+        self.turn = _turns.setdefault(device.index, _Turns(device))      # what a launch, or a replay of one, goes within
 
     def takes(self, ctx, rows: int) -> bool:
         """Whether this step runs in one launch: one new token for each of few requests."""
         return rows <= self.MOST_ROWS and ctx.max_q_len == 1 and len(ctx.spans) == rows
-
-    def turn(self, entries: list):
-        """What a step of these entries is launched within."""
-        return _Turn(self.device) if len(entries) <= self.MOST_ROWS and all(len(e.tokens) == 1 for e in entries) else contextlib.nullcontext()
 
     def gave_up(self) -> bool:
         return bool(self._failed[0])
 
     def forward(self, ctx, hidden: torch.Tensor) -> None:
         cos, sin = self.position.table(ctx.n_positions)
-        ops.decode_resident(hidden, self.layers, ctx.positions, ctx._tables[self.group], ctx._slots[self.group], cos, sin, self.area.address, self.failed, self.intermediate,
-                            self.heads, self.kv_heads, self.d, self.page, self.biased, self.scale, self.eps)
+        with contextlib.nullcontext() if torch.cuda.is_current_stream_capturing() else self.turn:      # (one that is captured takes its turn at every replay)
+            ops.decode_resident(hidden, self.layers, ctx.positions, ctx._tables[self.group], ctx._slots[self.group], cos, sin, self.area.address, self.failed, self.intermediate,
+                                self.heads, self.kv_heads, self.d, self.page, self.biased, self.scale, self.eps)

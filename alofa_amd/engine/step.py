@@ -6,8 +6,10 @@ the order given (src/alofa/engine/executor.mojo:555-609 for the row layout,
 :665-859 for the pass)."""
 from __future__ import annotations
 
+import contextlib
 import gc
 import os
+import threading
 from dataclasses import dataclass, field
 from typing import Optional
 
@@ -23,6 +25,8 @@ from .resident import ResidentLayers
 def _pow2_ceil(n: int) -> int:
     return max(64, 1 << (int(n) - 1).bit_length())
 
+
+_capturing = threading.Lock()
 
 TOKEN_ON_DEVICE = -1     # as a StepEntry's only token: the token the last choice for this request left on the device
 
@@ -406,7 +410,8 @@ class StepFunction:
                 gc.collect()
                 gc.disable()
                 try:
-                    with torch.cuda.graph(graph), ops.stream_scope():
+                    # (one capture at a time in the process: torch has one stream for them; steps of other threads go on meanwhile)
+                    with _capturing, torch.cuda.graph(graph, capture_error_mode="thread_local"), ops.stream_scope():
                         hidden = self.model.forward(ctx, buf["ids"])
                         captured = outcome(hidden)
                 finally:
@@ -418,7 +423,8 @@ class StepFunction:
                 # the capture itself ran nothing: the eager results stand
             else:
                 graph, logits = self._graphs[key]
-                graph.replay()
+                with self.resident.turn if self.resident is not None and self.resident.takes(ctx, B) else contextlib.nullcontext():
+                    graph.replay()
                 self.graph_replays += 1
         finally:
             self._scratch = saved
@@ -435,25 +441,6 @@ class StepFunction:
         The buffer is re-used by the next step. The step runs when the GPU gets there; ``check`` says
         afterwards whether its results stand."""
         self.check()
-        if self.resident is None:
-            return self._run(entries, greedy)
-        with self.resident.turn(entries):
-            return self._run(entries, greedy)
-
-    def check(self) -> None:
-        """An error (``LostResults``) if a step that has run lost its results. To be called behind a copy or an event that
-        waits for the step, before what it left is used; every ``run`` asks for the steps before it. It is said once: from
-        then on all steps run kernel by kernel, which wait for nobody. What the lost steps wrote to their requests' pages is no
-        history to go on from."""
-        if self.resident is None or not self.resident.gave_up():
-            return
-        torch.cuda.synchronize(self.device)      # (what is in flight may be such a launch)
-        most = self.resident.MOST_ROWS
-        self._graphs = {key: graph for key, graph in self._graphs.items() if key[0] > most}
-        self.resident = None
-        raise LostResults("a decode step gave up waiting for blocks that another kernel kept off the GPU; its results are lost")
-
-    def _run(self, entries: list, greedy: bool) -> Optional[torch.Tensor]:
         with ops.stream_scope():
             if self.use_graphs and self.watch is None and all(len(e.tokens) == 1 and list(e.want) == [0] for e in entries):
                 return self._run_decode_graph(entries, greedy)
@@ -468,3 +455,16 @@ class StepFunction:
             self.finish(ctx)
             self.last_context = ctx
             return out
+
+    def check(self) -> None:
+        """An error (``LostResults``) if a step that has run lost its results. To be called behind a copy or an event that
+        waits for the step, before what it left is used; every ``run`` asks for the steps before it. It is said once: from
+        then on all steps run kernel by kernel, which wait for nobody. What the lost steps wrote to their requests' pages is no
+        history to go on from."""
+        if self.resident is None or not self.resident.gave_up():
+            return
+        torch.cuda.synchronize(self.device)      # (what is in flight may be such a launch)
+        most = self.resident.MOST_ROWS
+        self._graphs = {key: graph for key, graph in self._graphs.items() if key[0] > most}
+        self.resident = None
+        raise LostResults("a decode step gave up waiting for blocks that another kernel kept off the GPU; its results are lost")

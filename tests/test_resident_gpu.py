@@ -373,3 +373,55 @@ def test_no_number_comes_from_a_wait_that_was_given_up(shape, rows):
     ops.clear_resident_area(res.area.address)
     res.failed.zero_()
     assert torch.equal(run(0)[0], want)
+
+
+def ends(work):
+    """``work`` in a thread of its own, whose end is waited for, but not for ever; what it returned."""
+    import threading
+    got = []
+
+    def run():
+        try:
+            got.append(work())
+        except BaseException as e:
+            got.append(e)
+    th = threading.Thread(target=run, daemon=True)
+    th.start()
+    th.join(30)
+    assert got, "still waiting"
+    assert not isinstance(got[0], BaseException), got[0]
+    return got[0]
+
+
+def test_a_step_within_a_step_that_is_watched():
+    m = model(256, 4, 1, 512, "bfloat16", layers=2)
+    outer, inner = (engine(m, 2, 64, "bfloat16") for _ in range(2))
+    stand(outer, [5, 9], 1), stand(inner, [12], 1)
+    seen = []
+    outer.step_fn.watch = lambda i, hidden: seen.append(decode(inner, [[i]])[0])
+    got = ends(lambda: decode(outer, [[1, 2]]))
+    assert len(seen) == 2 and all(torch.isfinite(x).all() for x in [*seen, *got])
+
+
+def test_a_step_that_is_being_laid_out_keeps_no_other_waiting():
+    import threading
+    m = model(256, 4, 1, 512, "bfloat16", layers=2)
+    slow, other = (engine(m, 1, 64, "bfloat16") for _ in range(2))
+    stand(slow, [5], 1), stand(other, [9], 1)
+    decode(other, [[3]])      # (captured)
+    inside, go_on, plan = threading.Event(), threading.Event(), slow.step_fn.plan
+
+    def plan_slowly(entries):
+        inside.set()
+        go_on.wait(60)
+        return plan(entries)
+    slow.step_fn.plan = plan_slowly
+    th = threading.Thread(target=lambda: decode(slow, [[1]]), daemon=True)
+    th.start()
+    assert inside.wait(30)
+    try:
+        ends(lambda: decode(other, [[4], [5]]))
+    finally:
+        go_on.set()
+        th.join(30)
+    assert not th.is_alive()
