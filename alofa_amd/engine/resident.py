@@ -3,6 +3,7 @@ function: the table of the layers' matrices and caches, an area of memory that t
 kernel sets if it gives a wait up."""
 from __future__ import annotations
 
+import collections
 import contextlib
 import fcntl
 import os
@@ -34,13 +35,18 @@ class _Areas:
     whose owner failed is cleared then: the word that stops its launches is still set, and its counter and its values may not belong together."""
 
     def __init__(self):
-        self._lock = threading.Lock()
-        self._idle: dict = {}      # device -> areas
+        # device -> areas. No lock: ``give_back`` runs wherever the garbage collector does, in the middle of a ``take`` or of another ``give_back`` of the same
+        # thread too (a deque's own operations are whole ones)
+        self._idle: dict = {}
+
+    def _of(self, device: torch.device) -> collections.deque:
+        return self._idle.setdefault(device.index, collections.deque())
 
     def take(self, device: torch.device) -> _Area:
-        with self._lock:
-            idle = self._idle.get(device.index)
-            area = idle.pop() if idle else None
+        try:
+            area = self._of(device).pop()
+        except IndexError:
+            area = None
         with torch.cuda.device(device):
             if area is None:
                 return _Area()
@@ -51,8 +57,7 @@ class _Areas:
         return area
 
     def give_back(self, device: torch.device, area: _Area) -> None:
-        with self._lock:
-            self._idle.setdefault(device.index, []).append(area)
+        self._of(device).append(area)
 
 
 _areas = _Areas()

@@ -1,10 +1,14 @@
 """Decode steps in one launch: what lies around the launch, without a GPU."""
+import gc
 import os
 import signal
 import threading
+import weakref
 from types import SimpleNamespace
 
-from alofa_amd.engine.resident import _Seats
+import torch
+
+from alofa_amd.engine.resident import _Areas, _Seats
 
 
 def another(folder):
@@ -103,3 +107,32 @@ def test_a_scope_of_one_thread_leaves_the_streams_of_others_alone(monkeypatch):
     assert seen == {"before": 2, "within": 2, "behind": 2}
     current.stream = 3
     assert ops._stream() == 3
+
+
+def test_an_area_is_given_back_while_another_is_being_given_back():
+    """By a finalizer that the collector runs in the middle of it, on the same thread."""
+    areas, device = _Areas(), torch.device("cuda:0")
+
+    class Collecting(dict):
+        def setdefault(self, key, value):
+            gc.collect()
+            return super().setdefault(key, value)
+    areas._idle = Collecting()
+
+    class Owner:
+        def __init__(self):
+            self.me = self      # (goes only when the collector comes)
+            weakref.finalize(self, areas.give_back, device, object())
+
+    def work():
+        gc.disable()
+        Owner()
+        areas.give_back(device, object())
+    t = threading.Thread(target=work, daemon=True)
+    try:
+        t.start()
+        t.join(10)
+    finally:
+        gc.enable()
+    assert not t.is_alive()
+    assert sum(len(a) for a in areas._idle.values()) == 2
