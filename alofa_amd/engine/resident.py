@@ -15,7 +15,6 @@ from typing import Optional
 import torch
 
 from .. import ops
-from ..errors import AlofaError
 from ..parts.attention import GQAAttention
 from ..parts.block import PreNormBlock
 from ..parts.feed_forward import SwiGLU
@@ -175,28 +174,44 @@ class ResidentLayers:
         m = first.mixer
         if not ops.resident_takes(m.hidden, first.feed_forward.intermediate, m.heads, m.kv_heads, m.d, cache.block_size):
             return None
+        tables = [cls._tensors(b, cache.tensors[(i, 0)]) for i, b in enumerate(blocks)]
+        if not all(cls._reads(m, first.feed_forward.intermediate, t) for t in tables):
+            return None
         if not _seats.take(str(torch.cuda.get_device_properties(rt.device).uuid)):
             return None
-        return cls(blocks, cache, rt.device)
+        return cls(blocks, cache, rt.device, tables)
 
-    def __init__(self, blocks: list, cache, device):
-        self.blocks, self.device = blocks, device
+    @staticmethod
+    def _tensors(b, kv: dict) -> list:
+        """What the kernel reads of a layer, in its order: matrices and bias, norms, caches."""
+        return [b.mixer.w_qkv, b.mixer.b_qkv, b.mixer.w_o, b.feed_forward.w_gate, b.feed_forward.w_up, b.feed_forward.w_down,
+                b.norms[0].as_rmsnorm()[0], b.norms[1].as_rmsnorm()[0], kv["k"], kv["v"]]
+
+    @staticmethod
+    def _reads(m, intermediate: int, tensors: list) -> bool:
+        """Whether a layer's tensors are what the kernel takes them for: matrices are kept in the type they were stored in and where their owner has them, so they may
+        be float32, or begin where no load of sixteen bytes can (the products one by one take those too)."""
+        qkv, out, h = (m.heads + 2 * m.kv_heads) * m.d, m.heads * m.d, m.hidden
+        shapes = [(qkv, h), (qkv,), (h, out), (intermediate, h), (intermediate, h), (h, intermediate), (h,), (h,), None, None]
+        for t, shape in zip(tensors, shapes):
+            if t is None:      # (no bias)
+                continue
+            dtype = torch.float32 if shape is not None and len(shape) == 1 else torch.bfloat16
+            if not t.is_cuda or t.dtype is not dtype or not t.is_contiguous() or t.data_ptr() % 16 or (shape is not None and tuple(t.shape) != shape):
+                return False
+        return True
+
+    def __init__(self, blocks: list, cache, device, tables: list):
+        self.device = device
         m = blocks[0].mixer
         self.heads, self.kv_heads, self.d, self.scale, self.position = m.heads, m.kv_heads, m.d, m.scale, m.position
         self.hidden, self.intermediate, self.biased = m.hidden, blocks[0].feed_forward.intermediate, m.b_qkv is not None
         self.eps = tuple(float(n.as_rmsnorm()[1]) for n in blocks[0].norms)
         self.page, self.group = cache.block_size, cache.group_of_entry[(0, 0)]
-        # (what the table points to: the model's matrices and the cache's pages, which live as long as the step function that holds both)
-        rows = []
-        for i, b in enumerate(blocks):
-            kv = cache.tensors[(i, 0)]
-            ops.check_caches(kv["k"], kv["v"], self.kv_heads, self.d)
-            tensors = [b.mixer.w_qkv, b.mixer.b_qkv, b.mixer.w_o, b.feed_forward.w_gate, b.feed_forward.w_up, b.feed_forward.w_down,
-                       b.norms[0].as_rmsnorm()[0], b.norms[1].as_rmsnorm()[0], kv["k"], kv["v"]]
-            if any(t is not None and (not t.is_cuda or not t.is_contiguous()) for t in tensors):
-                raise AlofaError("shape_mismatch", "the layers' tensors must be contiguous and on the GPU", f"layer={i}")
-            rows.append([0 if t is None else t.data_ptr() for t in tensors])
-        self.layers = torch.tensor(rows, dtype=torch.int64, device=device)
+        for t in tables:
+            ops.check_caches(t[-2], t[-1], self.kv_heads, self.d)
+        self._tables = tables      # (kept: the table on the GPU holds their addresses)
+        self.layers = torch.tensor([[0 if t is None else t.data_ptr() for t in ts] for ts in tables], dtype=torch.int64, device=device)
         self.area = _areas.take(device)
         weakref.finalize(self, _areas.give_back, device, self.area)
         self.failed = self.area.failed

@@ -425,3 +425,38 @@ def test_a_step_that_is_being_laid_out_keeps_no_other_waiting():
         go_on.set()
         th.join(30)
     assert not th.is_alive()
+
+
+@pytest.mark.parametrize("how", ["stored in 32 bits", "one matrix in 32 bits", "off its place"])
+def test_matrices_that_the_launch_cannot_read_run_kernel_by_kernel(how, monkeypatch):
+    """Matrices keep the type they were stored in and the place they were given: the results are those of the kernels one by one."""
+    config, first = model(256, 4, 1, 512, "bfloat16", layers=2)
+    from alofa_amd.model import Model, runtime
+
+    def shifted(t):
+        room = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")
+        return room[1:].view(t.shape).copy_(t)
+    weights = {}
+    for i, b in enumerate(first.blocks):
+        pre, q, kv = f"model.layers.{i}.", 4 * 64, 64
+        for n, t in zip("qkv", b.mixer.w_qkv.split([q, kv, kv])):
+            weights[pre + f"self_attn.{n}_proj.weight"] = t
+        for n, t in zip("qkv", b.mixer.b_qkv.split([q, kv, kv])):
+            weights[pre + f"self_attn.{n}_proj.bias"] = t
+        weights.update({pre + "self_attn.o_proj.weight": b.mixer.w_o, pre + "mlp.gate_proj.weight": b.feed_forward.w_gate, pre + "mlp.up_proj.weight": b.feed_forward.w_up,
+                        pre + "mlp.down_proj.weight": b.feed_forward.w_down, pre + "input_layernorm.weight": b.norms[0].weight, pre + "post_attention_layernorm.weight": b.norms[1].weight})
+    weights.update({"model.embed_tokens.weight": first.embedding.table, "model.norm.weight": first.final_norm.weight})
+    for n, t in weights.items():
+        if t.dim() == 2 and (how == "stored in 32 bits" or (how == "one matrix in 32 bits" and n == "model.layers.1.mlp.down_proj.weight")):
+            weights[n] = t.float()
+        elif how == "off its place" and n == "model.layers.1.self_attn.o_proj.weight":
+            weights[n] = shifted(t)
+    m = config, Model(config.spec(), weights, runtime("bfloat16"))
+    got = {}
+    for switch in ("1", "0"):
+        monkeypatch.setenv("ALOFA_ONE_LAUNCH", switch)
+        eng = engine(m, 2, 64, "bfloat16")
+        assert eng.step_fn.resident is None
+        stand(eng, [5, 20], 3)
+        got[switch] = decode(eng, [[1, 2], [3, 4]])
+    assert all(torch.equal(a, b) and torch.isfinite(a).all() for a, b in zip(got["1"], got["0"]))
