@@ -752,6 +752,7 @@ extern "C" int alofa_resident_area(void** area) {
   using namespace alofa;
   *area = nullptr;
   const hipError_t e = hipExtMallocWithFlags(area, kAreaPlaces * 8, hipDeviceMallocUncached);
+  if (e != hipSuccess) static_cast<void>(hipGetLastError());      // (the caller goes on without one: not the next launch's error)
   ALOFA_REQUIRE(e == hipSuccess, "resident_area: %s", hipGetErrorString(e));
   return alofa_resident_area_clear(*area);
 }

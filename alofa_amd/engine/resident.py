@@ -15,6 +15,7 @@ from typing import Optional
 import torch
 
 from .. import ops
+from ..errors import AlofaError
 from ..parts.attention import GQAAttention
 from ..parts.block import PreNormBlock
 from ..parts.feed_forward import SwiGLU
@@ -24,8 +25,8 @@ class _Area:
     """Memory that the blocks of a launch exchange values in, and the pinned word that the kernel sets if it gives a wait up."""
 
     def __init__(self):
-        self.address = ops.resident_area()
         self.failed = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self.address = ops.resident_area()
 
 
 class _Areas:
@@ -179,7 +180,11 @@ class ResidentLayers:
             return None
         if not _seats.take(str(torch.cuda.get_device_properties(rt.device).uuid)):
             return None
-        return cls(blocks, cache, rt.device, tables)
+        try:
+            area = _areas.take(rt.device)
+        except (AlofaError, RuntimeError):      # (no memory for one: the kernels one by one need none)
+            return None
+        return cls(blocks, cache, rt.device, tables, area)
 
     @staticmethod
     def _tensors(b, kv: dict) -> list:
@@ -201,8 +206,9 @@ class ResidentLayers:
                 return False
         return True
 
-    def __init__(self, blocks: list, cache, device, tables: list):
-        self.device = device
+    def __init__(self, blocks: list, cache, device, tables: list, area: "_Area"):
+        self.device, self.area = device, area
+        weakref.finalize(self, _areas.give_back, device, area)
         m = blocks[0].mixer
         self.heads, self.kv_heads, self.d, self.scale, self.position = m.heads, m.kv_heads, m.d, m.scale, m.position
         self.hidden, self.intermediate, self.biased = m.hidden, blocks[0].feed_forward.intermediate, m.b_qkv is not None
@@ -212,9 +218,7 @@ class ResidentLayers:
             ops.check_caches(t[-2], t[-1], self.kv_heads, self.d)
         self._tables = tables      # (kept: the table on the GPU holds their addresses)
         self.layers = torch.tensor([[0 if t is None else t.data_ptr() for t in ts] for ts in tables], dtype=torch.int64, device=device)
-        self.area = _areas.take(device)
-        weakref.finalize(self, _areas.give_back, device, self.area)
-        self.failed = self.area.failed
+        self.failed = area.failed
         self._failed = self.failed.numpy()
         self.turn = _turns.setdefault(device.index, _Turns(device))      # what a launch, or a replay of one, goes within
 

@@ -460,3 +460,19 @@ def test_matrices_that_the_launch_cannot_read_run_kernel_by_kernel(how, monkeypa
         stand(eng, [5, 20], 3)
         got[switch] = decode(eng, [[1, 2], [3, 4]])
     assert all(torch.equal(a, b) and torch.isfinite(a).all() for a, b in zip(got["1"], got["0"]))
+
+
+def test_without_memory_for_an_area_steps_run_kernel_by_kernel(monkeypatch):
+    from alofa_amd import ops
+    from alofa_amd.engine import resident
+    from alofa_amd.errors import AlofaError
+
+    def none():
+        raise AlofaError("capacity", "no memory for an area")
+    m = model(256, 4, 1, 512, "bfloat16", layers=1)
+    monkeypatch.setattr(resident, "_areas", resident._Areas())
+    monkeypatch.setattr(ops, "resident_area", none)
+    eng = engine(m, 1, 32, "bfloat16")
+    assert eng.step_fn.resident is None
+    stand(eng, [3], 1)
+    assert torch.isfinite(decode(eng, [[1]])[0]).all()
