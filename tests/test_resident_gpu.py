@@ -178,11 +178,17 @@ def test_areas_are_used_again():
     import gc
     from alofa_amd.engine.resident import _areas
     m = model(256, 4, 1, 512, "bfloat16", layers=1)
-    area = engine(m, 1, 32, "bfloat16").step_fn.resident.area
+    eng = engine(m, 1, 32, "bfloat16")
+    stand(eng, [3], 1)
+    area, want = eng.step_fn.resident.area, decode(eng, [[1], [2]])
+    del eng
     gc.collect()
     idle = [a for areas in _areas._idle.values() for a in areas]
     assert area in idle
-    assert engine(m, 1, 32, "bfloat16").step_fn.resident.area in idle
+    eng = engine(m, 1, 32, "bfloat16")
+    assert eng.step_fn.resident.area in idle
+    stand(eng, [3], 1)
+    assert all(torch.equal(a, b) for a, b in zip(decode(eng, [[1], [2]]), want))
 
 
 def write(address, words):
