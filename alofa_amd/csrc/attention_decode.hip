@@ -79,8 +79,9 @@ struct MapsForm {
 // Blocks dealt out by length (`deal` blocks a token on average, at most 64 tokens, one lane each): a token's keys are cut into as many parts as it takes for none to have
 // more than a quota of tiles, the least of five quotas between an even share of all tiles and one that always fits for which the blocks suffice. Every wave finds the
 // same from the positions alone (four sums over the lanes, independent of one another, some 0.2 us). One number of parts for all leaves the launch
-// waiting for the longest request. us a step of the 0.5B sizes (24 layers, 14/2 heads of 64), so many parts each / dealt out: 64 tokens of 128 to 2,048 keys 1,410 / 1,379, 64 of 700
-// 1,317 / 1,314, 64 of 32 to 500 1,255 / 1,255, 48 of 16 to 300 1,213 / 1,215. Not where a token has four parts or more on average: 32 of 512 to 768 1,160 / 1,175 (24 of 64 to 1,500 1,178 / 1,154), and not
+// waiting for the longest request. us a step of the 0.5B sizes (24 layers, 14/2 heads of 64), so many parts each / dealt out, two runs of
+// one side within 0.1 %: 40 tokens of 32 to 3,000 keys 1,331 / 1,275, 64 of 128 to 2,048 1,392 / 1,361; 64 of 700 1,301 / 1,304, 64 of 16 to 700 1,288 / 1,291, 48 of 64 to 1,024 1,304 / 1,309, 33 of 128 to 512
+// 1,211 / 1,217 (there it is what finding the parts takes). Not where a token has four parts or more on average: 32 of 512 to 768 1,160 / 1,175 (24 of 64 to 1,500 1,178 / 1,154), and not
 // for heads of 128: 32 tokens of 28/4 heads, 128 to 1,024 keys, even; 8 of 500 to 800 1.4 % slower.
 constexpr int kMostDealt = 8;
 struct Dealt {

@@ -28,9 +28,9 @@
 // LDS), so that 256 of them fit beside 256 of another such launch, whatever process it belongs to; kernels that wait for nobody make room by ending.
 // No wait is without end: a wave that has asked kLimit times sets `stop` and `failed`, which end every other wait, and what it waited for is NaN from then on.
 //
-// A step of the 0.5B sizes (24 layers of 896, 14/2 heads, 4,864; the head's 70 us among them), us, kernel by kernel / this: 1 row of 512 keys 643 / 455, 2 667 / 476,
-// 4 of 512 to 768 715 / 510, 8 785 / 549, 12 of 64 to 700 890 / 616, 16 of 128 to 1,024 937 / 663, 1 of 4,000 707 / 481, 8 of 3,000 to 4,000 860 / 589. What a layer takes (16 us at
-// one row, 20 at eight) is the exchanges, 1.1 to 2.2 us each with the loads that are waited for before them, and 0.5 to 1.3 us of dependent instructions in every phase. Where the
+// A step of the 0.5B sizes (24 layers of 896, 14/2 heads, 4,864; the head's 70 us among them), us, kernel by kernel / this: 1 row of 512 keys 643 / 450, 2 667 / 469,
+// 4 of 512 to 768 715 / 500, 8 785 / 529, 12 of 64 to 700 890 / 599, 16 of 128 to 1,024 937 / 644, 1 of 4,000 707 / 472, 8 of 3,000 to 4,000 860 / 574. What a layer takes (16 us at
+// one row, 19 at eight) is the exchanges, 1.1 to 2.2 us each with the loads that are waited for before them, and 0.5 to 1.3 us of dependent instructions in every phase. Where the
 // weights are asked for was found by trying: behind a phase's products and before its barrier, before the values leave, a phase earlier or later cost 1 to 5 %, a single register
 // that the compiler keeps in memory 10 (it is read back behind the weights on their way), and weights by pointers of any kind, which LDS's waits wait for too, 15.
 //

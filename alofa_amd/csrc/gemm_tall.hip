@@ -19,7 +19,7 @@
 //
 // A tile's way out counts as much as its way in where K is short. bfloat16 outputs are written as whole lines of rows by way of LDS (rows_epilogue), the gate's division takes what its range needs
 // (common.h), and gate and up share a group of 32 rows of W eight and eight, so that any tile does for them: 4,864 x 896 with the gate against 2,048 rows 47.6 us (tiles of 128 x 64 of gemm_mfma.hip; 53.1
-// with 256 x 128 here) -> 40.3 (256 x 160, one round of the chip) -> 37.2 (the division); 8,960 x 1,536 against 2,048 133 -> 102, 18,944 x 3,584 against 1,970 460 -> 441, 27,648 x 5,120
+// with 256 x 128 here) -> 40.3 (256 x 160, one round of the chip) -> 37.2 (the division; with the general one's bits for every gate 0.4 to 0.7 % more); 8,960 x 1,536 against 2,048 133 -> 102, 18,944 x 3,584 against 1,970 460 -> 441, 27,648 x 5,120
 // against 4,096 1,797 -> 1,756; stored as bfloat16 7,168 x 5,120 against 4,096 266 -> 243, 4,608 x 3,584 against 1,970 72.0 -> 65.7.
 //
 // Tiles (Tall<rows, columns, waves along rows, along columns, slabs in the ring, column groups of the phases>): the wider, the less a
