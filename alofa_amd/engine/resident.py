@@ -178,13 +178,14 @@ class ResidentLayers:
         tables = [cls._tensors(b, cache.tensors[(i, 0)]) for i, b in enumerate(blocks)]
         if not all(cls._reads(m, first.feed_forward.intermediate, t) for t in tables):
             return None
-        if not _seats.take(str(torch.cuda.get_device_properties(rt.device).uuid)):
+        device = rt.device if rt.device.index is not None else torch.device(rt.device.type, torch.cuda.current_device())      # (by number, so that all of a GPU's launches meet)
+        if not _seats.take(str(torch.cuda.get_device_properties(device).uuid)):
             return None
         try:
-            area = _areas.take(rt.device)
+            area = _areas.take(device)
         except (AlofaError, RuntimeError):      # (no memory for one: the kernels one by one need none)
             return None
-        return cls(blocks, cache, rt.device, tables, area)
+        return cls(blocks, cache, device, tables, area)
 
     @staticmethod
     def _tensors(b, kv: dict) -> list:

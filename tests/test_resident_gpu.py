@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 VOCAB, LAYERS = 512, 3
 
 
-def model(width, heads, kv_heads, ff, dtype, layers=LAYERS, window=None):
+def model(width, heads, kv_heads, ff, dtype, layers=LAYERS, window=None, device="cuda:0"):
     from alofa_amd.config import config_from_dict
     from alofa_amd.model import Model, runtime
     config = config_from_dict({"architectures": ["Qwen2ForCausalLM"], "model_type": "qwen2", "num_hidden_layers": layers, "hidden_size": width, "num_attention_heads": heads,
@@ -32,7 +32,7 @@ def model(width, heads, kv_heads, ff, dtype, layers=LAYERS, window=None):
                 w[pre + n + ".bias"] = draw(rows, scale=0.5)
         for n in ("input_layernorm", "post_attention_layernorm"):
             w[pre + n + ".weight"] = draw(width, scale=0.1, shift=1.0)
-    return config, Model(config.spec(), w, runtime(dtype))
+    return config, Model(config.spec(), w, runtime(dtype, device))
 
 
 def engine(m, rows, context, dtype, page=16):
@@ -482,3 +482,9 @@ def test_without_memory_for_an_area_steps_run_kernel_by_kernel(monkeypatch):
     assert eng.step_fn.resident is None
     stand(eng, [3], 1)
     assert torch.isfinite(decode(eng, [[1]])[0]).all()
+
+
+def test_a_gpu_named_without_its_number_is_the_same_gpu():
+    config, first = model(256, 4, 1, 512, "bfloat16", layers=1)
+    turns = [engine(m, 1, 32, "bfloat16").step_fn.resident.turn for m in ((config, first), model(256, 4, 1, 512, "bfloat16", layers=1, device="cuda"))]
+    assert turns[0] is turns[1]
