@@ -150,6 +150,11 @@ class ResidentLayers:
     """All layers of ``model`` over ``cache`` as one launch, for steps of at most ``MOST_ROWS`` rows of one new token each."""
     MOST_ROWS = 16
     MOST_LAYERS = 64      # whose addresses the kernel keeps at hand
+    # (rows x key heads below, keys that the longest request sees): the launch cuts a row and key head's keys into sixteen parts, the kernels one by one into as many as the chip has
+    # compute units for, up to 64. us a step, one launch / kernel by kernel: one row, two key heads of the 0.5B sizes, 16,000 keys 629 / 764, 31,000 813 / 779; one row and key head, 256
+    # wide (24 layers), 15,000 491 / 542, 31,000 668 / 562, 512 wide (16) 344 / 382 and 469 / 398; three key heads, 576 wide (30), 682 / 793 and 919 / 820; rows x key heads of four or five,
+    # 31,000 keys: 840 / 846, 299 / 297, 802 / 804, 560 / 573; of eight 924 / 1,022; of sixteen 1,076 / 1,335, 484 / 617. Even at 20,000 to 28,000 below four, at 30,000 from there on.
+    MOST_KEYS = ((4, 20000), (16, 28000))
 
     @classmethod
     def of(cls, model, cache) -> Optional["ResidentLayers"]:
@@ -224,8 +229,10 @@ class ResidentLayers:
         self.turn = _turns.setdefault(device.index, _Turns(device))      # what a launch, or a replay of one, goes within
 
     def takes(self, ctx, rows: int) -> bool:
-        """Whether this step runs in one launch: one new token for each of few requests."""
-        return rows <= self.MOST_ROWS and ctx.max_q_len == 1 and len(ctx.spans) == rows
+        """Whether this step runs in one launch: one new token for each of few requests, and keys that it is the faster one for."""
+        if rows > self.MOST_ROWS or ctx.max_q_len != 1 or len(ctx.spans) != rows:
+            return False
+        return ctx.longest <= next((keys for below, keys in self.MOST_KEYS if rows * self.kv_heads < below), ctx.longest)
 
     def gave_up(self) -> bool:
         return bool(self._failed[0])

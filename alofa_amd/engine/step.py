@@ -82,9 +82,9 @@ class StepContext:
         self.positions_host = positions_host
         self.tokens = int(positions_host.shape[0])
         self.max_q_len = max(s.n for s in spans)            # most rows of one request
-        # longest context after this step, rounded up to a power of two: it only shapes
-        # launches, and a coarse value lets captured decode graphs be used again
-        self.max_context = _pow2_ceil(max(s.pos0 + s.n for s in spans))
+        self.longest = max(s.pos0 + s.n for s in spans)     # longest context after this step
+        # ... rounded up to a power of two: it only shapes launches, and a coarse value lets captured decode graphs be used again
+        self.max_context = _pow2_ceil(self.longest)
         self.n_positions = fn.n_positions
         self.entry_slots = self.entry_tokens = None   # request slot and token count per entry, as arrays
         self.positions: torch.Tensor = None
@@ -384,7 +384,8 @@ class StepFunction:
         buf["dev"].copy_(host["block"], non_blocking=True)
         host["copied"].record()
         ctx.want_slots = buf["request_slots"]
-        key = (B, ctx.max_context, greedy)
+        one_launch = self.resident is not None and self.resident.takes(ctx, B)
+        key = (B, ctx.max_context, greedy, one_launch)
         saved, self._scratch = self._scratch, buf["scratch"]   # graphs of one batch size share their own buffers
         chosen = self._chosen[:B]
 
@@ -423,7 +424,7 @@ class StepFunction:
                 # the capture itself ran nothing: the eager results stand
             else:
                 graph, logits = self._graphs[key]
-                with self.resident.turn if self.resident is not None and self.resident.takes(ctx, B) else contextlib.nullcontext():
+                with self.resident.turn if one_launch else contextlib.nullcontext():
                     graph.replay()
                 self.graph_replays += 1
         finally:
@@ -464,7 +465,6 @@ class StepFunction:
         if self.resident is None or not self.resident.gave_up():
             return
         torch.cuda.synchronize(self.device)      # (what is in flight may be such a launch)
-        most = self.resident.MOST_ROWS
-        self._graphs = {key: graph for key, graph in self._graphs.items() if key[0] > most}
+        self._graphs = {key: graph for key, graph in self._graphs.items() if not key[3]}
         self.resident = None
         raise LostResults("a decode step gave up waiting for blocks that another kernel kept off the GPU; its results are lost")

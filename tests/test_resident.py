@@ -8,7 +8,7 @@ from types import SimpleNamespace
 
 import torch
 
-from alofa_amd.engine.resident import _Areas, _Seats
+from alofa_amd.engine.resident import ResidentLayers, _Areas, _Seats
 
 
 def another(folder):
@@ -136,3 +136,17 @@ def test_an_area_is_given_back_while_another_is_being_given_back():
         gc.enable()
     assert not t.is_alive()
     assert sum(len(a) for a in areas._idle.values()) == 2
+
+
+def test_steps_of_few_rows_over_very_many_keys_are_left_to_the_kernels_one_by_one():
+    layers = ResidentLayers.__new__(ResidentLayers)
+
+    def takes(rows, kv_heads, longest, new=1):
+        layers.kv_heads = kv_heads
+        return layers.takes(SimpleNamespace(max_q_len=new, spans=[None] * rows, longest=longest), rows)
+    assert takes(1, 2, 20000) and not takes(1, 2, 20001)
+    assert takes(3, 1, 20000) and not takes(3, 1, 20001)
+    assert takes(2, 2, 28000) and not takes(2, 2, 28001)
+    assert takes(5, 3, 28000) and not takes(5, 3, 28001)
+    assert takes(8, 2, 1000000) and takes(1, 16, 1000000) and takes(16, 1, 1000000)
+    assert not takes(17, 1, 10) and not takes(1, 1, 10, new=2)

@@ -488,3 +488,19 @@ def test_a_gpu_named_without_its_number_is_the_same_gpu():
     config, first = model(256, 4, 1, 512, "bfloat16", layers=1)
     turns = [engine(m, 1, 32, "bfloat16").step_fn.resident.turn for m in ((config, first), model(256, 4, 1, 512, "bfloat16", layers=1, device="cuda"))]
     assert turns[0] is turns[1]
+
+
+def test_a_step_that_grows_past_the_keys_it_is_for(monkeypatch):
+    """In the middle of a captured length (one graph for either way), laid out eagerly and captured: the same bits."""
+    from alofa_amd.engine.resident import ResidentLayers
+    monkeypatch.setattr(ResidentLayers, "MOST_KEYS", ((4, 40), (16, 1000)))
+    m = model(256, 4, 1, 512, "bfloat16", layers=2)
+    got = {}
+    for captured in (True, False):
+        eng = engine(m, 2, 100, "bfloat16")
+        eng.step_fn.use_graphs = captured
+        stand(eng, [37, 20], 5)
+        got[captured] = decode(eng, np.arange(14).reshape(7, 2))
+        if captured:
+            assert {key[3] for key in eng.step_fn._graphs} == {True, False} and eng.step_fn.graph_replays == 5
+    assert all(torch.equal(a, b) and torch.isfinite(a).all() for a, b in zip(got[True], got[False]))
