@@ -11,7 +11,7 @@ from .cache.manager import CacheManager
 from .engine.core import EngineCore
 from .engine.scheduler import SchedConfig
 from .engine.step import StepFunction
-from .errors import AlofaError
+from .errors import AlofaError, LostResults
 from .model import load_model
 from .sampling.sampler import SampleParams
 
@@ -111,19 +111,24 @@ class Engine:
             waiting.append((self._next_id, list(p)))
             self._next_id += 1
         ticks = 0
-        while waiting or self.core.has_work():
-            # requests the watermark cannot hold yet wait here until earlier ones end
-            while waiting and self.core.can_admit(len(waiting[0][1]), max_new):
-                rid, p = waiting.pop(0)
-                self.core.submit(rid, p, max_new, params, use_seed)
-            if not self.core.has_work():
-                raise AlofaError("capacity", "a request can never be admitted: it does not fit under the kv watermark",
-                                 f"prompt={len(waiting[0][1])} max_new={max_new}")
-            self.core.tick()
-            ticks += 1
-            if ticks > max_ticks:
-                raise AlofaError("capacity", "generation did not finish within the tick limit", f"max_ticks={max_ticks}")
-        self.core.flush()
+        try:
+            while waiting or self.core.has_work():
+                # requests the watermark cannot hold yet wait here until earlier ones end
+                while waiting and self.core.can_admit(len(waiting[0][1]), max_new):
+                    rid, p = waiting.pop(0)
+                    self.core.submit(rid, p, max_new, params, use_seed)
+                if not self.core.has_work():
+                    raise AlofaError("capacity", "a request can never be admitted: it does not fit under the kv watermark",
+                                     f"prompt={len(waiting[0][1])} max_new={max_new}")
+                self.core.tick()
+                ticks += 1
+                if ticks > max_ticks:
+                    raise AlofaError("capacity", "generation did not finish within the tick limit", f"max_ticks={max_ticks}")
+            self.core.flush()
+        except LostResults:      # (those of these requests that had not begun are not the next call's)
+            for rid in ids:
+                self.core.cancel(rid)
+            raise
         outs = {}
         for rid in ids:
             outs[rid] = self.core.output(rid)

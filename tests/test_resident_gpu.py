@@ -504,3 +504,28 @@ def test_a_step_that_grows_past_the_keys_it_is_for(monkeypatch):
         if captured:
             assert {key[3] for key in eng.step_fn._graphs} == {True, False} and eng.step_fn.graph_replays == 5
     assert all(torch.equal(a, b) and torch.isfinite(a).all() for a, b in zip(got[True], got[False]))
+
+
+def test_generate_again_behind_a_step_that_gave_up():
+    """More prompts than the pages hold at once, so that some have not begun when it happens: the next call's results are its own."""
+    from alofa_amd import Engine
+    from alofa_amd.errors import LostResults
+    m = model(256, 4, 1, 512, "bfloat16", layers=2)
+    prompts = np.random.default_rng(6).integers(0, VOCAB, (6, 40)).tolist()
+    engines = [Engine(None, dtype="bfloat16", max_tokens=64, max_batch=6, kv_blocks=9, block_size=16, token_budget=64, watermark_permille=1000, model=m) for _ in range(2)]
+    engines[0].step_fn.resident = None
+    want = engines[0].generate(prompts[3:], max_new=6)
+    eng, run = engines[1], engines[1].step_fn.run
+    steps = []
+
+    def failing(entries, greedy=False):
+        out = run(entries, greedy)
+        steps.append(entries)
+        if len(steps) == 6:
+            eng.step_fn.resident.failed[0] = 1
+        return out
+    eng.step_fn.run = failing
+    with pytest.raises(LostResults):
+        eng.generate(prompts, max_new=6)
+    assert eng.generate(prompts[3:], max_new=6) == want
+    assert not eng.core.has_work() and not eng.core.cache.requests
