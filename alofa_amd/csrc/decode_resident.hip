@@ -36,123 +36,10 @@
 //
 // Numbers as in the kernels this replaces: the norm's weight on the row rounded to bfloat16 as an operand and the row's factor on the finished
 // sum, queries and keys (once, when they have been turned), values, attention's result and act rounded to bfloat16, everything else float.
-#include "common.h"
-
-#include <float.h>
-
-#include <type_traits>
+#include "resident.h"
 
 namespace alofa {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned long long u64;
-
-// (pointers that are read from memory are told to lead to global memory: a load by a pointer of any kind is waited for with LDS's own, at every barrier)
-#define ALOFA_GLOBAL __attribute__((address_space(1)))
-typedef ALOFA_GLOBAL const char* gbytes;
-
-// one per layer, in device memory
-struct ResidentLayer {
-  gbytes w_qkv;
-  ALOFA_GLOBAL const float* b_qkv;
-  gbytes w_o;
-  gbytes w_gate;
-  gbytes w_up;
-  gbytes w_down;
-  ALOFA_GLOBAL const float* norm0;
-  ALOFA_GLOBAL const float* norm1;
-  ALOFA_GLOBAL bf16_t* k_cache;
-  ALOFA_GLOBAL bf16_t* v_cache;
-};
-
-template <typename V>
-__device__ __forceinline__ V load_global(gbytes at) { return *reinterpret_cast<ALOFA_GLOBAL const V*>(at); }
-
-constexpr int kLayerWords = sizeof(ResidentLayer) / 4, kResMaxLayers = 64;
-struct LayerWords {
-  uint32_t w[kLayerWords];
-};
-
-constexpr int kResBlocks = 256, kResThreads = 512, kResWaves = 8;
-constexpr int kResMaxWidth = 1024, kResMaxFF = 6144, kResMaxRows = 16, kResMaxParts = 16, kResShares = 8, kResMaxGroup = 8;
-constexpr int kLimit = 4 << 20;      // asks of about a microsecond
-
-// where the values lie in the area, in places of eight bytes (the first 32 hold the step counter and `stop`)
-constexpr int kAtRowsA = 32, kAtRowsB = kAtRowsA + kResMaxRows * kResMaxWidth, kAtQkv = kAtRowsB + kResMaxRows * kResMaxWidth,
-              kAtParts = kAtQkv + kResMaxRows * 4096, kAtAttn = kAtParts + kResBlocks * kResMaxGroup * 66, kAtAct = kAtAttn + kResMaxRows * kResMaxWidth / 2,
-              kAtDown = kAtAct + kResMaxRows * kResMaxFF / 2, kAreaPlaces = kAtDown + kResMaxWidth * kResMaxRows * kResShares;
-
-struct ResidentArgs {
-  float* hidden;
-  const ResidentLayer* layers;
-  const int32_t* positions;
-  const int32_t* table;
-  const int64_t* slots;
-  const float* cos_t;
-  const float* sin_t;
-  u64* area;
-  int* failed;
-  int n_layers, M, H, FF, heads, kv_heads, max_blocks, bs_shift, parts, has_bias, limit;
-  float scale, eps0, eps1;
-};
-
-__device__ __forceinline__ void put(u64* at, uint32_t value, uint32_t stamp) {
-  __hip_atomic_store(at, (static_cast<u64>(stamp) << 32) | value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void put(u64* at, float value, uint32_t stamp) { put(at, __float_as_uint(value), stamp); }
-
-struct Wait {      // of one wave: the area as a buffer resource (reads past the caches), the stamp waited for, whether waits are over
-  __amdgpu_buffer_rsrc_t area;
-  u64* words;
-  int* failed;
-  int limit;      // asks until a wait is given up
-  uint32_t stamp;
-  bool dead;
-
-  // Two places at once (16 bytes), `at`: the first one's number, even. That such a load sees each of the two stores of eight bytes whole, never a new stamp beside an old
-  // value, is how memory serves an aligned piece of sixteen bytes, and taken for granted here (none of 3.9e10 loads beside stores saw half of one): what is promised of a load ends at eight bytes. With loads of eight (64 lanes
-  // a run of 64 places, no register in memory) a step of 1, 4, 8, 12 and 16 rows takes 454, 522, 581, 663 and 713 us instead of 449, 499, 529, 599 and 641.
-  __device__ __forceinline__ u32x4 two(int at) const {
-    constexpr int kPastCaches = 1 | 16;      // sc0, sc1
-    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(area, at * 8, 0, kPastCaches));
-  }
-  // whether to go on asking (uniform over the wave)
-  __device__ __forceinline__ bool again(int& asked) {
-    if ((++asked & 255) == 0 || asked >= limit) {
-      dead = asked >= limit || __any(__hip_atomic_load(words + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0);
-      if (dead) {
-        __hip_atomic_store(words + 1, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      }
-    }
-    return !dead;
-  }
-  // N pairs of places at at(i), until all bear the stamp. Where waits are over the values are NaN, in 32 bits and as two numbers of 16: whatever is computed from
-  // them is NaN and leaves as such, so that no number that a row ends with comes from a wait that was given up, whichever wave gave it up and when.
-  // (told which way is the usual one, the compiler keeps no register in memory: a step of 8 rows 545 -> 529 us, of 12 617 -> 599)
-  template <int N, typename At>
-  __device__ __forceinline__ void pairs(u32x4 (&v)[N], At&& at) {
-    constexpr uint32_t kNaN = 0x7fc07fc0u;
-    int asked = 0;
-    if (__builtin_expect(!dead, 1)) do {
-      asm volatile("" ::: "memory");      // (read anew every time)
-#pragma unroll
-      for (int i = 0; i < N; ++i)
-        v[i] = two(at(i));
-      bool here = true;
-#pragma unroll
-      for (int i = 0; i < N; ++i) here &= v[i][1] == stamp && v[i][3] == stamp;
-      if (__builtin_expect(__all(here), 1)) return;
-    } while (again(asked));
-#pragma unroll
-    for (int i = 0; i < N; ++i) v[i][0] = kNaN, v[i][2] = kNaN;
-  }
-};
-
-// MB: rows computed (1, 2, 4, 8 or 16; M of them count)
 template <int MB>
 __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(ResidentArgs a) {
   constexpr int d = 64;
@@ -735,14 +622,14 @@ static int launch_resident(const ResidentArgs& a, hipStream_t stream) {
 }  // namespace alofa
 
 // Bytes of an area (uncached device memory; it is never given back to the runtime: tensors that took the place of such memory have held wrong values).
-extern "C" int64_t alofa_resident_area_bytes() { return static_cast<int64_t>(alofa::kAreaPlaces) * 8; }
+extern "C" int64_t alofa_resident_area_bytes() { return static_cast<int64_t>(alofa::kAreaPlaces) * 8 * alofa::kResGroups; }
 
 // An area as it was when new, zeros, behind everything that the device has been given. Not to be called under graph capture.
 extern "C" int alofa_resident_area_clear(void* area) {
   using namespace alofa;
   ALOFA_REQUIRE(area, "resident_area_clear: no area");
   hipError_t e = hipDeviceSynchronize();
-  if (e == hipSuccess) e = hipMemset(area, 0, kAreaPlaces * 8);
+  if (e == hipSuccess) e = hipMemset(area, 0, alofa_resident_area_bytes());
   if (e == hipSuccess) e = hipDeviceSynchronize();
   ALOFA_REQUIRE(e == hipSuccess, "resident_area_clear: %s", hipGetErrorString(e));
   return 0;
@@ -752,7 +639,7 @@ extern "C" int alofa_resident_area_clear(void* area) {
 extern "C" int alofa_resident_area(void** area) {
   using namespace alofa;
   *area = nullptr;
-  const hipError_t e = hipExtMallocWithFlags(area, kAreaPlaces * 8, hipDeviceMallocUncached);
+  const hipError_t e = hipExtMallocWithFlags(area, alofa_resident_area_bytes(), hipDeviceMallocUncached);
   if (e != hipSuccess) static_cast<void>(hipGetLastError());      // (the caller goes on without one: not the next launch's error)
   ALOFA_REQUIRE(e == hipSuccess, "resident_area: %s", hipGetErrorString(e));
   return alofa_resident_area_clear(*area);
@@ -779,13 +666,14 @@ extern "C" int alofa_decode_resident(float* hidden, const void* layers, const in
                                      const float* sin_t, void* area, int* failed, int n_layers, int M, int H, int FF, int heads, int kv_heads, int d, int page, int max_blocks,
                                      int has_bias, int limit, float scale, float eps0, float eps1, hipStream_t stream) {
   using namespace alofa;
-  ALOFA_REQUIRE(alofa_resident_takes(H, FF, heads, kv_heads, d, page) && M >= 1 && M <= kResMaxRows && M * kv_heads <= kResBlocks && M * heads <= kResBlocks && n_layers > 0 && n_layers <= kResMaxLayers && max_blocks > 0,
+  ALOFA_REQUIRE(alofa_resident_takes(H, FF, heads, kv_heads, d, page) && M >= 1 && M <= alofa_resident_rows(H, FF, heads, kv_heads) && (M > kResMaxRows || (M * kv_heads <= kResBlocks && M * heads <= kResBlocks)) && n_layers > 0 && n_layers <= kResMaxLayers && max_blocks > 0,
                 "decode_resident: sizes beyond what a block holds (M=%d H=%d FF=%d heads=%d/%d d=%d page=%d)", M, H, FF, heads, kv_heads, d, page);
   ALOFA_REQUIRE(hidden && layers && positions && table && slots && cos_t && sin_t && area && failed, "decode_resident: an operand is missing");
   int shift = 0;
   while ((1 << shift) < page) ++shift;
   const ResidentArgs a = {hidden, static_cast<const ResidentLayer*>(layers), positions, table, slots, cos_t, sin_t, static_cast<u64*>(area), failed, n_layers, M, H, FF, heads, kv_heads,
                           max_blocks, shift, alofa_resident_parts(M, kv_heads), has_bias, limit > 0 ? limit : kLimit, scale, eps0, eps1};
+  if (M > kResMaxRows) return launch_groups(a, stream);
   if (M == 1) return launch_resident<1>(a, stream);
   if (M == 2) return launch_resident<2>(a, stream);
   if (M <= 4) return launch_resident<4>(a, stream);

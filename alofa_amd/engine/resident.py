@@ -148,7 +148,7 @@ _turns: dict = {}      # GPU -> its launches' turns
 
 class ResidentLayers:
     """All layers of ``model`` over ``cache`` as one launch, for steps of at most ``MOST_ROWS`` rows of one new token each."""
-    MOST_ROWS = 16
+    MOST_ROWS = most_rows = 16      # (``most_rows``: of this model, up to 64: csrc/decode_groups.hip)
     MOST_LAYERS = 64      # whose addresses the kernel keeps at hand
     # (rows x key heads below, keys that the longest request sees): the launch cuts a row and key head's keys into sixteen parts, the kernels one by one into as many as the chip has
     # compute units for, up to 64. us a step, one launch / kernel by kernel: one row, two key heads of the 0.5B sizes, 16,000 keys 629 / 764, 31,000 813 / 779; one row and key head, 256
@@ -218,6 +218,7 @@ class ResidentLayers:
         m = blocks[0].mixer
         self.heads, self.kv_heads, self.d, self.scale, self.position = m.heads, m.kv_heads, m.d, m.scale, m.position
         self.hidden, self.intermediate, self.biased = m.hidden, blocks[0].feed_forward.intermediate, m.b_qkv is not None
+        self.most_rows = ops.resident_rows(self.hidden, self.intermediate, self.heads, self.kv_heads)
         self.eps = tuple(float(n.as_rmsnorm()[1]) for n in blocks[0].norms)
         self.page, self.group = cache.block_size, cache.group_of_entry[(0, 0)]
         for t in tables:
@@ -230,7 +231,7 @@ class ResidentLayers:
 
     def takes(self, ctx, rows: int) -> bool:
         """Whether this step runs in one launch: one new token for each of few requests, and keys that it is the faster one for."""
-        if rows > self.MOST_ROWS or ctx.max_q_len != 1 or len(ctx.spans) != rows:
+        if rows > self.most_rows or ctx.max_q_len != 1 or len(ctx.spans) != rows:
             return False
         return ctx.longest <= next((keys for below, keys in self.MOST_KEYS if rows * self.kv_heads < below), ctx.longest)
 

@@ -859,6 +859,11 @@ def resident_takes(hidden: int, intermediate: int, heads: int, kv_heads: int, d:
     return bool(_answer("alofa_resident_takes", _I(hidden), _I(intermediate), _I(heads), _I(kv_heads), _I(d), _I(page)))
 
 
+def resident_rows(hidden: int, intermediate: int, heads: int, kv_heads: int) -> int:
+    """The most rows of a decode step that ``decode_resident`` takes of a model that ``resident_takes``."""
+    return _answer("alofa_resident_rows", _I(hidden), _I(intermediate), _I(heads), _I(kv_heads))
+
+
 def resident_area() -> int:
     """A new area that the blocks of ``decode_resident`` exchange values in: its address. It is never freed."""
     place = ctypes.c_void_p()
