@@ -11,11 +11,12 @@
 // D column l % 16 and rows 4 * (l / 16) .. + 3):
 //   S^T[key, head] = K[key, :] . Q[head, :]        A = keys straight from the cache, B = queries (registers)
 //   O^T[c, head]  += V^T[c, key] * P^T[key, head]   A = values straight from the cache, B = weights (registers)
-// The cache holds the values transposed, so four consecutive keys of a channel
-// are one 8-byte load. After the first product of a step lane l holds, for head
-// l % 16, the scores of keys 4 g + r of either tile (g = l / 16, r = 0..3); these
-// eight are its reduction slots of the second product when the values are read
-// in the same order, so the weights never leave their registers. Scores, the
+// The cache holds the values transposed, so eight consecutive keys of a channel
+// are one 16-byte load. Row i of the first product kt is key 8 (i / 4 % 2) + 4 kt
+// + i % 4 of the step's tile i / 8: after both products lane l holds, for head
+// l % 16, the scores of eight consecutive keys (from 8 (g % 2) on of tile g / 2,
+// g = l / 16), which are its reduction slots of the second product: the weights
+// never leave their registers. Scores, the
 // running maximum, the weights and their sum are float (in units of log2 e);
 // the weights are rounded to bfloat16 only as MFMA operands.
 //
@@ -44,6 +45,9 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kMaxSplits = 64;
+
+// (values may lie on a boundary of eight bytes)
+typedef uint32_t values8 __attribute__((ext_vector_type(4), aligned(8)));
 
 // A result goes to the bfloat16 rows, or, where `out32` is given, unrounded to float rows of the same shape.
 __device__ __forceinline__ void put_out(bf16_t* out, float* out32, int64_t at, float v) {
@@ -142,8 +146,11 @@ __device__ __forceinline__ Pair8 rotate8(uint4 lo, uint4 hi, float4 c_lo, float4
   return Pair8{make_uint4(ra[0], ra[1], ra[2], ra[3]), make_uint4(rb[0], rb[1], rb[2], rb[3])};
 }
 
-// Heads of 128: two blocks to a compute unit (the rotary form's 295 registers come out as 256 and five that are spilled): us, one / two, 28/4 heads, 32 tokens of 128 to 1,028 keys 21.9 / 21.2,
-// 48 of 64 to 512 16.0 / 15.6.
+// Heads of 128: two blocks to a compute unit (us, one / two, 28/4 heads, 32 tokens of 128 to 1,028 keys 21.9 / 21.2, 48 of 64 to 512 16.0 / 15.6).
+// Loads of sixteen bytes of values (a lane's pieces of a page, 32 bytes a channel, lie side by side: 512 bytes in one piece; of eight bytes they were twice as many loads of 16 pieces each, and it is
+// pieces that a compute unit's loads are bound by) and the new token's key and value in LDS (no register of the kernel that turns it is kept in memory any more), us, before / now: 28/4 heads of 128,
+// 32 tokens of 128 to 1,024 keys 19.3 / 18.4, 64 of 128 to 2,048 37.7 / 35.8, in pages of 64 tokens 61.2 / 47.4; 40/8 heads, 16 of 1,000 to 4,000 45.3 / 42.4; 14/2 heads of 64, 64 of 128 to 2,048
+// 14.3 / 14.0, in pages of 64 18.0 / 15.8. The loads alone, with the new token in registers: 22.5, 50.1, 57.2 and 54.9 (heads of 128: eleven registers kept in memory, read back behind the keys on their way).
 // DT = d / 16; NW: waves per block. blockIdx.y = key head * chunks + chunk of up to `block_heads` (<= 16) heads of its group.
 // kSplit: a weight enters the second product as two bfloat16 numbers, its rounding and what the rounding took away: sixteen bits of every weight count.
 template <int DT, int NW, bool kRope, bool kSplit = false, bool kMaps = false>
@@ -222,7 +229,9 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
     qf[ds] = __builtin_bit_cast(bf16x8, v);
   }
 
-  // the new token's key (this lane's channel slices, rotated) and value (channels 16 nt + c16), kRope only
+  // the new token's key (this lane's channel slices, rotated) and value (channels 16 nt + c16), kRope only; from the rotation on they lie in LDS, in the room that the wave's state takes
+  // at the end (held in registers they are 24 at a head size of 128, and what does not fit is read back from memory behind the keys on their way)
+  bf16_t* fresh = reinterpret_cast<bf16_t*>(state[threadIdx.x / 64]);
   uint4 new_k[DS];
   uint32_t new_v[DT];
   constexpr int kPairs = !kRope ? 1 : kMaps ? DS / 4 : DS / 2;      // slices of pairs' first channels; a pair's second lies kPairs slices on (kMaps: in either map's half)
@@ -272,9 +281,11 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
   // them and wait for the oldest step only, so that two later steps stay on their way.
   struct Step {
     uint4 k[2][DS];
-    uint2 v[2][DT];
+    values8 v[DT];
   };
-  const int lo4 = lo & ~3, p4 = p & ~3;
+  const int lo8 = lo & ~7, p8 = p & ~7;
+  const int k_tile = c16 >> 3, k_row = 8 * (c16 >> 2 & 1) + (c16 & 3);      // this lane's row of the first product kt: key k_row + 4 kt of the step's tile k_tile
+  const int v_tile = g >> 1, v_row = 8 * (g & 1);                            // this lane's eight keys of the second: from v_row on of the step's tile v_tile
   auto fetch = [&](int tile, Step& s) __attribute__((always_inline)) {
     const int tile1 = tile_at(tile + 1);
     const bool in_window = !kMaps || tile + 1 >= kept_tiles;      // (kMaps: of the step's two tiles at least the second lies there)
@@ -284,19 +295,22 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
       my_page = (page_base + lane <= last_page) ? table[page_base + lane] : 0;
       my_page = my_page < 0 ? 0 : my_page;
     }
+    // the keys of this lane's rows of K, and the first of this lane's eight keys of V^T, brought into lo..p
+    auto page_of = [&](int key, bool kept) {
+      // (a step past the end of the share may lie before the window of pages held in the lanes: its operands are not used)
+      const int at = (key >> bs_shift) - (kept ? 0 : page_base);
+      const int here = at < 0 ? 0 : (at > 63 ? 63 : at);
+      const int page = __shfl(my_page, here, 64);
+      if constexpr (!kMaps) return static_cast<int64_t>(page);
+      const int kept_one = __shfl(kept_page, here, 64);
+      return static_cast<int64_t>(kept ? kept_one : page);
+    };
+    const bool k_kept = kMaps && tile + k_tile < kept_tiles, v_kept = kMaps && tile + v_tile < kept_tiles;      // (a tile of kept tokens: its pages are all held, and it may hold tokens of the window too)
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt) {
-      // the key of this lane's row of K, and the first of this lane's four keys of V^T, brought into lo..p
-      const int at16 = tile_at(tile + kt) << 4;
-      const bool kept = kMaps && tile + kt < kept_tiles;      // (a tile of kept tokens: its pages are all held, and it may hold tokens of the window too)
-      int key = at16 + c16, key4 = at16 + 4 * g;
-      key = (key < lo && !kept) ? lo : (key > p ? p : key);
-      key4 = (key4 < lo4 && !kept) ? lo4 : (key4 > p4 ? p4 : key4);
-      // (a step past the end of the share may lie before the window of pages held in the lanes: its operands are not used)
-      const int base = kept ? 0 : page_base, pages = kept ? kept_page : my_page;
-      const int kpage = (key >> bs_shift) - base, vpage = (key4 >> bs_shift) - base;
-      const int64_t kblk = __shfl(pages, kpage < 0 ? 0 : (kpage > 63 ? 63 : kpage), 64);
-      const int64_t vblk = __shfl(pages, vpage < 0 ? 0 : (vpage > 63 ? 63 : vpage), 64);
+      int key = (tile_at(tile + k_tile) << 4) + k_row + 4 * kt;
+      key = (key < lo && !k_kept) ? lo : (key > p ? p : key);
+      const int64_t kblk = page_of(key, k_kept);
 #pragma unroll
       for (int ds = 0; ds < DS; ++ds) {
         const int c = ds * 32 + g * 8;
@@ -307,10 +321,12 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
           s.k[kt][ds] = *reinterpret_cast<const uint4*>(k_cache + ((((kblk * kv_heads + hk) << bs_shift) + (key & bs_mask)) * d) + (c < d ? c : 0));
         }
       }
-#pragma unroll
-      for (int nt = 0; nt < DT; ++nt)
-        s.v[kt][nt] = *reinterpret_cast<const uint2*>(v_cache + ((((vblk * kv_heads + hv) * d + nt * 16 + c16) << bs_shift) + (key4 & bs_mask)));
     }
+    int key8 = (tile_at(tile + v_tile) << 4) + v_row;
+    key8 = (key8 < lo8 && !v_kept) ? lo8 : (key8 > p8 ? p8 : key8);
+    const int64_t vblk = page_of(key8, v_kept);
+#pragma unroll
+    for (int nt = 0; nt < DT; ++nt) s.v[nt] = *reinterpret_cast<const values8*>(v_cache + ((((vblk * kv_heads + hv) * d + nt * 16 + c16) << bs_shift) + (key8 & bs_mask)));
   };
 
   // one step: the running state takes the two tiles from `tile` on (tiles past the share's end change nothing)
@@ -320,7 +336,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
     // Most steps of a long context touch neither end of the visible keys nor the new token: they skip the masks and
     // the new token's insertion (branches of the whole wave with no loads inside; the results are the same bits).
     const bool last_here = kRope && tile + 1 >= last;                                                   // the step holds the new token's tile
-    const int at0 = tile_at(tile) << 4, at1 = tile_at(tile + 1) << 4;
+    const int at0 = tile_at(tile) << 4, at1 = tile_at(tile + 1) << 4, first_key = (v_tile == 0 ? at0 : at1) + v_row;      // (this lane's scores are of keys first_key .. + 7)
     auto tile_seen = [&](int at) { return at >= lo || (kMaps && at + 16 <= keep); };
     const bool inner = tile_seen(at0) && (!kMaps || tile_seen(at1)) && at1 + 15 <= p && tile + 1 < tile_end;        // every key of the step is seen
     f32x4 s[2];
@@ -328,15 +344,16 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
     for (int kt = 0; kt < 2; ++kt) {
       s[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
       // (kRope: the new token's key is not in the cache yet: its row of the last tile comes from the registers)
-      const bool new_row = last_here && tile + kt == last && c16 == (p & 15);
+      const bool new_row = last_here && tile + k_tile == last && k_row + 4 * kt == (p & 15);
 #pragma unroll
       for (int ds = 0; ds < DS; ++ds) {
         uint4 kf = st.k[kt][ds];
         if (last_here) {      // (word by word: a choice between two whole operands would be made through memory)
-          kf.x = new_row ? new_k[ds].x : kf.x;
-          kf.y = new_row ? new_k[ds].y : kf.y;
-          kf.z = new_row ? new_k[ds].z : kf.z;
-          kf.w = new_row ? new_k[ds].w : kf.w;
+          const uint4 nk = *reinterpret_cast<const uint4*>(fresh + ds * 32 + g * 8);
+          kf.x = new_row ? nk.x : kf.x;
+          kf.y = new_row ? nk.y : kf.y;
+          kf.z = new_row ? nk.z : kf.z;
+          kf.w = new_row ? nk.w : kf.w;
         }
         s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf), qf[ds], s[kt], 0, 0, 0);
       }
@@ -360,8 +377,8 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
     } else {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const int key = (i < 4 ? at0 : at1) + 4 * g + i % 4;
-        const bool seen = (key >= lo || (kMaps && key < keep)) && key <= p && tile + i / 4 < tile_end;
+        const int key = first_key + i;
+        const bool seen = (key >= lo || (kMaps && key < keep)) && key <= p && tile + v_tile < tile_end;
         pw[i] = seen ? scored(s[i / 4][i % 4]) : -FLT_MAX;
         step_max = fmaxf(step_max, pw[i]);
       }
@@ -386,33 +403,24 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
     }
     // What lies beyond the visible keys is not data: it is cleared, so that a weight of zero times it is zero.
     // (Within lo..p a weight of zero meets a visible key's values.)
-    uint32_t keep_x[2] = {0xffffffffu, 0xffffffffu}, keep_y[2] = {0xffffffffu, 0xffffffffu};
+    uint32_t shown[4] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu};
     if (!inner) {
+      auto hidden = [&](int key) { return (key < lo && (!kMaps || key >= keep)) || key > p; };
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        const int key4 = (kt == 0 ? at0 : at1) + 4 * g;
-        if constexpr (kMaps) {
-          auto hidden = [&](int key) { return (key < lo && key >= keep) || key > p; };
-          keep_x[kt] = (hidden(key4) ? 0u : 0x0000ffffu) | (hidden(key4 + 1) ? 0u : 0xffff0000u);
-          keep_y[kt] = (hidden(key4 + 2) ? 0u : 0x0000ffffu) | (hidden(key4 + 3) ? 0u : 0xffff0000u);
-          continue;
-        }
-        const int lo_e = lo - key4, hi_e = p - key4 + 1;       // elements lo_e .. hi_e - 1 are visible
-        keep_x[kt] = ((0 < lo_e || 0 >= hi_e) ? 0u : 0x0000ffffu) | ((1 < lo_e || 1 >= hi_e) ? 0u : 0xffff0000u);
-        keep_y[kt] = ((2 < lo_e || 2 >= hi_e) ? 0u : 0x0000ffffu) | ((3 < lo_e || 3 >= hi_e) ? 0u : 0xffff0000u);
-      }
+      for (int i = 0; i < 4; ++i) shown[i] = (hidden(first_key + 2 * i) ? 0u : 0x0000ffffu) | (hidden(first_key + 2 * i + 1) ? 0u : 0xffff0000u);
     }
     // O^T += V^T P^T
 #pragma unroll
     for (int nt = 0; nt < DT; ++nt) {
       o[nt] *= corr;
-      uint32_t vw[4] = {st.v[0][nt].x & keep_x[0], st.v[0][nt].y & keep_y[0], st.v[1][nt].x & keep_x[1], st.v[1][nt].y & keep_y[1]};
+      uint32_t vw[4] = {st.v[nt].x & shown[0], st.v[nt].y & shown[1], st.v[nt].z & shown[2], st.v[nt].w & shown[3]};
       if (last_here) {
-        // the new token's value takes its place among this lane's four keys of the last tile
+        // the new token's value takes its place among this lane's eight keys
+        const uint32_t nv = fresh[d + nt * 16 + c16];
 #pragma unroll
         for (int w2 = 0; w2 < 4; ++w2) {
-          const bool hit = tile + w2 / 2 == last && g == ((p & 15) >> 2) && ((p & 3) >> 1) == (w2 & 1);
-          const uint32_t ins = (p & 1) ? ((vw[w2] & 0x0000ffffu) | (new_v[nt] << 16)) : ((vw[w2] & 0xffff0000u) | new_v[nt]);
+          const bool hit = tile + v_tile == last && v_row == (p & 8) && (p & 7) >> 1 == w2;
+          const uint32_t ins = (p & 1) ? ((vw[w2] & 0x0000ffffu) | (nv << 16)) : ((vw[w2] & 0xffff0000u) | nv);
           vw[w2] = hit ? ins : vw[w2];
         }
       }
@@ -447,6 +455,15 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
       new_k[a] = rk.lo;
       new_k[b] = rk.hi;
     }
+    if (c16 == 0) {
+#pragma unroll
+      for (int ds = 0; ds < DS; ++ds) *reinterpret_cast<uint4*>(fresh + ds * 32 + g * 8) = new_k[ds];
+    }
+    if (g == 0) {
+#pragma unroll
+      for (int nt = 0; nt < DT; ++nt) fresh[d + nt * 16 + c16] = static_cast<bf16_t>(new_v[nt]);
+    }
+    wave_lds_sync();
     // the wave that owns the last tile of keys (in the first chunk of heads) writes the token's cache slot
     if (h0 == 0 && tile_begin <= last && last < tile_end) {
       const int64_t blk = new_slot >> bs_shift, off = new_slot & bs_mask;
@@ -490,6 +507,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
   }
   l = rows_sum(l);
 
+  if constexpr (kRope) wave_lds_sync();      // (the new token's key and value have been read)
   // the wave's state: head c16; this lane holds channels 16 nt + 4 g + r
   {
     float* mine = state[wave][c16];

@@ -642,6 +642,27 @@ def test_decode_attention_that_rotates_and_writes_the_new_token(heads, kv_heads,
         o.attention_decode(again, t(qkv, torch.bfloat16), kc, vc, c["table"][:n - 1], None, c["pos"], heads, kv_heads, d, window, scale, bucket, scratch)
 
 
+@pytest.mark.parametrize("d,bs,window", [(64, 8, None), (64, 16, 21), (128, 32, None), (48, 16, 9)])
+def test_decode_attention_at_every_place_of_the_last_key_in_its_step(d, bs, window):
+    """Contexts of 1 to 34 and of 257 to 290 keys: the last key, and the first that a window shows, at every place of a step of 32, values within pages that hold NaN beyond them;
+    and the same bits where the values begin on a boundary of eight bytes."""
+    heads, kv_heads = 6, 2
+    lens = [*range(1, 35), *range(257, 291)]
+    n = len(lens)
+    c = paged_case(np.random.default_rng(31), lens, [1] * n, heads, kv_heads, d, bs, torch.bfloat16)
+    scale = float(np.float32(1) / np.sqrt(np.float32(d)))
+    ref = np.concatenate([pm.attention(c["q"][r], c["k"][r], c["v"][r], heads, kv_heads, d, window) for r in range(n)])
+    room = torch.empty(c["vc"].numel() + 4, device=DEV, dtype=torch.bfloat16)
+    shifted = room[4:].view(c["vc"].shape)
+    shifted.copy_(c["vc"])
+    assert shifted.data_ptr() % 16 == 8
+    out, again = (torch.empty(n, heads * d, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    for to, values in ((out, c["vc"]), (again, shifted)):
+        ops().attention_decode(to, c["qcat"], c["kc"], values, c["table"], c["req"], c["pos"], heads, kv_heads, d, window, scale, 300, None, n_splits=1)
+    close(out, ref, BF16, "decode attention")
+    assert torch.equal(out, again)
+
+
 @pytest.mark.parametrize("heads,kv_heads", [(14, 2), (20, 1), (3, 3)])
 @pytest.mark.parametrize("parts", [2, 3])
 @pytest.mark.parametrize("n,kind", [(33, "spread"), (33, "one long"), (40, "alike"), (63, "spread"), (64, "spread"), (64, "one long"), (64, "single keys")])
