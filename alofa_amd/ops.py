@@ -1475,7 +1475,7 @@ def recurrence_max_parts(dk: int) -> int:
 
 def linear_recurrence(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Tensor, rows: RowsOfRequests,
                       heads: int, dk: int, dv: int, decay_kind: int, decay: torch.Tensor, tau: float = 1.0, bonus: Optional[torch.Tensor] = None,
-                      q_scale: float = 1.0, k_scale: float = 1.0, before_update: bool = False) -> int:
+                      q_scale: float = 1.0, k_scale: float = 1.0, before_update: bool = False, finish: Optional[tuple] = None, rope: Optional[tuple] = None) -> int:
     """Per request (in its rows' order) and head: S = diag(w_t) S + k_t v_t^T and out_t = S^T q_t, or with
     ``before_update`` out_t = (S + diag(bonus) k_t v_t^T)^T q_t first and the update after it. S float32
     [slots, heads, dk, dv] is read and left in ``state``. q, k [T, heads * dk] and v [T, heads * dv] are rows in one
@@ -1484,7 +1484,11 @@ def linear_recurrence(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: to
     (1 otherwise), and ``headnorm_gate(parts=)`` adds them. The decay w_t: ``DECAY_PER_HEAD`` with ``decay``
     float32 [heads]; ``DECAY_SIGMOID_ROOT`` sigmoid(z)^(1/tau) or ``DECAY_EXP_NEG_EXP`` exp(-exp(z)) with ``decay`` = z
     float32 [T, heads * dk] rows, which a step of many rows overwrites with the decays made of them; ``DECAY_GIVEN``:
-    ``decay`` holds the w_t themselves."""
+    ``decay`` holds the w_t themselves. ``finish`` = (gate, weight, eps), and ``rope`` = (cos, sin, positions) with it: ``recurrence_step``, what stands around the
+    recurrence of single rows in the same launch."""
+    if finish is not None:
+        recurrence_step(out, q, k, v, finish[0], finish[1], state, rows, heads, dk, dv, finish[2], decay_kind, decay, tau, bonus, q_scale, k_scale, before_update, rope)
+        return 1
     _gpu("out", out, torch.float32), _contig("out", out), _gpu("q", q, None, 2), _gpu("k", k, q.dtype, 2), _gpu("v", v, q.dtype, 2)
     _gpu("state", state, torch.float32, 4), _contig("state", state)
     T = q.shape[0]
@@ -1512,6 +1516,47 @@ def linear_recurrence(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: to
           _ptr(rows.slots), _ptr(rows.offsets), _I(rows.requests), _I(T), _I(heads), _I(dk), _I(dv), _I(decay_kind), _F(tau), _F(q_scale), _F(k_scale),
           _I(int(before_update)), _stream())
     return used.value
+
+
+def recurrence_step_takes(rows: RowsOfRequests, dk: int, dv: int, dtype: torch.dtype, q: torch.Tensor) -> bool:
+    """Whether ``recurrence_step`` takes a step: one row of every request, bfloat16 rows, heads of at most 256 key and value channels, the latter in fours."""
+    return rows.offsets is None and dtype is torch.bfloat16 and q.dtype is torch.bfloat16 and 0 < dk <= 256 and 4 <= dv <= 256 and dv % 4 == 0
+
+
+def recurrence_step(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torch.Tensor, weight: Optional[torch.Tensor], state: torch.Tensor, rows: RowsOfRequests,
+                    heads: int, dk: int, dv: int, eps: float, decay_kind: int, decay: torch.Tensor, tau: float = 1.0, bonus: Optional[torch.Tensor] = None, q_scale: float = 1.0,
+                    k_scale: float = 1.0, before_update: bool = False, rope: Optional[tuple] = None) -> None:
+    """``linear_recurrence`` for steps in which every request brings one row, with what stands around it in one launch: with ``rope`` = (cos, sin, positions) the rotation
+    of queries and keys (``rope_kv_write`` of both, which are left as they are), and ``headnorm_gate`` (silu) of the read-outs, which ``out`` [T, heads * dv] receives. All rows bfloat16."""
+    T = q.shape[0]
+    for name, t, width in (("out", out, heads * dv), ("q", q, heads * dk), ("k", k, heads * dk), ("v", v, heads * dv), ("gate", gate, heads * dv)):
+        if tuple(_gpu(name, t, torch.bfloat16, 2).shape) != (T, width):
+            raise AlofaError("shape_mismatch", "recurrence operands do not fit", f"operand={name} shape={tuple(t.shape)} rows={T} heads={heads} dk={dk} dv={dv}")
+    _gpu("state", state, torch.float32, 4), _contig("state", state)
+    if tuple(state.shape[1:]) != (heads, dk, dv) or T != rows.rows or not recurrence_step_takes(rows, dk, dv, out.dtype, q):
+        raise AlofaError("shape_mismatch", "a step of one row a request, heads of at most 256 channels", f"state={tuple(state.shape)} heads={heads} dk={dk} dv={dv} rows={rows.rows}")
+    rows.fits("state", state)
+    per_head = decay_kind == DECAY_PER_HEAD
+    _gpu("decay", decay, torch.float32, 1 if per_head else 2)
+    if per_head:
+        _contig("decay", decay)
+    if decay_kind not in (DECAY_PER_HEAD, DECAY_SIGMOID_ROOT, DECAY_EXP_NEG_EXP) or tuple(decay.shape) != ((heads,) if per_head else (T, heads * dk)):
+        raise AlofaError("shape_mismatch", "the decay does not fit its kind", f"decay={tuple(decay.shape)} kind={decay_kind} heads={heads} dk={dk}")
+    if bonus is not None and (tuple(_contig("bonus", _gpu("bonus", bonus, torch.float32, 2)).shape) != (heads, dk) or not before_update):
+        raise AlofaError("shape_mismatch", "the bonus is [heads, dk] and goes with the read-out before the update", f"bonus={tuple(bonus.shape)}")
+    if weight is not None and tuple(_contig("weight", _gpu("weight", weight, torch.float32, 1)).shape) != (heads * dv,):
+        raise AlofaError("shape_mismatch", "one weight per head and channel", f"weight={tuple(weight.shape)} heads={heads} dv={dv}")
+    cos = sin = positions = None
+    if rope is not None:
+        cos, sin, positions = rope
+        for name, t in (("cos", cos), ("sin", sin)):
+            if dk % 2 or _contig(name, _gpu(name, t, torch.float32, 2)).shape[1] != dk // 2 or t.shape[0] != cos.shape[0]:
+                raise AlofaError("shape_mismatch", "rotary table must be [positions, dk / 2]", f"operand={name} shape={tuple(t.shape)} dk={dk}")
+        if tuple(_contig("positions", _gpu("positions", positions, torch.int32, 1)).shape) != (T,):
+            raise AlofaError("shape_mismatch", "one position per row", f"positions={tuple(positions.shape)} rows={T}")
+    _call("alofa_recurrence_step", _ptr(out), _L(_rows("out", out)), _ptr(q), _L(_rows("q", q)), _ptr(k), _L(_rows("k", k)), _ptr(v), _L(_rows("v", v)), _ptr(gate), _L(_rows("gate", gate)),
+          _ptr(decay), _L(0 if per_head else _rows("decay", decay)), _ptr(bonus), _ptr(weight), _ptr(state), _ptr(rows.slots), _ptr(cos), _ptr(sin), _ptr(positions),
+          _I(T), _I(heads), _I(dk), _I(dv), _I(decay_kind), _F(tau), _F(q_scale), _F(k_scale), _F(eps), _I(int(before_update)), _stream())
 
 
 CHUNK_ROWS = 64           # rows of a chunk of ``chunked_recurrence``

@@ -10,6 +10,7 @@ gated_linear    w_t = sigmoid(z_t)^(1/tau) per key channel, z = W_a2 (W_a1 x) + 
 time_mix        RWKV-style: each of r, k, v, g, w reads its own mix of the token with the one before it,
                 x + (x' - x) mu_s; w_t = exp(-exp(W_w2 tanh(W_w1 mix_w) + w0)); o_t = (S_(t-1) + diag(u) k_t v_t^T)^T r_t,
                 then the update; o / rms(o) per head, times a weight per channel, times silu(g), output projection.
+(In steps of one row a request these three run rotation, recurrence, norm and gate as one launch, ``ops.recurrence_step``.)
 
 lightning_attention  w = a constant per head; q, k, v through silu; o_t = S_t^T q_t; the heads together through an RMS norm with a
                 weight, times sigmoid(gate), output projection.
@@ -82,10 +83,23 @@ class RecurrentMixer(Mixer):
         """Head norm, gate and output projection of the read-outs ``o`` (float32 [P, T, heads * dv], the first ``parts`` to be added)."""
         y = ctx.scratch("recurrent_gated", (o.shape[1], self.heads * self.dv), self.rt.dtype)
         ops.headnorm_gate(y, o, gate, weight, self.heads, self.dv, self.eps, self.rt.exact, parts=parts)
+        self._project(ctx, y, residual, out)
+
+    def _project(self, ctx, y, residual, out):
         if out is not None:
             ops.gemm(out, y, self.w_o, exact=self.rt.exact, scratch=ctx.scratch)
         else:
             ops.gemm(residual, y, self.w_o, add_to_out=True, exact=self.rt.exact, scratch=ctx.scratch)
+
+    def _single_step(self, ctx, where, q, k, v, gate, weight, residual, out, decay_kind, decay, **how) -> bool:
+        """Where every request brings one row: the recurrence, the head norm and the gate in one launch, and the output projection. False (and nothing done) where it is no such step."""
+        rows = rows_of_requests(ctx)
+        if not ops.recurrence_step_takes(rows, self.dk, self.dv, self.rt.dtype, q):
+            return False
+        y = ctx.scratch("recurrent_gated", (q.shape[0], self.heads * self.dv), self.rt.dtype)
+        ops.linear_recurrence(y, q, k, v, ctx.state(where), rows, self.heads, self.dk, self.dv, decay_kind, decay, finish=(gate, weight, self.eps), **how)
+        self._project(ctx, y, residual, out)
+        return True
 
 
 class Retention(RecurrentMixer):
@@ -128,11 +142,12 @@ class Retention(RecurrentMixer):
         proj = ctx.scratch("recurrent_proj", (T, 2 * kd + 2 * vd), self.rt.dtype)
         ops.gemm(proj, x, self.w_in, exact=self.rt.exact, scratch=ctx.scratch)
         table = self.position.table(ctx.n_positions) if self.position is not None else None
-        if self.position is None:
-            pass
-        elif table is None:
+        if self.position is not None and table is None:
             self.position.apply(ctx, proj[:, :kd].unflatten(1, (self.heads, self.dk)), proj[:, kd:2 * kd].unflatten(1, (self.heads, self.dk)))
-        else:      # queries and keys alike: 2 * heads heads to rotate, nothing to write to pages
+        if self._single_step(ctx, where, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:2 * kd + vd], proj[:, 2 * kd + vd:], None, residual, out, ops.DECAY_PER_HEAD, self.decay,
+                             k_scale=self.k_scale, rope=None if table is None else (*table, ctx.positions)):
+            return
+        if table is not None:      # queries and keys alike: 2 * heads heads to rotate, nothing to write to pages
             ops.rope_kv_write(proj, table[0], table[1], ctx.positions, 2 * self.heads, 0, self.dk)
         o = self._readouts(ctx, T)
         parts = self._constant_decay(ctx, where, o, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:2 * kd + vd], self.k_scale)
@@ -170,6 +185,9 @@ class GatedLinearAttention(RecurrentMixer):
         ops.gemm(proj, x, self.w_in, exact=self.rt.exact, scratch=ctx.scratch)
         z = ctx.scratch("recurrent_decay", (T, kd), torch.float32)
         ops.gemm(z, proj[:, 2 * kd + 2 * vd:], self.w_a2, self.b_a2, exact=self.rt.exact, scratch=ctx.scratch)
+        if self._single_step(ctx, where, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:2 * kd + vd], proj[:, 2 * kd + vd:2 * kd + 2 * vd], self.norm, residual, out, ops.DECAY_SIGMOID_ROOT, z,
+                             tau=self.tau, q_scale=self.q_scale):
+            return
         o = self._readouts(ctx, T)
         parts = ops.linear_recurrence(o, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:2 * kd + vd], ctx.state(where), rows_of_requests(ctx),
                                       self.heads, self.dk, self.dv, ops.DECAY_SIGMOID_ROOT, z, tau=self.tau, q_scale=self.q_scale)
@@ -439,6 +457,9 @@ class TimeMix(RecurrentMixer):
         ops.activation(low, low, ops.TANH, exact=exact)
         z = ctx.scratch("recurrent_decay", (T, kd), torch.float32)
         ops.gemm(z, low, self.w["w2"], self.w0, exact=exact, scratch=ctx.scratch)
+        if self._single_step(ctx, (entry, k), proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:3 * kd], proj[:, 3 * kd:], self.norm, residual, out, ops.DECAY_EXP_NEG_EXP, z,
+                             bonus=self.bonus, before_update=True):
+            return
         o = self._readouts(ctx, T)
         parts = ops.linear_recurrence(o, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:3 * kd], ctx.state((entry, k)), rows_of_requests(ctx),
                                       self.heads, self.dk, self.dv, ops.DECAY_EXP_NEG_EXP, z, bonus=self.bonus, before_update=True)

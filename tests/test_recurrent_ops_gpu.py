@@ -301,3 +301,58 @@ def test_a_slot_is_cleared_on_the_callers_stream():
         scope.__exit__(None, None, None)
     busy.synchronize()
     assert bool((got[1] == 0).all()) and bool((got[[0, 2]] == 1).all())
+
+
+@pytest.mark.parametrize("heads,dk,dv", [(1, 1, 4), (3, 63, 20), (16, 64, 64), (5, 96, 40), (2, 128, 256), (3, 256, 252), (2, 256, 256)])
+@pytest.mark.parametrize("kind", ["per head", "sigmoid root", "exp of exp, bonus"])
+@pytest.mark.parametrize("turned", [False, True])
+def test_single_row_step_in_one_launch(heads, dk, dv, kind, turned):
+    """Rotation, recurrence, head norm and gate in one launch beside the launches it replaces and beside float64; slots in any order, others left alone."""
+    from alofa_amd import ops
+    if turned and dk % 2:
+        return
+    rng = np.random.default_rng(heads * dk + dv)
+    T, n_slots, used = 5, 9, (7, 0, 3, 8, 4)
+    rows = rows_of([(s, 1) for s in used], n_slots)
+    proj = dev(rng.normal(0, 1, (T, heads * (2 * dk + 2 * dv) + 8)), torch.bfloat16)
+    kd, vd = heads * dk, heads * dv
+    q, k, v, gate = proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:2 * kd + vd], proj[:, 2 * kd + vd:2 * kd + 2 * vd]
+    state = dev(rng.normal(0, 1, (n_slots, heads, dk, dv)))
+    weight = None if kind == "per head" else dev(rng.normal(1, 0.2, vd))
+    bonus = dev(rng.normal(0, 1, (heads, dk))) if kind.startswith("exp") else None
+    code = {"per head": ops.DECAY_PER_HEAD, "sigmoid root": ops.DECAY_SIGMOID_ROOT}.get(kind, ops.DECAY_EXP_NEG_EXP)
+    decay = dev(rng.uniform(0.5, 0.99, heads)) if code == ops.DECAY_PER_HEAD else dev(rng.normal(0, 1, (T, kd)))
+    how = dict(tau=4.0, bonus=bonus, q_scale=0.5, k_scale=0.25, before_update=bonus is not None)
+    cos, sin = (dev(rng.uniform(-1, 1, (11, max(dk // 2, 1)))) for _ in range(2))
+    positions = torch.tensor([10, 0, 3, 5, 5], dtype=torch.int32, device=DEV)
+    out, got_state, kept = torch.empty(T, vd, device=DEV, dtype=torch.bfloat16), state.clone(), proj.clone()
+    ops.recurrence_step(out, q, k, v, gate, weight, got_state, rows, heads, dk, dv, 1e-5, code, decay, rope=(cos, sin, positions) if turned else None, **how)
+    assert torch.equal(proj, kept)
+
+    # launch by launch
+    if turned:
+        ops.rope_kv_write(proj, cos, sin, positions, 2 * heads, 0, dk)
+    o, old_state, old = torch.empty(T, vd, device=DEV), state.clone(), torch.empty_like(out)
+    ops.linear_recurrence(o, q, k, v, old_state, rows, heads, dk, dv, code, decay.clone(), **how)
+    ops.headnorm_gate(old, o, gate, weight, heads, dv, 1e-5, False)
+    # (a number of the state is one product and one sum in either, two roundings of at most 2^-24 of terms below 8)
+    assert torch.allclose(got_state, old_state, rtol=1e-6, atol=1e-6)
+
+    # in float64
+    S = state.double()[rows.slots.long()]
+    qd, kh, vh = (t.double().unflatten(1, (heads, -1)) for t in (q, k, v))
+    qd, kh = qd * 0.5, kh * 0.25
+    if code == ops.DECAY_PER_HEAD:
+        w = decay.double()[None, :, None].expand(T, heads, dk)
+    else:
+        w = (torch.sigmoid(decay.double()) ** 0.25 if code == ops.DECAY_SIGMOID_ROOT else torch.exp(-torch.exp(decay.double()))).unflatten(1, (heads, -1))
+    kv = kh[..., None] * vh[:, :, None]
+    new = w[..., None] * S + kv
+    read = ((S + bonus.double()[None, :, :, None] * kv if bonus is not None else new) * qd[..., None]).sum(2)
+    y = (read / torch.sqrt((read * read).mean(2, keepdim=True) + 1e-5)).flatten(1) * (1 if weight is None else weight.double()) * torch.nn.functional.silu(gate.double())
+    assert ((got_state[rows.slots.long()].double() - new).norm() / new.norm()).item() < 1e-6
+    untouched = [s for s in range(n_slots) if s not in used]
+    assert torch.equal(got_state[untouched], state[untouched])
+    # a result is rounded once, to bfloat16: by at most 2^-9 of it; both ways are off by those roundings, and where a sum falls close to the middle of two of them they differ
+    off = {n: ((x.double() - y).norm() / y.norm()).item() for n, x in (("one launch", out), ("launch by launch", old))}
+    assert off["one launch"] < 2 ** -9 and off["one launch"] <= off["launch by launch"] * 1.01 + 1e-5, off
