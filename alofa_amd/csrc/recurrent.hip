@@ -74,43 +74,64 @@ __global__ void __launch_bounds__(256) keep_last_rows_kernel(TI* __restrict__ st
 // which then moves on by n. A block owns 256 channels of a row (every block of a row takes the row's two sums itself: the
 // row is a few kilobytes), a thread one channel of the request's state: it fetches what the state holds at once, and
 // writes afterwards.
-template <typename TO, typename Acc>
+// kTaps: the filter's taps where the host knows them (4 and fewer, of which the loads then set out together, none under a condition), 0: up to kMaxKeep + 1. kOwn: values of the row that a thread
+// keeps between the sums (wider rows are read again). A dependent read is what such a launch waits for, so the row, the state and the weights set out before the first sum: 4 rows of 1,024, four
+// taps, in a captured step: 4.7 us as one loop over the row a sum and sixteen conditional loads, 2.8 so; the same bits.
+template <typename TO, typename Acc, int kTaps, int kOwn>
 __global__ void __launch_bounds__(256) norm_conv_step_kernel(TO* __restrict__ out, const float* __restrict__ x, const float* __restrict__ nw,
                                                              const float* __restrict__ nb, float eps, const float* __restrict__ w,
-                                                             float* __restrict__ state, const int32_t* __restrict__ req_slot, int width, int taps) {
-  __shared__ Acc scratch[4];
-  const int r = blockIdx.y, c = blockIdx.x * 256 + threadIdx.x;
+                                                             float* __restrict__ state, const int32_t* __restrict__ req_slot, int width, int any_taps) {
+  __shared__ Acc scratch[2][4];
+  const int taps = kTaps > 0 ? kTaps : any_taps;
+  constexpr int kKeep = kTaps > 0 ? kTaps - 1 : kMaxKeep;
+  const int r = blockIdx.y, c = blockIdx.x * 256 + threadIdx.x, own_c = c < width ? c : width - 1;
   const float* src = x + static_cast<int64_t>(r) * width;
-  float* st = state + static_cast<int64_t>(req_slot[r]) * (taps - 1) * width;
-  float kept[kMaxKeep], wc[kMaxKeep + 1];
+  const int slot = req_slot[r];
+  float own[kOwn > 0 ? kOwn : 1];
 #pragma unroll
-  for (int jj = 0; jj < kMaxKeep; ++jj) kept[jj] = (c < width && jj < taps - 1) ? st[static_cast<int64_t>(jj) * width + c] : 0.f;
+  for (int i = 0; i < kOwn; ++i) own[i] = src[min(static_cast<int>(threadIdx.x) + i * 256, width - 1)];
+  const float mine = src[own_c], weight = nw[own_c], shift = nb[own_c];
+  float* st = state + static_cast<int64_t>(slot) * (taps - 1) * width;
+  float kept[kKeep > 0 ? kKeep : 1], wc[kKeep + 1];
 #pragma unroll
-  for (int jj = 0; jj <= kMaxKeep; ++jj) wc[jj] = (c < width && jj < taps) ? w[static_cast<int64_t>(c) * taps + jj] : 0.f;
+  for (int jj = 0; jj <= kKeep; ++jj) wc[jj] = (kTaps > 0 || jj < taps) ? w[static_cast<int64_t>(own_c) * taps + jj] : 0.f;
+#pragma unroll
+  for (int jj = 0; jj < kKeep; ++jj) kept[jj] = (kTaps > 0 || jj < taps - 1) ? st[static_cast<int64_t>(jj) * width + own_c] : 0.f;
   Acc s = 0;
-  for (int e = threadIdx.x; e < width; e += 256) s += static_cast<Acc>(src[e]);
-  const Acc mean = block_sum<Acc, 256>(s, scratch) / static_cast<Acc>(width);
-  Acc ss = 0;
-  for (int e = threadIdx.x; e < width; e += 256) {
-    const Acc d = static_cast<Acc>(src[e]) - mean;
-    ss += d * d;
+  if constexpr (kOwn > 0) {
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) s += static_cast<int>(threadIdx.x) + i * 256 < width ? static_cast<Acc>(own[i]) : static_cast<Acc>(0);
+  } else {
+    for (int e = threadIdx.x; e < width; e += 256) s += static_cast<Acc>(src[e]);
   }
-  const Acc var = block_sum<Acc, 256>(ss, scratch) / static_cast<Acc>(width);
+  const Acc mean = block_sum<Acc, 256>(s, scratch[0]) / static_cast<Acc>(width);
+  Acc ss = 0;
+  auto squared = [&](float v) {
+    const Acc d = static_cast<Acc>(v) - mean;
+    return d * d;
+  };
+  if constexpr (kOwn > 0) {
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) ss += static_cast<int>(threadIdx.x) + i * 256 < width ? squared(own[i]) : static_cast<Acc>(0);
+  } else {
+    for (int e = threadIdx.x; e < width; e += 256) ss += squared(src[e]);
+  }
+  const Acc var = block_sum<Acc, 256>(ss, scratch[1]) / static_cast<Acc>(width);
   if (c >= width) return;
   const Acc inv = static_cast<Acc>(1) / sqrt(var + static_cast<Acc>(eps));
-  const float n = static_cast<float>((static_cast<Acc>(src[c]) - mean) * inv * static_cast<Acc>(nw[c]) + static_cast<Acc>(nb[c]));
+  const float n = static_cast<float>((static_cast<Acc>(mine) - mean) * inv * static_cast<Acc>(weight) + static_cast<Acc>(shift));
   Acc acc = static_cast<Acc>(n);
-  float last = n;      // the filter's own tap on the row itself comes last, as in the kernel for any rows
 #pragma unroll
-  for (int jj = 0; jj < kMaxKeep; ++jj) {
-    if (jj < taps - 1) {
+  for (int jj = 0; jj < kKeep; ++jj) {
+    if (kTaps > 0 || jj < taps - 1) {
       acc += static_cast<Acc>(wc[jj]) * static_cast<Acc>(kept[jj]);
       if (jj > 0) st[static_cast<int64_t>(jj - 1) * width + c] = kept[jj];
     }
   }
+  // (the filter's own tap on the row itself comes last, as in the kernel for any rows)
 #pragma unroll
-  for (int jj = 0; jj <= kMaxKeep; ++jj)
-    if (jj == taps - 1) acc += static_cast<Acc>(wc[jj]) * static_cast<Acc>(last);
+  for (int jj = 0; jj <= kKeep; ++jj)
+    if (jj == taps - 1) acc += static_cast<Acc>(wc[jj]) * static_cast<Acc>(n);
   if (taps > 1) st[static_cast<int64_t>(taps - 2) * width + c] = n;
   store_f32(out + static_cast<int64_t>(r) * width + c, static_cast<float>(acc));
 }
@@ -550,9 +571,18 @@ extern "C" int alofa_norm_conv_step(void* out, int out_dtype, const float* x, co
   ALOFA_REQUIRE(!exact || out_dtype == kF32, "norm_conv_step: the exact path writes float32");
   if (rows == 0) return 0;
   const dim3 grid((width + 255) / 256, rows);
-  if (exact) norm_conv_step_kernel<float, double><<<grid, 256, 0, stream>>>(static_cast<float*>(out), x, nw, nb, eps, w, state, req_slot, width, taps);
-  else if (out_dtype == kF32) norm_conv_step_kernel<float, float><<<grid, 256, 0, stream>>>(static_cast<float*>(out), x, nw, nb, eps, w, state, req_slot, width, taps);
-  else norm_conv_step_kernel<bf16_t, float><<<grid, 256, 0, stream>>>(static_cast<bf16_t*>(out), x, nw, nb, eps, w, state, req_slot, width, taps);
+#define ALOFA_STEP_AS(TO, ACC, TAPS, OWN) norm_conv_step_kernel<TO, ACC, TAPS, OWN><<<grid, 256, 0, stream>>>(static_cast<TO*>(out), x, nw, nb, eps, w, state, req_slot, width, taps)
+#define ALOFA_STEP(TO, ACC)                                                                     \
+  if (width > 2048) ALOFA_STEP_AS(TO, ACC, 0, 0);                                               \
+  else if (taps == 2) ALOFA_STEP_AS(TO, ACC, 2, 8);                                             \
+  else if (taps == 3) ALOFA_STEP_AS(TO, ACC, 3, 8);                                             \
+  else if (taps == 4) ALOFA_STEP_AS(TO, ACC, 4, 8);                                             \
+  else ALOFA_STEP_AS(TO, ACC, 0, 8)
+  if (exact) { ALOFA_STEP(float, double); }
+  else if (out_dtype == kF32) { ALOFA_STEP(float, float); }
+  else { ALOFA_STEP(bf16_t, float); }
+#undef ALOFA_STEP
+#undef ALOFA_STEP_AS
   return check_launch("norm_conv_step");
 }
 

@@ -356,3 +356,24 @@ def test_single_row_step_in_one_launch(heads, dk, dv, kind, turned):
     # a result is rounded once, to bfloat16: by at most 2^-9 of it; both ways are off by those roundings, and where a sum falls close to the middle of two of them they differ
     off = {n: ((x.double() - y).norm() / y.norm()).item() for n, x in (("one launch", out), ("launch by launch", old))}
     assert off["one launch"] < 2 ** -9 and off["one launch"] <= off["launch by launch"] * 1.01 + 1e-5, off
+
+
+@pytest.mark.parametrize("width", [1, 255, 1025, 2048, 2049, 4100])
+@pytest.mark.parametrize("taps", [2, 3, 4, 5])
+def test_norm_filter_and_state_at_the_edges_of_its_forms(width, taps):
+    """Widths around a block's channels and what a thread keeps of a row, the taps that have a form of their own and the next: norm, filter and state beside the launches for any rows."""
+    from alofa_amd import ops
+    rng = np.random.default_rng(width + taps)
+    n_slots, rows = 6, rows_of([(4, 1), (0, 1), (5, 1)], 6)
+    x, w, b, f = dev(rng.normal(1, 2, (3, width))), dev(rng.normal(1, 0.2, width)), dev(rng.normal(0, 0.5, width)), dev(rng.normal(0, 0.5, (width, taps)))
+    state = dev(rng.normal(0, 1, (n_slots, taps - 1, width)))
+    for dtype in (torch.float32, torch.bfloat16):
+        one, got = state.clone(), torch.empty(3, width, device=DEV, dtype=dtype)
+        ops.norm_conv_step(got, x, w, b, 1e-5, f, one, rows)
+        apart, n, want = state.clone(), torch.empty(3, width, device=DEV), torch.empty(3, width, device=DEV)
+        ops.layernorm(n, x, w, b, 1e-5, False)
+        ops.short_conv(want, n, f, apart, rows)
+        ops.keep_last_rows(apart, n, rows)
+        # (a norm's sums of up to 4,100 numbers in another order: 1e-6 of numbers around 3; a rounding to bfloat16 is 2^-9 of a number)
+        assert torch.allclose(one, apart, rtol=1e-5, atol=1e-5)
+        assert torch.allclose(got.float(), want, rtol=2 ** -8 if dtype is torch.bfloat16 else 1e-5, atol=1e-4)
