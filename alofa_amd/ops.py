@@ -1017,6 +1017,30 @@ def attention_tall(out, q, k_cache, v_cache, block_table, runs, heads, kv_heads,
           _ptr(runs), _I(runs.shape[0]), _I(heads), _I(kv_heads), _I(d), _I(bs), _I(int(window or 0)), _F(scale), _stream())
 
 
+def attention_teams_pays(heads: int, kv_heads: int, d: int, block_size: int, scale: float, runs: int, window: Optional[int] = None) -> bool:
+    """Whether ``runs`` runs of up to 64 rows go to the kernel of heads of 64 whose waves own 32 rows: always where the other kernel's heads have blocks of their own (14/2 heads, 30
+    launches of portions from 5 to 8,192 rows, us, the other / this: 0.99 to 1.37 times as fast, 40 portions of 40 rows 20.7 / 20.9), and without a window also where a group's heads share its
+    tiles with 16 rows a wave (two prompts of 2,048 47.4 / 42.1, one of 4,096 85.6 / 63.6). Where they share them with 32 rows a wave a tile serves 224 (row, head) pairs instead of 64:
+    four of 2,048 68 / 80, one of 8,192 even; and with a window (four of 1,024 on 500 keys, window 300) 25.2 / 34.6."""
+    if d != 64 or block_size < 16 or not scale > 0:
+        return False
+    share = prefill_share(heads, kv_heads, d, runs)
+    return not share or (not window and prefill_rows(heads, kv_heads, d, share, runs) == 16)
+
+
+def attention_teams(out, q, k_cache, v_cache, block_table, tiles, heads, kv_heads, d, window, scale) -> None:
+    """bfloat16 attention for portions of prompts, heads of 64, pages of 16 tokens or more: 64 query rows of one head a block. ``tiles`` as ``attention_prefill`` takes them
+    (paired for ``heads`` blocks a run)."""
+    T, bs = _attention_operands(out, q, k_cache, v_cache, block_table, heads, kv_heads, d)
+    if out.dtype is not torch.bfloat16:
+        raise AlofaError("unsupported", "this attention kernel leaves bfloat16 rows", f"out={out.dtype}")
+    _gpu("tiles", tiles, torch.int32, 3), _contig("tiles", tiles)
+    if tuple(tiles.shape[1:]) != (2, 4) or tiles.shape[0] == 0:
+        raise AlofaError("shape_mismatch", "tiles must be [n, 2, 4]", f"tiles={tuple(tiles.shape)}")
+    _call("alofa_attention_teams", _ptr(out), _L(_rows("out", out)), _ptr(q), _L(_rows("q", q)), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), _I(block_table.shape[1]),
+          _ptr(tiles), _I(tiles.shape[0]), _I(heads), _I(kv_heads), _I(d), _I(bs), _I(int(window or 0)), _F(scale), _stream())
+
+
 def attention_prefill(out, q, k_cache, v_cache, block_table, tiles, heads, kv_heads, d, window, scale, share: int = 0,
                       rows: int = 16, v_head: Optional[int] = None, fine_weights: bool = False, all_value_heads: bool = False,
                       sink: Optional[torch.Tensor] = None) -> None:

@@ -38,6 +38,7 @@ class RowPlan:
         self.long_runs = None       # (request index, first row, rows, first position) per run; None when every row is short
         self._tiles: dict = {}
         self._tall: dict = {}
+        self._teams: dict = {}
         if self.n_short < ctx.tokens:
             self.long_runs = [(i, s.row0 + q0, min(TILE_ROWS, s.n - q0), s.pos0 + q0)
                               for i, s in enumerate(spans) if s.n > SHORT for q0 in range(0, s.n, TILE_ROWS)]
@@ -50,6 +51,13 @@ class RowPlan:
         if key not in self._tall:
             self._tall[key] = ops.attention_tall_pays(*key[:-1], [(s.n, s.pos0 + s.n) for s in self.spans if s.n > SHORT], window)
         return self._tall[key]
+
+    def in_team_blocks(self, heads: int, kv_heads: int, d: int, block_size: int, scale: float, window) -> bool:
+        """Whether the runs go to the kernel of heads of 64 whose waves own 32 rows."""
+        key = (heads, kv_heads, d, block_size, scale, window)
+        if key not in self._teams:
+            self._teams[key] = ops.attention_teams_pays(*key[:-1], len(self.long_runs), window)
+        return self._teams[key]
 
     def tall_runs(self):
         """The long portions in runs of up to ``ops.TALL_ROWS`` rows, the ones that see most keys first: int32 [n, 4] (request index, first row, rows, position of the first row)."""
@@ -111,6 +119,8 @@ def paged_attend(ctx, entry, qkv, attn, heads, kv_heads, d, window, scale, posit
     else:
         if plan.long_runs is not None and plan.in_tall_blocks(heads, kv_heads, d, kv.k.shape[2], scale, window):      # portions of prompts, many rows
             ops.attention_tall(attn, qkv, kv.k, kv.v, kv.block_table, ctx.memo("gqa_attention.tall_runs", plan.tall_runs), *common)
+        elif plan.long_runs is not None and plan.in_team_blocks(heads, kv_heads, d, kv.k.shape[2], scale, window):
+            ops.attention_teams(attn, qkv, kv.k, kv.v, kv.block_table, plan.tiles(heads, kv_heads, d, window, plain=True)[0], *common)
         elif plan.long_runs is not None:      # portions of prompts
             tiles, share, rows = plan.tiles(heads, kv_heads, d, window)
             ops.attention_prefill(attn, qkv, kv.k, kv.v, kv.block_table, tiles, *common, share=share, rows=rows)

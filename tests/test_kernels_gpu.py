@@ -952,6 +952,49 @@ def test_prefill_attention(heads, kv_heads, d, bs, window):
                                 share=5)
 
 
+@pytest.mark.parametrize("heads,kv_heads,bs", [(14, 2, 16), (5, 1, 64), (4, 4, 32), (9, 3, 128)])
+@pytest.mark.parametrize("window", [None, 1, 21, 64, 300])
+def test_attention_of_heads_of_64_in_teams(heads, kv_heads, bs, window):
+    """The kernel whose waves own 32 rows of heads of 64: runs of 1, 31 to 33, 63 to 65 rows, portions that begin in the middle of a tile, contexts that end at every edge of a
+    tile and a round of four, two runs a block and one; NaN in all pages that no table names and beyond the last key of those that do."""
+    d = 64
+    lens, q_lens = [1, 37, 130, 700, 64, 65, 200, 257, 512, 321, 319], [1, 32, 5, 100, 64, 65, 200, 33, 31, 63, 64]
+    c = paged_case(np.random.default_rng(29), lens, q_lens, heads, kv_heads, d, bs, torch.bfloat16)
+    scale = float(np.float32(1) / np.sqrt(np.float32(d)))
+    tiles, row = [], 0
+    for r, (L, n) in enumerate(zip(lens, q_lens)):
+        tiles += [(r, row + q0, min(64, n - q0), L - n + q0) for q0 in range(0, n, 64)]
+        row += n
+    ref = np.concatenate([pm.attention(c["q"][r], c["k"][r], c["v"][r], heads, kv_heads, d, window) for r in range(len(lens))])
+    got = []
+    for blocks in (ops().pair_tiles(tiles, window), ops().pair_tiles(tiles, window, 1)):
+        out = torch.full((row + 1, heads * d), 3.0, device=DEV, dtype=torch.bfloat16)
+        ops().attention_teams(out[:row], c["qcat"], c["kc"], c["vc"], c["table"], t(np.array(blocks, np.int32), torch.int32), heads, kv_heads, d, window, scale)
+        close(out[:row], ref, BF16, "attention in teams")
+        assert (out[row] == 3.0).all()
+        got.append(out)
+    assert torch.equal(*got)
+
+
+def test_attention_in_teams_is_as_near_64_bits_as_the_kernel_it_replaces():
+    """Scores times 1, 3 and 8 (a row's weight on few keys or on many): the distance of either from the plain attention in float64."""
+    heads, kv_heads, d, bs = 14, 2, 64, 16
+    lens, q_lens = [900, 333], [200, 333]
+    tiles = [(0, q0, min(64, 200 - q0), 700 + q0) for q0 in range(0, 200, 64)] + [(1, 200 + q0, min(64, 333 - q0), q0) for q0 in range(0, 333, 64)]
+    blocks = t(np.array(ops().pair_tiles(tiles), np.int32), torch.int32)
+    for times in (1.0, 3.0, 8.0):
+        c = paged_case(np.random.default_rng(37), lens, q_lens, heads, kv_heads, d, bs, torch.bfloat16)
+        scale = float(np.float32(times) / np.sqrt(np.float32(d)))
+        ref = np.concatenate([pm.attention(times * c["q"][r].astype(np.float64), c["k"][r], c["v"][r], heads, kv_heads, d, None) for r in range(2)])
+        off = {}
+        for name, run in (("teams", ops().attention_teams), ("before", ops().attention_prefill)):
+            out = torch.empty(533, heads * d, device=DEV, dtype=torch.bfloat16)
+            run(out, c["qcat"], c["kc"], c["vc"], c["table"], blocks, heads, kv_heads, d, None, scale)
+            off[name] = np.linalg.norm(out.double().cpu().numpy() - ref) / np.linalg.norm(ref)
+        # (either rounds each weight and each result once, to bfloat16, with four running states a row over the same tiles: the same roundings but for sums in another order)
+        assert off["teams"] <= 1.01 * off["before"], (times, off)
+
+
 def test_prefill_attention_far_key():
     rng = np.random.default_rng(29)
     heads, kv_heads, d, bs, L, far = 6, 2, 64, 16, 700, 3
