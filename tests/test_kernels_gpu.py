@@ -194,6 +194,12 @@ def test_norm_behind_a_product_that_adds_to_the_residual_stream(M, N, K):
         o.gemm(torch.empty(M, N, device=DEV, dtype=torch.bfloat16), at, wt, then_norm=(nwt, eps, rows))       # not the residual stream
 
 
+@pytest.mark.parametrize("M,N,K", [(32, 1028, 8192), (65, 2048, 8192), (256, 2052, 8192), (257, 2052, 8192), (33, 4096, 8192), (64, 4100, 4096), (40, 8192, 4096)])
+def test_norm_behind_such_a_product_at_the_edges_of_its_forms(M, N, K):
+    """Widths at which the launch that adds the shares takes other numbers of threads, and rows at which it takes another form: the same values."""
+    test_norm_behind_a_product_that_adds_to_the_residual_stream(M, N, K)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 1152, 896), (8, 896, 4864), (3, 97, 80), (7, 1000, 1544), (5, 130, 6144), (2, 64, 8), (4, 4864, 896), (6, 35, 520)])
 def test_product_for_very_few_rows(M, N, K):
     """The vector-unit product for at most eight rows, every form of it (store with bias, float32 store,
