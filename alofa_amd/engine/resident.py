@@ -1,4 +1,5 @@
-"""Decode steps whose layers run in one launch (csrc/decode_resident.hip): what the launch needs beside the step's own tensors, kept by a step
+"""Decode steps whose layers run in one launch (csrc/decode_resident.hip, and csrc/decode_groups.hip for more
+than 16 rows): what the launch needs beside the step's own tensors, kept by a step
 function: the table of the layers' matrices and caches, an area of memory that the launch's blocks exchange values in, and a word that the
 kernel sets if it gives a wait up."""
 from __future__ import annotations
@@ -155,6 +156,12 @@ class ResidentLayers:
     # wide (24 layers), 15,000 491 / 542, 31,000 668 / 562, 512 wide (16) 344 / 382 and 469 / 398; three key heads, 576 wide (30), 682 / 793 and 919 / 820; rows x key heads of four or five,
     # 31,000 keys: 840 / 846, 299 / 297, 802 / 804, 560 / 573; of eight 924 / 1,022; of sixteen 1,076 / 1,335, 484 / 617. Even at 20,000 to 28,000 below four, at 30,000 from there on.
     MOST_KEYS = ((4, 20000), (16, 28000))
+    # Groups (more than MOST_ROWS rows) deal their blocks to their rows' key heads, a block at least to each. Where a row of more than LONG_KEYS keys is left with one block a key head, the
+    # layer waits for that block while others idle. us a step of 6 layers, kernel by kernel / groups, blocks with keys of 64: four key heads, 33 rows of 16,000 keys (36) 1,017 / 1,111, 48
+    # (48) 1,126 / 1,196, 56 (56) 1,270 / 1,209; 24 of 14,000 beside 24 short ones 906 / 962; 28 beside five, two blocks to each, 926 / 700; three key heads, 48 of 24,000 (36) 1,338 / 1,561,
+    # 40 (30, twice) 1,055 / 971, 64 of 14,000 (48) 1,017 / 1,088. So groups where every long row has two blocks a key head, or where such rows fill thirteen of sixteen blocks (52 rows of
+    # 14,000 with four key heads 1,090 / 1,076). Rows of 4,000 gain 1.08 to 1.24 throughout, of 8,000 0.97 to 1.19.
+    LONG_KEYS, BLOCKS = 7000, 256      # (blocks of a launch)
 
     @classmethod
     def of(cls, model, cache) -> Optional["ResidentLayers"]:
@@ -233,6 +240,12 @@ class ResidentLayers:
         """Whether this step runs in one launch: one new token for each of few requests, and keys that it is the faster one for."""
         if rows > self.most_rows or ctx.max_q_len != 1 or len(ctx.spans) != rows:
             return False
+        if rows > self.MOST_ROWS and ctx.longest > self.LONG_KEYS:
+            groups = 2 if rows <= 2 * self.MOST_ROWS else 4
+            blocks = self.BLOCKS // groups
+            pairs, long = (-(-n // groups) * self.kv_heads for n in (rows, sum(s.pos0 + s.n > self.LONG_KEYS for s in ctx.spans)))
+            if pairs + long > blocks and 16 * long < 13 * blocks:
+                return False
         return ctx.longest <= next((keys for below, keys in self.MOST_KEYS if rows * self.kv_heads < below), ctx.longest)
 
     def gave_up(self) -> bool:

@@ -6,6 +6,7 @@ import threading
 import weakref
 from types import SimpleNamespace
 
+import pytest
 import torch
 
 from alofa_amd.engine.resident import ResidentLayers, _Areas, _Seats
@@ -150,3 +151,16 @@ def test_steps_of_few_rows_over_very_many_keys_are_left_to_the_kernels_one_by_on
     assert takes(5, 3, 28000) and not takes(5, 3, 28001)
     assert takes(8, 2, 1000000) and takes(1, 16, 1000000) and takes(16, 1, 1000000)
     assert not takes(17, 1, 10) and not takes(1, 1, 10, new=2)
+
+
+@pytest.mark.parametrize("kv_heads,long,short,taken", [
+    (4, 33, 0, False), (4, 48, 0, False), (4, 52, 0, True), (4, 64, 0, True), (4, 24, 24, False), (4, 28, 5, True), (4, 0, 64, True),     # 64 blocks a group
+    (3, 40, 0, True), (3, 48, 0, False), (3, 64, 0, False), (3, 28, 20, True), (2, 48, 0, True), (2, 64, 0, True), (1, 64, 0, True),
+    (4, 32, 0, True), (8, 17, 0, False), (8, 28, 0, True), (8, 0, 17, True),     # 128
+    (4, 16, 0, True),     # one group
+])
+def test_groups_where_long_rows_have_two_blocks_a_key_head(kv_heads, long, short, taken):
+    rule = SimpleNamespace(MOST_ROWS=16, most_rows=64, kv_heads=kv_heads, MOST_KEYS=ResidentLayers.MOST_KEYS, LONG_KEYS=ResidentLayers.LONG_KEYS, BLOCKS=ResidentLayers.BLOCKS)
+    keys = [ResidentLayers.LONG_KEYS + 1] * long + [ResidentLayers.LONG_KEYS] * short
+    ctx = SimpleNamespace(max_q_len=1, longest=max(keys), spans=[SimpleNamespace(pos0=n - 1, n=1) for n in keys])
+    assert ResidentLayers.takes(rule, ctx, len(keys)) is taken
