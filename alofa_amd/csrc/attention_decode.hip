@@ -895,8 +895,9 @@ extern "C" int alofa_attention_decode_v(void* out, int64_t out_stride, float* pa
   ALOFA_REQUIRE(tokens > 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0,
                 "attention_decode: tokens=%d heads=%d kv_heads=%d (kv_heads must divide heads)", tokens, heads, kv_heads);
   ALOFA_REQUIRE(d >= 16 && d <= 256 && d % 16 == 0, "attention_decode: head size %d must be 16..256 in steps of 16", d);
-  ALOFA_REQUIRE(block_size >= 4 && (block_size & (block_size - 1)) == 0 && max_blocks > 0 && window >= 0,
-                "attention_decode: block_size=%d must be a power of two, at least 4; max_blocks=%d window=%d", block_size, max_blocks, window);
+  // (a load of values takes eight keys of a channel, which have to lie in one page)
+  ALOFA_REQUIRE(block_size >= 8 && (block_size & (block_size - 1)) == 0 && max_blocks > 0 && window >= 0,
+                "attention_decode: block_size=%d must be a power of two, at least 8; max_blocks=%d window=%d", block_size, max_blocks, window);
   int bs_shift = 0;
   while ((1 << bs_shift) < block_size) ++bs_shift;
   ALOFA_REQUIRE(n_splits >= 1 && n_splits <= kMaxSplits && (n_splits == 1 || partial || hand_over), "attention_decode: n_splits=%d (1..%d) needs scratch when above 1", n_splits, kMaxSplits);
@@ -908,7 +909,7 @@ extern "C" int alofa_attention_decode_v(void* out, int64_t out_stride, float* pa
     counters = workspace().counters;
   }
   ALOFA_REQUIRE(q_stride % 8 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0, "attention_decode: q rows must be 16-byte aligned");
-  ALOFA_REQUIRE(reinterpret_cast<uintptr_t>(k_cache) % 16 == 0 && reinterpret_cast<uintptr_t>(v_cache) % 8 == 0, "attention_decode: caches must be 16-byte aligned");
+  ALOFA_REQUIRE(reinterpret_cast<uintptr_t>(k_cache) % 16 == 0 && reinterpret_cast<uintptr_t>(v_cache) % 8 == 0, "attention_decode: the cache of keys must be 16-byte aligned, that of values 8-byte aligned");
   const MapsForm maps{keep_first, cap, lambda, gain, eps, d_true};
   if (two_maps) {      // heads counts both maps of every head; parts that a second kernel combines leave both maps' sums as they are in out32 ([tokens, heads * d])
     ALOFA_REQUIRE(split && (!cos_t || d % 128 == 0) && !sink && v_head < 0 && value_heads == 0 && heads % (2 * kv_heads) == 0 && block_heads % 2 == 0 && d_true > 0 && d_true <= d,

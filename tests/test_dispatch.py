@@ -3,6 +3,7 @@ a shape, how decode attention shares a context out, how runs of rows are paired 
 import pytest
 
 from alofa_amd import ops
+from alofa_amd.csrc.build import load
 from alofa_amd.errors import AlofaError
 
 
@@ -103,3 +104,13 @@ def test_runs_are_paired_long_with_short():
     assert len(odd) == 2 and odd[1][1] == [0, 0, 0, 0]
     windowed = ops.pair_tiles(runs, window=100)                                   # with a window every run walks two or three tiles
     assert sorted(tuple(r) for b in windowed for r in b) == sorted(runs)
+
+
+@pytest.mark.parametrize("page,taken", [(1, False), (2, False), (4, False), (8, True), (12, False), (16, True)])
+@pytest.mark.parametrize("entry", ["alofa_attention_decode", "alofa_attention_decode_v"])
+def test_decode_attention_refuses_pages_that_a_load_of_its_values_does_not_fit(entry, page, taken):
+    """The entry itself, whoever calls it: eight keys of a channel are one load. (Rows of queries that no load fits either: a check behind that of the pages, so that nothing is launched.)"""
+    q_stride, tail = 4, () if entry.endswith("decode") else (-1, None, 0, 0, 0, None, 16, 0, 0, 0.0, 0.0, 0.0, 0.0, 64)
+    assert ops._answer(entry, None, 128, None, None, q_stride, None, None, None, 8, None, None, None, 1, 2, 1, 64, page, 0, 0.125, 1, None, None, None, 0, *tail, 0) != 0
+    said = load().alofa_last_error().decode()
+    assert ("block_size" not in said and "16-byte aligned" in said) if taken else f"block_size={page} must be a power of two, at least 8" in said
