@@ -48,6 +48,8 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_groups_kernel(ResidentA
   __shared__ __attribute__((aligned(16))) float angles[2][32];
   __shared__ __attribute__((aligned(16))) float hs[MB * 16];     // the block's columns of the stream
   __shared__ int rows_of[MB], parts_of[MB], first_of[MB], order[64], n_rows;
+  static_assert(kLdsOf<decltype(xs), decltype(red), decltype(ssq), decltype(table), decltype(angles), decltype(hs), decltype(rows_of), decltype(parts_of), decltype(first_of), decltype(order),
+                       decltype(n_rows)> <= kResMostLds, "two launches' blocks fit a compute unit");
   bf16_t* qs = reinterpret_cast<bf16_t*>(red + kQsAt);           // B: the turned queries of the key head (rows 0..), behind them the new key and value
   const int b = blockIdx.x;
   int s = b / (8 * G) * 8 + b % 8, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), tid = threadIdx.x, lane = tid % 64, c16 = lane % 16, g = lane / 16;

@@ -24,7 +24,7 @@
 // A place is written again a layer later by a block that has seen all of G's values, which every block leaves after its last read of the layer
 // before: nothing is overwritten that is still waited for.
 //
-// All blocks have to be on the chip at once. A block takes at most half of a compute unit (eight waves of up to 128 registers, under 80 KB of
+// All blocks have to be on the chip at once. A block takes at most half of a compute unit (eight waves of up to 128 registers, at most 80 KB of
 // LDS), so that 256 of them fit beside 256 of another such launch, whatever process it belongs to; kernels that wait for nobody make room by ending.
 // No wait is without end: a wave that has asked kLimit times sets `stop` and `failed`, which end every other wait, and what it waited for is NaN from then on.
 //
@@ -58,6 +58,8 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(Residen
   __shared__ __attribute__((aligned(16))) float angles[2][32];
   __shared__ float hs[4 * MB];                               // the block's columns of the stream
   __shared__ __attribute__((aligned(16))) bf16_t qs[(kResMaxGroup + 2) * 72];      // B: the turned queries of the key head (rows 0..), behind them the new key and value
+  static_assert(kLdsOf<decltype(xs), decltype(red), decltype(norms), decltype(ssq), decltype(table), decltype(angles), decltype(hs), decltype(qs)> <= kResMostLds,
+                "two launches' blocks fit a compute unit");
   // (what follows from these is formed anew in every phase: kept from layer to layer it would take the registers of the weights, and a register that is
   // read back from memory is waited for behind the weights that are on their way)
   int b = blockIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), tid = threadIdx.x, lane = tid % 64, c16 = lane % 16, g = lane / 16;

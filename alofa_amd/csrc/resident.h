@@ -44,6 +44,11 @@ struct LayerWords {
 
 constexpr int kResBlocks = 256, kResThreads = 512, kResWaves = 8;
 constexpr int kResMaxWidth = 1024, kResMaxFF = 6144, kResMaxRows = 16, kResMaxParts = 16, kResShares = 8, kResMaxGroup = 8;
+// A launch waits until all its blocks are on the chip, and two processes may have one each on their way: a block takes at most half of a compute unit's registers (the launch bounds) and LDS.
+// kLdsOf: the bytes of a kernel's __shared__ arrays, all of which are named to it; one that does not fit beside another launch's blocks must not build (its waits would end at their limit).
+constexpr int kResMostLds = 80 * 1024;
+template <typename... Arrays>
+constexpr int kLdsOf = (((static_cast<int>(sizeof(Arrays)) + 15) / 16 * 16) + ...);
 constexpr int kLimit = 4 << 20;      // asks of about a microsecond
 
 // where the values lie in the area, in places of eight bytes (the first 32 hold the step counter and `stop`)
