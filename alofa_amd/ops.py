@@ -1499,7 +1499,7 @@ def recurrence_max_parts(dk: int) -> int:
 
 def linear_recurrence(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Tensor, rows: RowsOfRequests,
                       heads: int, dk: int, dv: int, decay_kind: int, decay: torch.Tensor, tau: float = 1.0, bonus: Optional[torch.Tensor] = None,
-                      q_scale: float = 1.0, k_scale: float = 1.0, before_update: bool = False, finish: Optional[tuple] = None, rope: Optional[tuple] = None) -> int:
+                      q_scale: float = 1.0, k_scale: float = 1.0, before_update: bool = False) -> int:
     """Per request (in its rows' order) and head: S = diag(w_t) S + k_t v_t^T and out_t = S^T q_t, or with
     ``before_update`` out_t = (S + diag(bonus) k_t v_t^T)^T q_t first and the update after it. S float32
     [slots, heads, dk, dv] is read and left in ``state``. q, k [T, heads * dk] and v [T, heads * dv] are rows in one
@@ -1508,11 +1508,7 @@ def linear_recurrence(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: to
     (1 otherwise), and ``headnorm_gate(parts=)`` adds them. The decay w_t: ``DECAY_PER_HEAD`` with ``decay``
     float32 [heads]; ``DECAY_SIGMOID_ROOT`` sigmoid(z)^(1/tau) or ``DECAY_EXP_NEG_EXP`` exp(-exp(z)) with ``decay`` = z
     float32 [T, heads * dk] rows, which a step of many rows overwrites with the decays made of them; ``DECAY_GIVEN``:
-    ``decay`` holds the w_t themselves. ``finish`` = (gate, weight, eps), and ``rope`` = (cos, sin, positions) with it: ``recurrence_step``, what stands around the
-    recurrence of single rows in the same launch."""
-    if finish is not None:
-        recurrence_step(out, q, k, v, finish[0], finish[1], state, rows, heads, dk, dv, finish[2], decay_kind, decay, tau, bonus, q_scale, k_scale, before_update, rope)
-        return 1
+    ``decay`` holds the w_t themselves."""
     _gpu("out", out, torch.float32), _contig("out", out), _gpu("q", q, None, 2), _gpu("k", k, q.dtype, 2), _gpu("v", v, q.dtype, 2)
     _gpu("state", state, torch.float32, 4), _contig("state", state)
     T = q.shape[0]
@@ -1543,8 +1539,8 @@ def linear_recurrence(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: to
 
 
 def recurrence_step_takes(rows: RowsOfRequests, dk: int, dv: int, dtype: torch.dtype, q: torch.Tensor) -> bool:
-    """Whether ``recurrence_step`` takes a step: one row of every request, bfloat16 rows, heads of at most 256 key and value channels, the latter in fours."""
-    return rows.offsets is None and dtype is torch.bfloat16 and q.dtype is torch.bfloat16 and 0 < dk <= 256 and 4 <= dv <= 256 and dv % 4 == 0
+    """Whether ``recurrence_step`` takes a step: one row of every request, bfloat16 rows, heads of at most 256 key and value channels, the latter in fours (the kernel's own rule)."""
+    return rows.offsets is None and dtype is torch.bfloat16 and q.dtype is torch.bfloat16 and bool(_answer("alofa_recurrence_step_takes", _I(dk), _I(dv)))
 
 
 def recurrence_step(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torch.Tensor, weight: Optional[torch.Tensor], state: torch.Tensor, rows: RowsOfRequests,

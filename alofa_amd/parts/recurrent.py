@@ -97,7 +97,7 @@ class RecurrentMixer(Mixer):
         if not ops.recurrence_step_takes(rows, self.dk, self.dv, self.rt.dtype, q):
             return False
         y = ctx.scratch("recurrent_gated", (q.shape[0], self.heads * self.dv), self.rt.dtype)
-        ops.linear_recurrence(y, q, k, v, ctx.state(where), rows, self.heads, self.dk, self.dv, decay_kind, decay, finish=(gate, weight, self.eps), **how)
+        ops.recurrence_step(y, q, k, v, gate, weight, ctx.state(where), rows, self.heads, self.dk, self.dv, self.eps, decay_kind, decay, **how)
         self._project(ctx, y, residual, out)
         return True
 

@@ -1,6 +1,9 @@
 """Host-side choices that shape kernel launches (no GPU needed): which bfloat16 product takes
 a shape, how decode attention shares a context out, how runs of rows are paired into blocks."""
+from types import SimpleNamespace
+
 import pytest
+import torch
 
 from alofa_amd import ops
 from alofa_amd.csrc.build import load
@@ -114,3 +117,14 @@ def test_decode_attention_refuses_pages_that_a_load_of_its_values_does_not_fit(e
     assert ops._answer(entry, None, 128, None, None, q_stride, None, None, None, 8, None, None, None, 1, 2, 1, 64, page, 0, 0.125, 1, None, None, None, 0, *tail, 0) != 0
     said = load().alofa_last_error().decode()
     assert ("block_size" not in said and "16-byte aligned" in said) if taken else f"block_size={page} must be a power of two, at least 8" in said
+
+
+def test_single_rows_of_layers_with_state_in_one_launch():
+    def takes(dk, dv, dtype=torch.bfloat16, q=torch.bfloat16, offsets=None):
+        return ops.recurrence_step_takes(SimpleNamespace(offsets=offsets), dk, dv, dtype, torch.empty(0, dtype=q))
+    assert all(takes(dk, dv) for dk in (1, 63, 256) for dv in (4, 252, 256))
+    assert not any(takes(*sizes) for sizes in ((0, 64), (257, 64), (64, 0), (64, 2), (64, 66), (64, 260)))
+    assert not takes(64, 64, dtype=torch.float32) and not takes(64, 64, q=torch.float32) and not takes(64, 64, offsets=torch.zeros(2, dtype=torch.int32))
+    for how in ("rope", "finish"):      # (the recurrence alone neither turns queries and keys nor norms what it reads out)
+        with pytest.raises(TypeError):
+            ops.linear_recurrence(None, None, None, None, None, None, 1, 64, 64, ops.DECAY_PER_HEAD, None, **{how: (None, None, None)})
