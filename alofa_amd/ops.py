@@ -1017,15 +1017,26 @@ def attention_tall(out, q, k_cache, v_cache, block_table, runs, heads, kv_heads,
           _ptr(runs), _I(runs.shape[0]), _I(heads), _I(kv_heads), _I(d), _I(bs), _I(int(window or 0)), _F(scale), _stream())
 
 
-def attention_teams_pays(heads: int, kv_heads: int, d: int, block_size: int, scale: float, runs: int, window: Optional[int] = None) -> bool:
-    """Whether ``runs`` runs of up to 64 rows go to the kernel of heads of 64 whose waves own 32 rows: always where the other kernel's heads have blocks of their own (14/2 heads, 30
-    launches of portions from 5 to 8,192 rows, us, the other / this: 0.99 to 1.37 times as fast, 40 portions of 40 rows 20.7 / 20.9), and without a window also where a group's heads share its
-    tiles with 16 rows a wave (two prompts of 2,048 47.4 / 42.1, one of 4,096 85.6 / 63.6). Where they share them with 32 rows a wave a tile serves 224 (row, head) pairs instead of 64:
-    four of 2,048 68 / 80, one of 8,192 even; and with a window (four of 1,024 on 500 keys, window 300) 25.2 / 34.6."""
+def attention_teams_pays(heads: int, kv_heads: int, d: int, block_size: int, scale: float, portions: list, window: Optional[int] = None) -> bool:
+    """Whether ``portions``, (rows brought, keys that the last of them sees) each, go to the kernel of heads of 64 whose waves own 32 rows. How many times as fast it is as the other one,
+    launches of portions of 5 to 8,192 rows on 0 to 4,000 keys, twelve head counts, pages of 16 to 64:
+    Where the other kernel's heads have blocks of their own: 0.94 to 1.4, 1.13 on average, and with a window of 384 keys or more 0.92 to 1.34, 1.04 to 1.12. A smaller window leaves a run few rounds of
+    tiles: with a block a compute unit or fewer still 0.94 to 1.27, 1.07; with more blocks, whose beginnings and ends are then most of it, 0.89 to 1.2, below 1 for one launch in three: not those.
+    Where six or seven heads of a group share that kernel's tiles with 16 rows a wave, without a window: whole runs that see sixteen tiles of 64 keys or more on average, 1.04 to 2.5 (14/2 heads, two prompts of
+    2,048 47.4 / 42.1 us, one of 4,096 85.6 / 63.6). A block there that has no rows of its sixteen ends at once and a tile serves all heads, while a block here takes as long for five rows as for 64 and
+    3 us beside its tiles: 14/2 heads, 64 portions of 33 rows on 200 keys 17 / 23, launches of partly filled runs or few keys 0.3 to 1.7. Eight heads share at a lower price, 0.84 to 1.15 for whole runs over
+    many keys, 32/2 heads, 40 portions of 40 rows 9.7 / 29.6. Where they share them with 32 rows a wave a tile serves 224 (row, head) pairs instead of 64: four of 2,048 68 / 80, one of 8,192
+    even; and with a window (four of 1,024 on 500 keys, window 300) 25.2 / 34.6."""
     if d != 64 or block_size < 16 or not scale > 0:
         return False
+    runs = sum(-(-n // 64) for n, _ in portions)
     share = prefill_share(heads, kv_heads, d, runs)
-    return not share or (not window and prefill_rows(heads, kv_heads, d, share, runs) == 16)
+    if not share:
+        return not window or window >= 384 or runs * heads <= compute_units()
+    if window or share > 7 or prefill_rows(heads, kv_heads, d, share, runs) != 16:
+        return False
+    tiles = sum((keys - n + min(q0 + 64, n) - 1) // 64 + 1 for n, keys in portions for q0 in range(0, n, 64))
+    return sum(n for n, _ in portions) >= 60 * runs and tiles >= 16 * runs
 
 
 def attention_teams(out, q, k_cache, v_cache, block_table, tiles, heads, kv_heads, d, window, scale) -> None:

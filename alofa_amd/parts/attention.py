@@ -56,7 +56,7 @@ class RowPlan:
         """Whether the runs go to the kernel of heads of 64 whose waves own 32 rows."""
         key = (heads, kv_heads, d, block_size, scale, window)
         if key not in self._teams:
-            self._teams[key] = ops.attention_teams_pays(*key[:-1], len(self.long_runs), window)
+            self._teams[key] = ops.attention_teams_pays(*key[:-1], [(s.n, s.pos0 + s.n) for s in self.spans if s.n > SHORT], window)
         return self._teams[key]
 
     def tall_runs(self):

@@ -128,3 +128,22 @@ def test_single_rows_of_layers_with_state_in_one_launch():
     for how in ("rope", "finish"):      # (the recurrence alone neither turns queries and keys nor norms what it reads out)
         with pytest.raises(TypeError):
             ops.linear_recurrence(None, None, None, None, None, None, 1, 64, 64, ops.DECAY_PER_HEAD, None, **{how: (None, None, None)})
+
+
+def test_runs_of_heads_of_64_that_go_to_teams(monkeypatch):
+    monkeypatch.setattr(ops, "_compute_units", 256)
+
+    def teams(heads, kv_heads, *portions, window=None, page=16, d=64, scale=0.125):
+        return ops.attention_teams_pays(heads, kv_heads, d, page, scale, list(portions), window)
+    prompt = (2048, 2048)
+    assert teams(14, 2, prompt) and teams(14, 2, (5, 5)) and teams(8, 8, *[prompt] * 8) and teams(16, 4, *[(40, 40)] * 40)       # heads with blocks of their own
+    assert teams(16, 4, *[(64, 500)] * 16, window=100) and not teams(16, 4, *[(64, 500)] * 17, window=383) and teams(16, 4, *[(64, 500)] * 17, window=384)
+    assert not teams(14, 2, prompt, page=8) and not teams(14, 2, prompt, d=128) and not teams(14, 2, prompt, scale=0.0)
+    # heads that share tiles, 16 rows a wave: whole runs over many keys
+    assert ops.prefill_share(14, 2, 64, 64) == 7 and ops.prefill_rows(14, 2, 64, 7, 64) == 16 and ops.prefill_rows(14, 2, 64, 7, 96) == 32
+    assert teams(14, 2, prompt, prompt) and teams(14, 2, (4096, 4096)) and not teams(14, 2, prompt, prompt, window=4096)
+    assert teams(14, 2, *[(64, 64 * 16)] * 64) and not teams(14, 2, *[(64, 64 * 15)] * 64)
+    assert teams(14, 2, *[(60, 60 + 64 * 15)] * 64) and not teams(14, 2, *[(60, 60 + 64 * 15)] * 63, (59, 59 + 64 * 15))
+    assert ops.prefill_share(16, 2, 64, 64) == 8 and not teams(16, 2, prompt, prompt) and not teams(32, 2, *[prompt] * 2)
+    assert not teams(32, 2, *[(40, 40)] * 40) and not teams(14, 2, *[(33, 233)] * 64) and not teams(12, 2, *[(5, 4005)] * 64) and not teams(12, 2, *[(512, 512)] * 8)
+    assert not teams(14, 2, *[prompt] * 3)                                         # ... with 32
