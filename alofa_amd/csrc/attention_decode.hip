@@ -151,10 +151,11 @@ __device__ __forceinline__ Pair8 rotate8(uint4 lo, uint4 hi, float4 c_lo, float4
 // pieces that a compute unit's loads are bound by) and the new token's key and value in LDS (no register of the kernel that turns it is kept in memory any more), us, before / now: 28/4 heads of 128,
 // 32 tokens of 128 to 1,024 keys 19.3 / 18.4, 64 of 128 to 2,048 37.7 / 35.8, in pages of 64 tokens 61.2 / 47.4; 40/8 heads, 16 of 1,000 to 4,000 45.3 / 42.4; 14/2 heads of 64, 64 of 128 to 2,048
 // 14.3 / 14.0, in pages of 64 18.0 / 15.8. The loads alone, with the new token in registers: 22.5, 50.1, 57.2 and 54.9 (heads of 128: eleven registers kept in memory, read back behind the keys on their way).
+// Heads of 32: two blocks (128 registers; left to itself the compiler takes 132): 8/8 heads, 64 tokens of 60 to 600 keys 11.5 / 10.1 us, in pages of 64 12.7 / 10.5, behind a window of 100 7.5 / 6.2.
 // DT = d / 16; NW: waves per block. blockIdx.y = key head * chunks + chunk of up to `block_heads` (<= 16) heads of its group.
 // kSplit: a weight enters the second product as two bfloat16 numbers, its rounding and what the rounding took away: sixteen bits of every weight count.
 template <int DT, int NW, bool kRope, bool kSplit = false, bool kMaps = false>
-__global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1) attention_decode_kernel(
+__global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : DT == 2 && !kSplit ? 4 : 1) attention_decode_kernel(
     bf16_t* __restrict__ out, int64_t out_stride, float* __restrict__ partial, const bf16_t* __restrict__ q,
     int64_t q_stride, bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache,
     const int32_t* __restrict__ block_table, int max_blocks, const int32_t* __restrict__ req_of_token,
@@ -230,7 +231,9 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
   }
 
   // the new token's key (this lane's channel slices, rotated) and value (channels 16 nt + c16), kRope only; from the rotation on they lie in LDS, in the room that the wave's state takes
-  // at the end (held in registers they are 24 at a head size of 128, and what does not fit is read back from memory behind the keys on their way)
+  // at the end (held in registers they are 24 at a head size of 128, and what does not fit is read back from memory behind the keys on their way; at 192 all of it fits, and the way through LDS
+  // would cost more than it saves: 8/8 heads, us, in LDS / in registers, one token of 700 keys 10.7 / 10.3, eight behind a window of 100 9.6 / 9.1)
+  constexpr bool kFresh = kRope && DT != 12;
   bf16_t* fresh = reinterpret_cast<bf16_t*>(state[threadIdx.x / 64]);
   uint4 new_k[DS];
   uint32_t new_v[DT];
@@ -343,13 +346,14 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt) {
       s[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
-      // (kRope: the new token's key is not in the cache yet: its row of the last tile comes from the registers)
+      // (kRope: the new token's key is not in the cache yet: its row of the last tile is put in here)
       const bool new_row = last_here && tile + k_tile == last && k_row + 4 * kt == (p & 15);
 #pragma unroll
       for (int ds = 0; ds < DS; ++ds) {
         uint4 kf = st.k[kt][ds];
         if (last_here) {      // (word by word: a choice between two whole operands would be made through memory)
-          const uint4 nk = *reinterpret_cast<const uint4*>(fresh + ds * 32 + g * 8);
+          uint4 nk = new_k[ds];
+          if constexpr (kFresh) nk = *reinterpret_cast<const uint4*>(fresh + ds * 32 + g * 8);
           kf.x = new_row ? nk.x : kf.x;
           kf.y = new_row ? nk.y : kf.y;
           kf.z = new_row ? nk.z : kf.z;
@@ -416,7 +420,8 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
       uint32_t vw[4] = {st.v[nt].x & shown[0], st.v[nt].y & shown[1], st.v[nt].z & shown[2], st.v[nt].w & shown[3]};
       if (last_here) {
         // the new token's value takes its place among this lane's eight keys
-        const uint32_t nv = fresh[d + nt * 16 + c16];
+        uint32_t nv = new_v[nt];
+        if constexpr (kFresh) nv = fresh[d + nt * 16 + c16];
 #pragma unroll
         for (int w2 = 0; w2 < 4; ++w2) {
           const bool hit = tile + v_tile == last && v_row == (p & 8) && (p & 7) >> 1 == w2;
@@ -455,15 +460,17 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
       new_k[a] = rk.lo;
       new_k[b] = rk.hi;
     }
-    if (c16 == 0) {
+    if constexpr (kFresh) {
+      if (c16 == 0) {
 #pragma unroll
-      for (int ds = 0; ds < DS; ++ds) *reinterpret_cast<uint4*>(fresh + ds * 32 + g * 8) = new_k[ds];
-    }
-    if (g == 0) {
+        for (int ds = 0; ds < DS; ++ds) *reinterpret_cast<uint4*>(fresh + ds * 32 + g * 8) = new_k[ds];
+      }
+      if (g == 0) {
 #pragma unroll
-      for (int nt = 0; nt < DT; ++nt) fresh[d + nt * 16 + c16] = static_cast<bf16_t>(new_v[nt]);
+        for (int nt = 0; nt < DT; ++nt) fresh[d + nt * 16 + c16] = static_cast<bf16_t>(new_v[nt]);
+      }
+      wave_lds_sync();
     }
-    wave_lds_sync();
     // the wave that owns the last tile of keys (in the first chunk of heads) writes the token's cache slot
     if (h0 == 0 && tile_begin <= last && last < tile_end) {
       const int64_t blk = new_slot >> bs_shift, off = new_slot & bs_mask;
@@ -507,7 +514,7 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : 1)
   }
   l = rows_sum(l);
 
-  if constexpr (kRope) wave_lds_sync();      // (the new token's key and value have been read)
+  if constexpr (kFresh) wave_lds_sync();      // (the new token's key and value have been read)
   // the wave's state: head c16; this lane holds channels 16 nt + 4 g + r
   {
     float* mine = state[wave][c16];
