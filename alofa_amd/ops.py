@@ -1554,6 +1554,13 @@ def recurrence_step_takes(rows: RowsOfRequests, dk: int, dv: int, dtype: torch.d
     return rows.offsets is None and dtype is torch.bfloat16 and q.dtype is torch.bfloat16 and bool(_answer("alofa_recurrence_step_takes", _I(dk), _I(dv)))
 
 
+def recurrence_step_pays(requests: int, heads: int, dk: int, dv: int, turned: bool) -> bool:
+    """Whether ``recurrence_step`` is the faster way for a step that it takes. It reads and writes a head's state, up to 256 KB, by one block, the recurrence alone deals the columns out over several: where
+    that is most of the work, a few (request, head) pairs of the widest heads without a rotation, whose launch would be saved too. Times as fast, pairs of 256 x 256: one 0.85 to 0.92, four 0.90 to 0.94, six 0.97 to
+    1.00, sixteen 1.02, 64 1.4; of 256 x 192: one 0.96, five 0.97, six 1.02; of 224 x 224 and 192 x 256 from 1.01, of 128 x 128 from 1.6, of 64 x 64 from 1.95 on."""
+    return turned or requests * heads > 6 or dk <= 224 or dv < 192
+
+
 def recurrence_step(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torch.Tensor, weight: Optional[torch.Tensor], state: torch.Tensor, rows: RowsOfRequests,
                     heads: int, dk: int, dv: int, eps: float, decay_kind: int, decay: torch.Tensor, tau: float = 1.0, bonus: Optional[torch.Tensor] = None, q_scale: float = 1.0,
                     k_scale: float = 1.0, before_update: bool = False, rope: Optional[tuple] = None) -> None:

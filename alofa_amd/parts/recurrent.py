@@ -92,9 +92,9 @@ class RecurrentMixer(Mixer):
             ops.gemm(residual, y, self.w_o, add_to_out=True, exact=self.rt.exact, scratch=ctx.scratch)
 
     def _single_step(self, ctx, where, q, k, v, gate, weight, residual, out, decay_kind, decay, **how) -> bool:
-        """Where every request brings one row: the recurrence, the head norm and the gate in one launch, and the output projection. False (and nothing done) where it is no such step."""
+        """Where every request brings one row: the recurrence, the head norm and the gate in one launch, and the output projection. False (and nothing done) where it is no such step, or one that is slower so."""
         rows = rows_of_requests(ctx)
-        if not ops.recurrence_step_takes(rows, self.dk, self.dv, self.rt.dtype, q):
+        if not ops.recurrence_step_takes(rows, self.dk, self.dv, self.rt.dtype, q) or not ops.recurrence_step_pays(rows.rows, self.heads, self.dk, self.dv, how.get("rope") is not None):
             return False
         y = ctx.scratch("recurrent_gated", (q.shape[0], self.heads * self.dv), self.rt.dtype)
         ops.recurrence_step(y, q, k, v, gate, weight, ctx.state(where), rows, self.heads, self.dk, self.dv, self.eps, decay_kind, decay, **how)

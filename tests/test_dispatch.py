@@ -147,3 +147,9 @@ def test_runs_of_heads_of_64_that_go_to_teams(monkeypatch):
     assert ops.prefill_share(16, 2, 64, 64) == 8 and not teams(16, 2, prompt, prompt) and not teams(32, 2, *[prompt] * 2)
     assert not teams(32, 2, *[(40, 40)] * 40) and not teams(14, 2, *[(33, 233)] * 64) and not teams(12, 2, *[(5, 4005)] * 64) and not teams(12, 2, *[(512, 512)] * 8)
     assert not teams(14, 2, *[prompt] * 3)                                         # ... with 32
+
+
+def test_few_wide_heads_with_state_go_launch_by_launch():
+    pays = ops.recurrence_step_pays
+    assert not pays(1, 1, 256, 256, False) and not pays(2, 3, 225, 192, False) and pays(1, 7, 256, 256, False) and pays(7, 1, 256, 256, False)
+    assert pays(1, 1, 256, 256, True) and pays(1, 1, 224, 256, False) and pays(1, 1, 256, 188, False) and pays(4, 16, 64, 64, False)
