@@ -10,12 +10,12 @@ pytestmark = pytest.mark.gpu
 VOCAB, LAYERS = 512, 3
 
 
-def model(width, heads, kv_heads, ff, dtype, layers=LAYERS, window=None, device="cuda:0"):
+def model(width, heads, kv_heads, ff, dtype, layers=LAYERS, window=None, device="cuda:0", positions=4096):
     from alofa_amd.config import config_from_dict
     from alofa_amd.model import Model, runtime
     config = config_from_dict({"architectures": ["Qwen2ForCausalLM"], "model_type": "qwen2", "num_hidden_layers": layers, "hidden_size": width, "num_attention_heads": heads,
                                "num_key_value_heads": kv_heads, "head_dim": width // heads, "intermediate_size": ff, "vocab_size": VOCAB, "rope_theta": 10000.0, "rms_norm_eps": 1e-6,
-                               "tie_word_embeddings": True, "use_sliding_window": window is not None, "max_position_embeddings": 4096,
+                               "tie_word_embeddings": True, "use_sliding_window": window is not None, "max_position_embeddings": positions,
                                **({"sliding_window": window, "max_window_layers": 0} if window else {})})
     gen = torch.Generator(device="cuda").manual_seed(7)
 
@@ -45,8 +45,8 @@ def stand(eng, lengths, seed):
     rng = np.random.default_rng(seed)
     for i, n in enumerate(lengths):
         eng.cache.admit(i)
-        if n:
-            eng.step_fn.run([StepEntry(i, rng.integers(0, VOCAB, n).tolist())])
+        for at in range(0, n, 4096):      # (no more than a step's tokens at once)
+            eng.step_fn.run([StepEntry(i, rng.integers(0, VOCAB, min(n - at, 4096)).tolist())])
 
 
 def decode(eng, tokens):
@@ -539,13 +539,27 @@ GROUP_SHAPES = [(256, 4, 1, 512), (320, 5, 5, 768), (576, 9, 3, 1536), (896, 14,
 @pytest.mark.parametrize("page", [16, 64])
 @pytest.mark.parametrize("rows", [17, 31, 32, 33, 50, 64])
 @pytest.mark.parametrize("shape", GROUP_SHAPES)
-def test_groups_are_as_near_the_32_bit_path_as_the_kernels_they_replace(shape, rows, page):
+def test_groups_are_as_near_the_32_bit_path_as_the_kernels_they_replace(shape, rows, page, monkeypatch):
     lengths = (CONTEXTS * 4)[rows % 5:][:rows] + [33] * (rows - len((CONTEXTS * 4)[rows % 5:][:rows]))
+    groups_beside_the_32_bit_path(shape, lengths, page, monkeypatch)
+
+
+@pytest.mark.parametrize("rows", [17, 33])
+@pytest.mark.parametrize("shape", [(256, 4, 1, 512), (512, 8, 2, 1024)])
+def test_a_row_of_more_keys_than_its_parts_are_for_beside_short_ones(shape, rows, monkeypatch):
+    """The most parts that a row and key head has, sixteen, each of more tiles of keys than the group's other blocks, and all rounds of the launch's sums over parts."""
+    groups_beside_the_32_bit_path(shape, [40 + 13 * i for i in range(rows // 2)] + [6100] + [15 + i for i in range(rows - rows // 2 - 1)], 16, monkeypatch)
+
+
+def groups_beside_the_32_bit_path(shape, lengths, page, monkeypatch):
+    from alofa_amd import ops
+    rows, launches, one_launch = len(lengths), [], ops.decode_resident
+    monkeypatch.setattr(ops, "decode_resident", lambda hidden, *a, **how: (launches.append(hidden.shape[0]), one_launch(hidden, *a, **how))[1])
     tokens = np.random.default_rng(rows).integers(0, VOCAB, (2, rows))
     got = {}
     for how in ("float32", "one by one", "one launch", "one launch, captured"):
         dtype = "float32" if how == "float32" else "bfloat16"
-        eng = engine(model(*shape, dtype, layers=2), rows, max(lengths) + 4, dtype, page)
+        eng = engine(model(*shape, dtype, layers=2, positions=8192), rows, max(lengths) + 4, dtype, page)
         fn = eng.step_fn
         if how.startswith("one launch"):
             assert fn.resident.most_rows == (32 if shape[2] > 4 else 64)
@@ -553,7 +567,12 @@ def test_groups_are_as_near_the_32_bit_path_as_the_kernels_they_replace(shape, r
             fn.resident = None
         fn.use_graphs = how.endswith("captured")
         stand(eng, lengths, 1)
+        launches.clear()
         got[how] = decode(eng, tokens)
+        # (captured: a step that replays no graph launches once for its results and once for the graph)
+        steps = 2 * (len(tokens) - fn.graph_replays) if how.endswith("captured") else len(tokens)
+        # (five key heads: 32 rows at most, and kernel by kernel beyond)
+        assert launches == ([rows] * steps if how.startswith("one launch") and rows <= fn.resident.most_rows else []), (how, launches)
     for step in range(len(tokens)):
         exact = got["float32"][step]
         # (per row: a row that took another's place would hide among so many; the spread of the norm of 512 logits' roundings, as above, is less than a third of it)
