@@ -18,6 +18,10 @@
 //   * The rows are dealt to the groups by length (the longest to one after the other, then back), and a group's blocks to its rows' keys in proportion to their number, so that groups and
 //     blocks end at about the same time whatever the lengths.
 //   * Several output tiles a wave and K over four waves instead of eight: gate's tiles are four waves', up's the other four's.
+//   * Phase B is decode_resident.hip's with values by sixteen bytes: masks, the new token's place and the states' end are the same in both.
+//
+// The compiler keeps two registers of a lane in memory with two groups and three with four (12 and 16 bytes; decode_resident.hip has none, whose comment says what one costs there; here it was not
+// measured apart). A block's LDS, 64,580 and 80,964 bytes, leaves room for another launch's block in the compute unit (kLdsOf).
 #include "resident.h"
 
 namespace alofa {
@@ -97,7 +101,7 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_groups_kernel(ResidentA
     quota = fit == 0 || quota > all ? all : quota;
     quota = quota < 2 * kResWaves ? 2 * kResWaves : quota;      // (a part with less than a step for every wave saves nothing)
     int parts = (tiles + quota - 1) / quota;
-    parts = parts < kResMaxParts ? parts : kResMaxParts;
+    parts = parts < kResMaxParts ? parts : kResMaxParts;      // (such a row's parts are longer than the quota, and what the phase waits for: blocks that it leaves would shorten others' parts only)
     int first = 0;
     for (int k = 0; k < MB; ++k) {
       const int p = __builtin_amdgcn_readlane(parts, k);

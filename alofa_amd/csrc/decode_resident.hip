@@ -40,6 +40,7 @@
 
 namespace alofa {
 
+// MB: rows computed (1, 2, 4, 8 or 16; M of them count)
 template <int MB>
 __global__ void __launch_bounds__(kResThreads, 4) decode_resident_kernel(ResidentArgs a) {
   constexpr int d = 64;

@@ -3,6 +3,8 @@
 //
 // Launch by launch these were three, which hand a few hundred numbers on: rotation 2.4 to 4.4 us, the recurrence 6.2 to 8.8 (made for many rows: operands by way of LDS in chunks, read-outs in
 // parts), norm and gate 2.2 to 4 (4 requests, 16 heads of 64 x 64 in a captured step). What the work cannot do without is the state, read and written once: 16 KB a head.
+// 1 to 64 requests of 1 to 32 heads, 1.01 to 2.2 times as fast, but a few (request, head) pairs of the widest heads, whose state one block reads and writes here: those go launch by launch
+// (recurrence_step_pays in ops.py has the figures).
 // A block takes a head of a request. The state's loads set out first (a thread has four neighbouring columns of every so-manieth row, 16 bytes a load), the row's operands are made meanwhile, each
 // once, in LDS; the read-outs' shares meet in LDS in row order. Read-outs stay float up to the norm's end, as they are between the launches.
 #include "common.h"

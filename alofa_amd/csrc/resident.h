@@ -128,8 +128,6 @@ struct Wait {      // of one wave: the area as a buffer resource (reads past the
   }
 };
 
-// MB: rows computed (1, 2, 4, 8 or 16; M of them count)
-
 // (decode_groups.hip) more than sixteen rows
 int launch_groups(const ResidentArgs& a, hipStream_t stream);
 

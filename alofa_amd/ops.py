@@ -764,7 +764,7 @@ def attention_decode(out, q, k_cache, v_cache, block_table, req_of_token, positi
     With ``rope`` = (cos, sin, slots) the rows of ``q`` are the fused projection's
     [queries | keys | values] of ONE new token per request, not yet rotated: the
     kernel rotates queries and the new key itself, uses the new key and value from
-    registers and writes them to the token's cache slot (``can_fuse_rope_into_decode``).
+    the rows and writes them to the token's cache slot (``can_fuse_rope_into_decode``).
     ``n_splits`` (default ``decode_splits``): blocks that share the keys of a (token, key head);
     ``hand_over`` (default ``decode_hand_over``): the last of them to arrive combines their states,
     else the states go to ``scratch`` and a second kernel combines them.
