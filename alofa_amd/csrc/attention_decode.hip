@@ -230,10 +230,10 @@ __global__ void __launch_bounds__(64 * NW, DT == 8 && !(kMaps && kRope) ? 2 : DT
     qf[ds] = __builtin_bit_cast(bf16x8, v);
   }
 
-  // the new token's key (this lane's channel slices, rotated) and value (channels 16 nt + c16), kRope only; from the rotation on they lie in LDS, in the room that the wave's state takes
-  // at the end (held in registers they are 24 at a head size of 128, and what does not fit is read back from memory behind the keys on their way; at 192 all of it fits, and the way through LDS
-  // would cost more than it saves: 8/8 heads, us, in LDS / in registers, one token of 700 keys 10.7 / 10.3, eight behind a window of 100 9.6 / 9.1)
-  constexpr bool kFresh = kRope && DT != 12;
+  // the new token's key (this lane's channel slices, rotated) and value (channels 16 nt + c16), kRope only. Where not all registers would fit (24 of them at a head size of 128; what does not fit is read
+  // back from memory behind the keys on their way) they lie in LDS from the rotation on, in the room that the wave's state takes at the end. Where all fit, the way through LDS costs more than it saves: us, in
+  // LDS / in registers, one token of 700 keys, 8/8 heads of 64 7.9 / 7.7, of 192 10.7 / 10.3, of two maps of 64 9.8 / 9.2.
+  constexpr bool kFresh = kRope && (DT == 16 || (DT == 8 && !kMaps));
   bf16_t* fresh = reinterpret_cast<bf16_t*>(state[threadIdx.x / 64]);
   uint4 new_k[DS];
   uint32_t new_v[DT];

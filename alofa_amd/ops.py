@@ -2584,7 +2584,7 @@ def maps_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cac
     share the keys and values a block reads. ``req_of_token`` None: token i is the one token of request i. ``scratch`` and ``sums`` (float32 [T, 2 heads * d]): needed
     where ``maps_decode_plan`` asks for floats of scratch (a second kernel then combines the parts and ``combine_maps`` ends the heads). ``plan``: that
     function's answer, if another is wanted. With ``rope`` = (cos, sin, slots) the rows of ``q`` are the projection's [queries | keys | values] of one new token per request, not
-    yet turned: the kernel turns queries and the new key itself, uses the new key and value from registers and writes them to the token's cache slot
+    yet turned: the kernel turns queries and the new key itself, uses the new key and value from the rows and writes them to the token's cache slot
     (``can_turn_in_maps_decode``)."""
     T, bs = _maps_operands(out, q, k_cache, v_cache, block_table, heads, kv_heads, d, window, keep_first, softcap, end)
     _gpu("positions", positions, torch.int32, 1), _contig("positions", positions)
