@@ -551,10 +551,16 @@ def test_a_row_of_more_keys_than_its_parts_are_for_beside_short_ones(shape, rows
     groups_beside_the_32_bit_path(shape, [40 + 13 * i for i in range(rows // 2)] + [6100] + [15 + i for i in range(rows - rows // 2 - 1)], 16, monkeypatch)
 
 
-def groups_beside_the_32_bit_path(shape, lengths, page, monkeypatch):
+def counted(monkeypatch) -> list:
+    """The rows of every launch from here on."""
     from alofa_amd import ops
-    rows, launches, one_launch = len(lengths), [], ops.decode_resident
+    launches, one_launch = [], ops.decode_resident
     monkeypatch.setattr(ops, "decode_resident", lambda hidden, *a, **how: (launches.append(hidden.shape[0]), one_launch(hidden, *a, **how))[1])
+    return launches
+
+
+def groups_beside_the_32_bit_path(shape, lengths, page, monkeypatch):
+    rows, launches = len(lengths), counted(monkeypatch)
     tokens = np.random.default_rng(rows).integers(0, VOCAB, (2, rows))
     got = {}
     for how in ("float32", "one by one", "one launch", "one launch, captured"):
@@ -617,7 +623,8 @@ def test_no_number_of_a_group_comes_from_a_wait_that_was_given_up(shape, rows):
 
 
 @pytest.mark.parametrize("name", ["k", "v"])
-def test_a_cached_key_or_value_that_is_no_number_reaches_its_row_alone_in_a_group(name):
+def test_a_cached_key_or_value_that_is_no_number_reaches_its_row_alone_in_a_group(name, monkeypatch):
+    launches = counted(monkeypatch)
     lengths, page = [300, 40, 600] + [25 + i for i in range(17)], 16
     tokens = [list(range(5, 25))]
     m = model(896, 14, 2, 4864, "bfloat16")
@@ -633,15 +640,17 @@ def test_a_cached_key_or_value_that_is_no_number_reaches_its_row_alone_in_a_grou
         (t[block, 1, at % page] if name == "k" else t[block, 1, :, at % page]).fill_(float("nan"))
         got = decode(eng, tokens)[0]
         assert torch.isnan(got[2]).all() and torch.equal(got[others], clean[others]), at
+    assert set(launches) == {20}
 
 
-def test_steps_of_few_and_of_many_rows_in_turn():
+def test_steps_of_few_and_of_many_rows_in_turn(monkeypatch):
     """One step function whose steps have 20, 3, 40 and 20 rows: the groups' counters go on apart from one another."""
     m = model(896, 14, 2, 4864, "bfloat16", layers=2)
     rng = np.random.default_rng(5)
     lengths = [30 + 3 * i for i in range(40)]
     counts = [20, 3, 40, 20, 3, 40, 40]
     tokens = [rng.integers(0, VOCAB, n).tolist() for n in counts]
+    launches = counted(monkeypatch)
 
     def run(one_launch, graphs):
         eng = engine(m, 40, 300, "bfloat16")
@@ -650,6 +659,10 @@ def test_steps_of_few_and_of_many_rows_in_turn():
         eng.step_fn.use_graphs = graphs
         stand(eng, lengths, 3)
         return [eng.step_fn.run([StepEntry(i, [t], [0]) for i, t in enumerate(ts)]).double().cpu() for ts in tokens]
-    want, got, captured = run(False, False), run(True, False), run(True, True)
+    want = run(False, False)
+    assert not launches
+    got = run(True, False)
+    assert launches == counts
+    captured = run(True, True)
     for a, b, c in zip(want, got, captured):
         assert ((a - b).norm() / a.norm()).item() < 0.02 and torch.equal(b, c)      # (two bfloat16 roundings of two layers: some 0.003 each)
