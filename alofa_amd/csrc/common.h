@@ -35,6 +35,7 @@ __device__ __forceinline__ uint32_t pack_bf16x2_rest(float a, float b, uint32_t 
 }
 
 __device__ __forceinline__ bf16_t f32_to_bf16(float f) { return static_cast<bf16_t>(pack_bf16x2(f, 0.f) & 0xffffu); }
+__device__ __forceinline__ float round_bf16(float f) { return bf16_to_f32(f32_to_bf16(f)); }
 
 template <typename T> __device__ __forceinline__ float load_f32(const T* p);
 template <> __device__ __forceinline__ float load_f32<float>(const float* p) { return *p; }
@@ -70,6 +71,17 @@ __device__ __forceinline__ double gate_of(double z, bool gelu) {
 }
 __device__ __forceinline__ float gate_of(float z, bool gelu) {
   return z / (1.f + expf(-(gelu ? 1.5957691216057308f * (z + 0.044715f * z * z * z) : z)));
+}
+
+// ---- activations of feed-forwards with one matrix in front --------------------
+// kind 0: xIELU with a = softplus(p) and b = 1/2 + softplus(q) given: z > 0: a z^2 + z/2; else b (exp(z) - 1 - z) + z/2.
+// kind 1: tanh. kind 2: silu, z sigmoid(z). kind 3: the tanh form of gelu, z/2 (1 + tanh(sqrt(2/pi) (z + 0.044715 z^3))).
+template <typename Acc>
+__device__ __forceinline__ Acc activation_of(Acc z, int kind, Acc a, Acc b) {
+  if (kind == 0) return z > 0 ? a * z * z + z / 2 : b * (expm1(z) - z) + z / 2;
+  if (kind == 1) return tanh(z);
+  if (kind == 2) return z / (static_cast<Acc>(1) + exp(-z));
+  return z / 2 * (static_cast<Acc>(1) + tanh(static_cast<Acc>(0.7978845608028654) * (z + static_cast<Acc>(0.044715) * z * z * z)));
 }
 
 // ---- reductions ------------------------------------------------------------

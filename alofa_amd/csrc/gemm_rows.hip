@@ -30,7 +30,22 @@ namespace alofa {
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-enum RowsEpilogue : int { kRwStore = 0, kRwResidual = 1, kRwSwiglu = 2, kRwGeglu = 4 };
+enum RowsEpilogue : int { kRwStore = 0, kRwResidual = 1, kRwSwiglu = 2, kRwGeglu = 4, kRwActivated = 5, kRwDepth = 6 };
+
+// What kRwActivated does to an output once it is rounded to bfloat16 (as the activation's own launch reads it: the same bits), activation_of in common.h.
+struct RowsActivation {
+  int kind;      // -1: none
+  float a, b;
+};
+
+// kRwDepth: behind the sum into the residual stream the average over depth (depth_average_kernel in pointwise.hip: the same sums in the same order): the new value goes to level n - 1 of the stack
+// [levels][level_stride], and the stream receives the sum of w[j] times level j. An output's levels are read by the thread that finishes it, with the rest of its loads.
+struct RowsDepth {
+  float* stack;
+  int64_t level_stride, ld;
+  const float* w;
+  int n;
+};
 
 constexpr int kRowsMaxWaves = 12;     // runs of 512 along K, one per wave
 constexpr int kRowsMaxK = kRowsMaxWaves * 512;
@@ -95,19 +110,47 @@ __device__ __forceinline__ void lanes_sum(float (&v)[n], int lane) {
 }
 constexpr int log2_of(int n) { return n <= 1 ? 0 : 1 + log2_of(n / 2); }
 
+// The levels of an output's average over depth (kOn: kRwDepth): asked for with the thread's other loads, eight of them (a stack of fewer: its last one again), and the weights with them;
+// more are read at the end.
+template <bool kOn>
+struct DepthOf {
+  static constexpr int kHeld = 8;
+  float held[kOn ? kHeld : 1], weight[kOn ? kHeld + 1 : 1];
+  __device__ __forceinline__ void ask(const RowsDepth& d, int m, int n) {
+    if constexpr (kOn) {
+      const float* at = d.stack + static_cast<int64_t>(m) * d.ld + n;
+#pragma unroll
+      for (int j = 0; j < kHeld; ++j) held[j] = at[max(min(j, d.n - 2), 0) * d.level_stride];
+#pragma unroll
+      for (int j = 0; j < kHeld; ++j) weight[j] = d.w[min(j, d.n - 1)];
+      weight[kHeld] = d.w[d.n - 1];
+    }
+  }
+  __device__ __forceinline__ float average(const RowsDepth& d, int m, int n, float mine) const {
+    float* at = d.stack + static_cast<int64_t>(m) * d.ld + n;
+    at[(d.n - 1) * d.level_stride] = mine;
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j)
+      if (j < d.n - 1) acc += weight[j] * held[j];
+    for (int j = kHeld; j < d.n - 1; ++j) acc += d.w[j] * at[j * d.level_stride];
+    return acc + weight[kHeld] * mine;
+  }
+};
+
 // MR: rows computed (1, 2, 4, 8, or 16 for plain products; rows beyond M are not stored); C: columns per block; kRwSwiglu: W is the gate
 // matrix and W2 the up matrix, same columns; TO: float or bf16_t; kMaxWaves: bound of the block's waves.
 template <int MR, int C, int kEpilogue, typename TO, bool kNorm, int kMaxWaves>
-__global__ void __launch_bounds__(64 * kMaxWaves) gemm_rows_kernel(
+__device__ __forceinline__ void rows_block(
     TO* __restrict__ out, int64_t ldo, const void* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W,
     const bf16_t* __restrict__ W2, int64_t ldw, const float* __restrict__ bias, int M, int N, int K,
-    const float* __restrict__ norm_w, float eps) {
+    const float* __restrict__ norm_w, float eps, int block, const RowsActivation& act, const RowsDepth& depth) {
   constexpr int kMats = is_gated(kEpilogue) ? 2 : 1;
   constexpr int V = C * MR;                                // partial sums per lane and matrix
   __shared__ float red[kMaxWaves][kMats][V];
   __shared__ float ssq[kNorm ? kMaxWaves : 1][MR];
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, n_waves = blockDim.x / 64;
-  const int n0 = blockIdx.x * C;
+  const int n0 = block * C;
   const int k0 = (wave * 64 + lane) * 8;
   const bool k_ok = k0 < K;
 
@@ -145,9 +188,11 @@ __global__ void __launch_bounds__(64 * kMaxWaves) gemm_rows_kernel(
   const int my_c = threadIdx.x / MR, my_m = threadIdx.x % MR;
   const bool finisher = threadIdx.x < V && my_m < M && n0 + my_c < N;
   float add = 0.f;
+  DepthOf<kEpilogue == kRwDepth> levels;
   if (finisher) {
-    if (kEpilogue == kRwStore && bias) add = bias[n0 + my_c];
-    if (kEpilogue == kRwResidual) add = load_f32(out + static_cast<int64_t>(my_m) * ldo + n0 + my_c);
+    if ((kEpilogue == kRwStore || kEpilogue == kRwActivated) && bias) add = bias[n0 + my_c];
+    if (kEpilogue == kRwResidual || kEpilogue == kRwDepth) add = load_f32(out + static_cast<int64_t>(my_m) * ldo + n0 + my_c);
+    levels.ask(depth, my_m, n0 + my_c);
   }
   // a lane past the end of K adds nothing: its weights and its rows' values are cleared
   if (!k_ok) {
@@ -219,13 +264,48 @@ __global__ void __launch_bounds__(64 * kMaxWaves) gemm_rows_kernel(
     up *= factor;
   }
   TO* dst = out + static_cast<int64_t>(my_m) * ldo + n0 + my_c;
-  if (kEpilogue == kRwStore) {
+  if constexpr (kEpilogue == kRwStore) {
     store_f32(dst, sum + add);
-  } else if (kEpilogue == kRwResidual) {
+  } else if constexpr (kEpilogue == kRwResidual) {
     store_f32(dst, add + sum);
+  } else if constexpr (kEpilogue == kRwDepth) {
+    store_f32(dst, levels.average(depth, my_m, n0 + my_c, add + sum));
+  } else if constexpr (kEpilogue == kRwActivated) {
+    store_f32(dst, act.kind < 0 ? sum + add : activation_of(round_bf16(sum + add), act.kind, act.a, act.b));
   } else {
     store_f32(dst, gate_of<kEpilogue == kRwGeglu>(sum) * up);
   }
+}
+
+template <int MR, int C, int kEpilogue, typename TO, bool kNorm, int kMaxWaves>
+__global__ void __launch_bounds__(64 * kMaxWaves) gemm_rows_kernel(
+    TO* __restrict__ out, int64_t ldo, const void* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W,
+    const bf16_t* __restrict__ W2, int64_t ldw, const float* __restrict__ bias, int M, int N, int K,
+    const float* __restrict__ norm_w, float eps, RowsDepth depth) {
+  rows_block<MR, C, kEpilogue, TO, kNorm, kMaxWaves>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, norm_w, eps, blockIdx.x, RowsActivation{}, depth);
+}
+
+// Up to kRowsMany products of the same count of rows and K side by side, each with its own rows, weights, columns and activation, a range of the grid's blocks each: bfloat16 rows and results.
+// Such a launch is mostly the launch: the five of a time-mixing layer and an activation (1,024 x 1,024 four times, 64 x 1,024; in a captured run, us, one by one / this): one row 11.5 / 3.0, four 13.0 / 3.6,
+// eight 14.7 / 4.5; of width 2,048 four rows 16.8 / 5.8. An activation behind 4,096 x 1,024 against four rows 5.0 / 3.4, eight 5.7 / 4.0; the average over nine levels behind 1,024 x 4,096 5.8 / 3.7 and
+// 6.5 / 4.4 (kRwDepth).
+constexpr int kRowsMany = 5;
+struct RowsProducts {
+  bf16_t* out[kRowsMany];
+  const bf16_t *a[kRowsMany], *w[kRowsMany];
+  int64_t ldo[kRowsMany], lda[kRowsMany], ldw[kRowsMany];
+  int columns[kRowsMany], blocks_upto[kRowsMany];      // blocks of the products up to this one
+  RowsActivation act[kRowsMany];
+  const float* bias;                                    // of a product that stands alone
+};
+template <int MR, int kMaxWaves>
+__global__ void __launch_bounds__(64 * kMaxWaves) gemm_rows_many_kernel(RowsProducts p, int M, int K) {
+  int i = 0;
+#pragma unroll
+  for (int j = 0; j < kRowsMany - 1; ++j) i += static_cast<int>(blockIdx.x) >= p.blocks_upto[j] ? 1 : 0;
+  i = __builtin_amdgcn_readfirstlane(i);
+  rows_block<MR, 4, kRwActivated, bf16_t, false, kMaxWaves>(p.out[i], p.ldo[i], p.a[i], p.lda[i], p.w[i], nullptr, p.ldw[i], p.bias, M, p.columns[i], K, nullptr, 0.f,
+                                                            static_cast<int>(blockIdx.x) - (i > 0 ? p.blocks_upto[i - 1] : 0), p.act[i], RowsDepth{});
 }
 
 // K beyond kRowsMaxK: the block's eight waves (eight rows' operands leave no registers for more, and the number
@@ -238,7 +318,7 @@ constexpr int rows_long_waves(int) { return 8; }
 template <int MR, int C, int kEpilogue, typename TO>
 __global__ void __launch_bounds__(64 * rows_long_waves(MR)) gemm_rows_long_kernel(
     TO* __restrict__ out, int64_t ldo, const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int64_t ldw,
-    const float* __restrict__ bias, int M, int N, int K) {
+    const float* __restrict__ bias, int M, int N, int K, RowsDepth depth) {
   constexpr int V = C * MR, kWaves = rows_long_waves(MR);
   __shared__ float red[kWaves][V];
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
@@ -281,9 +361,11 @@ __global__ void __launch_bounds__(64 * rows_long_waves(MR)) gemm_rows_long_kerne
   const int my_c = threadIdx.x / MR, my_m = threadIdx.x % MR;
   const bool finisher = threadIdx.x < V && my_m < M && n0 + my_c < N;
   float add = 0.f;
+  DepthOf<kEpilogue == kRwDepth> levels;
   if (finisher) {
-    if (kEpilogue == kRwStore && bias) add = bias[n0 + my_c];
-    if (kEpilogue == kRwResidual) add = load_f32(out + static_cast<int64_t>(my_m) * ldo + n0 + my_c);
+    if ((kEpilogue == kRwStore || kEpilogue == kRwActivated) && bias) add = bias[n0 + my_c];
+    if (kEpilogue == kRwResidual || kEpilogue == kRwDepth) add = load_f32(out + static_cast<int64_t>(my_m) * ldo + n0 + my_c);
+    levels.ask(depth, my_m, n0 + my_c);
   }
   const int runs = (K + 511) / 512;
   Set s0, s1;
@@ -306,18 +388,19 @@ __global__ void __launch_bounds__(64 * rows_long_waves(MR)) gemm_rows_long_kerne
 #pragma unroll
   for (int w = 1; w < kWaves; ++w) sum += red[w][threadIdx.x];
   TO* dst = out + static_cast<int64_t>(my_m) * ldo + n0 + my_c;
-  store_f32(dst, kEpilogue == kRwStore ? sum + add : add + sum);
+  if constexpr (kEpilogue == kRwDepth) store_f32(dst, levels.average(depth, my_m, n0 + my_c, add + sum));
+  else store_f32(dst, kEpilogue == kRwStore ? sum + add : add + sum);
 }
 
 template <int MR, int C, int kEpilogue, typename TO, bool kNorm>
 static int launch_rows(void* out, int64_t ldo, const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw,
-                       const float* bias, int M, int N, int K, const float* norm_w, float eps, hipStream_t stream) {
+                       const float* bias, int M, int N, int K, const float* norm_w, float eps, const RowsDepth& depth, hipStream_t stream) {
   const int waves = (K + 511) / 512;
   const dim3 grid((N + C - 1) / C);
   if (waves > kRowsMaxWaves) {
     if constexpr (!kNorm && !is_gated(kEpilogue) && MR <= 8) {
       gemm_rows_long_kernel<MR, C, kEpilogue, TO><<<grid, 64 * rows_long_waves(MR), 0, stream>>>(
-          static_cast<TO*>(out), ldo, static_cast<const bf16_t*>(A), lda, static_cast<const bf16_t*>(W), ldw, bias, M, N, K);
+          static_cast<TO*>(out), ldo, static_cast<const bf16_t*>(A), lda, static_cast<const bf16_t*>(W), ldw, bias, M, N, K, depth);
       return check_launch("gemm_rows (long K)");
     }
     ALOFA_REQUIRE(false, "gemm_rows: K=%d beyond %d goes with the store and residual epilogues of bfloat16 rows only", K, kRowsMaxK);
@@ -326,7 +409,7 @@ static int launch_rows(void* out, int64_t ldo, const void* A, int64_t lda, const
 #define ALOFA_ROWS(MAXW)                                                                                               \
   gemm_rows_kernel<MR, C, kEpilogue, TO, kNorm, MAXW><<<grid, 64 * waves, 0, stream>>>(                                \
       static_cast<TO*>(out), ldo, A, lda, static_cast<const bf16_t*>(W), static_cast<const bf16_t*>(W2), ldw, bias, M, \
-      N, K, norm_w, eps)
+      N, K, norm_w, eps, depth)
   if (waves <= 4) {
     ALOFA_ROWS(4);
   } else {
@@ -338,17 +421,17 @@ static int launch_rows(void* out, int64_t ldo, const void* A, int64_t lda, const
 
 template <int kEpilogue, typename TO, bool kNorm>
 static int dispatch_rows(void* out, int64_t ldo, const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw,
-                         const float* bias, int M, int N, int K, const float* norm_w, float eps, hipStream_t stream) {
+                         const float* bias, int M, int N, int K, const float* norm_w, float eps, hipStream_t stream, const RowsDepth& depth = RowsDepth{}) {
   // (gate and up: eight columns of either, so that the rows, which every block reads and, with a norm, converts,
   // are read half as often where the blocks are many)
   constexpr int C = is_gated(kEpilogue) ? 8 : 4;
-  if (M <= 1) return launch_rows<1, C, kEpilogue, TO, kNorm>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, norm_w, eps, stream);
-  if (M <= 2) return launch_rows<2, C, kEpilogue, TO, kNorm>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, norm_w, eps, stream);
-  if (M <= 4) return launch_rows<4, C, kEpilogue, TO, kNorm>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, norm_w, eps, stream);
-  if constexpr (!kNorm && !is_gated(kEpilogue)) {
-    if (M > 8) return launch_rows<16, C, kEpilogue, TO, kNorm>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, norm_w, eps, stream);
+  if (M <= 1) return launch_rows<1, C, kEpilogue, TO, kNorm>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, norm_w, eps, depth, stream);
+  if (M <= 2) return launch_rows<2, C, kEpilogue, TO, kNorm>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, norm_w, eps, depth, stream);
+  if (M <= 4) return launch_rows<4, C, kEpilogue, TO, kNorm>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, norm_w, eps, depth, stream);
+  if constexpr (!kNorm && !is_gated(kEpilogue) && kEpilogue != kRwDepth) {
+    if (M > 8) return launch_rows<16, C, kEpilogue, TO, kNorm>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, norm_w, eps, depth, stream);
   }
-  return launch_rows<8, C, kEpilogue, TO, kNorm>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, norm_w, eps, stream);
+  return launch_rows<8, C, kEpilogue, TO, kNorm>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, norm_w, eps, depth, stream);
 }
 
 }  // namespace alofa
@@ -390,4 +473,53 @@ extern "C" int alofa_gemm_rows(void* out, int o_dtype, int64_t ldo, const void* 
   if (epilogue == kRwGeglu && o_dtype == kBF16 && W2) return dispatch_rows<kRwGeglu, bf16_t, false>(out, ldo, A, lda, W, W2, ldw, bias, M, N, K, nullptr, 0.f, stream);
   ALOFA_REQUIRE(false, "gemm_rows: no kernel for epilogue %d with output type %d", epilogue, o_dtype);
   return 1;
+}
+
+// Products of up to eight rows side by side, out_i [M, columns_i] = act_i(a_i [M, K] w_i^T), bfloat16 throughout, in one launch (count 1 to 5; what comes behind is not read). kind: -1 as it is, else an
+// activation of pointwise.hip with its numbers act_a, act_b (the same for all of them). bias: of a product that stands alone.
+extern "C" int alofa_gemm_rows_many(int count, int M, int K, const float* bias, float act_a, float act_b,
+                                    void* o0, int64_t ldo0, const void* a0, int64_t lda0, const void* w0, int64_t ldw0, int n0, int kind0,
+                                    void* o1, int64_t ldo1, const void* a1, int64_t lda1, const void* w1, int64_t ldw1, int n1, int kind1,
+                                    void* o2, int64_t ldo2, const void* a2, int64_t lda2, const void* w2, int64_t ldw2, int n2, int kind2,
+                                    void* o3, int64_t ldo3, const void* a3, int64_t lda3, const void* w3, int64_t ldw3, int n3, int kind3,
+                                    void* o4, int64_t ldo4, const void* a4, int64_t lda4, const void* w4, int64_t ldw4, int n4, int kind4, hipStream_t stream) {
+  ALOFA_REQUIRE(count >= 1 && count <= kRowsMany && M >= 1 && M <= 8 && K >= 8 && K % 8 == 0 && K <= kRowsMaxK && (!bias || count == 1),
+                "gemm_rows_many: %d products (1..%d; a bias with one only), M=%d (1..8), K=%d (a multiple of 8, at most %d)", count, kRowsMany, M, K, kRowsMaxK);
+  void* const os[] = {o0, o1, o2, o3, o4};
+  const void *const as[] = {a0, a1, a2, a3, a4}, *const ws[] = {w0, w1, w2, w3, w4};
+  const int64_t ldos[] = {ldo0, ldo1, ldo2, ldo3, ldo4}, ldas[] = {lda0, lda1, lda2, lda3, lda4}, ldws[] = {ldw0, ldw1, ldw2, ldw3, ldw4};
+  const int ns[] = {n0, n1, n2, n3, n4}, kinds[] = {kind0, kind1, kind2, kind3, kind4};
+  RowsProducts p{};
+  p.bias = bias;
+  int blocks = 0;
+  for (int i = 0; i < kRowsMany; ++i) {
+    if (i < count) {
+      ALOFA_REQUIRE(ns[i] >= 1 && ldas[i] >= K && ldws[i] >= K && ldos[i] >= ns[i] && ldas[i] % 8 == 0 && ldws[i] % 8 == 0 && reinterpret_cast<uintptr_t>(as[i]) % 16 == 0 &&
+                        reinterpret_cast<uintptr_t>(ws[i]) % 16 == 0, "gemm_rows_many: product %d: columns %d, rows of A and W must be 16-byte aligned, strides no shorter than the rows", i, ns[i]);
+      ALOFA_REQUIRE(kinds[i] >= -1 && kinds[i] <= 3, "gemm_rows_many: no such activation (%d)", kinds[i]);
+      p.out[i] = static_cast<bf16_t*>(os[i]), p.a[i] = static_cast<const bf16_t*>(as[i]), p.w[i] = static_cast<const bf16_t*>(ws[i]);
+      p.ldo[i] = ldos[i], p.lda[i] = ldas[i], p.ldw[i] = ldws[i], p.columns[i] = ns[i], p.act[i] = RowsActivation{kinds[i], act_a, act_b};
+      blocks += (ns[i] + 3) / 4;
+    }
+    p.blocks_upto[i] = i < count ? blocks : 0x7fffffff;
+  }
+  const int waves = (K + 511) / 512;
+#define ALOFA_MANY(MR)                                                                                         \
+  if (waves <= 4) gemm_rows_many_kernel<MR, 4><<<blocks, 64 * waves, 0, stream>>>(p, M, K);                    \
+  else gemm_rows_many_kernel<MR, kRowsMaxWaves><<<blocks, 64 * waves, 0, stream>>>(p, M, K)
+  if (M <= 1) { ALOFA_MANY(1); }
+  else if (M <= 2) { ALOFA_MANY(2); }
+  else if (M <= 4) { ALOFA_MANY(4); }
+  else { ALOFA_MANY(8); }
+#undef ALOFA_MANY
+  return check_launch("gemm_rows_many");
+}
+
+// alofa_gemm_rows with the residual epilogue, and behind it the average over depth (see RowsDepth): stack [levels][level_stride], rows of it `ld` apart, w [n].
+extern "C" int alofa_gemm_rows_depth(float* out, int64_t ldo, const void* A, int64_t lda, const void* W, int64_t ldw, int M, int N, int K, float* stack, int64_t level_stride, int64_t ld,
+                                     const float* w, int n, hipStream_t stream) {
+  ALOFA_REQUIRE(M <= 8 && alofa_gemm_rows_fits(M, N, K, 1), "gemm_rows_depth: M=%d (1..8) N=%d K=%d (a multiple of 8)", M, N, K);
+  ALOFA_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0, "gemm_rows_depth: rows of A and W must be 16-byte aligned");
+  ALOFA_REQUIRE(lda >= K && ldw >= K && ldo >= N && ld >= N && n >= 1 && w && stack, "gemm_rows_depth: strides shorter than the rows, or no levels (%d)", n);
+  return dispatch_rows<kRwDepth, float, false>(out, ldo, A, lda, W, nullptr, ldw, nullptr, M, N, K, nullptr, 0.f, stream, RowsDepth{stack, level_stride, ld, w, n});
 }

@@ -237,9 +237,7 @@ __global__ void __launch_bounds__(256) headnorm_gate_wide_kernel(T* __restrict__
 }
 
 // ---- activations -------------------------------------------------------------------------------
-// kind 0: xIELU with a = softplus(p) and b = 1/2 + softplus(q) given: z > 0: a z^2 + z/2; else b (exp(z) - 1 - z) + z/2.
-// kind 1: tanh. kind 2: silu, z sigmoid(z). kind 3: the tanh form of gelu, z/2 (1 + tanh(sqrt(2/pi) (z + 0.044715 z^3))).
-// In place or not; rows of `width` values with a row stride.
+// activation_of (common.h), element by element. In place or not; rows of `width` values with a row stride.
 template <typename T, typename Acc>
 __global__ void __launch_bounds__(256) activation_kernel(T* __restrict__ out, int64_t out_stride, const T* __restrict__ x, int64_t x_stride,
                                                          int64_t rows, int width, int kind, float a, float b) {
@@ -247,18 +245,7 @@ __global__ void __launch_bounds__(256) activation_kernel(T* __restrict__ out, in
   if (idx >= rows * width) return;
   const int64_t r = idx / width;
   const int c = static_cast<int>(idx % width);
-  const Acc z = static_cast<Acc>(load_f32(x + r * x_stride + c));
-  Acc y;
-  if (kind == 0) {
-    y = z > 0 ? static_cast<Acc>(a) * z * z + z / 2 : static_cast<Acc>(b) * (expm1(z) - z) + z / 2;
-  } else if (kind == 1) {
-    y = tanh(z);
-  } else if (kind == 2) {
-    y = z / (static_cast<Acc>(1) + exp(-z));
-  } else {
-    y = z / 2 * (static_cast<Acc>(1) + tanh(static_cast<Acc>(0.7978845608028654) * (z + static_cast<Acc>(0.044715) * z * z * z)));
-  }
-  store_f32(out + r * out_stride + c, static_cast<float>(y));
+  store_f32(out + r * out_stride + c, static_cast<float>(activation_of(static_cast<Acc>(load_f32(x + r * x_stride + c)), kind, static_cast<Acc>(a), static_cast<Acc>(b))));
 }
 
 // ---- weighted average over depth -----------------------------------------------------------------

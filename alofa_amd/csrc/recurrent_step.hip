@@ -5,6 +5,8 @@
 // parts), norm and gate 2.2 to 4 (4 requests, 16 heads of 64 x 64 in a captured step). What the work cannot do without is the state, read and written once: 16 KB a head.
 // 1 to 64 requests of 1 to 32 heads, 1.01 to 2.2 times as fast, but a few (request, head) pairs of the widest heads, whose state one block reads and writes here: those go launch by launch
 // (recurrence_step_pays in ops.py has the figures).
+// Where the decays come from a projection of few channels (its rank), the block makes its head's share of it too: the launch that was saved took 2.6 us of a captured step, the products hide behind the
+// state's loads.
 // A block takes a head of a request. The state's loads set out first (a thread has four neighbouring columns of every so-manieth row, 16 bytes a load), the row's operands are made meanwhile, each
 // once, in LDS; the read-outs' shares meet in LDS in row order. Read-outs stay float up to the norm's end, as they are between the launches.
 #include "common.h"
@@ -18,8 +20,11 @@ struct StepArgs {
   int64_t out_stride;
   const bf16_t *q, *k, *v, *gate;
   int64_t q_stride, k_stride, v_stride, gate_stride;
-  const float* decay;      // per head [heads], or z [rows, heads * dk]
+  const float* decay;      // per head [heads], or z [rows, heads * dk], or (low not null) z's bias [heads * dk]
   int64_t decay_stride;
+  const bf16_t *low, *low_w;      // z = low [rows, rank] low_w^T + bias, low_w [heads * dk, rank]; null: z is given
+  int64_t low_stride, low_ld;
+  int rank;                       // a multiple of 8, at most kStepRank
   const float* bonus;
   const float* weight;     // of the norm [heads * dv]; null: none
   float* state;
@@ -30,7 +35,7 @@ struct StepArgs {
   float inv_tau, q_scale, k_scale, eps;
 };
 
-constexpr int kStepThreads = 512, kStepMost = 256;      // kStepMost: key and value channels of a head
+constexpr int kStepThreads = 512, kStepMost = 256, kStepRank = 64;      // kStepMost: key and value channels of a head
 
 // kRows: rows of the state a thread has at most
 template <int kRows>
@@ -47,6 +52,19 @@ __global__ void __launch_bounds__(kStepThreads) recurrence_step_kernel(StepArgs 
   for (int n = 0; n < kRows; ++n) {
     const int i = first + n * every;
     s[n] = works && i < dk ? S[static_cast<int64_t>(i) * quads + quad] : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  // the decays' projection: a thread of the second half has a key channel; its weights and the row set out with the state
+  uint4 lw[kStepRank / 8], lx[kStepRank / 8];
+  const int key = tid - kStepMost;
+  const bool projects = a.low != nullptr && key >= 0 && key < dk;
+  if (a.low != nullptr) {      // (uniform)
+    const int own = projects ? key : 0;
+#pragma unroll
+    for (int i = 0; i < kStepRank / 8; ++i) {
+      const int at = 8 * i < a.rank ? 8 * i : 0;
+      lw[i] = *reinterpret_cast<const uint4*>(a.low_w + static_cast<int64_t>(h * dk + own) * a.low_ld + at);
+      lx[i] = *reinterpret_cast<const uint4*>(a.low + r * a.low_stride + at);
+    }
   }
   float z = 0.f, weight = 1.f;      // of the channel that this thread finishes
   if (tid < dv) {
@@ -80,7 +98,20 @@ __global__ void __launch_bounds__(kStepThreads) recurrence_step_kernel(StepArgs 
         if (a.decay_kind == kStepPerHead) {
           ws[i] = a.decay[h];
         } else {
-          const float x = a.decay[r * a.decay_stride + h * dk + i];
+          float x = a.decay[r * a.decay_stride + h * dk + i];      // (low: the bias, decay_stride 0)
+          if (projects) {
+#pragma unroll
+            for (int n = 0; n < kStepRank / 8; ++n) {
+              const uint32_t u[4] = {lw[n].x, lw[n].y, lw[n].z, lw[n].w}, v[4] = {lx[n].x, lx[n].y, lx[n].z, lx[n].w};
+              if (8 * n < a.rank) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                  x += __uint_as_float(u[e] << 16) * __uint_as_float(v[e] << 16);
+                  x += __uint_as_float(u[e] & 0xffff0000u) * __uint_as_float(v[e] & 0xffff0000u);
+                }
+              }
+            }
+          }
           ws[i] = a.decay_kind == kStepSigmoidRoot ? expf(-(fmaxf(-x, 0.f) + log1pf(expf(-fabsf(x)))) * a.inv_tau) : expf(-expf(x));
         }
         us[i] = a.bonus ? a.bonus[h * dk + i] : 0.f;
@@ -127,9 +158,11 @@ using namespace alofa;
 
 extern "C" int alofa_recurrence_step_takes(int dk, int dv) { return dk >= 1 && dk <= kStepMost && dv >= 4 && dv <= kStepMost && dv % 4 == 0; }
 
-// out [rows, heads * dv]: the read-outs of one row a request, normed per head, gated. decay: [heads] (decay_kind 0) or z [rows, heads * dk] (1: sigmoid(z)^(1 / tau), 2: exp(-exp(z))).
+// out [rows, heads * dv]: the read-outs of one row a request, normed per head, gated. decay: [heads] (decay_kind 0) or z [rows, heads * dk] (1: sigmoid(z)^(1 / tau), 2: exp(-exp(z))); low not null:
+// z = low [rows, rank] low_w [heads * dk, rank]^T + decay [heads * dk], in bfloat16 products and float sums.
 extern "C" int alofa_recurrence_step(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v, int64_t v_stride,
-                                     const void* gate, int64_t gate_stride, const float* decay, int64_t decay_stride, const float* bonus, const float* weight, float* state,
+                                     const void* gate, int64_t gate_stride, const float* decay, int64_t decay_stride, const void* low, int64_t low_stride, const void* low_w, int64_t low_ld, int rank,
+                                     const float* bonus, const float* weight, float* state,
                                      const int32_t* req_slot, const float* cos_t, const float* sin_t, const int32_t* positions, int rows, int heads, int dk, int dv,
                                      int decay_kind, float tau, float q_scale, float k_scale, float eps, int before_update, hipStream_t stream) {
   ALOFA_REQUIRE(rows >= 0 && rows <= 65535 && heads > 0 && alofa_recurrence_step_takes(dk, dv), "recurrence_step: bad sizes (rows=%d heads=%d dk=%d dv=%d)", rows, heads, dk, dv);
@@ -137,9 +170,11 @@ extern "C" int alofa_recurrence_step(void* out, int64_t out_stride, const void* 
                 "recurrence_step: decay kind %d, tau %g, eps %g", decay_kind, static_cast<double>(tau), static_cast<double>(eps));
   ALOFA_REQUIRE(!cos_t || (sin_t && positions && dk % 2 == 0), "recurrence_step: a rotation needs both tables, positions, and an even number of key channels (%d)", dk);
   ALOFA_REQUIRE(reinterpret_cast<uintptr_t>(state) % 16 == 0, "recurrence_step: the state must be 16-byte aligned");
+  ALOFA_REQUIRE(!low || (low_w && decay_kind != kStepPerHead && decay_stride == 0 && rank >= 8 && rank <= kStepRank && rank % 8 == 0 && low_stride % 8 == 0 && low_ld % 8 == 0 && low_ld >= rank &&
+                         reinterpret_cast<uintptr_t>(low) % 16 == 0 && reinterpret_cast<uintptr_t>(low_w) % 16 == 0), "recurrence_step: the decays' projection takes aligned rows of 8 to %d channels in eights (%d)", kStepRank, rank);
   if (rows == 0) return 0;
   const StepArgs a = {static_cast<bf16_t*>(out), out_stride, static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k), static_cast<const bf16_t*>(v), static_cast<const bf16_t*>(gate),
-                      q_stride, k_stride, v_stride, gate_stride, decay, decay_stride, bonus, weight, state, req_slot, cos_t, sin_t, positions, heads, dk, dv, decay_kind, before_update,
+                      q_stride, k_stride, v_stride, gate_stride, decay, decay_stride, static_cast<const bf16_t*>(low), static_cast<const bf16_t*>(low_w), low_stride, low_ld, rank, bonus, weight, state, req_slot, cos_t, sin_t, positions, heads, dk, dv, decay_kind, before_update,
                       decay_kind == kStepSigmoidRoot ? 1.f / tau : 0.f, q_scale, k_scale, eps};
   const int every = kStepThreads / (dv / 4), most = (dk + every - 1) / every;
   const dim3 grid(heads, rows);

@@ -186,6 +186,7 @@ GATED = {"silu": 2, "gelu_tanh": 4}      # epilogues of the products of gate and
 
 
 ROWS_MAX_M, ROWS_MAX_K = 8, 6144      # what the vector-unit kernel for very few rows takes (longer rows: plain products only)
+ROWS_SIDE_BY_SIDE = 5                 # products that one launch of it takes side by side
 ROWS_MAX_M_PLAIN = 16                 # ... and up to so many rows for plain products of rows up to ROWS_MAX_K
 
 
@@ -380,7 +381,7 @@ def _exact_operands(**operands) -> None:
 
 def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
          add_to_out: bool = False, exact: bool = False, kernel: Optional[str] = None, norm: Optional[tuple] = None,
-         then_norm: Optional[tuple] = None, scratch=None) -> None:
+         then_norm: Optional[tuple] = None, scratch=None, act: Optional[tuple] = None, depth: Optional[tuple] = None) -> None:
     """out = a @ w.T (+ bias), or out += a @ w.T when ``add_to_out`` (out is then
     the float32 residual stream). w is [out_features, in_features]. ``kernel``
     names the bfloat16 kernel ("rows", "stream" or "tiled") instead of ``few_rows_kernel``.
@@ -391,7 +392,12 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[tor
     rows in hand (the tiled kernel with K shared out and a launch that adds the shares) the norm rides
     on it; everywhere else it is the norm kernel, run here: the values are the same either way.
     ``scratch``: (name, shape, dtype) -> a buffer of the caller's stream that the call may use and leave (a step's, which its captured graphs share and
-    the memory account sees); without it, the products that need one allocate it."""
+    the memory account sees); without it, the products that need one allocate it.
+    ``act`` = (kind, a, b): ``activation`` of the result; ``depth`` = (stack, weights, n) with ``add_to_out``: ``depth_average`` of out's new rows. Both ride on the
+    vector-unit kernel of up to eight rows and are launches of their own behind every other: the values are the same either way."""
+    if act is not None or depth is not None:
+        _gemm_and(out, a, w, bias, add_to_out, exact, kernel, norm, then_norm, scratch, act, depth)
+        return
     sizes = None if exact or norm is not None else _native().product(out, a, w, None, bias)      # (bfloat16 operands that 16-byte loads along K can read)
     if sizes is not None:
         M, N, K, ldo, lda, ldw, code = sizes
@@ -461,6 +467,60 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[tor
           _I(ADD_TO_RESIDUAL if add_to_out else STORE), _stream())
     if then_rows is not None:
         rmsnorm(then_rows, out, then_w, then_eps, exact)
+
+
+def _gemm_and(out, a, w, bias, add_to_out, exact, kernel, norm, then_norm, scratch, act, depth) -> None:
+    """``gemm`` with an activation or an average over depth behind it: one launch where the kernel of choice is the vector-unit kernel."""
+    if (act is not None and (add_to_out or depth is not None)) or (depth is not None and (not add_to_out or then_norm is not None or norm is not None)):
+        raise AlofaError("invalid_argument", "an activation goes with a product that stores its result, an average over depth with one that adds to the stream")
+    sizes = None if exact or norm is not None else _native().product(out, a, w, None, bias)
+    if sizes is not None:
+        M, N, K, ldo, lda, ldw, _ = sizes
+        if act is not None and out.dtype is torch.bfloat16 and act[0] in ACTIVATIONS and kernel is None and _rows_product(M, N, K) and K <= ROWS_MAX_K:
+            _rows_side_by_side(M, K, bias, act[1], act[2], [(out, ldo, a, lda, w, ldw, N, act[0])])
+            return
+        if depth is not None and out.dtype is torch.float32 and kernel is None and _rows_product(M, N, K) and bias is None:
+            stack, weights, n = depth
+            if _level_stack(out, stack, weights, n):
+                _call("alofa_gemm_rows_depth", out, ldo, a, lda, w, ldw, M, N, K, stack, out.numel(), N, weights, n, _stream())
+                return
+    gemm(out, a, w, bias, add_to_out, exact, kernel, norm, then_norm, scratch)
+    if act is not None:
+        activation(out, out, *act, exact=exact)
+    else:
+        depth_average(out, *depth, exact=exact)
+
+
+def _rows_product(M: int, N: int, K: int) -> bool:
+    """Whether a plain product is the vector-unit kernel's, with at most eight rows (its forms with something behind the sum)."""
+    return M <= ROWS_MAX_M and _product_entry(None, M, N, K) == "alofa_gemm_rows"
+
+
+def _rows_side_by_side(M: int, K: int, bias: Optional[torch.Tensor], act_a: float, act_b: float, products: list) -> None:
+    """``products``: (out, ldo, a, lda, w, ldw, columns, activation or -1) each, at most ``ROWS_SIDE_BY_SIDE``, checked."""
+    flat = [x for p in products for x in p] + [None, 0, None, 0, None, 0, 0, -1] * (ROWS_SIDE_BY_SIDE - len(products))
+    _call("alofa_gemm_rows_many", len(products), M, K, bias, act_a, act_b, *flat, _stream())
+
+
+def gemm_side_by_side(products: list, exact: bool = False, scratch=None) -> None:
+    """Products of the same count of rows that do not depend on one another: (out, a, w, activation kind or None (``TANH``, ``SILU``, ``GELU_TANH``)) each, as ``gemm(act=)``. One launch
+    where all of them are bfloat16 products of the same K that the vector-unit kernel of up to eight rows would take one by one; the values are the same either way."""
+    if not exact and 2 <= len(products) <= ROWS_SIDE_BY_SIDE:
+        flat = []
+        for out, a, w, act in products:
+            sizes = _native().product(out, a, w, None, None)
+            if sizes is None or out.dtype is not torch.bfloat16 or act not in (None, TANH, SILU, GELU_TANH):
+                break
+            M, N, K, ldo, lda, ldw, _ = sizes
+            if not _rows_product(M, N, K) or K > ROWS_MAX_K or (flat and (M, K) != same):
+                break
+            same = (M, K)
+            flat.append((out, ldo, a, lda, w, ldw, N, -1 if act is None else act))
+        else:
+            _rows_side_by_side(*same, None, 0.0, 0.0, flat)
+            return
+    for out, a, w, act in products:
+        gemm(out, a, w, exact=exact, scratch=scratch, act=None if act is None else (act, 0.0, 0.0))
 
 
 def gemm_swiglu(out: torch.Tensor, a: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, exact: bool = False,
@@ -1361,7 +1421,7 @@ def headnorm_gate(out: torch.Tensor, o: torch.Tensor, gate: torch.Tensor, weight
           _I(int(gate_kind == "sigmoid")), _I(extra), _ptr(floor), _stream())
 
 
-XIELU, TANH, SILU, GELU_TANH = 0, 1, 2, 3
+ACTIVATIONS = XIELU, TANH, SILU, GELU_TANH = 0, 1, 2, 3
 
 
 def activation(out: torch.Tensor, x: torch.Tensor, kind: int, a: float = 0.0, b: float = 0.0, exact: bool = False) -> None:
@@ -1375,6 +1435,12 @@ def activation(out: torch.Tensor, x: torch.Tensor, kind: int, a: float = 0.0, b:
         raise AlofaError("invalid_argument", "the exact path is float32 throughout", f"out={out.dtype}")
     _call("alofa_activation", _ptr(out), _L(_rows("out", out)), _ptr(x), _L(_rows("x", x)), _I(dtype_code(out)), _L(x.shape[0]), _I(x.shape[1]),
           _I(kind), _F(a), _F(b), _I(int(exact)), _stream())
+
+
+def _level_stack(x: torch.Tensor, stack: torch.Tensor, weights: Optional[torch.Tensor], n: int) -> bool:
+    """Whether the operands of an average over depth are such as a product's kernel takes along (``depth_average`` names what is wrong with others)."""
+    return (weights is not None and x.is_contiguous() and stack.is_cuda and stack.dtype is torch.float32 and stack.is_contiguous() and tuple(stack.shape[1:]) == tuple(x.shape)
+            and 1 <= n <= stack.shape[0] and weights.is_cuda and weights.dtype is torch.float32 and weights.is_contiguous() and tuple(weights.shape) == (n,))
 
 
 def depth_average(x: torch.Tensor, stack: torch.Tensor, weights: Optional[torch.Tensor], n: int, exact: bool = False) -> None:
@@ -1561,10 +1627,17 @@ def recurrence_step_pays(requests: int, heads: int, dk: int, dv: int, turned: bo
     return turned or requests * heads > 6 or dk <= 224 or dv < 192
 
 
+def recurrence_step_makes_decays(low: torch.Tensor, w: torch.Tensor, bias: torch.Tensor, rows: int, channels: int) -> bool:
+    """Whether ``recurrence_step`` takes the decays' projection along: bfloat16 rows ``low`` [rows, rank] and ``w`` [channels, rank] that 16-byte loads can read, a bias. Up to 64 channels of rank: a
+    channel's are one thread's, whose loads are all on their way at once."""
+    return (low.is_cuda and _aligned_rows(low) and low.dim() == 2 and low.shape[0] == rows and w.is_cuda and w.dim() == 2 and _aligned_rows(w) and tuple(w.shape) == (channels, low.shape[1])
+            and low.shape[1] % 8 == 0 and low.shape[1] <= 64 and bias is not None and bias.is_cuda and bias.dtype is torch.float32 and bias.is_contiguous() and tuple(bias.shape) == (channels,))
+
+
 def recurrence_step(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torch.Tensor, weight: Optional[torch.Tensor], state: torch.Tensor, rows: RowsOfRequests,
                     heads: int, dk: int, dv: int, eps: float, decay_kind: int, decay: torch.Tensor, tau: float = 1.0, bonus: Optional[torch.Tensor] = None, q_scale: float = 1.0,
                     k_scale: float = 1.0, before_update: bool = False, rope: Optional[tuple] = None) -> None:
-    """``linear_recurrence`` for steps in which every request brings one row, with what stands around it in one launch: with ``rope`` = (cos, sin, positions) the rotation
+    """``decay`` may be (low, w, bias) in place of z: z = low @ w.T + bias, made in the same launch (``recurrence_step_makes_decays``). ``linear_recurrence`` for steps in which every request brings one row, with what stands around it in one launch: with ``rope`` = (cos, sin, positions) the rotation
     of queries and keys (``rope_kv_write`` of both, which are left as they are), and ``headnorm_gate`` (silu) of the read-outs, which ``out`` [T, heads * dv] receives. All rows bfloat16."""
     T = q.shape[0]
     for name, t, width in (("out", out, heads * dv), ("q", q, heads * dk), ("k", k, heads * dk), ("v", v, heads * dv), ("gate", gate, heads * dv)):
@@ -1575,11 +1648,18 @@ def recurrence_step(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torc
         raise AlofaError("shape_mismatch", "a step of one row a request, heads of at most 256 channels", f"state={tuple(state.shape)} heads={heads} dk={dk} dv={dv} rows={rows.rows}")
     rows.fits("state", state)
     per_head = decay_kind == DECAY_PER_HEAD
-    _gpu("decay", decay, torch.float32, 1 if per_head else 2)
-    if per_head:
-        _contig("decay", decay)
-    if decay_kind not in (DECAY_PER_HEAD, DECAY_SIGMOID_ROOT, DECAY_EXP_NEG_EXP) or tuple(decay.shape) != ((heads,) if per_head else (T, heads * dk)):
-        raise AlofaError("shape_mismatch", "the decay does not fit its kind", f"decay={tuple(decay.shape)} kind={decay_kind} heads={heads} dk={dk}")
+    low = low_w = low_b = None
+    if isinstance(decay, tuple):
+        low, low_w, low_b = decay
+        if not recurrence_step_makes_decays(low, low_w, low_b, T, heads * dk) or decay_kind not in (DECAY_SIGMOID_ROOT, DECAY_EXP_NEG_EXP):
+            raise AlofaError("shape_mismatch", "the decays' projection does not fit", f"low={tuple(low.shape)} w={tuple(low_w.shape)} kind={decay_kind} heads={heads} dk={dk}")
+        decay = low_b
+    else:
+        _gpu("decay", decay, torch.float32, 1 if per_head else 2)
+        if per_head:
+            _contig("decay", decay)
+        if decay_kind not in (DECAY_PER_HEAD, DECAY_SIGMOID_ROOT, DECAY_EXP_NEG_EXP) or tuple(decay.shape) != ((heads,) if per_head else (T, heads * dk)):
+            raise AlofaError("shape_mismatch", "the decay does not fit its kind", f"decay={tuple(decay.shape)} kind={decay_kind} heads={heads} dk={dk}")
     if bonus is not None and (tuple(_contig("bonus", _gpu("bonus", bonus, torch.float32, 2)).shape) != (heads, dk) or not before_update):
         raise AlofaError("shape_mismatch", "the bonus is [heads, dk] and goes with the read-out before the update", f"bonus={tuple(bonus.shape)}")
     if weight is not None and tuple(_contig("weight", _gpu("weight", weight, torch.float32, 1)).shape) != (heads * dv,):
@@ -1593,7 +1673,8 @@ def recurrence_step(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torc
         if tuple(_contig("positions", _gpu("positions", positions, torch.int32, 1)).shape) != (T,):
             raise AlofaError("shape_mismatch", "one position per row", f"positions={tuple(positions.shape)} rows={T}")
     _call("alofa_recurrence_step", _ptr(out), _L(_rows("out", out)), _ptr(q), _L(_rows("q", q)), _ptr(k), _L(_rows("k", k)), _ptr(v), _L(_rows("v", v)), _ptr(gate), _L(_rows("gate", gate)),
-          _ptr(decay), _L(0 if per_head else _rows("decay", decay)), _ptr(bonus), _ptr(weight), _ptr(state), _ptr(rows.slots), _ptr(cos), _ptr(sin), _ptr(positions),
+          _ptr(decay), _L(0 if per_head or low is not None else _rows("decay", decay)), _ptr(low), _L(0 if low is None else _rows("low", low)), _ptr(low_w), _L(0 if low is None else _rows("w", low_w)),
+          _I(0 if low is None else low.shape[1]), _ptr(bonus), _ptr(weight), _ptr(state), _ptr(rows.slots), _ptr(cos), _ptr(sin), _ptr(positions),
           _I(T), _I(heads), _I(dk), _I(dv), _I(decay_kind), _F(tau), _F(q_scale), _F(k_scale), _F(eps), _I(int(before_update)), _stream())
 
 

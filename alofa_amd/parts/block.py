@@ -160,6 +160,9 @@ class FilteredPreNormBlock(Block):
                 ops.depth_average(hidden, stack, None, 1, self.rt.exact)
         self.mixer.forward(ctx, (entry, 0), self._read(ctx, entry, 0, hidden), hidden)
         if self.feed_forward is not None:
+            if stack is not None and getattr(self.feed_forward, "takes_depth", False):      # the average rides on the product that adds to the stream
+                self.feed_forward.forward(ctx, self._read(ctx, entry, 1, hidden), hidden, depth=(stack, self.depth_weights, self.level + 1))
+                return
             self.feed_forward.forward(ctx, self._read(ctx, entry, 1, hidden), hidden)
         if stack is not None:
             ops.depth_average(hidden, stack, self.depth_weights, self.level + 1, self.rt.exact)

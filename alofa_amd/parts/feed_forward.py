@@ -112,19 +112,23 @@ class DenseActivated(FeedForward):
     def fuses_norm(self, norm, rows):
         return not self.rt.exact and norm.as_rmsnorm() is not None and ops.can_fuse_norm(rows, self.w_up, self.rt.dtype)
 
-    def forward(self, ctx, x, residual, scale=None, norm=None, then=None):
+    @property
+    def takes_depth(self):
+        return self.b_down is None
+
+    def forward(self, ctx, x, residual, scale=None, norm=None, then=None, depth=None):
+        """``depth`` = (stack, weights, n) (where the part ``takes_depth``): the average over depth of the stream's new rows, ``ops.depth_average``, behind the sum."""
         act = ctx.scratch("ff_act", (residual.shape[0], self.intermediate), self.rt.dtype)
+        kind = {"xielu": (ops.XIELU, getattr(self, "a", 0.0), getattr(self, "b", 0.0)), "gelu_tanh": (ops.GELU_TANH, 0.0, 0.0)}.get(self.activation)
         if norm is not None:      # the norm in front rides on the product
-            ops.gemm(act, residual, self.w_up, self.b_up, norm=norm.as_rmsnorm())
+            ops.gemm(act, residual, self.w_up, self.b_up, norm=norm.as_rmsnorm(), act=kind)
         else:
-            ops.gemm(act, x, self.w_up, self.b_up, exact=self.rt.exact, scratch=ctx.scratch)
-        if self.activation == "xielu":
-            ops.activation(act, act, ops.XIELU, self.a, self.b, self.rt.exact)
-        elif self.activation == "gelu_tanh":
-            ops.activation(act, act, ops.GELU_TANH, exact=self.rt.exact)
-        else:
+            ops.gemm(act, x, self.w_up, self.b_up, exact=self.rt.exact, scratch=ctx.scratch, act=kind)
+        if kind is None:
             ops.relu_squared(act, act)
-        if scale is None and self.b_down is None:
+        if depth is not None:
+            ops.gemm(residual, act, self.w_down, add_to_out=True, exact=self.rt.exact, scratch=ctx.scratch, depth=depth)
+        elif scale is None and self.b_down is None:
             ops.gemm(residual, act, self.w_down, add_to_out=True, exact=self.rt.exact, scratch=ctx.scratch)
             if then is not None:
                 ops.rmsnorm(then[2], residual, then[0], then[1], self.rt.exact)

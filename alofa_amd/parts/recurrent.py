@@ -103,11 +103,19 @@ class RecurrentMixer(Mixer):
         else:
             ops.gemm(residual, y, self.w_o, add_to_out=True, exact=self.rt.exact, scratch=ctx.scratch)
 
+    def _projected(self, ctx, low, w, bias):
+        """What the decays are made of, z = low @ w.T + bias, float32."""
+        z = ctx.scratch("recurrent_decay", (low.shape[0], self.heads * self.dk), torch.float32)
+        ops.gemm(z, low, w, bias, exact=self.rt.exact, scratch=ctx.scratch)
+        return z
+
     def _single_step(self, ctx, where, q, k, v, gate, weight, residual, out, decay_kind, decay, **how) -> bool:
-        """Where every request brings one row: the recurrence, the head norm and the gate in one launch, and the output projection. False (and nothing done) where it is no such step, or one that is slower so."""
+        """``decay``: one per head, or (low, w, bias), which z is projected from. Where every request brings one row: the recurrence, the head norm and the gate in one launch, and the output projection. False (and nothing done) where it is no such step, or one that is slower so."""
         rows = rows_of_requests(ctx)
         if not ops.recurrence_step_takes(rows, self.dk, self.dv, self.rt.dtype, q) or not ops.recurrence_step_pays(rows.rows, self.heads, self.dk, self.dv, how.get("rope") is not None):
             return False
+        if isinstance(decay, tuple) and not ops.recurrence_step_makes_decays(*decay, q.shape[0], self.heads * self.dk):
+            decay = self._projected(ctx, *decay)
         y = ctx.scratch("recurrent_gated", (q.shape[0], self.heads * self.dv), self.rt.dtype)
         ops.recurrence_step(y, q, k, v, gate, weight, ctx.state(where), rows, self.heads, self.dk, self.dv, self.eps, decay_kind, decay, **how)
         self._project(ctx, y, residual, out)
@@ -195,13 +203,12 @@ class GatedLinearAttention(RecurrentMixer):
         T, kd, vd = x.shape[0], self.heads * self.dk, self.heads * self.dv
         proj = ctx.scratch("recurrent_proj", (T, 2 * kd + 2 * vd + self.rank), self.rt.dtype)
         ops.gemm(proj, x, self.w_in, exact=self.rt.exact, scratch=ctx.scratch)
-        z = ctx.scratch("recurrent_decay", (T, kd), torch.float32)
-        ops.gemm(z, proj[:, 2 * kd + 2 * vd:], self.w_a2, self.b_a2, exact=self.rt.exact, scratch=ctx.scratch)
-        if self._single_step(ctx, where, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:2 * kd + vd], proj[:, 2 * kd + vd:2 * kd + 2 * vd], self.norm, residual, out, ops.DECAY_SIGMOID_ROOT, z,
+        low = (proj[:, 2 * kd + 2 * vd:], self.w_a2, self.b_a2)
+        if self._single_step(ctx, where, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:2 * kd + vd], proj[:, 2 * kd + vd:2 * kd + 2 * vd], self.norm, residual, out, ops.DECAY_SIGMOID_ROOT, low,
                              tau=self.tau, q_scale=self.q_scale):
             return
         o = self._readouts(ctx, T)
-        parts = self._decays(ctx, where, o, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:2 * kd + vd], ops.DECAY_SIGMOID_ROOT, z, tau=self.tau, q_scale=self.q_scale)
+        parts = self._decays(ctx, where, o, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:2 * kd + vd], ops.DECAY_SIGMOID_ROOT, self._projected(ctx, *low), tau=self.tau, q_scale=self.q_scale)
         self._leave(ctx, o, parts, proj[:, 2 * kd + vd:2 * kd + 2 * vd], self.norm, residual, out)
 
 
@@ -461,18 +468,15 @@ class TimeMix(RecurrentMixer):
         mixes = ctx.scratch("time_mix_inputs", (len(MIXES), T, self.hidden), self.rt.dtype)
         self.shift.forward(ctx, (entry, k + 1), mixes, x)
         proj = ctx.scratch("time_mix_proj", (T, 4 * kd), self.rt.dtype)
-        for i, n in enumerate(("r", "k", "v", "g")):
-            ops.gemm(proj[:, i * kd:(i + 1) * kd], mixes[i], self.w[n], exact=exact, scratch=ctx.scratch)
         low = ctx.scratch("time_mix_low", (T, self.rank), self.rt.dtype)
-        ops.gemm(low, mixes[4], self.w["w1"], exact=exact, scratch=ctx.scratch)
-        ops.activation(low, low, ops.TANH, exact=exact)
-        z = ctx.scratch("recurrent_decay", (T, kd), torch.float32)
-        ops.gemm(z, low, self.w["w2"], self.w0, exact=exact, scratch=ctx.scratch)
-        if self._single_step(ctx, (entry, k), proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:3 * kd], proj[:, 3 * kd:], self.norm, residual, out, ops.DECAY_EXP_NEG_EXP, z,
+        ops.gemm_side_by_side([(proj[:, i * kd:(i + 1) * kd], mixes[i], self.w[n], None) for i, n in enumerate(("r", "k", "v", "g"))] + [(low, mixes[4], self.w["w1"], ops.TANH)],
+                              exact=exact, scratch=ctx.scratch)
+        low = (low, self.w["w2"], self.w0)
+        if self._single_step(ctx, (entry, k), proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:3 * kd], proj[:, 3 * kd:], self.norm, residual, out, ops.DECAY_EXP_NEG_EXP, low,
                              bonus=self.bonus, before_update=True):
             return
         o = self._readouts(ctx, T)
-        parts = self._decays(ctx, (entry, k), o, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:3 * kd], ops.DECAY_EXP_NEG_EXP, z, bonus=self.bonus, before_update=True)
+        parts = self._decays(ctx, (entry, k), o, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:3 * kd], ops.DECAY_EXP_NEG_EXP, self._projected(ctx, *low), bonus=self.bonus, before_update=True)
         self._leave(ctx, o, parts, proj[:, 3 * kd:], self.norm, residual, out)
 
 
@@ -523,6 +527,11 @@ class ParallelMixers(Mixer):
 
     def forward(self, ctx, where, x, residual, out=None, scale=None, then=None):
         entry, k = where if isinstance(where, tuple) else (where, 0)
+        if not self.norms and out is None and not self.rt.exact and all(s == 1.0 for s in self.scales):      # (nothing between a branch and the stream: each adds to it with its last product)
+            for b in self.branches:
+                b.forward(ctx, (entry, k), x, residual)
+                k += len(b.stateful_parts())
+            return
         outs = []
         for j, b in enumerate(self.branches):
             buf = ctx.scratch(f"branch_{j}", tuple(residual.shape), torch.float32)

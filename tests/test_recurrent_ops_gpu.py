@@ -422,3 +422,72 @@ def test_recurrence_in_chunks_with_decays_per_row(heads, dk, dv, lengths, kind):
             # float sums of some hundred terms, products of up to 64 decays
             assert np.abs(got[part, vc] - want).max() <= 2e-5 * max(1.0, np.abs(want).max()), (r, h)
             assert np.abs(after[slot, h] - S).max() <= 2e-5 * max(1.0, np.abs(S).max()), (r, h)
+
+
+# what rides on the vector-unit product is the same bits as the launches one behind the other: K of one run, several, ragged and (depth) the long form; rows up to eight and, launch by launch, beyond; columns of no whole block
+@pytest.mark.parametrize("M,N,K", [(1, 64, 512), (4, 4096, 1024), (5, 37, 520), (8, 130, 6144), (3, 64, 8192), (12, 96, 1024), (2, 8, 16)])
+def test_products_with_what_follows_them(M, N, K):
+    from alofa_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(M + N)
+    draw = lambda *s: torch.randn(s, generator=gen, device=DEV)      # noqa: E731
+    a, w, bias = draw(M, K).bfloat16(), (draw(N, K) * K ** -0.5).bfloat16(), draw(N)
+    for b in (None, bias):
+        for kind in ops.ACTIVATIONS:
+            want, got = torch.empty(M, N, device=DEV, dtype=torch.bfloat16), torch.empty(M, N + 5, device=DEV, dtype=torch.bfloat16).fill_(7.0)
+            ops.gemm(want, a, w, b)
+            ops.activation(want, want, kind, 0.7, 1.1)
+            ops.gemm(got[:, :N], a, w, b, act=(kind, 0.7, 1.1))
+            assert torch.equal(got[:, :N], want) and bool((got[:, N:] == 7.0).all()), kind
+    for n in (1, 2, 8, 9, 13):
+        levels, weights, x = draw(14, M, N), draw(n), draw(M, N)
+        stacks, xs = [levels.clone(), levels.clone()], [x.clone(), x.clone()]
+        ops.gemm(xs[0], a, w, add_to_out=True)
+        ops.depth_average(xs[0], stacks[0], weights, n)
+        ops.gemm(xs[1], a, w, add_to_out=True, depth=(stacks[1], weights, n))
+        assert torch.equal(xs[0], xs[1]) and torch.equal(*stacks), n
+
+
+@pytest.mark.parametrize("M,K,columns", [(1, 512, (64, 64)), (4, 1024, (1024, 1024, 1024, 1024, 64)), (8, 520, (5, 130, 4)), (3, 4096, (33, 7, 64, 1)), (9, 256, (64, 32))])
+def test_products_side_by_side(M, K, columns):
+    from alofa_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(K)
+    products, want = [], []
+    wide = torch.zeros(M, sum(columns) + 8, device=DEV, dtype=torch.bfloat16)      # (results beside one another in one buffer)
+    at = 0
+    for i, n in enumerate(columns):
+        a, w = torch.randn(M, K, generator=gen, device=DEV).bfloat16(), (torch.randn(n, K, generator=gen, device=DEV) * K ** -0.5).bfloat16()
+        kind = (None, ops.TANH, ops.SILU, None, ops.GELU_TANH)[i]
+        products.append((wide[:, at:at + n], a, w, kind))
+        alone = torch.empty(M, n, device=DEV, dtype=torch.bfloat16)
+        ops.gemm(alone, a, w)
+        if kind is not None:
+            ops.activation(alone, alone, kind)
+        want.append(alone)
+        at += n
+    ops.gemm_side_by_side(products)
+    assert torch.equal(wide[:, :at], torch.cat(want, 1)) and not bool(wide[:, at:].any())
+
+
+@pytest.mark.parametrize("rank", [8, 16, 40, 64])
+@pytest.mark.parametrize("heads,dk,dv,kind", [(3, 64, 64, "sigmoid_root"), (2, 40, 72, "exp_neg_exp"), (1, 256, 8, "exp_neg_exp")])
+def test_single_row_step_that_makes_its_decays(heads, dk, dv, kind, rank):
+    from alofa_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(rank + dk)
+    draw = lambda *s: torch.randn(s, generator=gen, device=DEV)      # noqa: E731
+    n = 5
+    wide = draw(n, 2 * heads * dk + 2 * heads * dv + rank).bfloat16()
+    q, k, v, gate, low = wide.split([heads * dk, heads * dk, heads * dv, heads * dv, rank], 1)
+    w, bias = (draw(heads * dk, rank) * rank ** -0.5).bfloat16(), draw(heads * dk)
+    z = (low.double() @ w.double().T.contiguous() + bias.double()).float()      # (products of bfloat16 numbers and sums of up to 64: a float rounding from what the kernel makes)
+    before = kind == "exp_neg_exp"
+    code, rows = (ops.DECAY_EXP_NEG_EXP if before else ops.DECAY_SIGMOID_ROOT), rows_of([(s, 1) for s in (3, 0, 5, 1, 2)], 6)
+    bonus, first = draw(heads, dk) if before else None, draw(6, heads, dk, dv)
+    got = []
+    for decay in (z, (low, w, bias)):
+        state, out = first.clone(), torch.empty(n, heads * dv, device=DEV, dtype=torch.bfloat16)
+        ops.recurrence_step(out, q, k, v, gate, None, state, rows, heads, dk, dv, 1e-6, code, decay, tau=5.0, bonus=bonus, before_update=before)
+        got.append((out.float(), state))
+    # a decay moves by its exponent's rounding (sums of up to 64 products: some 2e-6 of z), the state by that times itself; an output by that or a rounding to bfloat16
+    assert (got[0][1] - got[1][1]).abs().max().item() <= 2e-5 * first.abs().max().item()
+    assert (got[0][0] - got[1][0]).abs().max().item() <= 2.0 ** -7 * got[0][0].abs().max().item()
+    assert torch.equal(got[0][1][4], first[4]) and torch.equal(got[1][1][4], first[4])
