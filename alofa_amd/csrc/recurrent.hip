@@ -137,6 +137,109 @@ __global__ void __launch_bounds__(256) norm_conv_step_kernel(TO* __restrict__ ou
   store_f32(out + static_cast<int64_t>(r) * width + c, static_cast<float>(acc));
 }
 
+// The same for portions of any lengths: a block takes kConvRows rows of one request, whose norms' sums its wavefronts make first, those of the kTaps - 1 rows in front of them too; a thread then has four
+// channels, filters down the rows and keeps the rows before in registers. The state's old rows are read, and its new ones written, by the request's first block alone (which makes the norms of
+// the request's last rows once more for it), so no other block can find them changed. Three launches did this by way of a float copy of the normed rows: 1,050 rows of 1,024 in four requests, us,
+// launch by launch 20.9 (5.5 + 11 + 4.4, each in a step under the profiler), this 8.3.
+constexpr int kConvRows = 8;
+template <typename TO, int kTaps, int kOwn>
+__global__ void __launch_bounds__(256) norm_conv_rows_kernel(TO* __restrict__ out, const float* __restrict__ x, const float* __restrict__ nw, const float* __restrict__ nb, float eps,
+                                                             const float* __restrict__ w, float* __restrict__ state, const int32_t* __restrict__ req_slot, const int32_t* __restrict__ row_off, int width) {
+  constexpr int kKeep = kTaps - 1, kAll = kConvRows + kKeep, kEach = (kAll + 3) / 4;
+  __shared__ float means[kAll], invs[kAll];
+  const int r = blockIdx.y, row0 = row_off[r], end = row_off[r + 1], c0 = row0 + static_cast<int>(blockIdx.x) * kConvRows;
+  if (c0 >= end) return;      // (uniform over the block)
+  const int n = min(kConvRows, end - c0), lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, quads = width / 4;
+  // mean and 1 / deviation of rows first + i, i = wave, wave + 4, ..: of those that are there, kEach a wavefront, their values on their way together; rows up to 256 kOwn wide stay in registers
+  auto norms = [&](int first, int count) __attribute__((always_inline)) {
+    float4 own[kEach][kOwn > 0 ? kOwn : 1];
+    const float4* rows[kEach];
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+      rows[e] = reinterpret_cast<const float4*>(x + static_cast<int64_t>(min(max(first + min(wave + 4 * e, count - 1), row0), end - 1)) * width);
+#pragma unroll
+      for (int i = 0; i < kOwn; ++i) own[e][i] = rows[e][min(lane + kWave * i, quads - 1)];
+    }
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+      if (wave + 4 * e >= count) break;      // (uniform over the wavefront)
+      float s = 0.f, ss = 0.f;
+      if constexpr (kOwn > 0) {
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i) s += lane + kWave * i < quads ? own[e][i].x + own[e][i].y + (own[e][i].z + own[e][i].w) : 0.f;
+      } else {
+        for (int i = lane; i < quads; i += kWave) s += rows[e][i].x + rows[e][i].y + (rows[e][i].z + rows[e][i].w);
+      }
+      const float mean = wave_sum(s) / static_cast<float>(width);
+      auto squares = [&](float4 v) { return (v.x - mean) * (v.x - mean) + (v.y - mean) * (v.y - mean) + ((v.z - mean) * (v.z - mean) + (v.w - mean) * (v.w - mean)); };
+      if constexpr (kOwn > 0) {
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i) ss += lane + kWave * i < quads ? squares(own[e][i]) : 0.f;
+      } else {
+        for (int i = lane; i < quads; i += kWave) ss += squares(rows[e][i]);
+      }
+      const float var = wave_sum(ss) / static_cast<float>(width);
+      if (lane == 0) means[wave + 4 * e] = mean, invs[wave + 4 * e] = 1.f / sqrtf(var + eps);
+    }
+  };
+  norms(c0 - kKeep, n + kKeep);
+  __syncthreads();
+  float* st = state + static_cast<int64_t>(req_slot[r]) * kKeep * width;
+  auto normed = [&](float4 v, int i, float4 weight, float4 shift) {      // i: which of the rows whose sums lie in LDS
+    const float m = means[i], f = invs[i];
+    return make_float4((v.x - m) * f * weight.x + shift.x, (v.y - m) * f * weight.y + shift.y, (v.z - m) * f * weight.z + shift.z, (v.w - m) * f * weight.w + shift.w);
+  };
+  auto row = [&](int t, int q) { return reinterpret_cast<const float4*>(x + static_cast<int64_t>(t) * width)[q]; };
+  for (int q = threadIdx.x; q < quads; q += 256) {
+    float4 xs[kAll], taps[kTaps];
+#pragma unroll
+    for (int i = 0; i < kAll; ++i) {      // (in front of the request's first row: what the state holds; past the last: the last again)
+      const int t = c0 - kKeep + i;
+      xs[i] = t >= row0 ? row(min(t, c0 + n - 1), q) : reinterpret_cast<const float4*>(st + static_cast<int64_t>(kKeep + t - row0) * width)[q];
+    }
+    float raw[4 * kTaps];
+#pragma unroll
+    for (int i = 0; i < kTaps; ++i) *reinterpret_cast<float4*>(raw + 4 * i) = reinterpret_cast<const float4*>(w + static_cast<int64_t>(4 * q) * kTaps)[i];
+#pragma unroll
+    for (int j = 0; j < kTaps; ++j) taps[j] = make_float4(raw[j], raw[kTaps + j], raw[2 * kTaps + j], raw[3 * kTaps + j]);
+    const float4 weight = reinterpret_cast<const float4*>(nw)[q], shift = reinterpret_cast<const float4*>(nb)[q];
+#pragma unroll
+    for (int i = 0; i < kAll; ++i)
+      if (c0 - kKeep + i >= row0) xs[i] = normed(xs[i], i, weight, shift);
+#pragma unroll
+    for (int i = 0; i < kConvRows; ++i) {
+      if (i >= n) break;      // (uniform)
+      const float4 mine = xs[i + kKeep];
+      float4 acc = mine;
+#pragma unroll
+      for (int j = 0; j < kTaps; ++j) {      // (the row's own tap last)
+        const float4 v = xs[i + j];
+        acc.x += taps[j].x * v.x, acc.y += taps[j].y * v.y, acc.z += taps[j].z * v.z, acc.w += taps[j].w * v.w;
+      }
+      TO* dst = out + static_cast<int64_t>(c0 + i) * width + 4 * q;
+      if constexpr (sizeof(TO) == 2) *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(acc.x, acc.y), pack_bf16x2(acc.z, acc.w));
+      else *reinterpret_cast<float4*>(dst) = acc;
+    }
+  }
+  if (blockIdx.x != 0) return;
+  // ---- the request's last rows, normed, into the state (a thread has the channels that it has read above)
+  __syncthreads();
+  const int from = max(end - kKeep, row0);
+  norms(from, end - from);
+  __syncthreads();
+  for (int q = threadIdx.x; q < quads; q += 256) {
+    const float4 weight = reinterpret_cast<const float4*>(nw)[q], shift = reinterpret_cast<const float4*>(nb)[q];
+    float4 kept[kKeep];
+#pragma unroll
+    for (int i = 0; i < kKeep; ++i) {
+      const int t = end - kKeep + i;
+      kept[i] = t >= row0 ? normed(row(t, q), t - from, weight, shift) : reinterpret_cast<const float4*>(st + static_cast<int64_t>(kKeep + t - row0) * width)[q];
+    }
+#pragma unroll
+    for (int i = 0; i < kKeep; ++i) reinterpret_cast<float4*>(st + static_cast<int64_t>(i) * width)[q] = kept[i];
+  }
+}
+
 // ---- mix with the token before --------------------------------------------------------------------------
 // out[s, t, c] = x[t, c] + (x[t-1, c] - x[t, c]) * mu[s, c] for s < n_mixes; the row before a request's first row
 // of this step is state[slot, c] (zeros for a new request). The state is kept by keep_last_rows (keep = 1), or, in steps of
@@ -585,6 +688,28 @@ extern "C" int alofa_norm_conv_step(void* out, int out_dtype, const float* x, co
 #undef ALOFA_STEP
 #undef ALOFA_STEP_AS
   return check_launch("norm_conv_step");
+}
+
+extern "C" int alofa_norm_conv_rows_takes(int width, int taps) { return taps >= 2 && taps <= 4 && width >= 4 && width % 4 == 0; }
+
+// longest: rows of the request that brings the most.
+extern "C" int alofa_norm_conv_rows(void* out, int out_dtype, const float* x, const float* nw, const float* nb, float eps, const float* w, float* state, const int32_t* req_slot,
+                                    const int32_t* row_off, int requests, int longest, int width, int taps, hipStream_t stream) {
+  ALOFA_REQUIRE(requests >= 0 && requests <= 65535 && longest >= 1 && alofa_norm_conv_rows_takes(width, taps) && eps > 0.f, "norm_conv_rows: bad sizes (requests=%d longest=%d width=%d taps=%d)", requests, longest, width, taps);
+  for (const void* p : {static_cast<const void*>(out), static_cast<const void*>(x), static_cast<const void*>(nw), static_cast<const void*>(nb), static_cast<const void*>(w), static_cast<const void*>(state)})
+    ALOFA_REQUIRE(reinterpret_cast<uintptr_t>(p) % 16 == 0, "norm_conv_rows: operands must be 16-byte aligned");
+  if (requests == 0) return 0;
+  const dim3 grid((longest + kConvRows - 1) / kConvRows, requests);
+#define ALOFA_NC(TO, TAPS, OWN) norm_conv_rows_kernel<TO, TAPS, OWN><<<grid, 256, 0, stream>>>(static_cast<TO*>(out), x, nw, nb, eps, w, state, req_slot, row_off, width)
+#define ALOFA_NC_TAPS(TO, TAPS) if (width <= 1024) ALOFA_NC(TO, TAPS, 4); else if (width <= 2048) ALOFA_NC(TO, TAPS, 8); else ALOFA_NC(TO, TAPS, 0)
+  if (out_dtype == kF32) {
+    if (taps == 2) { ALOFA_NC_TAPS(float, 2); } else if (taps == 3) { ALOFA_NC_TAPS(float, 3); } else { ALOFA_NC_TAPS(float, 4); }
+  } else {
+    if (taps == 2) { ALOFA_NC_TAPS(bf16_t, 2); } else if (taps == 3) { ALOFA_NC_TAPS(bf16_t, 3); } else { ALOFA_NC_TAPS(bf16_t, 4); }
+  }
+#undef ALOFA_NC_TAPS
+#undef ALOFA_NC
+  return check_launch("norm_conv_rows");
 }
 
 extern "C" int alofa_keep_last_rows(void* state, const void* h, int dtype, const int32_t* req_slot, const int32_t* row_off, int requests, int width,

@@ -1538,6 +1538,27 @@ def norm_conv_step(out: torch.Tensor, x: torch.Tensor, norm_w: torch.Tensor, nor
           _I(T), _I(width), _I(taps), _I(int(exact)), _stream())
 
 
+def norm_conv_rows_takes(x: torch.Tensor, norm_w: torch.Tensor, norm_b: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``norm_conv_rows`` takes these operands: two to four taps, rows in fours of channels, 16-byte aligned."""
+    return bool(_answer("alofa_norm_conv_rows_takes", x.shape[1], w.shape[1])) and all(t.data_ptr() % 16 == 0 and t.is_contiguous() for t in (x, norm_w, norm_b, w))
+
+
+def norm_conv_rows(out: torch.Tensor, x: torch.Tensor, norm_w: torch.Tensor, norm_b: torch.Tensor, eps: float, w: torch.Tensor, state: torch.Tensor, rows: RowsOfRequests, longest: int) -> None:
+    """``layernorm``, ``short_conv`` and ``keep_last_rows`` in one launch for portions of any lengths (``longest``: the most rows a request brings), in float: out[t] = n[t] + conv(n)[t], n the layer
+    norm of x; the state (float32 [slots, taps - 1, width]) moves on by n."""
+    _gpu("out", out, None, 2), _gpu("x", x, torch.float32, 2), _gpu("w", w, torch.float32, 2), _gpu("state", state, torch.float32, 3)
+    _gpu("norm_w", norm_w, torch.float32, 1), _gpu("norm_b", norm_b, torch.float32, 1)
+    for n, t in (("out", out), ("x", x), ("w", w), ("state", state), ("norm_w", norm_w), ("norm_b", norm_b)):
+        _contig(n, t)
+    T, width = x.shape
+    taps = w.shape[1]
+    if (tuple(out.shape) != (T, width) or w.shape[0] != width or tuple(state.shape[1:]) != (taps - 1, width) or norm_w.shape[0] != width or norm_b.shape[0] != width
+            or rows.offsets is None or rows.rows != T or not 1 <= longest <= T):
+        raise AlofaError("shape_mismatch", "norm and convolution operands do not fit (portions of requests)", f"out={tuple(out.shape)} x={tuple(x.shape)} w={tuple(w.shape)} state={tuple(state.shape)} longest={longest}")
+    rows.fits("state", state)
+    _call("alofa_norm_conv_rows", out, dtype_code(out), x, norm_w, norm_b, _F(eps), w, state, rows.slots, rows.offsets, rows.requests, longest, width, taps, _stream())
+
+
 def keep_last_rows(state: torch.Tensor, h: torch.Tensor, rows: RowsOfRequests) -> None:
     """state[slot] [keep, width] = the last ``keep`` rows its request has seen once this step's rows ``h`` are in (older
     ones from the state itself where the step brought fewer)."""

@@ -195,7 +195,7 @@ class TimeConv(Part):
     def prepare(self, n_positions: int) -> None:
         pass
 
-    def fuses_norm(self, ctx, norm) -> bool:
+    def fuses_norm(self, ctx, norm, x) -> bool:
         """Whether, in this step, the filter would rather apply ``norm`` to the stream itself, in the same launch. A filter
         that says yes is called as ``forward(ctx, where, out, stream, norm=norm)``."""
         return False

@@ -32,14 +32,19 @@ class ShortCausalConv(TimeConv):
     def state_need(self):
         return StateNeed((self.taps - 1, self.width), torch.float32) if self.taps > 1 else None
 
-    def fuses_norm(self, ctx, norm):
-        # single rows (decoding): norm, filter and the state's step are one launch
-        return ctx.max_q_len == 1 and self.taps > 1 and norm.as_layernorm() is not None
+    def fuses_norm(self, ctx, norm, x):
+        # norm, filter and the state's step are one launch: for single rows (decoding), and for portions where the kernel takes the sizes (not on the exact path, whose sums are float64)
+        if self.taps <= 1 or norm.as_layernorm() is None:
+            return False
+        return ctx.max_q_len == 1 or (not self.rt.exact and ops.norm_conv_rows_takes(x, *norm.as_layernorm()[:2], self.weight))
 
     def forward(self, ctx, where, out, x, norm=None):
         """out = x + conv(x) for float32 rows x (with ``norm``: for the norm of the rows x); the state moves on by this step's rows."""
         if norm is not None:
             weight, bias, eps = norm.as_layernorm()
+            if ctx.max_q_len > 1:
+                ops.norm_conv_rows(out, x, weight, bias, eps, self.weight, ctx.state(where), rows_of_requests(ctx), ctx.max_q_len)
+                return
             ops.norm_conv_step(out, x, weight, bias, eps, self.weight, ctx.state(where), rows_of_requests(ctx), self.rt.exact)
             return
         if self.taps == 1:      # a filter of one tap sees the row itself only

@@ -491,3 +491,38 @@ def test_single_row_step_that_makes_its_decays(heads, dk, dv, kind, rank):
     assert (got[0][1] - got[1][1]).abs().max().item() <= 2e-5 * first.abs().max().item()
     assert (got[0][0] - got[1][0]).abs().max().item() <= 2.0 ** -7 * got[0][0].abs().max().item()
     assert torch.equal(got[0][1][4], first[4]) and torch.equal(got[1][1][4], first[4])
+
+
+# portions of one row, of fewer rows than the state keeps, of a block's rows and one more, and long ones; widths that stay in registers and wider ones
+@pytest.mark.parametrize("width", [4, 1020, 1024, 1028, 2048, 2052])
+@pytest.mark.parametrize("taps", [2, 3, 4])
+def test_norm_filter_and_state_of_portions_in_one_launch(width, taps):
+    from alofa_amd import ops
+    rng = np.random.default_rng(width + taps)
+    lengths, slots = (1, 2, 3, 8, 9, 35, 16), (6, 0, 3, 7, 1, 2, 5)
+    T = sum(lengths)
+    x, nw, nb, w = dev(rng.normal(1.0, 2.0, (T, width))), dev(rng.normal(1, 0.2, width)), dev(rng.normal(0, 0.5, width)), dev(rng.normal(0, 0.5, (width, taps)))
+    state = dev(rng.normal(0, 1, (8, taps - 1, width)))
+    rows = rows_of(list(zip(slots, lengths)), 8)
+    assert ops.norm_conv_rows_takes(x, nw, nb, w)
+    # launch by launch, and in float64
+    wide, old, old_state = torch.empty_like(x), torch.empty_like(x), state.clone()
+    ops.layernorm(wide, x, nw, nb, 1e-5, False)
+    ops.short_conv(old, wide, w, old_state, rows)
+    ops.keep_last_rows(old_state, wide, rows)
+    xd = x.double()
+    dev2 = xd - xd.mean(1, keepdim=True)
+    n = dev2 / torch.sqrt((dev2 * dev2).mean(1, keepdim=True) + 1e-5) * nw.double() + nb.double()
+    want, want_state, at = torch.empty_like(n), state.double(), 0
+    for s, m in zip(slots, lengths):
+        both = torch.cat([want_state[s], n[at:at + m]])
+        want[at:at + m] = both[taps - 1:] + sum(both[j:j + m] * w.double()[:, j] for j in range(taps))
+        want_state[s] = both[m:]
+        at += m
+    for dtype in (torch.float32, torch.bfloat16):
+        out, got_state = torch.empty(T, width, device=DEV, dtype=dtype), state.clone()
+        ops.norm_conv_rows(out, x, nw, nb, 1e-5, w, got_state, rows, max(lengths))
+        off, off_old = (out.double() - want).norm() / want.norm(), (old.to(dtype).double() - want).norm() / want.norm()
+        assert off < 2 ** -8 and off <= 1.5 * off_old + 1e-7      # (as close to 64 bits as the launches one behind the other, whose sums run in another order)
+        assert (got_state.double() - want_state).abs().max() <= 1.5 * (old_state.double() - want_state).abs().max() + 1e-6
+        assert torch.equal(got_state[4], state[4])
