@@ -4,6 +4,7 @@ in Python. Some 12 us a product instead of 3."""
 from __future__ import annotations
 
 import ctypes
+import threading
 
 import torch
 
@@ -30,6 +31,43 @@ def call(address, *args) -> int:
         else:
             raise TypeError(f"call: a {type(a).__name__} is no tensor, number or None")
     return entry(*passed)
+
+
+class _Noting(threading.local):
+    calls = None
+
+
+_noting = _Noting()
+
+
+def note(address, *args) -> int:
+    rc = call(address, *args)
+    if _noting.calls is not None and rc == 0:
+        _noting.calls.append((address, [a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args]))
+    return rc
+
+
+def tape() -> None:
+    _noting.calls = []
+
+
+def taped(*ranges):
+    calls, _noting.calls = _noting.calls, None
+    if calls is None:
+        raise RuntimeError("taped: no tape is being written")
+    inside = lambda x: next(((r, x - at) for r, (at, size) in enumerate(ranges) if 0 <= x - at < size), None) if isinstance(x, int) else None      # noqa: E731
+    return len(ranges), [(address, args, {k: inside(x) for k, x in enumerate(args) if inside(x) is not None}) for address, args in calls]
+
+
+def play(tape, at) -> int:
+    ranges, calls = tape
+    if len(at) != ranges:
+        raise ValueError("play: another count of ranges than the tape's")
+    for address, args, places in calls:
+        rc = call(address, *[at[places[k][0]] + places[k][1] if k in places else x for k, x in enumerate(args)])
+        if rc != 0:
+            return rc
+    return 0
 
 
 def _leading(t) -> int:

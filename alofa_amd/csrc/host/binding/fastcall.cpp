@@ -1,6 +1,7 @@
 // The way from Python to the kernels' C entries: the call itself without an argument object per parameter (ctypes took some 4 us a
 // call), and the operand checks of what every layer runs without an interpreter's step per question (another 4 us a product). A
-// step of a few short prompts (24 layers of 0.5B sizes, 172 calls) waited for the host: 2.21 ms with 1.27 ms of kernels, 1.47 so.
+// step of a few short prompts (24 layers of 0.5B sizes, 172 calls) waited for the host: 2.21 ms with 1.27 ms of kernels, 1.47 so. The layers of a step that are alike make one layer's calls again
+// (tape, play below; engine/tapes.py).
 // A check here answers the sizes that the launch needs, or nothing: what it does not pass goes to the checks in Python, which take what is
 // left to other kernels and say what is wrong with the rest. Nothing is remembered from call to call.
 #define PY_SSIZE_T_CLEAN
@@ -10,6 +11,9 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <memory>
+#include <utility>
+#include <vector>
 
 namespace {
 
@@ -151,44 +155,149 @@ using F = float;
 using Entry = int (*)(I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I,
                       I, I, I, I, I, F, F, F, F, F, F, F, F);
 
-PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  I i[kInts] = {};
-  F f[kFloats] = {};
+// A call as it was made: for `note` and `play`.
+struct Call {
+  Entry entry;
+  I i[kInts];
+  F f[kFloats];
+  int ni;
+};
+int make(const Call& c) {
+  const I* i = c.i;
+  const F* f = c.f;
+  return c.entry(i[0], i[1], i[2], i[3], i[4], i[5], i[6], i[7], i[8], i[9], i[10], i[11], i[12], i[13], i[14], i[15], i[16], i[17], i[18], i[19], i[20],
+                 i[21], i[22], i[23], i[24], i[25], i[26], i[27], i[28], i[29], i[30], i[31], i[32], i[33], i[34], i[35], i[36], i[37], i[38], i[39],
+                 i[40], i[41], i[42], i[43], i[44], i[45], i[46], i[47], f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7]);
+}
+
+// A tape: calls in their order, and which of their parameters lie in a memory range of the layer that they were made for (range, offset); `play` makes them for another layer.
+struct Tape {
+  struct Patch {
+    int call, parameter, range;
+    I offset;
+  };
+  std::vector<Call> calls;
+  std::vector<Patch> patches;
+  int ranges = 0;
+};
+thread_local Tape* noting = nullptr;
+
+bool read_call(PyObject* const* args, Py_ssize_t n, Call& c) {
+  I* i = c.i;
+  F* f = c.f;
   int ni = 0, nf = 0;
   if (n < 1) {
     PyErr_SetString(PyExc_TypeError, "call: an address comes first");
-    return nullptr;
+    return false;
   }
   const Entry entry = reinterpret_cast<Entry>(PyLong_AsVoidPtr(args[0]));
   if (PyErr_Occurred() || entry == nullptr) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "call: no such entry");
-    return nullptr;
+    return false;
   }
   for (Py_ssize_t k = 1; k < n; ++k) {
     PyObject* o = args[k];
     if (PyFloat_Check(o)) {
-      if (nf == kFloats) { PyErr_SetString(PyExc_TypeError, "call: too many floats"); return nullptr; }
+      if (nf == kFloats) { PyErr_SetString(PyExc_TypeError, "call: too many floats"); return false; }
       f[nf++] = static_cast<float>(PyFloat_AS_DOUBLE(o));
       continue;
     }
-    if (ni == kInts) { PyErr_SetString(PyExc_TypeError, "call: too many parameters"); return nullptr; }
+    if (ni == kInts) { PyErr_SetString(PyExc_TypeError, "call: too many parameters"); return false; }
     if (PyLong_Check(o)) {
       i[ni] = PyLong_AsLongLong(o);
-      if (i[ni++] == -1 && PyErr_Occurred()) return nullptr;
+      if (i[ni++] == -1 && PyErr_Occurred()) return false;
     } else if (o == Py_None) {
       i[ni++] = 0;
     } else if (THPVariable_Check(o)) {
       i[ni++] = reinterpret_cast<I>(THPVariable_Unpack(o).data_ptr());
     } else {
       PyErr_Format(PyExc_TypeError, "call: parameter %zd is no tensor, number or None", k);
-      return nullptr;
+      return false;
     }
   }
+  c.entry = entry, c.ni = ni;
+  return true;
+}
+
+PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  Call c{};
+  if (!read_call(args, n, c)) return nullptr;
   int rc;
   Py_BEGIN_ALLOW_THREADS
-  rc = entry(i[0], i[1], i[2], i[3], i[4], i[5], i[6], i[7], i[8], i[9], i[10], i[11], i[12], i[13], i[14], i[15], i[16], i[17], i[18], i[19], i[20],
-             i[21], i[22], i[23], i[24], i[25], i[26], i[27], i[28], i[29], i[30], i[31], i[32], i[33], i[34], i[35], i[36], i[37], i[38], i[39],
-             i[40], i[41], i[42], i[43], i[44], i[45], i[46], i[47], f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7]);
+  rc = make(c);
+  Py_END_ALLOW_THREADS
+  return PyLong_FromLong(rc);
+}
+
+// note(address, ...): call, kept on this thread's tape as well (if it is being written and the call went well)
+PyObject* note(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  Call c{};
+  if (!read_call(args, n, c)) return nullptr;
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = make(c);
+  Py_END_ALLOW_THREADS
+  if (noting && rc == 0) noting->calls.push_back(c);
+  return PyLong_FromLong(rc);
+}
+
+void drop_tape(PyObject* capsule) { delete static_cast<Tape*>(PyCapsule_GetPointer(capsule, "alofa.tape")); }
+
+// tape(): this thread's calls are noted from now on (what an interrupted step left is dropped)
+PyObject* tape(PyObject*, PyObject* const*, Py_ssize_t) {
+  delete noting;
+  noting = nullptr;
+  noting = new Tape;
+  Py_RETURN_NONE;
+}
+
+// taped((address, bytes), ...): the calls since, for `play`; the ranges are the memory of the layer that they were made for
+PyObject* taped(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (!noting) {
+    PyErr_SetString(PyExc_RuntimeError, "taped: no tape is being written");
+    return nullptr;
+  }
+  std::unique_ptr<Tape> t(noting);
+  noting = nullptr;
+  std::vector<std::pair<I, I>> ranges;
+  for (Py_ssize_t k = 0; k < n; ++k) {
+    if (!PyTuple_Check(args[k]) || PyTuple_GET_SIZE(args[k]) != 2) { PyErr_SetString(PyExc_TypeError, "taped: ranges are pairs"); return nullptr; }
+    ranges.emplace_back(PyLong_AsLongLong(PyTuple_GET_ITEM(args[k], 0)), PyLong_AsLongLong(PyTuple_GET_ITEM(args[k], 1)));
+  }
+  if (PyErr_Occurred()) return nullptr;
+  t->ranges = static_cast<int>(ranges.size());
+  for (size_t c = 0; c < t->calls.size(); ++c)
+    for (int k = 0; k < t->calls[c].ni; ++k)
+      for (size_t r = 0; r < ranges.size(); ++r) {
+        const I off = t->calls[c].i[k] - ranges[r].first;
+        if (off >= 0 && off < ranges[r].second) {
+          t->patches.push_back({static_cast<int>(c), k, static_cast<int>(r), off});
+          break;
+        }
+      }
+  PyObject* capsule = PyCapsule_New(t.get(), "alofa.tape", drop_tape);
+  if (capsule) t.release();
+  return capsule;
+}
+
+// play(tape, (address, ...)): the tape's calls for a layer whose memory ranges begin there; the first answer that is not zero, or zero
+PyObject* play(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (n != 2 || !PyCapsule_IsValid(args[0], "alofa.tape") || !PyTuple_Check(args[1])) {
+    PyErr_SetString(PyExc_TypeError, "play: a tape and the addresses of a layer");
+    return nullptr;
+  }
+  Tape& t = *static_cast<Tape*>(PyCapsule_GetPointer(args[0], "alofa.tape"));
+  if (PyTuple_GET_SIZE(args[1]) != t.ranges) { PyErr_SetString(PyExc_ValueError, "play: another count of ranges than the tape's"); return nullptr; }
+  std::vector<I> at(t.ranges);
+  for (int r = 0; r < t.ranges; ++r) at[r] = PyLong_AsLongLong(PyTuple_GET_ITEM(args[1], r));
+  if (PyErr_Occurred()) return nullptr;
+  for (const Tape::Patch& p : t.patches) t.calls[p.call].i[p.parameter] = at[p.range] + p.offset;
+  int rc = 0;
+  Py_BEGIN_ALLOW_THREADS
+  for (const Call& c : t.calls) {
+    rc = make(c);
+    if (rc != 0) break;
+  }
   Py_END_ALLOW_THREADS
   return PyLong_FromLong(rc);
 }
@@ -202,9 +311,10 @@ PyObject* guarded(PyObject* self, PyObject* const* args, Py_ssize_t n) {
     Py_RETURN_NONE;
   }
 }
+template <PyObject* (*kCall)(PyObject*, PyObject* const*, Py_ssize_t)>
 PyObject* guarded_call(PyObject* self, PyObject* const* args, Py_ssize_t n) {
   try {
-    return call(self, args, n);
+    return kCall(self, args, n);
   } catch (const std::exception& e) {
     PyErr_SetString(PyExc_RuntimeError, e.what());
     return nullptr;
@@ -213,7 +323,8 @@ PyObject* guarded_call(PyObject* self, PyObject* const* args, Py_ssize_t n) {
 
 #define METHOD(name, function) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(function)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {METHOD("product", guarded<product>), METHOD("norm", guarded<norm>), METHOD("caches", guarded<caches>), METHOD("turn", guarded<turn>), METHOD("attention", guarded<attention>),
-                         METHOD("call", guarded_call), {nullptr, nullptr, 0, nullptr}};
+                         METHOD("call", guarded_call<call>), METHOD("note", guarded_call<note>), METHOD("tape", guarded_call<tape>), METHOD("taped", guarded_call<taped>),
+                         METHOD("play", guarded_call<play>), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "alofa_fastcall", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

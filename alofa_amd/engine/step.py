@@ -20,6 +20,7 @@ from .. import ops
 from ..cache.manager import CacheManager
 from ..errors import AlofaError, LostResults
 from .resident import ResidentLayers
+from .tapes import LayerTapes
 
 
 def _pow2_ceil(n: int) -> int:
@@ -95,6 +96,7 @@ class StepContext:
         self.token_store = fn.token_store
         self.watch = fn.watch
         self.resident = fn.resident
+        self.tapes = getattr(fn, "tapes", None)
         self.request_slots: Optional[torch.Tensor] = None   # int32 [entries] on the device: the request slot of every entry
         self.row_offsets: Optional[torch.Tensor] = None     # int32 [entries + 1] on the device: entry i owns the rows [i] .. [i+1]-1; None: one row each (decode graphs)
         self.want_slots: Optional[torch.Tensor] = None      # int32 [wanted rows] on the device: the request slot behind every wanted row
@@ -186,6 +188,7 @@ class StepFunction:
         self.graph_replays = 0
         # what must not move once steps run (position tables up to the context bound) is built now
         model.prepare(self.n_positions)
+        self.tapes = LayerTapes.of(model, cache)             # None, or which layers are alike
         self.resident = ResidentLayers.of(model, cache)      # None, or what runs the layers of small decode steps in one launch
 
     # ------------------------------------------------------------- scratch

@@ -57,6 +57,7 @@ class Model:
         self.head = build_part("head", spec.head, weights, rt, embedding=self.embedding)
         self.joins = [build_part("join", j, weights, rt) for j in spec.joins]
         self.order = list(spec.order)
+        self.descriptions = None      # (of the blocks, for engine/tapes.py)
         self.streams = int(spec.streams)
         if any(b.on_streams != bool(self.streams) for b in self.blocks) or (self.streams and self.joins):
             raise AlofaError("unsupported", "blocks on copies of the stream go with a model that keeps copies, and with no joins", f"streams={self.streams}")
@@ -135,8 +136,14 @@ class Model:
             read = self.blocks[self.order[0].layer].wants_normed(rows)
             normed = ctx.scratch("normed", tuple(hidden.shape), self.rt.dtype)
             ops.streams_step(stream, source=hidden, w_in=read.weights, norm=read.norm, out=normed, exact=self.rt.exact)
+        tapes = getattr(ctx, "tapes", None) if watch is None else None
+        tape = None      # (the launches of the last entry that others are alike, whether a norm was left for it, and what it left)
         for i, e in enumerate(self.order):
             block = self.blocks[e.layer]
+            if tapes is not None and tape is not None and tapes.source.get(i) == tape[0] and (normed is not None) == tape[2]:
+                tape[1].play(tapes.addresses(i))
+                normed = tape[3]
+                continue
             if e.join is not None:
                 self.joins[e.join].forward(ctx, hidden, first)
                 normed = None
@@ -155,6 +162,12 @@ class Model:
             then = (norm, ctx.scratch("normed", tuple(hidden.shape), self.rt.dtype)) if leaves else None
             if self.streams and nxt is None:
                 then = (self.sum_of_streams, hidden)
+            if tapes is not None and i in tapes.sources:
+                given = normed is not None
+                with tapes.note(i) as noted:
+                    normed = then[1] if block.forward(ctx, i, stream, normed, then) else None
+                tape = (i, noted, given, normed)
+                continue
             normed = then[1] if block.forward(ctx, i, stream, normed, then) else None
         return hidden
 

@@ -65,6 +65,10 @@ def _contig(name: str, t: torch.Tensor) -> torch.Tensor:
 
 class _Scope(threading.local):
     stream: Optional[int] = None
+    taping = False      # (tape_calls)
+
+    def __init__(self):
+        self.done = ctypes.c_int(0)      # where a product says whether it has seen to the norm behind it: memory that outlives the call, which a tape makes again
 
 
 _scope = _Scope()      # (a thread's own, as torch's current stream is)
@@ -110,17 +114,45 @@ def _native():
     return _binding
 
 
-def _answer(fn_name: str, *args) -> int:
-    """The entry's own answer. A parameter is a tensor (its memory), None (a null pointer), an integer or a float, as ``_ptr``, ``_I``, ``_L`` and ``_F`` leave them."""
+def _address(fn_name: str) -> int:
     address = _entries.get(fn_name)
     if address is None:
         address = _entries[fn_name] = ctypes.cast(getattr(load(), fn_name), ctypes.c_void_p).value
-    return _native().call(address, *args)
+    return address
+
+
+def _answer(fn_name: str, *args) -> int:
+    """The entry's own answer. A parameter is a tensor (its memory), None (a null pointer), an integer or a float, as ``_ptr``, ``_I``, ``_L`` and ``_F`` leave them."""
+    return _native().call(_address(fn_name), *args)
 
 
 def _call(fn_name: str, *args) -> None:
-    if _answer(fn_name, *args) != 0:
+    native = _native()
+    if (native.note if _scope.taping else native.call)(_address(fn_name), *args) != 0:
         raise AlofaError("invalid_argument", "kernel refused its arguments", load().alofa_last_error().decode())
+
+
+class tape_calls:
+    """Within the scope this thread's launches are noted; ``tape.play(addresses)`` makes them again for another layer. ``ranges``: (address, bytes) of the layer's own tensors: a parameter that lies in
+    one of them is moved to the same place of the other layer's, every other one stays as it was. Only for code whose work on the device is launches by way of ``_call`` with memory that outlives the scope."""
+
+    def __init__(self, ranges: tuple):
+        self._ranges, self._tape = ranges, None
+
+    def __enter__(self):
+        _native().tape()
+        _scope.taping = True
+        return self
+
+    def __exit__(self, kind, *exc):
+        _scope.taping = False
+        if kind is None:
+            self._tape = _native().taped(*self._ranges)
+        return False
+
+    def play(self, addresses: tuple) -> None:
+        if _native().play(self._tape, addresses) != 0:
+            raise AlofaError("invalid_argument", "kernel refused its arguments", load().alofa_last_error().decode())
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
@@ -441,7 +473,8 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[tor
         if kernel is None and then_rows is not None and then_rows.dtype is torch.bfloat16 and FUSE_NORMS and norm_rides_on_shares(M, N, K):
             kernel = "tiled"
         entry = _product_entry(kernel, M, N, K)
-        done = ctypes.c_int(0)
+        done = _scope.done
+        done.value = 0
         if entry == "alofa_gemm_mfma":
             ride = then_rows is not None and then_rows.dtype is torch.bfloat16 and FUSE_NORMS
             more = (then_w if ride else None, _F(then_eps), then_rows if ride else None, N, ctypes.addressof(done))

@@ -267,6 +267,10 @@ class GQAAttention(Mixer):
     def gives_normed(self):
         return self.b_o is None
 
+    @property
+    def repeatable(self):
+        return self.b_o is None and self.position.table(1) is not None      # (no sum and no rotation of torch's)
+
     def forward(self, ctx, entry, x, residual, norm=None, then=None, out=None):
         """``out`` (float32, the residual's shape): the mix is stored there instead of being added to the residual."""
         T = residual.shape[0]

@@ -59,6 +59,12 @@ class PreNormBlock(Block):
     def wants_normed(self, rows):
         return None if self.mixer.fuses_norm(self.norms[0], rows) else self.norms[0]
 
+    @property
+    def repeatable(self):
+        """Whether all that the block does on the device is launches of this package's kernels on its own tensors, its cache and buffers that the step keeps, chosen by sizes alone: another block like it
+        may then be run by making them again (``engine/tapes.py``)."""
+        return all(n.as_rmsnorm() is not None for n in self.norms) and all(getattr(p, "repeatable", False) for p in (self.mixer, self.feed_forward))
+
     def forward(self, ctx, entry, hidden, normed=None, then=None):
         """``normed``: the first norm's rows, where the block before has left them; ``then`` = (norm, rows): the norm
         the next block starts with, to be left in ``rows``. Returns whether that was done."""

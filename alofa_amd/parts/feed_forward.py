@@ -53,6 +53,7 @@ class SwiGLU(FeedForward):
                 and ops.can_fuse_norm(rows, self.w_gate, self.rt.dtype, swiglu=True))
 
     gives_normed = True
+    repeatable = True
 
     def forward(self, ctx, x, residual, norm=None, then=None, out=None):
         act = ctx.scratch("ff_act", (residual.shape[0], self.intermediate), self.rt.dtype)

@@ -1,0 +1,92 @@
+"""Layers that are alike: one layer's launches made again for the others."""
+import ctypes
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+import torch
+
+from alofa_amd.csrc import calls
+from alofa_amd.csrc.build import load_binding
+
+SOURCE = """
+#include <stdint.h>
+static int64_t seen[64];
+static int n;
+int64_t* places(void) { return seen; }
+int keep(int64_t a, float x, int64_t b, int64_t c, float y) { seen[n++] = a, seen[n++] = b, seen[n++] = c, seen[n++] = (int64_t)(x * 2), seen[n++] = (int64_t)(y * 2); return 0; }
+void forget(void) { n = 0; }
+int odd(int64_t a) { return (int)(a & 1); }
+"""
+
+
+@pytest.fixture(scope="module")
+def library(tmp_path_factory):
+    cc = shutil.which("gcc") or shutil.which("cc") or shutil.which("clang")
+    if cc is None:
+        pytest.skip("no C compiler")
+    d = tmp_path_factory.mktemp("tapes")
+    (d / "tapes.c").write_text(SOURCE)
+    subprocess.run([cc, "-O2", "-shared", "-fPIC", "-o", str(d / "tapes.so"), str(d / "tapes.c")], check=True)
+    return ctypes.CDLL(str(d / "tapes.so"))
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_calls_are_made_again_with_another_layers_addresses(library, native):
+    ways = load_binding() if native else calls
+    address = lambda name: ctypes.cast(getattr(library, name), ctypes.c_void_p).value      # noqa: E731
+    library.places.restype = ctypes.POINTER(ctypes.c_int64)
+    library.forget()
+    t = torch.zeros(4)
+    assert ways.note(address("keep"), 1, 0.5, 2, 3, 1.5) == 0      # (no tape is being written: a call like any other)
+    ways.tape()
+    assert ways.note(address("odd"), 7) == 1                       # (a call that failed is not made again)
+    assert ways.note(address("keep"), 1000, 2.5, 1099, None, 3.5) == 0
+    assert ways.note(address("keep"), 1100, 4.5, 2007, t, -1.5) == 0
+    tape = ways.taped((1000, 100), (2000, 8), (5000, 0))
+    for at in ((30, 70000, 0), (1 << 40, -5, 1)):
+        assert ways.play(tape, at) == 0
+    got = np.ctypeslib.as_array(library.places(), (64,))[:40].reshape(8, 5).tolist()
+    del tape
+    mem = t.data_ptr()
+    assert got[:7] == [[1, 2, 3, 1, 3], [1000, 1099, 0, 5, 7], [1100, 2007, mem, 9, -3],
+                       [30, 129, 0, 5, 7], [1100, 70007, mem, 9, -3], [1 << 40, (1 << 40) + 99, 0, 5, 7], [1100, 2, mem, 9, -3]]
+    with pytest.raises(RuntimeError):
+        ways.taped()
+    ways.tape()
+    ways.note(address("odd"), 8)
+    tape = ways.taped((8, 1))
+    assert ways.play(tape, (11,)) == 1      # (the first answer that is not zero)
+    with pytest.raises(ValueError):
+        ways.play(tape, ())
+
+
+MODEL = {"architectures": ["Qwen2ForCausalLM"], "model_type": "qwen2", "num_hidden_layers": 7, "hidden_size": 256, "num_attention_heads": 4, "num_key_value_heads": 2, "intermediate_size": 512,
+         "vocab_size": 500, "rope_theta": 10000.0, "rms_norm_eps": 1e-6, "tie_word_embeddings": True, "use_sliding_window": False, "max_position_embeddings": 2048}
+WINDOWS = {**MODEL, "use_sliding_window": True, "sliding_window": 40, "max_window_layers": 3}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("config", [MODEL, WINDOWS], ids=["alike", "two kinds of layers"])
+def test_steps_are_the_same_bits_with_and_without_tapes(tmp_path, config, dtype, monkeypatch):
+    from alofa_amd.engine import tapes
+    from alofa_amd.replay import Replayer
+    from alofa_amd.weights import write_random_model
+    write_random_model(config, tmp_path, seed=5)
+    rng = np.random.default_rng(3)
+    ids = lambda n: [int(x) for x in rng.integers(0, 500, n)]      # noqa: E731
+    # short prompts, a longer one, portions beside tokens that decode, and decode steps (which run once launch by launch and are then captured)
+    steps = [[("a", ids(5)), ("b", ids(33))], [("c", ids(150))], [("a", ids(1)), ("b", ids(7)), ("c", ids(90))], [("a", ids(1)), ("b", ids(1)), ("c", ids(1))]] + [[("a", ids(1)), ("b", ids(1)), ("c", ids(1))]] * 2
+    got = {}
+    for on in (False, True):
+        monkeypatch.setattr(tapes, "SWITCHED_ON", on)
+        r = Replayer(str(tmp_path), dtype, 512)
+        r.fn.resident = None
+        assert (r.fn.tapes is not None) == on
+        if on:
+            assert r.fn.tapes.source == ({i: 1 for i in range(2, 6)} if config is MODEL else {4: 3, 5: 3})
+        got[on] = [r.step({"step": k, "entries": [{"id": n, "tokens": t, "want": [len(t) - 1]} for n, t in s], "end": []}) for k, s in enumerate(steps)]
+    for a, b in zip(got[False], got[True]):
+        assert a.size and np.array_equal(a, b)
