@@ -25,12 +25,31 @@ namespace alofa {
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
+// What the kernel needs to take a decode step's projections as they come out of the product (kRope; one token a request): q then points to rows [queries | keys | values] not yet turned, one token
+// a request. Queries and the new key are turned here as rope_kv_write_kernel turns them (elementwise.hip: the same bits), the new key and value take their place among the cache's from registers, and
+// the wave that has their tile writes them to the token's slot. Needs d a multiple of 32: a channel and its partner, d / 2 on, lie in the same lane. us in captured runs, a launch for it / here, 14/2 heads of 64: one token of 128 keys 10.5 / 8.6,
+// eight of 60 7.9 / 6.5, of 250 12.4 / 11.1, three of 2,000 54.8 / 52.9.
+constexpr int kTurnedTiles = 6;      // heads of up to 96: beyond, the registers of a wave do not hold the new token beside the rest
+struct ExactRope {
+  const float *cos_t, *sin_t;      // [position, d / 2]
+  const int64_t* slots;
+  float *k_cache, *v_cache;
+};
+
+__device__ __forceinline__ void turn_quads(float4& lo, float4& hi, float4 c, float4 s) {
+#pragma clang fp contract(off)
+  const float4 a = lo, b = hi;
+  lo = make_float4(a.x * c.x - b.x * s.x, a.y * c.y - b.y * s.y, a.z * c.z - b.z * s.z, a.w * c.w - b.w * s.w);
+  hi = make_float4(b.x * c.x + a.x * s.x, b.y * c.y + a.y * s.y, b.z * c.z + a.z * s.z, b.w * c.w + a.w * s.w);
+}
+
 // NT = d / 16, NW waves; blockIdx.y = key head * chunks + chunk of up to 16 heads of its group
-template <int NT, int NW>
+template <int NT, int NW, bool kRope>
 __global__ void __launch_bounds__(64 * NW) attention_exact_kernel(
     float* __restrict__ out, int64_t out_stride, const float* __restrict__ q, int64_t q_stride, const float* __restrict__ k_cache,
     const float* __restrict__ v_cache, const int32_t* __restrict__ block_table, int max_blocks, const int32_t* __restrict__ req_of_token,
-    const int32_t* __restrict__ positions, int heads, int kv_heads, int block_size, int window, float scale) {
+    const int32_t* __restrict__ positions, int heads, int kv_heads, int block_size, int window, float scale, ExactRope rope) {
+  static_assert(!kRope || NT % 2 == 0, "a channel and its partner in the same lane");
   constexpr int d = NT * 16;
   __shared__ double sums[NW][16][d + 1];      // per wave and head: the channels' sums, then the weights'
   __shared__ float maxima[NW][16];
@@ -47,6 +66,30 @@ __global__ void __launch_bounds__(64 * NW) attention_exact_kernel(
   for (int i = 0; i < NT; ++i)
     qf[i] = head_ok ? *reinterpret_cast<const float4*>(q + static_cast<int64_t>(t) * q_stride + static_cast<int64_t>(hk * group + h0 + r) * d + i * 16 + g * 4)
                     : make_float4(0.f, 0.f, 0.f, 0.f);
+  float4 new_k[kRope ? NT : 1];      // the new token's key (this lane's channels, as of a query) and value (channels 16 i + r)
+  float new_v[kRope ? NT : 1];
+  if constexpr (kRope) {
+    const float* k_row = q + static_cast<int64_t>(t) * q_stride + static_cast<int64_t>(heads + hk) * d;
+    const float* v_row = k_row + static_cast<int64_t>(kv_heads) * d;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) new_k[i] = *reinterpret_cast<const float4*>(k_row + i * 16 + g * 4), new_v[i] = v_row[i * 16 + r];
+#pragma unroll
+    for (int i = 0; i < NT / 2; ++i) {
+      const int64_t at = static_cast<int64_t>(p) * (d / 2) + i * 16 + g * 4;
+      const float4 c = *reinterpret_cast<const float4*>(rope.cos_t + at), sn = *reinterpret_cast<const float4*>(rope.sin_t + at);
+      turn_quads(qf[i], qf[i + NT / 2], c, sn);
+      turn_quads(new_k[i], new_k[i + NT / 2], c, sn);
+    }
+    // (first of all, so that the step behind this one does not wait for it; no wave reads the slot)
+    if (h0 == 0 && wave == ((p >> 4) - (lo >> 4)) % NW) {
+      const int64_t page = rope.slots[t] / block_size, off = rope.slots[t] % block_size;
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        if (r == 0) *reinterpret_cast<float4*>(rope.k_cache + ((page * kv_heads + hk) * block_size + off) * d + i * 16 + g * 4) = new_k[i];
+        if (g == 0) rope.v_cache[((page * kv_heads + hk) * d + i * 16 + r) * block_size + off] = new_v[i];
+      }
+    }
+  }
   f64x4 o[NT];
 #pragma unroll
   for (int i = 0; i < NT; ++i) o[i] = f64x4{0, 0, 0, 0};
@@ -66,6 +109,21 @@ __global__ void __launch_bounds__(64 * NW) attention_exact_kernel(
     for (int i = 0; i < NT; ++i) kf[i] = *reinterpret_cast<const float4*>(kr + i * 16);
 #pragma unroll
     for (int i = 0; i < NT; ++i) vf[i] = *reinterpret_cast<const float4*>(vr + static_cast<int64_t>(i) * 16 * block_size);
+    if constexpr (kRope) {      // (what the cache holds at the new token's place is not looked at)
+      if (tile == p >> 4) {     // (uniform over the wave)
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+          if (key == p) kf[i] = new_k[i];
+          if (key4 == (p & ~3)) {
+            const int at4 = p & 3;
+            vf[i].x = at4 == 0 ? new_v[i] : vf[i].x;
+            vf[i].y = at4 == 1 ? new_v[i] : vf[i].y;
+            vf[i].z = at4 == 2 ? new_v[i] : vf[i].z;
+            vf[i].w = at4 == 3 ? new_v[i] : vf[i].w;
+          }
+        }
+      }
+    }
     f64x4 s = {0, 0, 0, 0};
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
@@ -131,12 +189,19 @@ __global__ void __launch_bounds__(64 * NW) attention_exact_kernel(
 template <int NT>
 static void launch_attention_exact(float* out, int64_t out_stride, const float* q, int64_t q_stride, const float* k_cache, const float* v_cache,
                                    const int32_t* block_table, int max_blocks, const int32_t* req_of_token, const int32_t* positions, int tokens, int heads,
-                                   int kv_heads, int block_size, int window, float scale, hipStream_t stream) {
+                                   int kv_heads, int block_size, int window, float scale, const ExactRope& rope, hipStream_t stream) {
   // (the number of waves, which decides whose running maximum a key's weight is taken against, follows from the head size alone: as many as the registers and LDS allow)
   constexpr int kWaves = NT <= 8 ? 8 : 4;
   dim3 grid(tokens, kv_heads * ((heads / kv_heads + 15) / 16));
-  attention_exact_kernel<NT, kWaves><<<grid, 64 * kWaves, 0, stream>>>(out, out_stride, q, q_stride, k_cache, v_cache, block_table, max_blocks, req_of_token, positions, heads, kv_heads,
-                                                                       block_size, window, scale);
+  if constexpr (NT % 2 == 0 && NT <= kTurnedTiles) {
+    if (rope.cos_t) {
+      attention_exact_kernel<NT, kWaves, true><<<grid, 64 * kWaves, 0, stream>>>(out, out_stride, q, q_stride, k_cache, v_cache, block_table, max_blocks, req_of_token, positions, heads, kv_heads,
+                                                                                 block_size, window, scale, rope);
+      return;
+    }
+  }
+  attention_exact_kernel<NT, kWaves, false><<<grid, 64 * kWaves, 0, stream>>>(out, out_stride, q, q_stride, k_cache, v_cache, block_table, max_blocks, req_of_token, positions, heads, kv_heads,
+                                                                              block_size, window, scale, rope);
 }
 
 }  // namespace alofa
@@ -150,18 +215,22 @@ extern "C" int alofa_attention_exact_takes(const void* q, int64_t q_stride, cons
   return d > 0 && d <= 256 && d % 16 == 0 && block_size > 0 && block_size % 4 == 0 && q_stride % 4 == 0 && aligned(q) && aligned(k_cache) && aligned(v_cache);
 }
 
+// cos_t, sin_t, slots: null for queries that are turned and a cache that is written already; else see ExactRope.
 extern "C" int alofa_attention_exact(float* out, int64_t out_stride, const float* q, int64_t q_stride, const float* k_cache, const float* v_cache,
                                      const int32_t* block_table, int max_blocks, const int32_t* req_of_token, const int32_t* positions, int tokens, int heads,
-                                     int kv_heads, int d, int block_size, int window, float scale, hipStream_t stream) {
+                                     int kv_heads, int d, int block_size, int window, float scale, const float* cos_t, const float* sin_t, const int64_t* slots, hipStream_t stream) {
   ALOFA_REQUIRE(tokens > 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0,
                 "attention: tokens=%d heads=%d kv_heads=%d (kv_heads must divide heads)", tokens, heads, kv_heads);
   ALOFA_REQUIRE(alofa_attention_exact_takes(q, q_stride, k_cache, v_cache, d, block_size), "attention: head size %d, pages of %d or the operands' places do not fit", d, block_size);
   ALOFA_REQUIRE(max_blocks > 0 && window >= 0, "attention: max_blocks=%d window=%d", max_blocks, window);
+  ALOFA_REQUIRE(!cos_t || (sin_t && slots && d % 32 == 0 && d <= 16 * kTurnedTiles && q_stride >= static_cast<int64_t>(heads + 2 * kv_heads) * d && reinterpret_cast<uintptr_t>(cos_t) % 16 == 0 && reinterpret_cast<uintptr_t>(sin_t) % 16 == 0),
+                "attention: the form that turns the new token takes sin, slots, rows of queries, keys and values, a head size in steps of 32 up to 96 (%d), aligned tables", d);
+  const ExactRope rope{cos_t, sin_t, slots, const_cast<float*>(k_cache), const_cast<float*>(v_cache)};
   switch (d / 16) {
 #define ALOFA_EXACT_HEAD(NT)                                                                                                                                      \
   case NT:                                                                                                                                                        \
     launch_attention_exact<NT>(out, out_stride, q, q_stride, k_cache, v_cache, block_table, max_blocks, req_of_token, positions, tokens, heads, kv_heads,        \
-                               block_size, window, scale, stream);                                                                                               \
+                               block_size, window, scale, rope, stream);                                                                                               \
     break;
     ALOFA_EXACT_HEAD(1) ALOFA_EXACT_HEAD(2) ALOFA_EXACT_HEAD(3) ALOFA_EXACT_HEAD(4) ALOFA_EXACT_HEAD(5) ALOFA_EXACT_HEAD(6) ALOFA_EXACT_HEAD(7) ALOFA_EXACT_HEAD(8)
     ALOFA_EXACT_HEAD(9) ALOFA_EXACT_HEAD(10) ALOFA_EXACT_HEAD(11) ALOFA_EXACT_HEAD(12) ALOFA_EXACT_HEAD(13) ALOFA_EXACT_HEAD(14) ALOFA_EXACT_HEAD(15) ALOFA_EXACT_HEAD(16)

@@ -771,8 +771,9 @@ def paged_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v
                     block_table: torch.Tensor, req_of_token: torch.Tensor, positions: torch.Tensor,
                     heads: int, kv_heads: int, d: int, window: Optional[int], scale: float, exact: bool,
                     max_q_len: Optional[int] = None, max_context: Optional[int] = None,
-                    scratch: Optional[torch.Tensor] = None) -> None:
-    """out[t] = attention of query token t (q [T, >= heads*d] rows, heads packed)
+                    scratch: Optional[torch.Tensor] = None, rope: Optional[tuple] = None) -> None:
+    """``rope`` = (cos, sin, slots) on the exact path (``can_turn_exactly``), for steps of one token a request: ``q`` holds rows [queries | keys | values] as they are projected; queries and keys are turned, and
+    keys and values written to their slots, in the same launch (``rope_kv_write``'s bits; the rows stay as they are). out[t] = attention of query token t (q [T, >= heads*d] rows, heads packed)
     over the keys lo..positions[t] of its request's pages. ``max_q_len`` (most
     query tokens of one request in this step) and ``max_context`` (longest
     context) only choose the kernel and its launch shape; with them the caller
@@ -798,11 +799,30 @@ def paged_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v
         return
     if exact and q.dtype is torch.float32 and _answer("alofa_attention_exact_takes", _ptr(q), _L(_rows("q", q)), _ptr(k_cache), _ptr(v_cache), _I(d), _I(bs)):
         _call("alofa_attention_exact", _ptr(out), _L(_rows("out", out)), _ptr(q), _L(_rows("q", q)), _ptr(k_cache), _ptr(v_cache), _ptr(block_table),
-              _I(block_table.shape[1]), _ptr(req_of_token), _ptr(positions), _I(T), _I(heads), _I(kv_heads), _I(d), _I(bs), _I(int(window or 0)), _F(scale), _stream())
+              _I(block_table.shape[1]), _ptr(req_of_token), _ptr(positions), _I(T), _I(heads), _I(kv_heads), _I(d), _I(bs), _I(int(window or 0)), _F(scale),
+              *_turned_here(rope, q, positions, heads, kv_heads, d), _stream())
         return
+    if rope is not None:
+        raise AlofaError("unsupported", "the kernel for any sizes takes rows that are turned", f"heads={heads} d={d} page={bs}")
     _call("alofa_attention_simple", _ptr(out), _L(_rows("out", out)), _ptr(q), _L(_rows("q", q)), _ptr(k_cache), _ptr(v_cache),
           _I(dtype_code(q)), _ptr(block_table), _I(block_table.shape[1]), _ptr(req_of_token), _ptr(positions), _I(T),
           _I(heads), _I(kv_heads), _I(d), _I(bs), _I(int(window or 0)), _F(scale), _I(int(exact)), _stream())
+
+
+def can_turn_exactly(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, d: int) -> bool:
+    """Whether the exact path's attention takes a decode step's rows as they are projected (``paged_attention(rope=)``)."""
+    return q.dtype is torch.float32 and d % 32 == 0 and d <= 96 and bool(_answer("alofa_attention_exact_takes", q, _rows("q", q), k_cache, v_cache, d, k_cache.shape[2]))
+
+
+def _turned_here(rope: Optional[tuple], q: torch.Tensor, positions: torch.Tensor, heads: int, kv_heads: int, d: int) -> tuple:
+    if rope is None:
+        return None, None, None
+    cos, sin, slots = rope
+    _angles(positions, cos, sin, q.shape[0])
+    _gpu("slots", slots, torch.int64, 1), _contig("slots", slots)
+    if slots.shape[0] != q.shape[0] or cos.shape[1] != d // 2 or q.shape[1] < (heads + 2 * kv_heads) * d:
+        raise AlofaError("shape_mismatch", "rows of queries, keys and values, a slot each, tables [positions, d / 2]", f"q={tuple(q.shape)} slots={tuple(slots.shape)} cos={tuple(cos.shape)}")
+    return cos, sin, slots
 
 
 def _attention_operands(out, q, k_cache, v_cache, block_table, heads, kv_heads, d):

@@ -107,7 +107,9 @@ def paged_attend(ctx, entry, qkv, attn, heads, kv_heads, d, window, scale, posit
     # one new token per request: the decode kernel rotates it and writes its cache slot itself
     fused = (not exact and pow2_pages and mfma_heads and kv.owner and ctx.max_q_len == 1 and plan.long_runs is None
              and ops.can_fuse_rope_into_decode(d))
-    if fused:
+    # (the exact path likewise)
+    turned = exact and kv.owner and ctx.max_q_len == 1 and plan.long_runs is None and ops.can_turn_exactly(qkv, kv.k, kv.v, d)
+    if fused or turned:
         pass
     elif kv.owner:
         ops.rope_kv_write(qkv, cos, sin, ctx.positions, heads, kv_heads, d, kv.slots, kv.k, kv.v)
@@ -115,7 +117,7 @@ def paged_attend(ctx, entry, qkv, attn, heads, kv_heads, d, window, scale, posit
         ops.rope_kv_write(qkv, cos, sin, ctx.positions, heads, kv_heads, d)
     if exact or not pow2_pages or not mfma_heads or (plan.long_runs is not None and not fast_prefill):
         # the exact path, and page or head sizes the bfloat16 kernels are not built for
-        ops.paged_attention(attn, qkv, kv.k, kv.v, kv.block_table, ctx.req_of_token, ctx.positions, *common, exact)
+        ops.paged_attention(attn, qkv, kv.k, kv.v, kv.block_table, ctx.req_of_token, ctx.positions, *common, exact, rope=(cos, sin, kv.slots) if turned else None)
     else:
         if plan.long_runs is not None and plan.in_tall_blocks(heads, kv_heads, d, kv.k.shape[2], scale, window):      # portions of prompts, many rows
             ops.attention_tall(attn, qkv, kv.k, kv.v, kv.block_table, ctx.memo("gqa_attention.tall_runs", plan.tall_runs), *common)

@@ -207,3 +207,39 @@ def test_exact_products_name_the_operand_that_is_not_float32():
     for operands, name in (((out, h, f, f), "operand=a"), ((out, f, h, h), "operand=w_gate"), ((out.bfloat16(), f, f, f), "operand=out")):
         with pytest.raises(AlofaError, match=name):
             ops().gemm_swiglu(*operands, exact=True)
+
+
+# the new token at a tile's, a page's and a quad's first and last place, alone, behind a window; more heads to a key head than a tile holds
+@pytest.mark.parametrize("heads,kv_heads,d,bs", [(14, 2, 64, 16), (20, 1, 32, 4), (4, 4, 96, 16), (6, 2, 64, 12)])
+@pytest.mark.parametrize("window", [None, 19])
+def test_a_decode_step_of_the_exact_path_turns_its_tokens(heads, kv_heads, d, bs, window):
+    positions = [0, 1, 3, 4, 15, 16, 17, 31, 63, 64, 130, 255]
+    n = len(positions)
+    gen = torch.Generator(device=DEV).manual_seed(heads)
+    draw = lambda *s: torch.randn(s, generator=gen, device=DEV)      # noqa: E731
+    per = [p // bs + 1 for p in positions]
+    pages = torch.randperm(sum(per), generator=gen, device=DEV).to(torch.int32)
+    table = torch.full((n, max(per)), -1, dtype=torch.int32, device=DEV)
+    used, slots = 0, []
+    for i, p in enumerate(positions):
+        mine = pages[used:used + per[i]]
+        lowest = 0 if window is None else max(0, p - window + 1)
+        table[i, :per[i]] = torch.where((torch.arange(per[i], device=DEV) + 1) * bs <= lowest, -1, mine)
+        slots.append(int(mine[-1]) * bs + p % bs)
+        used += per[i]
+    kc, vc = draw(sum(per), kv_heads, bs, d), draw(sum(per), kv_heads, d, bs)
+    for slot in slots:      # (what stands at a new token's place, and behind it, is not data)
+        kc[slot // bs, :, slot % bs:], vc[slot // bs, :, :, slot % bs:] = float("nan"), float("nan")
+    qkv, cos, sin = draw(n, (heads + 2 * kv_heads) * d), draw(300, d // 2), draw(300, d // 2)
+    to = lambda x, t=torch.int32: torch.tensor(x, dtype=t, device=DEV)      # noqa: E731
+    pos, req, slots = to(positions), to(range(n)), to(slots, torch.int64)
+    got = []
+    for turned in (False, True):
+        rows, k, v, out = qkv.clone(), kc.clone(), vc.clone(), torch.empty(n, heads * d, device=DEV)
+        if not turned:
+            ops().rope_kv_write(rows, cos, sin, pos, heads, kv_heads, d, slots, k, v)
+        assert ops().can_turn_exactly(rows, k, v, d)
+        ops().paged_attention(out, rows, k, v, table, req, pos, heads, kv_heads, d, window, d ** -0.5, True, rope=(cos, sin, slots) if turned else None)
+        got.append((out, k.nan_to_num(7.0), v.nan_to_num(7.0)))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and bool(torch.isfinite(got[0][0]).all())
+    assert torch.equal(rows, qkv)
