@@ -286,4 +286,5 @@ def load() -> ctypes.CDLL:
             raise AlofaError("not_initialized", "the HIP library cannot be loaded", f"path={path} reason={e}") from None
         _lib.alofa_last_error.restype = ctypes.c_char_p
         _lib.alofa_gemm_exact_parts.restype = ctypes.c_int64
+        _lib.alofa_gemm_exact_norm_parts.restype = ctypes.c_int64
     return _lib

@@ -191,13 +191,13 @@ __global__ void __launch_bounds__(64 * NW) exact_rows_kernel(float* __restrict__
   }
 }
 
-// A block of WM x (4 / WM) waves, each 32 rows x 32 weight rows; kMats = 2: the weight rows of a wave are 16 of gate and the same 16 of up.
+// A block of WM x (4 / WM) waves, each 16 RF rows x 32 weight rows; kMats = 2: the weight rows of a wave are 16 of gate and the same 16 of up.
 // kFold: the block takes all chains and adds them up; else chain blockIdx.z, whose sums go to parts, [chain][M][N], and the epilogue is the second launch's.
-template <int WM, int kMats, int kEpilogue, bool kVec, bool kFold>
+template <int WM, int RF, int kMats, int kEpilogue, bool kVec, bool kFold>
 __global__ void __launch_bounds__(256, WM == 2 && !kFold ? 3 : 2) exact_tile_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ A, int64_t lda,
                                                          const float* __restrict__ W, const float* __restrict__ W2, int64_t ldw,
                                                          const float* __restrict__ bias, double* __restrict__ parts, Cut cut, int M, int N, int K, int gelu) {
-  constexpr int WN = 4 / WM, BM = 32 * WM, BW = 32 * WN, BK = 32, kPad = 4;
+  constexpr int WN = 4 / WM, BM = 16 * RF * WM, BW = 32 * WN, BK = 32, kPad = 4;
   constexpr int kOwn = 32 / kMats;                     // outputs of a wave along N
   __shared__ __attribute__((aligned(16))) float As[2][BM][BK + kPad], Ws[2][BW][BK + kPad];      // (as doubles, widened once as they are brought: 174 us where this took 169)
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
@@ -218,9 +218,9 @@ __global__ void __launch_bounds__(256, WM == 2 && !kFold ? 3 : 2) exact_tile_ker
   const int k_own = threadIdx.x % 8 * 4;      // (threadIdx.x + 256 i has the same place in its row)
   const int k_begin = kFold ? 0 : blockIdx.z * cut.length, k_end = kFold ? K : min(k_begin + cut.length, K);
   static_assert(kFold || kMats == 1, "gate and up meet in the block");
-  f64x4 acc[2][2], sum[2][2];      // [rows of A][weight rows]: of this chain, of the chains before (kFold)
+  f64x4 acc[RF][2], sum[RF][2];      // [rows of A][weight rows]: of this chain, of the chains before (kFold)
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < RF; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = sum[i][j] = f64x4{0, 0, 0, 0};
   if constexpr (kFold && kMats == 1)
@@ -230,12 +230,12 @@ __global__ void __launch_bounds__(256, WM == 2 && !kFold ? 3 : 2) exact_tile_ker
         const int n = n0 + wn * 32 + j * 16 + r;
         const double b = n < N ? bias[n] : 0.0;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) sum[i][j] = f64x4{b, b, b, b};
+        for (int i = 0; i < RF; ++i) sum[i][j] = f64x4{b, b, b, b};
       }
     }
   auto end_chain = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < RF; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j) sum[i][j] += acc[i][j], acc[i][j] = f64x4{0, 0, 0, 0};
   };
@@ -260,14 +260,13 @@ __global__ void __launch_bounds__(256, WM == 2 && !kFold ? 3 : 2) exact_tile_ker
     constexpr int x = decltype(set)::value;
 #pragma unroll
     for (int q = 0; q < BK / 16; ++q) {
-      float4 a[2], w[2];
+      float4 a[RF], w[2];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        a[i] = *reinterpret_cast<const float4*>(&As[x][wm * 32 + i * 16 + r][q * 16 + g * 4]);
-        w[i] = *reinterpret_cast<const float4*>(&Ws[x][wn * 32 + i * 16 + r][q * 16 + g * 4]);
-      }
+      for (int i = 0; i < RF; ++i) a[i] = *reinterpret_cast<const float4*>(&As[x][(wm * RF + i) * 16 + r][q * 16 + g * 4]);
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < 2; ++i) w[i] = *reinterpret_cast<const float4*>(&Ws[x][wn * 32 + i * 16 + r][q * 16 + g * 4]);
+#pragma unroll
+      for (int i = 0; i < RF; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = fma_quad(a[i], w[j], acc[i][j]);
     }
@@ -325,10 +324,10 @@ __global__ void __launch_bounds__(256, WM == 2 && !kFold ? 3 : 2) exact_tile_ker
   end_chain();      // (the last one; zeros where its end was a pair's)
   // D: rows of A 4 v + g, weight row r
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < RF; ++i)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int m = m0 + wm * 32 + i * 16 + 4 * v + g;
+      const int m = m0 + (wm * RF + i) * 16 + 4 * v + g;
       if (m >= M) continue;
       if constexpr (kMats == 2) {
         const int n = n0 + wn * 16 + r;
@@ -362,9 +361,67 @@ __global__ void __launch_bounds__(256) exact_sum_kernel(float* __restrict__ out,
   put<kEpilogue>(out + i / N * ldo + n, s);
 }
 
+// The same behind a product that adds to the residual stream, and the RMSNorm that follows: a block per row adds its chains up, writes the stream's new row and leaves it normed (w, eps, float64) in
+// `normed` [M, N] rows, the bits that exact_sum_kernel and rmsnorm_kernel leave one behind the other (the squares in that kernel's order). K4: groups of four columns a thread, N at most 1,024 K4.
+// A launch less; us in captured runs, launch by launch / this: 896 x 4,864 against one row 9.8 / 9.1, eight 10.9 / 10.0, 64 22.5 / 20.7, 450 91 / 89; 896 x 896 against 8 rows 7.6 / 7.5
+// (which is cut over blocks for it), 64 13.2 / 11.9, 450 32.2 / 30.3.
+template <int K4>
+__global__ void __launch_bounds__(256) exact_sum_norm_kernel(float* __restrict__ out, int64_t ldo, const double* __restrict__ parts, const float* __restrict__ w, float eps,
+                                                             float* __restrict__ normed, int64_t rows_out, int M, int N, int chains) {
+  __shared__ double scratch[4];
+  const int m = blockIdx.x, groups = N / 4;
+  const int64_t all = static_cast<int64_t>(M) * N;
+  float* row = out + static_cast<int64_t>(m) * ldo;
+  float4 xs[K4], ws[K4];
+  double ss = 0;
+#pragma unroll
+  for (int i = 0; i < K4; ++i) {
+    const int g = threadIdx.x + 256 * i, at = 4 * (g < groups ? g : 0);      // (every thread loads; what lies beyond the row is cleared)
+    const double2* p = reinterpret_cast<const double2*>(parts + static_cast<int64_t>(m) * N + at);
+    const float4 old = *reinterpret_cast<const float4*>(row + at);
+    ws[i] = *reinterpret_cast<const float4*>(w + at);
+    double2 lo[kMaxChains], hi[kMaxChains];
+#pragma unroll
+    for (int x = 0; x < kMaxChains; ++x) lo[x] = p[(x < chains ? x : 0) * (all / 2)], hi[x] = p[(x < chains ? x : 0) * (all / 2) + 1];
+    double a = 0, b = 0, c = 0, d = 0;
+#pragma unroll
+    for (int x = 0; x < kMaxChains; ++x)
+      if (x < chains) a += lo[x].x, b += lo[x].y, c += hi[x].x, d += hi[x].y;
+    xs[i] = g < groups ? make_float4(old.x + static_cast<float>(a), old.y + static_cast<float>(b), old.z + static_cast<float>(c), old.w + static_cast<float>(d)) : make_float4(0.f, 0.f, 0.f, 0.f);
+    if (g < groups) *reinterpret_cast<float4*>(row + at) = xs[i];
+  }
+#pragma unroll
+  for (int i = 0; i < K4; ++i) {
+    const double a = xs[i].x, b = xs[i].y, c = xs[i].z, d = xs[i].w;
+    ss += a * a;
+    ss += b * b;
+    ss += c * c;
+    ss += d * d;
+  }
+  ss = block_sum<double, 256>(ss, scratch);
+  const double scale = 1.0 / sqrt(ss / static_cast<double>(N) + static_cast<double>(eps));
+  float* dst = normed + static_cast<int64_t>(m) * rows_out;
+#pragma unroll
+  for (int i = 0; i < K4; ++i) {
+    const int g = threadIdx.x + 256 * i;
+    if (g < groups)
+      *reinterpret_cast<float4*>(dst + 4 * g) = make_float4(static_cast<float>(static_cast<double>(xs[i].x) * scale * static_cast<double>(ws[i].x)), static_cast<float>(static_cast<double>(xs[i].y) * scale * static_cast<double>(ws[i].y)),
+                                                            static_cast<float>(static_cast<double>(xs[i].z) * scale * static_cast<double>(ws[i].z)), static_cast<float>(static_cast<double>(xs[i].w) * scale * static_cast<double>(ws[i].w)));
+  }
+}
+
 // Up to 16 rows: chains a block takes. Four where the blocks of 16 weight rows are fewer than half the compute units and the chains more than a block's eight
 // waves, else all of them.
-static int chains_per_block(int N, const Cut& cut) { return cut.count > 8 && (N + 15) / 16 * 2 < compute_units() ? 4 : cut.count; }
+// With a norm behind the sum there is a second launch either way: blocks of four chains from five chains on.
+static int chains_per_block(int N, const Cut& cut, bool norm) { return cut.count > (norm ? 4 : 8) && (N + 15) / 16 * 2 < compute_units() ? 4 : cut.count; }
+
+// The norm behind a product (null weights: none).
+struct ExactNorm {
+  const float* w;
+  float eps;
+  float* rows;
+  int64_t ld;
+};
 
 // More rows: whether the chains are dealt out over blocks, for the least time of the compute unit that has the most blocks: 35.5 ns a k of a block (30 of them its SIMDs'
 // matrix cores) and some 0.5 us a block, a twentieth more with one block to a compute unit, and for the second launch 4 us and 0.7 us a million sums.
@@ -384,8 +441,14 @@ static int rows_at_once(int M, int N, const Cut& cut) {
 }
 
 template <int kEpilogue>
-static void launch_exact_sum(float* out, int64_t ldo, const double* parts, const float* bias, int M, int N, int chains, hipStream_t stream) {
+static void launch_exact_sum(float* out, int64_t ldo, const double* parts, const float* bias, int M, int N, int chains, const ExactNorm& norm, hipStream_t stream) {
   const int64_t all = static_cast<int64_t>(M) * N;
+  if (norm.w) {      // (N a multiple of four, aligned rows: alofa_gemm_exact_norm sees to it)
+    if (N <= 1024) exact_sum_norm_kernel<1><<<M, 256, 0, stream>>>(out, ldo, parts, norm.w, norm.eps, norm.rows, norm.ld, M, N, chains);
+    else if (N <= 2048) exact_sum_norm_kernel<2><<<M, 256, 0, stream>>>(out, ldo, parts, norm.w, norm.eps, norm.rows, norm.ld, M, N, chains);
+    else exact_sum_norm_kernel<4><<<M, 256, 0, stream>>>(out, ldo, parts, norm.w, norm.eps, norm.rows, norm.ld, M, N, chains);
+    return;
+  }
   exact_sum_kernel<kEpilogue><<<static_cast<unsigned>((all + 255) / 256), 256, 0, stream>>>(out, ldo, parts, bias, M, N, chains);
 }
 
@@ -393,12 +456,12 @@ static void launch_exact_sum(float* out, int64_t ldo, const double* parts, const
 // often (8 rows, 151,936 x 896: 113 us; four tiles 130, eight waves 143).
 template <int kMats, int kEpilogue, bool kVec>
 static int launch_exact_rows(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, const float* W2, int64_t ldw, const float* bias,
-                             double* parts, int M, int N, int K, int gelu, hipStream_t stream) {
+                             double* parts, int M, int N, int K, int gelu, const ExactNorm& norm, hipStream_t stream) {
   const Cut cut = cut_of(K);
   const int tiles = (N + 15) / 16;
-  if (kMats == 1 && chains_per_block(N, cut) < cut.count) {
+  if (kMats == 1 && chains_per_block(N, cut, norm.w != nullptr) < cut.count) {
     exact_rows_kernel<4, 1, 1, kEpilogue, kVec><<<dim3(tiles, (cut.count + 3) / 4), 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, parts, cut, 4, M, N, K, gelu);
-    launch_exact_sum<kEpilogue>(out, ldo, parts, bias, M, N, cut.count, stream);
+    launch_exact_sum<kEpilogue>(out, ldo, parts, bias, M, N, cut.count, norm, stream);
   } else if (kMats == 1 && tiles >= 16 * compute_units()) {
     exact_rows_kernel<4, 2, 1, kEpilogue, kVec><<<(tiles + 2 - 1) / 2, 64 * 4, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, nullptr, cut, cut.count, M, N, K, gelu);
   } else {
@@ -407,10 +470,10 @@ static int launch_exact_rows(float* out, int64_t ldo, const float* A, int64_t ld
   return check_launch("gemm_exact_rows");
 }
 
-template <int WM, int kMats, int kEpilogue, bool kVec>
+template <int WM, int RF, int kMats, int kEpilogue, bool kVec>
 static int launch_exact_tile(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, const float* W2, int64_t ldw, const float* bias,
-                             double* parts, int M, int N, int K, int gelu, hipStream_t stream) {
-  constexpr int BM = 32 * WM, kOut = 32 * (4 / WM) / kMats;
+                             double* parts, int M, int N, int K, int gelu, const ExactNorm& norm, hipStream_t stream) {
+  constexpr int BM = 16 * RF * WM, kOut = 32 * (4 / WM) / kMats;
   const Cut cut = cut_of(K);
   if constexpr (kMats == 1) {
     if (chains_apart(M, N, K, cut)) {
@@ -418,30 +481,43 @@ static int launch_exact_tile(float* out, int64_t ldo, const float* A, int64_t ld
       for (int m = 0; m < M; m += at_once) {
         const int rows = std::min(at_once, M - m);
         float* dst = out + static_cast<int64_t>(m) * ldo;
-        exact_tile_kernel<WM, 1, kEpilogue, kVec, false><<<dim3((N + kOut - 1) / kOut, (rows + BM - 1) / BM, cut.count), 256, 0, stream>>>(
+        exact_tile_kernel<WM, RF, 1, kEpilogue, kVec, false><<<dim3((N + kOut - 1) / kOut, (rows + BM - 1) / BM, cut.count), 256, 0, stream>>>(
             nullptr, 0, A + static_cast<int64_t>(m) * lda, lda, W, W2, ldw, bias, parts, cut, rows, N, K, gelu);
-        launch_exact_sum<kEpilogue>(dst, ldo, parts, bias, rows, N, cut.count, stream);
+        launch_exact_sum<kEpilogue>(dst, ldo, parts, bias, rows, N, cut.count, norm.w ? ExactNorm{norm.w, norm.eps, norm.rows + static_cast<int64_t>(m) * norm.ld, norm.ld} : norm, stream);
       }
       return check_launch("gemm_exact_tile");
     }
   }
-  exact_tile_kernel<WM, kMats, kEpilogue, kVec, true><<<dim3((N + kOut - 1) / kOut, (M + BM - 1) / BM), 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, nullptr, cut, M, N, K, gelu);
+  exact_tile_kernel<WM, RF, kMats, kEpilogue, kVec, true><<<dim3((N + kOut - 1) / kOut, (M + BM - 1) / BM), 256, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, nullptr, cut, M, N, K, gelu);
   return check_launch("gemm_exact_tile");
+}
+
+// Gate and up of more than 64 rows: whether tiles of 96 rows come out sooner than those of 64. A compute unit takes a round's time for each of its blocks, whether they lie side by side or not, 31.5 us
+// a block of 64 rows and 47 of 96 against K of 896 (56 of whose registers are kept in memory), so it is the whole rounds that count: 9,728 x 896 against 66 to 96 rows (304 blocks of 64 rows, 152 of 96)
+// 64.9 / 51, 385 to 480 (1,064 and more, 760) 154 / 142; 130 (456, 304) 65 / 93, 300 (760, 608) 96 / 142.
+static bool taller_tiles(int M, int N) {
+  if (M <= 64) return false;
+  const int64_t columns = (N + 31) / 32, cus = compute_units();
+  auto rounds = [&](int rows) { return (columns * ((M + rows - 1) / rows) + cus - 1) / cus; };
+  return 47 * rounds(96) < 31.5 * rounds(64);
 }
 
 template <int kMats, int kEpilogue>
 static int launch_exact(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, const float* W2, int64_t ldw, const float* bias,
-                        double* parts, int M, int N, int K, int gelu, hipStream_t stream) {
+                        double* parts, int M, int N, int K, int gelu, const ExactNorm& norm, hipStream_t stream) {
   auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && aligned(A) && aligned(W) && aligned(W2);
   if (M <= kExactRows)
-    return vec ? launch_exact_rows<kMats, kEpilogue, true>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, stream)
-               : launch_exact_rows<kMats, kEpilogue, false>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, stream);
+    return vec ? launch_exact_rows<kMats, kEpilogue, true>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, norm, stream)
+               : launch_exact_rows<kMats, kEpilogue, false>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, norm, stream);
+  if constexpr (kMats == 2) {
+    if (vec && taller_tiles(M, N)) return launch_exact_tile<2, 3, kMats, kEpilogue, true>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, norm, stream);
+  }
   if (M <= 32)
-    return vec ? launch_exact_tile<1, kMats, kEpilogue, true>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, stream)
-               : launch_exact_tile<1, kMats, kEpilogue, false>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, stream);
-  return vec ? launch_exact_tile<2, kMats, kEpilogue, true>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, stream)
-             : launch_exact_tile<2, kMats, kEpilogue, false>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, stream);
+    return vec ? launch_exact_tile<1, 2, kMats, kEpilogue, true>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, norm, stream)
+               : launch_exact_tile<1, 2, kMats, kEpilogue, false>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, norm, stream);
+  return vec ? launch_exact_tile<2, 2, kMats, kEpilogue, true>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, norm, stream)
+             : launch_exact_tile<2, 2, kMats, kEpilogue, false>(out, ldo, A, lda, W, W2, ldw, bias, parts, M, N, K, gelu, norm, stream);
 }
 
 }  // namespace alofa
@@ -449,12 +525,16 @@ static int launch_exact(float* out, int64_t ldo, const float* A, int64_t lda, co
 using namespace alofa;
 
 // Float64 sums that alofa_gemm_exact needs room for with these sizes (0: none).
-extern "C" int64_t alofa_gemm_exact_parts(int M, int N, int K) {
+static int64_t exact_parts(int M, int N, int K, bool norm) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const Cut cut = cut_of(K);
-  if (M <= kExactRows ? chains_per_block(N, cut) == cut.count : !chains_apart(M, N, K, cut)) return 0;
+  if (M <= kExactRows ? chains_per_block(N, cut, norm) == cut.count : !chains_apart(M, N, K, cut)) return 0;
   return static_cast<int64_t>(cut.count) * (M <= kExactRows ? M : rows_at_once(M, N, cut)) * N;
 }
+extern "C" int64_t alofa_gemm_exact_parts(int M, int N, int K) { return exact_parts(M, N, K, false); }
+
+// The same for alofa_gemm_exact_norm; 0: it does not take the sizes (no sums go to memory whose launch the norm could ride on, or rows that are no whole fours or too wide).
+extern "C" int64_t alofa_gemm_exact_norm_parts(int M, int N, int K) { return N % 4 == 0 && N <= 4096 ? exact_parts(M, N, K, true) : 0; }
 
 extern "C" int alofa_gemm_exact(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, int64_t ldw, const float* bias, double* parts, int64_t room,
                                 int M, int N, int K, int epilogue, hipStream_t stream) {
@@ -462,13 +542,24 @@ extern "C" int alofa_gemm_exact(float* out, int64_t ldo, const float* A, int64_t
   ALOFA_REQUIRE(epilogue == kExactStore || epilogue == kExactResidual, "gemm: unknown epilogue %d", epilogue);
   ALOFA_REQUIRE(lda >= K && ldw >= K && ldo >= N, "gemm: a leading dimension is shorter than its row");
   ALOFA_REQUIRE(room >= alofa_gemm_exact_parts(M, N, K), "gemm: no room for the sums of the chains of K");
-  if (epilogue == kExactStore) return launch_exact<1, kExactStore>(out, ldo, A, lda, W, W, ldw, bias, parts, M, N, K, 0, stream);
-  return launch_exact<1, kExactResidual>(out, ldo, A, lda, W, W, ldw, bias, parts, M, N, K, 0, stream);
+  if (epilogue == kExactStore) return launch_exact<1, kExactStore>(out, ldo, A, lda, W, W, ldw, bias, parts, M, N, K, 0, ExactNorm{}, stream);
+  return launch_exact<1, kExactResidual>(out, ldo, A, lda, W, W, ldw, bias, parts, M, N, K, 0, ExactNorm{}, stream);
+}
+
+// The product added to the residual stream, and the RMSNorm of the stream's new rows in `normed` (`ld` apart).
+extern "C" int alofa_gemm_exact_norm(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, int64_t ldw, double* parts, int64_t room, const float* norm_w, float eps,
+                                     float* normed, int64_t ld, int M, int N, int K, hipStream_t stream) {
+  ALOFA_REQUIRE(M > 0 && N > 0 && K > 0 && lda >= K && ldw >= K && ldo >= N && ld >= N, "gemm: M=%d N=%d K=%d must be positive, leading dimensions no shorter than the rows", M, N, K);
+  const int64_t need = alofa_gemm_exact_norm_parts(M, N, K);
+  ALOFA_REQUIRE(need > 0 && room >= need && parts && norm_w && normed && eps > 0.f, "gemm: no room for the sums of the chains of K, or sizes that no norm rides on (M=%d N=%d K=%d)", M, N, K);
+  auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  ALOFA_REQUIRE(aligned(out) && aligned(parts) && aligned(norm_w) && aligned(normed) && ldo % 4 == 0 && ld % 4 == 0, "gemm: the norm behind the product takes 16-byte aligned rows");
+  return launch_exact<1, kExactResidual>(out, ldo, A, lda, W, W, ldw, nullptr, parts, M, N, K, 0, ExactNorm{norm_w, eps, normed, ld}, stream);
 }
 
 extern "C" int alofa_gemm_swiglu_exact(float* out, int64_t ldo, const float* A, int64_t lda, const float* Wg, const float* Wu, int64_t ldw, int M, int N, int K,
                                        int gelu, hipStream_t stream) {
   ALOFA_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_swiglu: M=%d N=%d K=%d must be positive", M, N, K);
   ALOFA_REQUIRE(lda >= K && ldw >= K && ldo >= N, "gemm_swiglu: a leading dimension is shorter than its row");
-  return launch_exact<2, kExactStore>(out, ldo, A, lda, Wg, Wu, ldw, nullptr, nullptr, M, N, K, gelu, stream);
+  return launch_exact<2, kExactStore>(out, ldo, A, lda, Wg, Wu, ldw, nullptr, nullptr, M, N, K, gelu, ExactNorm{}, stream);
 }

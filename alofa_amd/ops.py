@@ -486,6 +486,12 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[tor
         return
     if exact:
         _exact_operands(a=a, w=w, out=out)
+        if then_rows is not None and then_rows.dtype is torch.float32 and FUSE_NORMS and out.data_ptr() % 16 == 0 and _rows("out", out) % 4 == 0 and then_rows.data_ptr() % 16 == 0 and then_w.data_ptr() % 16 == 0:
+            room = load().alofa_gemm_exact_norm_parts(_I(M), _I(N), _I(K))
+            if room:      # (the norm rides on the launch that adds the chains' sums up)
+                parts = torch.empty(room, dtype=torch.float64, device=out.device) if scratch is None else scratch("product_sums", (room,), torch.float64)
+                _call("alofa_gemm_exact_norm", out, _rows("out", out), a, _rows("a", a), w, _rows("w", w), parts, room, then_w, _F(then_eps), then_rows, N, M, N, K, _stream())
+                return
         room = load().alofa_gemm_exact_parts(_I(M), _I(N), _I(K))      # (sums of the chains of K, where the tiles are too few for the chip)
         parts = None
         if room:

@@ -83,6 +83,23 @@ def test_exact_attention(heads, kv_heads, d, bs, requests, window):
     within(out, torch.stack(want).numpy(), 12.0)
 
 
+# gate and up of tiles of 96 rows (where they are the fewer rounds of the chip): their edges, K ragged, columns of no whole tile
+@pytest.mark.parametrize("M,N,K", [(66, 4864, 896), (96, 4864, 100), (95, 4833, 68), (450, 4864, 128), (385, 4810, 36)])
+def test_exact_gate_and_up_of_taller_tiles(M, N, K):
+    gen = torch.Generator(device=DEV).manual_seed(M)
+    a, g, u = (torch.randn(s, generator=gen, device=DEV) * K ** -0.25 for s in ((M, K), (N, K), (N, K)))
+    out = torch.full((M, N + 1), 7.0, device=DEV)
+    ops().gemm_swiglu(out[:, :N], a, g, u, exact=True)
+    gate, up = ((a.double() @ w.double().T.contiguous()).cpu().numpy() for w in (g, u))
+    want = gate / (1.0 + np.exp(-gate)) * up
+    within(out[:, :N], want, 4 * np.abs(want) * (1 + np.abs(gate)) + 1e-7)
+    assert bool((out[:, N:] == 7.0).all())
+    for first, n in ((0, 1), (60, 5), (1, 40), (0, 64)):      # (the same bits as in the other forms)
+        part = torch.empty(n, N, device=DEV)
+        ops().gemm_swiglu(part, a[first:first + n], g, u, exact=True)
+        assert torch.equal(part, out[first:first + n, :N])
+
+
 # slabs of 32 k: none whole, one to seven, with and without a rest, rows that are not 16-byte aligned, shares of unequal length
 @pytest.mark.parametrize("M,N,K,shift", [(17, 40, 20, 0), (33, 70, 32, 0), (33, 70, 52, 0), (65, 70, 64, 0), (20, 140, 96, 0), (65, 70, 99, 0), (40, 64, 128, 0), (64, 64, 160, 1), (90, 70, 190, 1),
                                          (40, 70, 228, 0), (200, 64, 1100, 0)])
@@ -207,6 +224,24 @@ def test_exact_products_name_the_operand_that_is_not_float32():
     for operands, name in (((out, h, f, f), "operand=a"), ((out, f, h, h), "operand=w_gate"), ((out.bfloat16(), f, f, f), "operand=out")):
         with pytest.raises(AlofaError, match=name):
             ops().gemm_swiglu(*operands, exact=True)
+
+
+# rows up to 16, 32, 64 and beyond, sums in one piece and in several, columns that fill a block's threads and more; where no sums go to memory the norm is a launch of its own
+@pytest.mark.parametrize("M,N,K", [(1, 896, 896), (8, 896, 4864), (16, 64, 4864), (8, 1028, 2048), (3, 2052, 700), (17, 896, 4864), (64, 1024, 1024), (450, 896, 896), (1100, 500, 16384), (5, 4100, 1024), (9, 131, 3000)])
+def test_exact_products_with_the_norm_behind_them(M, N, K):
+    gen = torch.Generator(device=DEV).manual_seed(M + N)
+    draw = lambda *s: torch.randn(s, generator=gen, device=DEV)      # noqa: E731
+    a, w, weight, stream = draw(M, K), draw(N, K) * K ** -0.5, draw(N), draw(M, N)
+    got = []
+    for rides in (False, True):
+        out, rows = stream.clone(), torch.empty(M, N, device=DEV)
+        if rides:
+            ops().gemm(out, a, w, add_to_out=True, exact=True, then_norm=(weight, 1e-6, rows))
+        else:
+            ops().gemm(out, a, w, add_to_out=True, exact=True)
+            ops().rmsnorm(rows, out, weight, 1e-6, True)
+        got.append((out, rows))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
 # the new token at a tile's, a page's and a quad's first and last place, alone, behind a window; more heads to a key head than a tile holds
