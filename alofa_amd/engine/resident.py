@@ -147,6 +147,43 @@ class _Turns:
 _turns: dict = {}      # GPU -> its launches' turns
 
 
+class _Tiles:
+    """Copies of a model's gate, up and down matrices as more than sixteen rows read them (``ops.in_tiles``): made once per model, for all its step functions, and again where the matrices have been
+    written since."""
+
+    def __init__(self, sources: list):
+        self._sources = sources
+        versions = self._now()
+        self.copies = [ops.in_tiles(w) for w in sources]
+        torch.cuda.current_stream(sources[0].device).synchronize()      # (steps on other streams read them too)
+        self._versions = versions
+
+    def _now(self) -> list:
+        return [None if w.is_inference() else w._version for w in self._sources]
+
+    def bytes(self) -> int:
+        return sum(t.numel() * t.element_size() for t in self.copies)
+
+    def follow(self) -> None:
+        now = self._now()
+        if now != self._versions:
+            for w, to in zip(self._sources, self.copies):
+                ops.in_tiles(w, to)
+            torch.cuda.current_stream(self._sources[0].device).synchronize()
+            self._versions = now
+
+    @staticmethod
+    def of(model, sources: list) -> Optional["_Tiles"]:
+        """None where there is no memory for them (the kernels one by one need none)."""
+        have = model.tiles
+        if have is None or len(have._sources) != len(sources) or any(a is not b for a, b in zip(have._sources, sources)):
+            try:
+                model.tiles = _Tiles(sources)
+            except torch.cuda.OutOfMemoryError:
+                return None
+        return model.tiles
+
+
 class ResidentLayers:
     """All layers of ``model`` over ``cache`` as one launch, for steps of at most ``MOST_ROWS`` rows of one new token each."""
     MOST_ROWS = most_rows = 16      # (``most_rows``: of this model, up to 64: csrc/decode_groups.hip)
@@ -197,7 +234,7 @@ class ResidentLayers:
             area = _areas.take(device)
         except (AlofaError, RuntimeError):      # (no memory for one: the kernels one by one need none)
             return None
-        return cls(blocks, cache, device, tables, area)
+        return cls(model, blocks, cache, device, tables, area)
 
     @staticmethod
     def _tensors(b, kv: dict) -> list:
@@ -219,7 +256,7 @@ class ResidentLayers:
                 return False
         return True
 
-    def __init__(self, blocks: list, cache, device, tables: list, area: "_Area"):
+    def __init__(self, model, blocks: list, cache, device, tables: list, area: "_Area"):
         self.device, self.area = device, area
         weakref.finalize(self, _areas.give_back, device, area)
         m = blocks[0].mixer
@@ -231,7 +268,8 @@ class ResidentLayers:
         for t in tables:
             ops.check_caches(t[-2], t[-1], self.kv_heads, self.d)
         self._tables = tables      # (kept: the table on the GPU holds their addresses)
-        self.layers = torch.tensor([[0 if t is None else t.data_ptr() for t in ts] for ts in tables], dtype=torch.int64, device=device)
+        self._model, self._tiles, self._addresses = model, None, [[0 if t is None else t.data_ptr() for t in ts] for ts in tables]
+        self._table = torch.tensor(self._addresses, dtype=torch.int64, device=device)
         self.failed = area.failed
         self._failed = self.failed.numpy()
         self.turn = _turns.setdefault(device.index, _Turns(device))      # what a launch, or a replay of one, goes within
@@ -248,11 +286,32 @@ class ResidentLayers:
                 return False
         return ctx.longest <= next((keys for below, keys in self.MOST_KEYS if rows * self.kv_heads < below), ctx.longest)
 
+    @property
+    def layers(self) -> torch.Tensor:
+        """The layers' addresses on the GPU, the second time with gate, up and down in tiles, which more rows than sixteen read: laid out when they are first asked for."""
+        if self._tiles is None and self.most_rows > self.MOST_ROWS:
+            self._tiles = _Tiles.of(self._model, [w for ts in self._tables for w in ts[3:6]])
+            if self._tiles is None:
+                self.most_rows = self.MOST_ROWS
+            else:
+                places = [t.data_ptr() for t in self._tiles.copies]
+                self._table = torch.tensor([self._addresses, [[*a[:3], *places[3 * i:3 * i + 3], *a[6:]] for i, a in enumerate(self._addresses)]], dtype=torch.int64, device=self.device)
+        return self._table
+
+    def ready(self, rows: int) -> bool:
+        """In front of a step that is taken, or a replay of one: what is laid out of the matrices is what they hold. False: there is no memory for it."""
+        if rows > self.MOST_ROWS and not torch.cuda.is_current_stream_capturing():
+            self.layers
+            if self._tiles is None:
+                return False
+            self._tiles.follow()
+        return True
+
     def gave_up(self) -> bool:
         return bool(self._failed[0])
 
     def forward(self, ctx, hidden: torch.Tensor) -> None:
         cos, sin = self.position.table(ctx.n_positions)
         with contextlib.nullcontext() if torch.cuda.is_current_stream_capturing() else self.turn:      # (one that is captured takes its turn at every replay)
-            ops.decode_resident(hidden, self.layers, ctx.positions, ctx._tables[self.group], ctx._slots[self.group], cos, sin, self.area.address, self.failed, self.intermediate,
+            ops.decode_resident(hidden, self._table, ctx.positions, ctx._tables[self.group], ctx._slots[self.group], cos, sin, self.area.address, self.failed, self.intermediate,
                                 self.heads, self.kv_heads, self.d, self.page, self.biased, self.scale, self.eps)

@@ -58,6 +58,7 @@ class Model:
         self.joins = [build_part("join", j, weights, rt) for j in spec.joins]
         self.order = list(spec.order)
         self.descriptions = None      # (of the blocks, for engine/tapes.py)
+        self.tiles = None             # (of matrices that were laid out again, for engine/resident.py)
         self.streams = int(spec.streams)
         if any(b.on_streams != bool(self.streams) for b in self.blocks) or (self.streams and self.joins):
             raise AlofaError("unsupported", "blocks on copies of the stream go with a model that keeps copies, and with no joins", f"streams={self.streams}")
@@ -114,7 +115,7 @@ class Model:
                         total += t.numel() * t.element_size()
                     elif hasattr(t, "rt") and hasattr(t, "spec") and t is not part:
                         stack.append(t)
-        return total
+        return total + (self.tiles.bytes() if self.tiles is not None else 0)
 
     def forward(self, ctx, ids: torch.Tensor) -> torch.Tensor:
         """Run the tokens of the step through every entry; returns the float32
@@ -127,7 +128,7 @@ class Model:
             first.copy_(hidden)
         watch = getattr(ctx, "watch", None)      # (for tests and debugging: called with the stream after every run entry)
         resident = getattr(ctx, "resident", None)
-        if resident is not None and watch is None and resident.takes(ctx, rows):      # few rows of one new token each: every layer in one launch
+        if resident is not None and watch is None and resident.takes(ctx, rows) and resident.ready(rows):      # few rows of one new token each: every layer in one launch
             resident.forward(ctx, hidden)
             return hidden
         stream = hidden

@@ -978,6 +978,19 @@ def resident_takes(hidden: int, intermediate: int, heads: int, kv_heads: int, d:
     return bool(_answer("alofa_resident_takes", _I(hidden), _I(intermediate), _I(heads), _I(kv_heads), _I(d), _I(page)))
 
 
+RESIDENT_ROWS = 16      # rows that ``decode_resident`` takes with the matrices as they are
+
+
+def in_tiles(w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``w`` [rows, columns], multiples of 16 and 32, laid out for ``decode_resident``: sixteen rows by 32 columns after one another, each as the matrix cores take it (sixteen bytes a lane: row l % 16,
+    columns 8 (l / 16) ..), along the columns first."""
+    n, k = w.shape
+    tiles = w.view(n // 16, 16, k // 32, 4, 8).permute(0, 2, 3, 1, 4)
+    out = torch.empty_like(w, memory_format=torch.contiguous_format) if out is None else out
+    out.view(tiles.shape).copy_(tiles)
+    return out
+
+
 def resident_rows(hidden: int, intermediate: int, heads: int, kv_heads: int) -> int:
     """The most rows of a decode step that ``decode_resident`` takes of a model that ``resident_takes``."""
     return _answer("alofa_resident_rows", _I(hidden), _I(intermediate), _I(heads), _I(kv_heads))
@@ -998,15 +1011,20 @@ def clear_resident_area(area: int) -> None:
 
 def decode_resident(hidden: torch.Tensor, layers: torch.Tensor, positions: torch.Tensor, block_table: torch.Tensor, slots: torch.Tensor, cos: torch.Tensor,
                     sin: torch.Tensor, area: int, failed: torch.Tensor, intermediate: int, heads: int, kv_heads: int, d: int, page: int, biased: bool, scale: float, eps: tuple, limit: int = 0) -> None:
-    """Every layer of a decode step, one new token per row, row i request i: ``hidden`` float32 [rows, width], in and out. ``layers`` int64 [layers, 10]: the addresses of a
-    layer's matrices, norms and caches, which the caller keeps alive and has checked; ``area``: of ``resident_area``, used by one launch at a time; ``failed``: int32 [1] in
+    """Every layer of a decode step, one new token per row, row i request i: ``hidden`` float32 [rows, width], in and out. ``layers`` int64 [2, layers, 10] (or [layers, 10], for up to
+    sixteen rows): the addresses of a layer's matrices, norms and caches, which the caller keeps alive and has checked, the second time with gate, up and down laid out in tiles (``in_tiles``), as more rows
+    than sixteen read them; ``area``: of ``resident_area``, used by one launch at a time; ``failed``: int32 [1] in
     pinned memory, set if the kernel gives a wait up: the numbers that hang on it are NaN then.
     ``limit``: after how many asks, some microsecond each (0: the kernel's own limit, seconds)."""
     _contig("hidden", _gpu("hidden", hidden, torch.float32, 2))
     M, H = hidden.shape
-    _contig("layers", _gpu("layers", layers, torch.int64, 2))
-    if layers.shape[1] != 10:
+    _contig("layers", _gpu("layers", layers, torch.int64, None))
+    if layers.dim() not in (2, 3) or layers.shape[-1] != 10 or (layers.dim() == 3 and layers.shape[0] != 2):
         raise AlofaError("shape_mismatch", "a layer has ten addresses", f"layers={tuple(layers.shape)}")
+    if layers.dim() == 3:
+        layers = layers[int(M > RESIDENT_ROWS)]
+    elif M > RESIDENT_ROWS:
+        raise AlofaError("shape_mismatch", "more than sixteen rows read matrices laid out in tiles", f"rows={M} layers={tuple(layers.shape)}")
     _contig("block_table", _gpu("block_table", block_table, torch.int32, 2))
     for name, t, dtype in (("positions", positions, torch.int32), ("slots", slots, torch.int64)):
         if tuple(_contig(name, _gpu(name, t, dtype, 1)).shape) != (M,):

@@ -1,0 +1,76 @@
+"""Matrices laid out in tiles for decode steps of more than sixteen rows in one launch."""
+import numpy as np
+import pytest
+import torch
+
+
+@pytest.mark.parametrize("n,k", [(16, 32), (48, 96), (80, 32)])
+def test_where_a_value_lies_in_tiles(n, k):
+    from alofa_amd import ops
+    w = torch.arange(n * k).view(n, k)
+    flat = ops.in_tiles(w).view(-1)
+    for row in range(n):
+        for col in range(k):
+            lane = col % 32 // 8 * 16 + row % 16
+            assert flat[((row // 16 * (k // 32) + col // 32) * 64 + lane) * 8 + col % 8] == w[row, col]
+    again = torch.zeros_like(w)
+    assert ops.in_tiles(w, again) is again and torch.equal(again.view(-1), flat)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [17, 40])
+def test_matrices_written_in_place_are_laid_out_again(rows):
+    from test_resident_gpu import decode, engine, model, stand
+    shape, lengths = (256, 4, 1, 512), [9 * i for i in range(rows)]
+    tokens = np.random.default_rng(3).integers(0, 500, (3, rows))
+    m = model(*shape, "bfloat16")
+    two = [engine(m, rows, max(lengths) + 12, "bfloat16") for _ in range(2)]
+    for e in two:
+        stand(e, lengths, 1)
+    before = [decode(e, tokens) for e in two]
+    assert all(torch.equal(a, b) for a, b in zip(*before)) and two[0].step_fn.resident._tiles is two[1].step_fn.resident._tiles is not None      # (once per model)
+    w = m[1].blocks[1].feed_forward
+    with torch.no_grad():
+        w.w_down.mul_(0.5), w.w_gate.neg_()
+    got = [decode(e, tokens) for e in two]      # (captured steps, replayed)
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and not torch.equal(got[0][0], before[0][0])
+    other = model(*shape, "bfloat16")
+    with torch.no_grad():
+        other[1].blocks[1].feed_forward.w_down.mul_(0.5), other[1].blocks[1].feed_forward.w_gate.neg_()
+    fresh = engine(other, rows, max(lengths) + 12, "bfloat16")
+    stand(fresh, lengths, 1)
+    first = decode(fresh, tokens[:1])
+    late = engine(m, rows, max(lengths) + 12, "bfloat16")
+    stand(late, lengths, 1)
+    assert torch.equal(decode(late, tokens[:1])[0], first[0])
+
+
+@pytest.mark.gpu
+def test_nothing_is_laid_out_before_a_step_of_more_than_sixteen_rows():
+    from test_resident_gpu import decode, engine, model, stand
+    m = model(256, 4, 1, 512, "bfloat16")
+    size = m[1].weight_bytes()
+    e = engine(m, 17, 100, "bfloat16")
+    stand(e, [5] * 17, 1)
+    decode(e, [[1] * 16])
+    assert m[1].tiles is None and m[1].weight_bytes() == size
+    decode(e, [[1] * 17])
+    assert m[1].weight_bytes() == size + 3 * 256 * 512 * 2 * len(m[1].order)
+
+
+@pytest.mark.gpu
+def test_without_memory_for_tiles_steps_run_kernel_by_kernel(monkeypatch):
+    from alofa_amd import ops
+    from test_resident_gpu import decode, engine, model, stand
+
+    def none(*a):
+        raise torch.cuda.OutOfMemoryError("no memory")
+    monkeypatch.setattr(ops, "in_tiles", none)
+    e = engine(model(256, 4, 1, 512, "bfloat16"), 20, 100, "bfloat16")
+    stand(e, [5] * 20, 1)
+    launches, one_launch = [], ops.decode_resident
+    monkeypatch.setattr(ops, "decode_resident", lambda hidden, *a, **how: (launches.append(hidden.shape[0]), one_launch(hidden, *a, **how))[1])
+    out = decode(e, [[1] * 20])
+    assert not launches and bool(torch.isfinite(out[0]).all()) and e.step_fn.resident.most_rows == 16
+    decode(e, [[1] * 16])
+    assert set(launches) == {16}
