@@ -273,6 +273,18 @@ __global__ void __launch_bounds__(256) gemm_mfma_kernel(TO* __restrict__ out, in
   }
 }
 
+// Where nothing more is to be set out: the last slabs, each as it comes (those behind it, R at most, stay on their way).
+template <int R, int kLoads, typename F>
+__device__ __forceinline__ void last_slabs(int& k, int slabs, const F& step) {
+  if (slabs - k > R) {
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kLoads * R) : "memory");
+    __syncthreads();
+    step(k);
+    ++k;
+  }
+  if constexpr (R > 0) last_slabs<R - 1, kLoads>(k, slabs, step);
+}
+
 // The same product with the slabs brought from memory straight into LDS (global_load_lds_dwordx4: every lane's
 // 16 bytes land at consecutive LDS addresses, 1 KB per wave and instruction, no registers and no LDS writes in
 // between) into a ring of S slabs, S - 1 of them on their way while one is multiplied. For K a multiple of 64; with
@@ -283,7 +295,6 @@ __global__ void __launch_bounds__(256) gemm_mfma_kernel(TO* __restrict__ out, in
 // of row r undoes by fetching chunk p ^ swz(r), so that the 16 or 32 rows whose fragments are read together
 // fall on distinct banks.
 // Rows beyond M or N are fetched from the last valid row (their results are never stored).
-
 // kSplitK = 2: a block leaves its share's sums as they are, tile by tile, in part `share` of `out` (float
 // [shares, M, ldo]); a second kernel (split_sum_kernel) adds the parts and runs the epilogue.
 template <int kEpilogue, typename TO, int WTM, int WTN, int S, int kSplitK = 0>
@@ -404,12 +415,10 @@ __global__ void __launch_bounds__(256) gemm_dma_kernel(TO* __restrict__ out, int
     fetch(k + kLead);
     multiply();
   }
-  for (; k < slabs; ++k) {      // nothing more to set out: the last slabs as they come
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    read(k);
+  last_slabs<kLead - 1, kLoads>(k, slabs, [&](int slab) __attribute__((always_inline)) {
+    read(slab);
     multiply();
-  }
+  });
   if constexpr (is_gated(kEpilogue) && WTN == 1) {
     __syncthreads();      // every wave has read the last slab: the ring is free
     float* meet = reinterpret_cast<float*>(ring);     // [wm][i][e][lane]
@@ -720,6 +729,15 @@ static int launch_dma_sliced(void* out, int64_t ldo, const void* A, int64_t lda,
   return 0;
 }
 
+// S: where the blocks are no more than the compute units, as many slabs as fit a compute unit's LDS. With a short K most
+// or all of it is on its way at once, and a block waits for memory about once, not every few slabs (us, weights from
+// memory, rings of three or four / these): tiles of 64 x 64, ring of eight, 1,152 x 896 at 65 to 400 rows 9.8 / 7.9, at
+// 768 9.7 / 8.4; 896 x 896 with the norm behind it 12.5-13.8 / 10.5-12.5; 1,024 x 1,024 10.5 / 8.2; 2,048 x 1,536 at 65
+// to 400 rows 14.0 / 10.3; gate and up of 4,864 x 896 at 17, 32, 64 rows 9.2, 9.7, 9.1 / 8.0, 8.5, 8.7; 11,008 x 2,048 at
+// 17 to 64 rows (64 x 128, six) 24.8-25.8 / 21.8-23.0. With K in shares: N = 896, K = 4,864 at 17 to 64 rows (six) 11.0-11.8 /
+// 10.5-11.3, N = 3,584, K = 18,944 at 200 and 400 rows (128 x 128, four) 58.4, 96.5 / 55.3, 90.3. With more blocks than
+// that a shallow ring leaves room for two or three of them in a compute unit: 288 and 336 blocks of 64 x 64, rings of three /
+// five 10.4, 15.9 / 10.8, 15.5; shares that meet in the workspace, two blocks a compute unit, 20.4 / 24.4 for 3,584 x 3,584 at 100 rows.
 template <int kEpilogue, typename TO, int WTM, int WTN, int S>
 static int launch_dma(void* out, int64_t ldo, const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, int M, int N, int K,
                       hipStream_t stream, const void* W2 = nullptr, int own = 0) {
@@ -781,10 +799,9 @@ static int launch_mfma(void* out, int64_t ldo, const void* A, int64_t lda, const
     // that brings them in through registers with 128-row tiles, one slab ahead):
     //  * up to 64 rows, and further while the tiles of 64 rows are no more than the compute units: such tiles
     //    (64 gate + 64 up columns; 128 + 128 for a long and wide pair of matrices, see below),
-    //    a ring of four where K is short (one block per compute unit), of three otherwise (9.9, 10.6, 11.4, 11.4
-    //    at 17, 32, 64, 192 rows against 11.8, 12.2, 12.3 through registers and 22.4; 7B sizes at 64 rows: 70.8
-    //    against 72.5);
-    //  * then, while the tiles of 128 rows are no more than the compute units: those, a ring of three (14.5 at
+    //    one block per compute unit and the ring as deep as LDS holds (with one of four 9.9, 10.6, 11.4, 11.4
+    //    at 17, 32, 64, 192 rows against 11.8, 12.2, 12.3 through registers and 22.4);
+    //  * then, while the tiles of 128 rows are no more than the compute units: those, a ring of four (three: 14.5 at
     //    256 rows, 14.8 at 384 against 22.6 and 22.8);
     //  * up to two such tiles per compute unit: a ring of two, two blocks per compute unit (22.5 at 512 rows,
     //    23.6 at 768 against 24.1 and 25.4);
@@ -795,15 +812,15 @@ static int launch_mfma(void* out, int64_t ldo, const void* A, int64_t lda, const
     const int own = M <= 64 ? owned_columns(N) : 0;     // (one tile of rows: what a block owns if the blocks are dealt out evenly, 0 if whole tiles fill the chip)
     if (ring && own > 0 && K >= 2048) {
       if (own <= 64) {
-        if (launch_dma<kEpilogue, TO, 1, 2, 3>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2, own)) return 1;
+        if (launch_dma<kEpilogue, TO, 1, 2, 6>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2, own)) return 1;
       } else {
         if (launch_dma<kEpilogue, TO, 1, 4, 3>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2, own)) return 1;
       }
     } else if (ring && own > 0 && own <= 64) {
       if (own <= 32) {
-        if (launch_dma<kEpilogue, TO, 1, 1, 4>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2, own)) return 1;
+        if (launch_dma<kEpilogue, TO, 1, 1, 8>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2, own)) return 1;
       } else {
-        if (launch_dma<kEpilogue, TO, 1, 2, 4>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2, own)) return 1;
+        if (launch_dma<kEpilogue, TO, 1, 2, 6>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2, own)) return 1;
       }
     } else
     if (ring && (M <= 64 || tiles_64 <= 256)) {
@@ -813,19 +830,16 @@ static int launch_mfma(void* out, int64_t ldo, const void* A, int64_t lda, const
         // 114, 120, 125; with fewer such tiles than three quarters of the compute units only from 33 rows on: 7B
         // sizes, 148 tiles, 64.1 against 62.4 at 16 rows, 67.6 against 70.7 at 64)
         if (launch_dma<kEpilogue, TO, 1, 4, 3>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2, 0)) return 1;
-      } else if (K < 2048) {
+      } else if (K < 2048 && M <= 64 && (N + 63) / 64 < 128) {
         // (up to 64 rows and fewer tiles than half the compute units: tiles of 32 outputs, whose gate and up halves
         // are computed by different waves and meet in LDS; N = 4,864, K = 896 at 17 to 64 rows 8.5-9.4 us against
-        // 9.9-11.2)
-        if (M <= 64 && (N + 63) / 64 < 128) {
-          if (launch_dma<kEpilogue, TO, 1, 1, 4>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2, 0)) return 1;
-        } else
-        if (launch_dma<kEpilogue, TO, 1, 2, 4>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2, 0)) return 1;
+        // 9.9-11.2, either with a ring of four)
+        if (launch_dma<kEpilogue, TO, 1, 1, 8>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2, 0)) return 1;
       } else {
-        if (launch_dma<kEpilogue, TO, 1, 2, 3>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2, 0)) return 1;
+        if (launch_dma<kEpilogue, TO, 1, 2, 6>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2, 0)) return 1;
       }
     } else if (ring && tiles_128 <= 256) {
-      if (launch_dma<kEpilogue, TO, 2, 2, 3>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2)) return 1;
+      if (launch_dma<kEpilogue, TO, 2, 2, 4>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2)) return 1;
     } else if (ring && tiles_128 < 512) {
       if (launch_dma<kEpilogue, TO, 2, 2, 2>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream, W2)) return 1;
     } else if (ring && K >= 2048 && fills_rounds(static_cast<int64_t>((N + 127) / 128) * ((M + 127) / 128))) {
@@ -895,22 +909,22 @@ static int launch_mfma(void* out, int64_t ldo, const void* A, int64_t lda, const
       if (!is_gated(kEpilogue) && ring && long_k && (M <= 64 || (M <= 256 && !tall && K >= 3072)) && wide_tiles <= 36 && N % 4 == 0 && slices > 1 &&
           static_cast<int64_t>(slices) * M * N <= workspace().tile_floats) {
         if constexpr (!is_gated(kEpilogue)) {
-          if (launch_dma_sliced<kEpilogue, TO, 2, 4>(out, ldo, A, lda, W, ldw, bias, M, N, K, slices, stream, then, then_done)) return 1;
+          if (launch_dma_sliced<kEpilogue, TO, 2, 6>(out, ldo, A, lda, W, ldw, bias, M, N, K, slices, stream, then, then_done)) return 1;
         }
       } else
       if (tall && !is_gated(kEpilogue) && ring && N % 4 == 0 &&
           static_cast<int64_t>(tall_shares) * M * N <= workspace().tile_floats) {
         if constexpr (!is_gated(kEpilogue)) {
-          if (launch_dma_sliced<kEpilogue, TO, 2, 3, 2>(out, ldo, A, lda, W, ldw, bias, M, N, K, tall_shares, stream, then, then_done)) return 1;
+          if (launch_dma_sliced<kEpilogue, TO, 2, 4, 2>(out, ldo, A, lda, W, ldw, bias, M, N, K, tall_shares, stream, then, then_done)) return 1;
         }
       } else
       if (ring && long_k && tiles_128x64 >= 144 && tiles_128x64 <= 256) {
         // Tiles of 128 x 64 that fill most of the chip once, and a long K: one block per compute unit with a ring
-        // of four (35.8 against 38.8 us for N = 896, K = 4,864 at 2,048 rows; 28.8 against 36.1 with K shared out
+        // of six (of four 35.8 against 38.8 us for N = 896, K = 4,864 at 2,048 rows; 28.8 against 36.1 with K shared out
         // for N = 4,608, K = 3,584 at 256 rows, 121 against 151 for N = 3,584, K = 18,944 at 384 rows; fewer tiles
         // do better with K shared out, 26.1 against 30.3 for 3,584 x 3,584 at 256 rows; with a short K, or with
         // more tiles than compute units, the small tiles below do better: 11.6 against 10.4 us for 896 x 896)
-        if (launch_dma<kEpilogue, TO, 2, 1, 4>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream)) return 1;
+        if (launch_dma<kEpilogue, TO, 2, 1, 6>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream)) return 1;
       } else if (shares > 1) {
         // K shared out among blocks: with weights of 32 MB or more the slabs go straight into a ring of three in
         // LDS here too (N = 5,120, K = 27,648 at 32 rows: 75 against 85 us; N = 3,584, K = 18,944 at 16 rows: 34.4
@@ -921,10 +935,13 @@ static int launch_mfma(void* out, int64_t ldo, const void* A, int64_t lda, const
         } else
         if (launch_tile<kEpilogue, TO, 1, 1, 2, true>(tiles_n, tiles_m, shares, out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream)) return 1;
       } else if (ring) {
-        // small tiles, slabs straight from memory into a ring of three (against the kernel below, same conditions:
+        // small tiles, slabs straight from memory, up to one block per compute unit into a ring of eight (launch_dma), with more
+        // of them a ring of three (against the kernel below, same conditions:
         // 13.3 against 15.8 us for N = 1,152, K = 896; 10.4 against 12.2 for 896 x 896; 38.8 against 44.6 for
         // N = 896, K = 4,864; a ring of two is slower than either when the weights come from memory: 60 us)
-        if (launch_dma<kEpilogue, TO, 1, 1, 3>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream)) return 1;
+        if (static_cast<int64_t>(tiles_n) * tiles_m <= 256) {
+          if (launch_dma<kEpilogue, TO, 1, 1, 8>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream)) return 1;
+        } else if (launch_dma<kEpilogue, TO, 1, 1, 3>(out, ldo, A, lda, W, ldw, bias, M, N, K, stream)) return 1;
       } else {
         if (launch_tile<kEpilogue, TO, 1, 1, 2, false>(tiles_n, tiles_m, 1, out, ldo, A, lda, W, W2, ldw, bias, M, N, K, stream)) return 1;
       }
