@@ -29,6 +29,23 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
 }
 
+// Eight pairs (a[j], b[j]) of bfloat16 turned by the angles whose cosines and sines are c and s: products and sum are separate float operations
+__device__ __forceinline__ void turn_eight(const uint4& a, const uint4& b, const float4 (&c)[2], const float4 (&s)[2], uint4& lo, uint4& hi) {
+#pragma clang fp contract(off)
+  const uint32_t aw[4] = {a.x, a.y, a.z, a.w}, bw[4] = {b.x, b.y, b.z, b.w};
+  const float cv[8] = {c[0].x, c[0].y, c[0].z, c[0].w, c[1].x, c[1].y, c[1].z, c[1].w}, sv[8] = {s[0].x, s[0].y, s[0].z, s[0].w, s[1].x, s[1].y, s[1].z, s[1].w};
+  uint32_t l[4], h[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    // two elements per 32-bit word, the lower one first
+    const float a0 = __uint_as_float(aw[e] << 16), a1 = __uint_as_float(aw[e] & 0xffff0000u);
+    const float b0 = __uint_as_float(bw[e] << 16), b1 = __uint_as_float(bw[e] & 0xffff0000u);
+    l[e] = pack_bf16x2(a0 * cv[2 * e] - b0 * sv[2 * e], a1 * cv[2 * e + 1] - b1 * sv[2 * e + 1]);
+    h[e] = pack_bf16x2(b0 * cv[2 * e] + a0 * sv[2 * e], b1 * cv[2 * e + 1] + a1 * sv[2 * e + 1]);
+  }
+  lo = make_uint4(l[0], l[1], l[2], l[3]), hi = make_uint4(h[0], h[1], h[2], h[3]);
+}
+
 // what pack_bf16x2 rounded away of a and b, as a second pair: the two pairs together keep sixteen bits of each
 __device__ __forceinline__ uint32_t pack_bf16x2_rest(float a, float b, uint32_t packed) {
   return pack_bf16x2(a - __uint_as_float(packed << 16), b - __uint_as_float(packed & 0xffff0000u));

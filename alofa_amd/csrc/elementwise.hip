@@ -141,7 +141,6 @@ __global__ void __launch_bounds__(256) rope_kv_write_vec_kernel(
     bf16_t* __restrict__ qkv, int64_t row_stride, const float* __restrict__ cos_t, const float* __restrict__ sin_t,
     const int32_t* __restrict__ positions, const int64_t* __restrict__ slots, bf16_t* __restrict__ k_cache,
     bf16_t* __restrict__ v_cache, int tokens, int heads, int kv_heads, int d, int block_size, int write_cache) {
-#pragma clang fp contract(off)
   const int half = d / 2;
   const int rot_units = (heads + kv_heads) * (half / 8);
   const int64_t rot_threads = static_cast<int64_t>(tokens) * rot_units;
@@ -155,27 +154,18 @@ __global__ void __launch_bounds__(256) rope_kv_write_vec_kernel(
     const float* sn = sin_t + static_cast<int64_t>(pos) * half + j;
     bf16_t* x = row + static_cast<int64_t>(head) * d + j;
     const uint4 av = *reinterpret_cast<const uint4*>(x), bv = *reinterpret_cast<const uint4*>(x + half);
-    const float4 c0 = *reinterpret_cast<const float4*>(cs), c1 = *reinterpret_cast<const float4*>(cs + 4);
-    const float4 s0 = *reinterpret_cast<const float4*>(sn), s1 = *reinterpret_cast<const float4*>(sn + 4);
-    const uint32_t aw[4] = {av.x, av.y, av.z, av.w}, bw[4] = {bv.x, bv.y, bv.z, bv.w};
-    const float c[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w}, sv[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-    uint32_t lo[4], hi[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      // two elements per 32-bit word, the lower one first
-      const float a0 = __uint_as_float(aw[e] << 16), a1 = __uint_as_float(aw[e] & 0xffff0000u);
-      const float b0 = __uint_as_float(bw[e] << 16), b1 = __uint_as_float(bw[e] & 0xffff0000u);
-      lo[e] = pack_bf16x2(a0 * c[2 * e] - b0 * sv[2 * e], a1 * c[2 * e + 1] - b1 * sv[2 * e + 1]);
-      hi[e] = pack_bf16x2(b0 * c[2 * e] + a0 * sv[2 * e], b1 * c[2 * e + 1] + a1 * sv[2 * e + 1]);
-    }
+    const float4 c[2] = {*reinterpret_cast<const float4*>(cs), *reinterpret_cast<const float4*>(cs + 4)};
+    const float4 sv[2] = {*reinterpret_cast<const float4*>(sn), *reinterpret_cast<const float4*>(sn + 4)};
+    uint4 lo, hi;
+    turn_eight(av, bv, c, sv, lo, hi);
     bf16_t* dst = x;
     if (head >= heads) {
       if (!write_cache) return;
       const int64_t slot = slots[t];
       dst = k_cache + ((slot / block_size * kv_heads + (head - heads)) * block_size + slot % block_size) * d + j;
     }
-    *reinterpret_cast<uint4*>(dst) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-    *reinterpret_cast<uint4*>(dst + half) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+    *reinterpret_cast<uint4*>(dst) = lo;
+    *reinterpret_cast<uint4*>(dst + half) = hi;
     return;
   }
   if (!write_cache) return;

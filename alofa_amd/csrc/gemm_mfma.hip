@@ -26,6 +26,9 @@
 // W slab holds as many rows of each) and writes silu(gate) * up (or the tanh form of gelu in silu's place).
 #include "gemm_tiles.h"
 
+#include <initializer_list>
+#include <type_traits>
+
 namespace alofa {
 
 constexpr int TK = 64, PAD = 8;
@@ -295,6 +298,79 @@ __device__ __forceinline__ void last_slabs(int& k, int slabs, const F& step) {
 // of row r undoes by fetching chunk p ^ swz(r), so that the 16 or 32 rows whose fragments are read together
 // fall on distinct banks.
 // Rows beyond M or N are fetched from the last valid row (their results are never stored).
+// kMfTurn: the columns are heads of 64 channels, query heads, then key heads, then value heads, and a tile is 64 rows of one of them. What rope_kv_write_kernel (elementwise.hip) would do to the rounded
+// outputs happens here on their way out, by way of LDS and with its arithmetic: queries are turned, keys are turned and go to their rows' slots of the cache, values to theirs (`out` keeps
+// neither). Rows' positions and slots are asked for before the first slab, cosines and sines behind the last. What bounds such a product is as before; the rotation's launch, its start and its way through memory are saved. Product and
+// rotation by launches of their own / together, us, weights from memory, 1,152 x 896 at 17, 64, 65, 512, 1,024, 2,048 and 3,072 rows 8.0 / 6.3, 9.9 / 7.7, 10.7 / 7.0, 11.5 / 7.6, 13.9 / 9.8, 19.5 / 13.9,
+// 20.4 / 17.3; 3,072 x 1,536 at 17, 65, 512, 1,024 rows 10.3 / 8.8, 13.5 / 9.4, 20.9 / 16.6, 27.4 / 22.4; 384 x 256 at 17 and 2,048 6.0 / 3.7, 8.3 / 4.6.
+struct TurnArgs {
+  const float* cos_t;          // [positions, 32]
+  const float* sin_t;
+  const int32_t* positions;    // of the rows
+  const int64_t* slots;
+  bf16_t* k_cache;             // [page, key head, slot, 64]
+  bf16_t* v_cache;             // [page, key head, 64, slot]
+  int heads, kv_heads, page_shift;
+};
+struct NoTurn {};
+constexpr int kTurnRow = 72;   // elements of a row in LDS
+
+__device__ __forceinline__ void turn_epilogue(const f32x16& acc, bf16_t* tile, bf16_t* __restrict__ out, int64_t ldo, const float* __restrict__ bias, int M, int m0, int n0, int wm, int wn,
+                                              int tid, int position, int64_t slot, const TurnArgs& turn) {
+  const int lane = tid % 64, head = n0 / 64, r = tid / 4, j = tid % 4 * 8, page = 1 << turn.page_shift;
+  const bool turned = head < turn.heads + turn.kv_heads;
+  float4 c[2], s[2];
+  if (turned) {
+    const int64_t at = static_cast<int64_t>(position) * 32 + j;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      c[i] = *reinterpret_cast<const float4*>(turn.cos_t + at + 4 * i);
+      s[i] = *reinterpret_cast<const float4*>(turn.sin_t + at + 4 * i);
+    }
+  }
+  const float b = bias ? bias[n0 + wn * 32 + lane % 32] : 0.f;
+  __syncthreads();      // every wave has read the last slab: the ring is free
+#pragma unroll
+  for (int e = 0; e < 16; ++e) tile[(wm * 32 + 8 * (e / 4) + 4 * (lane / 32) + e % 4) * kTurnRow + wn * 32 + lane % 32] = f32_to_bf16(acc[e] + b);
+  __syncthreads();
+  if (turned) {
+    const int m = m0 + r;
+    if (m >= M) return;
+    uint4 lo, hi;
+    turn_eight(*reinterpret_cast<const uint4*>(tile + r * kTurnRow + j), *reinterpret_cast<const uint4*>(tile + r * kTurnRow + 32 + j), c, s, lo, hi);
+    bf16_t* dst = head < turn.heads ? out + static_cast<int64_t>(m) * ldo + n0 + j
+                                    : turn.k_cache + ((((slot >> turn.page_shift) * turn.kv_heads + (head - turn.heads)) << turn.page_shift) + (slot & (page - 1))) * 64 + j;
+    *reinterpret_cast<uint4*>(dst) = lo;
+    *reinterpret_cast<uint4*>(dst + 32) = hi;
+    return;
+  }
+  // values: a channel of eight rows a lane; where these lie in eight aligned slots side by side they leave in one piece
+  const int hk = head - turn.heads - turn.kv_heads, ch = lane;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int r0 = (tid / 64 + 4 * u) * 8, n = min(8, M - m0 - r0);
+    if (n <= 0) continue;
+    int64_t to[8];
+    uint32_t v[8];
+    bool run = n == 8 && page >= 8;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      to[e] = turn.slots[m0 + r0 + min(e, n - 1)];
+      v[e] = tile[(r0 + e) * kTurnRow + ch];
+      run = run && to[e] == to[0] + e;
+    }
+    run = run && to[0] % 8 == 0 && reinterpret_cast<uintptr_t>(turn.v_cache) % 16 == 0;
+    auto place = [&](int64_t at) { return turn.v_cache + ((((at >> turn.page_shift) * turn.kv_heads + hk) * 64 + ch) << turn.page_shift) + (at & (page - 1)); };
+    if (run) {
+      *reinterpret_cast<uint4*>(place(to[0])) = make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (e < n) *place(to[e]) = static_cast<bf16_t>(v[e]);
+    }
+  }
+}
+
 // kSplitK = 2: a block leaves its share's sums as they are, tile by tile, in part `share` of `out` (float
 // [shares, M, ldo]); a second kernel (split_sum_kernel) adds the parts and runs the epilogue.
 template <int kEpilogue, typename TO, int WTM, int WTN, int S, int kSplitK = 0>
@@ -302,7 +378,8 @@ __global__ void __launch_bounds__(256) gemm_dma_kernel(TO* __restrict__ out, int
                                                        const bf16_t* __restrict__ W, const bf16_t* __restrict__ W2, int64_t ldw,
                                                        const float* __restrict__ bias, int M, int N, int K, int tiles_m,
                                                        int tiles_n, int by_die, int shares = 1, float* __restrict__ ws = nullptr,
-                                                       int* __restrict__ counters = nullptr, int own = 0) {
+                                                       int* __restrict__ counters = nullptr, int own = 0,
+                                                       std::conditional_t<kEpilogue == kMfTurn, TurnArgs, NoTurn> turn = {}) {
   constexpr int TM = 64 * WTM, TN = 64 * WTN;
   constexpr int kGateTiles = WTN / 2;
   // (swiglu with WTN = 1: the waves of column 0 take 32 gate columns, those of column 1 the up columns of the same
@@ -340,6 +417,13 @@ __global__ void __launch_bounds__(256) gemm_dma_kernel(TO* __restrict__ out, int
       }
       src[j] = base + static_cast<int64_t>(min(n, n_end - 1)) * ldw + c * 8;
     }
+  }
+  [[maybe_unused]] int position = 0;
+  [[maybe_unused]] int64_t slot = 0;
+  if constexpr (kEpilogue == kMfTurn) {
+    const int m = min(m0 + tid / 4, M - 1);
+    position = turn.positions[m];
+    slot = turn.slots[m];
   }
   // The fetches are written out as instructions: the compiler, which cannot tell the ring's slabs apart, would wait
   // for every fetch on its way before any read from LDS, and the slabs set out ahead would be waited for at once.
@@ -442,6 +526,11 @@ __global__ void __launch_bounds__(256) gemm_dma_kernel(TO* __restrict__ out, int
         }
       }
     }
+    return;
+  }
+  if constexpr (kEpilogue == kMfTurn) {
+    static_assert(WTM == 1 && WTN == 1 && sizeof(TO) == 2 && kSplitK == 0, "a tile is a head of 64 channels");
+    turn_epilogue(acc[0][0], reinterpret_cast<bf16_t*>(ring), out, ldo, bias, M, m0, n0, wm, wn, tid, position, slot, turn);
     return;
   }
   if constexpr (kSplitK == 2) {
@@ -990,6 +1079,35 @@ extern "C" int alofa_gemm_mfma(void* out, int o_dtype, int64_t ldo, const void* 
     return launch_mfma<kMfGeglu, bf16_t>(out, ldo, A, lda, W, W2, ldw, nullptr, M, N, K, stream, kNoNorm, done);
   }
   ALOFA_REQUIRE(false, "gemm_mfma: unsupported epilogue %d with out dtype %d", epilogue, o_dtype);
+}
+
+// Whether alofa_gemm_turn takes a product of M rows of [queries | keys | values]: heads of 64 channels and the small tiles, whose 64 columns are then a head. Those are what such a product takes where
+// K is short and the tiles of 128 x 128 are fewer than the compute units (launch_mfma; also where gemm_tall.hip is the faster product by itself: 2,304 x 768 at 1,500 rows 21.0 by two launches, 16.1 so). Up to sixteen
+// rows, and with a long K, the products that share K out are further ahead of these tiles than a launch takes.
+extern "C" int alofa_gemm_turns(int M, int N, int K, int d) {
+  return d == 64 && M > 16 && N > 0 && N % 64 == 0 && K > 0 && K % TK == 0 && K < 32 * TK && static_cast<int64_t>((N + 127) / 128) * ((M + 127) / 128) < 256;
+}
+
+// out = A @ W^T + bias, rounded, [queries | keys | values] of M rows in heads of 64 channels, with rope_kv_write's work behind it in the same launch: queries turned, keys turned in their rows' slots of the cache,
+// values in theirs (out's columns of keys and values are left as they are). Only where alofa_gemm_turns says so; pages of a power of two of tokens.
+extern "C" int alofa_gemm_turn(void* out, int64_t ldo, const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, const float* cos_t, const float* sin_t,
+                               const int32_t* positions, const int64_t* slots, void* k_cache, void* v_cache, int M, int N, int K, int heads, int kv_heads, int block_size, hipStream_t stream) {
+  ALOFA_REQUIRE(alofa_gemm_turns(M, N, K, 64) && heads > 0 && kv_heads > 0 && N == (heads + 2 * kv_heads) * 64, "gemm_turn: M=%d N=%d K=%d does not fit %d and %d heads of 64", M, N, K, heads, kv_heads);
+  ALOFA_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && ldo % 8 == 0 && lda >= K && ldw >= K && ldo >= N, "gemm_turn: leading dimensions %lld, %lld, %lld", static_cast<long long>(lda),
+                static_cast<long long>(ldw), static_cast<long long>(ldo));
+  ALOFA_REQUIRE(block_size > 0 && (block_size & (block_size - 1)) == 0, "gemm_turn: pages of %d tokens", block_size);
+  ALOFA_REQUIRE(cos_t && sin_t && positions && slots && k_cache && v_cache, "gemm_turn: a table, the rows' places or a cache is missing");
+  for (const void* p : {static_cast<const void*>(out), A, W, static_cast<const void*>(cos_t), static_cast<const void*>(sin_t), static_cast<const void*>(k_cache)})
+    ALOFA_REQUIRE(reinterpret_cast<uintptr_t>(p) % 16 == 0, "gemm_turn: operands must be 16-byte aligned");
+  const TurnArgs turn{cos_t, sin_t, positions, slots, static_cast<bf16_t*>(k_cache), static_cast<bf16_t*>(v_cache), heads, kv_heads, __builtin_ctz(block_size)};
+  const int tiles_n = N / 64, tiles_m = (M + 63) / 64;
+  auto launch = [&](auto kernel) {
+    kernel<<<tiles_n * tiles_m, 256, 0, stream>>>(static_cast<bf16_t*>(out), ldo, static_cast<const bf16_t*>(A), lda, static_cast<const bf16_t*>(W), nullptr, ldw, bias, M, N, K, tiles_m, tiles_n, 1, 1,
+                                                  nullptr, nullptr, 0, turn);
+  };
+  if (tiles_n * tiles_m <= 256) launch(gemm_dma_kernel<kMfTurn, bf16_t, 1, 1, 8>);      // (rings: launch_dma)
+  else launch(gemm_dma_kernel<kMfTurn, bf16_t, 1, 1, 3>);
+  return check_launch("gemm_turn");
 }
 
 // out[m] = the column n with the highest sum_k A[m, k] * W[n, k] (the lowest n among equals), for M <= 64 rows

@@ -9,7 +9,7 @@ namespace alofa {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-enum MfmaEpilogue : int { kMfStore = 0, kMfResidual = 1, kMfSwiglu = 2, kMfArgmax = 3, kMfGeglu = 4 };
+enum MfmaEpilogue : int { kMfStore = 0, kMfResidual = 1, kMfSwiglu = 2, kMfArgmax = 3, kMfGeglu = 4, kMfTurn = 5 };
 
 // Which tile a block computes. The chip is eight dies, each with an L2 of its own, and blocks go to the
 // dies in turn (block i to die i % 8). Dealt out row by row, every die computes tiles from all over the

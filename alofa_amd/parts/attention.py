@@ -84,11 +84,11 @@ class RowPlan:
         return self._tiles[key]
 
 
-def paged_attend(ctx, entry, qkv, attn, heads, kv_heads, d, window, scale, position, rt) -> None:
+def paged_attend(ctx, entry, qkv, attn, heads, kv_heads, d, window, scale, position, rt, written=False) -> None:
     """The rows of one step through attention over the pages of the mixer at ``entry``: ``qkv`` [T, (heads + 2 kv_heads) d] holds
     the step's queries, keys and values, heads of one size d side by side; queries and keys take ``position``, keys and values go
     to their rows' cache slots (where the mixer owns the cache), and ``attn`` [T, heads d] receives softmax(scale q k) v over the
-    keys each row may see. Which kernels run follows from the step's layout, the dtype and the sizes."""
+    keys each row may see (``written``: the queries are turned and the keys and values in their slots already). Which kernels run follows from the step's layout, the dtype and the sizes."""
     T = qkv.shape[0]
     exact = rt.exact
     mfma_heads = d % 16 == 0
@@ -109,7 +109,7 @@ def paged_attend(ctx, entry, qkv, attn, heads, kv_heads, d, window, scale, posit
              and ops.can_fuse_rope_into_decode(d))
     # (the exact path likewise)
     turned = exact and kv.owner and ctx.max_q_len == 1 and plan.long_runs is None and ops.can_turn_exactly(qkv, kv.k, kv.v, d)
-    if fused or turned:
+    if fused or turned or written:
         pass
     elif kv.owner:
         ops.rope_kv_write(qkv, cos, sin, ctx.positions, heads, kv_heads, d, kv.slots, kv.k, kv.v)
@@ -278,12 +278,17 @@ class GQAAttention(Mixer):
         T = residual.shape[0]
         exact = self.rt.exact
         qkv = ctx.scratch("qkv", (T, self.qkv_width), self.rt.dtype)
+        table = self.position.table(ctx.n_positions)
+        written = norm is None and not exact and ctx.max_q_len > 1 and table is not None and ctx.kv(entry).owner
         if norm is not None:      # the input norm rides on the product
             ops.gemm(qkv, residual, self.w_qkv, self.b_qkv, norm=norm.as_rmsnorm())
+        elif written:      # (portions of prompts: what stands between the product and attention rides on the product where it can)
+            kv = ctx.kv(entry)
+            ops.gemm_turned(qkv, x, self.w_qkv, self.b_qkv, *table, ctx.positions, kv.slots, kv.k, kv.v, self.heads, self.kv_heads, self.d)
         else:
             ops.gemm(qkv, x, self.w_qkv, self.b_qkv, exact=exact, scratch=ctx.scratch)
         attn = ctx.scratch("attn", (T, self.heads * self.d), self.rt.dtype)
-        paged_attend(ctx, entry, qkv, attn, self.heads, self.kv_heads, self.d, self.window, self.scale, self.position, self.rt)
+        paged_attend(ctx, entry, qkv, attn, self.heads, self.kv_heads, self.d, self.window, self.scale, self.position, self.rt, written)
         if out is not None:
             ops.gemm(out, attn, self.w_o, self.b_o, exact=exact, scratch=ctx.scratch)
         elif self.b_o is not None:
