@@ -79,25 +79,36 @@ static Cut cut_of(int K) {
 }
 
 // NW waves; kMats = 2: gate and up. NT tiles of 16 weight rows a block (of each matrix). blockIdx.y: which `per` chains; parts, where those are not all: the chains' sums, [chain][M][N].
-template <int NW, int NT, int kMats, int kEpilogue, bool kVec>
+// kDealt > 0 (gate and up): a block owns `own` outputs, the rows of gate and then those of up side by side in kDealt tiles: see launch_exact_rows.
+template <int NW, int NT, int kMats, int kEpilogue, bool kVec, int kDealt = 0>
 __global__ void __launch_bounds__(64 * NW) exact_rows_kernel(float* __restrict__ out, int64_t ldo, const float* __restrict__ A, int64_t lda,
                                                              const float* __restrict__ W, const float* __restrict__ W2, int64_t ldw,
-                                                             const float* __restrict__ bias, double* __restrict__ parts, Cut cut, int per, int M, int N, int K, int gelu) {
-  constexpr int kTiles = NT * kMats, kOut = (NT * 256 + 64 * NW - 1) / (64 * NW);
+                                                             const float* __restrict__ bias, double* __restrict__ parts, Cut cut, int per, int M, int N, int K, int gelu, int own = 0) {
+  constexpr int kTiles = kDealt ? kDealt : NT * kMats, kOut = kDealt ? (kDealt * 128 + 64 * NW - 1) / (64 * NW) : (NT * 256 + 64 * NW - 1) / (64 * NW);
   __shared__ double sums[NW][kTiles][4][64];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
-  const int n0 = blockIdx.x * 16 * NT;
+  const int n0 = blockIdx.x * (kDealt ? own : 16 * NT);
   const bool row_ok = r < M;
   const float* a_row = A + static_cast<int64_t>(row_ok ? r : 0) * lda;
   const float* w_row[kTiles];
 #pragma unroll
   for (int t = 0; t < kTiles; ++t) {
-    const int n = n0 + (t / kMats) * 16 + r;
-    w_row[t] = (t % kMats ? W2 : W) + static_cast<int64_t>(n < N ? n : N - 1) * ldw;      // (rows beyond N: the last one again, not stored)
+    if constexpr (kDealt) {
+      const int q = min(t * 16 + r, 2 * own - 1), n = n0 + (q < own ? q : q - own);
+      w_row[t] = (q < own ? W : W2) + static_cast<int64_t>(n < N ? n : N - 1) * ldw;
+    } else {
+      const int n = n0 + (t / kMats) * 16 + r;
+      w_row[t] = (t % kMats ? W2 : W) + static_cast<int64_t>(n < N ? n : N - 1) * ldw;      // (rows beyond N: the last one again, not stored)
+    }
   }
   // what this thread adds up: output o is place i = threadIdx.x + 64 NW o: tile, weight row 4 v + g', row of A j: (v, 16 g' + j)
   auto place = [&](int o, int& tile, int& v, int& at, int& m, int& n) __attribute__((always_inline)) {
     const int i = threadIdx.x + 64 * NW * o;
+    if constexpr (kDealt) {      // (of gate's row: up's is `own` rows on)
+      const int q = i / 16;
+      tile = q / 16, v = q / 4 % 4, m = i % 16, at = q % 4 * 16 + m, n = n0 + q;
+      return q < own && m < M && n < N;
+    }
     tile = i / 256, v = i / 64 % 4, at = i % 64, m = at % 16, n = n0 + tile * 16 + 4 * v + at / 16;
     return i < NT * 256 && m < M && n < N;
   };
@@ -173,7 +184,8 @@ __global__ void __launch_bounds__(64 * NW) exact_rows_kernel(float* __restrict__
         if (first + w >= last) break;      // (uniform)
 #pragma unroll
         for (int x = 0; x < kMats; ++x) {
-          const double sum = sums[w][tile * kMats + x][v][at];
+          const int up = n - n0 + own;
+          const double sum = !kDealt ? sums[w][tile * kMats + x][v][at] : x == 0 ? sums[w][tile][v][at] : sums[w][up / 16][up / 4 % 4][up % 4 * 16 + m];
           if (parts) parts[(static_cast<int64_t>(first + w) * M + m) * N + n] = sum;
           else total[o][x] += sum;
         }
@@ -453,7 +465,10 @@ static void launch_exact_sum(float* out, int64_t ldo, const double* parts, const
 }
 
 // Up to 16 rows: blocks of eight waves; two tiles of weight rows and four waves a block against a matrix as long as a vocabulary, so that the rows of A are read half as
-// often (8 rows, 151,936 x 896: 113 us; four tiles 130, eight waves 143).
+// often (8 rows, 151,936 x 896: 113 us; four tiles 130, eight waves 143). Gate and up: where their tiles of 16 outputs are more than the compute units but no more than one and a half times as many, a
+// compute unit with two blocks had up to twice the others' work (what it brings in, 37 bytes a nanosecond, and 72 cycles for each float64 instruction). There the outputs are dealt out evenly, 17 to 24 a block, in three tiles
+// that hold gate's rows and then up's (a fourth would be the two blocks' work again). us, blocks of sixteen / dealt out, 1, 8, 16 rows: 4,864 x 896 15.1, 15.4, 16.0 / 12.6, 12.5, 13.0; 5,632 x 2,048
+// 28.4, 30.2, 31.7 / 25.0, 25.4, 26.7; 4,352 x 1,024 15.9, 16.2, 17.0 / 13.1, 13.2, 14.0; 6,144 x 1,024 16.3, 16.6, 17.5 / 15.1, 15.2, 15.6. The bits do not change: a sum's chains are cut by K alone.
 template <int kMats, int kEpilogue, bool kVec>
 static int launch_exact_rows(float* out, int64_t ldo, const float* A, int64_t lda, const float* W, const float* W2, int64_t ldw, const float* bias,
                              double* parts, int M, int N, int K, int gelu, const ExactNorm& norm, hipStream_t stream) {
@@ -464,6 +479,9 @@ static int launch_exact_rows(float* out, int64_t ldo, const float* A, int64_t ld
     launch_exact_sum<kEpilogue>(out, ldo, parts, bias, M, N, cut.count, norm, stream);
   } else if (kMats == 1 && tiles >= 16 * compute_units()) {
     exact_rows_kernel<4, 2, 1, kEpilogue, kVec><<<(tiles + 2 - 1) / 2, 64 * 4, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, nullptr, cut, cut.count, M, N, K, gelu);
+  } else if (const int units = compute_units(); kMats == 2 && tiles > units && 2 * tiles <= 3 * units) {
+    const int own = (N + units - 1) / units;      // (17 to 24)
+    exact_rows_kernel<8, 1, kMats, kEpilogue, kVec, kMats == 2 ? 3 : 0><<<(N + own - 1) / own, 512, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, nullptr, cut, cut.count, M, N, K, gelu, own);
   } else {
     exact_rows_kernel<8, 1, kMats, kEpilogue, kVec><<<tiles, 512, 0, stream>>>(out, ldo, A, lda, W, W2, ldw, bias, nullptr, cut, cut.count, M, N, K, gelu);
   }

@@ -278,3 +278,21 @@ def test_a_decode_step_of_the_exact_path_turns_its_tokens(heads, kv_heads, d, bs
         got.append((out, k.nan_to_num(7.0), v.nan_to_num(7.0)))
     assert all(torch.equal(a, b) for a, b in zip(*got)) and bool(torch.isfinite(got[0][0]).all())
     assert torch.equal(rows, qkv)
+
+
+# gate and up of up to 16 rows dealt out over the compute units (256 here): 17 to 24 outputs a block, the last block with fewer, one before and one behind the range; K ragged and of several rounds of chains
+@pytest.mark.parametrize("M", [1, 8, 16])
+@pytest.mark.parametrize("N,K", [(4096, 64), (4097, 64), (4113, 896), (4864, 896), (4865, 99), (6144, 132), (6145, 64), (5000, 2100)])
+def test_exact_gate_and_up_of_few_rows_dealt_out(M, N, K):
+    gen = torch.Generator(device=DEV).manual_seed(N + K)
+    a, g, u = (torch.randn(s, generator=gen, device=DEV) * K ** -0.25 for s in ((M, K), (N, K), (N, K)))
+    out = torch.full((M, N + 1), 7.0, device=DEV)
+    ops().gemm_swiglu(out[:, :N], a, g, u, exact=True)
+    gate, up = ((a.double() @ w.double().T.contiguous()).cpu().numpy() for w in (g, u))
+    want = gate / (1.0 + np.exp(-gate)) * up
+    within(out[:, :N], want, 4 * np.abs(want) * (1 + np.abs(gate)) + 1e-7)
+    assert bool((out[:, N:] == 7.0).all())
+    for first in (0, N - 1000):      # (the same bits as in blocks of sixteen outputs)
+        part = torch.empty(M, 1000, device=DEV)
+        ops().gemm_swiglu(part, a, g[first:first + 1000].contiguous(), u[first:first + 1000].contiguous(), exact=True)
+        assert torch.equal(part, out[:, first:first + 1000])
