@@ -9,10 +9,10 @@
 // an instruction, and the chains' float64 sums are added in their order. Every form below does so, whichever wave or block has a chain: a row's
 // result is the same bits whatever rows are computed with it.
 //
-//   up to 16 rows (exact_rows_kernel): a block owns 16 weight rows (16 of gate and 16 of up), its waves take a chain each, in runs of 32 k
+//   up to 16 rows (exact_rows_kernel): a block owns 16 weight rows (16 to 24 of gate and as many of up), its waves take a chain each, in runs of 32 k
 //   straight from memory, and meet in LDS. Bound by the rate at which a compute unit takes its weights in and, within it, by the matrix
 //   cores (64 cycles an instruction, 64 weights), so the chains are dealt out over blocks where blocks are few. 8 rows, us, a tile of 64 x 64
-//   on the vector units (one block per 64 columns) / this: 9,728 x 896 with the gate 270 / 14.9, 896 x 4,864 920 / 10.2 with the second
+//   on the vector units (one block per 64 columns) / this: 9,728 x 896 with the gate 270 / 14.9 (12.5 dealt out evenly, launch_exact_rows), 896 x 4,864 920 / 10.2 with the second
 //   launch, 896 x 896 168 / 6.5, 1,152 x 896 170 / 6.5, 151,936 x 896 658 / 113.
 //
 //   more rows (exact_tile_kernel): slabs of 32 k through LDS, a wave owns 32 rows x 32 weight rows (four instructions for two
@@ -466,7 +466,7 @@ static void launch_exact_sum(float* out, int64_t ldo, const double* parts, const
 
 // Up to 16 rows: blocks of eight waves; two tiles of weight rows and four waves a block against a matrix as long as a vocabulary, so that the rows of A are read half as
 // often (8 rows, 151,936 x 896: 113 us; four tiles 130, eight waves 143). Gate and up: where their tiles of 16 outputs are more than the compute units but no more than one and a half times as many, a
-// compute unit with two blocks had up to twice the others' work (what it brings in, 37 bytes a nanosecond, and 72 cycles for each float64 instruction). There the outputs are dealt out evenly, 17 to 24 a block, in three tiles
+// compute unit with two blocks had up to twice the others' work (what it brings in, 37 bytes a nanosecond, and 64 cycles for each float64 instruction). There the outputs are dealt out evenly, 17 to 24 a block, in three tiles
 // that hold gate's rows and then up's (a fourth would be the two blocks' work again). us, blocks of sixteen / dealt out, 1, 8, 16 rows: 4,864 x 896 15.1, 15.4, 16.0 / 12.6, 12.5, 13.0; 5,632 x 2,048
 // 28.4, 30.2, 31.7 / 25.0, 25.4, 26.7; 4,352 x 1,024 15.9, 16.2, 17.0 / 13.1, 13.2, 14.0; 6,144 x 1,024 16.3, 16.6, 17.5 / 15.1, 15.2, 15.6. The bits do not change: a sum's chains are cut by K alone.
 template <int kMats, int kEpilogue, bool kVec>
