@@ -301,8 +301,9 @@ __device__ __forceinline__ void last_slabs(int& k, int slabs, const F& step) {
 // kMfTurn: the columns are heads of 64 channels, query heads, then key heads, then value heads, and a tile is 64 rows of one of them. What rope_kv_write_kernel (elementwise.hip) would do to the rounded
 // outputs happens here on their way out, by way of LDS and with its arithmetic: queries are turned, keys are turned and go to their rows' slots of the cache, values to theirs (`out` keeps
 // neither). Rows' positions and slots are asked for before the first slab, cosines and sines behind the last. What bounds such a product is as before; the rotation's launch, its start and its way through memory are saved. Product and
-// rotation by launches of their own / together, us, weights from memory, 1,152 x 896 at 17, 64, 65, 512, 1,024, 2,048 and 3,072 rows 8.0 / 6.3, 9.9 / 7.7, 10.7 / 7.0, 11.5 / 7.6, 13.9 / 9.8, 19.5 / 13.9,
-// 20.4 / 17.3; 3,072 x 1,536 at 17, 65, 512, 1,024 rows 10.3 / 8.8, 13.5 / 9.4, 20.9 / 16.6, 27.4 / 22.4; 384 x 256 at 17 and 2,048 6.0 / 3.7, 8.3 / 4.6.
+// rotation by launches of their own / together, us, weights from memory, 1,152 x 896 at 65, 512, 1,024, 2,048 and 3,072 rows 10.7 / 7.0, 11.5 / 7.6, 13.9 / 9.8, 19.5 / 13.9,
+// 20.4 / 17.3; 3,072 x 1,536 at 65, 512, 1,024 rows 13.5 / 9.4, 20.9 / 16.6, 27.4 / 22.4; 384 x 256 at 2,048 8.3 / 4.6. For products that are tiled ones by themselves: up to 64 rows of smaller matrices are
+// gemm_skinny.hip's, whose shares of K make other bits (1,152 x 896 at 17 and 64 rows 8.0 / 6.3, 9.9 / 7.7, and the outputs of whole layers 3.50e-3 of their norm from 64 bits where they were 3.35e-3).
 struct TurnArgs {
   const float* cos_t;          // [positions, 32]
   const float* sin_t;
@@ -1082,7 +1083,8 @@ extern "C" int alofa_gemm_mfma(void* out, int o_dtype, int64_t ldo, const void* 
 }
 
 // Whether alofa_gemm_turn takes a product of M rows of [queries | keys | values]: heads of 64 channels and the small tiles, whose 64 columns are then a head. Those are what such a product takes where
-// K is short and the tiles of 128 x 128 are fewer than the compute units (launch_mfma; also where gemm_tall.hip is the faster product by itself: 2,304 x 768 at 1,500 rows 21.0 by two launches, 16.1 so). Up to sixteen
+// K is short and the tiles of 128 x 128 are fewer than the compute units (launch_mfma, whose bits these are; also where gemm_tall.hip is the faster product by itself: 2,304 x 768 at 1,500 rows 21.0 by two launches, 16.1 so). The caller
+// asks only where the tiled kernel is the product's. Up to sixteen
 // rows, and with a long K, the products that share K out are further ahead of these tiles than a launch takes.
 extern "C" int alofa_gemm_turns(int M, int N, int K, int d) {
   return d == 64 && M > 16 && N > 0 && N % 64 == 0 && K > 0 && K % TK == 0 && K < 32 * TK && static_cast<int64_t>((N + 127) / 128) * ((M + 127) / 128) < 256;

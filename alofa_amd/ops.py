@@ -668,15 +668,15 @@ def rope_kv_write(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, posit
 
 def gemm_turned(qkv: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], cos: torch.Tensor, sin: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor,
                 k_cache: torch.Tensor, v_cache: torch.Tensor, heads: int, kv_heads: int, d: int) -> None:
-    """``gemm`` of the rows' queries, keys and values and ``rope_kv_write`` of them. Where the product's tiles are heads (``alofa_gemm_turns``) both are one launch, which leaves the turned queries in ``qkv``,
-    keys and values in the cache alone; otherwise two. The bits are the same."""
+    """``gemm`` of the rows' queries, keys and values and ``rope_kv_write`` of them. Where ``gemm`` takes the tiled kernel and its tiles are heads (``alofa_gemm_turns``) both are one launch, which leaves the
+    turned queries in ``qkv``, keys and values in the cache alone; otherwise two. The bits are the same: up to 64 rows of smaller matrices are the streaming kernel's, which adds K up in another order, and stay with it."""
     sizes = turned = None
     if qkv.dtype is torch.bfloat16:
         sizes, turned = _native().product(qkv, a, w, None, bias), _native().turn(qkv, cos, sin, positions, slots, k_cache, v_cache, heads, kv_heads, d)
     if sizes is not None and turned is not None:
         M, N, K, ldo, lda, ldw, _ = sizes
         page = turned[3]
-        if (load().alofa_gemm_turns(M, N, K, d) and page & (page - 1) == 0 and ldo % 8 == 0 and not (qkv.data_ptr() | cos.data_ptr() | sin.data_ptr() | k_cache.data_ptr()) % 16):
+        if (few_rows_kernel(M, N, K) == "tiled" and load().alofa_gemm_turns(M, N, K, d) and page & (page - 1) == 0 and ldo % 8 == 0 and not (qkv.data_ptr() | cos.data_ptr() | sin.data_ptr() | k_cache.data_ptr()) % 16):
             _call("alofa_gemm_turn", qkv, ldo, a, lda, w, ldw, bias, cos, sin, positions, slots, k_cache, v_cache, M, N, K, heads, kv_heads, page, _stream())
             return
     gemm(qkv, a, w, bias)
