@@ -1817,11 +1817,9 @@ def decay_powers(decay: torch.Tensor) -> torch.Tensor:
     return torch.pow(decay.double()[:, None], torch.arange(CHUNK_ROWS + 1, dtype=torch.float64, device=decay.device)[None, :]).float().contiguous()
 
 
-def can_chunk(q: torch.Tensor, k: torch.Tensor, dk: int, longest: int, per_row: bool = False) -> bool:
-    """Whether a step whose longest portion has so many rows should take a constant decay, or (``per_row``) decays per row and key channel, in chunks, and the kernels take its rows.
-    Decays per row: us, row by row / in chunks, 16 heads of 64 x 64, one request: 64 rows 27 / 29, 96 27 / 30, 128 38 / 30, 192 47 / 30, 500 113 / 33, 2,048 450 / 57; eight of 64 28 / 34, of 96
-    38 / 40; four of 96 to 500 121 / 47; of 128 x 128, one of 96 29 / 40, of 128 36 / 40, of 500 121 / 53, four of 500 192 / 141; two heads of 256 x 256, 128 rows 41 / 54."""
-    return USE_CHUNKS and longest >= (96 + dk // 2 if per_row else CHUNKED_FROM) and q.dtype is torch.bfloat16 and dk % 8 == 0 and _aligned_rows(q) and _aligned_rows(k)
+def can_chunk(q: torch.Tensor, k: torch.Tensor, dk: int, longest: int) -> bool:
+    """Whether a step whose longest portion has so many rows should take a constant decay in chunks, and the kernels take its rows."""
+    return USE_CHUNKS and longest >= CHUNKED_FROM and dk % 8 == 0 and _aligned_rows(q) and _aligned_rows(k)
 
 
 def chunked_recurrence(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Tensor, rows: RowsOfRequests, chunks: Chunks, heads: int,
@@ -1840,30 +1838,6 @@ def chunked_recurrence(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: t
     rows.fits("state", state)
     _call("alofa_chunked_recurrence", _ptr(out), _L(_rows("out", out)), _ptr(q), _L(_rows("q", q)), _ptr(k), _L(_rows("k", k)), _ptr(v), _L(_rows("v", v)), _ptr(state), _ptr(rows.slots),
           _ptr(chunks.chunks), _I(chunks.count), _ptr(chunks.of_request), _I(chunks.requests), _ptr(powers), _ptr(added), _I(heads), _I(dk), _I(dv), _F(q_scale), _F(k_scale), _stream())
-
-
-def chunked_recurrence_decays(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Tensor, rows: RowsOfRequests, chunks: Chunks, heads: int, dk: int, dv: int,
-                              decay_kind: int, decay: torch.Tensor, made: torch.Tensor, totals: torch.Tensor, added: torch.Tensor, tau: float = 1.0, bonus: Optional[torch.Tensor] = None,
-                              q_scale: float = 1.0, k_scale: float = 1.0, before_update: bool = False) -> None:
-    """``chunked_recurrence`` with a decay per row and key channel, as ``linear_recurrence`` takes it (kinds ``DECAY_SIGMOID_ROOT``, ``DECAY_EXP_NEG_EXP``, and ``DECAY_GIVEN`` of decays from 0 to 1;
-    ``decay`` is left as it is). ``made`` float32 [T, heads * dk] and ``totals`` float32 [chunks, heads, dk]: room for the decays and their products over the chunks."""
-    _gpu("out", out, torch.float32, 2), _contig("out", out), _gpu("q", q, torch.bfloat16, 2), _gpu("k", k, torch.bfloat16, 2), _gpu("v", v, torch.bfloat16, 2), _gpu("decay", decay, torch.float32, 2)
-    for name, t, dim in (("state", state, 4), ("made", made, 2), ("totals", totals, 3), ("added", added, 4)):
-        _gpu(name, t, torch.float32, dim), _contig(name, t)
-    T = q.shape[0]
-    if (tuple(q.shape) != (T, heads * dk) or tuple(k.shape) != (T, heads * dk) or tuple(v.shape) != (T, heads * dv) or tuple(out.shape) != (T, heads * dv)
-            or tuple(state.shape[1:]) != (heads, dk, dv) or T != rows.rows or T != chunks.rows or rows.requests != chunks.requests or tuple(decay.shape) != (T, heads * dk)
-            or tuple(made.shape) != (T, heads * dk) or tuple(totals.shape) != (chunks.count, heads, dk) or tuple(added.shape) != (chunks.count, heads, dk, dv)):
-        raise AlofaError("shape_mismatch", "recurrence operands do not fit", f"q={tuple(q.shape)} k={tuple(k.shape)} v={tuple(v.shape)} out={tuple(out.shape)} state={tuple(state.shape)} "
-                         f"decay={tuple(decay.shape)} made={tuple(made.shape)} totals={tuple(totals.shape)} added={tuple(added.shape)} heads={heads} dk={dk} dv={dv} rows={rows.rows} chunks={chunks.count}")
-    if decay_kind not in (DECAY_SIGMOID_ROOT, DECAY_EXP_NEG_EXP, DECAY_GIVEN) or (bonus is None) == before_update:
-        raise AlofaError("shape_mismatch", "a decay per row and channel, and the bonus where the read-out comes before the update", f"kind={decay_kind} bonus={bonus is not None} before={before_update}")
-    if bonus is not None and tuple(_contig("bonus", _gpu("bonus", bonus, torch.float32, 2)).shape) != (heads, dk):
-        raise AlofaError("shape_mismatch", "the bonus is [heads, dk]", f"bonus={tuple(bonus.shape)}")
-    rows.fits("state", state)
-    _call("alofa_chunked_recurrence_decays", _ptr(out), _L(_rows("out", out)), _ptr(q), _L(_rows("q", q)), _ptr(k), _L(_rows("k", k)), _ptr(v), _L(_rows("v", v)), _ptr(decay), _L(_rows("decay", decay)),
-          _ptr(bonus), _ptr(state), _ptr(rows.slots), _ptr(chunks.chunks), _I(chunks.count), _ptr(chunks.of_request), _I(chunks.requests), _ptr(made), _ptr(totals), _ptr(added),
-          _I(heads), _I(dk), _I(dv), _I(decay_kind), _F(tau), _F(q_scale), _F(k_scale), _I(int(before_update)), _stream())
 
 
 def gate_scan(gates: torch.Tensor, z: torch.Tensor, state: torch.Tensor, rows: RowsOfRequests, heads: int, cap: float) -> None:

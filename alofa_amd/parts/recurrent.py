@@ -1,7 +1,7 @@
 """Mixers that keep a state of fixed size per request instead of keys: per head a matrix S [dk, dv] in float32 that
 every token decays and adds to, S_t = diag(w_t) S_(t-1) + k_t v_t^T, and reads out with its query. They differ in
 where the decay comes from and in the order of read-out and update; the recurrence itself is one kernel
-(``ops.linear_recurrence``; for a long portion of a prompt ``ops.chunked_recurrence`` and ``ops.chunked_recurrence_decays``), and so are the norm of every head's read-out with the gate (``ops.headnorm_gate``).
+(``ops.linear_recurrence``; with a constant decay and a long portion of a prompt, ``ops.chunked_recurrence``), and so are the norm of every head's read-out with the gate (``ops.headnorm_gate``).
 
 retention       w = a constant per head; rotary positions on q and k, or none; k scaled by dk^(-1/2); o_t = S_t^T q_t;
                 o / rms(o) per head, times silu(gate), output projection.
@@ -78,18 +78,6 @@ class RecurrentMixer(Mixer):
             ops.chunked_recurrence(o[0], q, k, v, ctx.state(where), rows, chunks, self.heads, self.dk, self.dv, self.powers, added, k_scale=k_scale)
             return 1
         return ops.linear_recurrence(o, q, k, v, ctx.state(where), rows, self.heads, self.dk, self.dv, ops.DECAY_PER_HEAD, self.decay, k_scale=k_scale)
-
-    def _decays(self, ctx, where, o, q, k, v, kind, z, **how) -> int:
-        """The same with decays per row and key channel, made of ``z`` as ``kind`` says."""
-        rows = rows_of_requests(ctx)
-        if ops.can_chunk(q, k, self.dk, ctx.max_q_len, per_row=True):
-            chunks, T = chunks_of_requests(ctx), q.shape[0]
-            made = ctx.scratch("recurrent_decays_made", (T, self.heads * self.dk), torch.float32)
-            totals = ctx.scratch("recurrent_decay_products", (chunks.count, self.heads, self.dk), torch.float32)
-            added = ctx.scratch("recurrent_chunks", (chunks.count, self.heads, self.dk, self.dv), torch.float32)
-            ops.chunked_recurrence_decays(o[0], q, k, v, ctx.state(where), rows, chunks, self.heads, self.dk, self.dv, kind, z, made, totals, added, **how)
-            return 1
-        return ops.linear_recurrence(o, q, k, v, ctx.state(where), rows, self.heads, self.dk, self.dv, kind, z, **how)
 
     def _leave(self, ctx, o, parts, gate, weight, residual, out):
         """Head norm, gate and output projection of the read-outs ``o`` (float32 [P, T, heads * dv], the first ``parts`` to be added)."""
@@ -208,7 +196,8 @@ class GatedLinearAttention(RecurrentMixer):
                              tau=self.tau, q_scale=self.q_scale):
             return
         o = self._readouts(ctx, T)
-        parts = self._decays(ctx, where, o, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:2 * kd + vd], ops.DECAY_SIGMOID_ROOT, self._projected(ctx, *low), tau=self.tau, q_scale=self.q_scale)
+        parts = ops.linear_recurrence(o, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:2 * kd + vd], ctx.state(where), rows_of_requests(ctx),
+                                      self.heads, self.dk, self.dv, ops.DECAY_SIGMOID_ROOT, self._projected(ctx, *low), tau=self.tau, q_scale=self.q_scale)
         self._leave(ctx, o, parts, proj[:, 2 * kd + vd:2 * kd + 2 * vd], self.norm, residual, out)
 
 
@@ -476,7 +465,8 @@ class TimeMix(RecurrentMixer):
                              bonus=self.bonus, before_update=True):
             return
         o = self._readouts(ctx, T)
-        parts = self._decays(ctx, (entry, k), o, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:3 * kd], ops.DECAY_EXP_NEG_EXP, self._projected(ctx, *low), bonus=self.bonus, before_update=True)
+        parts = ops.linear_recurrence(o, proj[:, :kd], proj[:, kd:2 * kd], proj[:, 2 * kd:3 * kd], ctx.state((entry, k)), rows_of_requests(ctx),
+                                      self.heads, self.dk, self.dv, ops.DECAY_EXP_NEG_EXP, self._projected(ctx, *low), bonus=self.bonus, before_update=True)
         self._leave(ctx, o, parts, proj[:, 3 * kd:], self.norm, residual, out)
 
 

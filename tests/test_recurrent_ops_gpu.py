@@ -379,51 +379,6 @@ def test_norm_filter_and_state_at_the_edges_of_its_forms(width, taps):
         assert torch.allclose(got.float(), want, rtol=2 ** -8 if dtype is torch.bfloat16 else 1e-5, atol=1e-4)
 
 
-# runs of sixteen rows and chunks of 64, whole and not; key channels of less than, exactly and more than 64; decays of every size down to zero
-@pytest.mark.parametrize("kind", ["sigmoid_root", "exp_neg_exp", "given"])
-@pytest.mark.parametrize("heads,dk,dv,lengths", [(2, 64, 64, (1, 130)), (1, 8, 16, (17, 64)), (3, 40, 72, (63, 16, 65)), (1, 128, 128, (96, 15)), (2, 72, 20, (200,)), (1, 264, 66, (33, 79))])
-def test_recurrence_in_chunks_with_decays_per_row(heads, dk, dv, lengths, kind):
-    from alofa_amd import ops
-    rng = np.random.default_rng(dk + dv)
-    q, k, v = (pt.to_bfloat16(rng.normal(0, 1, (sum(lengths), heads * n))).astype(np.float32) for n in (dk, dk, dv))
-    z = rng.normal(0.5, 2.0, q.shape).astype(np.float32)
-    bonus = rng.normal(0, 1, (heads, dk)).astype(np.float32) if kind == "exp_neg_exp" else None
-    tau, qs, ks = 3.0, 0.37, 1.9
-    z64 = z.astype(np.float64)
-    if kind == "given":      # zeros, ones and what lies between
-        z = np.where(z > 2.5, 1.0, np.where(z < -2.0, 0.0, 1 / (1 + np.exp(-z64)))).astype(np.float32)
-    w = {"sigmoid_root": lambda: (1 / (1 + np.exp(-z64))) ** (1 / tau), "exp_neg_exp": lambda: np.exp(-np.exp(z64)), "given": lambda: z.astype(np.float64)}[kind]()
-    first = rng.normal(0, 1, (len(lengths) + 1, heads, dk, dv)).astype(np.float32)
-    slots = list(range(len(lengths), 0, -1))      # (slot 0 belongs to nobody)
-    state = dev(first)
-    rows = rows_of(list(zip(slots, lengths)), len(lengths) + 1)
-    offsets = np.concatenate([[0], np.cumsum(lengths)])
-    chunks = ops.Chunks([(int(a), n) for a, n in zip(offsets, lengths)], DEV)
-    room = [torch.full(s, float("nan"), device=DEV) for s in ((len(q), heads * dk), (chunks.count, heads, dk), (chunks.count, heads, dk, dv))]
-    out = torch.full((len(q), heads * dv), float("nan"), device=DEV)
-    code = {"sigmoid_root": ops.DECAY_SIGMOID_ROOT, "exp_neg_exp": ops.DECAY_EXP_NEG_EXP, "given": ops.DECAY_GIVEN}[kind]
-    ops.chunked_recurrence_decays(out, dev(q, torch.bfloat16), dev(k, torch.bfloat16), dev(v, torch.bfloat16), state, rows, chunks, heads, dk, dv, code, dev(z), *room, tau=tau,
-                                  bonus=None if bonus is None else dev(bonus), q_scale=qs, k_scale=ks, before_update=bonus is not None)
-    got, after = out.cpu().numpy(), state.cpu().numpy()
-    assert (after[0] == first[0]).all()
-    for r, (slot, n) in enumerate(zip(slots, lengths)):
-        part = slice(int(offsets[r]), int(offsets[r]) + n)
-        for h in range(heads):
-            kc, vc = slice(h * dk, (h + 1) * dk), slice(h * dv, (h + 1) * dv)
-            S, want = first[slot, h].astype(np.float64), []
-            for t in range(part.start, part.stop):
-                qt, kv = q[t, kc].astype(np.float64) * qs, np.outer(k[t, kc].astype(np.float64) * ks, v[t, vc].astype(np.float64))
-                if bonus is not None:
-                    want.append(qt @ (S + bonus[h].astype(np.float64)[:, None] * kv))
-                S = w[t, kc][:, None] * S + kv
-                if bonus is None:
-                    want.append(qt @ S)
-            want = np.array(want)
-            # float sums of some hundred terms, products of up to 64 decays
-            assert np.abs(got[part, vc] - want).max() <= 2e-5 * max(1.0, np.abs(want).max()), (r, h)
-            assert np.abs(after[slot, h] - S).max() <= 2e-5 * max(1.0, np.abs(S).max()), (r, h)
-
-
 # what rides on the vector-unit product is the same bits as the launches one behind the other: K of one run, several, ragged and (depth) the long form; rows up to eight and, launch by launch, beyond; columns of no whole block
 @pytest.mark.parametrize("M,N,K", [(1, 64, 512), (4, 4096, 1024), (5, 37, 520), (8, 130, 6144), (3, 64, 8192), (12, 96, 1024), (2, 8, 16)])
 def test_products_with_what_follows_them(M, N, K):

@@ -5,6 +5,7 @@ import json
 
 import numpy as np
 import pytest
+import torch
 
 from helpers import assert_close, bulk_and_tail, collect, mixed, portions, random_ids, whole
 from plain import tugalix as pt
@@ -45,7 +46,6 @@ def test_whole_prompt(replayers, tugalix_dirs, name, dtype):
 
 def test_the_stream_after_every_layer(replayers, tugalix_dirs):
     """float32, layer by layer: the engine keeps every layer's output in a stack for its average over depth."""
-    import torch
     name = "A"
     ids = ids_of(name, n=33)
     r = replayers(name, "float32")
@@ -206,6 +206,29 @@ def test_decode_steps_replay_a_captured_graph(replayers, tugalix_dirs):
     got = collect(r, bulk_and_tail("t", ids, tail=30))["t"]
     assert r.fn.graph_replays > before
     assert_close(got, plain_logits(tugalix_dirs[name], tuple(ids)), "bfloat16", "graph decode")
+
+
+def test_decays_per_row_are_taken_row_after_row(replayers, monkeypatch):
+    """Whatever a portion's length: sums over chunks are further from 64 bits than a row's own step (1.1 to 2.2e-7 of the read-outs' norm, 0.8 to 1.3e-7), and a value that is not finite would reach rows in front of it."""
+    from alofa_amd import ops
+    calls, real = [], ops.linear_recurrence
+
+    def counted(o, q, k, v, state, rows, heads, dk, dv, kind, *a, **how):
+        calls.append(kind)
+        if kind != ops.DECAY_PER_HEAD:      # an infinity near the end of a copy of the step: the rows in front of it are what they are without
+            z, row, outs = a[0], q.shape[0] - 7, []
+            for value in (1.0, float("inf")):
+                values, room = v.clone(), torch.empty_like(o)
+                values[row, 0] = value
+                parts = real(room, q, k, values, state.clone(), rows, heads, dk, dv, kind, z.clone(), *a[1:], **how)
+                outs.append(room[:parts])
+            assert torch.equal(outs[0][:, :row], outs[1][:, :row]) and not bool(torch.isfinite(outs[1][:, row, 0]).all())
+        return real(o, q, k, v, state, rows, heads, dk, dv, kind, *a, **how)
+    monkeypatch.setattr(ops, "linear_recurrence", counted)
+    for n in (70, 200):
+        calls.clear()
+        collect(replayers("D", "bfloat16"), whole("w", ids_of("D", n=n)))
+        assert sorted(k for k in calls if k != ops.DECAY_PER_HEAD) == [ops.DECAY_SIGMOID_ROOT, ops.DECAY_EXP_NEG_EXP, ops.DECAY_EXP_NEG_EXP], n
 
 
 def test_the_programs_take_the_design_by_its_config(tugalix_dirs, tmp_path):
