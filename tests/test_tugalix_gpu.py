@@ -231,6 +231,23 @@ def test_decays_per_row_are_taken_row_after_row(replayers, monkeypatch):
         assert sorted(k for k in calls if k != ops.DECAY_PER_HEAD) == [ops.DECAY_SIGMOID_ROOT, ops.DECAY_EXP_NEG_EXP, ops.DECAY_EXP_NEG_EXP], n
 
 
+def test_branches_meet_before_they_join_the_stream(replayers, monkeypatch):
+    """The stream's new rows are its old ones and the branches' sum, rounded once, whatever the branches' scales (E's second pair has scales of one)."""
+    from alofa_amd import ops
+    scales, real = [], ops.add_scaled
+
+    def checked(residual, x, a, y=None, b=0.0, exact=False):
+        want = (residual.double() + (a * x.double() + b * y.double()).float().double()).float() if a == b == 1.0 else None
+        real(residual, x, a, y, b, exact)
+        assert want is None or torch.equal(residual, want)
+        scales.append((a, b))
+    monkeypatch.setattr(ops, "add_scaled", checked)
+    for ids in (ids_of("E", n=40), ids_of("E", n=3)):
+        scales.clear()
+        collect(replayers("E", "bfloat16"), [{"step": 0, "entries": [{"id": "w", "tokens": ids, "want": [len(ids) - 1]}], "end": ["w"]}])
+        assert scales == [(0.3, 2.0), (1.0, 1.0)]
+
+
 def test_the_programs_take_the_design_by_its_config(tugalix_dirs, tmp_path):
     """bin/generate and bin/trace_run on a folder whose config.json names the architecture plainly and leaves the ranks of
     the decay projections to the tensors' shapes."""
