@@ -51,6 +51,12 @@ __device__ __forceinline__ uint32_t pack_bf16x2_rest(float a, float b, uint32_t 
   return pack_bf16x2(a - __uint_as_float(packed << 16), b - __uint_as_float(packed & 0xffff0000u));
 }
 
+// c + a.lo b.lo + a.hi b.hi of bfloat16 pairs (v_dot2_f32_bf16)
+__device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
+  typedef __bf16 pair_t __attribute__((ext_vector_type(2)));
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(pair_t, a), __builtin_bit_cast(pair_t, b), c, false);
+}
+
 __device__ __forceinline__ bf16_t f32_to_bf16(float f) { return static_cast<bf16_t>(pack_bf16x2(f, 0.f) & 0xffffu); }
 __device__ __forceinline__ float round_bf16(float f) { return bf16_to_f32(f32_to_bf16(f)); }
 

@@ -28,8 +28,6 @@
 
 namespace alofa {
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
 enum RowsEpilogue : int { kRwStore = 0, kRwResidual = 1, kRwSwiglu = 2, kRwGeglu = 4, kRwActivated = 5, kRwDepth = 6 };
 
 // What kRwActivated does to an output once it is rounded to bfloat16 (as the activation's own launch reads it: the same bits), activation_of in common.h.
@@ -49,10 +47,6 @@ struct RowsDepth {
 
 constexpr int kRowsMaxWaves = 12;     // runs of 512 along K, one per wave
 constexpr int kRowsMaxK = kRowsMaxWaves * 512;
-
-__device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a), __builtin_bit_cast(bf16x2, b), c, false);
-}
 
 // v of lane l ^ 4 (within a row of 16): the lanes of banks 0 and 2 (four lanes each) read four lanes up,
 // those of banks 1 and 3 four lanes down

@@ -5,8 +5,8 @@
 // parts), norm and gate 2.2 to 4 (4 requests, 16 heads of 64 x 64 in a captured step). What the work cannot do without is the state, read and written once: 16 KB a head.
 // 1 to 64 requests of 1 to 32 heads, 1.01 to 2.2 times as fast, but a few (request, head) pairs of the widest heads, whose state one block reads and writes here: those go launch by launch
 // (recurrence_step_pays in ops.py has the figures).
-// Where the decays come from a projection of few channels (its rank), the block makes its head's share of it too: the launch that was saved took 2.6 us of a captured step, the products hide behind the
-// state's loads.
+// Where the decays come from a projection of few channels (its rank), the block makes its head's share of it too, with the bits of the vector-unit product that makes it by itself: the launch that was
+// saved took 2.6 us of a captured step, the products hide behind the state's loads.
 // A block takes a head of a request. The state's loads set out first (a thread has four neighbouring columns of every so-manieth row, 16 bytes a load), the row's operands are made meanwhile, each
 // once, in LDS; the read-outs' shares meet in LDS in row order. Read-outs stay float up to the norm's end, as they are between the launches.
 #include "common.h"
@@ -36,6 +36,7 @@ struct StepArgs {
 };
 
 constexpr int kStepThreads = 512, kStepMost = 256, kStepRank = 64;      // kStepMost: key and value channels of a head
+static_assert(kStepRank == 64, "eight sums of eight channels meet");
 
 // kRows: rows of the state a thread has at most
 template <int kRows>
@@ -99,18 +100,14 @@ __global__ void __launch_bounds__(kStepThreads) recurrence_step_kernel(StepArgs 
           ws[i] = a.decay[h];
         } else {
           float x = a.decay[r * a.decay_stride + h * dk + i];      // (low: the bias, decay_stride 0)
-          if (projects) {
+          if (projects) {      // (gemm_rows_kernel's sum: eight channels in order, then the lanes' tree)
+            float p[kStepRank / 8];
 #pragma unroll
             for (int n = 0; n < kStepRank / 8; ++n) {
-              const uint32_t u[4] = {lw[n].x, lw[n].y, lw[n].z, lw[n].w}, v[4] = {lx[n].x, lx[n].y, lx[n].z, lx[n].w};
-              if (8 * n < a.rank) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                  x += __uint_as_float(u[e] << 16) * __uint_as_float(v[e] << 16);
-                  x += __uint_as_float(u[e] & 0xffff0000u) * __uint_as_float(v[e] & 0xffff0000u);
-                }
-              }
+              p[n] = dot2(lx[n].w, lw[n].w, dot2(lx[n].z, lw[n].z, dot2(lx[n].y, lw[n].y, dot2(lx[n].x, lw[n].x, 0.f))));
+              if (8 * n >= a.rank) p[n] = 0.f;
             }
+            x = (((p[0] + p[4]) + (p[2] + p[6])) + ((p[1] + p[5]) + (p[3] + p[7]))) + x;
           }
           ws[i] = a.decay_kind == kStepSigmoidRoot ? expf(-(fmaxf(-x, 0.f) + log1pf(expf(-fabsf(x)))) * a.inv_tau) : expf(-expf(x));
         }
@@ -159,7 +156,7 @@ using namespace alofa;
 extern "C" int alofa_recurrence_step_takes(int dk, int dv) { return dk >= 1 && dk <= kStepMost && dv >= 4 && dv <= kStepMost && dv % 4 == 0; }
 
 // out [rows, heads * dv]: the read-outs of one row a request, normed per head, gated. decay: [heads] (decay_kind 0) or z [rows, heads * dk] (1: sigmoid(z)^(1 / tau), 2: exp(-exp(z))); low not null:
-// z = low [rows, rank] low_w [heads * dk, rank]^T + decay [heads * dk], in bfloat16 products and float sums.
+// z = low [rows, rank] low_w [heads * dk, rank]^T + decay [heads * dk] (alofa_gemm_rows' bits).
 extern "C" int alofa_recurrence_step(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v, int64_t v_stride,
                                      const void* gate, int64_t gate_stride, const float* decay, int64_t decay_stride, const void* low, int64_t low_stride, const void* low_w, int64_t low_ld, int rank,
                                      const float* bonus, const float* weight, float* state,

@@ -1744,8 +1744,8 @@ def recurrence_step_pays(requests: int, heads: int, dk: int, dv: int, turned: bo
 
 def recurrence_step_makes_decays(low: torch.Tensor, w: torch.Tensor, bias: torch.Tensor, rows: int, channels: int) -> bool:
     """Whether ``recurrence_step`` takes the decays' projection along: bfloat16 rows ``low`` [rows, rank] and ``w`` [channels, rank] that 16-byte loads can read, a bias. Up to 64 channels of rank: a
-    channel's are one thread's, whose loads are all on their way at once."""
-    return (low.is_cuda and _aligned_rows(low) and low.dim() == 2 and low.shape[0] == rows and w.is_cuda and w.dim() == 2 and _aligned_rows(w) and tuple(w.shape) == (channels, low.shape[1])
+    channel's are one thread's, whose loads are all on their way at once. Only where ``gemm`` would take the vector-unit kernel, whose bits they are."""
+    return (few_rows_kernel(rows, channels, low.shape[-1]) == "rows" and low.is_cuda and _aligned_rows(low) and low.dim() == 2 and low.shape[0] == rows and w.is_cuda and w.dim() == 2 and _aligned_rows(w) and tuple(w.shape) == (channels, low.shape[1])
             and low.shape[1] % 8 == 0 and low.shape[1] <= 64 and bias is not None and bias.is_cuda and bias.dtype is torch.float32 and bias.is_contiguous() and tuple(bias.shape) == (channels,))
 
 
