@@ -139,8 +139,10 @@ __global__ void __launch_bounds__(256) norm_conv_step_kernel(TO* __restrict__ ou
 
 // The same for portions of any lengths: a block takes kConvRows rows of one request, whose norms' sums its wavefronts make first, those of the kTaps - 1 rows in front of them too; a thread then has four
 // channels, filters down the rows and keeps the rows before in registers. The state's old rows are read, and its new ones written, by the request's first block alone (which makes the norms of
-// the request's last rows once more for it), so no other block can find them changed. Three launches did this by way of a float copy of the normed rows: 1,050 rows of 1,024 in four requests, us,
-// launch by launch 20.9 (5.5 + 11 + 4.4, each in a step under the profiler), this 8.3.
+// the request's last rows once more for it), so no other block can find them changed. Three launches did this by way of a float copy
+// of the normed rows, whose bits these are. Rows of up to 2,048 only, which stay in registers; us in captured runs, three launches / this: 1,050 rows of 1,024 in four requests 17.0 / 8.0, one
+// request of 2,048 26.5 / 8.1, of 20 7.7 / 7.7, 1,000 rows of 2,048 23.2 / 11.8, 300 of 64 6.6 / 7.2 (two launches less for the host); read twice, wider rows lose: 512 of 2,052 16.3 / 18.9, of 4,096
+// 25.2 / 25.7, 200 of 8,192 27.1 / 43.
 constexpr int kConvRows = 8;
 template <typename TO, int kTaps, int kOwn>
 __global__ void __launch_bounds__(256) norm_conv_rows_kernel(TO* __restrict__ out, const float* __restrict__ x, const float* __restrict__ nw, const float* __restrict__ nb, float eps,
@@ -150,35 +152,29 @@ __global__ void __launch_bounds__(256) norm_conv_rows_kernel(TO* __restrict__ ou
   const int r = blockIdx.y, row0 = row_off[r], end = row_off[r + 1], c0 = row0 + static_cast<int>(blockIdx.x) * kConvRows;
   if (c0 >= end) return;      // (uniform over the block)
   const int n = min(kConvRows, end - c0), lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, quads = width / 4;
-  // mean and 1 / deviation of rows first + i, i = wave, wave + 4, ..: of those that are there, kEach a wavefront, their values on their way together; rows up to 256 kOwn wide stay in registers
+  // mean and 1 / deviation of rows first + i, i = wave, wave + 4, ..: of those that are there, kEach a wavefront, their values (up to 256 kOwn a row) on their way together.
+  // The sums are layernorm_kernel's (pointwise.hip), bit for bit: four, of channels 64 w .. + 63 of every 256, each over the lanes, then added up in their order.
   auto norms = [&](int first, int count) __attribute__((always_inline)) {
-    float4 own[kEach][kOwn > 0 ? kOwn : 1];
-    const float4* rows[kEach];
+    float own[kEach][4 * kOwn];
 #pragma unroll
     for (int e = 0; e < kEach; ++e) {
-      rows[e] = reinterpret_cast<const float4*>(x + static_cast<int64_t>(min(max(first + min(wave + 4 * e, count - 1), row0), end - 1)) * width);
+      const float* from = x + static_cast<int64_t>(min(max(first + min(wave + 4 * e, count - 1), row0), end - 1)) * width;
 #pragma unroll
-      for (int i = 0; i < kOwn; ++i) own[e][i] = rows[e][min(lane + kWave * i, quads - 1)];
+      for (int j = 0; j < 4 * kOwn; ++j) own[e][j] = from[min(lane + kWave * j, width - 1)];
     }
 #pragma unroll
     for (int e = 0; e < kEach; ++e) {
       if (wave + 4 * e >= count) break;      // (uniform over the wavefront)
-      float s = 0.f, ss = 0.f;
-      if constexpr (kOwn > 0) {
+      auto total = [&](auto term) __attribute__((always_inline)) {
+        float s[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < kOwn; ++i) s += lane + kWave * i < quads ? own[e][i].x + own[e][i].y + (own[e][i].z + own[e][i].w) : 0.f;
-      } else {
-        for (int i = lane; i < quads; i += kWave) s += rows[e][i].x + rows[e][i].y + (rows[e][i].z + rows[e][i].w);
-      }
-      const float mean = wave_sum(s) / static_cast<float>(width);
-      auto squares = [&](float4 v) { return (v.x - mean) * (v.x - mean) + (v.y - mean) * (v.y - mean) + ((v.z - mean) * (v.z - mean) + (v.w - mean) * (v.w - mean)); };
-      if constexpr (kOwn > 0) {
+        for (int j = 0; j < 4 * kOwn; ++j) s[j % 4] = term(s[j % 4], own[e][j], lane + kWave * j < width);
 #pragma unroll
-        for (int i = 0; i < kOwn; ++i) ss += lane + kWave * i < quads ? squares(own[e][i]) : 0.f;
-      } else {
-        for (int i = lane; i < quads; i += kWave) ss += squares(rows[e][i]);
-      }
-      const float var = wave_sum(ss) / static_cast<float>(width);
+        for (int w = 0; w < 4; ++w) s[w] = wave_sum(s[w]);
+        return (((s[0] + s[1]) + s[2]) + s[3]) / static_cast<float>(width);
+      };
+      const float mean = total([](float sum, float v, bool in) { return sum + (in ? v : 0.f); });
+      const float var = total([&](float sum, float v, bool in) { const float d = in ? v - mean : 0.f; return __builtin_fmaf(d, d, sum); });
       if (lane == 0) means[wave + 4 * e] = mean, invs[wave + 4 * e] = 1.f / sqrtf(var + eps);
     }
   };
@@ -690,7 +686,7 @@ extern "C" int alofa_norm_conv_step(void* out, int out_dtype, const float* x, co
   return check_launch("norm_conv_step");
 }
 
-extern "C" int alofa_norm_conv_rows_takes(int width, int taps) { return taps >= 2 && taps <= 4 && width >= 4 && width % 4 == 0; }
+extern "C" int alofa_norm_conv_rows_takes(int width, int taps) { return taps >= 2 && taps <= 4 && width >= 4 && width % 4 == 0 && width <= 2048; }
 
 // longest: rows of the request that brings the most.
 extern "C" int alofa_norm_conv_rows(void* out, int out_dtype, const float* x, const float* nw, const float* nb, float eps, const float* w, float* state, const int32_t* req_slot,
@@ -701,7 +697,7 @@ extern "C" int alofa_norm_conv_rows(void* out, int out_dtype, const float* x, co
   if (requests == 0) return 0;
   const dim3 grid((longest + kConvRows - 1) / kConvRows, requests);
 #define ALOFA_NC(TO, TAPS, OWN) norm_conv_rows_kernel<TO, TAPS, OWN><<<grid, 256, 0, stream>>>(static_cast<TO*>(out), x, nw, nb, eps, w, state, req_slot, row_off, width)
-#define ALOFA_NC_TAPS(TO, TAPS) if (width <= 1024) ALOFA_NC(TO, TAPS, 4); else if (width <= 2048) ALOFA_NC(TO, TAPS, 8); else ALOFA_NC(TO, TAPS, 0)
+#define ALOFA_NC_TAPS(TO, TAPS) if (width <= 1024) ALOFA_NC(TO, TAPS, 4); else ALOFA_NC(TO, TAPS, 8)
   if (out_dtype == kF32) {
     if (taps == 2) { ALOFA_NC_TAPS(float, 2); } else if (taps == 3) { ALOFA_NC_TAPS(float, 3); } else { ALOFA_NC_TAPS(float, 4); }
   } else {

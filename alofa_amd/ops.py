@@ -1633,12 +1633,12 @@ def norm_conv_step(out: torch.Tensor, x: torch.Tensor, norm_w: torch.Tensor, nor
 
 
 def norm_conv_rows_takes(x: torch.Tensor, norm_w: torch.Tensor, norm_b: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether ``norm_conv_rows`` takes these operands: two to four taps, rows in fours of channels, 16-byte aligned."""
+    """Whether ``norm_conv_rows`` takes these operands: two to four taps, rows in fours of up to 2,048 channels, 16-byte aligned."""
     return bool(_answer("alofa_norm_conv_rows_takes", x.shape[1], w.shape[1])) and all(t.data_ptr() % 16 == 0 and t.is_contiguous() for t in (x, norm_w, norm_b, w))
 
 
 def norm_conv_rows(out: torch.Tensor, x: torch.Tensor, norm_w: torch.Tensor, norm_b: torch.Tensor, eps: float, w: torch.Tensor, state: torch.Tensor, rows: RowsOfRequests, longest: int) -> None:
-    """``layernorm``, ``short_conv`` and ``keep_last_rows`` in one launch for portions of any lengths (``longest``: the most rows a request brings), in float: out[t] = n[t] + conv(n)[t], n the layer
+    """``layernorm``, ``short_conv`` and ``keep_last_rows`` in one launch for portions of any lengths (``longest``: the most rows a request brings), in float, with their bits: out[t] = n[t] + conv(n)[t], n the layer
     norm of x; the state (float32 [slots, taps - 1, width]) moves on by n."""
     _gpu("out", out, None, 2), _gpu("x", x, torch.float32, 2), _gpu("w", w, torch.float32, 2), _gpu("state", state, torch.float32, 3)
     _gpu("norm_w", norm_w, torch.float32, 1), _gpu("norm_b", norm_b, torch.float32, 1)

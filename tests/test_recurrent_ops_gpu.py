@@ -447,8 +447,8 @@ def test_single_row_step_that_makes_its_decays(heads, dk, dv, kind, rank, n):
     assert torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][0], got[1][0]) and torch.equal(got[1][1][0], first[0])
 
 
-# portions of one row, of fewer rows than the state keeps, of a block's rows and one more, and long ones; widths that stay in registers and wider ones
-@pytest.mark.parametrize("width", [4, 1020, 1024, 1028, 2048, 2052])
+# portions of one row, of fewer rows than the state keeps, of a block's rows and one more, and long ones; the widths at the edges of either form; the bits of three launches
+@pytest.mark.parametrize("width", [4, 64, 260, 1020, 1024, 1028, 2044, 2048])
 @pytest.mark.parametrize("taps", [2, 3, 4])
 def test_norm_filter_and_state_of_portions_in_one_launch(width, taps):
     from alofa_amd import ops
@@ -459,6 +459,7 @@ def test_norm_filter_and_state_of_portions_in_one_launch(width, taps):
     state = dev(rng.normal(0, 1, (8, taps - 1, width)))
     rows = rows_of(list(zip(slots, lengths)), 8)
     assert ops.norm_conv_rows_takes(x, nw, nb, w)
+    assert not ops.norm_conv_rows_takes(torch.empty(3, 2052, device=DEV), torch.empty(2052, device=DEV), torch.empty(2052, device=DEV), torch.empty(2052, taps, device=DEV))      # (three launches are faster)
     # launch by launch, and in float64
     wide, old, old_state = torch.empty_like(x), torch.empty_like(x), state.clone()
     ops.layernorm(wide, x, nw, nb, 1e-5, False)
@@ -476,7 +477,7 @@ def test_norm_filter_and_state_of_portions_in_one_launch(width, taps):
     for dtype in (torch.float32, torch.bfloat16):
         out, got_state = torch.empty(T, width, device=DEV, dtype=dtype), state.clone()
         ops.norm_conv_rows(out, x, nw, nb, 1e-5, w, got_state, rows, max(lengths))
-        off, off_old = (out.double() - want).norm() / want.norm(), (old.to(dtype).double() - want).norm() / want.norm()
-        assert off < 2 ** -8 and off <= 1.5 * off_old + 1e-7      # (as close to 64 bits as the launches one behind the other, whose sums run in another order)
-        assert (got_state.double() - want_state).abs().max() <= 1.5 * (old_state.double() - want_state).abs().max() + 1e-6
+        assert torch.equal(out, old.to(dtype)) and torch.equal(got_state, old_state)
+        assert (out.double() - want).norm() / want.norm() < (2 ** -8 if dtype is torch.bfloat16 else 1e-6)
+        assert (got_state.double() - want_state).abs().max() <= 1e-5 * want_state.abs().max()
         assert torch.equal(got_state[4], state[4])
