@@ -269,7 +269,9 @@ class ResidentLayers:
             ops.check_caches(t[-2], t[-1], self.kv_heads, self.d)
         self._tables = tables      # (kept: the table on the GPU holds their addresses)
         self._model, self._tiles, self._addresses = model, None, [[0 if t is None else t.data_ptr() for t in ts] for ts in tables]
-        self._table = torch.tensor(self._addresses, dtype=torch.int64, device=device)
+        # the layers' addresses on the GPU, and behind them, for more rows than sixteen, those with gate, up and down in tiles (once these are laid out). Launches read it whenever they run, captured ones as
+        # long as their graphs live: it is made once and never moves
+        self._table = torch.tensor([self._addresses] * 2 if self.most_rows > self.MOST_ROWS else self._addresses, dtype=torch.int64, device=device)
         self.failed = area.failed
         self._failed = self.failed.numpy()
         self.turn = _turns.setdefault(device.index, _Turns(device))      # what a launch, or a replay of one, goes within
@@ -288,14 +290,14 @@ class ResidentLayers:
 
     @property
     def layers(self) -> torch.Tensor:
-        """The layers' addresses on the GPU, the second time with gate, up and down in tiles, which more rows than sixteen read: laid out when they are first asked for."""
+        """The layers' addresses on the GPU. Gate, up and down in tiles, which more rows than sixteen read, are laid out when they are first asked for."""
         if self._tiles is None and self.most_rows > self.MOST_ROWS:
             self._tiles = _Tiles.of(self._model, [w for ts in self._tables for w in ts[3:6]])
             if self._tiles is None:
                 self.most_rows = self.MOST_ROWS
             else:
                 places = [t.data_ptr() for t in self._tiles.copies]
-                self._table = torch.tensor([self._addresses, [[*a[:3], *places[3 * i:3 * i + 3], *a[6:]] for i, a in enumerate(self._addresses)]], dtype=torch.int64, device=self.device)
+                self._table[1].copy_(torch.tensor([[*a[:3], *places[3 * i:3 * i + 3], *a[6:]] for i, a in enumerate(self._addresses)], dtype=torch.int64))
         return self._table
 
     def ready(self, rows: int) -> bool:

@@ -17,6 +17,53 @@ def test_where_a_value_lies_in_tiles(n, k):
     assert ops.in_tiles(w, again) is again and torch.equal(again.view(-1), flat)
 
 
+def test_the_addresses_that_captured_steps_read_stay_where_they_are(monkeypatch):
+    """A captured launch has the place of the layers' addresses in it: laying the tiles out moves nothing that it reads."""
+    from types import SimpleNamespace as Some
+    from alofa_amd import ops
+    from alofa_amd.engine import resident
+    monkeypatch.setattr(resident, "_areas", resident._Areas()), monkeypatch.setattr(resident, "_turns", {})
+    monkeypatch.setattr(ops, "resident_rows", lambda *a: 64), monkeypatch.setattr(ops, "check_caches", lambda *a: None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: Some(synchronize=lambda: None)), monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: None)
+    mixer = Some(heads=4, kv_heads=1, d=64, scale=1.0, position=None, hidden=256, b_qkv=None)
+    block = Some(mixer=mixer, feed_forward=Some(intermediate=512), norms=[Some(as_rmsnorm=lambda: (None, 1e-6))] * 2)
+    tables = [[torch.zeros(1), None, torch.zeros(1), torch.zeros(512, 256), torch.zeros(512, 256), torch.zeros(256, 512), *(torch.zeros(1) for _ in range(4))] for _ in range(3)]
+    model, cache = Some(tiles=None, written=0), Some(block_size=16, group_of_entry={(0, 0): 0})
+    layers = resident.ResidentLayers(model, [block] * 3, cache, torch.device("cpu"), tables, Some(failed=torch.zeros(1, dtype=torch.int32), address=0))
+    held, at = layers._table, layers._table.data_ptr()
+    before = held[0].clone()
+    assert layers.ready(16) and layers._tiles is None
+    assert layers.ready(17) and layers._tiles is not None
+    assert layers._table is held and held.data_ptr() == at and torch.equal(held[0], before)
+    assert [held[1, i, 3:6].tolist() for i in range(3)] == [[t.data_ptr() for t in layers._tiles.copies[3 * i:3 * i + 3]] for i in range(3)]
+    assert torch.equal(held[1][:, [0, 1, 2, 6, 7, 8, 9]], before[:, [0, 1, 2, 6, 7, 8, 9]])
+
+
+@pytest.mark.gpu
+def test_a_captured_step_of_few_rows_behind_one_of_many():
+    """Sixteen rows captured, seventeen, for which tiles are laid out, small tensors that take whatever memory was given back, and the captured steps of sixteen again: beside an engine whose tiles were
+    there before its first step."""
+    from test_resident_gpu import decode, engine, model, stand
+    m, lengths = model(896, 14, 2, 1024, "bfloat16"), [11 * i for i in range(17)]
+    tokens = np.random.default_rng(5).integers(0, 500, (9, 17)).tolist()
+    steps = [tokens[i][:17 if i in (3, 7) else 16] for i in range(9)]
+    got = []
+    for first in (False, True):
+        m[1].tiles = None
+        e = engine(m, 17, 400, "bfloat16")
+        if first:
+            assert e.step_fn.resident.ready(17)
+        stand(e, lengths, 1)
+        out = decode(e, steps[:4])
+        replays = e.step_fn.graph_replays
+        held = [torch.full((n,), -1, dtype=torch.int64, device="cuda") for n in (30, 60, 60, 120, 250)]
+        out += decode(e, steps[4:])
+        assert e.step_fn.graph_replays == replays + 5 and all(bool((t == -1).all()) for t in held)
+        got.append(out)
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows", [17, 40])
 def test_matrices_written_in_place_are_laid_out_again(rows):
