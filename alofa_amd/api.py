@@ -38,7 +38,8 @@ class Engine:
         tick before only after its own step is launched (``EngineCore``); off, every tick is synchronous.
         ``memory_fraction`` (with no ``kv_blocks``): the pool of the layers that keep every key takes this share
         of the device memory that is free once the weights are loaded (less what the windowed layers' pools take),
-        instead of what ``max_batch`` requests of ``max_tokens`` need.
+        instead of what ``max_batch`` requests of ``max_tokens`` need. What it leaves is what the steps' scratch grows into and, where that is twice
+        their size, what copies of the feed-forward matrices are laid out in when decode steps of more than sixteen requests first come (engine/resident.py).
         ``max_chunk``: the most prompt tokens of one request in a tick; by default the whole ``token_budget``,
         so that a lone long prompt takes one step (requests are served in order of arrival either way, and the
         budget alone bounds a tick's length)."""

@@ -7,9 +7,11 @@
 // weights no longer fit the registers: gate, up and down go through a ring of fragments in a phase, the first of them asked for before the phase's values are waited for, as all weights are there.
 // A compute unit takes a fragment of a row-major matrix (1 KB, sixteen rows' 64 bytes: sixteen lanes in a row bring sixteen lines) in 27 ns however many are on their way, 37 bytes a nanosecond, 1 KB
 // in one piece in 10 to 17: gate and up's 280 fragments of a block at four groups 7.5 us, down's 140 3.8. So these matrices come laid out in tiles, fragment behind fragment as the matrix cores take them
-// (ops.in_tiles: copies, 26 MB a layer at the 0.5B sizes, made once per model when a step first needs them), and blocks take whole tiles of them. Eight steps of the 0.5B sizes with logits behind
+// (kTiled; ops.in_tiles: copies, 26 MB a layer at the 0.5B sizes, made once per model when a step first needs them), and blocks take whole tiles of them; where there is no room for copies
+// a step reads these as they are: the same bits. Eight steps of the 0.5B sizes with logits behind
 // the last, us, rows of the matrices / tiles: 64 rows of 128 to 2,048 keys 8,194 / 7,300, of 64 to 256 7,502 / 6,543, of 3,300 to 4,000 11,361 / 10,381, 48 of 128 to 1,024 7,372 / 6,485, 33 of 64 to 512
-// 7,068 / 6,195, 32 of 128 to 1,024 6,055 / 5,795, 17 of 64 to 700 5,711 / 5,405. Loads marked as read once (nt) lose half of it at four groups (7,806 for 7,374): the L2's other three readers; past the L1 (sc0) is even.
+// 7,068 / 6,195, 32 of 128 to 1,024 6,055 / 5,795, 17 of 64 to 700 5,711 / 5,405. Other widths (256 to 1,024) and feed-forwards (512 to 5,120), 12 layers, rows of 100 to 290 keys: 1.00 to 1.07 times as fast
+// at 17 and 32 rows, 1.06 to 1.18 at 33 and 64. Loads marked as read once (nt) lose half of it at four groups (7,806 for 7,374): the L2's other three readers; past the L1 (sc0) is even.
 //
 // A step of the 0.5B sizes before that (24 layers; the head's 70 us among them), us, kernel by kernel / this: 17 rows of 64 to 700 keys 1,101 / 712, 32 of 128 to 1,024 1,185 / 754, 48 of 128 to 1,024
 // 1,312 / 917, 64 of 128 to 2,048 1,363 / 1,023, 64 of 3,300 to 4,000 1,676 / 1,360. Other widths from 256 (one key head) to 1,024 (four), 24 layers, 17 to 64 rows of 200 to 1,000 keys: 1.25 to 1.83 times
@@ -23,7 +25,7 @@
 //   * Several output tiles a wave and K over four waves instead of eight: gate's tiles are four waves', up's the other four's.
 //   * Phase B is decode_resident.hip's with values by sixteen bytes: masks, the new token's place and the states' end are the same in both.
 //
-// The compiler keeps two registers of a lane in memory (12 bytes; decode_resident.hip has none, whose comment says what one costs there; here it was not
+// The compiler keeps two registers of a lane in memory (12 bytes; three, 16, with four groups and the matrices as they are; decode_resident.hip has none, whose comment says what one costs there; here it was not
 // measured apart). A block's LDS, 64,580 and 80,964 bytes, leaves room for another launch's block in the compute unit (kLdsOf).
 #include "resident.h"
 
@@ -38,13 +40,14 @@ constexpr int kColumnPlaces = kResMaxWidth;             // of down's sums: a sha
 constexpr int kQkvMost = 2048;                          // columns of queries, keys and values
 static_assert(kRowPlaces <= kResMaxWidth && kQkvMost <= 4096, "the places lie where decode_resident.hip has them");
 
-template <int G, int GS>
+// kTiled: gate, up and down laid out in tiles
+template <int G, int GS, bool kTiled>
 __global__ void __launch_bounds__(kResThreads, 4) decode_groups_kernel(ResidentArgs a) {
   constexpr int d = 64, MB = kResMaxRows, NB = kResBlocks / G;      // NB: blocks of a group
   constexpr int QT = G == 4 ? 2 : 1, QK = 8 / QT, QS = 32 / QK;     // queries, keys, values: tiles, waves that share K, steps of a wave
   constexpr int GT = G == 4 ? 5 : 3;                                // gate and up: tiles of either; K over four waves, GS steps each at most
   constexpr int DT = G == 4 ? 4 : 2, DS = 5;                        // down: tiles of half of the waves, steps of a wave
-  constexpr int kRing = 16, kFirst = G == 4 ? 4 : 8, kBefore = G == 4 ? 8 : 10;                             // fragments of a wave on their way, and of them before attention's values are there
+  constexpr int kRing = 16, kFirst = kTiled && G == 4 ? 4 : 8, kBefore = kTiled && G == 4 ? 8 : 10;                             // fragments of a wave on their way, and of them before attention's values are there
   constexpr int kLdx = kResMaxWidth + 8;
   constexpr int kStates = kResWaves * kResMaxGroup * (d + 4), kSums = 2 * GT * 4 * 256, kQsAt = kStates;
   static_assert(kSums * 4 >= (kStates + 10 * 72 / 2) * 4, "queries lie behind the attention states");
@@ -127,15 +130,23 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_groups_kernel(ResidentA
   };
   auto qkv_columns = [&]() __attribute__((always_inline)) { return run_of(NQ); };
   auto own_pairs = [&]() __attribute__((always_inline)) { return run_of(H / 2); };
-  // gate, up and down are dealt out in whole tiles of sixteen rows of theirs
+  // gate, up and down in tiles are dealt out in whole ones, of sixteen rows of theirs
   auto act_tiles = [&]() __attribute__((always_inline)) { return run_of(FF / 16); };      // (none where the tiles are fewer than the blocks)
-  auto act_pairs = [&]() __attribute__((always_inline)) { const auto [t0, nt] = act_tiles(); return Run{8 * t0, 8 * nt}; };
+  auto act_pairs = [&]() __attribute__((always_inline)) {
+    if constexpr (!kTiled) return run_of(FF / 2);
+    const auto [t0, nt] = act_tiles();
+    return Run{8 * t0, 8 * nt};
+  };
   auto down_tiles = [&]() __attribute__((always_inline)) {
     constexpr int kParts = NB / kResShares;
     const int part = s / kResShares, first = static_cast<int>(static_cast<uint32_t>(part * (H / 16)) / kParts);
     return Run{first, static_cast<int>(static_cast<uint32_t>((part + 1) * (H / 16)) / kParts) - first};
   };
-  auto down_columns = [&]() __attribute__((always_inline)) { const auto [t0, nt] = down_tiles(); return Run{16 * t0, 16 * nt}; };
+  auto down_columns = [&]() __attribute__((always_inline)) {
+    if constexpr (!kTiled) return Run{(s / kResShares) * (H * kResShares / NB), H * kResShares / NB};
+    const auto [t0, nt] = down_tiles();
+    return Run{16 * t0, 16 * nt};
+  };
   auto share_of = [&]() __attribute__((always_inline)) { return s % kResShares; };
   auto share_length = [&]() __attribute__((always_inline)) { return FF / kResShares; };
 
@@ -192,13 +203,25 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_groups_kernel(ResidentA
   constexpr auto step_at = [](int i, int tiles, int n) { return i / (2 * tiles) * 2 + 1 < n ? i / (2 * tiles) * 2 + i % 2 : n - 1; };
   constexpr auto tile_at = [](int i, int tiles, int n) { return i / (2 * tiles) * 2 + 1 < n ? i / 2 % tiles : i % (2 * tiles); };
   auto fetch_gate_up = [&](u32x4& to, const ResidentLayer& layer, int i) __attribute__((always_inline)) {
-    const auto [t0, nt] = act_tiles();
     const int step = run_step(step_at(i, GT, GS), H / 32), tile = tile_at(i, GT, GS);
+    if constexpr (!kTiled) {
+      const auto [p0, np] = act_pairs();
+      gbytes from = (wave < 4 ? layer.w_gate : layer.w_up) + static_cast<int64_t>(2 * p0) * H * 2;
+      to = load_global<u32x4>(from + (step >= 0 ? step : 0) * 64 + row_at(tile * 16 + c16, 2 * np, H));
+      return;
+    }
+    const auto [t0, nt] = act_tiles();
     to = load_global<u32x4>((wave < 4 ? layer.w_gate : layer.w_up) + static_cast<uint32_t>((t0 + (tile < nt ? tile : nt > 0 ? nt - 1 : 0)) * (H / 32) + (step >= 0 ? step : 0)) * 1024u + lane * 16);
   };
   auto fetch_down = [&](u32x4& to, const ResidentLayer& layer, int i) __attribute__((always_inline)) {
-    const auto [t0, nt] = down_tiles();
     const int steps = share_length() / 32, step = run_step(step_at(i, DT, DS), steps), tile = (wave >> 2) * DT + tile_at(i, DT, DS);
+    if constexpr (!kTiled) {
+      const auto [f0, nf] = down_columns();
+      gbytes from = layer.w_down + (static_cast<int64_t>(f0) * FF + share_of() * share_length()) * 2;
+      to = load_global<u32x4>(from + (step >= 0 ? step : 0) * 64 + row_at(tile * 16 + c16, nf, FF));
+      return;
+    }
+    const auto [t0, nt] = down_tiles();
     to = load_global<u32x4>(layer.w_down + static_cast<uint32_t>((t0 + (tile < nt ? tile : nt - 1)) * (FF / 32) + share_of() * steps + (step >= 0 ? step : 0)) * 1024u + lane * 16);
   };
 
@@ -681,29 +704,30 @@ __global__ void __launch_bounds__(kResThreads, 4) decode_groups_kernel(ResidentA
   if (s == 0 && tid == 0) __hip_atomic_store(area, static_cast<u64>(base + a.n_layers), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int G>
+template <int G, bool kTiled>
 static void launch_steps(const ResidentArgs& a, hipStream_t stream) {      // (by the steps of a wave's run of a row: 512, 896 and 1,024 columns)
-  if (a.H <= 512) decode_groups_kernel<G, 4><<<kResBlocks, kResThreads, 0, stream>>>(a);
-  else if (a.H <= 896) decode_groups_kernel<G, 7><<<kResBlocks, kResThreads, 0, stream>>>(a);
-  else decode_groups_kernel<G, 8><<<kResBlocks, kResThreads, 0, stream>>>(a);
+  if (a.H <= 512) decode_groups_kernel<G, 4, kTiled><<<kResBlocks, kResThreads, 0, stream>>>(a);
+  else if (a.H <= 896) decode_groups_kernel<G, 7, kTiled><<<kResBlocks, kResThreads, 0, stream>>>(a);
+  else decode_groups_kernel<G, 8, kTiled><<<kResBlocks, kResThreads, 0, stream>>>(a);
 }
 
-int launch_groups(const ResidentArgs& a, hipStream_t stream) {
-  if (a.M <= 32) launch_steps<2>(a, stream);
-  else launch_steps<4>(a, stream);
+int launch_groups(const ResidentArgs& a, bool tiled, hipStream_t stream) {
+  if (a.M <= 32) tiled ? launch_steps<2, true>(a, stream) : launch_steps<2, false>(a, stream);
+  else tiled ? launch_steps<4, true>(a, stream) : launch_steps<4, false>(a, stream);
   return check_launch("decode_groups");
 }
 
 }  // namespace alofa
 
-// The most rows of a step of a model that alofa_resident_takes: sixteen, or as many as the groups hold of it.
+// The most rows of a step of a model that alofa_resident_takes: sixteen, or as many as the groups hold of it, with the matrices as they are and in tiles alike.
 extern "C" int alofa_resident_rows(int H, int FF, int heads, int kv_heads) {
   using namespace alofa;
   auto fits = [&](int groups) {
     const int blocks = kResBlocks / groups, gate_tiles = groups == 4 ? 5 : 3, down_tiles = groups == 4 ? 4 : 2, qkv_tiles = groups == 4 ? 2 : 1;
     auto most = [&](int n) { return (n + blocks - 1) / blocks; };
-    return H / 2 >= blocks && 2 * most(H / 2) <= 16 && (heads + 2 * kv_heads) * 64 <= kQkvMost && most((heads + 2 * kv_heads) * 64) <= 16 * qkv_tiles && FF % 16 == 0 && most(FF / 16) <= gate_tiles &&
-           FF / kResShares <= 20 * 32 && H % 16 == 0 && (H / 16 * kResShares + blocks - 1) / blocks <= 2 * down_tiles && kv_heads * kResMaxRows <= blocks && kResMaxRows * heads <= kResWaves * blocks;
+    return H / 2 >= blocks && 2 * most(H / 2) <= 16 && (heads + 2 * kv_heads) * 64 <= kQkvMost && most((heads + 2 * kv_heads) * 64) <= 16 * qkv_tiles && FF % 16 == 0 && 2 * most(FF / 2) <= 16 * gate_tiles &&
+           most(FF / 16) <= gate_tiles && FF / kResShares <= 20 * 32 && H % 16 == 0 && H * kResShares / blocks <= 32 * down_tiles && (H / 16 * kResShares + blocks - 1) / blocks <= 2 * down_tiles &&
+           kv_heads * kResMaxRows <= blocks && kResMaxRows * heads <= kResWaves * blocks;
   };
   return !fits(2) ? kResMaxRows : !fits(4) ? 2 * kResMaxRows : 4 * kResMaxRows;
 }

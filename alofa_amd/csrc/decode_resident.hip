@@ -664,19 +664,20 @@ extern "C" int alofa_resident_takes(int H, int FF, int heads, int kv_heads, int 
 
 // hidden [M, H] float32, in and out; layers: n_layers x ten pointers (ResidentLayer) in device memory; positions [M], table [M, max_blocks], slots [M]: the new token's
 // place per row, row i request i; cos, sin [positions, 32]; area: of alofa_resident_area, of one launch at a time; failed: an int in memory that the host reads, set if a wait is given up;
-// limit: after how many asks (0: kLimit).
+// limit: after how many asks (0: kLimit). tiled (more than sixteen rows): the layers' gate, up and down are laid out in tiles (decode_groups.hip).
 extern "C" int alofa_decode_resident(float* hidden, const void* layers, const int32_t* positions, const int32_t* table, const int64_t* slots, const float* cos_t,
                                      const float* sin_t, void* area, int* failed, int n_layers, int M, int H, int FF, int heads, int kv_heads, int d, int page, int max_blocks,
-                                     int has_bias, int limit, float scale, float eps0, float eps1, hipStream_t stream) {
+                                     int has_bias, int limit, int tiled, float scale, float eps0, float eps1, hipStream_t stream) {
   using namespace alofa;
   ALOFA_REQUIRE(alofa_resident_takes(H, FF, heads, kv_heads, d, page) && M >= 1 && M <= alofa_resident_rows(H, FF, heads, kv_heads) && (M > kResMaxRows || (M * kv_heads <= kResBlocks && M * heads <= kResBlocks)) && n_layers > 0 && n_layers <= kResMaxLayers && max_blocks > 0,
                 "decode_resident: sizes beyond what a block holds (M=%d H=%d FF=%d heads=%d/%d d=%d page=%d)", M, H, FF, heads, kv_heads, d, page);
+  ALOFA_REQUIRE(!tiled || M > kResMaxRows, "decode_resident: up to %d rows read the matrices as they are", kResMaxRows);
   ALOFA_REQUIRE(hidden && layers && positions && table && slots && cos_t && sin_t && area && failed, "decode_resident: an operand is missing");
   int shift = 0;
   while ((1 << shift) < page) ++shift;
   const ResidentArgs a = {hidden, static_cast<const ResidentLayer*>(layers), positions, table, slots, cos_t, sin_t, static_cast<u64*>(area), failed, n_layers, M, H, FF, heads, kv_heads,
                           max_blocks, shift, alofa_resident_parts(M, kv_heads), has_bias, limit > 0 ? limit : kLimit, scale, eps0, eps1};
-  if (M > kResMaxRows) return launch_groups(a, stream);
+  if (M > kResMaxRows) return launch_groups(a, tiled != 0, stream);
   if (M == 1) return launch_resident<1>(a, stream);
   if (M == 2) return launch_resident<2>(a, stream);
   if (M <= 4) return launch_resident<4>(a, stream);

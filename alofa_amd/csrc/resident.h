@@ -128,8 +128,8 @@ struct Wait {      // of one wave: the area as a buffer resource (reads past the
   }
 };
 
-// (decode_groups.hip) more than sixteen rows
-int launch_groups(const ResidentArgs& a, hipStream_t stream);
+// (decode_groups.hip) more than sixteen rows; tiled: the layers' gate, up and down are laid out in tiles
+int launch_groups(const ResidentArgs& a, bool tiled, hipStream_t stream);
 
 }  // namespace alofa
 

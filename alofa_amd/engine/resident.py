@@ -150,9 +150,10 @@ _turns: dict = {}      # GPU -> its launches' turns
 class _Tiles:
     """Copies of a model's gate, up and down matrices as more than sixteen rows read them (``ops.in_tiles``): made once per model, for all its step functions, and again where the matrices have been
     written since."""
+    ROOM = 2      # times their size that must be free before they are laid out: the rest is what a service's scratch grows into
 
     def __init__(self, sources: list):
-        self._sources = sources
+        self._sources, self._lock = sources, threading.Lock()
         versions = self._now()
         self.copies = [ops.in_tiles(w) for w in sources]
         torch.cuda.current_stream(sources[0].device).synchronize()      # (steps on other streams read them too)
@@ -165,23 +166,36 @@ class _Tiles:
         return sum(t.numel() * t.element_size() for t in self.copies)
 
     def follow(self) -> None:
-        now = self._now()
-        if now != self._versions:
-            for w, to in zip(self._sources, self.copies):
-                ops.in_tiles(w, to)
-            torch.cuda.current_stream(self._sources[0].device).synchronize()
-            self._versions = now
+        if self._now() == self._versions:
+            return
+        with self._lock:
+            now = self._now()
+            if now != self._versions:
+                device = self._sources[0].device
+                torch.cuda.synchronize(device)      # (steps of other streams that are on their way read what is there now)
+                for w, to in zip(self._sources, self.copies):
+                    ops.in_tiles(w, to)
+                torch.cuda.current_stream(device).synchronize()
+                self._versions = now
 
     @staticmethod
     def of(model, sources: list) -> Optional["_Tiles"]:
-        """None where there is no memory for them (the kernels one by one need none)."""
-        have = model.tiles
-        if have is None or len(have._sources) != len(sources) or any(a is not b for a, b in zip(have._sources, sources)):
-            try:
-                model.tiles = _Tiles(sources)
-            except torch.cuda.OutOfMemoryError:
-                return None
-        return model.tiles
+        """None where the matrices are read as they are instead: where there is no memory to spare."""
+        with _laying_out:
+            have = model.tiles
+            if have is None or len(have._sources) != len(sources) or any(a is not b for a, b in zip(have._sources, sources)):
+                device = sources[0].device
+                free = torch.cuda.mem_get_info(device)[0] + torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+                if free < _Tiles.ROOM * sum(w.numel() * w.element_size() for w in sources):
+                    return None
+                try:
+                    model.tiles = _Tiles(sources)
+                except torch.cuda.OutOfMemoryError:
+                    return None
+            return model.tiles
+
+
+_laying_out = threading.Lock()
 
 
 class ResidentLayers:
@@ -268,10 +282,11 @@ class ResidentLayers:
         for t in tables:
             ops.check_caches(t[-2], t[-1], self.kv_heads, self.d)
         self._tables = tables      # (kept: the table on the GPU holds their addresses)
-        self._model, self._tiles, self._addresses = model, None, [[0 if t is None else t.data_ptr() for t in ts] for ts in tables]
+        self._model, self._tiles, self._asked, self._addresses = model, None, False, [[0 if t is None else t.data_ptr() for t in ts] for ts in tables]
         # the layers' addresses on the GPU, and behind them, for more rows than sixteen, those with gate, up and down in tiles (once these are laid out). Launches read it whenever they run, captured ones as
         # long as their graphs live: it is made once and never moves
         self._table = torch.tensor([self._addresses] * 2 if self.most_rows > self.MOST_ROWS else self._addresses, dtype=torch.int64, device=device)
+        self._few = self._table if self._table.dim() == 2 else self._table[0]
         self.failed = area.failed
         self._failed = self.failed.numpy()
         self.turn = _turns.setdefault(device.index, _Turns(device))      # what a launch, or a replay of one, goes within
@@ -290,24 +305,21 @@ class ResidentLayers:
 
     @property
     def layers(self) -> torch.Tensor:
-        """The layers' addresses on the GPU. Gate, up and down in tiles, which more rows than sixteen read, are laid out when they are first asked for."""
-        if self._tiles is None and self.most_rows > self.MOST_ROWS:
-            self._tiles = _Tiles.of(self._model, [w for ts in self._tables for w in ts[3:6]])
-            if self._tiles is None:
-                self.most_rows = self.MOST_ROWS
-            else:
-                places = [t.data_ptr() for t in self._tiles.copies]
+        """The layers' addresses as ``ops.decode_resident`` takes them. Gate, up and down in tiles, which more rows than sixteen read where there is room for them, are laid out when they are first asked for."""
+        if not self._asked and self.most_rows > self.MOST_ROWS and not torch.cuda.is_current_stream_capturing():
+            tiles = _Tiles.of(self._model, [w for ts in self._tables for w in ts[3:6]])
+            if tiles is not None:
+                places = [t.data_ptr() for t in tiles.copies]
                 self._table[1].copy_(torch.tensor([[*a[:3], *places[3 * i:3 * i + 3], *a[6:]] for i, a in enumerate(self._addresses)], dtype=torch.int64))
-        return self._table
+            self._tiles, self._asked = tiles, True      # (once: captured steps of more rows are of one kind)
+        return self._table if self._tiles is not None or self._table.dim() == 2 else self._table[0]
 
-    def ready(self, rows: int) -> bool:
-        """In front of a step that is taken, or a replay of one: what is laid out of the matrices is what they hold. False: there is no memory for it."""
-        if rows > self.MOST_ROWS and not torch.cuda.is_current_stream_capturing():
+    def ready(self, rows: int) -> None:
+        """In front of a step that is taken, or a replay of one: what is laid out of the matrices is what they hold."""
+        if rows > self.MOST_ROWS:
             self.layers
-            if self._tiles is None:
-                return False
-            self._tiles.follow()
-        return True
+            if self._tiles is not None and not torch.cuda.is_current_stream_capturing():
+                self._tiles.follow()
 
     def gave_up(self) -> bool:
         return bool(self._failed[0])
@@ -315,5 +327,5 @@ class ResidentLayers:
     def forward(self, ctx, hidden: torch.Tensor) -> None:
         cos, sin = self.position.table(ctx.n_positions)
         with contextlib.nullcontext() if torch.cuda.is_current_stream_capturing() else self.turn:      # (one that is captured takes its turn at every replay)
-            ops.decode_resident(hidden, self._table, ctx.positions, ctx._tables[self.group], ctx._slots[self.group], cos, sin, self.area.address, self.failed, self.intermediate,
+            ops.decode_resident(hidden, self.layers if hidden.shape[0] > self.MOST_ROWS else self._few, ctx.positions, ctx._tables[self.group], ctx._slots[self.group], cos, sin, self.area.address, self.failed, self.intermediate,
                                 self.heads, self.kv_heads, self.d, self.page, self.biased, self.scale, self.eps)

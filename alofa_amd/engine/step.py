@@ -387,7 +387,9 @@ class StepFunction:
         buf["dev"].copy_(host["block"], non_blocking=True)
         host["copied"].record()
         ctx.want_slots = buf["request_slots"]
-        one_launch = self.resident is not None and self.resident.takes(ctx, B) and self.resident.ready(B)
+        one_launch = self.resident is not None and self.resident.takes(ctx, B)
+        if one_launch:
+            self.resident.ready(B)
         key = (B, ctx.max_context, greedy, one_launch)
         saved, self._scratch = self._scratch, buf["scratch"]   # graphs of one batch size share their own buffers
         chosen = self._chosen[:B]

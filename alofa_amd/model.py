@@ -103,7 +103,7 @@ class Model:
             b.prepare(n_positions)
 
     def weight_bytes(self) -> int:
-        """Bytes of device memory the model's tensors take (a tensor shared by two parts counts once)."""
+        """Bytes of device memory the model's tensors take (a tensor shared by two parts counts once), with the copies that decode steps of more than sixteen rows read once there are any."""
         seen, total = set(), 0
         stack = [self.embedding, self.final_norm, self.head, *self.joins, *self.blocks]
         while stack:
@@ -128,7 +128,8 @@ class Model:
             first.copy_(hidden)
         watch = getattr(ctx, "watch", None)      # (for tests and debugging: called with the stream after every run entry)
         resident = getattr(ctx, "resident", None)
-        if resident is not None and watch is None and resident.takes(ctx, rows) and resident.ready(rows):      # few rows of one new token each: every layer in one launch
+        if resident is not None and watch is None and resident.takes(ctx, rows):      # few rows of one new token each: every layer in one launch
+            resident.ready(rows)
             resident.forward(ctx, hidden)
             return hidden
         stream = hidden

@@ -1028,9 +1028,9 @@ def clear_resident_area(area: int) -> None:
 
 def decode_resident(hidden: torch.Tensor, layers: torch.Tensor, positions: torch.Tensor, block_table: torch.Tensor, slots: torch.Tensor, cos: torch.Tensor,
                     sin: torch.Tensor, area: int, failed: torch.Tensor, intermediate: int, heads: int, kv_heads: int, d: int, page: int, biased: bool, scale: float, eps: tuple, limit: int = 0) -> None:
-    """Every layer of a decode step, one new token per row, row i request i: ``hidden`` float32 [rows, width], in and out. ``layers`` int64 [2, layers, 10] (or [layers, 10], for up to
-    sixteen rows): the addresses of a layer's matrices, norms and caches, which the caller keeps alive and has checked, the second time with gate, up and down laid out in tiles (``in_tiles``), as more rows
-    than sixteen read them; ``area``: of ``resident_area``, used by one launch at a time; ``failed``: int32 [1] in
+    """Every layer of a decode step, one new token per row, row i request i: ``hidden`` float32 [rows, width], in and out. ``layers`` int64 [layers, 10]: the addresses of a
+    layer's matrices, norms and caches, which the caller keeps alive and has checked; or [2, layers, 10], the second time with gate, up and down laid out in tiles (``in_tiles``), which more rows than
+    sixteen then read; ``area``: of ``resident_area``, used by one launch at a time; ``failed``: int32 [1] in
     pinned memory, set if the kernel gives a wait up: the numbers that hang on it are NaN then.
     ``limit``: after how many asks, some microsecond each (0: the kernel's own limit, seconds)."""
     _contig("hidden", _gpu("hidden", hidden, torch.float32, 2))
@@ -1038,10 +1038,9 @@ def decode_resident(hidden: torch.Tensor, layers: torch.Tensor, positions: torch
     _contig("layers", _gpu("layers", layers, torch.int64, None))
     if layers.dim() not in (2, 3) or layers.shape[-1] != 10 or (layers.dim() == 3 and layers.shape[0] != 2):
         raise AlofaError("shape_mismatch", "a layer has ten addresses", f"layers={tuple(layers.shape)}")
+    tiled = layers.dim() == 3 and M > RESIDENT_ROWS
     if layers.dim() == 3:
-        layers = layers[int(M > RESIDENT_ROWS)]
-    elif M > RESIDENT_ROWS:
-        raise AlofaError("shape_mismatch", "more than sixteen rows read matrices laid out in tiles", f"rows={M} layers={tuple(layers.shape)}")
+        layers = layers[int(tiled)]
     _contig("block_table", _gpu("block_table", block_table, torch.int32, 2))
     for name, t, dtype in (("positions", positions, torch.int32), ("slots", slots, torch.int64)):
         if tuple(_contig(name, _gpu(name, t, dtype, 1)).shape) != (M,):
@@ -1052,7 +1051,7 @@ def decode_resident(hidden: torch.Tensor, layers: torch.Tensor, positions: torch
     if block_table.shape[0] < M or failed.dtype is not torch.int32 or not failed.is_pinned():
         raise AlofaError("shape_mismatch", "a row of pages per request, and a pinned word", f"table={tuple(block_table.shape)} rows={M}")
     _call("alofa_decode_resident", hidden, layers, positions, block_table, slots, cos, sin, _L(area), _L(failed.data_ptr()), _I(layers.shape[0]), _I(M), _I(H), _I(intermediate),
-          _I(heads), _I(kv_heads), _I(d), _I(page), _I(block_table.shape[1]), _I(bool(biased)), _I(limit), _F(scale), _F(eps[0]), _F(eps[1]), _L(_stream()))
+          _I(heads), _I(kv_heads), _I(d), _I(page), _I(block_table.shape[1]), _I(bool(biased)), _I(limit), _I(tiled), _F(scale), _F(eps[0]), _F(eps[1]), _L(_stream()))
 
 
 def can_fuse_rope_into_decode(d: int) -> bool:

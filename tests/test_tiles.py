@@ -22,19 +22,23 @@ def test_the_addresses_that_captured_steps_read_stay_where_they_are(monkeypatch)
     from types import SimpleNamespace as Some
     from alofa_amd import ops
     from alofa_amd.engine import resident
+    from alofa_amd.model import Model
     monkeypatch.setattr(resident, "_areas", resident._Areas()), monkeypatch.setattr(resident, "_turns", {})
     monkeypatch.setattr(ops, "resident_rows", lambda *a: 64), monkeypatch.setattr(ops, "check_caches", lambda *a: None)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: Some(synchronize=lambda: None)), monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
-    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: None)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda *a: (1 << 40, 1 << 40)), monkeypatch.setattr(torch.cuda, "memory_reserved", lambda *a: 0), monkeypatch.setattr(torch.cuda, "memory_allocated", lambda *a: 0)
     mixer = Some(heads=4, kv_heads=1, d=64, scale=1.0, position=None, hidden=256, b_qkv=None)
     block = Some(mixer=mixer, feed_forward=Some(intermediate=512), norms=[Some(as_rmsnorm=lambda: (None, 1e-6))] * 2)
     tables = [[torch.zeros(1), None, torch.zeros(1), torch.zeros(512, 256), torch.zeros(512, 256), torch.zeros(256, 512), *(torch.zeros(1) for _ in range(4))] for _ in range(3)]
-    model, cache = Some(tiles=None, written=0), Some(block_size=16, group_of_entry={(0, 0): 0})
+    model, cache = Model.__new__(Model), Some(block_size=16, group_of_entry={(0, 0): 0})
+    model.tiles = None
     layers = resident.ResidentLayers(model, [block] * 3, cache, torch.device("cpu"), tables, Some(failed=torch.zeros(1, dtype=torch.int32), address=0))
     held, at = layers._table, layers._table.data_ptr()
     before = held[0].clone()
-    assert layers.ready(16) and layers._tiles is None
-    assert layers.ready(17) and layers._tiles is not None
+    layers.ready(16)
+    assert layers._tiles is None
+    layers.ready(17)
+    assert layers._tiles is not None
     assert layers._table is held and held.data_ptr() == at and torch.equal(held[0], before)
     assert [held[1, i, 3:6].tolist() for i in range(3)] == [[t.data_ptr() for t in layers._tiles.copies[3 * i:3 * i + 3]] for i in range(3)]
     assert torch.equal(held[1][:, [0, 1, 2, 6, 7, 8, 9]], before[:, [0, 1, 2, 6, 7, 8, 9]])
@@ -53,7 +57,8 @@ def test_a_captured_step_of_few_rows_behind_one_of_many():
         m[1].tiles = None
         e = engine(m, 17, 400, "bfloat16")
         if first:
-            assert e.step_fn.resident.ready(17)
+            e.step_fn.resident.ready(17)
+            assert m[1].tiles is not None
         stand(e, lengths, 1)
         out = decode(e, steps[:4])
         replays = e.step_fn.graph_replays
@@ -105,19 +110,39 @@ def test_nothing_is_laid_out_before_a_step_of_more_than_sixteen_rows():
     assert m[1].weight_bytes() == size + 3 * 256 * 512 * 2 * len(m[1].order)
 
 
-@pytest.mark.gpu
-def test_without_memory_for_tiles_steps_run_kernel_by_kernel(monkeypatch):
+def steps_of(e, rows, launches):
+    from test_resident_gpu import decode, stand
+    stand(e, [5 + i for i in range(rows)], 1)
+    del launches[:]
+    out = decode(e, np.random.default_rng(rows).integers(0, 500, (3, rows)).tolist())
+    assert set(launches) <= {rows} and e.step_fn.graph_replays + len(launches) >= 3      # (all layers in one launch)
+    return out
+
+
+@pytest.fixture
+def launches(monkeypatch):
     from alofa_amd import ops
-    from test_resident_gpu import decode, engine, model, stand
+    made, one_launch = [], ops.decode_resident
+    monkeypatch.setattr(ops, "decode_resident", lambda hidden, *a, **how: (made.append(hidden.shape[0]), one_launch(hidden, *a, **how))[1])
+    return made
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,rows", [((256, 4, 1, 512), 17), ((320, 5, 5, 768), 30), ((896, 14, 2, 4864), 33), ((896, 14, 2, 4864), 64), ((1024, 16, 2, 2304), 20)])
+@pytest.mark.parametrize("why", ["no memory", "little room"])
+def test_matrices_are_read_as_they_are_where_no_tiles_are(shape, rows, why, monkeypatch, launches):
+    """One launch for all layers either way, and the same bits."""
+    from alofa_amd import ops
+    from test_resident_gpu import engine, model
+    want = steps_of(engine(model(*shape, "bfloat16"), rows, 200, "bfloat16"), rows, launches)
 
     def none(*a):
         raise torch.cuda.OutOfMemoryError("no memory")
-    monkeypatch.setattr(ops, "in_tiles", none)
-    e = engine(model(256, 4, 1, 512, "bfloat16"), 20, 100, "bfloat16")
-    stand(e, [5] * 20, 1)
-    launches, one_launch = [], ops.decode_resident
-    monkeypatch.setattr(ops, "decode_resident", lambda hidden, *a, **how: (launches.append(hidden.shape[0]), one_launch(hidden, *a, **how))[1])
-    out = decode(e, [[1] * 20])
-    assert not launches and bool(torch.isfinite(out[0]).all()) and e.step_fn.resident.most_rows == 16
-    decode(e, [[1] * 16])
-    assert set(launches) == {16}
+    if why == "no memory":
+        monkeypatch.setattr(ops, "in_tiles", none)
+    elif why == "little room":
+        monkeypatch.setattr(torch.cuda, "mem_get_info", lambda *a: (0, 1 << 38)), monkeypatch.setattr(torch.cuda, "memory_reserved", lambda *a: torch.cuda.memory_allocated(*a))
+    m = model(*shape, "bfloat16")
+    e = engine(m, rows, 200, "bfloat16")
+    got = steps_of(e, rows, launches)
+    assert m[1].tiles is None and all(torch.equal(a, b) for a, b in zip(want, got))
