@@ -7,8 +7,8 @@
 // weights no longer fit the registers: gate, up and down go through a ring of fragments in a phase, the first of them asked for before the phase's values are waited for, as all weights are there.
 // A compute unit takes a fragment of a row-major matrix (1 KB, sixteen rows' 64 bytes: sixteen lanes in a row bring sixteen lines) in 27 ns however many are on their way, 37 bytes a nanosecond, 1 KB
 // in one piece in 10 to 17: gate and up's 280 fragments of a block at four groups 7.5 us, down's 140 3.8. So these matrices come laid out in tiles, fragment behind fragment as the matrix cores take them
-// (kTiled; ops.in_tiles: copies, 26 MB a layer at the 0.5B sizes, made once per model when a step first needs them), and blocks take whole tiles of them; where there is no room for copies
-// a step reads these as they are: the same bits. Eight steps of the 0.5B sizes with logits behind
+// (kTiled; ops.in_tiles: copies, 26 MB a layer at the 0.5B sizes, made once per model when a step first needs them), and blocks take whole tiles of them; where there is no room for copies, or none that
+// follow what is written to the matrices, a step reads these as they are: the same bits. Eight steps of the 0.5B sizes with logits behind
 // the last, us, rows of the matrices / tiles: 64 rows of 128 to 2,048 keys 8,194 / 7,300, of 64 to 256 7,502 / 6,543, of 3,300 to 4,000 11,361 / 10,381, 48 of 128 to 1,024 7,372 / 6,485, 33 of 64 to 512
 // 7,068 / 6,195, 32 of 128 to 1,024 6,055 / 5,795, 17 of 64 to 700 5,711 / 5,405. Other widths (256 to 1,024) and feed-forwards (512 to 5,120), 12 layers, rows of 100 to 290 keys: 1.00 to 1.07 times as fast
 // at 17 and 32 rows, 1.06 to 1.18 at 33 and 64. Loads marked as read once (nt) lose half of it at four groups (7,806 for 7,374): the L2's other three readers; past the L1 (sc0) is even.

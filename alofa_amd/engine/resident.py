@@ -149,18 +149,19 @@ _turns: dict = {}      # GPU -> its launches' turns
 
 class _Tiles:
     """Copies of a model's gate, up and down matrices as more than sixteen rows read them (``ops.in_tiles``): made once per model, for all its step functions, and again where the matrices have been
-    written since."""
+    written since: as far as torch counts the writes, and where ``Model.weights_written`` says so."""
     ROOM = 2      # times their size that must be free before they are laid out: the rest is what a service's scratch grows into
 
-    def __init__(self, sources: list):
-        self._sources, self._lock = sources, threading.Lock()
+    def __init__(self, model, sources: list):
+        self._model, self._sources, self._lock = weakref.ref(model), sources, threading.Lock()
         versions = self._now()
         self.copies = [ops.in_tiles(w) for w in sources]
         torch.cuda.current_stream(sources[0].device).synchronize()      # (steps on other streams read them too)
         self._versions = versions
 
     def _now(self) -> list:
-        return [None if w.is_inference() else w._version for w in self._sources]
+        model = self._model()
+        return [None if model is None else model.written, *(w._version for w in self._sources)]
 
     def bytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self.copies)
@@ -180,16 +181,18 @@ class _Tiles:
 
     @staticmethod
     def of(model, sources: list) -> Optional["_Tiles"]:
-        """None where the matrices are read as they are instead: where there is no memory to spare."""
+        """None where the matrices are read as they are instead: where torch does not count the writes to them (inference tensors), or there is no memory to spare."""
         with _laying_out:
             have = model.tiles
             if have is None or len(have._sources) != len(sources) or any(a is not b for a, b in zip(have._sources, sources)):
+                if any(w.is_inference() for w in sources):
+                    return None
                 device = sources[0].device
                 free = torch.cuda.mem_get_info(device)[0] + torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
                 if free < _Tiles.ROOM * sum(w.numel() * w.element_size() for w in sources):
                     return None
                 try:
-                    model.tiles = _Tiles(sources)
+                    model.tiles = _Tiles(model, sources)
                 except torch.cuda.OutOfMemoryError:
                     return None
             return model.tiles

@@ -59,6 +59,7 @@ class Model:
         self.order = list(spec.order)
         self.descriptions = None      # (of the blocks, for engine/tapes.py)
         self.tiles = None             # (of matrices that were laid out again, for engine/resident.py)
+        self.written = 0              # (how often ``weights_written`` was called)
         self.streams = int(spec.streams)
         if any(b.on_streams != bool(self.streams) for b in self.blocks) or (self.streams and self.joins):
             raise AlofaError("unsupported", "blocks on copies of the stream go with a model that keeps copies, and with no joins", f"streams={self.streams}")
@@ -101,6 +102,11 @@ class Model:
     def prepare(self, n_positions: int) -> None:
         for b in self.blocks:
             b.prepare(n_positions)
+
+    def weights_written(self) -> None:
+        """To be called behind writes to the model's matrices that torch does not count, before the next step: through ``w.data``, or from a pointer (another library, another process). Writes that it counts
+        (``w.copy_``, an optimizer's) are seen without. Decode steps of more than sixteen rows read gate, up and down from copies, which are laid out again then; everything else reads the matrices."""
+        self.written += 1
 
     def weight_bytes(self) -> int:
         """Bytes of device memory the model's tensors take (a tensor shared by two parts counts once), with the copies that decode steps of more than sixteen rows read once there are any."""

@@ -31,7 +31,7 @@ def test_the_addresses_that_captured_steps_read_stay_where_they_are(monkeypatch)
     block = Some(mixer=mixer, feed_forward=Some(intermediate=512), norms=[Some(as_rmsnorm=lambda: (None, 1e-6))] * 2)
     tables = [[torch.zeros(1), None, torch.zeros(1), torch.zeros(512, 256), torch.zeros(512, 256), torch.zeros(256, 512), *(torch.zeros(1) for _ in range(4))] for _ in range(3)]
     model, cache = Model.__new__(Model), Some(block_size=16, group_of_entry={(0, 0): 0})
-    model.tiles = None
+    model.tiles, model.written = None, 0
     layers = resident.ResidentLayers(model, [block] * 3, cache, torch.device("cpu"), tables, Some(failed=torch.zeros(1, dtype=torch.int32), address=0))
     held, at = layers._table, layers._table.data_ptr()
     before = held[0].clone()
@@ -129,7 +129,7 @@ def launches(monkeypatch):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape,rows", [((256, 4, 1, 512), 17), ((320, 5, 5, 768), 30), ((896, 14, 2, 4864), 33), ((896, 14, 2, 4864), 64), ((1024, 16, 2, 2304), 20)])
-@pytest.mark.parametrize("why", ["no memory", "little room"])
+@pytest.mark.parametrize("why", ["no memory", "little room", "writes are not counted"])
 def test_matrices_are_read_as_they_are_where_no_tiles_are(shape, rows, why, monkeypatch, launches):
     """One launch for all layers either way, and the same bits."""
     from alofa_amd import ops
@@ -142,7 +142,33 @@ def test_matrices_are_read_as_they_are_where_no_tiles_are(shape, rows, why, monk
         monkeypatch.setattr(ops, "in_tiles", none)
     elif why == "little room":
         monkeypatch.setattr(torch.cuda, "mem_get_info", lambda *a: (0, 1 << 38)), monkeypatch.setattr(torch.cuda, "memory_reserved", lambda *a: torch.cuda.memory_allocated(*a))
-    m = model(*shape, "bfloat16")
+    with torch.inference_mode(why == "writes are not counted"):
+        m = model(*shape, "bfloat16")
+    assert m[1].blocks[0].feed_forward.w_down.is_inference() == (why == "writes are not counted")
     e = engine(m, rows, 200, "bfloat16")
     got = steps_of(e, rows, launches)
     assert m[1].tiles is None and all(torch.equal(a, b) for a, b in zip(want, got))
+    if why == "writes are not counted":      # (such a write is seen)
+        from test_resident_gpu import decode
+        with torch.inference_mode():
+            m[1].blocks[0].feed_forward.w_down.neg_()
+        assert not torch.equal(decode(e, [[1] * rows])[0], got[0])
+
+
+@pytest.mark.gpu
+def test_writes_that_are_not_counted_and_said(launches):
+    """Through ``.data``: seen by steps of up to sixteen rows at once, by steps of more behind ``weights_written``."""
+    from test_resident_gpu import engine, model
+    m = model(256, 4, 1, 512, "bfloat16")
+    e = engine(m, 20, 200, "bfloat16")
+    before = steps_of(e, 20, launches)
+    for i in range(20):
+        e.cache.free(i)
+    m[1].blocks[1].feed_forward.w_gate.data.neg_(), m[1].blocks[2].feed_forward.w_down.data.mul_(0.5)
+    m[1].weights_written()
+    got = steps_of(e, 20, launches)
+    other = model(256, 4, 1, 512, "bfloat16")
+    with torch.no_grad():
+        other[1].blocks[1].feed_forward.w_gate.neg_(), other[1].blocks[2].feed_forward.w_down.mul_(0.5)
+    want = steps_of(engine(other, 20, 200, "bfloat16"), 20, launches)
+    assert all(torch.equal(a, b) for a, b in zip(want, got)) and not torch.equal(before[0], got[0])
