@@ -168,6 +168,7 @@ class StepFunction:
         self._scratch: dict = {}
         self._views: dict = {}                   # per set of buffers: (name, dtype, shape) -> (buffer, its view of that shape)
         self._eager_scratch = self._scratch      # buffers of steps that run kernel by kernel
+        self.buffers_moved = 0                   # how often one was outgrown
         self._retired: list = []                 # outgrown buffers that captured graphs may still use
         self._eager_hosts: list = []             # pinned blocks the eager steps are laid out in, taking turns
         self._eager_turn = 0
@@ -214,6 +215,7 @@ class StepFunction:
                 # buffers, and a longer context needs more room for attention's partial results):
                 # it is kept for good, so that replays of the older graph write where nothing else lives
                 self._retired.append(buf)
+            self.buffers_moved += buf is not None
             buf = torch.empty(max(n, 1), dtype=dtype, device=self.device)
             self._scratch[key] = buf
         if known is None or known[0] is not buf or len(known[1]) >= 64:

@@ -163,6 +163,7 @@ class Model:
                 if watch is not None:
                     watch(i, hidden)
                 continue
+            moved = None if tapes is None else ctx.fn.buffers_moved
             # the norm the next block starts with may be left by this block's last product (a launch less)
             nxt = self.blocks[self.order[i + 1].layer] if i + 1 < len(self.order) and self.order[i + 1].join is None else None
             norm = nxt.wants_normed(rows) if nxt is not None and nxt.takes_normed else None
@@ -174,7 +175,8 @@ class Model:
                 given = normed is not None
                 with tapes.note(i) as noted:
                     normed = then[1] if block.forward(ctx, i, stream, normed, then) else None
-                tape = (i, noted, given, normed)
+                # (a buffer that was outgrown on the way is gone, and launches before have its address: the layers alike go through their parts this once)
+                tape = (i, noted, given, normed) if ctx.fn.buffers_moved == moved else None
                 continue
             normed = then[1] if block.forward(ctx, i, stream, normed, then) else None
         return hidden

@@ -62,6 +62,49 @@ def test_calls_are_made_again_with_another_layers_addresses(library, native):
         ways.play(tape, ())
 
 
+@pytest.mark.parametrize("grows", [False, True])
+def test_a_buffer_outgrown_while_a_layer_is_noted(grows):
+    """The noted launches before have the old buffer's address: the layers alike run through their parts in that step, and from their notes in the next."""
+    from contextlib import contextmanager
+    from types import SimpleNamespace as Some
+    from alofa_amd.engine.step import StepFunction
+    from alofa_amd.model import Model
+    ran, played = [], []
+
+    class Block:
+        takes_normed, wants_normed, can_leave = True, staticmethod(lambda rows: None), staticmethod(lambda norm: False)
+
+        def forward(self, ctx, i, stream, normed, then):
+            ran.append(i)
+            ctx.scratch("sums", (8,), torch.float32)
+            ctx.scratch("sums", (16 if grows and i else 8,), torch.float32)
+
+    class Tapes:
+        sources, source = {1}, {2: 1, 3: 1}
+
+        def stand(self):
+            return True
+
+        @contextmanager
+        def note(self, i):
+            yield Some(play=played.append)
+
+        def addresses(self, i):
+            return i
+    fn = StepFunction.__new__(StepFunction)
+    fn._scratch, fn._views, fn._retired, fn.buffers_moved, fn.device = {}, {}, [], 0, torch.device("cpu")
+    fn._eager_scratch = fn._scratch
+    model = Model.__new__(Model)
+    model.embedding, model.joins, model.streams, model.blocks = Some(forward=lambda ctx, ids: torch.zeros(2, 4)), [], 0, [Block()]
+    model.order, model.rt = [Some(layer=0, join=None)] * 5, Some(dtype=torch.float32)
+    ctx = Some(fn=fn, scratch=fn.scratch, watch=None, resident=None, tapes=Tapes())
+    model.forward(ctx, None)
+    assert (ran, played) == (([0, 1, 2, 3, 4], []) if grows else ([0, 1, 4], [2, 3]))
+    del ran[:], played[:]
+    model.forward(ctx, None)
+    assert (ran, played) == ([0, 1, 4], [2, 3])
+
+
 MODEL = {"architectures": ["Qwen2ForCausalLM"], "model_type": "qwen2", "num_hidden_layers": 7, "hidden_size": 256, "num_attention_heads": 4, "num_key_value_heads": 2, "intermediate_size": 512,
          "vocab_size": 500, "rope_theta": 10000.0, "rms_norm_eps": 1e-6, "tie_word_embeddings": True, "use_sliding_window": False, "max_position_embeddings": 2048}
 WINDOWS = {**MODEL, "use_sliding_window": True, "sliding_window": 40, "max_window_layers": 3}
