@@ -145,6 +145,8 @@ class Model:
             normed = ctx.scratch("normed", tuple(hidden.shape), self.rt.dtype)
             ops.streams_step(stream, source=hidden, w_in=read.weights, norm=read.norm, out=normed, exact=self.rt.exact)
         tapes = getattr(ctx, "tapes", None) if watch is None else None
+        if tapes is not None and not tapes.stand():
+            tapes = None
         tape = None      # (the launches of the last entry that others are alike, whether a norm was left for it, and what it left)
         for i, e in enumerate(self.order):
             block = self.blocks[e.layer]

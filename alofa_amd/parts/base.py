@@ -141,6 +141,12 @@ class Part:
         self.rt = rt
 
 
+def repeats(part) -> bool:
+    """Whether the part's class says ``repeatable`` itself: that all it does on the device is launches of this package's kernels on its own tensors, its cache and buffers that the step keeps, chosen by
+    sizes alone, so that a part like it may be run by making them again (``engine/tapes.py``). Not what a class it derives from says: it may do something else."""
+    return "repeatable" in vars(type(part)) and bool(part.repeatable)
+
+
 class Mixer(Part):
     """``where`` names the mixer's place in the run: the run entry, or (entry, k) for the k-th
     mixer of a block that has several; it is what ``ctx.kv`` and ``ctx.state`` are asked with."""

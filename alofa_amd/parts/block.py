@@ -26,7 +26,7 @@ from .. import ops
 from ..config.base import PartSpec
 from ..errors import AlofaError
 from ..weights.loader import TensorRule
-from .base import Block, build_part, register_part, tensors_of
+from .base import Block, build_part, register_part, repeats, tensors_of
 
 
 class PreNormBlock(Block):
@@ -61,9 +61,7 @@ class PreNormBlock(Block):
 
     @property
     def repeatable(self):
-        """Whether all that the block does on the device is launches of this package's kernels on its own tensors, its cache and buffers that the step keeps, chosen by sizes alone: another block like it
-        may then be run by making them again (``engine/tapes.py``)."""
-        return all(n.as_rmsnorm() is not None for n in self.norms) and all(getattr(p, "repeatable", False) for p in (self.mixer, self.feed_forward))
+        return all(n.as_rmsnorm() is not None and repeats(n) for n in self.norms) and all(repeats(p) for p in (self.mixer, self.feed_forward))
 
     def forward(self, ctx, entry, hidden, normed=None, then=None):
         """``normed``: the first norm's rows, where the block before has left them; ``then`` = (norm, rows): the norm

@@ -27,6 +27,8 @@ class RMSNorm(Norm):
         weight = weights[spec.params["name"]]
         self.weight = rt.vector(weight.float().reshape(1).repeat(self.width) if spec.params.get("scalar", False) else weight)
 
+    repeatable = True
+
     def as_rmsnorm(self):
         return self.weight, self.eps
 

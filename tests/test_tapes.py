@@ -110,6 +110,87 @@ MODEL = {"architectures": ["Qwen2ForCausalLM"], "model_type": "qwen2", "num_hidd
 WINDOWS = {**MODEL, "use_sliding_window": True, "sliding_window": 40, "max_window_layers": 3}
 
 
+def alike(change=lambda model: None, layers=6):
+    """Which layers of a small model on the CPU are taken for alike once ``change`` has been at it, and the model and its notes."""
+    from types import SimpleNamespace as Some
+    from alofa_amd.config import config_from_dict
+    from alofa_amd.engine.tapes import LayerTapes
+    from alofa_amd.model import Model
+    from alofa_amd.parts.base import Runtime
+    config = config_from_dict({**MODEL, "num_hidden_layers": layers, "hidden_size": 64, "num_attention_heads": 2, "num_key_value_heads": 1, "intermediate_size": 64, "vocab_size": 20})
+    w = {"model.embed_tokens.weight": torch.zeros(20, 64), "model.norm.weight": torch.ones(64)}
+    for i in range(layers):
+        pre = f"model.layers.{i}."
+        for n, rows, cols in (("self_attn.q_proj", 64, 64), ("self_attn.k_proj", 32, 64), ("self_attn.v_proj", 32, 64), ("self_attn.o_proj", 64, 64), ("mlp.gate_proj", 64, 64), ("mlp.up_proj", 64, 64), ("mlp.down_proj", 64, 64)):
+            w[pre + n + ".weight"] = torch.zeros(rows, cols, dtype=torch.bfloat16)
+            if n[-6] in "qkv" and n.startswith("self"):
+                w[pre + n + ".bias"] = torch.zeros(rows)
+        for n in ("input_layernorm", "post_attention_layernorm"):
+            w[pre + n + ".weight"] = torch.ones(64)
+    model = Model(config.spec(), w, Runtime(torch.device("cpu"), torch.bfloat16))
+    cache = Some(tensors={(i, 0): {"k": torch.zeros(8), "v": torch.zeros(8)} for i in range(layers)}, group_of_entry={(i, 0): 0 for i in range(layers)})
+    change(model)
+    made = LayerTapes.of(model, cache)
+    return {} if made is None else made.source, model, made, cache
+
+
+def test_which_layers_are_alike():
+    assert alike()[0] == {2: 1, 3: 1, 4: 1}      # (the first has the embedding in front of it, the last no layer behind)
+
+    def other_numbers(model):
+        for i, b in enumerate(model.blocks):
+            b.mixer.numbers = np.arange(5000) * (2 if i == 3 else 1)      # (alike at either end, as an array is written out)
+            b.mixer.numbers[[*range(10), *range(-10, 0)]] = 0
+    assert alike(other_numbers)[0] == {2: 1} or alike(other_numbers)[0] == {}
+    assert 3 not in alike(other_numbers)[0]
+
+    def named(model):
+        for i, b in enumerate(model.blocks):
+            b.feed_forward.more = {"w": torch.zeros(4, 4) if i != 3 else torch.zeros(4, 5), "rest": [1.0, None]}
+    assert 3 not in alike(named)[0] and alike(lambda m: [setattr(b.feed_forward, "more", {"w": torch.zeros(4, 4)}) for b in m.blocks])[0] == {2: 1, 3: 1, 4: 1}
+    shared, own = object(), [object() for _ in range(6)]
+    assert alike(lambda m: [setattr(b.mixer, "x", shared) for b in m.blocks])[0] == {2: 1, 3: 1, 4: 1}
+    assert alike(lambda m: [setattr(b.mixer, "x", x) for b, x in zip(m.blocks, own)])[0] == {}
+
+
+def test_a_class_says_for_itself_that_it_may_be_run_so():
+    from alofa_amd.parts.feed_forward import SwiGLU
+
+    class Sum(SwiGLU):
+        def forward(self, ctx, x, residual, **how):
+            residual += x
+    assert alike(lambda m: [setattr(b.feed_forward, "__class__", Sum) for b in m.blocks])[0] == {}
+
+
+def test_matrices_that_are_replaced():
+    """Behind the step function: its steps go through the parts. Another step function of the model has the new one."""
+    from alofa_amd.engine.tapes import LayerTapes
+    source, model, made, cache = alike()
+    assert made.stand()
+    model.blocks[3].feed_forward.w_down = torch.ones(64, 64, dtype=torch.bfloat16)
+    assert not made.stand()
+    again = LayerTapes.of(model, cache)
+    assert again.source == source and again.stand() and model.blocks[3].feed_forward.w_down.data_ptr() in again.addresses(3) and model.blocks[3].feed_forward.w_down.data_ptr() not in made.addresses(3)
+    model.blocks[2].norms[1] = model.blocks[1].norms[1]
+    assert not again.stand()
+    _, model, made, cache = alike()
+    model.blocks[4].mixer.window = 40
+    assert LayerTapes.of(model, cache).source == {2: 1}      # (three has another layer behind it then)
+
+
+def test_what_is_asked_of_the_library_is_no_launch():
+    """Launches are noted by ``_call``: what ops asks by ``_answer`` takes no stream."""
+    import re
+    from conftest import ROOT
+    ops = (ROOT / "alofa_amd" / "ops.py").read_text()
+    code = "\n".join(f.read_text() for f in sorted((ROOT / "alofa_amd" / "csrc").glob("*.hip")))
+    asked = set(re.findall(r'_answer\("(\w+)"', ops)) | set(re.findall(r"load\(\)\.(alofa_\w+)\(", ops))
+    assert len(asked) >= 6
+    for name in asked:
+        found = re.search(r'extern "C" [\w* ]+?\b' + name + r"\(([^)]*)\)", code)
+        assert found and "hipStream_t" not in found.group(1), name
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
 @pytest.mark.parametrize("config", [MODEL, WINDOWS], ids=["alike", "two kinds of layers"])
