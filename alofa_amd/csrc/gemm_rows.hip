@@ -313,6 +313,7 @@ template <int MR, int C, int kEpilogue, typename TO>
 __global__ void __launch_bounds__(64 * rows_long_waves(MR)) gemm_rows_long_kernel(
     TO* __restrict__ out, int64_t ldo, const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int64_t ldw,
     const float* __restrict__ bias, int M, int N, int K, RowsDepth depth) {
+  static_assert(kEpilogue == kRwStore || kEpilogue == kRwResidual || kEpilogue == kRwDepth, "plain products, and an average over depth behind one");
   constexpr int V = C * MR, kWaves = rows_long_waves(MR);
   __shared__ float red[kWaves][V];
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
@@ -357,7 +358,7 @@ __global__ void __launch_bounds__(64 * rows_long_waves(MR)) gemm_rows_long_kerne
   float add = 0.f;
   DepthOf<kEpilogue == kRwDepth> levels;
   if (finisher) {
-    if ((kEpilogue == kRwStore || kEpilogue == kRwActivated) && bias) add = bias[n0 + my_c];
+    if (kEpilogue == kRwStore && bias) add = bias[n0 + my_c];
     if (kEpilogue == kRwResidual || kEpilogue == kRwDepth) add = load_f32(out + static_cast<int64_t>(my_m) * ldo + n0 + my_c);
     levels.ask(depth, my_m, n0 + my_c);
   }
