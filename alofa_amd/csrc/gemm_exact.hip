@@ -510,14 +510,15 @@ static int launch_exact_tile(float* out, int64_t ldo, const float* A, int64_t ld
   return check_launch("gemm_exact_tile");
 }
 
-// Gate and up of more than 64 rows: whether tiles of 96 rows come out sooner than those of 64. A compute unit takes a round's time for each of its blocks, whether they lie side by side or not, 31.5 us
-// a block of 64 rows and 47 of 96 against K of 896 (56 of whose registers are kept in memory), so it is the whole rounds that count: 9,728 x 896 against 66 to 96 rows (304 blocks of 64 rows, 152 of 96)
-// 64.9 / 51, 385 to 480 (1,064 and more, 760) 154 / 142; 130 (456, 304) 65 / 93, 300 (760, 608) 96 / 142.
+// Gate and up of more than 64 rows: whether tiles of 96 rows come out sooner than those of 64. A compute unit takes a round's time for each of its blocks, whether they lie side by side or not, so it is
+// the whole rounds that count, and a block of 96 rows (56 of whose registers are kept in memory) takes 1.55 times what one of 64 takes (31.5 us against K of 896). us, 64 / 96 rows a block, by their rounds:
+// 2 and 1, 66 rows of 4,864 x 896 64.9 / 51; 5 and 3, 96 of 18,944 x 1,536 1.10 times as fast; 11 and 7, 480 of 11,008 x 1,536 1.03; 3 and 2 of 64: 65 of 8,960 x 128 19.6 / 20.9, 96 of 8,960 x 896
+// 97.7 / 100.6, 240 of 4,864 x 3,584 357 / 371 (K from 128 to 5,120, 69 sizes: at the median 0.98 times as fast); 6 and 4 0.985; 3 and 3, 300 of 4,864 x 896 96 / 142.
 static bool taller_tiles(int M, int N) {
   if (M <= 64) return false;
   const int64_t columns = (N + 31) / 32, cus = compute_units();
   auto rounds = [&](int rows) { return (columns * ((M + rows - 1) / rows) + cus - 1) / cus; };
-  return 47 * rounds(96) < 31.5 * rounds(64);
+  return 31 * rounds(96) < 20 * rounds(64);
 }
 
 template <int kMats, int kEpilogue>
@@ -574,6 +575,9 @@ extern "C" int alofa_gemm_exact_norm(float* out, int64_t ldo, const float* A, in
   ALOFA_REQUIRE(aligned(out) && aligned(parts) && aligned(norm_w) && aligned(normed) && ldo % 4 == 0 && ld % 4 == 0, "gemm: the norm behind the product takes 16-byte aligned rows");
   return launch_exact<1, kExactResidual>(out, ldo, A, lda, W, W, ldw, nullptr, parts, M, N, K, 0, ExactNorm{norm_w, eps, normed, ld}, stream);
 }
+
+// Rows of a block's tile of gate and up.
+extern "C" int alofa_gemm_swiglu_exact_tile(int M, int N) { return M <= kExactRows ? 16 : taller_tiles(M, N) ? 96 : M <= 32 ? 32 : 64; }
 
 extern "C" int alofa_gemm_swiglu_exact(float* out, int64_t ldo, const float* A, int64_t lda, const float* Wg, const float* Wu, int64_t ldw, int M, int N, int K,
                                        int gelu, hipStream_t stream) {

@@ -101,6 +101,17 @@ def test_exact_gate_and_up_of_taller_tiles(M, N, K):
 
 
 # slabs of 32 k: none whole, one to seven, with and without a rest, rows that are not 16-byte aligned, shares of unequal length
+def test_taller_tiles_where_their_rounds_are_the_shorter():
+    """A tile of 96 rows takes 1.55 times as long as one of 64: two rounds of the one do not make up for three of the other."""
+    from alofa_amd.csrc.build import load
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for M in (65, 96, 130, 190, 240, 390, 450, 480, 576, 960):
+        for N in (1024, 2432, 4864, 5632, 8960, 11008, 13824, 18944):
+            low, tall = (-(-(-(-N // 32) * -(-M // rows)) // cus) for rows in (64, 96))
+            assert load().alofa_gemm_swiglu_exact_tile(M, N) == (96 if 1.55 * tall < low else 64), (M, N, low, tall)
+    assert [load().alofa_gemm_swiglu_exact_tile(M, 4864) for M in (16, 17, 32, 33, 64)] == [16, 32, 32, 64, 64]
+
+
 @pytest.mark.parametrize("M,N,K,shift", [(17, 40, 20, 0), (33, 70, 32, 0), (33, 70, 52, 0), (65, 70, 64, 0), (20, 140, 96, 0), (65, 70, 99, 0), (40, 64, 128, 0), (64, 64, 160, 1), (90, 70, 190, 1),
                                          (40, 70, 228, 0), (200, 64, 1100, 0)])
 def test_exact_products_by_slabs(M, N, K, shift):
