@@ -132,6 +132,14 @@ struct DepthOf {
   }
 };
 
+// The squares of four values added up. Written out, as left to itself the compiler starts with x or with y as the code around it happens to be: one unit in the last place of a row's factor, and with it now and
+// then an output's rounding. One row alone starts with x, several with y.
+template <bool kFirstX>
+__device__ __forceinline__ float squares_of(float4 v) {
+  const float two = kFirstX ? __builtin_fmaf(v.y, v.y, v.x * v.x) : __builtin_fmaf(v.x, v.x, v.y * v.y);
+  return __builtin_fmaf(v.w, v.w, __builtin_fmaf(v.z, v.z, two));
+}
+
 // MR: rows computed (1, 2, 4, 8, or 16 for plain products; rows beyond M are not stored); C: columns per block; kRwSwiglu: W is the gate
 // matrix and W2 the up matrix, same columns; TO: float or bf16_t; kMaxWaves: bound of the block's waves.
 template <int MR, int C, int kEpilogue, typename TO, bool kNorm, int kMaxWaves>
@@ -208,8 +216,7 @@ __device__ __forceinline__ void rows_block(
 #pragma unroll
     for (int m = 0; m < MR; ++m) {
       const float4 a = xlo[m], b = xhi[m];
-      ss[m] = a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w;
-      ss[m] += b.x * b.x + b.y * b.y + b.z * b.z + b.w * b.w;
+      ss[m] = squares_of<MR == 1>(a) + squares_of<MR == 1>(b);
       av[m] = make_uint4(pack_bf16x2(a.x * nlo.x, a.y * nlo.y), pack_bf16x2(a.z * nlo.z, a.w * nlo.w),
                          pack_bf16x2(b.x * nhi.x, b.y * nhi.y), pack_bf16x2(b.z * nhi.z, b.w * nhi.w));
     }

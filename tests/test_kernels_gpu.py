@@ -1529,3 +1529,46 @@ def test_attention_of_many_rows_is_as_exact_as_the_kernel_for_all_sizes(heads, k
             far[i] += ((got[:, h * d:(h + 1) * d].double() - want) ** 2).sum().item()
     # both follow the maxima of the even and of the odd tiles and round the same weights and results; what differs is the order of float sums
     assert far[1] <= 1.005 ** 2 * far[0], (far[0] ** 0.5, far[1] ** 0.5)
+
+
+def test_the_order_of_a_normed_rows_squares():
+    """The vector-unit product adds four neighbouring squares up by fused steps, from x on for a single row and from y on for several. A row (x, y, 0, 0) whose sum depends on that has a row (0, 0, z, 0) beside
+    it with the sum that it should have, and one with the other: all columns' outputs are the first's and not the second's (the columns' weights read the channels behind, which the rows share)."""
+    from alofa_amd import ops
+    rng, f32 = np.random.default_rng(0), np.float32
+
+    def fused(a, c):      # a * a + c with one rounding
+        return f32(np.float64(a) * np.float64(a) + np.float64(c))
+
+    def root(t):          # z with z * z == t, or None
+        z = f32(np.sqrt(np.float64(t)))
+        return next((c for c in (z, np.nextafter(z, f32(9)), np.nextafter(z, f32(0))) if c * c == t), None)
+    rows = []
+    while len(rows) < 24:
+        x, y = rng.uniform(0.7, 2.0, 2).astype(f32)
+        from_x, from_y = fused(y, x * x), fused(x, y * y)
+        roots = root(from_x), root(from_y)
+        if from_x != from_y and None not in roots:
+            tail = (rng.uniform(0.1, 0.3, 4)).astype(f32)
+            rows.append(np.stack([np.concatenate([head, tail]) for head in ((x, y, 0, 0), (0, 0, roots[0], 0), (0, 0, roots[1], 0))]).astype(f32))
+    w = torch.zeros(1 << 17, 8)
+    w[:, 4:] = torch.from_numpy(rng.standard_normal((1 << 17, 4)).astype(f32))
+    w, ones = w.bfloat16().to(DEV), torch.ones(8, device=DEV)
+
+    def outputs(a):
+        out = torch.empty(a.shape[0], w.shape[0], dtype=torch.bfloat16, device=DEV)
+        ops.gemm(out, torch.from_numpy(a).to(DEV), w, norm=(ones, 1e-30), kernel="rows")
+        return out
+    told_apart = {1: 0, 2: 0, 4: 0, 8: 0}
+    for r in rows:
+        for many in told_apart:
+            if many == 1:
+                mine, from_x, from_y = (outputs(r[i:i + 1])[0] for i in range(3))
+            elif many == 2:
+                mine, from_x, from_y = *outputs(r[:2]), outputs(r[1:])[1]
+            else:
+                mine, from_x, from_y = outputs(np.tile(r, (many // 3 + 1, 1))[:many - 1])[:3]
+            want, other = (from_x, from_y) if many == 1 else (from_y, from_x)
+            assert mine.equal(want), many
+            told_apart[many] += not mine.equal(other)
+    assert all(told_apart.values()), told_apart
