@@ -5,7 +5,8 @@
 //   its read-outs            o_t = g^(t+1) S^T q_t + sum_(s <= t) g^(t-s) (q_t . k_s) v_s     (chunk_read: every chunk by itself)
 // All products run in float on the matrix cores (v_mfma_f32_16x16x4_f32: lane l holds A row and B column l % 16 at reduction index l / 16,
 // and D column l % 16, rows 4 (l / 16) .. + 3), on operands that are bfloat16 numbers times a power of g, so nothing but float rounding
-// separates the result from the recurrence row by row. q, k, v come as bfloat16 rows; the powers g^0 .. g^64 from a table; q is
+// separates the result from the recurrence row by row, as long as values are finite: an infinity or NaN in a value meets the zeros that stand
+// for the queries in front of it, so that up to fifteen rows before it in its sixteen read out NaN too. q, k, v come as bfloat16 rows; the powers g^0 .. g^64 from a table; q is
 // scaled by q_scale and k by k_scale.
 //
 // Chunks: int32 [n_chunks, 4]: request, first row, rows (<= 64), 0; a request's chunks lie together, in its rows' order, and
